@@ -245,9 +245,12 @@ int of3_attn_pair_bias_fwd(const void* a, const void* pair_bias, const float* ma
  * single_transition, pairformer.py:118-122, :203-212): x, out contiguous [rows][C] (any leading
  * dimensions flattened; out may alias x), mask fp32 [rows] or null.  bf16: C = 384, HID a
  * multiple of 384 up to 1920, the workspace holds the hidden activations [rows][HID]; fp32: C <= 512,
- * HID <= 2048, no workspace (null, 0 is accepted). */
+ * HID <= 2048, no workspace needed (null, 0 is accepted).  With C and HID multiples of 32, 16-byte
+ * aligned tensors and a workspace of ..._fast_workspace_bytes the fp32 products run on the matrix
+ * instructions (the same for bf16 as ..._workspace_bytes). */
 int64_t of3_transition_rows_workspace_bytes(int64_t rows, int64_t C, int64_t HID);
 int64_t of3_transition_rows_workspace_bytes_for(int dtype, int64_t rows, int64_t C, int64_t HID);
+int64_t of3_transition_rows_fast_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t HID);
 int of3_transition_rows_fwd(const void* x, const float* mask, const void* ln_w, const void* ln_b, const void* w_a,
                             const void* w_b, const void* w_out, void* out, int64_t rows, int64_t C, int64_t HID,
                             int add_residual, void* workspace, int64_t workspace_bytes, int dtype, void* stream);

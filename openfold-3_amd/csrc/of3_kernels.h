@@ -165,7 +165,7 @@ struct RowTransitionArgs {
 };
 hipError_t row_transition_launch(const RowTransitionArgs& args, hipStream_t stream);
 
-// ---- fp32 versions of the single-representation kernels (single_f32.hip)
+// ---- fp32 versions of the single-representation kernels (single_f32.hip, single_x3_f32.hip)
 struct SingleAttnF32Args {
   const float* a;            // [B][N][C]
   const float* pair_bias;    // [B][H][N][N]
@@ -177,16 +177,22 @@ struct SingleAttnF32Args {
   int B, N, C, H, D, add_residual;
 };
 hipError_t single_attn_fwd_f32(const SingleAttnF32Args& args, hipStream_t stream);
+// the same on split operands; single_attn_fwd_f32 hands over what it serves
+bool single_attn_x3_serves(const SingleAttnF32Args& args);
+hipError_t single_attn_x3_fwd_f32(const SingleAttnF32Args& args, hipStream_t stream);
 
 struct RowTransitionF32Args {
   const float* x;
   const float* mask;
   const float *ln_w, *ln_b, *wa, *wb, *wout;
+  float* hidden;  // workspace, [rows][HID], 16-byte aligned; may be null (then the plain FMA kernel runs)
   float* out;
   long rows;
   int C, HID, add_residual;
 };
 hipError_t row_transition_fwd_f32(const RowTransitionF32Args& args, hipStream_t stream);
+bool row_transition_x3_serves(const RowTransitionF32Args& args);
+hipError_t row_transition_x3_fwd_f32(const RowTransitionF32Args& args, hipStream_t stream);
 
 // ---- fp32 path (pair_f32.hip): whole updates, any N, C and C_hidden <= 256, head width 16/32/64
 struct TrimulF32Args {

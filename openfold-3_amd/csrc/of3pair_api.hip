@@ -793,7 +793,13 @@ int64_t of3_transition_rows_workspace_bytes_for(int dtype, int64_t rows, int64_t
   if (dtype == OF3_DTYPE_BF16) return of3_transition_rows_workspace_bytes(rows, C, HID);
   if (dtype != OF3_DTYPE_F32 || rows < 1 || rows > (1ll << 31) || C < 1 || C > 512 || HID < 1 || HID > 2048)
     return OF3_EINVAL;
-  return 0;  // the hidden activations stay on chip
+  return 0;  // the hidden activations stay on chip (of3_transition_rows_fast_workspace_bytes: room for the faster kernels)
+}
+
+int64_t of3_transition_rows_fast_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t HID) {
+  const int64_t need = of3_transition_rows_workspace_bytes_for(dtype, rows, C, HID);
+  if (need < 0 || dtype == OF3_DTYPE_BF16) return need;
+  return C % 32 == 0 && HID % 32 == 0 ? align256(rows * HID * 4) : need;
 }
 
 int of3_transition_rows_fwd(const void* x, const float* mask, const void* ln_w, const void* ln_b, const void* w_a,
@@ -814,6 +820,9 @@ int of3_transition_rows_fwd(const void* x, const float* mask, const void* ln_w, 
     a.wa = f(w_a);
     a.wb = f(w_b);
     a.wout = f(w_out);
+    // with room for the hidden activations the matrix-instruction kernels run (where the shape allows)
+    const int64_t fast = of3_transition_rows_fast_workspace_bytes(dtype, rows, C, HID);
+    a.hidden = workspace && fast > 0 && workspace_bytes >= fast ? static_cast<float*>(workspace) : nullptr;
     a.out = static_cast<float*>(out);
     a.rows = (long)rows;
     a.C = (int)C;

@@ -1,8 +1,10 @@
 // fp32 versions of the single-representation kernels (AttentionPairBias of the trunk,
 // attention_pair_bias.py:189-244, and the SwiGLU transition over s, transition.py:225-271): plain
 // fp32 FMA arithmetic in the reference's order of operations, any N, C_s <= 512, head width
-// <= 64, hidden width <= 2048.  The precision path, not a fast one: the linear layers give a thread
-// one output channel and stage the weights through LDS, the attention gives a thread one query.
+// <= 64, hidden width <= 2048.  These serve the shapes that the matrix-instruction kernels of
+// single_x3_f32.hip do not (channel counts off the multiples of 32, unaligned tensors, a transition called
+// without a workspace): the linear layers give a thread one output channel and stage the weights through
+// LDS, the attention gives a thread one query.
 #include "of3_device.h"
 #include "of3_kernels.h"
 #include "of3_launch.h"
@@ -320,6 +322,7 @@ hipError_t single_attn_fwd_f32(const SingleAttnF32Args& a, hipStream_t stream) {
   if (a.C < 1 || a.C > kMaxCs || a.H < 1 || a.D < 1 || a.D > 64 || a.H * a.D > kMaxCs || a.N < 1 || a.B < 1 ||
       a.B > 65535 || a.H > 65535)
     return hipErrorInvalidValue;
+  if (single_attn_x3_serves(a)) return single_attn_x3_fwd_f32(a, stream);
   const long rows = (long)a.B * a.N;
   const long blocks = (rows + kRows - 1) / kRows;
   if (blocks > 0x7fffffffl) return hipErrorInvalidValue;
@@ -340,6 +343,7 @@ hipError_t single_attn_fwd_f32(const SingleAttnF32Args& a, hipStream_t stream) {
 
 hipError_t row_transition_fwd_f32(const RowTransitionF32Args& a, hipStream_t stream) {
   if (a.rows < 1 || a.C < 1 || a.C > kMaxCs || a.HID < 1 || a.HID > kMaxHidden) return hipErrorInvalidValue;
+  if (row_transition_x3_serves(a)) return row_transition_x3_fwd_f32(a, stream);
   const long blocks = (a.rows + kRows - 1) / kRows;
   if (blocks > 0x7fffffffl) return hipErrorInvalidValue;
   const hipError_t e = allow_dynamic_lds<row_transition_f32>(kWTileBytes);

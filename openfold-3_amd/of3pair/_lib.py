@@ -51,6 +51,7 @@ SIGNATURES = {
     "of3_attn_pair_bias_workspace_bytes": (c_int64, [c_int64] * 5),
     "of3_attn_pair_bias_workspace_bytes_for": (c_int64, [c_int] + [c_int64] * 5),
     "of3_transition_rows_workspace_bytes_for": (c_int64, [c_int] + [c_int64] * 3),
+    "of3_transition_rows_fast_workspace_bytes": (c_int64, [c_int] + [c_int64] * 3),
     "of3_attn_pair_bias_fwd": (c_int, [c_void_p] * 12 + [c_int64] * 5 + [ctypes.c_float, c_int, c_void_p, c_int64, c_int,
                                                                     c_void_p]),
     "of3_transition_rows_workspace_bytes": (c_int64, [c_int64] * 3),

@@ -262,7 +262,7 @@ def _swiglu_transition_rows(x, mask, norm_weight, norm_bias, a_weight, b_weight,
         if tuple(mask.shape) != tuple(x.shape[:-1]):
             mask = mask.expand(*x.shape[:-1])
         m = mask.to(torch.float32).contiguous()
-    need = lib.of3_transition_rows_workspace_bytes_for(code, rows, C, HID)
+    need = lib.of3_transition_rows_fast_workspace_bytes(code, rows, C, HID)
     if need < 0 and code == _lib.OF3_DTYPE_BF16 and lib.of3_transition_rows_workspace_bytes_for(_lib.OF3_DTYPE_F32, rows, C, HID) >= 0:
         # widths the bf16 kernels do not serve: the fp32 kernel on widened activations, rounded once at the end
         upd = _swiglu_transition_rows(x.float(), mask, norm_weight, norm_bias, a_weight, b_weight, out_weight, add_residual,
