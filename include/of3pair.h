@@ -272,6 +272,43 @@ int of3_layer_norm_fwd(const void* x, const void* ln_w, const void* ln_b, void* 
 int of3_template_tail_fwd(const void* t, const void* ln_w, const void* ln_b, const void* w, void* out, int64_t B,
                           int64_t T, int64_t P, int64_t C_t, int64_t C_z, int apply_ln, int dtype, void* stream);
 
+/* ---- whole blocks in one call ------------------------------------------------------------ */
+
+/* A PairBlock (base_blocks.py:307-480; a TemplatePairBlock, template_module.py:148-166) as one call: the
+ * two triangle multiplications (outgoing, incoming), the two triangle attentions (starting, ending node),
+ * each with its residual add, and the pair transition when HID is not 0.  out uses z's strides and may
+ * alias z; otherwise z is left intact.  weights: OF3_PAIR_BLOCK_WEIGHTS device pointers (the last five are
+ * not read when HID is 0) in the order of the arguments of the entry points above:
+ *   of3_trimul_fwd's ten (ln_in_w ... w_z) of the outgoing module, ten of the incoming one,
+ *   of3_triattn_fwd's eight (ln_w ... w_o) of the starting node, eight of the ending node,
+ *   of3_transition_fwd's five (ln_w ... w_out).
+ * flags: OF3_BLOCK_ATTENTION_FIRST runs the attentions before the multiplications,
+ * OF3_BLOCK_TRANSITION_UNMASKED gives the transition no mask.  Same shapes, results and launches as the
+ * single calls; everything is checked before the first launch. */
+#define OF3_PAIR_BLOCK_WEIGHTS 41
+#define OF3_BLOCK_ATTENTION_FIRST 1
+#define OF3_BLOCK_TRANSITION_UNMASKED 2
+int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
+                                       int64_t HID);
+int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t z_strides[3], const float* mask,
+                       const int64_t mask_strides[3], void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H,
+                       int64_t D, int64_t HID, float inf, int flags, void* workspace, int64_t workspace_bytes, int dtype,
+                       void* stream);
+
+/* A PairFormerBlock (pairformer.py:173-215) as one call: the PairBlock above on z, then s + attention with
+ * z's pair bias, then s + transition of s (unmasked with OF3_BLOCK_TRANSITION_UNMASKED).  s, s_out:
+ * contiguous [B][N][C_s], s_out may alias s; single_mask: fp32 [B][N] or null.  weights: the PairBlock's,
+ * then layer_norm_z weight and bias (may be null) and linear_z, layer_norm_a weight and bias, linear_q weight
+ * and bias, linear_k, linear_v, linear_g, linear_o, then of3_transition_rows_fwd's five. */
+#define OF3_PAIRFORMER_BLOCK_WEIGHTS 57
+int64_t of3_pairformer_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
+                                             int64_t HID, int64_t C_s, int64_t H_s, int64_t D_s, int64_t HID_s);
+int of3_pairformer_block_fwd(const void* const* weights, const void* s, const void* z, const int64_t z_strides[3],
+                             const float* single_mask, const float* pair_mask, const int64_t mask_strides[3], void* s_out,
+                             void* z_out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D, int64_t HID,
+                             int64_t C_s, int64_t H_s, int64_t D_s, int64_t HID_s, float inf, float inf_s, int flags,
+                             void* workspace, int64_t workspace_bytes, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

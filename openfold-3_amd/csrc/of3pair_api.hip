@@ -856,4 +856,115 @@ int of3_transition_rows_fwd(const void* x, const float* mask, const void* ln_w, 
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
+// ---- whole blocks in one call ---------------------------------------------------------------
+// A block is 12 to 24 kernel launches of 5 to 10 us each at the lengths of small proteins.  Issued module by
+// module from Python they cost 260 us of host time per PairFormerBlock, more than the kernels take; from one
+// call the launches themselves (2.5 us each) are what is left.
+
+int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
+                                       int64_t HID) {
+  int64_t need = of3_trimul_workspace_bytes_for(dtype, B, N, C, CH);
+  const int64_t att = of3_triattn_workspace_bytes_for(dtype, B, N, C, H, D);
+  if (need < 0 || att < 0) return OF3_EINVAL;
+  if (att > need) need = att;
+  if (HID != 0) {
+    if (dtype == OF3_DTYPE_BF16 && (HID < 128 || HID % 32 != 0 || HID > (1 << 16))) return OF3_EINVAL;
+    const int64_t tr = of3_transition_workspace_bytes_for(dtype, B, N, C, HID);
+    if (tr < 0) return OF3_EINVAL;
+    if (tr > need) need = tr;
+  }
+  return need;
+}
+
+int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t z_strides[3], const float* mask,
+                       const int64_t mask_strides[3], void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H,
+                       int64_t D, int64_t HID, float inf, int flags, void* workspace, int64_t workspace_bytes, int dtype,
+                       void* stream) {
+  // everything is checked before the first launch: a block is updated in place, half of one is of no use
+  const int64_t need = of3_pair_block_workspace_bytes(dtype, B, N, C, CH, H, D, HID);
+  if (need < 0 || !weights || !z || !out || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
+  const bool wide = dtype == OF3_DTYPE_F32;
+  if (wide ? !f32_strides_ok(z_strides) : !strides_ok(z_strides)) return OF3_EINVAL;
+  if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return OF3_EINVAL;
+  const int n_weights = OF3_PAIR_BLOCK_WEIGHTS - (HID == 0 ? 5 : 0);
+  for (int i = 0; i < n_weights; ++i)
+    if (!weights[i] || !(wide ? aligned4(weights[i]) : aligned16(weights[i]))) return OF3_EINVAL;
+  if (wide ? !(aligned4(z) && aligned4(out)) : !(aligned16(z) && aligned16(out))) return OF3_EINVAL;
+  if (workspace_bytes < need) return OF3_ENOSPC;
+
+  const void* src = z;  // the first module reads z, every later one updates out in place
+  auto trimul = [&](const void* const* w, int outgoing) {
+    const int st = of3_trimul_fwd(src, z_strides, mask, mask_strides, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8],
+                                  w[9], out, B, N, C, CH, outgoing, 1, workspace, workspace_bytes, dtype, stream);
+    src = out;
+    return st;
+  };
+  auto triattn = [&](const void* const* w, bool ending) {
+    const int64_t zt[3] = {z_strides[0], ending ? z_strides[2] : z_strides[1], ending ? z_strides[1] : z_strides[2]};
+    int64_t mt[3] = {0, 0, 0};
+    if (mask) mt[0] = mask_strides[0], mt[1] = mask_strides[ending ? 2 : 1], mt[2] = mask_strides[ending ? 1 : 2];
+    const int st = of3_triattn_fwd(src, zt, mask, mt, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], out, B, N, C, H, D,
+                                   inf, 1, workspace, workspace_bytes, dtype, stream);
+    src = out;
+    return st;
+  };
+  const void* const* w_mul = weights;
+  const void* const* w_att = weights + 20;
+  int st = OF3_OK;
+  for (int part = 0; part < 2 && st == OF3_OK; ++part) {
+    if ((part == 0) == !(flags & OF3_BLOCK_ATTENTION_FIRST)) {
+      st = trimul(w_mul, 1);
+      if (st == OF3_OK) st = trimul(w_mul + 10, 0);
+    } else {
+      st = triattn(w_att, false);
+      if (st == OF3_OK) st = triattn(w_att + 8, true);
+    }
+  }
+  if (st != OF3_OK || HID == 0) return st;
+  const void* const* t = weights + 36;
+  return of3_transition_fwd_ws(out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask, mask_strides, t[0],
+                               t[1], t[2], t[3], t[4], out, B, N, C, HID, 1, wide ? workspace : nullptr,
+                               wide ? workspace_bytes : 0, dtype, stream);
+}
+
+int64_t of3_pairformer_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
+                                             int64_t HID, int64_t C_s, int64_t H_s, int64_t D_s, int64_t HID_s) {
+  int64_t need = of3_pair_block_workspace_bytes(dtype, B, N, C, CH, H, D, HID);
+  const int64_t attn = of3_attn_pair_bias_workspace_bytes_for(dtype, B, N, C_s, H_s, D_s);
+  const int64_t rows = of3_transition_rows_fast_workspace_bytes(dtype, B * N, C_s, HID_s);
+  if (need < 0 || attn < 0 || rows < 0 || HID < 1 || H_s > (dtype == OF3_DTYPE_BF16 ? 32 : 64)) return OF3_EINVAL;
+  const int64_t single = align256(B * H_s * N * N * (dtype == OF3_DTYPE_BF16 ? 2 : 4)) + attn;  // the pair bias, then its consumer's
+  if (single > need) need = single;
+  return rows > need ? rows : need;
+}
+
+int of3_pairformer_block_fwd(const void* const* weights, const void* s, const void* z, const int64_t z_strides[3],
+                             const float* single_mask, const float* pair_mask, const int64_t mask_strides[3], void* s_out,
+                             void* z_out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D, int64_t HID,
+                             int64_t C_s, int64_t H_s, int64_t D_s, int64_t HID_s, float inf, float inf_s, int flags,
+                             void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
+  const int64_t need = of3_pairformer_block_workspace_bytes(dtype, B, N, C, CH, H, D, HID, C_s, H_s, D_s, HID_s);
+  if (need < 0 || B > 65535 || N > (1 << 16) || !weights || !s || !s_out) return OF3_EINVAL;
+  const bool wide = dtype == OF3_DTYPE_F32;
+  const void* const* ws_ = weights + OF3_PAIR_BLOCK_WEIGHTS;
+  for (int i = 0; i < OF3_PAIRFORMER_BLOCK_WEIGHTS - OF3_PAIR_BLOCK_WEIGHTS; ++i)
+    if ((!ws_[i] && i != 1) || !(wide ? aligned4(ws_[i]) : aligned16(ws_[i]))) return OF3_EINVAL;  // 1: no offset
+  if (wide ? !(aligned4(s) && aligned4(s_out)) : !(aligned16(s) && aligned16(s_out))) return OF3_EINVAL;
+  if (single_mask && !aligned4(single_mask)) return OF3_EINVAL;
+  if (workspace_bytes < need) return OF3_ENOSPC;
+  int st = of3_pair_block_fwd(weights, z, z_strides, pair_mask, mask_strides, z_out, B, N, C, CH, H, D, HID, inf, flags,
+                              workspace, workspace_bytes, dtype, stream);
+  if (st != OF3_OK) return st;
+  const int64_t bias_bytes = align256(B * H_s * N * N * (wide ? 4 : 2));
+  st = of3_pair_bias_fwd(z_out, z_strides, ws_[0], ws_[1], ws_[2], workspace, B, N, C, H_s, dtype, stream);
+  if (st != OF3_OK) return st;
+  st = of3_attn_pair_bias_fwd(s, workspace, single_mask, ws_[3], ws_[4], ws_[5], ws_[6], ws_[7], ws_[8], ws_[9], ws_[10],
+                              s_out, B, N, C_s, H_s, D_s, inf_s, 1, static_cast<char*>(workspace) + bias_bytes,
+                              workspace_bytes - bias_bytes, dtype, stream);
+  if (st != OF3_OK) return st;
+  return of3_transition_rows_fwd(s_out, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : single_mask, ws_[11], ws_[12],
+                                 ws_[13], ws_[14], ws_[15], s_out, B * N, C_s, HID_s, 1, workspace, workspace_bytes, dtype,
+                                 stream);
+}
+
 }  // extern "C"

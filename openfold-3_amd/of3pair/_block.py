@@ -1,0 +1,300 @@
+"""Whole blocks through one call of the C ABI (of3_pair_block_fwd, of3_pairformer_block_fwd).
+
+A block issued module by module costs some 200 us of Python (parameter lookups, views, stream and device
+queries for each of its seven modules) beside 50 us of launches, more than its kernels take below about 200
+tokens.  Here the parameters are gathered in one sweep and the arguments are prepared once per block.
+
+A block is served when it is built of this package's own modules as their constructors left them: anything a
+caller may have changed (a replaced or subclassed submodule, a hook on one, parameters of another dtype than
+the activations, layouts or widths that need a conversion) makes run_* return None, and the block then runs
+module by module.
+"""
+from __future__ import annotations
+
+import ctypes
+import weakref
+
+import torch
+from torch.nn.modules import module as _nn_module
+
+from . import _lib, layers
+from . import functional as F3
+
+_TRI_MUL = ("linear_a_p", "linear_a_g", "linear_b_p", "linear_b_g")
+_MULS = {
+    layers.TriangleMultiplicationOutgoing: True, layers.TriangleMultiplicationIncoming: False,
+    layers.FusedTriangleMultiplicationOutgoing: True, layers.FusedTriangleMultiplicationIncoming: False,
+}
+
+
+class _Refused(Exception):
+    """The block is not one that the single call serves."""
+
+
+class _Params:
+    """The parameters of a block in the order of the C ABI, looked up anew in every call: a parameter or a
+    submodule that was replaced since, or moved by .to(), is seen."""
+
+    def __init__(self):
+        self.links = []    # (children of a module, name, the child they held)
+        self.refs = []     # (parameters of a module, name)
+        self.shapes = []   # what refs must have; None where a parameter may be absent
+        self.entries = []  # (index into refs, first row): the pointers handed over
+        self.called = []   # submodules that the block calls as modules
+        self.attrs = []    # (attributes of a module, name, the value the dimensions were taken from)
+        self.last = (None, None, None)  # pointers of refs, dtype and pointer array of the last call
+
+    def child(self, parent, name, kinds=None):
+        sub = parent._modules.get(name)
+        if sub is None or (kinds is not None and type(sub) not in kinds):
+            raise _Refused
+        self.links.append((parent._modules, name, sub))
+        return sub
+
+    def attr(self, module, *names):
+        for name in names:
+            self.attrs.append((module.__dict__, name, getattr(module, name)))
+
+    def current(self):
+        """Whether the block still holds the submodules and attributes that it held."""
+        for owner, name, sub in self.links:
+            if owner.get(name) is not sub:
+                return False
+        for owner, name, value in self.attrs:
+            if owner.get(name) != value:
+                return False
+        return True
+
+    def param(self, module, name, shape, optional=False, rows=(0,)):
+        if name not in module._parameters:
+            raise _Refused
+        for first in rows:
+            self.entries.append((len(self.refs), first))
+        self.refs.append((module._parameters, name))
+        self.shapes.append((shape, optional))
+
+    def norm(self, module, name, c, optional_bias=False):
+        ln = self.child(module, name, (torch.nn.LayerNorm,))
+        self.param(ln, "weight", (c,))
+        self.param(ln, "bias", (c,), optional=optional_bias)
+
+    def linear(self, module, name, shape, bias=False):
+        lin = self.child(module, name, (torch.nn.Linear,))
+        self.param(lin, "weight", shape)
+        if bias:
+            self.param(lin, "bias", shape[:1])
+
+    def gather(self, dtype):
+        """The pointer array, or None when a parameter is not a plain contiguous tensor of `dtype`."""
+        ptrs = []
+        for owner, name in self.refs:
+            p = owner.get(name)
+            if p is None:
+                ptrs.append(0)
+            elif p.dtype is dtype and p.is_contiguous():
+                ptrs.append(p.data_ptr())
+            else:
+                return None
+        seen_ptrs, seen_dtype, array = self.last
+        if seen_ptrs != ptrs or seen_dtype is not dtype:
+            array = (ctypes.c_void_p * len(self.entries))()
+            for i, (owner, name) in enumerate(self.refs):
+                shape, optional = self.shapes[i]
+                p = owner.get(name)
+                if p is None:
+                    if not optional:
+                        return None
+                elif tuple(p.shape) != shape:
+                    return None
+            for i, (ref, row) in enumerate(self.entries):
+                shape = self.shapes[ref][0]
+                at = ptrs[ref] + row * (shape[1] if len(shape) > 1 else 1) * dtype.itemsize
+                array[i] = at or None
+            self.last = (ptrs, dtype, array)
+        return array
+
+
+def _pair_params(q, block):
+    """Appends what of3_pair_block_fwd takes; returns (C, CH, H, D, HID, inf)."""
+    mul_out, mul_in = q.child(block, "tri_mul_out", _MULS), q.child(block, "tri_mul_in", _MULS)
+    c, ch = mul_out.c_z, mul_out.c_hidden
+    for m, outgoing in ((mul_out, True), (mul_in, False)):
+        if _MULS[type(m)] is not outgoing or m._outgoing is not outgoing or (m.c_z, m.c_hidden) != (c, ch):
+            raise _Refused
+        q.attr(m, "c_z", "c_hidden", "_outgoing")
+        q.norm(m, "layer_norm_in", c)
+        q.norm(m, "layer_norm_out", ch)
+        if isinstance(m, layers.FusedTriangleMultiplicativeUpdate):
+            # the a and b matrices are the two halves of each stacked weight: a_p, a_g, b_p, b_g
+            n = len(q.refs)
+            for name in ("linear_ab_p", "linear_ab_g"):
+                lin = q.child(m, name, (torch.nn.Linear,))
+                q.param(lin, "weight", (2 * ch, c), rows=())
+            q.entries += [(n, 0), (n + 1, 0), (n, ch), (n + 1, ch)]
+        else:
+            for name in _TRI_MUL:
+                q.linear(m, name, (ch, c))
+        q.linear(m, "linear_g", (c, c))
+        q.linear(m, "linear_z", (c, ch))
+    start, end = (q.child(block, n, (layers.TriangleAttention,)) for n in ("tri_att_start", "tri_att_end"))
+    h, d, inf = start.no_heads, start.mha.c_hidden, start.inf
+    for m in (start, end):
+        mha = q.child(m, "mha", (layers._GatedAttentionParams,))
+        if (m.c_in, m.no_heads, mha.c_hidden, m.inf) != (c, h, d, inf):
+            raise _Refused
+        q.attr(m, "no_heads", "inf")
+        q.norm(m, "layer_norm", c)
+        q.linear(m, "linear_z", (h, c))
+        for name in ("linear_q", "linear_k", "linear_v", "linear_g"):
+            q.linear(mha, name, (h * d, c))
+        q.linear(mha, "linear_o", (c, h * d))
+    hid = 0
+    if "pair_transition" in block._modules:
+        hid = _transition_params(q, block, "pair_transition", c)
+    return c, ch, h, d, hid, inf
+
+
+def _transition_params(q, block, name, c):
+    t = q.child(block, name, (layers.SwiGLUTransition,))
+    q.called.append(t)
+    hid = t.n * c
+    q.norm(t, "layer_norm", c)
+    sw = q.child(t, "swiglu", (layers._SwiGLUParams,))
+    q.linear(sw, "linear_a", (hid, c))
+    q.linear(sw, "linear_b", (hid, c))
+    q.linear(t, "linear_out", (c, hid))
+    return hid
+
+
+def _pairformer_params(q, block, pair_block_type):
+    pair = q.child(block, "pair_stack", (pair_block_type,))
+    q.called.append(pair)
+    dims = _pair_params(q, pair)
+    a = q.child(block, "attn_pair_bias", (layers.AttentionPairBias,))
+    q.called.append(a)
+    mha = q.child(a, "mha", (layers._PairBiasAttentionParams,))
+    c_s, c_z, h = a.c_q, dims[0], a.no_heads
+    hd = mha.linear_q.weight.shape[0]
+    if a.c_z != c_z or h < 1 or hd % h:
+        raise _Refused
+    q.attr(a, "no_heads", "inf")
+    q.norm(a, "layer_norm_z", c_z, optional_bias=True)
+    q.linear(a, "linear_z", (h, c_z))
+    q.norm(a, "layer_norm_a", c_s)
+    q.linear(mha, "linear_q", (hd, c_s), bias=True)
+    for name in ("linear_k", "linear_v", "linear_g"):
+        q.linear(mha, name, (hd, c_s))
+    q.linear(mha, "linear_o", (c_s, hd))
+    hid_s = _transition_params(q, block, "single_transition", c_s)
+    return dims, (c_s, h, hd // h, hid_s, a.inf)
+
+
+_plans = weakref.WeakKeyDictionary()  # block -> (parameters, dimensions), or False where it is not served
+
+
+def _plan(block, build):
+    plan = _plans.get(block)
+    if plan is None:
+        q = _Params()
+        try:
+            plan = (q, build(q))
+        except (_Refused, AttributeError, TypeError):
+            plan = False
+        _plans[block] = plan
+    return plan
+
+
+def _gather(block, build, dtype):
+    """(pointer array, dimensions) of the block's parameters, or None."""
+    plan = _plan(block, build)
+    if plan and not plan[0].current():
+        _plans.pop(block, None)
+        plan = _plan(block, build)
+    if not plan:
+        return None
+    q, dims = plan
+    array = q.gather(dtype)
+    if array is None:
+        return None
+    for m in q.called:  # modules that the block would call: their hooks and their mode are theirs
+        if m.training or m._forward_hooks or m._forward_pre_hooks:
+            return None
+    if _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks:
+        return None
+    return array, dims
+
+
+def _pair_args(z, mask):
+    """(z as [B, N, N, C] without a copy, mask as fp32 [B, N, N] or None), or None."""
+    if not z.is_cuda or z.dtype not in (torch.bfloat16, torch.float32) or z.dim() < 3:
+        return None
+    z4, lead = F3._flatten_pair(z)
+    if z4.data_ptr() != z.data_ptr():  # a layout that is copied first
+        return None
+    return z4, F3._mask_arg(mask, lead, z4.shape[0], z4.shape[1], z.device)
+
+
+def _call(fn, what, device, *args):
+    if torch.cuda.current_device() == device.index:
+        st = fn(*args)
+    else:
+        with torch.cuda.device(device):
+            st = fn(*args)
+    _lib.check(st, what)
+
+
+def run_pair_block(block, z, mask, inplace, attention_first=False, mask_trans=True):
+    """z after the block's modules, or None when the single call does not serve it."""
+    found = _gather(block, lambda q: _pair_params(q, block), z.dtype)
+    args = found and _pair_args(z, mask)
+    if not args:
+        return None
+    array, (c, ch, h, d, hid, inf) = found
+    z4, (m, mptr, mstr) = args
+    B, N, _, C = z4.shape
+    if C != c:
+        return None
+    lib = _lib.load()
+    code = _lib.OF3_DTYPE_BF16 if z.dtype is torch.bfloat16 else _lib.OF3_DTYPE_F32
+    need = lib.of3_pair_block_workspace_bytes(code, B, N, C, ch, h, d, hid)
+    if need < 0:
+        return None
+    out4 = z4 if inplace else F3._out_like(z4)
+    stream = F3._stream(z)
+    ws = F3._workspace(z.device, need, stream)
+    flags = (_lib.OF3_BLOCK_ATTENTION_FIRST if attention_first else 0) | (0 if mask_trans else _lib.OF3_BLOCK_TRANSITION_UNMASKED)
+    _call(lib.of3_pair_block_fwd, "of3_pair_block_fwd", z.device, array, z4.data_ptr(), _lib.strides3(z4.stride()[:3]),
+          mptr, mstr, out4.data_ptr(), B, N, C, ch, h, d, hid, float(inf), flags, ws.data_ptr(), ws.numel(), code, stream)
+    return z if inplace else out4.view(z.shape)
+
+
+def run_pairformer_block(block, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
+    """(s, z) after the block, or None when the single call does not serve it."""
+    found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
+    if not found or not s.is_cuda or s.dtype is not z.dtype or not s.is_contiguous():
+        return None
+    args = _pair_args(z, pair_mask)
+    if not args or s.shape[:-1] != z.shape[:-2]:
+        return None
+    array, ((c, ch, h, d, hid, inf), (c_s, h_s, d_s, hid_s, inf_s)) = found
+    z4, (m, mptr, mstr) = args
+    B, N, _, C = z4.shape
+    if C != c or s.shape[-1] != c_s:
+        return None
+    lib = _lib.load()
+    code = _lib.OF3_DTYPE_BF16 if z.dtype is torch.bfloat16 else _lib.OF3_DTYPE_F32
+    need = lib.of3_pairformer_block_workspace_bytes(code, B, N, C, ch, h, d, hid, c_s, h_s, d_s, hid_s)
+    if need < 0:
+        return None
+    sm = None
+    if single_mask is not None:
+        sm = single_mask.to(torch.float32).expand(s.shape[:-1]).contiguous()
+    z_out = z4 if inplace else F3._out_like(z4)
+    s_out = s if inplace else torch.empty_like(s)
+    stream = F3._stream(z)
+    ws = F3._workspace(z.device, need, stream)
+    _call(lib.of3_pairformer_block_fwd, "of3_pairformer_block_fwd", z.device, array, s.data_ptr(), z4.data_ptr(),
+          _lib.strides3(z4.stride()[:3]), None if sm is None else sm.data_ptr(), mptr, mstr, s_out.data_ptr(),
+          z_out.data_ptr(), B, N, C, ch, h, d, hid, c_s, h_s, d_s, hid_s, float(inf), float(inf_s),
+          0 if mask_trans else _lib.OF3_BLOCK_TRANSITION_UNMASKED, ws.data_ptr(), ws.numel(), code, stream)
+    return s_out, z if inplace else z_out.view(z.shape)

@@ -12,28 +12,27 @@ import functools
 import torch
 
 
-def _tensors(values):
+def _wants_gradient(values):
     for v in values:
         if isinstance(v, torch.Tensor):
-            yield v
-        elif isinstance(v, (list, tuple)):
-            yield from _tensors(v)
+            if v.requires_grad:
+                return True
+        elif isinstance(v, (list, tuple)) and _wants_gradient(v):
+            return True
+    return False
 
 
 def refuse_training(module, args=(), kwargs=None):
     """Raises RuntimeError when `module` is in training mode, or when autograd is recording and an
     input tensor asks for a gradient."""
-    name = type(module).__name__
     if module.training:
         raise RuntimeError(
             "%s is forward-only (inference): call .eval() first.  In training mode the reference applies "
-            "dropout and records gradients; these kernels do neither." % name)
-    if torch.is_grad_enabled():
-        for t in _tensors(list(args) + list((kwargs or {}).values())):
-            if t.requires_grad:
-                raise RuntimeError(
-                    "%s is forward-only (inference): an input requires a gradient, and the kernels record no "
-                    "autograd graph.  Detach the input or call under torch.no_grad()." % name)
+            "dropout and records gradients; these kernels do neither." % type(module).__name__)
+    if torch.is_grad_enabled() and (_wants_gradient(args) or (kwargs and _wants_gradient(kwargs.values()))):
+        raise RuntimeError(
+            "%s is forward-only (inference): an input requires a gradient, and the kernels record no "
+            "autograd graph.  Detach the input or call under torch.no_grad()." % type(module).__name__)
 
 
 def forward_only(fn):

@@ -16,6 +16,9 @@ OF3_OK, OF3_EINVAL, OF3_ENOSPC, OF3_EHIP, OF3_ESTATIC = 0, -1, -2, -3, -4
 OF3_STATIC_SCRATCH_BYTES = 48 << 20
 OF3_DTYPE_F32, OF3_DTYPE_BF16 = 0, 1
 
+OF3_PAIR_BLOCK_WEIGHTS, OF3_PAIRFORMER_BLOCK_WEIGHTS = 41, 57
+OF3_BLOCK_ATTENTION_FIRST, OF3_BLOCK_TRANSITION_UNMASKED = 1, 2
+
 _I64x3 = ctypes.POINTER(c_int64)
 
 # name -> (restype, argtypes); mirrors include/of3pair.h one to one
@@ -57,6 +60,13 @@ SIGNATURES = {
     "of3_transition_rows_workspace_bytes": (c_int64, [c_int64] * 3),
     "of3_transition_rows_fwd": (c_int, [c_void_p] * 8 + [c_int64] * 3 + [c_int, c_void_p, c_int64, c_int, c_void_p]),
     "of3_layer_norm_fwd": (c_int, [c_void_p] * 4 + [c_int64] * 2 + [c_int, c_void_p]),
+    "of3_pair_block_workspace_bytes": (c_int64, [c_int] + [c_int64] * 7),
+    "of3_pair_block_fwd": (c_int, [ctypes.POINTER(c_void_p), c_void_p, _I64x3, c_void_p, _I64x3, c_void_p] + [c_int64] * 7
+                           + [c_float, c_int, c_void_p, c_int64, c_int, c_void_p]),
+    "of3_pairformer_block_workspace_bytes": (c_int64, [c_int] + [c_int64] * 11),
+    "of3_pairformer_block_fwd": (c_int, [ctypes.POINTER(c_void_p), c_void_p, c_void_p, _I64x3, c_void_p, c_void_p, _I64x3,
+                                         c_void_p, c_void_p] + [c_int64] * 11 + [c_float, c_float, c_int, c_void_p,
+                                                                                c_int64, c_int, c_void_p]),
     "of3_template_tail_fwd": (c_int, [c_void_p] * 5 + [c_int64] * 5 + [c_int, c_int, c_void_p]),
 }
 

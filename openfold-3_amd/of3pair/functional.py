@@ -20,14 +20,14 @@ _in_graph: set = set()  # keys of the buffers a stream capture has handed to ker
 _retired: list = []
 
 
-def _workspace(device, nbytes: int) -> torch.Tensor:
+def _workspace(device, nbytes: int, stream=None) -> torch.Tensor:
     """Grow-only scratch per (device, current stream), owned by this Python layer (the library
     allocates nothing).  Kernels on one stream are ordered, so all modules running on a stream share
     its buffer; another stream gets a buffer of its own.  A buffer that is outgrown is freed, unless a
     stream capture has used it: a HIP graph captured earlier still replays kernels that point into it
     and the caching allocator must not hand that memory to another tensor, so such a buffer is kept
-    alive until release_workspaces()."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    alive until release_workspaces().  stream: the current stream's handle, where the caller has it."""
+    key = (device, torch.cuda.current_stream(device).cuda_stream if stream is None else stream)
     capturing = torch.cuda.is_current_stream_capturing()
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:

@@ -12,6 +12,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from . import _block
 from . import functional as F3
 from ._guard import forward_only
 from .layers import (FusedTriangleMultiplicationIncoming, FusedTriangleMultiplicationOutgoing, SwiGLUTransition,
@@ -81,6 +82,17 @@ class PairStack(nn.Module):
         """z [*, N, N, C_z], pair_mask [*, N, N] -> z after the four residual updates.
         Leading dimensions (batch, templates) are independent and processed together.  With
         inplace_safe the input tensor is overwritten; otherwise it is left intact."""
+        if type(self) is PairStack:
+            done = _block.run_pair_block(self, z, pair_mask, inplace_safe)
+            if done is not None:
+                return done
+        return self._modules_forward(z, pair_mask, inplace_safe)
+
+    def _modules_forward(self, z, pair_mask, inplace_safe, attention_first=False):
+        """The four updates module by module."""
+        if attention_first:
+            z = self.tri_att_start_end(z, pair_mask, inplace_safe=inplace_safe)
+            return self.tri_mul_out_in(z, pair_mask, inplace_safe=True)
         z = self.tri_mul_out_in(z, pair_mask, inplace_safe=inplace_safe)
         # z is now a tensor this module owns (or the caller allowed overwriting)
         return self.tri_att_start_end(z, pair_mask, inplace_safe=True)
@@ -114,6 +126,10 @@ class PairBlock(PairStack):
                 _mask_trans: bool = True, _attn_chunk_size=None):
         """base_blocks.py:408-480.  _mask_trans=False runs the transition unmasked
         (base_blocks.py:445-448)."""
-        z = super().forward(z, pair_mask, inplace_safe=inplace_safe)
+        if type(self) is PairBlock:
+            done = _block.run_pair_block(self, z, pair_mask, inplace_safe, mask_trans=_mask_trans)
+            if done is not None:
+                return done
+        z = self._modules_forward(z, pair_mask, inplace_safe)
         # z is owned by this call (or may be overwritten): the transition updates it in place
         return self.pair_transition(z, mask=pair_mask if _mask_trans else None, _add_residual=True, _inplace=True)

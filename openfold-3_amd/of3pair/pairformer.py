@@ -9,6 +9,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from . import _block
 from ._guard import forward_only
 from .layers import AttentionPairBias, SwiGLUTransition
 from .pair_stack import PairBlock
@@ -48,6 +49,10 @@ class PairFormerBlock(nn.Module):
                 _attn_chunk_size=None):
         """s [*, N, C_s], z [*, N, N, C_z], single_mask [*, N], pair_mask [*, N, N] -> (s, z).
         With inplace_safe both inputs are overwritten; otherwise they are left intact."""
+        if type(self) is PairFormerBlock:
+            done = _block.run_pairformer_block(self, PairBlock, s, z, single_mask, pair_mask, inplace_safe, _mask_trans)
+            if done is not None:
+                return done
         z = self.pair_stack(z, pair_mask, inplace_safe=inplace_safe, _mask_trans=_mask_trans)
         s = self.attn_pair_bias(a=s, z=z, s=None, mask=single_mask, _add_residual=True, _inplace=inplace_safe)
         # s is now a tensor this call owns (or may be overwritten)

@@ -12,6 +12,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from . import _block
 from . import functional as F3
 from ._guard import forward_only
 from .layers import _init_linear, _init_name
@@ -37,12 +38,12 @@ class TemplatePairBlock(PairBlock):
                 use_lma=False, inplace_safe: bool = False, _mask_trans: bool = True, _attn_chunk_size=None):
         """z [*, N_templ, N, N, C_t], mask [*, N_templ, N, N] -> updated z.  Without inplace_safe
         the input is left intact."""
-        if self.tri_mul_first:
-            z = self.tri_mul_out_in(z, mask, inplace_safe=inplace_safe)
-            z = self.tri_att_start_end(z, mask, inplace_safe=True)
-        else:
-            z = self.tri_att_start_end(z, mask, inplace_safe=inplace_safe)
-            z = self.tri_mul_out_in(z, mask, inplace_safe=True)
+        attention_first = not self.tri_mul_first
+        if type(self) is TemplatePairBlock:
+            done = _block.run_pair_block(self, z, mask, inplace_safe, attention_first, _mask_trans)
+            if done is not None:
+                return done
+        z = self._modules_forward(z, mask, inplace_safe, attention_first)
         return self.pair_transition(z, mask=mask if _mask_trans else None, _add_residual=True, _inplace=True)
 
 
