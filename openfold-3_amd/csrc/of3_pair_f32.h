@@ -1,0 +1,72 @@
+// Arguments of the fp32 pair kernels, shared by pair_f32.hip (every shape) and pair_pass_f32.hip (the
+// position-wise passes at 64 and 128 channels).
+#pragma once
+
+#include "of3_kernels.h"
+
+namespace of3 {
+
+// split, operand-ordered copy of a weight matrix [rows][K]: three planes of ceil(rows / 32) * 32 * K bf16
+struct WeightX3 {
+  const bf16_t* h;
+  long plane;
+};
+__host__ __device__ constexpr long packed_elems(long rows, long K) { return (rows + 31) / 32 * 32 * K; }
+
+// Row of a k-panel that holds row r of channel c: the rows of a channel's panels are rotated by 4 c.  A store of the
+// projection pass writes 32 channels of one row at once; without the rotation these are Np * Np * 2 bytes apart, at
+// the usual lengths a multiple of the memory system's interleave, and all 32 pieces go to one L2 channel
+// (N = 768: see trimul_proj_pass).  rot = panel_rotation(c, Np), Np >= 32.
+__host__ __device__ inline int panel_rotation(int c, int Np) { return (4 * c) % Np; }
+__host__ __device__ inline int panel_row(int r, int rot, int Np) {
+  const int s = r + rot;
+  return s < Np ? s : s - Np;
+}
+
+// ---- triangle multiplication
+struct TrimulF32 {
+  const float *z, *mask;
+  PairView zv, mv;          // view used by the projection pass (swapped for the incoming update)
+  PairView zc;              // canonical view (output pass)
+  const float *ln_in_w, *ln_in_b, *ln_out_w, *ln_out_b;
+  const float *w_ap, *w_ag, *w_bp, *w_bg, *w_g, *w_z;
+  WeightX3 s_ap, s_ag, s_bp, s_bg, s_g, s_z;  // split copies (the *_x3 kernels only)
+  float *a, *b, *x, *out;
+  // a and b split into three bf16 terms in the k-panel layout (the split-operand contraction only):
+  // element (b, c, r, k) of a term sits at ((((b CH + c) Np / 32 + k / 32) Np + panel_row(r, c)) 32 + k % 32,
+  // the three terms ab_plane elements apart; Np = N rounded up to whole 32-wide panels
+  bf16_t *as, *bs;
+  long ab_plane;
+  int Np;
+  int B, N, C, CH, add_residual;
+};
+
+// ---- triangle attention
+struct TriattnF32 {
+  const float *x, *mask;
+  PairView xv, mv;
+  const float *ln_w, *ln_b, *w_q, *w_k, *w_v, *w_b, *w_g, *w_o;
+  WeightX3 s_q, s_k, s_v, s_g, s_o;  // split copies (the *_x3 kernels only)
+  float *q, *k, *v, *tb, *o, *out;
+  // q, k and v^T split into three bf16 terms and stored as MFMA operands (the split-operand core only):
+  // the 16 bytes of lane l for step s of 32-position tile t of (b, i, h) are slot
+  // (((b N + i) H + h) * Jp / 32 + t) * steps + s) * 64 + l of a plane.  q and k have D / 16 steps (16
+  // head channels each) and planes of qk_plane elements; v^T always has two steps (16 keys each) of 32
+  // rows, the rows from D on being zero, and planes of v_plane elements
+  bf16_t *qs, *ks, *vs;
+  long qk_plane, v_plane;
+  int Jp;  // N rounded up to whole 32-position tiles
+  int B, N, C, H, D, add_residual;
+  float inf;
+};
+
+// position-wise passes with the weights held in registers (pair_pass_f32.hip): which shapes they serve (the
+// caller has split the weights and asked for split intermediates), and their launches
+bool trimul_pass_serves(const TrimulF32& p);
+hipError_t trimul_proj_pass_f32(const TrimulF32& p, hipStream_t stream);
+hipError_t trimul_out_pass_f32(const TrimulF32& p, hipStream_t stream);
+bool triattn_pass_serves(const TriattnF32& p);
+hipError_t triattn_proj_pass_f32(const TriattnF32& p, hipStream_t stream);
+hipError_t triattn_out_pass_f32(const TriattnF32& p, hipStream_t stream);
+
+}  // namespace of3

@@ -20,6 +20,7 @@
 #include "of3_device.h"
 #include "of3_kernels.h"
 #include "of3_launch.h"
+#include "of3_pair_f32.h"
 #include "of3_split.h"
 
 namespace of3 {
@@ -189,13 +190,6 @@ __device__ __forceinline__ TileX3 make_tile_x3(void* base, int K, int tp) {
   return t;
 }
 __host__ __device__ constexpr size_t tile_bytes_x3(int K, int tp) { return (size_t)3 * tp * (K + 8) * sizeof(bf16_t); }
-
-// split, operand-ordered copy of a weight matrix [rows][K]: three planes of ceil(rows / 32) * 32 * K bf16
-struct WeightX3 {
-  const bf16_t* h;
-  long plane;
-};
-__host__ __device__ constexpr long packed_elems(long rows, long K) { return (rows + 31) / 32 * 32 * K; }
 
 // up to six matrices in one launch
 struct SplitJobs {
@@ -424,23 +418,6 @@ __device__ __forceinline__ void linear_tiles_x3(const TileX3& xs, const WeightX3
 }
 
 // ---- triangle multiplication -----------------------------------------------------------------
-struct TrimulF32 {
-  const float *z, *mask;
-  PairView zv, mv;          // view used by the projection pass (swapped for the incoming update)
-  PairView zc;              // canonical view (output pass)
-  const float *ln_in_w, *ln_in_b, *ln_out_w, *ln_out_b;
-  const float *w_ap, *w_ag, *w_bp, *w_bg, *w_g, *w_z;
-  WeightX3 s_ap, s_ag, s_bp, s_bg, s_g, s_z;  // split copies (the *_x3 kernels only)
-  float *a, *b, *x, *out;
-  // a and b split into three bf16 terms in the k-panel layout (the split-operand contraction only):
-  // element (b, c, r, k) of a term sits at ((((b CH + c) Np / 32 + k / 32) Np + r) 32 + k % 32, the
-  // three terms ab_plane elements apart; Np = N rounded up to whole 32-wide panels
-  bf16_t *as, *bs;
-  long ab_plane;
-  int Np;
-  int B, N, C, CH, add_residual;
-};
-
 __global__ __launch_bounds__(kThreads) void trimul_proj_f32(TrimulF32 p, int groups) {
   __shared__ float xn[kP][kMaxC];
   __shared__ float msk[kP];
@@ -758,7 +735,7 @@ __global__ __launch_bounds__(kThreads * PT) void trimul_proj_x3_f32(TrimulF32 p,
       for (int xt = 0; xt < XT; ++xt) {
         if (k0 + 32 * xt >= p.Np || !(FAST || c < CH)) continue;
         bf16_t* lp = (pair ? p.bs : p.as) + ((size_t)b * CH + c) * chan +
-                     ((size_t)((k0 + 32 * xt) >> 5) * p.Np + r) * 32 + 8 * lh;
+                     ((size_t)((k0 + 32 * xt) >> 5) * p.Np + panel_row(r, panel_rotation(c, p.Np), p.Np)) * 32 + 8 * lh;
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
           float x[8];
@@ -839,14 +816,16 @@ __global__ __launch_bounds__(512) void trimul_contract_x3_f32(TrimulF32 p, int t
   // slot t of a stage's a (b) part holds chunk (t & 3) ^ ((row >> 2) & 3) of tile row t >> 2; wave w
   // fills a slots 128 w .. + 127 (two instructions) and b slots 64 w .. + 63 of each term
   uint32_t a_off[2], b_off;
+  const int rot = panel_rotation(bc % p.CH, Np);
+  auto rotated = [&](int r) { return panel_row(r < Np ? r : Np - 1, rot, Np); };  // rows past the end: computed, not stored
 #pragma unroll
   for (int n = 0; n < 2; ++n) {
     const int t = 128 * wave + 64 * n + lane, row = t >> 2, c = (t & 3) ^ ((row >> 2) & 3);
-    a_off[n] = (uint32_t)(((i0 + row) * 32 + 8 * c) * sizeof(bf16_t));
+    a_off[n] = (uint32_t)((rotated(i0 + row) * 32 + 8 * c) * sizeof(bf16_t));
   }
   {
     const int t = 64 * wave + lane, row = t >> 2, c = (t & 3) ^ ((row >> 2) & 3);
-    b_off = (uint32_t)(((j0 + row) * 32 + 8 * c) * sizeof(bf16_t));
+    b_off = (uint32_t)((rotated(j0 + row) * 32 + 8 * c) * sizeof(bf16_t));
   }
   auto issue_loads = [&](int panel, int buf) {  // buf is a constant at every call site
     u32x4_t* st = lds4 + buf * kCtStage;
@@ -1056,24 +1035,6 @@ __global__ __launch_bounds__(kThreads * PT) void trimul_out_x3_f32(TrimulF32 p, 
 }
 
 // ---- triangle attention ----------------------------------------------------------------------
-struct TriattnF32 {
-  const float *x, *mask;
-  PairView xv, mv;
-  const float *ln_w, *ln_b, *w_q, *w_k, *w_v, *w_b, *w_g, *w_o;
-  WeightX3 s_q, s_k, s_v, s_g, s_o;  // split copies (the *_x3 kernels only)
-  float *q, *k, *v, *tb, *o, *out;
-  // q, k and v^T split into three bf16 terms and stored as MFMA operands (the split-operand core only):
-  // the 16 bytes of lane l for step s of 32-position tile t of (b, i, h) are slot
-  // (((b N + i) H + h) * Jp / 32 + t) * steps + s) * 64 + l of a plane.  q and k have D / 16 steps (16
-  // head channels each) and planes of qk_plane elements; v^T always has two steps (16 keys each) of 32
-  // rows, the rows from D on being zero, and planes of v_plane elements
-  bf16_t *qs, *ks, *vs;
-  long qk_plane, v_plane;
-  int Jp;  // N rounded up to whole 32-position tiles
-  int B, N, C, H, D, add_residual;
-  float inf;
-};
-
 __global__ __launch_bounds__(kThreads) void triattn_proj_f32(TriattnF32 p, int groups) {
   __shared__ float xn[kP][kMaxC];
   const int N = p.N, C = p.C, H = p.H, D = p.D, HD = H * D;
@@ -2338,6 +2299,12 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
     splitter.add(a.w_g, a.C, a.C, p.s_g);
     splitter.add(a.w_z, a.C, a.CH, p.s_z);
     if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
+  }
+  const bool pass = split_ab && trimul_pass_serves(p);
+  if (pass) {
+    if (hipError_t ep = trimul_proj_pass_f32(p, stream); ep != hipSuccess) return ep;
+    if (hipError_t ep = allow_lds<trimul_contract_x3_f32>(kLdsLimit); ep != hipSuccess) return ep;
+  } else if (x3) {
     auto proj = split_ab ? (fast ? trimul_proj_x3_f32<kXT, kPT, true, true> : trimul_proj_x3_f32<kXT, kPT, false, true>)
                          : (fast ? trimul_proj_x3_f32<kXT, kPT, true, false> : trimul_proj_x3_f32<kXT, kPT, false, false>);
     hipError_t e = allow_lds<trimul_proj_x3_f32<kXT, kPT, false, false>>(kLdsLimit);
@@ -2380,6 +2347,7 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
     hipLaunchKernelGGL(trimul_contract_f32, dim3(t, t, (unsigned)(a.B * a.CH)), dim3(kThreads), 0, stream, p.a, p.b,
                        p.x, a.N);
   }
+  if (pass) return trimul_out_pass_f32(p, stream);
   if (x3) {
     const size_t lds = tile_bytes_x3(a.C > a.CH ? a.C : a.CH, 32 * kXT * kPT) + 2 * kThreads * kPT * sizeof(float);
     const bool wide = a.C > 128 || a.CH > 128;
@@ -2455,6 +2423,13 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
     splitter.add(a.w_g, HD, a.C, p.s_g);
     splitter.add(a.w_o, a.C, HD, p.s_o);
     if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
+  }
+  const bool pass = core_x3 && triattn_pass_serves(p);
+  if (pass) {
+    if (hipError_t ep = triattn_proj_pass_f32(p, stream); ep != hipSuccess) return ep;
+    if (hipError_t ep = allow_lds<triattn_core_x3_f32<1>>(kCoreX3Lds); ep != hipSuccess) return ep;
+    if (hipError_t ep = allow_lds<triattn_core_x3_f32<2>>(kCoreX3Lds); ep != hipSuccess) return ep;
+  } else if (x3) {
     auto proj = core_x3 ? (fast ? triattn_proj_x3_f32<kXT, kPT, true, true> : triattn_proj_x3_f32<kXT, kPT, true, false>)
                         : (fast ? triattn_proj_x3_f32<kXT, kPT, false, true> : triattn_proj_x3_f32<kXT, kPT, false, false>);
     hipError_t e = allow_lds<triattn_proj_x3_f32<kXT, kPT, false, false>>(kLdsLimit);
@@ -2502,6 +2477,7 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
     }
     hipLaunchKernelGGL(core, dim3((unsigned)cblocks), dim3(kThreads), 0, stream, p, qgroups);
   }
+  if (pass) return triattn_out_pass_f32(p, stream);
   if (x3) {
     const int HD = a.H * a.D;
     const size_t lds = tile_bytes_x3(a.C > HD ? a.C : HD, 32 * kXT * kPT);

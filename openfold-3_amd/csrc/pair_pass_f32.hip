@@ -1,0 +1,816 @@
+// Position-wise passes of the two fp32 triangle modules at 64 and 128 channels (c_z = c_hidden = heads x width:
+// the template stack's and the trunk's), products on the bf16 matrix instructions with operands split into three
+// bf16 terms (of3_split.h).  pair_f32.hip has the passes for every other shape.
+//
+// What bounded the passes of pair_f32.hip at these widths: every group of 32 positions read all split weights
+// again from L2 (6 KB per k-step of a wave against 12 MFMAs, 64 bytes per clock and compute unit: the rate of the
+// L1), and LayerNorm, products and epilogue ran one after the other.  Here the weights stay on the chip:
+// persistent work-groups whose waves each own one 32-output tile of one or two matrices and keep its split
+// operands in registers (96 registers per matrix at 128 channels, 48 at 64) for all the tiles they process; a tile
+// of 32 positions goes through LDS once (three bf16 planes, 16-byte chunks XOR-swizzled by the position), read by
+// all waves.  The next tile's rows are in flight meanwhile, in registers.  At small N the weights are a
+// one-time 3 us instead of a latency in every k-step.
+#include <type_traits>
+
+#include "of3_device.h"
+#include "of3_kernels.h"
+#include "of3_launch.h"
+#include "of3_pair_f32.h"
+#include "of3_split.h"
+
+namespace of3 {
+
+namespace {
+
+constexpr float kEps = 1e-5f;
+constexpr float kLog2eF32 = 1.4426950408889634f;
+__device__ __forceinline__ float sigmoid_hw_f32(float x) {
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * kLog2eF32));
+}
+
+// four values as the halves of three MFMA operand chunks
+__device__ __forceinline__ void split4(const float4& x, u32x2_t& h, u32x2_t& m, u32x2_t& l) {
+  const float v[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    const float a = v[2 * w], b = v[2 * w + 1];
+    const uint32_t ph = pack_bf16(a, b);
+    const float ra = a - __uint_as_float(ph << 16), rb = b - __uint_as_float(ph & 0xffff0000u);
+    const uint32_t pm = pack_bf16(ra, rb);
+    h[w] = ph;
+    m[w] = pm;
+    l[w] = pack_bf16(ra - __uint_as_float(pm << 16), rb - __uint_as_float(pm & 0xffff0000u));
+  }
+}
+
+// LDS tile of 32 positions x C channels: three planes [position][C / 8 chunks of 8 bf16].  The 16 lanes of a read
+// phase hold 16 consecutive positions at one chunk index: the key spreads them over the banks.
+template <int C>
+struct PassTile {
+  static constexpr int NCH = C / 8, PLANE = 32 * NCH, SLOTS = 3 * PLANE;  // in 16-byte slots
+  u32x4_t* s;
+  __device__ __forceinline__ static int slot(int pos, int chunk) {
+    return pos * NCH + (chunk ^ (NCH == 16 ? (pos & 15) : ((pos >> 1) & 7)));
+  }
+  // channels 4 c4 .. + 3 of a position
+  __device__ __forceinline__ void store4(int pos, int c4, const float4& y) const {
+    u32x2_t h, m, l;
+    split4(y, h, m, l);
+    u32x2_t* d = reinterpret_cast<u32x2_t*>(s) + 2 * slot(pos, c4 >> 1) + (c4 & 1);
+    d[0] = h;
+    d[2 * PLANE] = m;
+    d[4 * PLANE] = l;
+  }
+  // channels 8 chunk .. + 7
+  __device__ __forceinline__ void store8(int pos, int chunk, const float (&y)[8]) const {
+    u32x4_t h, m, l;
+    split8(y, h, m, l);
+    u32x4_t* d = s + slot(pos, chunk);
+    d[0] = h;
+    d[PLANE] = m;
+    d[2 * PLANE] = l;
+  }
+};
+
+// The lane number, opaque to the compiler: what is derived from it inside a tile loop is recomputed there (a few
+// instructions) instead of being hoisted into registers that the weights occupy.
+struct Lane {
+  int l32, lh, li, lg;
+};
+__device__ __forceinline__ Lane lane_here() {
+  int lane = threadIdx.x & 63;
+  __asm__ volatile("" : "+v"(lane));
+  return {lane & 31, lane >> 5, lane & 15, lane >> 4};
+}
+
+// A row of C channels over 16 lanes: lane li holds channels 64 e + 4 li .. + 3 (a wave reads four rows at a time,
+// 256 contiguous bytes of each per instruction)
+template <int C>
+struct RowRegs {
+  float4 v[C / 64];
+};
+template <int C>
+__device__ __forceinline__ void load_row(const float* row, int li, RowRegs<C>& r) {
+#pragma unroll
+  for (int e = 0; e < C / 64; ++e) r.v[e] = *reinterpret_cast<const float4*>(row + 64 * e + 4 * li);
+}
+// LayerNorm of the row (two-pass statistics); ln: LDS, weights [C] then biases [C]
+template <int C>
+__device__ __forceinline__ void norm_row(const RowRegs<C>& r, bool has, const float* ln, int li, float4 (&y)[C / 64]) {
+  float s = 0.f;
+#pragma unroll
+  for (int e = 0; e < C / 64; ++e) s += (r.v[e].x + r.v[e].y) + (r.v[e].z + r.v[e].w);
+  const float mean = group_sum<16>(s) * (1.f / C);
+  float q = 0.f;
+#pragma unroll
+  for (int e = 0; e < C / 64; ++e) {
+    y[e].x = r.v[e].x - mean, y[e].y = r.v[e].y - mean, y[e].z = r.v[e].z - mean, y[e].w = r.v[e].w - mean;
+    q += y[e].x * y[e].x + y[e].y * y[e].y + y[e].z * y[e].z + y[e].w * y[e].w;
+  }
+  const float rstd = 1.0f / sqrtf(group_sum<16>(q) * (1.f / C) + kEps);
+#pragma unroll
+  for (int e = 0; e < C / 64; ++e) {
+    const float4 w = *reinterpret_cast<const float4*>(ln + 64 * e + 4 * li);
+    const float4 b = *reinterpret_cast<const float4*>(ln + C + 64 * e + 4 * li);
+    y[e].x = has ? y[e].x * rstd * w.x + b.x : 0.f;
+    y[e].y = has ? y[e].y * rstd * w.y + b.y : 0.f;
+    y[e].z = has ? y[e].z * rstd * w.z + b.z : 0.f;
+    y[e].w = has ? y[e].w * rstd * w.w + b.w : 0.f;
+  }
+}
+
+// the split operands of output rows 32 t .. + 31 of a weight matrix with K = C inputs; lane_src: whose packed
+// operand this lane takes (its own, or rowperm16's to deal the rows so that a lane ends with 16 consecutive ones)
+template <int C, int TERMS>
+__device__ __forceinline__ void load_unit(const WeightX3& W, int t, int lane_src, u32x4_t (&w)[C / 16][TERMS]) {
+  const u32x4_t* src = reinterpret_cast<const u32x4_t*>(W.h) + (size_t)t * (C / 16) * 64 + lane_src;
+#pragma unroll
+  for (int s = 0; s < C / 16; ++s)
+#pragma unroll
+    for (int pl = 0; pl < TERMS; ++pl) w[s][pl] = src[pl * (W.plane / 8) + 64 * s];
+}
+
+// one k-step: six products, smallest terms first.  W_ROWS: the outputs are the MFMA rows, otherwise the positions
+template <bool W_ROWS>
+__device__ __forceinline__ f32x16_t step6(u32x4_t w_h, u32x4_t w_m, u32x4_t w_l, const u32x4_t (&x)[3], f32x16_t acc) {
+  if (W_ROWS) {
+    acc = mfma_32x32x16(w_l, x[0], acc);
+    acc = mfma_32x32x16(w_h, x[2], acc);
+    acc = mfma_32x32x16(w_m, x[1], acc);
+    acc = mfma_32x32x16(w_m, x[0], acc);
+    acc = mfma_32x32x16(w_h, x[1], acc);
+    return mfma_32x32x16(w_h, x[0], acc);
+  }
+  acc = mfma_32x32x16(x[0], w_l, acc);
+  acc = mfma_32x32x16(x[2], w_h, acc);
+  acc = mfma_32x32x16(x[1], w_m, acc);
+  acc = mfma_32x32x16(x[0], w_m, acc);
+  acc = mfma_32x32x16(x[1], w_h, acc);
+  return mfma_32x32x16(x[0], w_h, acc);
+}
+template <int C, bool W_ROWS>
+__device__ __forceinline__ f32x16_t unit_product(const PassTile<C>& t, const u32x4_t (&w)[C / 16][3]) {
+  f32x16_t acc = zero16();
+  const Lane at = lane_here();
+#pragma unroll
+  for (int s = 0; s < C / 16; ++s) {
+    const u32x4_t* x = t.s + PassTile<C>::slot(at.l32, 2 * s + at.lh);
+    const u32x4_t op[3] = {x[0], x[PassTile<C>::PLANE], x[2 * PassTile<C>::PLANE]};
+    acc = step6<W_ROWS>(w[s][0], w[s][1], w[s][2], op, acc);
+  }
+  return acc;
+}
+
+// the value of the lane with the lowest bit flipped (quad_perm [1,0,3,2])
+__device__ __forceinline__ uint32_t swap_adjacent(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);
+}
+
+// logical number of a work-group: consecutive numbers run on one XCD where the grid deals evenly
+__device__ __forceinline__ int grid_slot() {
+  return gridDim.x % 8 == 0 ? xcd_logical_block(blockIdx.x, gridDim.x / 8) : blockIdx.x;
+}
+
+// ---- triangle multiplication, input pass: a, b = mask * sigmoid(LN(z) Wg^T) * (LN(z) Wp^T) ------------------
+// Wave = gate and projection of one 32-channel tile of a or b: two matrices, 192 registers of split operands at 128
+// channels, of which the gate's third terms (used by one product of six) sit in LDS.  A work-group has four waves: at
+// 64 channels a and b, at 128 one of the two, so that two work-groups share a CU and the products of one run beside
+// the LayerNorm and the stores of the other (one work-group of eight waves in step: 468 against 462 us at N = 768).  Tile = 32 columns k of one row; four
+// consecutive rows of a panel are consecutive tiles of one XCD, so that the 64-byte pieces a tile writes per channel
+// and term meet in L2 as whole lines.
+template <int C>
+struct ProjLds {
+  static constexpr bool kThirdInLds = C == 128;
+  static constexpr int kWl = kThirdInLds ? 4 * (C / 16) * 64 : 0;  // slots
+  static constexpr size_t kBytes = (size_t)(PassTile<C>::SLOTS + kWl) * 16 + (2 * C + 64) * sizeof(float);
+};
+
+template <int C>
+__global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int panels, int row_groups, int total) {
+  typedef PassTile<C> Tile;
+  constexpr int NW = 4, KS = C / 16, OT = C / 32, TASKS = 8 / NW;
+  constexpr bool kOneSide = OT == NW;  // a and b in work-groups of their own
+  constexpr bool TL = ProjLds<C>::kThirdInLds;
+  constexpr int GTERMS = TL ? 2 : 3;
+  extern __shared__ u32x4_t lds[];
+  const Tile xn = {lds};
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
+  u32x4_t* wl = lds + Tile::SLOTS + wave * (KS * 64) + lane;
+  float* ln = reinterpret_cast<float*>(lds + Tile::SLOTS + ProjLds<C>::kWl);  // [2][C]
+  float* msk = ln + 2 * C;                                                   // [2][32]
+  const int slot = grid_slot(), N = p.N, pair = kOneSide ? slot & 1 : wave / OT, ot = wave % OT;
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_in_w[c], ln[C + c] = p.ln_in_b[c];
+  const WeightX3 Wg = pair ? p.s_bg : p.s_ag, Wp = pair ? p.s_bp : p.s_ap;
+  u32x4_t wg[KS][GTERMS], wp[KS][3];
+  load_unit<C, GTERMS>(Wg, ot, lane, wg);
+  load_unit<C, 3>(Wp, ot, lane, wp);
+  if (TL) {
+    const u32x4_t* g = reinterpret_cast<const u32x4_t*>(Wg.h) + 2 * (Wg.plane / 8) + (size_t)ot * KS * 64 + lane;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) wl[64 * s] = g[64 * s];
+  }
+  __syncthreads();
+
+  struct Place {
+    int b, r, k0;
+  };
+  auto place = [&](int id) {
+    Place t;
+    const int q = id & 3, rest = id >> 2, per_b = row_groups * panels;
+    t.b = rest / per_b;
+    const int rem = rest - t.b * per_b, rg = rem / panels;
+    t.r = 4 * rg + q;
+    t.k0 = 32 * (rem - rg * panels);
+    return t;
+  };
+  RowRegs<C> raw[TASKS];
+  float mraw = 1.f;
+  auto load_tile = [&](int id) {  // addresses clamped to real positions: no load is under a condition
+    const Lane here = lane_here();
+    const int li = here.li, lg = here.lg, l32 = here.l32;
+    const Place t = place(id);
+    const int r = t.r < N ? t.r : N - 1;
+    const float* base = p.z + t.b * p.zv.stride_b + r * p.zv.stride_r;
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      int k = t.k0 + 4 * (wave + NW * u) + lg;
+      k = k < N ? k : N - 1;
+      load_row<C>(base + k * p.zv.stride_k, li, raw[u]);
+    }
+    int k = t.k0 + l32;
+    k = k < N ? k : N - 1;
+    if (p.mask) mraw = p.mask[t.b * p.mv.stride_b + r * p.mv.stride_r + k * p.mv.stride_k];
+  };
+
+  const int step = kOneSide ? gridDim.x / 2 : gridDim.x;
+  int id = kOneSide ? slot >> 1 : slot, buf = 0;
+  if (id < total) load_tile(id);
+  for (; id < total; id += step, buf ^= 1) {
+    const Place t = place(id);
+    const Lane here = lane_here();
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      const int li = here.li, pos = 4 * (wave + NW * u) + here.lg;
+      float4 y[C / 64];
+      norm_row<C>(raw[u], t.k0 + pos < N && t.r < N, ln, li, y);
+#pragma unroll
+      for (int e = 0; e < C / 64; ++e) xn.store4(pos, li + 16 * e, y[e]);
+    }
+    if (tid < 32) msk[32 * buf + tid] = mraw;
+    load_tile(id + step < total ? id + step : id);
+    __syncthreads();  // the tile is complete
+    f32x16_t ag = zero16(), ap = zero16();
+    const Lane at = lane_here();
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const u32x4_t* x = xn.s + Tile::slot(at.l32, 2 * s + at.lh);
+      const u32x4_t op[3] = {x[0], x[Tile::PLANE], x[2 * Tile::PLANE]};
+      ag = step6<false>(wg[s][0], wg[s][1], TL ? wl[64 * s] : wg[s][GTERMS - 1], op, ag);
+      ap = step6<false>(wp[s][0], wp[s][1], wp[s][2], op, ap);
+    }
+    __syncthreads();  // everybody has read it
+    // channels in the lanes, positions in the registers: registers 8 st .. + 7 are the k-values 16 st + 8 (e >> 2)
+    // + 4 lh + (e & 3), stored as the 8 consecutive columns 16 st + 8 lh .. of the panel row (a and b in the same
+    // order, which is all a sum over k needs); positions past N are zero rows and store the panel's padding
+    if (t.r < N) {
+      const Lane out = lane_here();
+      const int l32 = out.l32, lh = out.lh;
+      const bool odd = l32 & 1;
+      const int rot0 = panel_rotation(32 * ot + (l32 & ~1), p.Np), rot1 = panel_rotation(32 * ot + (l32 | 1), p.Np);
+      u32x4_t op[2][3];
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        float x[8];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          const float4 m4 = *reinterpret_cast<const float4*>(msk + 32 * buf + 16 * st + 8 * a + 4 * lh);
+          const float m[4] = {m4.x, m4.y, m4.z, m4.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int v = 8 * st + 4 * a + e;
+            x[4 * a + e] = m[e] * sigmoid_hw_f32(ag[v]) * ap[v];
+          }
+        }
+        split8(x, op[st][0], op[st][1], op[st][2]);
+      }
+      // The lanes of an even and an odd channel exchange a chunk, so that one store writes the 64 bytes of the even
+      // channels and the next those of the odd ones (32-byte pieces of every channel otherwise: twice the requests).
+      const size_t chan = (size_t)p.Np * p.Np, pn = (size_t)(t.k0 >> 5) * p.Np;
+      bf16_t* lp = (pair ? p.bs : p.as) + ((size_t)t.b * C + 32 * ot + (l32 & ~1)) * chan + 8 * lh + (odd ? 16 : 0);
+      bf16_t* lp0 = lp + (pn + panel_row(t.r, rot0, p.Np)) * 32;
+      bf16_t* lp1 = lp + chan + (pn + panel_row(t.r, rot1, p.Np)) * 32;
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) {
+        u32x4_t first, second;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const uint32_t mine = odd ? op[1][pl][w] : op[0][pl][w];
+          const uint32_t got = swap_adjacent(odd ? op[0][pl][w] : op[1][pl][w]);
+          first[w] = odd ? got : mine;
+          second[w] = odd ? mine : got;
+        }
+        *reinterpret_cast<u32x4_t*>(lp0 + pl * p.ab_plane) = first;
+        *reinterpret_cast<u32x4_t*>(lp1 + pl * p.ab_plane) = second;
+      }
+    }
+  }
+}
+
+// ---- output passes ------------------------------------------------------------------------------------------
+// Wave = one 32-channel tile of the gate and the same tile of the output projection (weights as in the input pass of
+// the multiplication: the gate's third terms in LDS at 128 channels).  The LDS tile holds LayerNorm(z) for the gates,
+// then LayerNorm(x) or the gated attention output in its place.  Four waves per work-group at 128 channels, two
+// work-groups per CU; two waves at 64.
+template <int C>
+struct OutLds {
+  static constexpr int NW = C / 32, KS = C / 16;
+  static constexpr bool kThirdInLds = C == 128;
+  static constexpr int kWl = kThirdInLds ? NW * KS * 64 : 0;  // slots
+  static constexpr size_t kTrimul = (size_t)(PassTile<C>::SLOTS + kWl) * 16 + (2 * 32 * 2 * NW + 4 * C) * sizeof(float);
+  static constexpr size_t kTriattn = (size_t)(PassTile<C>::SLOTS + kWl) * 16 + 2 * C * sizeof(float);
+};
+// the two matrices of an output wave, outputs dealt by rowperm16: lane (position l32, half lh) ends with the outputs
+// 32 ot + 16 lh + v
+template <int C>
+struct OutWeights {
+  static constexpr int KS = C / 16;
+  static constexpr bool TL = OutLds<C>::kThirdInLds;
+  static constexpr int GTERMS = TL ? 2 : 3;
+  u32x4_t g[KS][GTERMS], o[KS][3];
+  u32x4_t* wl;
+  __device__ __forceinline__ void load(const WeightX3& Wg, const WeightX3& Wo, int ot, int l32, int lh, u32x4_t* lds_wave) {
+    const int src = rowperm16(l32) + 32 * lh;
+    load_unit<C, GTERMS>(Wg, ot, src, g);
+    load_unit<C, 3>(Wo, ot, src, o);
+    wl = lds_wave + l32 + 32 * lh;
+    if (TL) {
+      const u32x4_t* t = reinterpret_cast<const u32x4_t*>(Wg.h) + 2 * (Wg.plane / 8) + (size_t)ot * KS * 64 + src;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) wl[64 * s] = t[64 * s];
+    }
+  }
+  __device__ __forceinline__ f32x16_t gate(const PassTile<C>& t) const {
+    f32x16_t acc = zero16();
+    const Lane at = lane_here();
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const u32x4_t* x = t.s + PassTile<C>::slot(at.l32, 2 * s + at.lh);
+      const u32x4_t op[3] = {x[0], x[PassTile<C>::PLANE], x[2 * PassTile<C>::PLANE]};
+      acc = step6<true>(g[s][0], g[s][1], TL ? wl[64 * s] : g[s][GTERMS - 1], op, acc);
+    }
+    return acc;
+  }
+};
+// out row (16 channels from op on) = [residual +] v * g
+__device__ __forceinline__ void store_row16(const float* zp, float* op, const f32x16_t& v, bool add_residual) {
+  float4 z[4];
+  if (add_residual) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) z[a] = *reinterpret_cast<const float4*>(zp + 4 * a);
+  }
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    float4 r = make_float4(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);
+    if (add_residual) r.x = z[a].x + r.x, r.y = z[a].y + r.y, r.z = z[a].z + r.z, r.w = z[a].w + r.w;
+    *reinterpret_cast<float4*>(op + 4 * a) = r;
+  }
+}
+
+// ---- triangle multiplication, output pass: out = [z +] (LN(x) Wz^T) * sigmoid(LN(z) Wg^T)
+// x is channel-major: thread (position tid % 32, group tid / 32) holds 16 channels of a position; the statistics are
+// combined from the groups' means and squared deviations (one exchange).
+template <int C>
+__global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int panels, int total) {
+  typedef PassTile<C> Tile;
+  constexpr int NW = C / 32, KS = C / 16, TASKS = 8 / NW, NG = 2 * NW;
+  extern __shared__ u32x4_t lds[];
+  const Tile tile = {lds};
+  float* red = reinterpret_cast<float*>(lds + Tile::SLOTS + OutLds<C>::kWl);  // [NG][32] means, [NG][32] squared deviations
+  float* ln = red + 2 * 32 * NG;                                             // LayerNorm of z [2][C], of x [2][C]
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
+  const int N = p.N;
+  for (int c = tid; c < C; c += 64 * NW)
+    ln[c] = p.ln_in_w[c], ln[C + c] = p.ln_in_b[c], ln[2 * C + c] = p.ln_out_w[c], ln[3 * C + c] = p.ln_out_b[c];
+  OutWeights<C> w;
+  w.load(p.s_g, p.s_z, wave, l32, lh, lds + Tile::SLOTS + wave * (KS * 64));
+  __syncthreads();
+
+  struct Place {
+    int b, i, j0;
+  };
+  auto place = [&](int id) {
+    Place t;
+    const int bi = id / panels;
+    t.j0 = 32 * (id - bi * panels);
+    t.b = bi / N;
+    t.i = bi - t.b * N;
+    return t;
+  };
+  const int xpos = tid & 31, xg = tid >> 5;
+  RowRegs<C> zraw[TASKS];
+  float xraw[16];  // channels 8 xg .. + 7 and C / 2 + 8 xg .. + 7
+  const size_t NN = (size_t)N * N;
+  auto load_tile = [&](int id) {
+    const Lane here = lane_here();
+    const int li = here.li, lg = here.lg;
+    const Place t = place(id);
+    const float* base = p.z + t.b * p.zc.stride_b + t.i * p.zc.stride_r;
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      int j = t.j0 + 4 * (wave + NW * u) + lg;
+      j = j < N ? j : N - 1;
+      load_row<C>(base + j * p.zc.stride_k, li, zraw[u]);
+    }
+    int j = t.j0 + xpos;
+    j = j < N ? j : N - 1;
+    const float* xp = p.x + (((size_t)t.b * C + 8 * xg) * N + t.i) * N + j;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) xraw[e] = xp[e * NN], xraw[8 + e] = xp[(C / 2 + e) * NN];
+  };
+
+  int id = grid_slot();
+  if (id < total) load_tile(id);
+  for (; id < total; id += gridDim.x) {
+    const Place t = place(id);
+    const Lane here = lane_here();
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      const int li = here.li, pos = 4 * (wave + NW * u) + here.lg;
+      float4 y[C / 64];
+      norm_row<C>(zraw[u], t.j0 + pos < N, ln, li, y);
+#pragma unroll
+      for (int e = 0; e < C / 64; ++e) tile.store4(pos, li + 16 * e, y[e]);
+    }
+    {
+      float s = 0.f, q = 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s += xraw[e];
+      s *= 0.0625f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) q += (xraw[e] - s) * (xraw[e] - s);
+      red[xg * 32 + xpos] = s;
+      red[(NG + xg) * 32 + xpos] = q;
+    }
+    __syncthreads();  // LayerNorm(z) is complete
+    f32x16_t gate = w.gate(tile);
+    __syncthreads();  // everybody has read it
+    {
+      // mean of the groups' means; squared deviations = within the groups + 16 x those of the groups' means
+      float mg[NG], mean = 0.f, q = 0.f;
+#pragma unroll
+      for (int g = 0; g < NG; ++g) mean += mg[g] = red[g * 32 + xpos];
+      mean *= 1.f / NG;
+#pragma unroll
+      for (int g = 0; g < NG; ++g) q += red[(NG + g) * 32 + xpos] + 16.f * ((mg[g] - mean) * (mg[g] - mean));
+      const float rstd = 1.0f / sqrtf(q * (1.f / C) + kEps);
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        const float* wv = ln + 2 * C + hf * (C / 2) + 8 * xg;
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = (xraw[8 * hf + e] - mean) * rstd * wv[e] + wv[C + e];
+        tile.store8(xpos, hf * (C / 16) + xg, y);
+      }
+    }
+    load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
+    __syncthreads();  // LayerNorm(x) is complete
+    f32x16_t acc = unit_product<C, true>(tile, w.o);
+    __syncthreads();  // everybody has read it
+    const Lane out = lane_here();
+    if (t.j0 + out.l32 < N) {
+      const int64_t off = t.b * p.zc.stride_b + t.i * p.zc.stride_r + (t.j0 + out.l32) * p.zc.stride_k + 32 * wave + 16 * out.lh;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[v] *= sigmoid_hw_f32(gate[v]);
+      store_row16(p.z + off, p.out + off, acc, p.add_residual);
+    }
+  }
+}
+
+// ---- triangle attention, input pass: q / sqrt(D), k, v^T as split operands of the core, triangle bias --------
+// Wave = one 32-channel tile of q, k or v (12 waves at 128 channels, three per SIMD).  Tile = one 32-position panel;
+// double buffered, one barrier per tile (three panels per barrier: 417 against 385 us at N = 768).  The H rows of the
+// triangle bias are dot products taken on the normalised rows while they are in registers.
+template <int C>
+struct AttProjLds {
+  static constexpr size_t kBytes = (size_t)2 * PassTile<C>::SLOTS * 16 + (2 * C + 8 * C) * sizeof(float);
+};
+
+template <int C>
+__global__ __launch_bounds__(6 * C) void triattn_proj_pass(TriattnF32 p, int panels, int total) {
+  typedef PassTile<C> Tile;
+  constexpr int OT = C / 32, NW = 3 * OT, KS = C / 16, TASKS = (8 + NW - 1) / NW;
+  extern __shared__ u32x4_t lds[];
+  float* ln = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS);  // [2][C]
+  float* wb = ln + 2 * C;                                       // [H][C], H <= 8
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int N = p.N, H = p.H, kind = wave / OT, ot = wave % OT;
+  const bool narrow = p.D == 16;
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c], ln[C + c] = p.ln_b[c];
+  for (int c = tid; c < H * C; c += 64 * NW) wb[c] = p.w_b[c];
+  u32x4_t w[KS][3];
+  load_unit<C, 3>(kind == 0 ? p.s_q : kind == 1 ? p.s_k : p.s_v, ot, tid & 63, w);
+  __syncthreads();
+  const float scale = 1.0f / sqrtf((float)p.D);
+
+  // panel -> its row (b N + i) and first position
+  auto row_of = [&](int pn, int& j0) {
+    const int bi = pn / panels;
+    j0 = 32 * (pn - bi * panels);
+    return bi;
+  };
+  RowRegs<C> raw[TASKS];  // task u of this wave: rows 4 (wave + NW u) .. + 3, where these are below 32
+  auto load_tile = [&](int pn) {
+    const Lane here = lane_here();
+    int j0;
+    const int bi = row_of(pn, j0), b = bi / N, i = bi - b * N;
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u)
+      if (wave + NW * u < 8) {
+        int j = j0 + 4 * (wave + NW * u) + here.lg;
+        j = j < N ? j : N - 1;
+        load_row<C>(p.x + b * p.xv.stride_b + i * p.xv.stride_r + j * p.xv.stride_k, here.li, raw[u]);
+      }
+  };
+  // the operands of a step are read one step ahead, no further: read as early as the compiler would have it, they do
+  // not fit the registers of three waves per SIMD
+  auto product = [&](auto w_rows, const Tile& t) {
+    f32x16_t acc = zero16();
+    u32x4_t nxt[3];
+    const Lane at = lane_here();
+    auto read = [&](int s) {
+      const u32x4_t* x = t.s + Tile::slot(at.l32, 2 * s + at.lh);
+      nxt[0] = x[0], nxt[1] = x[Tile::PLANE], nxt[2] = x[2 * Tile::PLANE];
+    };
+    read(0);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const u32x4_t op[3] = {nxt[0], nxt[1], nxt[2]};
+      if (s + 1 < KS) read(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      acc = step6<decltype(w_rows)::value>(w[s][0], w[s][1], w[s][2], op, acc);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return acc;
+  };
+  auto split_store = [&](bf16_t* dst, long plane8, size_t slot, const f32x16_t& acc, int st, float mul) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = acc[8 * st + e] * mul;
+    u32x4_t h, m, lo;
+    split8(x, h, m, lo);
+    u32x4_t* d4 = reinterpret_cast<u32x4_t*>(dst) + slot;
+    d4[0] = h;
+    d4[plane8] = m;
+    d4[2 * plane8] = lo;
+  };
+
+  int pn = grid_slot(), buf = 0;
+  if (pn < total) load_tile(pn);
+  for (; pn < total; pn += gridDim.x, buf ^= 1) {
+    const Tile xn = {lds + buf * Tile::SLOTS};
+    const Lane here = lane_here();
+    int j0;
+    const int bi = row_of(pn, j0);
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      if (wave + NW * u >= 8) continue;
+      const int li = here.li, pos = 4 * (wave + NW * u) + here.lg;
+      float4 y[C / 64];
+      norm_row<C>(raw[u], j0 + pos < N, ln, li, y);
+#pragma unroll
+      for (int e = 0; e < C / 64; ++e) xn.store4(pos, li + 16 * e, y[e]);
+      float bias = 0.f;  // of head li
+      for (int h = 0; h < H; ++h) {
+        float d = 0.f;
+#pragma unroll
+        for (int e = 0; e < C / 64; ++e) {
+          const float4 v = *reinterpret_cast<const float4*>(wb + h * C + 64 * e + 4 * li);
+          d += y[e].x * v.x, d += y[e].y * v.y, d += y[e].z * v.z, d += y[e].w * v.w;
+        }
+        d = group_sum<16>(d);
+        bias = li == h ? d : bias;
+      }
+      if (li < H) {  // rows padded to whole panels: zero rows store zeros
+        const int b = bi / N, i = bi - b * N;
+        p.tb[(((size_t)b * H + li) * N + i) * p.Jp + j0 + pos] = bias;
+      }
+    }
+    load_tile(pn + (int)gridDim.x < total ? pn + gridDim.x : pn);
+    __syncthreads();  // this tile is complete, and everybody has finished with the other buffer
+    const Lane out = lane_here();
+    const int l32 = out.l32, lh = out.lh, lane = l32 + 32 * lh, nt = p.Jp / 32, jt = j0 / 32;
+    const size_t row = bi;
+    // A 32-column tile of the projections is one head, or two of width 16.  q and k: head channels in the
+    // registers, positions in the lanes; v the other way round.  Registers 8 st .. + 7 of a lane are its operand
+    // for step st (narrow heads: q, k have one step, that of head 2 ot + st; lane l32 of the v tile is row
+    // l32 % 16 of head 2 ot + l32 / 16, whose rows 16 .. 31 are written as zeros).
+    if (kind < 2) {
+      const f32x16_t acc = product(std::true_type{}, xn);
+      const float mul = kind == 0 ? scale : 1.f;  // q / sqrt(c) after the projection (attention.py:283-284)
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        const size_t slot = narrow ? ((row * H + 2 * ot + st) * nt + jt) * 64 + lane : (((row * H + ot) * nt + jt) * 2 + st) * 64 + lane;
+        split_store(kind == 0 ? p.qs : p.ks, p.qk_plane / 8, slot, acc, st, mul);
+      }
+    } else {
+      const f32x16_t acc = product(std::false_type{}, xn);
+      const int head = narrow ? 2 * ot + (l32 >> 4) : ot, vrow = narrow ? (l32 & 15) : l32;
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        const size_t slot = (((row * H + head) * nt + jt) * 2 + st) * 64 + vrow + 32 * lh;
+        split_store(p.vs, p.v_plane / 8, slot, acc, st, 1.f);
+        if (narrow) {
+          const u32x4_t zero = {0u, 0u, 0u, 0u};
+          u32x4_t* d4 = reinterpret_cast<u32x4_t*>(p.vs) + slot + 16;
+          d4[0] = zero;
+          d4[p.v_plane / 8] = zero;
+          d4[2 * (p.v_plane / 8)] = zero;
+        }
+      }
+    }
+  }
+}
+
+// ---- triangle attention, output pass: out = [x +] (o * sigmoid(LN(x) Wg^T)) Wo^T
+// A wave's 16 channels of a position are consecutive: 64 bytes of o, and two chunks of the second product's operand.
+template <int C>
+__global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int panels, int total) {
+  typedef PassTile<C> Tile;
+  constexpr int NW = C / 32, KS = C / 16, TASKS = 8 / NW;
+  extern __shared__ u32x4_t lds[];
+  const Tile tile = {lds};
+  float* ln = reinterpret_cast<float*>(lds + Tile::SLOTS + OutLds<C>::kWl);  // [2][C]
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
+  const int N = p.N;
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c], ln[C + c] = p.ln_b[c];
+  OutWeights<C> w;
+  w.load(p.s_g, p.s_o, wave, l32, lh, lds + Tile::SLOTS + wave * (KS * 64));
+  __syncthreads();
+
+  auto place = [&](int id, int& b, int& i) {  // returns the first position
+    const int bi = id / panels;
+    b = bi / N;
+    i = bi - b * N;
+    return 32 * (id - bi * panels);
+  };
+  RowRegs<C> raw[TASKS];
+  float4 oraw[4];
+  auto load_tile = [&](int id) {
+    const Lane here = lane_here();
+    const int li = here.li, lg = here.lg;
+    int b, i;
+    const int j0 = place(id, b, i);
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      int j = j0 + 4 * (wave + NW * u) + lg;
+      j = j < N ? j : N - 1;
+      load_row<C>(p.x + b * p.xv.stride_b + i * p.xv.stride_r + j * p.xv.stride_k, li, raw[u]);
+    }
+    const int j = j0 + here.l32 < N ? j0 + here.l32 : N - 1;
+    const float* op = p.o + (((size_t)b * N + i) * N + j) * C + 32 * wave + 16 * here.lh;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) oraw[a] = *reinterpret_cast<const float4*>(op + 4 * a);
+  };
+
+  int id = grid_slot();
+  if (id < total) load_tile(id);
+  for (; id < total; id += gridDim.x) {
+    int b, i;
+    const int j0 = place(id, b, i);
+    const Lane here = lane_here();
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      const int li = here.li, pos = 4 * (wave + NW * u) + here.lg;
+      float4 y[C / 64];
+      norm_row<C>(raw[u], j0 + pos < N, ln, li, y);
+#pragma unroll
+      for (int e = 0; e < C / 64; ++e) tile.store4(pos, li + 16 * e, y[e]);
+    }
+    __syncthreads();  // LayerNorm(x) is complete
+    const f32x16_t gate = w.gate(tile);
+    __syncthreads();  // everybody has read it
+    const Lane mid = lane_here();
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const float4 o0 = oraw[2 * hf], o1 = oraw[2 * hf + 1];
+      const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
+      float y[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = ov[e] * sigmoid_hw_f32(gate[8 * hf + e]);
+      tile.store8(mid.l32, 4 * wave + 2 * mid.lh + hf, y);
+    }
+    load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
+    __syncthreads();  // the gated output is complete
+    const f32x16_t acc = unit_product<C, true>(tile, w.o);
+    __syncthreads();  // everybody has read it
+    const Lane out = lane_here();
+    if (j0 + out.l32 < N) {
+      const int64_t off = b * p.xv.stride_b + i * p.xv.stride_r + (j0 + out.l32) * p.xv.stride_k + 32 * wave + 16 * out.lh;
+      store_row16(p.x + off, p.out + off, acc, p.add_residual);
+    }
+  }
+}
+
+bool rows_aligned(const float* p, const PairView& v) {
+  return (reinterpret_cast<uintptr_t>(p) & 15u) == 0 && ((v.stride_b | v.stride_r | v.stride_k) & 3) == 0;
+}
+
+// persistent grid: what fits the device at once, at most one work-group per tile
+template <auto Kern>
+hipError_t resident_grid(int threads, size_t lds, long tiles, unsigned* grid) {
+  static int cache[kMaxDevices];
+  int fit = 0;
+  hipError_t e = allow_dynamic_lds<Kern>(lds);
+  if (e != hipSuccess) return e;
+  e = per_device(
+      cache,
+      [&](int dev, int* v) {
+        int cus = 0, per_cu = 0;
+        hipError_t s = cu_count(dev, &cus);
+        if (s == hipSuccess) s = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, Kern, threads, lds);
+        *v = cus * (per_cu > 0 ? per_cu : 1);
+        return s;
+      },
+      &fit);
+  *grid = (unsigned)(tiles < fit ? tiles : fit);
+  return e;
+}
+
+template <int C>
+hipError_t launch_trimul_proj(const TrimulF32& p, hipStream_t stream) {
+  const int panels = p.Np / 32, row_groups = (p.N + 3) / 4;
+  const long total = (long)p.B * row_groups * panels * 4;
+  if (total > 0x3fffffffL) return hipErrorInvalidValue;
+  unsigned grid = 0;
+  hipError_t e = resident_grid<trimul_proj_pass<C>>(256, ProjLds<C>::kBytes, C == 128 ? 2 * total : total, &grid);
+  if (e != hipSuccess) return e;
+  if (C == 128) grid &= ~1u;  // a and b
+  hipLaunchKernelGGL(trimul_proj_pass<C>, dim3(grid), dim3(256), ProjLds<C>::kBytes, stream, p, panels, row_groups, (int)total);
+  return hipGetLastError();
+}
+
+template <int C>
+hipError_t launch_trimul_out(const TrimulF32& p, hipStream_t stream) {
+  const int panels = p.Np / 32;
+  const long total = (long)p.B * p.N * panels;
+  if (total > 0x3fffffffL) return hipErrorInvalidValue;
+  unsigned grid = 0;
+  hipError_t e = resident_grid<trimul_out_pass<C>>(2 * C, OutLds<C>::kTrimul, total, &grid);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(trimul_out_pass<C>, dim3(grid), dim3(2 * C), OutLds<C>::kTrimul, stream, p, panels, (int)total);
+  return hipGetLastError();
+}
+
+template <int C>
+hipError_t launch_triattn_proj(const TriattnF32& p, hipStream_t stream) {
+  const int panels = p.Jp / 32;
+  const long total = (long)p.B * p.N * panels;
+  if (total > 0x3fffffffL) return hipErrorInvalidValue;
+  unsigned grid = 0;
+  hipError_t e = resident_grid<triattn_proj_pass<C>>(6 * C, AttProjLds<C>::kBytes, total, &grid);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(triattn_proj_pass<C>, dim3(grid), dim3(6 * C), AttProjLds<C>::kBytes, stream, p, panels, (int)total);
+  return hipGetLastError();
+}
+
+template <int C>
+hipError_t launch_triattn_out(const TriattnF32& p, hipStream_t stream) {
+  const int panels = p.Jp / 32;
+  const long total = (long)p.B * p.N * panels;
+  if (total > 0x3fffffffL) return hipErrorInvalidValue;
+  unsigned grid = 0;
+  hipError_t e = resident_grid<triattn_out_pass<C>>(2 * C, OutLds<C>::kTriattn, total, &grid);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(triattn_out_pass<C>, dim3(grid), dim3(2 * C), OutLds<C>::kTriattn, stream, p, panels, (int)total);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+bool trimul_pass_serves(const TrimulF32& p) {
+  return p.C == p.CH && (p.C == 64 || p.C == 128) && rows_aligned(p.z, p.zv) && rows_aligned(p.out, p.zc) &&
+         (long)p.B * (p.N + 3) * (p.Np / 32) <= 0x3fffffffL;
+}
+hipError_t trimul_proj_pass_f32(const TrimulF32& p, hipStream_t stream) {
+  return p.C == 128 ? launch_trimul_proj<128>(p, stream) : launch_trimul_proj<64>(p, stream);
+}
+hipError_t trimul_out_pass_f32(const TrimulF32& p, hipStream_t stream) {
+  return p.C == 128 ? launch_trimul_out<128>(p, stream) : launch_trimul_out<64>(p, stream);
+}
+
+bool triattn_pass_serves(const TriattnF32& p) {
+  return p.H * p.D == p.C && (p.C == 64 || p.C == 128) && p.H <= 8 && rows_aligned(p.x, p.xv) && rows_aligned(p.out, p.xv) &&
+         (long)p.B * p.N * (p.Jp / 32) <= 0x3fffffffL;
+}
+hipError_t triattn_proj_pass_f32(const TriattnF32& p, hipStream_t stream) {
+  return p.C == 128 ? launch_triattn_proj<128>(p, stream) : launch_triattn_proj<64>(p, stream);
+}
+hipError_t triattn_out_pass_f32(const TriattnF32& p, hipStream_t stream) {
+  return p.C == 128 ? launch_triattn_out<128>(p, stream) : launch_triattn_out<64>(p, stream);
+}
+
+}  // namespace of3

@@ -35,6 +35,7 @@ SOURCES = [
     "single_attn.hip",
     "single_transition.hip",
     "pair_f32.hip",
+    "pair_pass_f32.hip",
     "single_f32.hip",
     "single_x3_f32.hip",
 ]
