@@ -194,6 +194,8 @@ hipError_t row_transition_fwd_f32(const RowTransitionF32Args& args, hipStream_t 
 bool row_transition_x3_serves(const RowTransitionF32Args& args);
 hipError_t row_transition_x3_fwd_f32(const RowTransitionF32Args& args, hipStream_t stream);
 
+struct WeightX3;  // of3_pair_f32.h
+
 // ---- fp32 path (pair_f32.hip): whole updates, any N, C and C_hidden <= 256, head width 16/32/64
 struct TrimulF32Args {
   const float* z;
@@ -204,6 +206,7 @@ struct TrimulF32Args {
   const float *w_ap, *w_ag, *w_bp, *w_bg, *w_g, *w_z;
   float *a, *b, *x;                  // workspace, [B][CH][N][N] each
   void* wsplit;                      // workspace, trimul_wsplit_bytes(C, CH) bytes, 16-byte aligned; may be null
+  const WeightX3* presplit = nullptr;  // the weights as split before (of3_weight_split.h), or null: split by the call
   void* ab_split;                    // workspace, trimul_ab_split_bytes(B, N, CH) bytes, 16-byte aligned, may
                                      // overlap a and b; may be null
   float* out;
@@ -230,6 +233,7 @@ struct TriattnF32Args {
   float *tb;                         // workspace, [B][H][N][N rounded up to a multiple of 32]
   float *o;                          // workspace, [B][N][N][H*D]
   void* wsplit;                      // workspace, triattn_wsplit_bytes(C, H, D) bytes, 16-byte aligned; may be null
+  const WeightX3* presplit = nullptr;
   void* qkv_split;                   // workspace, triattn_qkv_split_bytes(B, N, H, D) bytes, 16-byte aligned, may
                                      // overlap q, k, v; may be null
   float* out;
@@ -252,6 +256,7 @@ struct TransitionF32Args {
   PairView x_view, mask_view;
   const float *ln_w, *ln_b, *w_a, *w_b, *w_out;  // [C], [C], [HID][C], [HID][C], [C][HID]
   void* wsplit;  // workspace, transition_wsplit_bytes(C, HID) bytes, 16-byte aligned; may be null (fp32 MFMA kernel)
+  const WeightX3* presplit = nullptr;
   float* out;
   int B, N, C, HID, add_residual;
 };

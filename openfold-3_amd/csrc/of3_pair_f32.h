@@ -68,5 +68,15 @@ hipError_t trimul_out_pass_f32(const TrimulF32& p, hipStream_t stream);
 bool triattn_pass_serves(const TriattnF32& p);
 hipError_t triattn_proj_pass_f32(const TriattnF32& p, hipStream_t stream);
 hipError_t triattn_out_pass_f32(const TriattnF32& p, hipStream_t stream);
+// the pair transition likewise (transition_f32.hip)
+bool transition_pass_serves(const TransitionF32Args& a);
+hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, const WeightX3& s_b, const WeightX3& s_out,
+                               hipStream_t stream);
+
+// projections off a pair tensor (pair_proj_f32.hip)
+bool pair_bias_pass_serves(const PairBiasF32Args& a);
+hipError_t pair_bias_pass_f32(const PairBiasF32Args& a, hipStream_t stream);
+bool template_tail_pass_serves(const TemplateTailF32Args& a);
+hipError_t template_tail_pass_f32(const TemplateTailF32Args& a, hipStream_t stream);
 
 }  // namespace of3

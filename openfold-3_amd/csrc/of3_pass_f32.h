@@ -1,0 +1,196 @@
+// Building blocks of the fp32 position-wise passes on split operands (pair_pass_f32.hip, transition_f32.hip): LDS tiles
+// of 32 positions in three bf16 planes, LayerNorm of rows spread over 16 lanes, six-product MFMA steps.
+#pragma once
+
+#include "of3_device.h"
+#include "of3_launch.h"
+#include "of3_pair_f32.h"
+#include "of3_split.h"
+
+namespace of3 {
+namespace pass_f32 {
+
+constexpr float kEps = 1e-5f;
+constexpr float kLog2eF32 = 1.4426950408889634f;
+__device__ __forceinline__ float sigmoid_hw_f32(float x) {
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * kLog2eF32));
+}
+
+// four values as the halves of three MFMA operand chunks
+__device__ __forceinline__ void split4(const float4& x, u32x2_t& h, u32x2_t& m, u32x2_t& l) {
+  const float v[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    const float a = v[2 * w], b = v[2 * w + 1];
+    const uint32_t ph = pack_bf16(a, b);
+    const float ra = a - __uint_as_float(ph << 16), rb = b - __uint_as_float(ph & 0xffff0000u);
+    const uint32_t pm = pack_bf16(ra, rb);
+    h[w] = ph;
+    m[w] = pm;
+    l[w] = pack_bf16(ra - __uint_as_float(pm << 16), rb - __uint_as_float(pm & 0xffff0000u));
+  }
+}
+
+// LDS tile of 32 positions x C channels: three planes [position][C / 8 chunks of 8 bf16].  The 16 lanes of a read
+// phase hold 16 consecutive positions at one chunk index: the key spreads them over the banks.
+template <int C>
+struct PassTile {
+  static constexpr int NCH = C / 8, PLANE = 32 * NCH, SLOTS = 3 * PLANE;  // in 16-byte slots
+  u32x4_t* s;
+  __device__ __forceinline__ static int slot(int pos, int chunk) {
+    return pos * NCH + (chunk ^ (NCH >= 16 ? (pos & 15) : ((pos >> 1) & 7)));
+  }
+  // channels 4 c4 .. + 3 of a position
+  __device__ __forceinline__ void store4(int pos, int c4, const float4& y) const {
+    u32x2_t h, m, l;
+    split4(y, h, m, l);
+    u32x2_t* d = reinterpret_cast<u32x2_t*>(s) + 2 * slot(pos, c4 >> 1) + (c4 & 1);
+    d[0] = h;
+    d[2 * PLANE] = m;
+    d[4 * PLANE] = l;
+  }
+  // channels 8 chunk .. + 7
+  __device__ __forceinline__ void store8(int pos, int chunk, const float (&y)[8]) const {
+    u32x4_t h, m, l;
+    split8(y, h, m, l);
+    u32x4_t* d = s + slot(pos, chunk);
+    d[0] = h;
+    d[PLANE] = m;
+    d[2 * PLANE] = l;
+  }
+};
+
+// The lane number, opaque to the compiler: what is derived from it inside a tile loop is recomputed there (a few
+// instructions) instead of being hoisted into registers that the weights occupy.
+struct Lane {
+  int l32, lh, li, lg;
+};
+__device__ __forceinline__ Lane lane_here() {
+  int lane = threadIdx.x & 63;
+  __asm__ volatile("" : "+v"(lane));
+  return {lane & 31, lane >> 5, lane & 15, lane >> 4};
+}
+
+// A row of C channels over 16 lanes: lane li holds channels 64 e + 4 li .. + 3 (a wave reads four rows at a time,
+// 256 contiguous bytes of each per instruction)
+template <int C>
+struct RowRegs {
+  float4 v[C / 64];
+};
+template <int C>
+__device__ __forceinline__ void load_row(const float* row, int li, RowRegs<C>& r) {
+#pragma unroll
+  for (int e = 0; e < C / 64; ++e) r.v[e] = *reinterpret_cast<const float4*>(row + 64 * e + 4 * li);
+}
+// LayerNorm of the row (two-pass statistics); ln: LDS, weights [C] then biases [C]
+template <int C>
+__device__ __forceinline__ void norm_row(const RowRegs<C>& r, bool has, const float* ln, int li, float4 (&y)[C / 64]) {
+  float s = 0.f;
+#pragma unroll
+  for (int e = 0; e < C / 64; ++e) s += (r.v[e].x + r.v[e].y) + (r.v[e].z + r.v[e].w);
+  const float mean = group_sum<16>(s) * (1.f / C);
+  float q = 0.f;
+#pragma unroll
+  for (int e = 0; e < C / 64; ++e) {
+    y[e].x = r.v[e].x - mean, y[e].y = r.v[e].y - mean, y[e].z = r.v[e].z - mean, y[e].w = r.v[e].w - mean;
+    q += y[e].x * y[e].x + y[e].y * y[e].y + y[e].z * y[e].z + y[e].w * y[e].w;
+  }
+  const float rstd = 1.0f / sqrtf(group_sum<16>(q) * (1.f / C) + kEps);
+#pragma unroll
+  for (int e = 0; e < C / 64; ++e) {
+    const float4 w = *reinterpret_cast<const float4*>(ln + 64 * e + 4 * li);
+    const float4 b = *reinterpret_cast<const float4*>(ln + C + 64 * e + 4 * li);
+    y[e].x = has ? y[e].x * rstd * w.x + b.x : 0.f;
+    y[e].y = has ? y[e].y * rstd * w.y + b.y : 0.f;
+    y[e].z = has ? y[e].z * rstd * w.z + b.z : 0.f;
+    y[e].w = has ? y[e].w * rstd * w.w + b.w : 0.f;
+  }
+}
+
+// the split operands of output rows 32 t .. + 31 of a weight matrix with K = C inputs; lane_src: whose packed
+// operand this lane takes (its own, or rowperm16's to deal the rows so that a lane ends with 16 consecutive ones)
+template <int C, int TERMS>
+__device__ __forceinline__ void load_unit(const WeightX3& W, int t, int lane_src, u32x4_t (&w)[C / 16][TERMS]) {
+  const u32x4_t* src = reinterpret_cast<const u32x4_t*>(W.h) + (size_t)t * (C / 16) * 64 + lane_src;
+#pragma unroll
+  for (int s = 0; s < C / 16; ++s)
+#pragma unroll
+    for (int pl = 0; pl < TERMS; ++pl) w[s][pl] = src[pl * (W.plane / 8) + 64 * s];
+}
+
+// one k-step: six products, smallest terms first (one chain of dependent MFMAs: two alternating chains were no
+// faster, their second accumulator is what some of the kernels spill for).  W_ROWS: the outputs are the MFMA rows,
+// otherwise the positions
+template <bool W_ROWS>
+__device__ __forceinline__ f32x16_t mm(u32x4_t w, u32x4_t x, f32x16_t acc) {
+  return W_ROWS ? mfma_32x32x16(w, x, acc) : mfma_32x32x16(x, w, acc);
+}
+template <bool W_ROWS>
+__device__ __forceinline__ f32x16_t step6(const u32x4_t (&w)[3], const u32x4_t (&x)[3], f32x16_t acc) {
+  acc = mm<W_ROWS>(w[2], x[0], acc);
+  acc = mm<W_ROWS>(w[0], x[2], acc);
+  acc = mm<W_ROWS>(w[1], x[1], acc);
+  acc = mm<W_ROWS>(w[1], x[0], acc);
+  acc = mm<W_ROWS>(w[0], x[1], acc);
+  return mm<W_ROWS>(w[0], x[0], acc);
+}
+template <int C, bool W_ROWS>
+__device__ __forceinline__ f32x16_t unit_product(const PassTile<C>& t, const u32x4_t (&w)[C / 16][3]) {
+  f32x16_t acc = zero16();
+  const Lane at = lane_here();
+#pragma unroll
+  for (int s = 0; s < C / 16; ++s) {
+    const u32x4_t* x = t.s + PassTile<C>::slot(at.l32, 2 * s + at.lh);
+    const u32x4_t op[3] = {x[0], x[PassTile<C>::PLANE], x[2 * PassTile<C>::PLANE]};
+    acc = step6<W_ROWS>(w[s], op, acc);
+  }
+  return acc;
+}
+
+// out row (16 channels from op on) = [residual +] v * g
+__device__ __forceinline__ void store_row16(const float* zp, float* op, const f32x16_t& v, bool add_residual) {
+  float4 z[4];
+  if (add_residual) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) z[a] = *reinterpret_cast<const float4*>(zp + 4 * a);
+  }
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    float4 r = make_float4(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);
+    if (add_residual) r.x = z[a].x + r.x, r.y = z[a].y + r.y, r.z = z[a].z + r.z, r.w = z[a].w + r.w;
+    *reinterpret_cast<float4*>(op + 4 * a) = r;
+  }
+}
+
+// logical number of a work-group: consecutive numbers run on one XCD where the grid deals evenly
+__device__ __forceinline__ int grid_slot() {
+  return gridDim.x % 8 == 0 ? xcd_logical_block(blockIdx.x, gridDim.x / 8) : blockIdx.x;
+}
+
+inline bool rows_aligned(const float* p, const PairView& v) {
+  return (reinterpret_cast<uintptr_t>(p) & 15u) == 0 && ((v.stride_b | v.stride_r | v.stride_k) & 3) == 0;
+}
+
+// persistent grid: what fits the device at once, at most one work-group per tile
+template <auto Kern>
+hipError_t resident_grid(int threads, size_t lds, long tiles, unsigned* grid) {
+  static int cache[kMaxDevices];
+  int fit = 0;
+  hipError_t e = allow_dynamic_lds<Kern>(lds);
+  if (e != hipSuccess) return e;
+  e = per_device(
+      cache,
+      [&](int dev, int* v) {
+        int cus = 0, per_cu = 0;
+        hipError_t s = cu_count(dev, &cus);
+        if (s == hipSuccess) s = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, Kern, threads, lds);
+        *v = cus * (per_cu > 0 ? per_cu : 1);
+        return s;
+      },
+      &fit);
+  *grid = (unsigned)(tiles < fit ? tiles : fit);
+  return e;
+}
+
+}  // namespace pass_f32
+}  // namespace of3

@@ -8,6 +8,7 @@
 
 #include "of3_kernels.h"
 #include "of3_launch.h"
+#include "of3_weight_split.h"
 
 // Built-in scratch of of3_trimul_fwd_static: one copy per GPU the library runs on, held until the
 // process ends.  In host code this name is only a handle for hipGetSymbolAddress; the device
@@ -255,8 +256,9 @@ int of3_trimul_out(const void* x, const void* z, const int64_t z_strides[3], voi
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
-int of3_trimul_fwd(const void* z, const int64_t z_strides[3], const float* mask, const int64_t mask_strides[3],
-                   const void* ln_in_w, const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
+// presplit: the fp32 weights as a block's call has split them, or null
+static int trimul_fwd(const of3::WeightX3* presplit, const void* z, const int64_t z_strides[3], const float* mask,
+                   const int64_t mask_strides[3], const void* ln_in_w, const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
                    const void* w_a_p, const void* w_a_g, const void* w_b_p, const void* w_b_g, const void* w_g,
                    const void* w_z, void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int outgoing,
                    int add_residual, void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
@@ -292,6 +294,7 @@ int of3_trimul_fwd(const void* z, const int64_t z_strides[3], const float* mask,
     a.ab_split = ws;  // in place of a and b
     a.x = reinterpret_cast<float*>(ws + ab);
     a.wsplit = ws + ab + part;
+    a.presplit = presplit;
     a.out = static_cast<float*>(out);
     a.B = (int)B;
     a.N = (int)N;
@@ -318,6 +321,15 @@ int of3_trimul_fwd(const void* z, const int64_t z_strides[3], const float* mask,
   if (st != OF3_OK) return st;
   return of3_trimul_out(x, z, z_strides, out, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_g, w_z, B, N, C, CH,
                         add_residual, stream);
+}
+
+int of3_trimul_fwd(const void* z, const int64_t z_strides[3], const float* mask, const int64_t mask_strides[3],
+                   const void* ln_in_w, const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
+                   const void* w_a_p, const void* w_a_g, const void* w_b_p, const void* w_b_g, const void* w_g,
+                   const void* w_z, void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int outgoing,
+                   int add_residual, void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
+  return trimul_fwd(nullptr, z, z_strides, mask, mask_strides, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_a_p, w_a_g, w_b_p,
+                    w_b_g, w_g, w_z, out, B, N, C, CH, outgoing, add_residual, workspace, workspace_bytes, dtype, stream);
 }
 
 int of3_trimul_fwd_static(const void* z, const int64_t z_strides[3], const float* mask,
@@ -432,8 +444,8 @@ int of3_triattn_out(const void* o, const void* x, const int64_t x_strides[3], vo
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
-int of3_triattn_fwd(const void* x, const int64_t x_strides[3], const float* mask, const int64_t mask_strides[3],
-                    const void* ln_w, const void* ln_b, const void* w_bias, const void* w_q, const void* w_k,
+static int triattn_fwd(const of3::WeightX3* presplit, const void* x, const int64_t x_strides[3], const float* mask,
+                    const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_bias, const void* w_q, const void* w_k,
                     const void* w_v, const void* w_g, const void* w_o, void* out, int64_t B, int64_t N, int64_t C,
                     int64_t H, int64_t D, float inf, int add_residual, void* workspace, int64_t workspace_bytes,
                     int dtype, void* stream) {
@@ -468,6 +480,7 @@ int of3_triattn_fwd(const void* x, const int64_t x_strides[3], const float* mask
     a.o = reinterpret_cast<float*>(ws + qkv);
     a.tb = reinterpret_cast<float*>(ws + qkv + part);
     a.wsplit = ws + qkv + part + f32_triattn_tb_bytes(B, N, H);
+    a.presplit = presplit;
     a.out = static_cast<float*>(out);
     a.B = (int)B;
     a.N = (int)N;
@@ -500,6 +513,15 @@ int of3_triattn_fwd(const void* x, const int64_t x_strides[3], const float* mask
   return of3_triattn_out(o, x, x_strides, out, ln_w, ln_b, w_g, w_o, B, N, C, H, D, add_residual, stream);
 }
 
+int of3_triattn_fwd(const void* x, const int64_t x_strides[3], const float* mask, const int64_t mask_strides[3],
+                    const void* ln_w, const void* ln_b, const void* w_bias, const void* w_q, const void* w_k,
+                    const void* w_v, const void* w_g, const void* w_o, void* out, int64_t B, int64_t N, int64_t C,
+                    int64_t H, int64_t D, float inf, int add_residual, void* workspace, int64_t workspace_bytes,
+                    int dtype, void* stream) {
+  return triattn_fwd(nullptr, x, x_strides, mask, mask_strides, ln_w, ln_b, w_bias, w_q, w_k, w_v, w_g, w_o, out, B, N, C,
+                     H, D, inf, add_residual, workspace, workspace_bytes, dtype, stream);
+}
+
 int64_t of3_transition_workspace_bytes_for(int dtype, int64_t B, int64_t N, int64_t C, int64_t HID) {
   if (dtype == OF3_DTYPE_BF16) return (B >= 1 && N >= 1) ? 0 : (int64_t)OF3_EINVAL;
   if (dtype != OF3_DTYPE_F32 || B < 1 || N < 1 || C < 1 || C > 256 || HID < 1 || HID > 1024) return OF3_EINVAL;
@@ -514,8 +536,8 @@ int of3_transition_fwd(const void* x, const int64_t x_strides[3], const float* m
                                add_residual, nullptr, 0, dtype, stream);
 }
 
-int of3_transition_fwd_ws(const void* x, const int64_t x_strides[3], const float* mask, const int64_t mask_strides[3],
-                          const void* ln_w, const void* ln_b, const void* w_a, const void* w_b, const void* w_out,
+static int transition_fwd(const of3::WeightX3* presplit, const void* x, const int64_t x_strides[3], const float* mask,
+                          const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_a, const void* w_b, const void* w_out,
                           void* out, int64_t B, int64_t N, int64_t C, int64_t HID, int add_residual, void* workspace,
                           int64_t workspace_bytes, int dtype, void* stream) {
   const void* ptrs[] = {x, ln_w, ln_b, w_a, w_b, w_out, out};
@@ -537,6 +559,7 @@ int of3_transition_fwd_ws(const void* x, const int64_t x_strides[3], const float
     a.w_out = f(w_out);
     // with room for the split weights the split-operand kernel runs (where the shape allows)
     a.wsplit = nullptr;
+    a.presplit = presplit;
     if (workspace) {
       if (reinterpret_cast<uintptr_t>(workspace) & 255u) return OF3_EINVAL;
       if (workspace_bytes < of3_transition_workspace_bytes_for(dtype, B, N, C, HID)) return OF3_ENOSPC;
@@ -587,6 +610,14 @@ int of3_transition_fwd_ws(const void* x, const int64_t x_strides[3], const float
   args.add_residual = add_residual ? 1 : 0;
   hipError_t e = of3::transition_launch(args, (int)C, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
+}
+
+int of3_transition_fwd_ws(const void* x, const int64_t x_strides[3], const float* mask, const int64_t mask_strides[3],
+                          const void* ln_w, const void* ln_b, const void* w_a, const void* w_b, const void* w_out,
+                          void* out, int64_t B, int64_t N, int64_t C, int64_t HID, int add_residual, void* workspace,
+                          int64_t workspace_bytes, int dtype, void* stream) {
+  return transition_fwd(nullptr, x, x_strides, mask, mask_strides, ln_w, ln_b, w_a, w_b, w_out, out, B, N, C, HID,
+                        add_residual, workspace, workspace_bytes, dtype, stream);
 }
 
 int of3_pair_bias_fwd(const void* z, const int64_t z_strides[3], const void* ln_w, const void* ln_b, const void* w,
@@ -861,7 +892,12 @@ int of3_transition_rows_fwd(const void* x, const float* mask, const void* ln_w, 
 // module from Python they cost 260 us of host time per PairFormerBlock, more than the kernels take; from one
 // call the launches themselves (2.5 us each) are what is left.
 
-int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
+// room for all matrices of a block split at once (fp32), after the modules' own workspace
+static int64_t block_split_bytes(int64_t C, int64_t CH, int64_t H, int64_t D, int64_t HID) {
+  return align256((int64_t)(2 * of3::trimul_wsplit_bytes(C, CH) + 2 * of3::triattn_wsplit_bytes(C, H, D) +
+                            (HID ? of3::transition_wsplit_bytes(C, HID) : 0)));
+}
+static int64_t pair_block_module_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
                                        int64_t HID) {
   int64_t need = of3_trimul_workspace_bytes_for(dtype, B, N, C, CH);
   const int64_t att = of3_triattn_workspace_bytes_for(dtype, B, N, C, H, D);
@@ -874,6 +910,12 @@ int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t 
     if (tr > need) need = tr;
   }
   return need;
+}
+
+int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
+                                       int64_t HID) {
+  const int64_t need = pair_block_module_bytes(dtype, B, N, C, CH, H, D, HID);
+  return need < 0 || dtype == OF3_DTYPE_BF16 ? need : need + block_split_bytes(C, CH, H, D, HID);
 }
 
 int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t z_strides[3], const float* mask,
@@ -892,9 +934,52 @@ int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t 
   if (wide ? !(aligned4(z) && aligned4(out)) : !(aligned16(z) && aligned16(out))) return OF3_EINVAL;
   if (workspace_bytes < need) return OF3_ENOSPC;
 
+  const void* const* w_mul = weights;
+  const void* const* w_att = weights + 20;
+  const void* const* w_tr = weights + 36;
+  // fp32 on split operands: all matrices of the block in one launch
+  of3::WeightX3 split[2 * of3::kTrimulMatrices + 2 * of3::kTriattnMatrices + of3::kTransitionMatrices];
+  const of3::WeightX3 *s_mul = nullptr, *s_att = nullptr, *s_tr = nullptr;
+  if (wide) {
+    of3::WeightSplitter splitter(static_cast<char*>(workspace) + pair_block_module_bytes(dtype, B, N, C, CH, H, D, HID));
+    auto f = [](const void* p) { return static_cast<const float*>(p); };
+    of3::WeightX3* next = split;
+    if (of3::trimul_split_widths(C, CH)) {
+      s_mul = next;
+      for (int d = 0; d < 2; ++d, next += of3::kTrimulMatrices) {
+        const void* const* w = w_mul + 10 * d;
+        of3::TrimulF32Args a;
+        a.w_ap = f(w[4]), a.w_ag = f(w[5]), a.w_bp = f(w[6]), a.w_bg = f(w[7]), a.w_g = f(w[8]), a.w_z = f(w[9]);
+        a.C = (int)C, a.CH = (int)CH;
+        of3::trimul_split_jobs(splitter, a, next);
+      }
+    }
+    if (of3::triattn_split_widths(C, H, D)) {
+      s_att = next;
+      for (int d = 0; d < 2; ++d, next += of3::kTriattnMatrices) {
+        const void* const* w = w_att + 8 * d;
+        of3::TriattnF32Args a;
+        a.w_q = f(w[3]), a.w_k = f(w[4]), a.w_v = f(w[5]), a.w_g = f(w[6]), a.w_o = f(w[7]);
+        a.C = (int)C, a.H = (int)H, a.D = (int)D;
+        of3::triattn_split_jobs(splitter, a, next);
+      }
+    }
+    if (HID && of3::transition_split_widths(C, HID)) {
+      s_tr = next;
+      of3::TransitionF32Args a;
+      a.w_a = f(w_tr[2]), a.w_b = f(w_tr[3]), a.w_out = f(w_tr[4]);
+      a.C = (int)C, a.HID = (int)HID;
+      of3::transition_split_jobs(splitter, a, next);
+    }
+    if (splitter.j.n > 0) {
+      const hipError_t e = splitter.launch(static_cast<hipStream_t>(stream));
+      if (e != hipSuccess) return fail_hip(e);
+    }
+  }
+
   const void* src = z;  // the first module reads z, every later one updates out in place
   auto trimul = [&](const void* const* w, int outgoing) {
-    const int st = of3_trimul_fwd(src, z_strides, mask, mask_strides, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8],
+    const int st = trimul_fwd(s_mul ? s_mul + (outgoing ? 0 : of3::kTrimulMatrices) : nullptr, src, z_strides, mask, mask_strides, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8],
                                   w[9], out, B, N, C, CH, outgoing, 1, workspace, workspace_bytes, dtype, stream);
     src = out;
     return st;
@@ -903,13 +988,11 @@ int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t 
     const int64_t zt[3] = {z_strides[0], ending ? z_strides[2] : z_strides[1], ending ? z_strides[1] : z_strides[2]};
     int64_t mt[3] = {0, 0, 0};
     if (mask) mt[0] = mask_strides[0], mt[1] = mask_strides[ending ? 2 : 1], mt[2] = mask_strides[ending ? 1 : 2];
-    const int st = of3_triattn_fwd(src, zt, mask, mt, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], out, B, N, C, H, D,
+    const int st = triattn_fwd(s_att ? s_att + (ending ? of3::kTriattnMatrices : 0) : nullptr, src, zt, mask, mt, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], out, B, N, C, H, D,
                                    inf, 1, workspace, workspace_bytes, dtype, stream);
     src = out;
     return st;
   };
-  const void* const* w_mul = weights;
-  const void* const* w_att = weights + 20;
   int st = OF3_OK;
   for (int part = 0; part < 2 && st == OF3_OK; ++part) {
     if ((part == 0) == !(flags & OF3_BLOCK_ATTENTION_FIRST)) {
@@ -921,10 +1004,9 @@ int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t 
     }
   }
   if (st != OF3_OK || HID == 0) return st;
-  const void* const* t = weights + 36;
-  return of3_transition_fwd_ws(out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask, mask_strides, t[0],
-                               t[1], t[2], t[3], t[4], out, B, N, C, HID, 1, wide ? workspace : nullptr,
-                               wide ? workspace_bytes : 0, dtype, stream);
+  return transition_fwd(s_tr, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask, mask_strides, w_tr[0],
+                        w_tr[1], w_tr[2], w_tr[3], w_tr[4], out, B, N, C, HID, 1, wide ? workspace : nullptr,
+                        wide ? workspace_bytes : 0, dtype, stream);
 }
 
 int64_t of3_pairformer_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,

@@ -21,6 +21,7 @@
 #include "of3_kernels.h"
 #include "of3_launch.h"
 #include "of3_pair_f32.h"
+#include "of3_weight_split.h"
 #include "of3_split.h"
 
 namespace of3 {
@@ -190,67 +191,6 @@ __device__ __forceinline__ TileX3 make_tile_x3(void* base, int K, int tp) {
   return t;
 }
 __host__ __device__ constexpr size_t tile_bytes_x3(int K, int tp) { return (size_t)3 * tp * (K + 8) * sizeof(bf16_t); }
-
-// up to six matrices in one launch
-struct SplitJobs {
-  static constexpr int kMax = 6;
-  const float* src[kMax];
-  bf16_t* dst[kMax];
-  int rows[kMax], K[kMax];
-  long first[kMax + 1];  // first item of each matrix; first[n] = all items
-  int n;
-};
-
-__global__ __launch_bounds__(kThreads) void split_weights_f32(SplitJobs j) {
-  // one thread per (matrix, row tile, step, lane): its 8 consecutive k-values
-  const long gitem = (long)blockIdx.x * kThreads + threadIdx.x;
-  if (gitem >= j.first[j.n]) return;
-  int q = 0;
-#pragma unroll
-  for (int i = 1; i < SplitJobs::kMax; ++i)
-    if (i < j.n && gitem >= j.first[i]) q = i;
-  const float* __restrict__ src = j.src[q];
-  bf16_t* __restrict__ dst = j.dst[q];
-  const int rows = j.rows[q], K = j.K[q];
-  const long item = gitem - j.first[q];
-  const int steps = K / 16;
-  const int lane = (int)(item & 63), l32 = lane & 31, lh = lane >> 5;
-  const long ts = item >> 6;
-  const int s = (int)(ts % steps), t = (int)(ts / steps);
-  int row = 32 * t + l32;
-  row = row < rows ? row : rows - 1;  // rows past the end repeat the last one (their results are dropped)
-  const long plane = packed_elems(rows, K);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const Split3 v = split3(src[(size_t)row * K + 16 * s + 8 * lh + e]);
-    dst[item * 8 + e] = v.h;
-    dst[plane + item * 8 + e] = v.m;
-    dst[2 * plane + item * 8 + e] = v.l;
-  }
-}
-
-// host side: matrices are added one after the other into the workspace, then split by one launch
-struct WeightSplitter {
-  SplitJobs j;
-  bf16_t* w;
-  explicit WeightSplitter(void* workspace) : j(), w(static_cast<bf16_t*>(workspace)) {}
-  void add(const float* src, int rows, int K, WeightX3& dst) {
-    dst.h = w;
-    dst.plane = packed_elems(rows, K);
-    j.src[j.n] = src;
-    j.dst[j.n] = w;
-    j.rows[j.n] = rows;
-    j.K[j.n] = K;
-    j.first[j.n + 1] = j.first[j.n] + dst.plane / 8;
-    ++j.n;
-    w += 3 * dst.plane;
-  }
-  hipError_t launch(hipStream_t stream) const {
-    const long items = j.first[j.n];
-    hipLaunchKernelGGL(split_weights_f32, dim3((unsigned)((items + kThreads - 1) / kThreads)), dim3(kThreads), 0, stream, j);
-    return hipGetLastError();
-  }
-};
 
 // LayerNorm of 32 * TILES positions by NT threads into a split tile, a row per 32 lanes, at most 256 channels (a
 // multiple of 16).  Lane l holds channels 2 l + 64 e and 2 l + 64 e + 1, e < 4.  A row is read once
@@ -2215,6 +2155,7 @@ hipError_t allow_lds(size_t max_bytes = 3 * (size_t)kTP * (kMaxC + 4) * sizeof(f
 
 hipError_t template_tail_fwd_f32(const TemplateTailF32Args& a, hipStream_t stream) {
   if (a.CT < 1 || a.CT > kMaxC || a.CZ < 1 || a.T < 1 || a.P < 1 || a.B < 1) return hipErrorInvalidValue;
+  if (template_tail_pass_serves(a)) return template_tail_pass_f32(a, stream);
   TemplateTailF32 p;
   p.t = a.t;
   p.ln_w = a.ln_w;
@@ -2278,7 +2219,7 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
   const unsigned mblocks = (unsigned)((long)a.B * a.N * mgroups);
   // split-operand kernels for the position-wise passes: channel counts in multiples of 16 and room for
   // the split weights
-  const bool x3 = a.C % 16 == 0 && a.CH % 16 == 0 && a.wsplit && aligned16({a.wsplit});
+  const bool x3 = trimul_split_widths(a.C, a.CH) && (a.presplit || (a.wsplit && aligned16({a.wsplit})));
   // channel counts in multiples of 64 and rows of z on 8-byte boundaries in both frames
   const bool fast = a.C % 64 == 0 && a.CH % 64 == 0 && (reinterpret_cast<uintptr_t>(a.z) & 7u) == 0 &&
                     even_strides(a.z_view) && even_strides(a.z_canonical);
@@ -2291,14 +2232,15 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
   const int xgroups = (a.N + 32 * kXT * kPT - 1) / (32 * kXT * kPT);
   const unsigned xblocks = (unsigned)((long)a.B * a.N * xgroups);
   if (x3) {
-    WeightSplitter splitter(a.wsplit);
-    splitter.add(a.w_ap, a.CH, a.C, p.s_ap);
-    splitter.add(a.w_ag, a.CH, a.C, p.s_ag);
-    splitter.add(a.w_bp, a.CH, a.C, p.s_bp);
-    splitter.add(a.w_bg, a.CH, a.C, p.s_bg);
-    splitter.add(a.w_g, a.C, a.C, p.s_g);
-    splitter.add(a.w_z, a.C, a.CH, p.s_z);
-    if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
+    WeightX3 w[kTrimulMatrices];
+    if (a.presplit) {
+      for (int i = 0; i < kTrimulMatrices; ++i) w[i] = a.presplit[i];
+    } else {
+      WeightSplitter splitter(a.wsplit);
+      trimul_split_jobs(splitter, a, w);
+      if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
+    }
+    p.s_ap = w[0], p.s_ag = w[1], p.s_bp = w[2], p.s_bg = w[3], p.s_g = w[4], p.s_z = w[5];
   }
   const bool pass = split_ab && trimul_pass_serves(p);
   if (pass) {
@@ -2398,7 +2340,7 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
   const bool mm = a.C % 8 == 0 && (a.H * a.D) % 8 == 0 && aligned16({a.w_q, a.w_k, a.w_v, a.w_b, a.w_g, a.w_o});
   const int mgroups = (a.N + kTP - 1) / kTP;
   const unsigned mblocks = (unsigned)((long)a.B * a.N * mgroups);
-  const bool x3 = a.C % 16 == 0 && (a.H * a.D) % 16 == 0 && a.wsplit && aligned16({a.wsplit});
+  const bool x3 = triattn_split_widths(a.C, a.H, a.D) && (a.presplit || (a.wsplit && aligned16({a.wsplit})));
   const bool fast = a.C % 64 == 0 && (a.H * a.D) % 64 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 7u) == 0 &&
                     even_strides(a.x_view);
   // head width 32 or 16 (then an even number of heads: a 32-channel tile of the projections is two of
@@ -2415,14 +2357,15 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
   const int xgroups = (a.N + 32 * kXT * kPT - 1) / (32 * kXT * kPT);
   const unsigned xblocks = (unsigned)((long)a.B * a.N * xgroups);
   if (x3) {
-    WeightSplitter splitter(a.wsplit);
-    const int HD = a.H * a.D;
-    splitter.add(a.w_q, HD, a.C, p.s_q);
-    splitter.add(a.w_k, HD, a.C, p.s_k);
-    splitter.add(a.w_v, HD, a.C, p.s_v);
-    splitter.add(a.w_g, HD, a.C, p.s_g);
-    splitter.add(a.w_o, a.C, HD, p.s_o);
-    if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
+    WeightX3 w[kTriattnMatrices];
+    if (a.presplit) {
+      for (int i = 0; i < kTriattnMatrices; ++i) w[i] = a.presplit[i];
+    } else {
+      WeightSplitter splitter(a.wsplit);
+      triattn_split_jobs(splitter, a, w);
+      if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
+    }
+    p.s_q = w[0], p.s_k = w[1], p.s_v = w[2], p.s_g = w[3], p.s_o = w[4];
   }
   const bool pass = core_x3 && triattn_pass_serves(p);
   if (pass) {
@@ -2512,12 +2455,17 @@ hipError_t transition_fwd_f32(const TransitionF32Args& a, hipStream_t stream) {
   p.C = a.C;
   p.HID = a.HID;
   p.add_residual = a.add_residual;
-  if (a.C % 16 == 0 && a.HID % kTrHC == 0 && a.wsplit && aligned16({a.wsplit})) {
-    WeightSplitter splitter(a.wsplit);
-    splitter.add(a.w_a, a.HID, a.C, p.s_a);
-    splitter.add(a.w_b, a.HID, a.C, p.s_b);
-    splitter.add(a.w_out, a.C, a.HID, p.s_out);
-    if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
+  if (transition_split_widths(a.C, a.HID) && (a.presplit || (a.wsplit && aligned16({a.wsplit})))) {
+    WeightX3 w[kTransitionMatrices];
+    if (a.presplit) {
+      for (int i = 0; i < kTransitionMatrices; ++i) w[i] = a.presplit[i];
+    } else {
+      WeightSplitter splitter(a.wsplit);
+      transition_split_jobs(splitter, a, w);
+      if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
+    }
+    p.s_a = w[0], p.s_b = w[1], p.s_out = w[2];
+    if (transition_pass_serves(a)) return transition_pass_f32(a, p.s_a, p.s_b, p.s_out, stream);
     const bool fast = a.C % 64 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 7u) == 0 && even_strides(a.x_view);
     const bool wide = a.C > 128;
     auto kern = wide ? (fast ? transition_x3_f32<true, true> : transition_x3_f32<true, false>)
@@ -2557,6 +2505,7 @@ hipError_t transition_fwd_f32(const TransitionF32Args& a, hipStream_t stream) {
 
 hipError_t pair_bias_fwd_f32(const PairBiasF32Args& a, hipStream_t stream) {
   if (a.C > kMaxC) return hipErrorInvalidValue;
+  if (pair_bias_pass_serves(a)) return pair_bias_pass_f32(a, stream);
   PairBiasF32 p;
   p.z = a.z;
   p.zv = a.z_view;

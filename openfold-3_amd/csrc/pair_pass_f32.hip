@@ -16,159 +16,18 @@
 #include "of3_kernels.h"
 #include "of3_launch.h"
 #include "of3_pair_f32.h"
+#include "of3_pass_f32.h"
 #include "of3_split.h"
 
 namespace of3 {
 
 namespace {
 
-constexpr float kEps = 1e-5f;
-constexpr float kLog2eF32 = 1.4426950408889634f;
-__device__ __forceinline__ float sigmoid_hw_f32(float x) {
-  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * kLog2eF32));
-}
-
-// four values as the halves of three MFMA operand chunks
-__device__ __forceinline__ void split4(const float4& x, u32x2_t& h, u32x2_t& m, u32x2_t& l) {
-  const float v[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-  for (int w = 0; w < 2; ++w) {
-    const float a = v[2 * w], b = v[2 * w + 1];
-    const uint32_t ph = pack_bf16(a, b);
-    const float ra = a - __uint_as_float(ph << 16), rb = b - __uint_as_float(ph & 0xffff0000u);
-    const uint32_t pm = pack_bf16(ra, rb);
-    h[w] = ph;
-    m[w] = pm;
-    l[w] = pack_bf16(ra - __uint_as_float(pm << 16), rb - __uint_as_float(pm & 0xffff0000u));
-  }
-}
-
-// LDS tile of 32 positions x C channels: three planes [position][C / 8 chunks of 8 bf16].  The 16 lanes of a read
-// phase hold 16 consecutive positions at one chunk index: the key spreads them over the banks.
-template <int C>
-struct PassTile {
-  static constexpr int NCH = C / 8, PLANE = 32 * NCH, SLOTS = 3 * PLANE;  // in 16-byte slots
-  u32x4_t* s;
-  __device__ __forceinline__ static int slot(int pos, int chunk) {
-    return pos * NCH + (chunk ^ (NCH == 16 ? (pos & 15) : ((pos >> 1) & 7)));
-  }
-  // channels 4 c4 .. + 3 of a position
-  __device__ __forceinline__ void store4(int pos, int c4, const float4& y) const {
-    u32x2_t h, m, l;
-    split4(y, h, m, l);
-    u32x2_t* d = reinterpret_cast<u32x2_t*>(s) + 2 * slot(pos, c4 >> 1) + (c4 & 1);
-    d[0] = h;
-    d[2 * PLANE] = m;
-    d[4 * PLANE] = l;
-  }
-  // channels 8 chunk .. + 7
-  __device__ __forceinline__ void store8(int pos, int chunk, const float (&y)[8]) const {
-    u32x4_t h, m, l;
-    split8(y, h, m, l);
-    u32x4_t* d = s + slot(pos, chunk);
-    d[0] = h;
-    d[PLANE] = m;
-    d[2 * PLANE] = l;
-  }
-};
-
-// The lane number, opaque to the compiler: what is derived from it inside a tile loop is recomputed there (a few
-// instructions) instead of being hoisted into registers that the weights occupy.
-struct Lane {
-  int l32, lh, li, lg;
-};
-__device__ __forceinline__ Lane lane_here() {
-  int lane = threadIdx.x & 63;
-  __asm__ volatile("" : "+v"(lane));
-  return {lane & 31, lane >> 5, lane & 15, lane >> 4};
-}
-
-// A row of C channels over 16 lanes: lane li holds channels 64 e + 4 li .. + 3 (a wave reads four rows at a time,
-// 256 contiguous bytes of each per instruction)
-template <int C>
-struct RowRegs {
-  float4 v[C / 64];
-};
-template <int C>
-__device__ __forceinline__ void load_row(const float* row, int li, RowRegs<C>& r) {
-#pragma unroll
-  for (int e = 0; e < C / 64; ++e) r.v[e] = *reinterpret_cast<const float4*>(row + 64 * e + 4 * li);
-}
-// LayerNorm of the row (two-pass statistics); ln: LDS, weights [C] then biases [C]
-template <int C>
-__device__ __forceinline__ void norm_row(const RowRegs<C>& r, bool has, const float* ln, int li, float4 (&y)[C / 64]) {
-  float s = 0.f;
-#pragma unroll
-  for (int e = 0; e < C / 64; ++e) s += (r.v[e].x + r.v[e].y) + (r.v[e].z + r.v[e].w);
-  const float mean = group_sum<16>(s) * (1.f / C);
-  float q = 0.f;
-#pragma unroll
-  for (int e = 0; e < C / 64; ++e) {
-    y[e].x = r.v[e].x - mean, y[e].y = r.v[e].y - mean, y[e].z = r.v[e].z - mean, y[e].w = r.v[e].w - mean;
-    q += y[e].x * y[e].x + y[e].y * y[e].y + y[e].z * y[e].z + y[e].w * y[e].w;
-  }
-  const float rstd = 1.0f / sqrtf(group_sum<16>(q) * (1.f / C) + kEps);
-#pragma unroll
-  for (int e = 0; e < C / 64; ++e) {
-    const float4 w = *reinterpret_cast<const float4*>(ln + 64 * e + 4 * li);
-    const float4 b = *reinterpret_cast<const float4*>(ln + C + 64 * e + 4 * li);
-    y[e].x = has ? y[e].x * rstd * w.x + b.x : 0.f;
-    y[e].y = has ? y[e].y * rstd * w.y + b.y : 0.f;
-    y[e].z = has ? y[e].z * rstd * w.z + b.z : 0.f;
-    y[e].w = has ? y[e].w * rstd * w.w + b.w : 0.f;
-  }
-}
-
-// the split operands of output rows 32 t .. + 31 of a weight matrix with K = C inputs; lane_src: whose packed
-// operand this lane takes (its own, or rowperm16's to deal the rows so that a lane ends with 16 consecutive ones)
-template <int C, int TERMS>
-__device__ __forceinline__ void load_unit(const WeightX3& W, int t, int lane_src, u32x4_t (&w)[C / 16][TERMS]) {
-  const u32x4_t* src = reinterpret_cast<const u32x4_t*>(W.h) + (size_t)t * (C / 16) * 64 + lane_src;
-#pragma unroll
-  for (int s = 0; s < C / 16; ++s)
-#pragma unroll
-    for (int pl = 0; pl < TERMS; ++pl) w[s][pl] = src[pl * (W.plane / 8) + 64 * s];
-}
-
-// one k-step: six products, smallest terms first.  W_ROWS: the outputs are the MFMA rows, otherwise the positions
-template <bool W_ROWS>
-__device__ __forceinline__ f32x16_t step6(u32x4_t w_h, u32x4_t w_m, u32x4_t w_l, const u32x4_t (&x)[3], f32x16_t acc) {
-  if (W_ROWS) {
-    acc = mfma_32x32x16(w_l, x[0], acc);
-    acc = mfma_32x32x16(w_h, x[2], acc);
-    acc = mfma_32x32x16(w_m, x[1], acc);
-    acc = mfma_32x32x16(w_m, x[0], acc);
-    acc = mfma_32x32x16(w_h, x[1], acc);
-    return mfma_32x32x16(w_h, x[0], acc);
-  }
-  acc = mfma_32x32x16(x[0], w_l, acc);
-  acc = mfma_32x32x16(x[2], w_h, acc);
-  acc = mfma_32x32x16(x[1], w_m, acc);
-  acc = mfma_32x32x16(x[0], w_m, acc);
-  acc = mfma_32x32x16(x[1], w_h, acc);
-  return mfma_32x32x16(x[0], w_h, acc);
-}
-template <int C, bool W_ROWS>
-__device__ __forceinline__ f32x16_t unit_product(const PassTile<C>& t, const u32x4_t (&w)[C / 16][3]) {
-  f32x16_t acc = zero16();
-  const Lane at = lane_here();
-#pragma unroll
-  for (int s = 0; s < C / 16; ++s) {
-    const u32x4_t* x = t.s + PassTile<C>::slot(at.l32, 2 * s + at.lh);
-    const u32x4_t op[3] = {x[0], x[PassTile<C>::PLANE], x[2 * PassTile<C>::PLANE]};
-    acc = step6<W_ROWS>(w[s][0], w[s][1], w[s][2], op, acc);
-  }
-  return acc;
-}
+using namespace pass_f32;
 
 // the value of the lane with the lowest bit flipped (quad_perm [1,0,3,2])
 __device__ __forceinline__ uint32_t swap_adjacent(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);
-}
-
-// logical number of a work-group: consecutive numbers run on one XCD where the grid deals evenly
-__device__ __forceinline__ int grid_slot() {
-  return gridDim.x % 8 == 0 ? xcd_logical_block(blockIdx.x, gridDim.x / 8) : blockIdx.x;
 }
 
 // ---- triangle multiplication, input pass: a, b = mask * sigmoid(LN(z) Wg^T) * (LN(z) Wp^T) ------------------
@@ -266,8 +125,9 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
     for (int s = 0; s < KS; ++s) {
       const u32x4_t* x = xn.s + Tile::slot(at.l32, 2 * s + at.lh);
       const u32x4_t op[3] = {x[0], x[Tile::PLANE], x[2 * Tile::PLANE]};
-      ag = step6<false>(wg[s][0], wg[s][1], TL ? wl[64 * s] : wg[s][GTERMS - 1], op, ag);
-      ap = step6<false>(wp[s][0], wp[s][1], wp[s][2], op, ap);
+      const u32x4_t g[3] = {wg[s][0], wg[s][1], TL ? wl[64 * s] : wg[s][GTERMS - 1]};
+      ag = step6<false>(g, op, ag);
+      ap = step6<false>(wp[s], op, ap);
     }
     __syncthreads();  // everybody has read it
     // channels in the lanes, positions in the registers: registers 8 st .. + 7 are the k-values 16 st + 8 (e >> 2)
@@ -357,26 +217,12 @@ struct OutWeights {
     for (int s = 0; s < KS; ++s) {
       const u32x4_t* x = t.s + PassTile<C>::slot(at.l32, 2 * s + at.lh);
       const u32x4_t op[3] = {x[0], x[PassTile<C>::PLANE], x[2 * PassTile<C>::PLANE]};
-      acc = step6<true>(g[s][0], g[s][1], TL ? wl[64 * s] : g[s][GTERMS - 1], op, acc);
+      const u32x4_t w[3] = {g[s][0], g[s][1], TL ? wl[64 * s] : g[s][GTERMS - 1]};
+      acc = step6<true>(w, op, acc);
     }
     return acc;
   }
 };
-// out row (16 channels from op on) = [residual +] v * g
-__device__ __forceinline__ void store_row16(const float* zp, float* op, const f32x16_t& v, bool add_residual) {
-  float4 z[4];
-  if (add_residual) {
-#pragma unroll
-    for (int a = 0; a < 4; ++a) z[a] = *reinterpret_cast<const float4*>(zp + 4 * a);
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    float4 r = make_float4(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);
-    if (add_residual) r.x = z[a].x + r.x, r.y = z[a].y + r.y, r.z = z[a].z + r.z, r.w = z[a].w + r.w;
-    *reinterpret_cast<float4*>(op + 4 * a) = r;
-  }
-}
-
 // ---- triangle multiplication, output pass: out = [z +] (LN(x) Wz^T) * sigmoid(LN(z) Wg^T)
 // x is channel-major: thread (position tid % 32, group tid / 32) holds 16 channels of a position; the statistics are
 // combined from the groups' means and squared deviations (one exchange).
@@ -550,7 +396,7 @@ __global__ __launch_bounds__(6 * C) void triattn_proj_pass(TriattnF32 p, int pan
       const u32x4_t op[3] = {nxt[0], nxt[1], nxt[2]};
       if (s + 1 < KS) read(s + 1);
       __builtin_amdgcn_sched_barrier(0);
-      acc = step6<decltype(w_rows)::value>(w[s][0], w[s][1], w[s][2], op, acc);
+      acc = step6<decltype(w_rows)::value>(w[s], op, acc);
       __builtin_amdgcn_sched_barrier(0);
     }
     return acc;
@@ -713,31 +559,6 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
       store_row16(p.x + off, p.out + off, acc, p.add_residual);
     }
   }
-}
-
-bool rows_aligned(const float* p, const PairView& v) {
-  return (reinterpret_cast<uintptr_t>(p) & 15u) == 0 && ((v.stride_b | v.stride_r | v.stride_k) & 3) == 0;
-}
-
-// persistent grid: what fits the device at once, at most one work-group per tile
-template <auto Kern>
-hipError_t resident_grid(int threads, size_t lds, long tiles, unsigned* grid) {
-  static int cache[kMaxDevices];
-  int fit = 0;
-  hipError_t e = allow_dynamic_lds<Kern>(lds);
-  if (e != hipSuccess) return e;
-  e = per_device(
-      cache,
-      [&](int dev, int* v) {
-        int cus = 0, per_cu = 0;
-        hipError_t s = cu_count(dev, &cus);
-        if (s == hipSuccess) s = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, Kern, threads, lds);
-        *v = cus * (per_cu > 0 ? per_cu : 1);
-        return s;
-      },
-      &fit);
-  *grid = (unsigned)(tiles < fit ? tiles : fit);
-  return e;
 }
 
 template <int C>

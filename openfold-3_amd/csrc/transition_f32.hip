@@ -1,0 +1,276 @@
+// fp32 pair transition (transition.py:225-271, activations.py:33-61) at 64 and 128 channels with a hidden width in
+// multiples of 128, products on the bf16 matrix instructions with operands split into three bf16 terms:
+//     out = [x +] ((silu(LN(x) Wa^T) * (LN(x) Wb^T)) Wout^T) * mask
+// pair_f32.hip has the kernels for every other shape.
+//
+// 36 flops per channel and hidden channel in bf16 products: 1.4 Tflop for N = 768 at n = 4, 730 us of the matrix
+// pipes at the rate they sustain.  The split weights (590 KB at C = 128, n = 4) do not fit a CU and stream from L2.
+// One wave per tile of 32 hidden channels and all of the tile's positions: a work-group of eight waves takes the
+// hidden dimension in slices of 32 S channels (S = 8, or 4 with a wave per position tile), so that an operand of Wa
+// and Wb is read once for 64 positions and a slice of 256 hidden channels costs two barriers, against 32 positions
+// and slices of 128 in pair_f32.hip's kernel.  The operands of a k-step are requested one to four steps ahead, those of
+// the other product before the barrier between them.  Below two tiles of 64 positions per CU, tiles of 32 positions (two
+// waves then share the sum of the second product).
+#include "of3_pass_f32.h"
+
+namespace of3 {
+
+namespace {
+
+using namespace pass_f32;
+
+struct TransitionPass {
+  const float *x, *mask;
+  PairView xv, mv;
+  const float *ln_w, *ln_b;
+  WeightX3 s_a, s_b, s_out;
+  float* out;
+  int R, L;     // rows per batch element, positions per row
+  int panels;   // 32-position panels per row
+  int total;    // panels in all
+  int HID, add_residual;
+};
+
+template <int C, int S, int NPT>
+constexpr size_t transition_lds() {
+  return (size_t)NPT * (PassTile<C>::SLOTS + PassTile<32 * S>::SLOTS) * 16 + 2 * C * sizeof(float);
+}
+
+template <int C, int S, int NPT>
+__global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
+  static_assert(S == 8 || (S == 4 && NPT == 2), "eight waves share the hidden tiles of a slice");
+  typedef PassTile<C> XTile;
+  typedef PassTile<32 * S> HTile;
+  constexpr int NW = 8, KS = C / 16, OT = C / 32;
+  constexpr int XT = S == 8 ? NPT : 1;             // position tiles of a wave in the first product
+  constexpr int KSPLIT = NW / (OT * NPT);          // waves sharing an output tile's sum in the second
+  constexpr int OSTEPS = 2 * S / KSPLIT;           // its k-steps per slice and wave
+  // steps that an operand is requested ahead: an L2 read takes about as long as 24 MFMAs of two waves per SIMD
+  constexpr int DA = XT == 1 ? 2 : 1, DO = 4;
+  static_assert(OSTEPS >= DO && KS >= DA, "");
+  extern __shared__ u32x4_t lds[];
+  u32x4_t* const hid = lds + NPT * XTile::SLOTS;
+  float* ln = reinterpret_cast<float*>(hid + NPT * HTile::SLOTS);  // [2][C]
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ht = S == 8 ? wave : wave & 3, pt_a = S == 8 ? 0 : wave >> 2;
+  const int ot = wave % OT, pt_b = (wave / OT) % NPT, kh = wave / (OT * NPT);
+  const int L = p.L, slices = p.HID / (32 * S);
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c], ln[C + c] = p.ln_b[c];
+
+  const int lane0 = tid & 63, src_lane = rowperm16(lane0 & 31) + (lane0 & 32);  // outputs dealt by rowperm16
+  const u32x4_t* wa = reinterpret_cast<const u32x4_t*>(p.s_a.h) + src_lane;
+  const u32x4_t* wb = reinterpret_cast<const u32x4_t*>(p.s_b.h) + src_lane;
+  const u32x4_t* wo = reinterpret_cast<const u32x4_t*>(p.s_out.h) + (size_t)(ot * (p.HID / 16) + kh * OSTEPS) * 64 + src_lane;
+  const long pa = p.s_a.plane / 8, po = p.s_out.plane / 8;
+
+  auto row_of = [&](int pn, int& j0) {  // element offsets of the panel's row in x and in the mask
+    const int r = pn / p.panels;
+    j0 = 32 * (pn - r * p.panels);
+    return r;
+  };
+  RowRegs<C> raw[NPT];
+  auto load_tile = [&](int tile) {
+    const Lane here = lane_here();
+#pragma unroll
+    for (int t = 0; t < NPT; ++t) {
+      int pn = NPT * tile + t, j0;
+      pn = pn < p.total ? pn : p.total - 1;
+      const int r = row_of(pn, j0), b = r / p.R, i = r - b * p.R;
+      int j = j0 + 4 * wave + here.lg;
+      j = j < L ? j : L - 1;
+      load_row<C>(p.x + b * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j * p.xv.stride_k, here.li, raw[t]);
+    }
+  };
+  u32x4_t na[DA][3], nb[DA][3], no[DO][3];  // operands of the next steps
+  auto fetch_ab = [&](int slice, int s) {
+    const size_t at = ((size_t)(slice * S + ht) * KS + s) * 64;
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) na[s % DA][pl] = wa[pl * pa + at], nb[s % DA][pl] = wb[pl * pa + at];
+  };
+  auto fetch_o = [&](int slice, int s) {
+    const size_t at = (size_t)(slice * 2 * S + s) * 64;
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) no[s % DO][pl] = wo[pl * po + at];
+  };
+
+  const int tiles = (p.total + NPT - 1) / NPT;
+  int tile = grid_slot();
+  if (tile < tiles) load_tile(tile);
+  __syncthreads();
+  for (; tile < tiles; tile += gridDim.x) {
+    {
+      const Lane here = lane_here();
+#pragma unroll
+      for (int t = 0; t < NPT; ++t) {
+        int j0;
+        const int pn = NPT * tile + t;
+        row_of(pn, j0);
+        const int pos = 4 * wave + here.lg;
+        float4 y[C / 64];
+        norm_row<C>(raw[t], pn < p.total && j0 + pos < L, ln, here.li, y);
+        const XTile xn = {lds + t * XTile::SLOTS};
+#pragma unroll
+        for (int e = 0; e < C / 64; ++e) xn.store4(pos, here.li + 16 * e, y[e]);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < DA; ++s) fetch_ab(0, s);
+    f32x16_t oacc = zero16();
+    for (int slice = 0; slice < slices; ++slice) {
+      __syncthreads();  // the activations (first slice), or: everybody has read the slice before
+      f32x16_t a[XT], b[XT];
+#pragma unroll
+      for (int t = 0; t < XT; ++t) a[t] = b[t] = zero16();
+      {
+        const Lane at = lane_here();
+        u32x4_t nx[XT][3];
+        auto read_x = [&](int s) {
+#pragma unroll
+          for (int t = 0; t < XT; ++t) {
+            const u32x4_t* x = lds + (pt_a + t) * XTile::SLOTS + XTile::slot(at.l32, 2 * s + at.lh);
+            nx[t][0] = x[0], nx[t][1] = x[XTile::PLANE], nx[t][2] = x[2 * XTile::PLANE];
+          }
+        };
+        read_x(0);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          u32x4_t x[XT][3], ca[3], cb[3];
+#pragma unroll
+          for (int pl = 0; pl < 3; ++pl) {
+            ca[pl] = na[s % DA][pl], cb[pl] = nb[s % DA][pl];
+#pragma unroll
+            for (int t = 0; t < XT; ++t) x[t][pl] = nx[t][pl];
+          }
+          if (s + 1 < KS) read_x(s + 1);
+          if (s + DA < KS) fetch_ab(slice, s + DA);
+          if (s + 1 == KS) {
+#pragma unroll
+            for (int q = 0; q < DO; ++q) fetch_o(slice, q);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int t = 0; t < XT; ++t) {
+            a[t] = step6<true>(ca, x[t], a[t]);
+            b[t] = step6<true>(cb, x[t], b[t]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      {
+        const Lane at = lane_here();
+#pragma unroll
+        for (int t = 0; t < XT; ++t) {
+          const HTile h = {hid + (pt_a + t) * HTile::SLOTS};
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {  // lane (position, half lh): hidden channels 32 ht + 16 lh + 8 hf + e
+            float y[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = (a[t][8 * hf + e] * sigmoid_hw_f32(a[t][8 * hf + e])) * b[t][8 * hf + e];
+            h.store8(at.l32, 4 * ht + 2 * at.lh + hf, y);
+          }
+        }
+      }
+      __syncthreads();  // the slice's hidden activations are complete
+      const bool last = slice + 1 == slices;
+      {
+        const Lane at = lane_here();
+        const u32x4_t* ht0 = hid + pt_b * HTile::SLOTS;
+        u32x4_t nx[3];
+        auto read_h = [&](int s) {
+          const u32x4_t* x = ht0 + HTile::slot(at.l32, 2 * (kh * OSTEPS + s) + at.lh);
+          nx[0] = x[0], nx[1] = x[HTile::PLANE], nx[2] = x[2 * HTile::PLANE];
+        };
+        read_h(0);
+#pragma unroll
+        for (int s = 0; s < OSTEPS; ++s) {
+          const u32x4_t x[3] = {nx[0], nx[1], nx[2]}, co[3] = {no[s % DO][0], no[s % DO][1], no[s % DO][2]};
+          if (s + 1 < OSTEPS) read_h(s + 1);
+          if (s + DO < OSTEPS) fetch_o(slice, s + DO);
+          if (s + DO == OSTEPS) {  // after the last weights: loads return in order
+            if (last) load_tile(tile + (int)gridDim.x < tiles ? tile + gridDim.x : tile);
+            else
+#pragma unroll
+              for (int q = 0; q < DA; ++q) fetch_ab(slice + 1, q);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          oacc = step6<true>(co, x, oacc);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    const Lane at = lane_here();
+    if (KSPLIT > 1) {  // the waves of an output tile add up through the hidden tile's memory
+      __syncthreads();
+      float* red = reinterpret_cast<float*>(hid) + (wave % (OT * NPT)) * 1024 + at.l32 + 32 * at.lh;
+      if (kh > 0) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) red[(kh - 1) * (OT * NPT * 1024) + 64 * v] = oacc[v];
+      }
+      __syncthreads();
+      if (kh > 0) continue;
+#pragma unroll
+      for (int q = 0; q < KSPLIT - 1; ++q)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) oacc[v] += red[q * (OT * NPT * 1024) + 64 * v];
+    }
+    int j0;
+    const int pn = NPT * tile + pt_b;
+    const int r = row_of(pn, j0), bb = r / p.R, i = r - bb * p.R, j = j0 + at.l32;
+    if (pn < p.total && j < L) {
+      const int64_t off = bb * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j * p.xv.stride_k + 32 * ot + 16 * at.lh;
+      if (p.mask) {
+        const float m = p.mask[bb * p.mv.stride_b + i * p.mv.stride_r + (int64_t)j * p.mv.stride_k];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) oacc[v] *= m;
+      }
+      store_row16(p.x + off, p.out + off, oacc, p.add_residual);
+    }
+  }
+}
+
+template <int C, int S, int NPT>
+hipError_t launch(const TransitionPass& p, hipStream_t stream) {
+  constexpr size_t lds = transition_lds<C, S, NPT>();
+  unsigned grid = 0;
+  hipError_t e = resident_grid<transition_pass<C, S, NPT>>(512, lds, (p.total + NPT - 1) / NPT, &grid);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((transition_pass<C, S, NPT>), dim3(grid), dim3(512), lds, stream, p);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+bool transition_pass_serves(const TransitionF32Args& a) {
+  return (a.C == 64 || a.C == 128) && a.HID % 128 == 0 && rows_aligned(a.x, a.x_view) && rows_aligned(a.out, a.x_view) &&
+         (long)a.B * a.N * ((a.N + 31) / 32) <= 0x3fffffffL;
+}
+
+hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, const WeightX3& s_b, const WeightX3& s_out,
+                               hipStream_t stream) {
+  TransitionPass p;
+  p.x = a.x;
+  p.mask = a.mask;
+  p.xv = a.x_view;
+  p.mv = a.mask_view;
+  p.ln_w = a.ln_w;
+  p.ln_b = a.ln_b;
+  p.s_a = s_a;
+  p.s_b = s_b;
+  p.s_out = s_out;
+  p.out = a.out;
+  // a tensor (and mask) whose rows follow one another without gaps is one row of N * N positions
+  const bool flat = a.x_view.stride_r == a.N * a.x_view.stride_k && (!a.mask || a.mask_view.stride_r == a.N * a.mask_view.stride_k);
+  p.R = flat ? 1 : a.N;
+  p.L = flat ? a.N * a.N : a.N;
+  p.panels = (p.L + 31) / 32;
+  p.total = a.B * p.R * p.panels;
+  p.HID = a.HID;
+  p.add_residual = a.add_residual;
+  const bool large = p.total >= 4 * 256;  // two tiles of 64 positions for every CU
+  if (a.HID % 256 != 0) return a.C == 128 ? launch<128, 4, 2>(p, stream) : launch<64, 4, 2>(p, stream);
+  if (a.C == 128) return large ? launch<128, 8, 2>(p, stream) : launch<128, 8, 1>(p, stream);
+  return large ? launch<64, 8, 2>(p, stream) : launch<64, 8, 1>(p, stream);
+}
+
+}  // namespace of3

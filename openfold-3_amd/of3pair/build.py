@@ -36,6 +36,9 @@ SOURCES = [
     "single_transition.hip",
     "pair_f32.hip",
     "pair_pass_f32.hip",
+    "pair_proj_f32.hip",
+    "transition_f32.hip",
+    "weight_split.hip",
     "single_f32.hip",
     "single_x3_f32.hip",
 ]
