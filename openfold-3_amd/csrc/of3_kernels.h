@@ -26,6 +26,7 @@ struct TrimulProjArgs {
   const bf16_t *w_ap, *w_ag, *w_bp, *w_bg;    // [CH][C]
   bf16_t *a, *b;                              // [B][CH][Np/32][Np][32]  (k-panels)
   int B, N, Np;
+  int packed = 0;                             // the weight matrices are in MFMA operand order (weight_pack.hip)
 };
 hipError_t trimul_proj_launch(const TrimulProjArgs& args, int C, int CH, hipStream_t stream);
 
@@ -46,6 +47,7 @@ struct TrimulOutArgs {
   const bf16_t *w_z;                  // [C][CH]
   int B, N, Np;
   int add_residual;
+  int packed = 0;
 };
 hipError_t trimul_out_launch(const TrimulOutArgs& args, int C, int CH, hipStream_t stream);
 
@@ -62,6 +64,7 @@ struct TriattnProjArgs {
   float *mbias;                       // [B][N][Jp]      (log2 e * inf * (mask-1); -inf for j >= N)
   int B, N, Jp, H;
   float inf;
+  int packed = 0;                     // w_q, w_k, w_v in MFMA operand order
 };
 hipError_t triattn_proj_launch(const TriattnProjArgs& args, int C, int D, hipStream_t stream);
 
@@ -83,8 +86,26 @@ struct TriattnOutArgs {
   const bf16_t *w_o;          // [C][H*D]
   int B, N;
   int add_residual;
+  int packed = 0;
 };
 hipError_t triattn_out_launch(const TriattnOutArgs& args, int C, int HD, hipStream_t stream);
+
+// the same four passes on tiles of 32 positions (pair_pass_bf16.hip), called by the launchers above for short sequences
+hipError_t trimul_proj_panels_launch(const TrimulProjArgs& args, int C, hipStream_t stream);
+hipError_t trimul_out_panels_launch(const TrimulOutArgs& args, int C, hipStream_t stream);
+hipError_t triattn_proj_panels_launch(const TriattnProjArgs& args, int C, hipStream_t stream);
+hipError_t triattn_out_panels_launch(const TriattnOutArgs& args, int C, hipStream_t stream);
+
+// Copies of bf16 weight matrices in MFMA operand order (weight_pack.hip): rows and K multiples of 32 and 16
+struct PackJobs {
+  static constexpr int kMax = 22;  // a pair block: 2 x 6 + 2 x 5
+  const bf16_t* src[kMax];
+  bf16_t* dst[kMax];
+  int K[kMax];
+  int first[kMax + 1];  // first item (8 values) of each matrix; first[n] = all items
+  int n;
+};
+hipError_t pack_weights_launch(const PackJobs& jobs, hipStream_t stream);
 
 struct TransitionArgs {
   const bf16_t* x;    // pair tensor, x_view addressing

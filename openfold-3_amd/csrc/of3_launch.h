@@ -35,6 +35,16 @@ inline hipError_t cu_count(int dev, int* n) {
   return hipDeviceGetAttribute(n, hipDeviceAttributeMultiprocessorCount, dev);
 }
 
+// Whether a bf16 position-wise pass over B tensors of N x N positions runs on 32-position tiles: up to `per_cu`
+// such tiles per CU.
+inline hipError_t small_pass(int B, int N, int per_cu, bool* small) {
+  static int cache[kMaxDevices];
+  int cus = 0;
+  hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  *small = (long)B * N * ((N + 31) / 32) <= (long)per_cu * cus;
+  return e;
+}
+
 // work-groups of `threads` threads (no dynamic LDS) that fit the device at once
 template <typename Kernel>
 inline hipError_t resident_blocks(Kernel kern, int threads, int dev, int* out) {

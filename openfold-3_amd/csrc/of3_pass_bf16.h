@@ -1,0 +1,125 @@
+// Building blocks of the bf16 position-wise passes: weight operands (row-major, or packed in operand order by
+// weight_pack.hip), LayerNorm lanes, LDS tiles of one 32-position panel.
+#pragma once
+
+#include "of3_device.h"
+
+namespace of3 {
+namespace pass_bf16 {
+
+// The lane number, opaque to the compiler: what is derived from it inside a tile loop is recomputed there (a few
+// instructions) instead of being hoisted into registers that the weights occupy.
+struct Lane {
+  int l32, lh;
+};
+__device__ __forceinline__ Lane lane_here() {
+  int lane = threadIdx.x & 63;
+  __asm__ volatile("" : "+v"(lane));
+  return {lane & 31, lane >> 5};
+}
+
+// MFMA operands of output rows 32 t .. + 31 of a matrix with K inputs: this lane takes row r of the tile, k-half lh.
+// packed: the 16 bytes of lane l for k-step s of tile t sit at ((t * K / 16 + s) * 64 + l) * 16, one contiguous
+// kilobyte per wave instruction; row-major the same operand touches 32 cache lines, and reading a pass's 64 to 128 KB of
+// weights that way takes 2 us longer (8.6 against 11.1 us for trimul_proj at N = 40, 15.8 against 18.1 at N = 200).
+struct UnitSource {
+  const bf16_t* base;
+  int step;  // elements between k-steps
+};
+template <int K>
+__device__ __forceinline__ UnitSource unit_source(const bf16_t* W, int t, int r, int lh, int packed) {
+  UnitSource u;
+  u.base = packed ? W + ((t * (K / 16)) * 64 + r + 32 * lh) * 8 : W + (32 * t + r) * K + 8 * lh;
+  u.step = packed ? 512 : 16;
+  return u;
+}
+template <int K>
+__device__ __forceinline__ void load_unit(const bf16_t* W, int t, int r, int lh, int packed, u32x4_t (&w)[K / 16]) {
+  const UnitSource u = unit_source<K>(W, t, r, lh, packed);
+#pragma unroll
+  for (int s = 0; s < K / 16; ++s) w[s] = *reinterpret_cast<const u32x4_t*>(u.base + s * u.step);
+}
+
+// A lane's part in the LayerNorm of rows of C channels: 16 bytes of one position, C / 8 lanes per position
+template <int C>
+struct LnLane {
+  static constexpr int NCH = C / 8, PPI = 64 / NCH;  // positions per wave instruction
+  u32x4_t w, b;
+  // chunk and position (inside the PPI of an instruction) of this lane, recomputed where they are used
+  __device__ __forceinline__ static int chunk() { return opaque_lane() % NCH; }
+  __device__ __forceinline__ static int pos() { return opaque_lane() / NCH; }
+  __device__ __forceinline__ static int opaque_lane() {
+    int lane = threadIdx.x & 63;
+    __asm__ volatile("" : "+v"(lane));
+    return lane;
+  }
+  // SCALED: the result feeds a gate only, weight and bias carry the factor -log2(e) of its base-2 exponential
+  template <bool SCALED>
+  __device__ __forceinline__ u32x4_t normalised(u32x4_t raw) const {
+    u32x4_t tw = w, tb = b;
+    __asm__ volatile("" : "+v"(tw), "+v"(tb));  // unpacked here rather than held as 16 floats
+    float lw[8], lb[8];
+    unpack8(tw, lw);
+    unpack8(tb, lb);
+    if (SCALED) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        lw[e] *= -kLog2e, lb[e] *= -kLog2e;
+        __asm__("" : "+v"(lb[e]));  // rounded here: the fused multiply-add is the one with the weight, as in the 128-position passes
+      }
+    }
+    return layer_norm_chunk<C>(raw, lw, lb);
+  }
+};
+template <int C>
+__device__ __forceinline__ LnLane<C> ln_lane(const bf16_t* w, const bf16_t* b, int lane) {
+  const int chunk = lane % LnLane<C>::NCH;
+  LnLane<C> l;
+  l.w = *reinterpret_cast<const u32x4_t*>(w + 8 * chunk);
+  l.b = *reinterpret_cast<const u32x4_t*>(b + 8 * chunk);
+  return l;
+}
+
+// LDS tile of 32 positions x C channels, 16-byte chunks.  PERMUTED: operand readers take the positions in rowperm16
+// order ({x .. x+3, x+16 .. x+19} per 8 lanes) as well as in natural order, otherwise in natural order only.
+template <int C, bool PERMUTED>
+struct PanelTile {
+  static constexpr int NCH = C / 8, SLOTS = 32 * NCH;
+  u32x4_t* s;
+  __device__ __forceinline__ static int slot(int pos, int chunk) {
+    // 128 channels: a position is one 256-byte bank window; 64: half of one
+    int key;
+    if (NCH == 16) key = PERMUTED ? (pos & 7) | ((pos ^ (pos >> 1)) & 8) : pos & 15;
+    else key = PERMUTED ? ((pos >> 1) & 3) | (((pos >> 2) ^ (pos >> 1)) & 4) : (pos >> 1) & 7;
+    return pos * NCH + (chunk ^ key);
+  }
+};
+
+// 16 consecutive bf16 values
+__device__ __forceinline__ void store16(bf16_t* dst, const float (&x)[16]) {
+  u32x4_t o0, o1;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    o0[q] = pack_bf16(x[2 * q], x[2 * q + 1]);
+    o1[q] = pack_bf16(x[8 + 2 * q], x[8 + 2 * q + 1]);
+  }
+  *reinterpret_cast<u32x4_t*>(dst) = o0;
+  *reinterpret_cast<u32x4_t*>(dst + 8) = o1;
+}
+__device__ __forceinline__ void add16(const bf16_t* src, float (&x)[16]) {
+  float r[8];
+  unpack8(*reinterpret_cast<const u32x4_t*>(src), r);
+#pragma unroll
+  for (int v = 0; v < 8; ++v) x[v] += r[v];
+  unpack8(*reinterpret_cast<const u32x4_t*>(src + 8), r);
+#pragma unroll
+  for (int v = 0; v < 8; ++v) x[8 + v] += r[v];
+}
+
+// logical number of a work-group: consecutive numbers run on one XCD where the grid deals evenly
+__device__ __forceinline__ int grid_slot() {
+  return gridDim.x % 8 == 0 ? xcd_logical_block(blockIdx.x, gridDim.x / 8) : blockIdx.x;
+}
+
+}  // namespace pass_bf16
+}  // namespace of3

@@ -191,10 +191,10 @@ int64_t of3_trimul_workspace_bytes_for(int dtype, int64_t B, int64_t N, int64_t 
   return f32_trimul_ab_bytes(B, N, CH) + align256(B * CH * N * N * 4) + align256((int64_t)of3::trimul_wsplit_bytes(C, CH));
 }
 
-int of3_trimul_proj(const void* z, const int64_t z_strides[3], const float* mask, const int64_t mask_strides[3],
-                    const void* ln_in_w, const void* ln_in_b, const void* w_a_p, const void* w_a_g,
-                    const void* w_b_p, const void* w_b_g, void* a, void* b, int64_t B, int64_t N, int64_t C,
-                    int64_t CH, int outgoing, void* stream) {
+static int trimul_proj(int packed, const void* z, const int64_t z_strides[3], const float* mask,
+                       const int64_t mask_strides[3], const void* ln_in_w, const void* ln_in_b, const void* w_a_p,
+                       const void* w_a_g, const void* w_b_p, const void* w_b_g, void* a, void* b, int64_t B, int64_t N,
+                       int64_t C, int64_t CH, int outgoing, void* stream) {
   if (!trimul_dims_ok(B, N, C, CH) || !strides_ok(z_strides) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
   const void* ptrs[] = {z, ln_in_w, ln_in_b, w_a_p, w_a_g, w_b_p, w_b_g, a, b};
   for (const void* p : ptrs)
@@ -215,8 +215,17 @@ int of3_trimul_proj(const void* z, const int64_t z_strides[3], const float* mask
   args.B = (int)B;
   args.N = (int)N;
   args.Np = (int)padded(N);
+  args.packed = packed;
   hipError_t e = of3::trimul_proj_launch(args, (int)C, (int)CH, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
+}
+
+int of3_trimul_proj(const void* z, const int64_t z_strides[3], const float* mask, const int64_t mask_strides[3],
+                    const void* ln_in_w, const void* ln_in_b, const void* w_a_p, const void* w_a_g,
+                    const void* w_b_p, const void* w_b_g, void* a, void* b, int64_t B, int64_t N, int64_t C,
+                    int64_t CH, int outgoing, void* stream) {
+  return trimul_proj(0, z, z_strides, mask, mask_strides, ln_in_w, ln_in_b, w_a_p, w_a_g, w_b_p, w_b_g, a, b, B, N,
+                     C, CH, outgoing, stream);
 }
 
 int of3_trimul_contract(const void* a, const void* b, void* x, int64_t B, int64_t N, int64_t CH, int variant,
@@ -230,9 +239,10 @@ int of3_trimul_contract(const void* a, const void* b, void* x, int64_t B, int64_
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
-int of3_trimul_out(const void* x, const void* z, const int64_t z_strides[3], void* out, const void* ln_in_w,
-                   const void* ln_in_b, const void* ln_out_w, const void* ln_out_b, const void* w_g,
-                   const void* w_z, int64_t B, int64_t N, int64_t C, int64_t CH, int add_residual, void* stream) {
+static int trimul_out(int packed, const void* x, const void* z, const int64_t z_strides[3], void* out,
+                      const void* ln_in_w, const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
+                      const void* w_g, const void* w_z, int64_t B, int64_t N, int64_t C, int64_t CH, int add_residual,
+                      void* stream) {
   if (!trimul_dims_ok(B, N, C, CH) || !strides_ok(z_strides)) return OF3_EINVAL;
   const void* ptrs[] = {x, z, out, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_g, w_z};
   for (const void* p : ptrs)
@@ -252,12 +262,21 @@ int of3_trimul_out(const void* x, const void* z, const int64_t z_strides[3], voi
   args.N = (int)N;
   args.Np = (int)padded(N);
   args.add_residual = add_residual ? 1 : 0;
+  args.packed = packed;
   hipError_t e = of3::trimul_out_launch(args, (int)C, (int)CH, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
-// presplit: the fp32 weights as a block's call has split them, or null
-static int trimul_fwd(const of3::WeightX3* presplit, const void* z, const int64_t z_strides[3], const float* mask,
+int of3_trimul_out(const void* x, const void* z, const int64_t z_strides[3], void* out, const void* ln_in_w,
+                   const void* ln_in_b, const void* ln_out_w, const void* ln_out_b, const void* w_g,
+                   const void* w_z, int64_t B, int64_t N, int64_t C, int64_t CH, int add_residual, void* stream) {
+  return trimul_out(0, x, z, z_strides, out, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_g, w_z, B, N, C, CH,
+                    add_residual, stream);
+}
+
+// presplit: the fp32 weights as a block's call has split them, or null; packed: the bf16 weight matrices are copies in
+// MFMA operand order
+static int trimul_fwd(const of3::WeightX3* presplit, int packed, const void* z, const int64_t z_strides[3], const float* mask,
                    const int64_t mask_strides[3], const void* ln_in_w, const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
                    const void* w_a_p, const void* w_a_g, const void* w_b_p, const void* w_b_g, const void* w_g,
                    const void* w_z, void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int outgoing,
@@ -314,12 +333,12 @@ static int trimul_fwd(const of3::WeightX3* presplit, const void* z, const int64_
   void* a = ws;
   void* b = ws + part;
   void* x = ws + 2 * part;
-  int st = of3_trimul_proj(z, z_strides, mask, mask_strides, ln_in_w, ln_in_b, w_a_p, w_a_g, w_b_p, w_b_g, a, b, B, N,
+  int st = trimul_proj(packed, z, z_strides, mask, mask_strides, ln_in_w, ln_in_b, w_a_p, w_a_g, w_b_p, w_b_g, a, b, B, N,
                            C, CH, outgoing, stream);
   if (st != OF3_OK) return st;
   st = of3_trimul_contract(a, b, x, B, N, CH, 0, stream);
   if (st != OF3_OK) return st;
-  return of3_trimul_out(x, z, z_strides, out, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_g, w_z, B, N, C, CH,
+  return trimul_out(packed, x, z, z_strides, out, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_g, w_z, B, N, C, CH,
                         add_residual, stream);
 }
 
@@ -328,7 +347,7 @@ int of3_trimul_fwd(const void* z, const int64_t z_strides[3], const float* mask,
                    const void* w_a_p, const void* w_a_g, const void* w_b_p, const void* w_b_g, const void* w_g,
                    const void* w_z, void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int outgoing,
                    int add_residual, void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
-  return trimul_fwd(nullptr, z, z_strides, mask, mask_strides, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_a_p, w_a_g, w_b_p,
+  return trimul_fwd(nullptr, 0, z, z_strides, mask, mask_strides, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_a_p, w_a_g, w_b_p,
                     w_b_g, w_g, w_z, out, B, N, C, CH, outgoing, add_residual, workspace, workspace_bytes, dtype, stream);
 }
 
@@ -366,10 +385,10 @@ int64_t of3_triattn_workspace_bytes_for(int dtype, int64_t B, int64_t N, int64_t
          align256((int64_t)of3::triattn_wsplit_bytes(C, H, D));
 }
 
-int of3_triattn_proj(const void* x, const int64_t x_strides[3], const float* mask, const int64_t mask_strides[3],
-                     const void* ln_w, const void* ln_b, const void* w_q, const void* w_k, const void* w_v,
-                     const void* w_bias, void* q, void* k, void* vt, float* tbias, float* mbias, int64_t B,
-                     int64_t N, int64_t C, int64_t H, int64_t D, float inf, void* stream) {
+static int triattn_proj(int packed, const void* x, const int64_t x_strides[3], const float* mask,
+                        const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_q,
+                        const void* w_k, const void* w_v, const void* w_bias, void* q, void* k, void* vt, float* tbias,
+                        float* mbias, int64_t B, int64_t N, int64_t C, int64_t H, int64_t D, float inf, void* stream) {
   if (!triattn_dims_ok(B, N, C, H, D) || !strides_ok(x_strides) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
   const void* ptrs[] = {x, ln_w, ln_b, w_q, w_k, w_v, w_bias, q, k, vt, tbias, mbias};
   for (const void* p : ptrs)
@@ -395,8 +414,17 @@ int of3_triattn_proj(const void* x, const int64_t x_strides[3], const float* mas
   args.Jp = (int)padded(N);
   args.H = (int)H;
   args.inf = inf;
+  args.packed = packed;
   hipError_t e = of3::triattn_proj_launch(args, (int)C, (int)D, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
+}
+
+int of3_triattn_proj(const void* x, const int64_t x_strides[3], const float* mask, const int64_t mask_strides[3],
+                     const void* ln_w, const void* ln_b, const void* w_q, const void* w_k, const void* w_v,
+                     const void* w_bias, void* q, void* k, void* vt, float* tbias, float* mbias, int64_t B,
+                     int64_t N, int64_t C, int64_t H, int64_t D, float inf, void* stream) {
+  return triattn_proj(0, x, x_strides, mask, mask_strides, ln_w, ln_b, w_q, w_k, w_v, w_bias, q, k, vt, tbias, mbias,
+                      B, N, C, H, D, inf, stream);
 }
 
 int of3_triattn_flash(const void* q, const void* k, const void* vt, const float* tbias, const float* mbias, void* o,
@@ -421,9 +449,9 @@ int of3_triattn_flash(const void* q, const void* k, const void* vt, const float*
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
-int of3_triattn_out(const void* o, const void* x, const int64_t x_strides[3], void* out, const void* ln_w,
-                    const void* ln_b, const void* w_g, const void* w_o, int64_t B, int64_t N, int64_t C, int64_t H,
-                    int64_t D, int add_residual, void* stream) {
+static int triattn_out(int packed, const void* o, const void* x, const int64_t x_strides[3], void* out,
+                       const void* ln_w, const void* ln_b, const void* w_g, const void* w_o, int64_t B, int64_t N,
+                       int64_t C, int64_t H, int64_t D, int add_residual, void* stream) {
   if (!triattn_dims_ok(B, N, C, H, D) || !strides_ok(x_strides)) return OF3_EINVAL;
   const void* ptrs[] = {o, x, out, ln_w, ln_b, w_g, w_o};
   for (const void* p : ptrs)
@@ -440,11 +468,18 @@ int of3_triattn_out(const void* o, const void* x, const int64_t x_strides[3], vo
   args.B = (int)B;
   args.N = (int)N;
   args.add_residual = add_residual ? 1 : 0;
+  args.packed = packed;
   hipError_t e = of3::triattn_out_launch(args, (int)C, (int)(H * D), static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
-static int triattn_fwd(const of3::WeightX3* presplit, const void* x, const int64_t x_strides[3], const float* mask,
+int of3_triattn_out(const void* o, const void* x, const int64_t x_strides[3], void* out, const void* ln_w,
+                    const void* ln_b, const void* w_g, const void* w_o, int64_t B, int64_t N, int64_t C, int64_t H,
+                    int64_t D, int add_residual, void* stream) {
+  return triattn_out(0, o, x, x_strides, out, ln_w, ln_b, w_g, w_o, B, N, C, H, D, add_residual, stream);
+}
+
+static int triattn_fwd(const of3::WeightX3* presplit, int packed, const void* x, const int64_t x_strides[3], const float* mask,
                     const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_bias, const void* w_q, const void* w_k,
                     const void* w_v, const void* w_g, const void* w_o, void* out, int64_t B, int64_t N, int64_t C,
                     int64_t H, int64_t D, float inf, int add_residual, void* workspace, int64_t workspace_bytes,
@@ -505,12 +540,12 @@ static int triattn_fwd(const of3::WeightX3* presplit, const void* x, const int64
   float* tbias = reinterpret_cast<float*>(ws + 3 * qkv);
   float* mbias = reinterpret_cast<float*>(ws + 3 * qkv + align256(B * H * N * Np * 4));
   void* o = ws + 3 * qkv + align256(B * H * N * Np * 4) + align256(B * N * Np * 4);
-  int st = of3_triattn_proj(x, x_strides, mask, mask_strides, ln_w, ln_b, w_q, w_k, w_v, w_bias, q, k, vt, tbias,
+  int st = triattn_proj(packed, x, x_strides, mask, mask_strides, ln_w, ln_b, w_q, w_k, w_v, w_bias, q, k, vt, tbias,
                             mbias, B, N, C, H, D, inf, stream);
   if (st != OF3_OK) return st;
   st = of3_triattn_flash(q, k, vt, tbias, mbias, o, B, N, H, D, stream);
   if (st != OF3_OK) return st;
-  return of3_triattn_out(o, x, x_strides, out, ln_w, ln_b, w_g, w_o, B, N, C, H, D, add_residual, stream);
+  return triattn_out(packed, o, x, x_strides, out, ln_w, ln_b, w_g, w_o, B, N, C, H, D, add_residual, stream);
 }
 
 int of3_triattn_fwd(const void* x, const int64_t x_strides[3], const float* mask, const int64_t mask_strides[3],
@@ -518,7 +553,7 @@ int of3_triattn_fwd(const void* x, const int64_t x_strides[3], const float* mask
                     const void* w_v, const void* w_g, const void* w_o, void* out, int64_t B, int64_t N, int64_t C,
                     int64_t H, int64_t D, float inf, int add_residual, void* workspace, int64_t workspace_bytes,
                     int dtype, void* stream) {
-  return triattn_fwd(nullptr, x, x_strides, mask, mask_strides, ln_w, ln_b, w_bias, w_q, w_k, w_v, w_g, w_o, out, B, N, C,
+  return triattn_fwd(nullptr, 0, x, x_strides, mask, mask_strides, ln_w, ln_b, w_bias, w_q, w_k, w_v, w_g, w_o, out, B, N, C,
                      H, D, inf, add_residual, workspace, workspace_bytes, dtype, stream);
 }
 
@@ -915,7 +950,10 @@ static int64_t pair_block_module_bytes(int dtype, int64_t B, int64_t N, int64_t 
 int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
                                        int64_t HID) {
   const int64_t need = pair_block_module_bytes(dtype, B, N, C, CH, H, D, HID);
-  return need < 0 || dtype == OF3_DTYPE_BF16 ? need : need + block_split_bytes(C, CH, H, D, HID);
+  if (need < 0) return need;
+  // fp32: the block's matrices split; bf16: the passes' matrices in operand order
+  if (dtype == OF3_DTYPE_F32) return need + block_split_bytes(C, CH, H, D, HID);
+  return need + align256(2 * 2 * (4 * CH * C + C * C + C * CH + 5 * H * D * C));
 }
 
 int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t z_strides[3], const float* mask,
@@ -977,10 +1015,44 @@ int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t 
     }
   }
 
+  // bf16: the passes' weight matrices in MFMA operand order, likewise
+  const void* packed_weights[OF3_PAIR_BLOCK_WEIGHTS];
+  const int packed = wide ? 0 : 1;
+  if (!wide) {
+    for (int i = 0; i < n_weights; ++i) packed_weights[i] = weights[i];
+    of3::PackJobs jobs;
+    jobs.n = jobs.first[0] = 0;
+    of3::bf16_t* dst = reinterpret_cast<of3::bf16_t*>(static_cast<char*>(workspace) +
+                                                      pair_block_module_bytes(dtype, B, N, C, CH, H, D, HID));
+    auto add = [&](int i, int64_t rows, int64_t K) {
+      const int n = jobs.n++;
+      jobs.src[n] = bf(weights[i]);
+      jobs.dst[n] = dst;
+      jobs.K[n] = (int)K;
+      jobs.first[n + 1] = jobs.first[n] + (int)(rows * K / 8);
+      packed_weights[i] = dst;
+      dst += rows * K;
+    };
+    for (int m = 0; m < 2; ++m) {
+      for (int i = 4; i < 8; ++i) add(10 * m + i, CH, C);
+      add(10 * m + 8, C, C);
+      add(10 * m + 9, C, CH);
+    }
+    for (int m = 0; m < 2; ++m) {
+      for (int i = 3; i < 7; ++i) add(20 + 8 * m + i, H * D, C);
+      add(20 + 8 * m + 7, C, H * D);
+    }
+    const hipError_t e = of3::pack_weights_launch(jobs, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail_hip(e);
+    w_mul = packed_weights;
+    w_att = packed_weights + 20;
+  }
+
   const void* src = z;  // the first module reads z, every later one updates out in place
   auto trimul = [&](const void* const* w, int outgoing) {
-    const int st = trimul_fwd(s_mul ? s_mul + (outgoing ? 0 : of3::kTrimulMatrices) : nullptr, src, z_strides, mask, mask_strides, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8],
-                                  w[9], out, B, N, C, CH, outgoing, 1, workspace, workspace_bytes, dtype, stream);
+    const int st = trimul_fwd(s_mul ? s_mul + (outgoing ? 0 : of3::kTrimulMatrices) : nullptr, packed, src, z_strides,
+                              mask, mask_strides, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8], w[9], out, B,
+                              N, C, CH, outgoing, 1, workspace, workspace_bytes, dtype, stream);
     src = out;
     return st;
   };
@@ -988,8 +1060,9 @@ int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t 
     const int64_t zt[3] = {z_strides[0], ending ? z_strides[2] : z_strides[1], ending ? z_strides[1] : z_strides[2]};
     int64_t mt[3] = {0, 0, 0};
     if (mask) mt[0] = mask_strides[0], mt[1] = mask_strides[ending ? 2 : 1], mt[2] = mask_strides[ending ? 1 : 2];
-    const int st = triattn_fwd(s_att ? s_att + (ending ? of3::kTriattnMatrices : 0) : nullptr, src, zt, mask, mt, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], out, B, N, C, H, D,
-                                   inf, 1, workspace, workspace_bytes, dtype, stream);
+    const int st = triattn_fwd(s_att ? s_att + (ending ? of3::kTriattnMatrices : 0) : nullptr, packed, src, zt, mask,
+                               mt, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], out, B, N, C, H, D, inf, 1,
+                               workspace, workspace_bytes, dtype, stream);
     src = out;
     return st;
   };

@@ -13,6 +13,7 @@
 #include "of3_device.h"
 #include "of3_kernels.h"
 #include "of3_launch.h"
+#include "of3_pass_bf16.h"
 
 namespace of3 {
 
@@ -53,12 +54,8 @@ __global__ __launch_bounds__(512) void triattn_out_kernel(TriattnOutArgs p, uint
   const int t0 = (wave / NOT) * TPW;
   u32x4_t wg[KS], wo[KS];
   {
-    const int row = 32 * ot + rowperm16(l32);
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      wg[s] = *reinterpret_cast<const u32x4_t*>(p.w_g + row * C + 16 * s + 8 * lh);
-      wo[s] = *reinterpret_cast<const u32x4_t*>(p.w_o + row * HD + 16 * s + 8 * lh);
-    }
+    pass_bf16::load_unit<C>(p.w_g, ot, rowperm16(l32), lh, p.packed, wg);
+    pass_bf16::load_unit<HD>(p.w_o, ot, rowperm16(l32), lh, p.packed, wo);
   }
 
   const int N = p.N;
@@ -182,13 +179,18 @@ hipError_t launch(const TriattnOutArgs& a, hipStream_t stream) {
 }  // namespace
 
 hipError_t triattn_out_launch(const TriattnOutArgs& args, int C, int HD, hipStream_t stream) {
+  if ((C != 128 && C != 64) || HD != C) return hipErrorInvalidValue;
+  // Short sequences on 32-position tiles, under the rule of the triangle multiplication's output pass (C = 128, packed, us,
+  // 128- against 32-position tiles: N = 40 7.7 / 4.5, 64 7.6 / 4.6, 96 8.4 / 6.7, 128 7.6 / 7.2, 160 8.8 / 9.4).
+  bool small = false;
+  const hipError_t e = small_pass(args.B, args.N, C == 128 ? 2 : 1, &small);
+  if (e != hipSuccess) return e;
+  if (small) return triattn_out_panels_launch(args, C, stream);
   // a 128-position tile lies in one row (N a multiple of 128), in at most two (N >= 128), or anywhere
   const int mode = args.N % 128 == 0 ? 0 : (args.N >= 128 ? 1 : 2);
-  if (C == 128 && HD == 128)
+  if (C == 128)
     return mode == 0 ? launch<128, 128, 0>(args, stream) : (mode == 1 ? launch<128, 128, 1>(args, stream) : launch<128, 128, 2>(args, stream));
-  if (C == 64 && HD == 64)
-    return mode == 0 ? launch<64, 64, 0>(args, stream) : (mode == 1 ? launch<64, 64, 1>(args, stream) : launch<64, 64, 2>(args, stream));
-  return hipErrorInvalidValue;
+  return mode == 0 ? launch<64, 64, 0>(args, stream) : (mode == 1 ? launch<64, 64, 1>(args, stream) : launch<64, 64, 2>(args, stream));
 }
 
 }  // namespace of3

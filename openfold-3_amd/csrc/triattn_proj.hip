@@ -22,6 +22,7 @@
 #include "of3_device.h"
 #include "of3_kernels.h"
 #include "of3_launch.h"
+#include "of3_pass_bf16.h"
 
 // Waves per work-group of the C = 128 kernel: 8 (two per SIMD, 248 registers) or 16 (four per SIMD,
 // 118 registers, one matrix per wave).  Measured at N = 768 inside the block: 126 us against 128 us,
@@ -148,9 +149,7 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
       const int m = m0 + jj;
       const bf16_t* W = (m == 0) ? p.w_q : (m == 1 ? p.w_k : p.w_v);
       // q, k (A operands): lane owns 16 consecutive channels (rowperm16); v (B operand): natural rows
-      const int row = 32 * ot + ((ROLE == 1) ? l32 : rowperm16(l32));
-#pragma unroll
-      for (int s = 0; s < KS; ++s) wj[jj][s] = *reinterpret_cast<const u32x4_t*>(W + row * C + 16 * s + 8 * lh);
+      pass_bf16::load_unit<C>(W, ot, (ROLE == 1) ? l32 : rowperm16(l32), lh, p.packed, wj[jj]);
     }
 
     auto do_tile = [&](int tile_id, int buf) {
@@ -292,12 +291,17 @@ hipError_t launch(const TriattnProjArgs& a, hipStream_t stream) {
 }  // namespace
 
 hipError_t triattn_proj_launch(const TriattnProjArgs& args, int C, int D, hipStream_t stream) {
-  if (args.H != 4) return hipErrorInvalidValue;
+  if (args.H != 4 || (C != 128 && C != 64) || 4 * D != C) return hipErrorInvalidValue;
+  // Short sequences on 32-position tiles, under the rule of the triangle multiplication's input pass (C = 128, packed, us,
+  // 128- against 32-position tiles: N = 40 8.1 / 6.0, 64 8.6 / 6.8, 80 10.5 / 8.7, 96 11.1 / 9.6, 128 12.1 / 13.0).
+  bool small = false;
+  const hipError_t e = small_pass(args.B, args.N, 1, &small);
+  if (e != hipSuccess) return e;
+  if (small) return triattn_proj_panels_launch(args, C, stream);
   // ragged pieces hold up to four rows, all of which must exist
   const bool ragged = args.N % 128 != 0 && args.N >= 4;
-  if (C == 128 && D == 32) return ragged ? launch<128, 32, OF3_TP_WAVES, true>(args, stream) : launch<128, 32, OF3_TP_WAVES, false>(args, stream);
-  if (C == 64 && D == 16) return ragged ? launch<64, 16, 8, true>(args, stream) : launch<64, 16, 8, false>(args, stream);
-  return hipErrorInvalidValue;
+  if (C == 128) return ragged ? launch<128, 32, OF3_TP_WAVES, true>(args, stream) : launch<128, 32, OF3_TP_WAVES, false>(args, stream);
+  return ragged ? launch<64, 16, 8, true>(args, stream) : launch<64, 16, 8, false>(args, stream);
 }
 
 }  // namespace of3

@@ -15,6 +15,7 @@
 #include "of3_device.h"
 #include "of3_kernels.h"
 #include "of3_launch.h"
+#include "of3_pass_bf16.h"
 
 namespace of3 {
 
@@ -61,12 +62,8 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
   const int t0 = (wave / NOT) * TPW;
   u32x4_t wz[KS], wgt[KS];
   {
-    const int row = 32 * ot + rowperm16(l32);
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      wz[s] = *reinterpret_cast<const u32x4_t*>(p.w_z + row * CH + 16 * s + 8 * lh);
-      wgt[s] = *reinterpret_cast<const u32x4_t*>(p.w_g + row * C + 16 * s + 8 * lh);
-    }
+    pass_bf16::load_unit<CH>(p.w_z, ot, rowperm16(l32), lh, p.packed, wz);
+    pass_bf16::load_unit<C>(p.w_g, ot, rowperm16(l32), lh, p.packed, wgt);
   }
 
   const int N = p.N, Np = p.Np;
@@ -213,10 +210,17 @@ hipError_t launch(const TrimulOutArgs& a, hipStream_t stream) {
 }  // namespace
 
 hipError_t trimul_out_launch(const TrimulOutArgs& args, int C, int CH, hipStream_t stream) {
+  if ((C != 128 && C != 64) || CH != C) return hipErrorInvalidValue;
+  // Short sequences on 32-position tiles, up to two of them per CU (C = 128, us per pass with packed weights, 128- against
+  // 32-position tiles: N = 40 8.3 / 5.4, 64 8.5 / 5.8, 96 9.0 / 7.6, 128 9.4 / 8.6, 160 9.9 / 10.4), one at 64 channels
+  // (B = 2: N = 64 5.2 / 4.8, 80 5.4 / 5.9).
+  bool small = false;
+  const hipError_t e = small_pass(args.B, args.N, C == 128 ? 2 : 1, &small);
+  if (e != hipSuccess) return e;
+  if (small) return trimul_out_panels_launch(args, C, stream);
   const bool ragged = args.N % 128 != 0;
-  if (C == 128 && CH == 128) return ragged ? launch<128, 128, true>(args, stream) : launch<128, 128, false>(args, stream);
-  if (C == 64 && CH == 64) return ragged ? launch<64, 64, true>(args, stream) : launch<64, 64, false>(args, stream);
-  return hipErrorInvalidValue;
+  if (C == 128) return ragged ? launch<128, 128, true>(args, stream) : launch<128, 128, false>(args, stream);
+  return ragged ? launch<64, 64, true>(args, stream) : launch<64, 64, false>(args, stream);
 }
 
 }  // namespace of3

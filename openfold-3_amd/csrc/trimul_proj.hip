@@ -21,6 +21,7 @@
 #include "of3_device.h"
 #include "of3_kernels.h"
 #include "of3_launch.h"
+#include "of3_pass_bf16.h"
 
 namespace of3 {
 
@@ -65,12 +66,8 @@ __global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int 
   {
     const bf16_t* Wg = pair ? p.w_bg : p.w_ag;
     const bf16_t* Wp = pair ? p.w_bp : p.w_ap;
-    const int row = 32 * ot + l32;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      wg[s] = *reinterpret_cast<const u32x4_t*>(Wg + row * C + 16 * s + 8 * lh);
-      wp[s] = *reinterpret_cast<const u32x4_t*>(Wp + row * C + 16 * s + 8 * lh);
-    }
+    pass_bf16::load_unit<C>(Wg, ot, l32, lh, p.packed, wg);
+    pass_bf16::load_unit<C>(Wp, ot, l32, lh, p.packed, wp);
     // the weights count as used here: the compiler waits for them once, before the tile loop,
     // instead of carrying "may still be in flight" into every iteration (where its wait for
     // them would also be a wait for the tile's prefetch and the previous tile's stores)
@@ -232,9 +229,16 @@ hipError_t launch(const TrimulProjArgs& a, hipStream_t stream) {
 }  // namespace
 
 hipError_t trimul_proj_launch(const TrimulProjArgs& args, int C, int CH, hipStream_t stream) {
-  if (C == 128 && CH == 128) return launch<128, 128>(args, stream);
-  if (C == 64 && CH == 64) return launch<64, 64>(args, stream);
-  return hipErrorInvalidValue;
+  if ((C != 128 && C != 64) || CH != C) return hipErrorInvalidValue;
+  // Short sequences on 32-position tiles.  256 CUs, C = 128, us per pass, packed weights, 128- against 32-position tiles:
+  // N = 40 8.3 / 6.3, 64 8.9 / 6.8, 80 9.8 / 7.8, 96 10.6 / 10.5, 160 11.4 / 13.8 (row-major weights 10.9 / 12.5 at 96): the
+  // line lies at one tile per CU.  At 64 channels (B = 2) 5.6 / 4.4 at N = 64, even at 80.
+  bool small = false;
+  const hipError_t e = small_pass(args.B, args.N, 1, &small);
+  if (e != hipSuccess) return e;
+  if (small) return trimul_proj_panels_launch(args, C, stream);
+  if (C == 128) return launch<128, 128>(args, stream);
+  return launch<64, 64>(args, stream);
 }
 
 }  // namespace of3

@@ -39,6 +39,8 @@ SOURCES = [
     "pair_proj_f32.hip",
     "transition_f32.hip",
     "weight_split.hip",
+    "weight_pack.hip",
+    "pair_pass_bf16.hip",
     "single_f32.hip",
     "single_x3_f32.hip",
 ]

@@ -1,0 +1,35 @@
+"""bf16 position-wise passes around the lines of their dispatch: tiles of 32 positions for short sequences, of 128 for the
+others, weights as they are (the stages) or in operand order (a block's call)."""
+import pytest
+import torch
+
+import test_gpu_stages as stages
+import test_gpu_block_call as blocks
+from gpu_util import lib  # noqa: F401
+
+import of3pair
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,batch", [(1, 1), (31, 2), (33, 1), (64, 1), (96, 1), (41, 3)])
+@pytest.mark.parametrize("c,d", [(128, 32), (64, 16)])
+def test_stages(c, d, n, batch):
+    for flag in (False, True):
+        stages.test_trimul_proj(flag, c, n, batch)
+        stages.test_trimul_out(int(flag), c, n, batch)
+        stages.test_triattn_proj(flag, c, d, n, batch)
+        stages.test_triattn_out(flag, int(flag), c, d, n, batch)
+
+
+@pytest.mark.parametrize("c,d,n", [(128, 32, 32), (128, 32, 65), (128, 32, 85), (128, 32, 86), (128, 32, 128), (128, 32, 129),
+                                   (64, 16, 33), (64, 16, 90), (64, 16, 91)])
+def test_packed_weights(monkeypatch, c, d, n):
+    """Bit for bit the same however the weights are laid out."""
+    lib()
+    m = blocks._fill(of3pair.PairStack(c, c, d, 4), n).to("cuda").to(torch.bfloat16).eval()
+    gen = torch.Generator().manual_seed(n)
+    z = torch.randn(1, n, n, c, generator=gen).to("cuda").to(torch.bfloat16)
+    mask = (torch.rand(1, n, n, generator=gen) > 0.2).float().to("cuda")
+    want = blocks._by_modules(monkeypatch, lambda: m(z, mask))
+    assert torch.equal(m(z, mask), want)
