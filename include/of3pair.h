@@ -309,6 +309,21 @@ int of3_pairformer_block_fwd(const void* const* weights, const void* s, const vo
                              int64_t C_s, int64_t H_s, int64_t D_s, int64_t HID_s, float inf, float inf_s, int flags,
                              void* workspace, int64_t workspace_bytes, int dtype, void* stream);
 
+/* `blocks` PairFormerBlocks one after the other (pairformer.py:217-470): weights[i] holds the
+ * OF3_PAIRFORMER_BLOCK_WEIGHTS pointers of block i, the other arguments are those of the single block.  side_stream, when
+ * not null, takes the single representation beside the pair representation of the next block; the call orders it after
+ * what `stream` holds at its start and `stream` after it at its end, so for the caller all work is `stream`'s.  Null (as
+ * under a stream capture that is to stay on one stream): everything runs on `stream`. */
+int64_t of3_pairformer_stack_workspace_bytes(int dtype, int64_t blocks, int64_t B, int64_t N, int64_t C, int64_t CH,
+                                             int64_t H, int64_t D, int64_t HID, int64_t C_s, int64_t H_s, int64_t D_s,
+                                             int64_t HID_s);
+int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, const void* s, const void* z,
+                             const int64_t z_strides[3], const float* single_mask, const float* pair_mask,
+                             const int64_t mask_strides[3], void* s_out, void* z_out, int64_t B, int64_t N, int64_t C,
+                             int64_t CH, int64_t H, int64_t D, int64_t HID, int64_t C_s, int64_t H_s, int64_t D_s,
+                             int64_t HID_s, float inf, float inf_s, int flags, void* workspace, int64_t workspace_bytes,
+                             int dtype, void* stream, void* side_stream);
+
 #ifdef __cplusplus
 }
 #endif

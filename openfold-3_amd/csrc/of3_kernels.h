@@ -98,7 +98,7 @@ hipError_t triattn_out_panels_launch(const TriattnOutArgs& args, int C, hipStrea
 
 // Copies of bf16 weight matrices in MFMA operand order (weight_pack.hip): rows and K multiples of 32 and 16
 struct PackJobs {
-  static constexpr int kMax = 22;  // a pair block: 2 x 6 + 2 x 5
+  static constexpr int kBlock = 22, kMax = 4 * kBlock;  // a pair block: 2 x 6 + 2 x 5
   const bf16_t* src[kMax];
   bf16_t* dst[kMax];
   int K[kMax];
@@ -157,6 +157,9 @@ hipError_t layer_norm_fwd_f32(const float* x, const float* w, const float* b, fl
                               hipStream_t stream);
 
 // ---- single-representation attention with pair bias (single_attn.hip), bf16, c_s = H*D = 384
+// The projections of s need no pair bias: a stack issues them ahead of the rest
+constexpr int kSingleProject = 1, kSingleAttend = 2;
+
 struct SingleAttnArgs {
   const bf16_t* a;            // [B][N][c_s]
   const bf16_t* pair_bias;    // [B][H][N][N], the pair-bias projection of z
@@ -169,6 +172,7 @@ struct SingleAttnArgs {
   bf16_t* out;                // [B][N][c_s]; may alias a
   float inf;
   int B, N, Np, H, D, add_residual;  // Np = N rounded up to a multiple of 32
+  int phases = kSingleProject | kSingleAttend;
 };
 hipError_t single_attn_launch(const SingleAttnArgs& args, hipStream_t stream);
 
@@ -196,6 +200,7 @@ struct SingleAttnF32Args {
   float* out;                 // [B][N][C]; may alias a
   float inf;
   int B, N, C, H, D, add_residual;
+  int phases = kSingleProject | kSingleAttend;
 };
 hipError_t single_attn_fwd_f32(const SingleAttnF32Args& args, hipStream_t stream);
 // the same on split operands; single_attn_fwd_f32 hands over what it serves

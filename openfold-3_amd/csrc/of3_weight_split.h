@@ -11,7 +11,7 @@ namespace of3 {
 // Matrices are added one after the other into the workspace, then split by one launch (a launch costs 4 to 5 us
 // whatever it splits: a whole block's matrices go together).
 struct SplitJobs {
-  static constexpr int kMax = 25;  // a pair block: 2 x 6 + 2 x 5 + 3
+  static constexpr int kBlock = 25, kMax = 4 * kBlock;  // a pair block: 2 x 6 + 2 x 5 + 3
   const float* src[kMax];
   bf16_t* dst[kMax];
   int rows[kMax], K[kMax];

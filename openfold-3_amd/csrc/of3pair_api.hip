@@ -766,7 +766,8 @@ int64_t of3_attn_pair_bias_workspace_bytes_for(int dtype, int64_t B, int64_t N, 
   return 5 * align256(B * N * H * D * 4);
 }
 
-int of3_attn_pair_bias_fwd(const void* a, const void* pair_bias, const float* mask, const void* ln_w,
+// phases: which of the launches (of3_kernels.h)
+static int attn_pair_bias(int phases, const void* a, const void* pair_bias, const float* mask, const void* ln_w,
                            const void* ln_b, const void* w_q, const void* b_q, const void* w_k, const void* w_v,
                            const void* w_g, const void* w_o, void* out, int64_t B, int64_t N, int64_t C_s, int64_t H,
                            int64_t D, float inf, int add_residual, void* workspace, int64_t workspace_bytes,
@@ -807,6 +808,7 @@ int of3_attn_pair_bias_fwd(const void* a, const void* pair_bias, const float* ma
     s.H = (int)H;
     s.D = (int)D;
     s.add_residual = add_residual ? 1 : 0;
+    s.phases = phases;
     hipError_t e = of3::single_attn_fwd_f32(s, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? OF3_OK : fail_hip(e);
   }
@@ -846,8 +848,18 @@ int of3_attn_pair_bias_fwd(const void* a, const void* pair_bias, const float* ma
   s.H = (int)H;
   s.D = (int)D;
   s.add_residual = add_residual ? 1 : 0;
+  s.phases = phases;
   hipError_t e = of3::single_attn_launch(s, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
+}
+
+int of3_attn_pair_bias_fwd(const void* a, const void* pair_bias, const float* mask, const void* ln_w,
+                           const void* ln_b, const void* w_q, const void* b_q, const void* w_k, const void* w_v,
+                           const void* w_g, const void* w_o, void* out, int64_t B, int64_t N, int64_t C_s, int64_t H,
+                           int64_t D, float inf, int add_residual, void* workspace, int64_t workspace_bytes,
+                           int dtype, void* stream) {
+  return attn_pair_bias(of3::kSingleProject | of3::kSingleAttend, a, pair_bias, mask, ln_w, ln_b, w_q, b_q, w_k, w_v, w_g,
+                        w_o, out, B, N, C_s, H, D, inf, add_residual, workspace, workspace_bytes, dtype, stream);
 }
 
 int64_t of3_transition_rows_workspace_bytes(int64_t rows, int64_t C, int64_t HID) {
@@ -947,139 +959,166 @@ static int64_t pair_block_module_bytes(int dtype, int64_t B, int64_t N, int64_t 
   return need;
 }
 
+// A block's weights as its kernels read them.  fp32 on split operands: all matrices split; bf16: those of the passes
+// in MFMA operand order.
+struct BlockDims {
+  int dtype;
+  int64_t B, N, C, CH, H, D, HID;
+  float inf;
+  bool wide() const { return dtype == OF3_DTYPE_F32; }
+  int weights() const { return OF3_PAIR_BLOCK_WEIGHTS - (HID == 0 ? 5 : 0); }
+  int64_t prepared_bytes() const {
+    return wide() ? block_split_bytes(C, CH, H, D, HID) : align256(2 * 2 * (4 * CH * C + C * C + C * CH + 5 * H * D * C));
+  }
+};
+struct BlockWeights {
+  const void* w[OF3_PAIR_BLOCK_WEIGHTS];
+  of3::WeightX3 split[of3::SplitJobs::kBlock];
+  const of3::WeightX3 *mul, *att, *tr;
+  int packed;
+};
+
+// Prepares the matrices of n <= kPrepared blocks at dst by one launch (4 to 5 us however many they are)
+constexpr int kPrepared = of3::PackJobs::kMax / of3::PackJobs::kBlock;
+static_assert(kPrepared * of3::SplitJobs::kBlock <= of3::SplitJobs::kMax, "");
+static hipError_t prepare_blocks(const void* const* const* weights, int n, const BlockDims& k, void* dst, BlockWeights* out,
+                                 hipStream_t stream) {
+  const int64_t C = k.C, CH = k.CH, HD = k.H * k.D;
+  if (k.wide()) {
+    of3::WeightSplitter splitter(dst);
+    auto f = [](const void* p) { return static_cast<const float*>(p); };
+    for (int q = 0; q < n; ++q) {
+      BlockWeights& o = out[q];
+      for (int i = 0; i < k.weights(); ++i) o.w[i] = weights[q][i];
+      o.packed = 0;
+      o.mul = o.att = o.tr = nullptr;
+      splitter.w = reinterpret_cast<of3::bf16_t*>(static_cast<char*>(dst) + q * k.prepared_bytes());
+      of3::WeightX3* next = o.split;
+      if (of3::trimul_split_widths(C, CH)) {
+        o.mul = next;
+        for (int d = 0; d < 2; ++d, next += of3::kTrimulMatrices) {
+          const void* const* w = o.w + 10 * d;
+          of3::TrimulF32Args a;
+          a.w_ap = f(w[4]), a.w_ag = f(w[5]), a.w_bp = f(w[6]), a.w_bg = f(w[7]), a.w_g = f(w[8]), a.w_z = f(w[9]);
+          a.C = (int)C, a.CH = (int)CH;
+          of3::trimul_split_jobs(splitter, a, next);
+        }
+      }
+      if (of3::triattn_split_widths(C, k.H, k.D)) {
+        o.att = next;
+        for (int d = 0; d < 2; ++d, next += of3::kTriattnMatrices) {
+          const void* const* w = o.w + 20 + 8 * d;
+          of3::TriattnF32Args a;
+          a.w_q = f(w[3]), a.w_k = f(w[4]), a.w_v = f(w[5]), a.w_g = f(w[6]), a.w_o = f(w[7]);
+          a.C = (int)C, a.H = (int)k.H, a.D = (int)k.D;
+          of3::triattn_split_jobs(splitter, a, next);
+        }
+      }
+      if (k.HID && of3::transition_split_widths(C, k.HID)) {
+        o.tr = next;
+        of3::TransitionF32Args a;
+        a.w_a = f(o.w[38]), a.w_b = f(o.w[39]), a.w_out = f(o.w[40]);
+        a.C = (int)C, a.HID = (int)k.HID;
+        of3::transition_split_jobs(splitter, a, next);
+      }
+    }
+    return splitter.j.n > 0 ? splitter.launch(stream) : hipSuccess;
+  }
+  of3::PackJobs jobs;
+  jobs.n = jobs.first[0] = 0;
+  for (int q = 0; q < n; ++q) {
+    BlockWeights& o = out[q];
+    for (int i = 0; i < k.weights(); ++i) o.w[i] = weights[q][i];
+    o.packed = 1;
+    o.mul = o.att = o.tr = nullptr;
+    of3::bf16_t* to = reinterpret_cast<of3::bf16_t*>(static_cast<char*>(dst) + q * k.prepared_bytes());
+    auto add = [&](int i, int64_t rows, int64_t K) {
+      const int m = jobs.n++;
+      jobs.src[m] = bf(o.w[i]);
+      jobs.dst[m] = to;
+      jobs.K[m] = (int)K;
+      jobs.first[m + 1] = jobs.first[m] + (int)(rows * K / 8);
+      o.w[i] = to;
+      to += rows * K;
+    };
+    for (int d = 0; d < 2; ++d) {
+      for (int i = 4; i < 8; ++i) add(10 * d + i, CH, C);
+      add(10 * d + 8, C, C);
+      add(10 * d + 9, C, CH);
+    }
+    for (int d = 0; d < 2; ++d) {
+      for (int i = 3; i < 7; ++i) add(20 + 8 * d + i, HD, C);
+      add(20 + 8 * d + 7, C, HD);
+    }
+  }
+  return of3::pack_weights_launch(jobs, stream);
+}
+
+static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void* z, const int64_t z_strides[3],
+                          const float* mask, const int64_t mask_strides[3], void* out, int flags, void* workspace,
+                          int64_t workspace_bytes, void* stream) {
+  const void* src = z;  // the first module reads z, every later one updates out in place
+  auto trimul = [&](int m) {
+    const void* const* w = k.w + 10 * m;
+    const int st = trimul_fwd(k.mul ? k.mul + m * of3::kTrimulMatrices : nullptr, k.packed, src, z_strides, mask, mask_strides,
+                              w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8], w[9], out, d.B, d.N, d.C, d.CH, m == 0,
+                              1, workspace, workspace_bytes, d.dtype, stream);
+    src = out;
+    return st;
+  };
+  auto triattn = [&](int m) {
+    const void* const* w = k.w + 20 + 8 * m;
+    const int64_t zt[3] = {z_strides[0], m ? z_strides[2] : z_strides[1], m ? z_strides[1] : z_strides[2]};
+    int64_t mt[3] = {0, 0, 0};
+    if (mask) mt[0] = mask_strides[0], mt[1] = mask_strides[m ? 2 : 1], mt[2] = mask_strides[m ? 1 : 2];
+    const int st = triattn_fwd(k.att ? k.att + m * of3::kTriattnMatrices : nullptr, k.packed, src, zt, mask, mt, w[0], w[1],
+                               w[2], w[3], w[4], w[5], w[6], w[7], out, d.B, d.N, d.C, d.H, d.D, d.inf, 1, workspace,
+                               workspace_bytes, d.dtype, stream);
+    src = out;
+    return st;
+  };
+  int st = OF3_OK;
+  for (int part = 0; part < 2; ++part)
+    for (int m = 0; m < 2 && st == OF3_OK; ++m)
+      st = (part == 0) == !(flags & OF3_BLOCK_ATTENTION_FIRST) ? trimul(m) : triattn(m);
+  if (st != OF3_OK || d.HID == 0) return st;
+  const void* const* w = k.w + 36;
+  return transition_fwd(k.tr, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask, mask_strides, w[0], w[1],
+                        w[2], w[3], w[4], out, d.B, d.N, d.C, d.HID, 1, d.wide() ? workspace : nullptr,
+                        d.wide() ? workspace_bytes : 0, d.dtype, stream);
+}
+
+// what a block's call checks before its first launch: a block is updated in place, half of one is of no use
+static bool pair_block_args_ok(const BlockDims& d, const void* const* weights, const void* z, const int64_t z_strides[3],
+                               const float* mask, const int64_t mask_strides[3], const void* out, const void* workspace) {
+  if (!weights || !z || !out || !mask_ok(mask, mask_strides)) return false;
+  if (d.wide() ? !f32_strides_ok(z_strides) : !strides_ok(z_strides)) return false;
+  if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return false;
+  for (int i = 0; i < d.weights(); ++i)
+    if (!weights[i] || !(d.wide() ? aligned4(weights[i]) : aligned16(weights[i]))) return false;
+  return d.wide() ? aligned4(z) && aligned4(out) : aligned16(z) && aligned16(out);
+}
+
 int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
                                        int64_t HID) {
   const int64_t need = pair_block_module_bytes(dtype, B, N, C, CH, H, D, HID);
-  if (need < 0) return need;
-  // fp32: the block's matrices split; bf16: the passes' matrices in operand order
-  if (dtype == OF3_DTYPE_F32) return need + block_split_bytes(C, CH, H, D, HID);
-  return need + align256(2 * 2 * (4 * CH * C + C * C + C * CH + 5 * H * D * C));
+  const BlockDims d = {dtype, B, N, C, CH, H, D, HID, 0.f};
+  return need < 0 ? need : need + d.prepared_bytes();
 }
 
 int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t z_strides[3], const float* mask,
                        const int64_t mask_strides[3], void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H,
                        int64_t D, int64_t HID, float inf, int flags, void* workspace, int64_t workspace_bytes, int dtype,
                        void* stream) {
-  // everything is checked before the first launch: a block is updated in place, half of one is of no use
   const int64_t need = of3_pair_block_workspace_bytes(dtype, B, N, C, CH, H, D, HID);
-  if (need < 0 || !weights || !z || !out || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
-  const bool wide = dtype == OF3_DTYPE_F32;
-  if (wide ? !f32_strides_ok(z_strides) : !strides_ok(z_strides)) return OF3_EINVAL;
-  if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return OF3_EINVAL;
-  const int n_weights = OF3_PAIR_BLOCK_WEIGHTS - (HID == 0 ? 5 : 0);
-  for (int i = 0; i < n_weights; ++i)
-    if (!weights[i] || !(wide ? aligned4(weights[i]) : aligned16(weights[i]))) return OF3_EINVAL;
-  if (wide ? !(aligned4(z) && aligned4(out)) : !(aligned16(z) && aligned16(out))) return OF3_EINVAL;
+  const BlockDims d = {dtype, B, N, C, CH, H, D, HID, inf};
+  if (need < 0 || !pair_block_args_ok(d, weights, z, z_strides, mask, mask_strides, out, workspace)) return OF3_EINVAL;
   if (workspace_bytes < need) return OF3_ENOSPC;
-
-  const void* const* w_mul = weights;
-  const void* const* w_att = weights + 20;
-  const void* const* w_tr = weights + 36;
-  // fp32 on split operands: all matrices of the block in one launch
-  of3::WeightX3 split[2 * of3::kTrimulMatrices + 2 * of3::kTriattnMatrices + of3::kTransitionMatrices];
-  const of3::WeightX3 *s_mul = nullptr, *s_att = nullptr, *s_tr = nullptr;
-  if (wide) {
-    of3::WeightSplitter splitter(static_cast<char*>(workspace) + pair_block_module_bytes(dtype, B, N, C, CH, H, D, HID));
-    auto f = [](const void* p) { return static_cast<const float*>(p); };
-    of3::WeightX3* next = split;
-    if (of3::trimul_split_widths(C, CH)) {
-      s_mul = next;
-      for (int d = 0; d < 2; ++d, next += of3::kTrimulMatrices) {
-        const void* const* w = w_mul + 10 * d;
-        of3::TrimulF32Args a;
-        a.w_ap = f(w[4]), a.w_ag = f(w[5]), a.w_bp = f(w[6]), a.w_bg = f(w[7]), a.w_g = f(w[8]), a.w_z = f(w[9]);
-        a.C = (int)C, a.CH = (int)CH;
-        of3::trimul_split_jobs(splitter, a, next);
-      }
-    }
-    if (of3::triattn_split_widths(C, H, D)) {
-      s_att = next;
-      for (int d = 0; d < 2; ++d, next += of3::kTriattnMatrices) {
-        const void* const* w = w_att + 8 * d;
-        of3::TriattnF32Args a;
-        a.w_q = f(w[3]), a.w_k = f(w[4]), a.w_v = f(w[5]), a.w_g = f(w[6]), a.w_o = f(w[7]);
-        a.C = (int)C, a.H = (int)H, a.D = (int)D;
-        of3::triattn_split_jobs(splitter, a, next);
-      }
-    }
-    if (HID && of3::transition_split_widths(C, HID)) {
-      s_tr = next;
-      of3::TransitionF32Args a;
-      a.w_a = f(w_tr[2]), a.w_b = f(w_tr[3]), a.w_out = f(w_tr[4]);
-      a.C = (int)C, a.HID = (int)HID;
-      of3::transition_split_jobs(splitter, a, next);
-    }
-    if (splitter.j.n > 0) {
-      const hipError_t e = splitter.launch(static_cast<hipStream_t>(stream));
-      if (e != hipSuccess) return fail_hip(e);
-    }
-  }
-
-  // bf16: the passes' weight matrices in MFMA operand order, likewise
-  const void* packed_weights[OF3_PAIR_BLOCK_WEIGHTS];
-  const int packed = wide ? 0 : 1;
-  if (!wide) {
-    for (int i = 0; i < n_weights; ++i) packed_weights[i] = weights[i];
-    of3::PackJobs jobs;
-    jobs.n = jobs.first[0] = 0;
-    of3::bf16_t* dst = reinterpret_cast<of3::bf16_t*>(static_cast<char*>(workspace) +
-                                                      pair_block_module_bytes(dtype, B, N, C, CH, H, D, HID));
-    auto add = [&](int i, int64_t rows, int64_t K) {
-      const int n = jobs.n++;
-      jobs.src[n] = bf(weights[i]);
-      jobs.dst[n] = dst;
-      jobs.K[n] = (int)K;
-      jobs.first[n + 1] = jobs.first[n] + (int)(rows * K / 8);
-      packed_weights[i] = dst;
-      dst += rows * K;
-    };
-    for (int m = 0; m < 2; ++m) {
-      for (int i = 4; i < 8; ++i) add(10 * m + i, CH, C);
-      add(10 * m + 8, C, C);
-      add(10 * m + 9, C, CH);
-    }
-    for (int m = 0; m < 2; ++m) {
-      for (int i = 3; i < 7; ++i) add(20 + 8 * m + i, H * D, C);
-      add(20 + 8 * m + 7, C, H * D);
-    }
-    const hipError_t e = of3::pack_weights_launch(jobs, static_cast<hipStream_t>(stream));
-    if (e != hipSuccess) return fail_hip(e);
-    w_mul = packed_weights;
-    w_att = packed_weights + 20;
-  }
-
-  const void* src = z;  // the first module reads z, every later one updates out in place
-  auto trimul = [&](const void* const* w, int outgoing) {
-    const int st = trimul_fwd(s_mul ? s_mul + (outgoing ? 0 : of3::kTrimulMatrices) : nullptr, packed, src, z_strides,
-                              mask, mask_strides, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8], w[9], out, B,
-                              N, C, CH, outgoing, 1, workspace, workspace_bytes, dtype, stream);
-    src = out;
-    return st;
-  };
-  auto triattn = [&](const void* const* w, bool ending) {
-    const int64_t zt[3] = {z_strides[0], ending ? z_strides[2] : z_strides[1], ending ? z_strides[1] : z_strides[2]};
-    int64_t mt[3] = {0, 0, 0};
-    if (mask) mt[0] = mask_strides[0], mt[1] = mask_strides[ending ? 2 : 1], mt[2] = mask_strides[ending ? 1 : 2];
-    const int st = triattn_fwd(s_att ? s_att + (ending ? of3::kTriattnMatrices : 0) : nullptr, packed, src, zt, mask,
-                               mt, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], out, B, N, C, H, D, inf, 1,
-                               workspace, workspace_bytes, dtype, stream);
-    src = out;
-    return st;
-  };
-  int st = OF3_OK;
-  for (int part = 0; part < 2 && st == OF3_OK; ++part) {
-    if ((part == 0) == !(flags & OF3_BLOCK_ATTENTION_FIRST)) {
-      st = trimul(w_mul, 1);
-      if (st == OF3_OK) st = trimul(w_mul + 10, 0);
-    } else {
-      st = triattn(w_att, false);
-      if (st == OF3_OK) st = triattn(w_att + 8, true);
-    }
-  }
-  if (st != OF3_OK || HID == 0) return st;
-  return transition_fwd(s_tr, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask, mask_strides, w_tr[0],
-                        w_tr[1], w_tr[2], w_tr[3], w_tr[4], out, B, N, C, HID, 1, wide ? workspace : nullptr,
-                        wide ? workspace_bytes : 0, dtype, stream);
+  BlockWeights k;
+  const hipError_t e = prepare_blocks(&weights, 1, d, static_cast<char*>(workspace) + need - d.prepared_bytes(), &k,
+                                      static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail_hip(e);
+  return run_pair_block(k, d, z, z_strides, mask, mask_strides, out, flags, workspace, workspace_bytes, stream);
 }
 
 int64_t of3_pairformer_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
@@ -1093,24 +1132,28 @@ int64_t of3_pairformer_block_workspace_bytes(int dtype, int64_t B, int64_t N, in
   return rows > need ? rows : need;
 }
 
+static bool single_args_ok(const BlockDims& d, const void* const* w, const void* s, const void* s_out, const float* single_mask) {
+  for (int i = 0; i < OF3_PAIRFORMER_BLOCK_WEIGHTS - OF3_PAIR_BLOCK_WEIGHTS; ++i)
+    if ((!w[i] && i != 1) || !(d.wide() ? aligned4(w[i]) : aligned16(w[i]))) return false;  // 1: no offset
+  if (!s || !s_out || !(d.wide() ? aligned4(s) && aligned4(s_out) : aligned16(s) && aligned16(s_out))) return false;
+  return !single_mask || aligned4(single_mask);
+}
+
 int of3_pairformer_block_fwd(const void* const* weights, const void* s, const void* z, const int64_t z_strides[3],
                              const float* single_mask, const float* pair_mask, const int64_t mask_strides[3], void* s_out,
                              void* z_out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D, int64_t HID,
                              int64_t C_s, int64_t H_s, int64_t D_s, int64_t HID_s, float inf, float inf_s, int flags,
                              void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
   const int64_t need = of3_pairformer_block_workspace_bytes(dtype, B, N, C, CH, H, D, HID, C_s, H_s, D_s, HID_s);
-  if (need < 0 || B > 65535 || N > (1 << 16) || !weights || !s || !s_out) return OF3_EINVAL;
-  const bool wide = dtype == OF3_DTYPE_F32;
+  const BlockDims d = {dtype, B, N, C, CH, H, D, HID, inf};
+  if (need < 0 || B > 65535 || N > (1 << 16) || !weights) return OF3_EINVAL;
   const void* const* ws_ = weights + OF3_PAIR_BLOCK_WEIGHTS;
-  for (int i = 0; i < OF3_PAIRFORMER_BLOCK_WEIGHTS - OF3_PAIR_BLOCK_WEIGHTS; ++i)
-    if ((!ws_[i] && i != 1) || !(wide ? aligned4(ws_[i]) : aligned16(ws_[i]))) return OF3_EINVAL;  // 1: no offset
-  if (wide ? !(aligned4(s) && aligned4(s_out)) : !(aligned16(s) && aligned16(s_out))) return OF3_EINVAL;
-  if (single_mask && !aligned4(single_mask)) return OF3_EINVAL;
+  if (!single_args_ok(d, ws_, s, s_out, single_mask)) return OF3_EINVAL;
   if (workspace_bytes < need) return OF3_ENOSPC;
   int st = of3_pair_block_fwd(weights, z, z_strides, pair_mask, mask_strides, z_out, B, N, C, CH, H, D, HID, inf, flags,
                               workspace, workspace_bytes, dtype, stream);
   if (st != OF3_OK) return st;
-  const int64_t bias_bytes = align256(B * H_s * N * N * (wide ? 4 : 2));
+  const int64_t bias_bytes = align256(B * H_s * N * N * (d.wide() ? 4 : 2));
   st = of3_pair_bias_fwd(z_out, z_strides, ws_[0], ws_[1], ws_[2], workspace, B, N, C, H_s, dtype, stream);
   if (st != OF3_OK) return st;
   st = of3_attn_pair_bias_fwd(s, workspace, single_mask, ws_[3], ws_[4], ws_[5], ws_[6], ws_[7], ws_[8], ws_[9], ws_[10],
@@ -1120,6 +1163,137 @@ int of3_pairformer_block_fwd(const void* const* weights, const void* s, const vo
   return of3_transition_rows_fwd(s_out, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : single_mask, ws_[11], ws_[12],
                                  ws_[13], ws_[14], ws_[15], s_out, B * N, C_s, HID_s, 1, workspace, workspace_bytes, dtype,
                                  stream);
+}
+
+// ---- a stack of PairFormerBlocks in one call --------------------------------------------------
+// The pair representation of block i + 1 needs nothing of block i's single representation: with a second stream the
+// attention and transition of s (44 us per block at 40 tokens, of 148) run beside the next block's pair updates, which
+// do not fill the chip at the lengths where that time counts.
+
+// Two streams of one call and the order between them; without a second stream nothing to order.  An event waited for on
+// another stream costs the host 15 us, five launches, so there are as few as can be.
+class StreamPair {
+ public:
+  enum { kBias, kFree, kJoin, kEvents };
+  StreamPair(hipStream_t main, hipStream_t side) : main(main), side(side ? side : main) {}
+  ~StreamPair() {
+    if (open_) join();
+    for (hipEvent_t e : events_)
+      if (e) (void)hipEventDestroy(e);  // released once the work recorded in it is done
+  }
+  // what is issued to `to` from now on waits for what `from` has been given so far
+  int order(hipStream_t from, hipStream_t to, int event) {
+    const int st = record(from, event);
+    return st == OF3_OK ? wait(to, event) : st;
+  }
+  int record(hipStream_t from, int event) {
+    if (main == side) return OF3_OK;
+    hipError_t e = hipSuccess;
+    // both streams are one device's: the fence that makes results visible to the host is not needed
+    if (!events_[event]) e = hipEventCreateWithFlags(&events_[event], hipEventDisableTiming | hipEventDisableSystemFence);
+    if (e == hipSuccess) e = hipEventRecord(events_[event], from);
+    return e == hipSuccess ? OF3_OK : fail_hip(e);
+  }
+  int wait(hipStream_t to, int event) {
+    if (main == side) return OF3_OK;
+    open_ |= to == side;
+    const hipError_t e = hipStreamWaitEvent(to, events_[event], 0);
+    return e == hipSuccess ? OF3_OK : fail_hip(e);
+  }
+  int join() {
+    if (!open_) return OF3_OK;
+    open_ = false;
+    return order(side, main, kJoin);
+  }
+  const hipStream_t main, side;
+
+ private:
+  hipEvent_t events_[kEvents] = {};
+  bool open_ = false;  // the side stream holds work that main does not wait for yet
+};
+
+// regions of a stack's workspace
+struct StackSpace {
+  int64_t module, prepared, bias, single, total;
+  int64_t buffers;  // pair biases: one per block up to 64 MB of them, at least two
+};
+static StackSpace stack_space(const BlockDims& d, int64_t blocks, int64_t C_s, int64_t H_s, int64_t D_s, int64_t HID_s) {
+  StackSpace w;
+  const int64_t attn = of3_attn_pair_bias_workspace_bytes_for(d.dtype, d.B, d.N, C_s, H_s, D_s);
+  const int64_t rows = of3_transition_rows_fast_workspace_bytes(d.dtype, d.B * d.N, C_s, HID_s);
+  w.module = pair_block_module_bytes(d.dtype, d.B, d.N, d.C, d.CH, d.H, d.D, d.HID);
+  w.total = OF3_EINVAL;
+  if (w.module < 0 || attn < 0 || rows < 0 || d.HID < 1 || H_s > (d.wide() ? 64 : 32) || blocks < 1) return w;
+  w.module = align256(w.module);
+  w.prepared = d.prepared_bytes() * (blocks < kPrepared ? blocks : kPrepared);
+  w.bias = align256(d.B * H_s * d.N * d.N * (d.wide() ? 4 : 2));
+  w.buffers = (64ll << 20) / w.bias;
+  if (w.buffers < 2) w.buffers = 2;
+  if (w.buffers > blocks) w.buffers = blocks;
+  w.single = align256(attn > rows ? attn : rows);
+  w.total = w.module + w.prepared + w.buffers * w.bias + w.single;
+  return w;
+}
+
+int64_t of3_pairformer_stack_workspace_bytes(int dtype, int64_t blocks, int64_t B, int64_t N, int64_t C, int64_t CH,
+                                             int64_t H, int64_t D, int64_t HID, int64_t C_s, int64_t H_s, int64_t D_s,
+                                             int64_t HID_s) {
+  const BlockDims d = {dtype, B, N, C, CH, H, D, HID, 0.f};
+  return stack_space(d, blocks, C_s, H_s, D_s, HID_s).total;
+}
+
+int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, const void* s, const void* z,
+                             const int64_t z_strides[3], const float* single_mask, const float* pair_mask,
+                             const int64_t mask_strides[3], void* s_out, void* z_out, int64_t B, int64_t N, int64_t C,
+                             int64_t CH, int64_t H, int64_t D, int64_t HID, int64_t C_s, int64_t H_s, int64_t D_s,
+                             int64_t HID_s, float inf, float inf_s, int flags, void* workspace, int64_t workspace_bytes,
+                             int dtype, void* stream, void* side_stream) {
+  const BlockDims d = {dtype, B, N, C, CH, H, D, HID, inf};
+  const StackSpace w = stack_space(d, blocks, C_s, H_s, D_s, HID_s);
+  if (w.total < 0 || B > 65535 || N > (1 << 16) || !weights) return OF3_EINVAL;
+  for (int64_t i = 0; i < blocks; ++i)
+    if (!pair_block_args_ok(d, weights[i], z, z_strides, pair_mask, mask_strides, z_out, workspace) ||
+        !single_args_ok(d, weights[i] + OF3_PAIR_BLOCK_WEIGHTS, s, s_out, single_mask))
+      return OF3_EINVAL;
+  if (workspace_bytes < w.total) return OF3_ENOSPC;
+  char* const prepared = static_cast<char*>(workspace) + w.module;
+  char* const bias0 = prepared + w.prepared;
+  char* const single = bias0 + w.buffers * w.bias;
+
+  StreamPair streams(static_cast<hipStream_t>(stream), static_cast<hipStream_t>(side_stream));
+  BlockWeights k[kPrepared];
+  int st = OF3_OK;
+  for (int64_t i = 0; i < blocks && st == OF3_OK; ++i) {
+    const int q = (int)(i % kPrepared);
+    const bool last = i + 1 == blocks;
+    if (q == 0) {
+      const int n = (int)(blocks - i < kPrepared ? blocks - i : kPrepared);
+      const hipError_t e = prepare_blocks(weights + i, n, d, prepared, k, streams.main);
+      if (e != hipSuccess) return fail_hip(e);
+    }
+    const void* const* ws_ = weights[i] + OF3_PAIR_BLOCK_WEIGHTS;
+    void* const bias = bias0 + (i % w.buffers) * w.bias;
+    auto attention = [&](int phases, hipStream_t on) {
+      return attn_pair_bias(phases, i ? s_out : s, bias, single_mask, ws_[3], ws_[4], ws_[5], ws_[6], ws_[7], ws_[8], ws_[9],
+                            ws_[10], s_out, B, N, C_s, H_s, D_s, inf_s, 1, single, w.single, dtype, on);
+    };
+    // the projections of s need no pair bias; those of the first block have nothing to wait behind on the side stream
+    if (i > 0 && (st = attention(of3::kSingleProject, streams.side)) != OF3_OK) break;
+    st = run_pair_block(k[q], d, i ? z_out : z, z_strides, pair_mask, mask_strides, z_out, flags, workspace, w.module, streams.main);
+    if (st != OF3_OK) break;
+    // a buffer is used again: the attentions issued so far have read theirs
+    if (i >= w.buffers && (st = streams.wait(streams.main, StreamPair::kFree)) != OF3_OK) break;
+    st = of3_pair_bias_fwd(z_out, z_strides, ws_[0], ws_[1], ws_[2], bias, B, N, C, H_s, dtype, streams.main);
+    if (st != OF3_OK) break;
+    // the last block has nothing beside it: it goes on where its bias was written
+    st = last ? streams.join() : streams.order(streams.main, streams.side, StreamPair::kBias);
+    const hipStream_t on = last ? streams.main : streams.side;
+    if (st != OF3_OK || (st = attention(i ? of3::kSingleAttend : of3::kSingleProject | of3::kSingleAttend, on)) != OF3_OK) break;
+    if (i + 2 < blocks && i + 2 >= w.buffers && (st = streams.record(on, StreamPair::kFree)) != OF3_OK) break;
+    st = of3_transition_rows_fwd(s_out, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : single_mask, ws_[11], ws_[12],
+                                 ws_[13], ws_[14], ws_[15], s_out, B * N, C_s, HID_s, 1, single, w.single, dtype, on);
+  }
+  return st;
 }
 
 }  // extern "C"

@@ -289,11 +289,14 @@ hipError_t single_attn_launch(const SingleAttnArgs& a, hipStream_t stream) {
     return hipErrorInvalidValue;
   if (a.Np != (a.N + 31) / 32 * 32) return hipErrorInvalidValue;
   const int row_blocks = a.Np / 32;
-  hipLaunchKernelGGL(single_proj_kernel, dim3(row_blocks, a.H, a.B), dim3(256), 0, stream, a);  // one tile per wave
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (a.phases & kSingleProject) {
+    hipLaunchKernelGGL(single_proj_kernel, dim3(row_blocks, a.H, a.B), dim3(256), 0, stream, a);  // one tile per wave
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (!(a.phases & kSingleAttend)) return hipSuccess;
   hipLaunchKernelGGL(single_attn_kernel, dim3(row_blocks, a.H, a.B), dim3(64 * kSplit), 0, stream, a, row_blocks);
-  e = hipGetLastError();
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(single_out_kernel, dim3(row_blocks, 3, a.B), dim3(256), 0, stream, a);
   return hipGetLastError();

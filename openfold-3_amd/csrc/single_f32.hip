@@ -329,9 +329,12 @@ hipError_t single_attn_fwd_f32(const SingleAttnF32Args& a, hipStream_t stream) {
   hipError_t e = allow_dynamic_lds<single_proj_f32>(kWTileBytes);
   if (e == hipSuccess) e = allow_dynamic_lds<single_out_f32>(kWTileBytes);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(single_proj_f32, dim3((unsigned)blocks), dim3(kThreads), kWTileBytes, stream, a);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (a.phases & kSingleProject) {
+    hipLaunchKernelGGL(single_proj_f32, dim3((unsigned)blocks), dim3(kThreads), kWTileBytes, stream, a);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (!(a.phases & kSingleAttend)) return hipSuccess;
   const dim3 grid((a.N + kAttnQ - 1) / kAttnQ, a.H, a.B);
   if (a.D <= 32) hipLaunchKernelGGL(single_attn_f32<32>, grid, dim3(kAttnQ * kAttnParts), 0, stream, a);
   else hipLaunchKernelGGL(single_attn_f32<64>, grid, dim3(kAttnQ * kAttnParts), 0, stream, a);

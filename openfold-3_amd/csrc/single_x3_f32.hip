@@ -494,12 +494,15 @@ hipError_t single_attn_x3_fwd_f32(const SingleAttnF32Args& a, hipStream_t stream
   const long row_tiles = (rows + 31) / 32;
   if (row_tiles > 0x7fffffffl) return hipErrorInvalidValue;
   const int HD = a.H * a.D;
-  hipLaunchKernelGGL(single_proj_x3_f32, dim3((unsigned)row_tiles, 4 * HD / 32), dim3(64 * kLnWaves), 0, stream, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (a.phases & kSingleProject) {
+    hipLaunchKernelGGL(single_proj_x3_f32, dim3((unsigned)row_tiles, 4 * HD / 32), dim3(64 * kLnWaves), 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (!(a.phases & kSingleAttend)) return hipSuccess;
   const int pb_vec = a.N % 4 == 0 && aligned16({a.pair_bias}) ? 1 : 0;
   hipLaunchKernelGGL(single_attn_x3_f32, dim3((a.N + 31) / 32, a.H, a.B), dim3(64 * kAttnWaves), 0, stream, a, pb_vec);
-  e = hipGetLastError();
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(single_out_x3_f32, dim3((unsigned)row_tiles, a.C / 32), dim3(64 * kOutWaves), 0, stream, a);
   return hipGetLastError();

@@ -13,8 +13,12 @@ __global__ __launch_bounds__(kThreads) void pack_weights(PackJobs j) {
   const int gitem = (int)blockIdx.x * kThreads + (int)threadIdx.x;
   const int wave_item = __builtin_amdgcn_readfirstlane(gitem);  // a matrix is a multiple of 64 items
   if (wave_item >= j.first[j.n]) return;
-  int q = 0;
-  while (q + 1 < j.n && wave_item >= j.first[q + 1]) ++q;
+  int q = 0, end = j.n;  // the matrix that holds the item
+  while (end - q > 1) {
+    const int mid = (q + end) / 2;
+    if (wave_item >= j.first[mid]) q = mid;
+    else end = mid;
+  }
   const int K = j.K[q], steps = K / 16, item = gitem - j.first[q];
   const int lane = item & 63, ts = item >> 6, s = ts % steps, t = ts / steps;
   reinterpret_cast<u32x4_t*>(j.dst[q])[item] =

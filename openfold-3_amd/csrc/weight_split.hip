@@ -15,8 +15,12 @@ __global__ __launch_bounds__(kThreads) void split_weights_f32(SplitJobs j) {
   // the 64 items of a wave belong to one matrix (every matrix has a multiple of 64)
   const int wave_item = __builtin_amdgcn_readfirstlane(gitem);
   if (wave_item >= j.first[j.n]) return;
-  int q = 0;
-  while (q + 1 < j.n && wave_item >= j.first[q + 1]) ++q;
+  int q = 0, end = j.n;  // the matrix that holds the item
+  while (end - q > 1) {
+    const int mid = (q + end) / 2;
+    if (wave_item >= j.first[mid]) q = mid;
+    else end = mid;
+  }
   const int rows = j.rows[q], K = j.K[q], steps = K / 16;
   const int item = gitem - j.first[q];
   const int lane = item & 63, ts = item >> 6;

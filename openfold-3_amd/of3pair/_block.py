@@ -1,4 +1,5 @@
-"""Whole blocks through one call of the C ABI (of3_pair_block_fwd, of3_pairformer_block_fwd).
+"""Whole blocks and stacks through one call of the C ABI (of3_pair_block_fwd, of3_pairformer_block_fwd,
+of3_pairformer_stack_fwd).
 
 A block issued module by module costs some 200 us of Python (parameter lookups, views, stream and device
 queries for each of its seven modules) beside 50 us of launches, more than its kernels take below about 200
@@ -268,33 +269,95 @@ def run_pair_block(block, z, mask, inplace, attention_first=False, mask_trans=Tr
     return z if inplace else out4.view(z.shape)
 
 
-def run_pairformer_block(block, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
-    """(s, z) after the block, or None when the single call does not serve it."""
-    found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
-    if not found or not s.is_cuda or s.dtype is not z.dtype or not s.is_contiguous():
+def _pairformer_args(s, z, single_mask, pair_mask, c, c_s):
+    """The tensors of a block's or a stack's call: (z4, mask arguments, single mask as fp32), or None."""
+    if not s.is_cuda or s.dtype is not z.dtype or not s.is_contiguous():
         return None
     args = _pair_args(z, pair_mask)
-    if not args or s.shape[:-1] != z.shape[:-2]:
-        return None
-    array, ((c, ch, h, d, hid, inf), (c_s, h_s, d_s, hid_s, inf_s)) = found
-    z4, (m, mptr, mstr) = args
-    B, N, _, C = z4.shape
-    if C != c or s.shape[-1] != c_s:
-        return None
-    lib = _lib.load()
-    code = _lib.OF3_DTYPE_BF16 if z.dtype is torch.bfloat16 else _lib.OF3_DTYPE_F32
-    need = lib.of3_pairformer_block_workspace_bytes(code, B, N, C, ch, h, d, hid, c_s, h_s, d_s, hid_s)
-    if need < 0:
+    if not args or s.shape[:-1] != z.shape[:-2] or args[0].shape[-1] != c or s.shape[-1] != c_s:
         return None
     sm = None
     if single_mask is not None:
         sm = single_mask.to(torch.float32).expand(s.shape[:-1]).contiguous()
+    return args + (sm,)
+
+
+def run_pairformer_block(block, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
+    """(s, z) after the block, or None when the single call does not serve it."""
+    found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
+    if not found:
+        return None
+    array, ((c, ch, h, d, hid, inf), (c_s, h_s, d_s, hid_s, inf_s)) = found
+    args = _pairformer_args(s, z, single_mask, pair_mask, c, c_s)
+    if not args:
+        return None
+    z4, (m, mptr, mstr), sm = args
+    B, N = z4.shape[:2]
+    lib = _lib.load()
+    code = _lib.OF3_DTYPE_BF16 if z.dtype is torch.bfloat16 else _lib.OF3_DTYPE_F32
+    need = lib.of3_pairformer_block_workspace_bytes(code, B, N, c, ch, h, d, hid, c_s, h_s, d_s, hid_s)
+    if need < 0:
+        return None
     z_out = z4 if inplace else F3._out_like(z4)
     s_out = s if inplace else torch.empty_like(s)
     stream = F3._stream(z)
     ws = F3._workspace(z.device, need, stream)
     _call(lib.of3_pairformer_block_fwd, "of3_pairformer_block_fwd", z.device, array, s.data_ptr(), z4.data_ptr(),
           _lib.strides3(z4.stride()[:3]), None if sm is None else sm.data_ptr(), mptr, mstr, s_out.data_ptr(),
-          z_out.data_ptr(), B, N, C, ch, h, d, hid, c_s, h_s, d_s, hid_s, float(inf), float(inf_s),
+          z_out.data_ptr(), B, N, c, ch, h, d, hid, c_s, h_s, d_s, hid_s, float(inf), float(inf_s),
           0 if mask_trans else _lib.OF3_BLOCK_TRANSITION_UNMASKED, ws.data_ptr(), ws.numel(), code, stream)
+    return s_out, z if inplace else z_out.view(z.shape)
+
+
+_sides = {}  # (device, stream) -> the stream of torch's pool that a stack's single representation runs on
+_MAX_SIDES = 16
+
+
+def _side_stream(device, stream):
+    """A second stream for work that is issued to `stream`; None while a stream is being captured (a graph would draw
+    in a stream that other threads may be using)."""
+    if torch.cuda.is_current_stream_capturing():
+        return None
+    side = _sides.get((device, stream))
+    if side is None:
+        if len(_sides) >= _MAX_SIDES:
+            _sides.clear()
+        side = _sides[(device, stream)] = torch.cuda.Stream(device=device)
+    return side.cuda_stream if side.cuda_stream != stream else None
+
+
+def run_pairformer_stack(blocks, block_type, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
+    """(s, z) after all blocks, or None when the single call does not serve them."""
+    arrays, dims = [], None
+    for block in blocks:
+        if type(block) is not block_type or block.training or block._forward_hooks or block._forward_pre_hooks:
+            return None
+        found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
+        if not found or (dims is not None and found[1] != dims):
+            return None
+        arrays.append(found[0])
+        dims = found[1]
+    if not arrays:
+        return None
+    (c, ch, h, d, hid, inf), (c_s, h_s, d_s, hid_s, inf_s) = dims
+    args = _pairformer_args(s, z, single_mask, pair_mask, c, c_s)
+    if not args:
+        return None
+    z4, (m, mptr, mstr), sm = args
+    B, N = z4.shape[:2]
+    lib = _lib.load()
+    code = _lib.OF3_DTYPE_BF16 if z.dtype is torch.bfloat16 else _lib.OF3_DTYPE_F32
+    need = lib.of3_pairformer_stack_workspace_bytes(code, len(arrays), B, N, c, ch, h, d, hid, c_s, h_s, d_s, hid_s)
+    if need < 0:
+        return None
+    table = (ctypes.POINTER(ctypes.c_void_p) * len(arrays))(*[ctypes.cast(a, ctypes.POINTER(ctypes.c_void_p)) for a in arrays])
+    z_out = z4 if inplace else F3._out_like(z4)
+    s_out = s if inplace else torch.empty_like(s)
+    stream = F3._stream(z)
+    ws = F3._workspace(z.device, need, stream)
+    _call(lib.of3_pairformer_stack_fwd, "of3_pairformer_stack_fwd", z.device, table, len(arrays), s.data_ptr(), z4.data_ptr(),
+          _lib.strides3(z4.stride()[:3]), None if sm is None else sm.data_ptr(), mptr, mstr, s_out.data_ptr(),
+          z_out.data_ptr(), B, N, c, ch, h, d, hid, c_s, h_s, d_s, hid_s, float(inf), float(inf_s),
+          0 if mask_trans else _lib.OF3_BLOCK_TRANSITION_UNMASKED, ws.data_ptr(), ws.numel(), code, stream,
+          _side_stream(z.device, stream))
     return s_out, z if inplace else z_out.view(z.shape)

@@ -87,6 +87,10 @@ class PairFormerStack(nn.Module):
                 use_cueq_triangle_kernels=False, use_lma=False, inplace_safe: bool = False, _mask_trans: bool = True):
         """s [*, N, C_s], z [*, N, N, C_z], single_mask [*, N], pair_mask [*, N, N] -> (s, z)
         (pairformer.py:398-470)."""
+        done = _block.run_pairformer_stack(self.blocks, PairFormerBlock, PairBlock, s, z, single_mask, pair_mask, inplace_safe,
+                                           _mask_trans)
+        if done is not None:
+            return done
         for i, blk in enumerate(self.blocks):
             # after the first block both tensors belong to this call
             s, z = blk(s, z, single_mask, pair_mask, inplace_safe=inplace_safe or i > 0, _mask_trans=_mask_trans)

@@ -110,3 +110,48 @@ def test_pair_stack_without_mask(monkeypatch):
     z = torch.randn(1, 21, 21, 128, generator=torch.Generator().manual_seed(8)).to(DEV).to(torch.bfloat16)
     want = _by_modules(monkeypatch, lambda: m(z, None))
     assert torch.equal(m(z, None), want) and calls == ["of3_pair_block_fwd"]
+
+
+@pytest.mark.parametrize("dtype,n,no_blocks", [(torch.bfloat16, 40, 1), (torch.bfloat16, 37, 2), (torch.bfloat16, 200, 3), (torch.bfloat16, 24, 9),
+                                               (torch.float32, 33, 5)])
+def test_pairformer_stack(monkeypatch, dtype, n, no_blocks):
+    """A stack's call, its single representation on a second stream, against its blocks one by one; again under a capture."""
+    lib()
+    calls = _count(monkeypatch)
+    m = _fill(of3pair.PairFormerStack(384, 128, 24, 16, 128, 32, 4, no_blocks=no_blocks), 11).to(DEV).to(dtype).eval()
+    gen = torch.Generator().manual_seed(12)
+    s, z = torch.randn(1, n, 384, generator=gen).to(DEV).to(dtype), torch.randn(1, n, n, 128, generator=gen).to(DEV).to(dtype)
+    tok = (torch.rand(1, n, generator=gen) > 0.2).float().to(DEV)
+    pair = tok[:, :, None] * tok[:, None, :]
+    want = (s, z)
+    for blk in m.blocks:
+        want = blk(*want, tok, pair)
+    del calls[:]
+    for _ in range(3):
+        got = m(s, z, tok, pair)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    a, b = s.clone(), z.clone()
+    m(a, b, tok, pair, inplace_safe=True)
+    assert torch.equal(a, want[0]) and torch.equal(b, want[1])
+    assert calls == ["of3_pairformer_stack_fwd"] * 4
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(other):
+        got = m(s, z, tok, pair)
+    torch.cuda.current_stream().wait_stream(other)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = m(s, z, tok, pair)
+    for _ in range(3):
+        out[0].zero_(), out[1].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], want[0]) and torch.equal(out[1], want[1])
+        m(s, z, tok, pair)
+    # blocks of other widths than the first, or a hook on one: block by block
+    if no_blocks > 1:
+        handle = m.blocks[1].register_forward_hook(lambda *args: None)
+        got = m(s, z, tok, pair)
+        assert torch.equal(got[0], want[0]) and calls[-1] == "of3_pairformer_block_fwd"
+        handle.remove()
