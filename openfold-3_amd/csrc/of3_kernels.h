@@ -98,7 +98,7 @@ hipError_t triattn_out_panels_launch(const TriattnOutArgs& args, int C, hipStrea
 
 // Copies of bf16 weight matrices in MFMA operand order (weight_pack.hip): rows and K multiples of 32 and 16
 struct PackJobs {
-  static constexpr int kBlock = 22, kMax = 4 * kBlock;  // a pair block: 2 x 6 + 2 x 5
+  static constexpr int kBlock = 25, kMax = 4 * kBlock;  // a pair block: 2 x 6 + 2 x 5 + 3
   const bf16_t* src[kMax];
   bf16_t* dst[kMax];
   int K[kMax];
@@ -119,8 +119,12 @@ struct TransitionArgs {
   int add_residual;
   int R;                      // rows per batch element (N for a pair tensor taken row by row; 1 when the
                               // caller hands a contiguous tensor over as one row of N*N positions)
+  const bf16_t* operands[3] = {};  // w_a, w_b, w_out in MFMA operand order, where a block's call has made them
 };
 hipError_t transition_launch(const TransitionArgs& args, int C, hipStream_t stream);
+// tiles of 32 or 64 positions (position_tiles 1 or 2), HID a multiple of 128
+// (transition_tiles_bf16.hip)
+hipError_t transition_tiles_launch(const TransitionArgs& args, int C, int position_tiles, hipStream_t stream);
 
 struct PairBiasArgs {
   const bf16_t* z;            // pair tensor, z_view addressing

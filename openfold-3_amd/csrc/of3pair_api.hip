@@ -571,7 +571,8 @@ int of3_transition_fwd(const void* x, const int64_t x_strides[3], const float* m
                                add_residual, nullptr, 0, dtype, stream);
 }
 
-static int transition_fwd(const of3::WeightX3* presplit, const void* x, const int64_t x_strides[3], const float* mask,
+// presplit as above; operands: w_a, w_b, w_out in MFMA operand order (bf16), or null
+static int transition_fwd(const of3::WeightX3* presplit, const void* const* operands, const void* x, const int64_t x_strides[3], const float* mask,
                           const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_a, const void* w_b, const void* w_out,
                           void* out, int64_t B, int64_t N, int64_t C, int64_t HID, int add_residual, void* workspace,
                           int64_t workspace_bytes, int dtype, void* stream) {
@@ -643,6 +644,7 @@ static int transition_fwd(const of3::WeightX3* presplit, const void* x, const in
   args.R = (int)rows;
   args.HID = (int)HID;
   args.add_residual = add_residual ? 1 : 0;
+  for (int i = 0; i < 3 && operands; ++i) args.operands[i] = bf(operands[i]);
   hipError_t e = of3::transition_launch(args, (int)C, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
@@ -651,7 +653,7 @@ int of3_transition_fwd_ws(const void* x, const int64_t x_strides[3], const float
                           const void* ln_w, const void* ln_b, const void* w_a, const void* w_b, const void* w_out,
                           void* out, int64_t B, int64_t N, int64_t C, int64_t HID, int add_residual, void* workspace,
                           int64_t workspace_bytes, int dtype, void* stream) {
-  return transition_fwd(nullptr, x, x_strides, mask, mask_strides, ln_w, ln_b, w_a, w_b, w_out, out, B, N, C, HID,
+  return transition_fwd(nullptr, nullptr, x, x_strides, mask, mask_strides, ln_w, ln_b, w_a, w_b, w_out, out, B, N, C, HID,
                         add_residual, workspace, workspace_bytes, dtype, stream);
 }
 
@@ -968,13 +970,15 @@ struct BlockDims {
   bool wide() const { return dtype == OF3_DTYPE_F32; }
   int weights() const { return OF3_PAIR_BLOCK_WEIGHTS - (HID == 0 ? 5 : 0); }
   int64_t prepared_bytes() const {
-    return wide() ? block_split_bytes(C, CH, H, D, HID) : align256(2 * 2 * (4 * CH * C + C * C + C * CH + 5 * H * D * C));
+    return wide() ? block_split_bytes(C, CH, H, D, HID)
+                  : align256(2 * (2 * (4 * CH * C + C * C + C * CH + 5 * H * D * C) + 3 * C * HID));
   }
 };
 struct BlockWeights {
   const void* w[OF3_PAIR_BLOCK_WEIGHTS];
   of3::WeightX3 split[of3::SplitJobs::kBlock];
   const of3::WeightX3 *mul, *att, *tr;
+  const void* tr_operands[3];  // bf16 transition, beside w
   int packed;
 };
 
@@ -1032,15 +1036,16 @@ static hipError_t prepare_blocks(const void* const* const* weights, int n, const
     o.packed = 1;
     o.mul = o.att = o.tr = nullptr;
     of3::bf16_t* to = reinterpret_cast<of3::bf16_t*>(static_cast<char*>(dst) + q * k.prepared_bytes());
-    auto add = [&](int i, int64_t rows, int64_t K) {
+    auto add_to = [&](const void*& packed, int i, int64_t rows, int64_t K) {
       const int m = jobs.n++;
       jobs.src[m] = bf(o.w[i]);
       jobs.dst[m] = to;
       jobs.K[m] = (int)K;
       jobs.first[m + 1] = jobs.first[m] + (int)(rows * K / 8);
-      o.w[i] = to;
+      packed = to;
       to += rows * K;
     };
+    auto add = [&](int i, int64_t rows, int64_t K) { add_to(o.w[i], i, rows, K); };
     for (int d = 0; d < 2; ++d) {
       for (int i = 4; i < 8; ++i) add(10 * d + i, CH, C);
       add(10 * d + 8, C, C);
@@ -1050,6 +1055,9 @@ static hipError_t prepare_blocks(const void* const* const* weights, int n, const
       for (int i = 3; i < 7; ++i) add(20 + 8 * d + i, HD, C);
       add(20 + 8 * d + 7, C, HD);
     }
+    for (int i = 0; i < 3; ++i) o.tr_operands[i] = nullptr;
+    if (k.HID)
+      for (int i = 0; i < 3; ++i) add_to(o.tr_operands[i], 38 + i, i < 2 ? k.HID : C, i < 2 ? C : k.HID);
   }
   return of3::pack_weights_launch(jobs, stream);
 }
@@ -1083,7 +1091,7 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
       st = (part == 0) == !(flags & OF3_BLOCK_ATTENTION_FIRST) ? trimul(m) : triattn(m);
   if (st != OF3_OK || d.HID == 0) return st;
   const void* const* w = k.w + 36;
-  return transition_fwd(k.tr, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask, mask_strides, w[0], w[1],
+  return transition_fwd(k.tr, d.wide() ? nullptr : k.tr_operands, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask, mask_strides, w[0], w[1],
                         w[2], w[3], w[4], out, d.B, d.N, d.C, d.HID, 1, d.wide() ? workspace : nullptr,
                         d.wide() ? workspace_bytes : 0, d.dtype, stream);
 }

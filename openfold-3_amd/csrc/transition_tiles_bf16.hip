@@ -1,0 +1,222 @@
+// bf16 pair transition (transition.hip has the operation and its rounding points) on tiles of 32 or 64 positions, for
+// short sequences.
+//
+// transition.hip gives a wave 32 positions and the whole hidden dimension: 256 positions per work-group and about 24 us
+// for one of them, whether a call has seven of them (40 tokens) or one for every CU.  Here the eight waves of a
+// work-group share a tile's hidden dimension, a wave to each tile of 32 hidden channels of a slice of 32 S; the hidden
+// activations go through LDS (double buffered, one barrier per slice), and a wave owns one 32-channel tile of the
+// output.  The sums run over the hidden channels in the same order and groups as there: the results are the same bits.
+// The weights come from L2 for every tile (384 KB at C = 128, n = 4, as long as its products on 64 positions), requested
+// one slice ahead.
+#include "of3_device.h"
+#include "of3_kernels.h"
+#include "of3_launch.h"
+#include "of3_pass_bf16.h"
+
+namespace of3 {
+
+namespace {
+
+using namespace pass_bf16;
+
+constexpr int kWaves = 8;
+
+// S hidden tiles per slice, P tiles of 32 positions per work-group
+template <int C, int S, int P>
+constexpr size_t lds_slots() {
+  return (size_t)P * (2 * PanelTile<C, false>::SLOTS + 2 * 32 * 4 * S);
+}
+
+template <int C, int S, int P>
+__global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p, int packed, int tiles_per_row, int total) {
+  typedef PanelTile<C, false> XTile;
+  constexpr int KS = C / 16, OT = C / 32, HCH = 4 * S;  // 16-byte chunks of a position's hidden slice
+  constexpr int TASKS = P * 32 / LnLane<C>::PPI;        // LayerNorm instructions of a tile
+  constexpr int LPW = (TASKS + kWaves - 1) / kWaves;
+  // first product: hidden tile of the wave and the position tiles it covers; second: output and position tile
+  constexpr int APT = S == 8 ? P : 1;
+  static_assert(S == 8 || S == 4, "");
+  extern __shared__ u32x4_t lds[];
+  u32x4_t* const xn = lds;                             // [P][XTile::SLOTS] LayerNorm(x)
+  u32x4_t* const xr = xn + P * XTile::SLOTS;           // x as loaded: the residual
+  u32x4_t* const hid = xr + P * XTile::SLOTS;          // [2][P][32 * HCH]
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int ht = wave % S, pt_a = S == 8 ? 0 : wave / S;
+  const int ot = wave % OT, pt_b = wave / OT;
+  const bool first = pt_a < P, second = pt_b < P;  // wave-uniform
+  const int L = p.N, slices = p.HID / (32 * S);
+  const LnLane<C> ln = ln_lane<C>(p.ln_w, p.ln_b, lane);
+  const int arow = rowperm16(lane & 31), half = lane >> 5;
+
+  auto hid_slot = [](int pos, int chunk) { return pos * HCH + (chunk ^ (pos & 15)); };
+  auto place = [&](int id, int& b, int& i) {
+    const int per_b = p.R * tiles_per_row;
+    b = id / per_b;
+    const int rem = id - b * per_b;
+    i = rem / tiles_per_row;
+    return (rem - i * tiles_per_row) * 32 * P;
+  };
+  u32x4_t raw[LPW];
+  float mval = 1.f;
+  auto load_tile = [&](int id) {
+    const int ln_chunk = ln.chunk(), ln_pos = ln.pos();
+    int b, i;
+    const int j0 = place(id, b, i);
+    const bf16_t* row = p.x + b * p.x_view.stride_b + i * p.x_view.stride_r + 8 * ln_chunk;
+#pragma unroll
+    for (int u = 0; u < LPW; ++u) {
+      const int task = wave + kWaves * u;
+      int j = j0 + (task < TASKS ? task : 0) * ln.PPI + ln_pos;
+      j = j < L ? j : L - 1;
+      raw[u] = *reinterpret_cast<const u32x4_t*>(row + j * p.x_view.stride_k);
+    }
+    if (p.mask) {
+      int j = j0 + (second ? 32 * pt_b : 0) + lane_here().l32;
+      j = j < L ? j : L - 1;
+      mval = p.mask[b * p.mask_view.stride_b + i * p.mask_view.stride_r + j * p.mask_view.stride_k];
+    }
+  };
+  // operands of hidden tile t of Wa and Wb, and of the output tile's columns of a slice.  The second product's k-step s
+  // of a hidden tile takes hidden channels 16 lh + 8 s + (0 .. 7) of it, the order in which a lane holds them.
+  u32x4_t wa[KS], wb[KS], wo[2 * S];
+  auto load_first = [&](int slice) {
+    const int t = slice * S + ht;
+    load_unit<C>(p.w_a, t, arow, half, packed, wa);
+    load_unit<C>(p.w_b, t, arow, half, packed, wb);
+  };
+  auto load_second = [&](int slice) {
+    const bf16_t* base = packed ? p.w_out + (((ot * (p.HID / 16) + half) * 64) + arow) * 8 : p.w_out + (32 * ot + arow) * p.HID + 16 * half;
+    const int step_t = packed ? 1024 : 32, step_s = packed ? 256 : 8;
+#pragma unroll
+    for (int t = 0; t < S; ++t)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) wo[2 * t + s] = *reinterpret_cast<const u32x4_t*>(base + (slice * S + t) * step_t + s * step_s);
+  };
+
+  int id = blockIdx.x;
+  if (id >= total) return;
+  load_tile(id);
+  if (first) load_first(0);
+  for (; id < total; id += gridDim.x) {
+    int b, i;
+    const int j0 = place(id, b, i);
+#pragma unroll
+    for (int u = 0; u < LPW; ++u) {
+      const int task = wave + kWaves * u;
+      if (task < TASKS) {
+        const int pos = task * ln.PPI + ln.pos(), slot = (pos >> 5) * XTile::SLOTS + XTile::slot(pos & 31, ln.chunk());
+        xn[slot] = ln.template normalised<false>(raw[u]);
+        xr[slot] = raw[u];
+      }
+    }
+    const float mtile = p.mask ? mval : 1.f;
+    __syncthreads();
+    f32x16_t oacc = zero16();
+    for (int slice = 0; slice < slices; ++slice) {
+      u32x4_t* const h = hid + (slice & 1) * P * 32 * HCH;
+      const Lane at = lane_here();
+      const int l32 = at.l32, lh = at.lh;
+      if (second) load_second(slice);
+      if (first) {
+#pragma unroll
+        for (int q = 0; q < APT; ++q) {
+          const u32x4_t* x = xn + (pt_a + q) * XTile::SLOTS;
+          f32x16_t ca = zero16(), cb = zero16();
+#pragma unroll
+          for (int s = 0; s < KS; ++s) {
+            const u32x4_t xb = x[XTile::slot(l32, 2 * s + lh)];
+            ca = mfma_32x32x16(wa[s], xb, ca);
+            cb = mfma_32x32x16(wb[s], xb, cb);
+          }
+          float hv[16];
+#pragma unroll
+          for (int e = 0; e < 16; ++e) hv[e] = ca[e] * fast_rcp(1.f + fast_exp2(-kLog2e * ca[e])) * cb[e];
+          u32x4_t* dst = h + (pt_a + q) * 32 * HCH;
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+            u32x4_t o;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o[v] = pack_bf16(hv[8 * s + 2 * v], hv[8 * s + 2 * v + 1]);
+            dst[hid_slot(l32, 4 * ht + 2 * lh + s)] = o;
+          }
+        }
+      }
+      __syncthreads();  // the slice is complete, and nobody reads the one before any more
+      if (first) load_first(slice + 1 < slices ? slice + 1 : 0);
+      if (slice + 1 == slices) load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
+      if (second) {
+        const u32x4_t* src = h + pt_b * 32 * HCH;
+#pragma unroll
+        for (int t = 0; t < S; ++t)
+#pragma unroll
+          for (int s = 0; s < 2; ++s) oacc = mfma_32x32x16(wo[2 * t + s], src[hid_slot(l32, 4 * t + 2 * lh + s)], oacc);
+      }
+    }
+    if (second) {
+      const Lane at = lane_here();
+      const int l32 = at.l32, lh = at.lh, j = j0 + 32 * pt_b + l32;
+      const u32x4_t* res = xr + pt_b * XTile::SLOTS;
+      float r0[8], r1[8];
+      unpack8(res[XTile::slot(l32, 4 * ot + 2 * lh)], r0);
+      unpack8(res[XTile::slot(l32, 4 * ot + 2 * lh + 1)], r1);
+      if (!p.add_residual) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r0[e] = r1[e] = 0.f;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        r0[e] += oacc[e] * mtile;
+        r1[e] += oacc[8 + e] * mtile;
+      }
+      if (j < L) {
+        bf16_t* dst = p.out + b * p.x_view.stride_b + i * p.x_view.stride_r + j * p.x_view.stride_k + 32 * ot + 16 * lh;
+        *reinterpret_cast<u32x4_t*>(dst) = pack8(r0);
+        *reinterpret_cast<u32x4_t*>(dst + 8) = pack8(r1);
+      }
+    }
+    __syncthreads();  // both tiles of x are rewritten by the next one
+  }
+}
+
+template <int C, int S, int P>
+hipError_t launch(const TransitionArgs& a, hipStream_t stream) {
+  constexpr size_t lds = lds_slots<C, S, P>() * 16;
+  static int cache[kMaxDevices];
+  int fit = 0;
+  hipError_t e = allow_dynamic_lds<transition_tiles<C, S, P>>(lds);
+  if (e == hipSuccess)
+    e = per_device(
+        cache,
+        [&](int dev, int* v) {
+          int cus = 0, per_cu = 0;
+          hipError_t s = cu_count(dev, &cus);
+          if (s == hipSuccess) s = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, transition_tiles<C, S, P>, 64 * kWaves, lds);
+          *v = cus * (per_cu > 0 ? per_cu : 1);
+          return s;
+        },
+        &fit);
+  if (e != hipSuccess) return e;
+  const int tiles_per_row = (a.N + 32 * P - 1) / (32 * P);
+  const long total = (long)a.B * a.R * tiles_per_row;
+  TransitionArgs k = a;
+  const int packed = a.operands[0] ? 1 : 0;
+  if (packed) k.w_a = a.operands[0], k.w_b = a.operands[1], k.w_out = a.operands[2];
+  hipLaunchKernelGGL((transition_tiles<C, S, P>), dim3((unsigned)(total < fit ? total : fit)), dim3(64 * kWaves), lds, stream, k,
+                     packed, tiles_per_row, (int)total);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t transition_tiles_launch(const TransitionArgs& a, int C, int position_tiles, hipStream_t stream) {
+  const bool one = position_tiles == 1;
+  if (a.HID % 256 == 0) {
+    if (C == 128) return one ? launch<128, 8, 1>(a, stream) : launch<128, 8, 2>(a, stream);
+    return one ? launch<64, 8, 1>(a, stream) : launch<64, 8, 2>(a, stream);
+  }
+  if (C == 128) return one ? launch<128, 4, 1>(a, stream) : launch<128, 4, 2>(a, stream);
+  return one ? launch<64, 4, 1>(a, stream) : launch<64, 4, 2>(a, stream);
+}
+
+}  // namespace of3

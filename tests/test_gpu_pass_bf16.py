@@ -5,6 +5,7 @@ import torch
 
 import test_gpu_stages as stages
 import test_gpu_block_call as blocks
+import test_gpu_transition as transition
 from gpu_util import lib  # noqa: F401
 
 import of3pair
@@ -33,3 +34,9 @@ def test_packed_weights(monkeypatch, c, d, n):
     mask = (torch.rand(1, n, n, generator=gen) > 0.2).float().to("cuda")
     want = blocks._by_modules(monkeypatch, lambda: m(z, mask))
     assert torch.equal(m(z, mask), want)
+
+
+@pytest.mark.parametrize("c,n_mult", [(128, 4), (128, 1), (128, 3), (64, 2), (64, 4)])
+@pytest.mark.parametrize("n,batch", [(2, 1), (7, 2), (33, 1), (64, 2), (90, 2), (91, 1), (141, 1)])
+def test_transition_tiles(c, n_mult, n, batch):
+    transition.test_transition_module(c, n_mult, n, (batch,))
