@@ -1334,8 +1334,13 @@ __global__ __launch_bounds__(kThreads * PT) void triattn_out_x3_f32(TriattnF32 p
 }
 
 // Attention core on split operands, head width 16 * STEPS (32 or 16; the narrow head leaves half of the
-// O^T tile's rows unused).  Work-group = 8 waves = 4 consecutive rows i x 2
-// halves of one (head, 128-query range); a wave owns 64 queries (two 32-query tiles) of one row.
+// O^T tile's rows unused).  Work-group = 4 waves = 2 consecutive rows i x 2
+// halves of one (head, 128-query range); a wave owns 64 queries (two 32-query tiles) of one row.  Two
+// work-groups share a CU, with exactly its 160 KB of LDS: a wave of each on every SIMD, so that the products of
+// one run under the exponentials and splits of the other (the barrier of a key tile holds the waves of a
+// work-group in the same phase).  They take turns better than the 8 waves of one work-group with four rows did,
+// although the bias slice is brought in for half as many rows: us per launch 10.8 -> 7.6 at N = 64, 243 -> 197 at
+// 384, 1560 -> 1443 at 768 (at 6 products a rate of 0.97 PFLOP/s), 119 -> 98 for three tensors of 200 with heads of 16.
 //   S^T = K Q^T  (rows = keys, columns = queries), six bf16 products per k-step, started from the
 //                triangle bias (the accumulator is loaded with it; logits stay in natural units, not
 //                pre-multiplied by log2(e): a row of masked keys has to lose its logits against -1e9 at
@@ -1344,7 +1349,7 @@ __global__ __launch_bounds__(kThreads * PT) void triattn_out_x3_f32(TriattnF32 p
 //                three bf16 terms, B = [1, 1, 1, 0 ...], taken only by tiles with a masked or padded key
 //   O^T = V^T P^T, the weights split in registers straight from the S^T accumulator into B operands
 // Per 32-key tile the work-group brings in the bias slice of its query range (it does not depend on
-// i: shared by the four rows) and each row's K and V^T operands (shared by the row's two waves) with
+// i: shared by its rows) and each row's K and V^T operands (shared by the row's two waves) with
 // direct-to-LDS buffer loads, one tile ahead, into double buffers: no registers are held for data in
 // flight, and the only wait is one vmcnt(0) + barrier per key tile, a whole tile of arithmetic after
 // the loads were issued.  The bias slice is XOR-swizzled on the global side (a lane picks which
@@ -1352,13 +1357,13 @@ __global__ __launch_bounds__(kThreads * PT) void triattn_out_x3_f32(TriattnF32 p
 // the offset 0 for every query that leaves out key tiles whose keys are all masked or padded, and a
 // second pass with running maxima for the work-groups whose row sums say the first was not exact;
 // keys past N carry a mask bias of -inf.
-constexpr int kXRows = 4;
+constexpr int kXRows = 2;
 constexpr int kXTbSlots = 128 * 8;                     // bias slice [128 queries][32 keys] fp32 in 16-byte slots
 constexpr int kXKvSlots = 12 * 64;                     // K step 0, 1 (h m l each), then V^T step 0, 1
 constexpr size_t kCoreX3Lds = (size_t)(2 * kXTbSlots + 2 * kXRows * kXKvSlots) * 16;
 
 template <int STEPS>
-__global__ __launch_bounds__(512) void triattn_core_x3_f32(TriattnF32 p, int n_qc, int n_rg, int total, int per_xcd) {
+__global__ __launch_bounds__(128 * kXRows, 2) void triattn_core_x3_f32(TriattnF32 p, int n_qc, int n_rg, int total, int per_xcd) {
   constexpr int QT = 2, D = 16 * STEPS;
   extern __shared__ u32x4_t lds4[];
   u32x4_t* tb_lds = lds4;                   // [2][kXTbSlots]
@@ -1392,12 +1397,13 @@ __global__ __launch_bounds__(512) void triattn_core_x3_f32(TriattnF32 p, int n_q
       for (int pl = 0; pl < 3; ++pl) qop[qt][st][pl] = Q[pl * plane + (jt * STEPS + st) * 64];
   }
 
-  // bias slice: instruction n of wave w fills slots 64 (2 w + n) .. + 63; slot t holds chunk
+  // bias slice: instruction n of wave w fills slots 64 (kTb w + n) .. + 63; slot t holds chunk
   // (t & 7) ^ ((q >> 1) & 7) of query q = t >> 3 of the work-group's range
-  uint32_t tb_off[2];
+  constexpr int kTb = kXTbSlots / (64 * 2 * kXRows);
+  uint32_t tb_off[kTb];
 #pragma unroll
-  for (int n = 0; n < 2; ++n) {
-    const int t = 64 * (2 * wave + n) + lane;
+  for (int n = 0; n < kTb; ++n) {
+    const int t = 64 * (kTb * wave + n) + lane;
     const int qloc = t >> 3, chunk = (t & 7) ^ ((qloc >> 1) & 7);
     int qrow = qc * 128 + qloc;
     qrow = qrow < N ? qrow : N - 1;
@@ -1415,10 +1421,10 @@ __global__ __launch_bounds__(512) void triattn_core_x3_f32(TriattnF32 p, int n_q
   const uint32_t lane_off = lane * 16;
   u32x4_t* kv_row = kv_lds + row * (2 * kXKvSlots);
   auto issue_loads = [&](int kt, int buf) {  // buf is a constant at every call site
-    u32x4_t* tdst = tb_lds + buf * kXTbSlots + 128 * wave;
+    u32x4_t* tdst = tb_lds + buf * kXTbSlots + 64 * kTb * wave;
     u32x4_t* kdst = kv_row + buf * kXKvSlots + 6 * 64 * qh;
 #pragma unroll
-    for (int n = 0; n < 2; ++n)
+    for (int n = 0; n < kTb; ++n)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(tb_rsrc, (void OF3_LDS_AS*)(tdst + 64 * n), 16, tb_off[n],
                                                kt * (32 * (int)sizeof(float)), 0, 0);
 #pragma unroll
@@ -1578,7 +1584,19 @@ __global__ __launch_bounds__(512) void triattn_core_x3_f32(TriattnF32 p, int n_q
       const bool in_range = l_tot[qt] >= 0x1p-60f && l_tot[qt] <= 0x1p60f;  // false for NaN too
       bad |= row_valid && (q0 + 32 * qt + l32 < N) && !in_range;
     }
-    if (__syncthreads_or(bad)) pass(std::true_type{});
+    // the vote goes through the bias buffers (no LDS beyond kCoreX3Lds: two work-groups fill a CU's exactly)
+    uint32_t* votes = reinterpret_cast<uint32_t*>(lds4);
+    __syncthreads();
+    const uint32_t wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+    if (lane == 0) votes[wave] = wave_bad;
+    __syncthreads();
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < 2 * kXRows; ++w) any |= votes[w];
+    if (any) {
+      __syncthreads();  // every wave has read the votes before loads land on them
+      pass(std::true_type{});
+    }
   }
 
   if (row_valid) {
@@ -2402,7 +2420,7 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
     const long total = (long)n_qc * n_rg * a.B * a.H;
     if (total > 0x7fffffffL - 8) return hipErrorInvalidValue;
     const int per_xcd = (int)((total + 7) / 8);
-    hipLaunchKernelGGL(a.D == 32 ? triattn_core_x3_f32<2> : triattn_core_x3_f32<1>, dim3(per_xcd * 8), dim3(512), kCoreX3Lds,
+    hipLaunchKernelGGL(a.D == 32 ? triattn_core_x3_f32<2> : triattn_core_x3_f32<1>, dim3(per_xcd * 8), dim3(128 * kXRows), kCoreX3Lds,
                        stream, p, n_qc, n_rg, (int)total, per_xcd);
   } else {
     // any head width up to 64, in LDS rounded up to a multiple of 8
