@@ -375,8 +375,9 @@ __global__ __launch_bounds__(64 * kWaves) void transition_kernel(TransitionArgs 
   wait_vmcnt<0>();
 }
 
+// tiles of 256 positions: at most `limit` of them, from the first one on
 template <int C>
-hipError_t launch(const TransitionArgs& a, hipStream_t stream) {
+hipError_t launch(const TransitionArgs& a, long limit, hipStream_t stream) {
   auto kern = transition_kernel<C>;
   constexpr int smem = (kStagesW * 2 * 32 * (C / 8) + kStagesO * C * 4 + kWaves * 32 * (C / 8)) * 16;
   static int cache[kMaxDevices];
@@ -395,8 +396,9 @@ hipError_t launch(const TransitionArgs& a, hipStream_t stream) {
     return hipErrorInvalidValue;
   const int tiles_per_row = (a.N + 32 * kWaves - 1) / (32 * kWaves);
   if (a.R < 1) return hipErrorInvalidValue;
-  const long total = (long)a.B * a.R * tiles_per_row;
+  long total = (long)a.B * a.R * tiles_per_row;
   if (total > 0x7fffffffl) return hipErrorInvalidValue;
+  total = total < limit ? total : limit;
   const int grid = (int)(total < cus ? total : cus);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kWaves), smem, stream, a, tiles_per_row, (int)total);
   return hipGetLastError();
@@ -418,9 +420,31 @@ hipError_t transition_launch(const TransitionArgs& args, int C, hipStream_t stre
   const long panels = (long)args.B * args.R * ((args.N + 31) / 32);
   const long per_cu = args.operands[0] ? (C == 128 ? 3 : 4) : (C == 128 ? 2 : 1);
   if (args.HID % 128 == 0 && panels <= per_cu * cus) return transition_tiles_launch(args, C, panels <= cus ? 1 : 2, stream);
-  if (C == 128) return launch<128>(args, stream);
-  if (C == 64) return launch<64>(args, stream);
-  return hipErrorInvalidValue;
+  // A last round with few tiles takes as long as a full one (29 us at C = 128, n = 4).  Its positions, where they are the
+  // end of one flat batch element, go to the shorter tiles instead if those are done in one go (15 us at two 32-position
+  // tiles per CU, 18 at one with the weights as they are).  Two trunk blocks, us: N = 260 728 -> 709, 365 1087 -> 1069,
+  // 384 1105 -> 1092; nothing to see at the 14 rounds of N = 929 and at C = 64, whose rounds take 12 us.
+  const long per_row = ((long)args.N + 32 * kWaves - 1) / (32 * kWaves);
+  long whole = (long)args.B * args.R * per_row;
+  const long last = whole % cus;
+  const long rest = args.N - (per_row - last) * (32 * kWaves);  // positions of the last round
+  TransitionArgs tail = args;
+  const bool split = C == 128 && args.HID % 128 == 0 && whole > cus && whole <= 5l * cus && last > 0 && args.R == 1 &&
+                     last <= per_row && (rest + 31) / 32 <= (args.operands[0] ? 2 : 1) * (long)cus;
+  if (split) {
+    const int64_t row = (int64_t)(args.B - 1), first = args.N - rest;
+    tail.x += row * args.x_view.stride_b + first * args.x_view.stride_k;
+    tail.out += row * args.x_view.stride_b + first * args.x_view.stride_k;
+    if (args.mask) tail.mask += row * args.mask_view.stride_b + first * args.mask_view.stride_k;
+    tail.B = 1;
+    tail.N = (int)rest;
+    whole -= last;
+  }
+  hipError_t st = hipErrorInvalidValue;
+  if (C == 128) st = launch<128>(args, whole, stream);
+  if (C == 64) st = launch<64>(args, whole, stream);
+  if (st != hipSuccess || !split) return st;
+  return transition_tiles_launch(tail, C, (rest + 31) / 32 <= cus ? 1 : 2, stream);
 }
 
 }  // namespace of3

@@ -40,3 +40,29 @@ def test_packed_weights(monkeypatch, c, d, n):
 @pytest.mark.parametrize("n,batch", [(2, 1), (7, 2), (33, 1), (64, 2), (90, 2), (91, 1), (141, 1)])
 def test_transition_tiles(c, n_mult, n, batch):
     transition.test_transition_module(c, n_mult, n, (batch,))
+
+
+@pytest.mark.parametrize("n_mult", [1, 4])
+@pytest.mark.parametrize("n,batch", [(257, 1), (259, 1), (300, 1), (182, 2), (263, 2)])
+def test_transition_last_round(n_mult, n, batch):
+    """Whole rounds of 256-position tiles and their rest on shorter ones: the second element of a batch, a last tile that
+    is not full, and (300, and 256-position tiles in whole rows of another stride) calls that stay in one piece.  The same
+    bits as the rows of the tensor one by one."""
+    lib()
+    gen = torch.Generator().manual_seed(n)
+    m = blocks._fill(of3pair.layers.SwiGLUTransition(128, n_mult), n).to("cuda").to(torch.bfloat16).eval()
+    x = torch.randn(batch, n, n, 128, generator=gen).to("cuda").to(torch.bfloat16)
+    mask = (torch.rand(batch, n, n, generator=gen) > 0.2).float().to("cuda")
+    got = m(x, mask=mask)
+    wide = torch.zeros(batch, n, n + 1, 128, device="cuda", dtype=torch.bfloat16)
+    wide[:, :, :n] = x
+    assert torch.equal(got, m(wide[:, :, :n], mask=mask))
+    small = torch.zeros(1, 8, 8, 128, device="cuda", dtype=torch.bfloat16)
+    small.view(-1, 128)[:64] = x[-1, -1, -64:]
+    small_mask = mask[-1, -1, -64:].reshape(1, 8, 8)
+    assert torch.equal(got[-1, -1, -64:], m(small, mask=small_mask).view(-1, 128))
+
+
+def test_transition_last_round_packed(monkeypatch):
+    """The same inside a block's call (weights in operand order, two short tiles per CU)."""
+    blocks.test_pairformer_stack(monkeypatch, torch.bfloat16, 260, 1)
