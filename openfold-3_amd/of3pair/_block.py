@@ -217,8 +217,8 @@ def _gather(block, build, dtype):
     array = q.gather(dtype)
     if array is None:
         return None
-    for m in q.called:  # modules that the block would call: their hooks and their mode are theirs
-        if m.training or m._forward_hooks or m._forward_pre_hooks:
+    for m in q.called:  # modules that the block would call: their hooks, their mode and a forward of their own are theirs
+        if m.training or m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
             return None
     if _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks:
         return None
@@ -330,7 +330,7 @@ def run_pairformer_stack(blocks, block_type, pair_block_type, s, z, single_mask,
     """(s, z) after all blocks, or None when the single call does not serve them."""
     arrays, dims = [], None
     for block in blocks:
-        if type(block) is not block_type or block.training or block._forward_hooks or block._forward_pre_hooks:
+        if type(block) is not block_type or block.training or block._forward_hooks or block._forward_pre_hooks or "forward" in block.__dict__:
             return None
         found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
         if not found or (dims is not None and found[1] != dims):

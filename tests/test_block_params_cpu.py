@@ -1,0 +1,26 @@
+"""Which blocks the single call takes (of3pair._block): the choice reads parameters and modules only, no device."""
+import os
+import sys
+
+import torch
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "openfold-3_amd"))
+
+import of3pair  # noqa: E402
+from of3pair import _block  # noqa: E402
+from of3pair.pair_stack import PairBlock  # noqa: E402
+
+
+def _taken(block):
+    return _block._gather(block, lambda q: _block._pairformer_params(q, block, PairBlock), torch.float32) is not None
+
+
+def test_forward_of_a_submodules_own():
+    """A forward set on an instance (as wrappers that move weights between devices do) is what the block has to call."""
+    block = of3pair.PairFormerBlock(384, 128, 24, 16, 128, 32, 4).eval()
+    assert _taken(block)
+    for sub in (block.single_transition, block.attn_pair_bias, block.pair_stack, block.pair_stack.pair_transition):
+        sub.forward = sub.forward
+        assert not _taken(block)
+        del sub.forward
+        assert _taken(block)
