@@ -22,6 +22,7 @@ from . import _lib, layers
 from . import functional as F3
 
 _TRI_MUL = ("linear_a_p", "linear_a_g", "linear_b_p", "linear_b_g")
+_NORM = (torch.nn.LayerNorm,)
 _MULS = {
     layers.TriangleMultiplicationOutgoing: True, layers.TriangleMultiplicationIncoming: False,
     layers.FusedTriangleMultiplicationOutgoing: True, layers.FusedTriangleMultiplicationIncoming: False,
@@ -66,24 +67,35 @@ class _Params:
                 return False
         return True
 
-    def param(self, module, name, shape, optional=False, rows=(0,)):
+    def param(self, module, name, shape, optional=False):
         if name not in module._parameters:
             raise _Refused
-        for first in rows:
-            self.entries.append((len(self.refs), first))
+        self.entries.append((len(self.refs), 0))
         self.refs.append((module._parameters, name))
         self.shapes.append((shape, optional))
 
     def norm(self, module, name, c, optional_bias=False):
-        ln = self.child(module, name, (torch.nn.LayerNorm,))
+        ln = self.child(module, name, _NORM)
         self.param(ln, "weight", (c,))
-        self.param(ln, "bias", (c,), optional=optional_bias)
+        self.param(ln, "bias", (c,), optional_bias)
 
-    def linear(self, module, name, shape, bias=False):
-        lin = self.child(module, name, (torch.nn.Linear,))
-        self.param(lin, "weight", shape)
-        if bias:
-            self.param(lin, "bias", shape[:1])
+    def linears(self, module, names, shape, bias=False):
+        """Of several layers of one shape, written out: they are most of a block."""
+        children, links, entries, refs, shapes = module._modules, self.links, self.entries, self.refs, self.shapes
+        want = (shape, False)
+        for name in names:
+            lin = children.get(name)
+            if type(lin) is not torch.nn.Linear:
+                raise _Refused
+            links.append((children, name, lin))
+            own = lin._parameters
+            if "weight" not in own:
+                raise _Refused
+            entries.append((len(refs), 0))
+            refs.append((own, "weight"))
+            shapes.append(want)
+            if bias:
+                self.param(lin, "bias", shape[:1])
 
     def gather(self, dtype):
         """The pointer array, or None when a parameter is not a plain contiguous tensor of `dtype`."""
@@ -98,19 +110,13 @@ class _Params:
                 return None
         seen_ptrs, seen_dtype, array = self.last
         if seen_ptrs != ptrs or seen_dtype is not dtype:
-            array = (ctypes.c_void_p * len(self.entries))()
-            for i, (owner, name) in enumerate(self.refs):
-                shape, optional = self.shapes[i]
+            for (owner, name), (shape, optional) in zip(self.refs, self.shapes):
                 p = owner.get(name)
-                if p is None:
-                    if not optional:
-                        return None
-                elif tuple(p.shape) != shape:
+                if not optional if p is None else p.shape != shape:
                     return None
-            for i, (ref, row) in enumerate(self.entries):
-                shape = self.shapes[ref][0]
-                at = ptrs[ref] + row * (shape[1] if len(shape) > 1 else 1) * dtype.itemsize
-                array[i] = at or None
+            size = dtype.itemsize
+            at = [ptrs[ref] + (row * self.shapes[ref][0][1] * size if row else 0) or None for ref, row in self.entries]
+            array = (ctypes.c_void_p * len(at))(*at)
             self.last = (ptrs, dtype, array)
         return array
 
@@ -130,13 +136,12 @@ def _pair_params(q, block):
             n = len(q.refs)
             for name in ("linear_ab_p", "linear_ab_g"):
                 lin = q.child(m, name, (torch.nn.Linear,))
-                q.param(lin, "weight", (2 * ch, c), rows=())
-            q.entries += [(n, 0), (n + 1, 0), (n, ch), (n + 1, ch)]
+                q.param(lin, "weight", (2 * ch, c))
+            q.entries[-2:] = [(n, 0), (n + 1, 0), (n, ch), (n + 1, ch)]
         else:
-            for name in _TRI_MUL:
-                q.linear(m, name, (ch, c))
-        q.linear(m, "linear_g", (c, c))
-        q.linear(m, "linear_z", (c, ch))
+            q.linears(m, _TRI_MUL, (ch, c))
+        q.linears(m, ("linear_g",), (c, c))
+        q.linears(m, ("linear_z",), (c, ch))
     start, end = (q.child(block, n, (layers.TriangleAttention,)) for n in ("tri_att_start", "tri_att_end"))
     h, d, inf = start.no_heads, start.mha.c_hidden, start.inf
     for m in (start, end):
@@ -145,10 +150,9 @@ def _pair_params(q, block):
             raise _Refused
         q.attr(m, "no_heads", "inf")
         q.norm(m, "layer_norm", c)
-        q.linear(m, "linear_z", (h, c))
-        for name in ("linear_q", "linear_k", "linear_v", "linear_g"):
-            q.linear(mha, name, (h * d, c))
-        q.linear(mha, "linear_o", (c, h * d))
+        q.linears(m, ("linear_z",), (h, c))
+        q.linears(mha, ("linear_q", "linear_k", "linear_v", "linear_g"), (h * d, c))
+        q.linears(mha, ("linear_o",), (c, h * d))
     hid = 0
     if "pair_transition" in block._modules:
         hid = _transition_params(q, block, "pair_transition", c)
@@ -161,9 +165,8 @@ def _transition_params(q, block, name, c):
     hid = t.n * c
     q.norm(t, "layer_norm", c)
     sw = q.child(t, "swiglu", (layers._SwiGLUParams,))
-    q.linear(sw, "linear_a", (hid, c))
-    q.linear(sw, "linear_b", (hid, c))
-    q.linear(t, "linear_out", (c, hid))
+    q.linears(sw, ("linear_a", "linear_b"), (hid, c))
+    q.linears(t, ("linear_out",), (c, hid))
     return hid
 
 
@@ -180,12 +183,11 @@ def _pairformer_params(q, block, pair_block_type):
         raise _Refused
     q.attr(a, "no_heads", "inf")
     q.norm(a, "layer_norm_z", c_z, optional_bias=True)
-    q.linear(a, "linear_z", (h, c_z))
+    q.linears(a, ("linear_z",), (h, c_z))
     q.norm(a, "layer_norm_a", c_s)
-    q.linear(mha, "linear_q", (hd, c_s), bias=True)
-    for name in ("linear_k", "linear_v", "linear_g"):
-        q.linear(mha, name, (hd, c_s))
-    q.linear(mha, "linear_o", (c_s, hd))
+    q.linears(mha, ("linear_q",), (hd, c_s), bias=True)
+    q.linears(mha, ("linear_k", "linear_v", "linear_g"), (hd, c_s))
+    q.linears(mha, ("linear_o",), (c_s, hd))
     hid_s = _transition_params(q, block, "single_transition", c_s)
     return dims, (c_s, h, hd // h, hid_s, a.inf)
 
@@ -328,6 +330,10 @@ def _side_stream(device, stream):
 
 def run_pairformer_stack(blocks, block_type, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
     """(s, z) after all blocks, or None when the single call does not serve them."""
+    if any(block not in _plans for block in blocks):
+        # First call: finding the parameters takes some 100 us per block.  Block by block that passes beside the kernels of
+        # the blocks before (4 blocks at N = 200: 1350 us in place of 1640).
+        return None
     arrays, dims = [], None
     for block in blocks:
         if type(block) is not block_type or block.training or block._forward_hooks or block._forward_pre_hooks or "forward" in block.__dict__:
