@@ -37,7 +37,8 @@
 //    loads and barriers go on).  A row without any unmasked key (a padded token) thereby sits the first
 //    pass out, ends it with the row sum 0 and takes the pass with running maxima, which gives the
 //    reference's uniform average (padded tokens come in runs, so the four rows of a work-group mostly
-//    agree and few other rows are dragged into a second pass).
+//    agree and few other rows are dragged into a second pass); a glance at four of its keys sends it there
+//    without the first.
 //  * head width 16 leaves rows 16..31 of the V^T operand free: row 16 holds ones, so the PV product
 //    itself accumulates the row sum (of the bf16 weights it multiplies) and the 16 additions per tile go.
 #include "of3_device.h"
@@ -155,6 +156,14 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
   const float* tb = p.tbias + ((size_t)b * H + h) * N * Jp;
   const float* mb = p.mbias + ((size_t)b * N + i) * Jp;
   const int nkt = (N + 31) / 32;
+
+  // four keys of every row of the work-group (lane 4 r + c: key c of row r), read before anything else: below
+  float sample;
+  {
+    const int r = rg * kRows + ((lane >> 2) & 3), c = lane & 3;
+    const int key = c == 0 ? r : c == 1 ? 0 : c == 2 ? N >> 1 : N - 1;
+    sample = r < N ? p.mbias[((size_t)b * N + r) * Jp + key] : 0.f;
+  }
 
   u32x4_t qop[kRQ][KSQ];
 #pragma unroll
@@ -359,6 +368,11 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
   };
 
   const uint32_t mb_off = krow * sizeof(float);
+  float mb_next;
+  auto first_loads = [&]() {
+    mb_next = __uint_as_float(load_mb(0, mb_off));
+    issue_loads(0, 0);
+  };
   auto pass = [&](auto track) {
 #pragma unroll
     for (int rq = 0; rq < kRQ; ++rq) {
@@ -367,8 +381,6 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
       oacc[rq] = zero16();
       lsum[rq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-    float mb_next = __uint_as_float(load_mb(0, mb_off));
-    issue_loads(0, 0);
     auto step = [&](int kt, int buf) {  // buf is a constant at both call sites: LDS addresses are immediates
       wait_vmcnt<0>();               // this wave's loads of tile kt (and its mask-bias values) have landed ...
       __builtin_amdgcn_s_barrier();  // ... and everybody's; nobody reads tile kt-1's buffers any more
@@ -405,16 +417,29 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
   // row sum itself tells: 2^-60 <= sum <= 2^60 (an overflow leaves +inf in the sum, a row of masked
   // keys leaves 0).  If any query of the work-group fails that test, the whole work-group (its
   // loads and barriers are collective) runs the pass again with running maxima.
-  pass(std::false_type{});
-  {
+  // A work-group with a row whose sampled keys (its own token, the first, the middle and the last) are all masked is
+  // taken for one with a padded token, which fails that test for certain, and goes to the second pass at once; a wrong
+  // guess costs it the offsets' arithmetic and nothing else.  A launch that fits the chip at once lasts as long as its
+  // work-groups with padded rows, of a larger one they are a share: two trunk blocks at N = 384, 38 of them padded,
+  // 1073 -> 1040 us; one at N = 2048, 256 padded, 25.1 -> 23.9 ms; two templates of 187, 12 padded, 391 -> 374 us; without
+  // padding no difference (N = 768).
+  first_loads();
+  const uint64_t masked = __builtin_amdgcn_ballot_w64(sample < kMaskedBelow);
+  bool again = false;
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) again |= ((masked >> (4 * r)) & 15u) == 15u;  // the same in every wave of the work-group
+  if (!again) {
+    pass(std::false_type{});
     bool bad = false;
 #pragma unroll
     for (int rq = 0; rq < kRQ; ++rq) {
       const bool in_range = l_tot[rq] >= 0x1p-60f && l_tot[rq] <= 0x1p60f;  // false for NaN too
       bad |= row_valid && (q0 + 32 * rq + l32 < N) && !in_range;
     }
-    if (__syncthreads_or(bad)) pass(std::true_type{});
+    again = __syncthreads_or(bad);
+    if (again) first_loads();
   }
+  if (again) pass(std::true_type{});
 
   if (row_valid && 16 * lh < D) {
 #pragma unroll
