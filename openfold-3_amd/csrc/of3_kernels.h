@@ -67,6 +67,10 @@ struct TriattnProjArgs {
   int packed = 0;                     // w_q, w_k, w_v in MFMA operand order
 };
 hipError_t triattn_proj_launch(const TriattnProjArgs& args, int C, int D, hipStream_t stream);
+// both in one, the attention on what the output pass writes, in the same orientation (pair_pass_bf16.hip): up to one
+// 32-position tile per CU, where either pass runs on such tiles by itself
+hipError_t trimul_out_triattn_proj_serves(int B, int N, bool* serves);
+hipError_t trimul_out_triattn_proj_launch(const TrimulOutArgs& out, const TriattnProjArgs& proj, int C, int D, hipStream_t stream);
 
 struct TriattnFlashArgs {
   const bf16_t *q, *k, *vt;

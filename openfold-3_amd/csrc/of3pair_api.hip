@@ -242,7 +242,7 @@ int of3_trimul_contract(const void* a, const void* b, void* x, int64_t B, int64_
 static int trimul_out(int packed, const void* x, const void* z, const int64_t z_strides[3], void* out,
                       const void* ln_in_w, const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
                       const void* w_g, const void* w_z, int64_t B, int64_t N, int64_t C, int64_t CH, int add_residual,
-                      void* stream) {
+                      void* stream, of3::TrimulOutArgs* deferred = nullptr) {
   if (!trimul_dims_ok(B, N, C, CH) || !strides_ok(z_strides)) return OF3_EINVAL;
   const void* ptrs[] = {x, z, out, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_g, w_z};
   for (const void* p : ptrs)
@@ -263,6 +263,10 @@ static int trimul_out(int packed, const void* x, const void* z, const int64_t z_
   args.Np = (int)padded(N);
   args.add_residual = add_residual ? 1 : 0;
   args.packed = packed;
+  if (deferred) {
+    *deferred = args;
+    return OF3_OK;
+  }
   hipError_t e = of3::trimul_out_launch(args, (int)C, (int)CH, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
@@ -275,12 +279,13 @@ int of3_trimul_out(const void* x, const void* z, const int64_t z_strides[3], voi
 }
 
 // presplit: the fp32 weights as a block's call has split them, or null; packed: the bf16 weight matrices are copies in
-// MFMA operand order
+// MFMA operand order; deferred (bf16): the output pass is not launched but handed on, to the `before` of triattn_fwd
 static int trimul_fwd(const of3::WeightX3* presplit, int packed, const void* z, const int64_t z_strides[3], const float* mask,
                    const int64_t mask_strides[3], const void* ln_in_w, const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
                    const void* w_a_p, const void* w_a_g, const void* w_b_p, const void* w_b_g, const void* w_g,
                    const void* w_z, void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int outgoing,
-                   int add_residual, void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
+                   int add_residual, void* workspace, int64_t workspace_bytes, int dtype, void* stream,
+                   of3::TrimulOutArgs* deferred = nullptr) {
   if (dtype == OF3_DTYPE_F32) {
     if (!f32_trimul_dims_ok(B, N, C, CH) || !f32_strides_ok(z_strides) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
     const void* ptrs[] = {z, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_a_p, w_a_g, w_b_p, w_b_g, w_g, w_z, out};
@@ -339,7 +344,7 @@ static int trimul_fwd(const of3::WeightX3* presplit, int packed, const void* z, 
   st = of3_trimul_contract(a, b, x, B, N, CH, 0, stream);
   if (st != OF3_OK) return st;
   return trimul_out(packed, x, z, z_strides, out, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_g, w_z, B, N, C, CH,
-                        add_residual, stream);
+                        add_residual, stream, deferred);
 }
 
 int of3_trimul_fwd(const void* z, const int64_t z_strides[3], const float* mask, const int64_t mask_strides[3],
@@ -388,7 +393,8 @@ int64_t of3_triattn_workspace_bytes_for(int dtype, int64_t B, int64_t N, int64_t
 static int triattn_proj(int packed, const void* x, const int64_t x_strides[3], const float* mask,
                         const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_q,
                         const void* w_k, const void* w_v, const void* w_bias, void* q, void* k, void* vt, float* tbias,
-                        float* mbias, int64_t B, int64_t N, int64_t C, int64_t H, int64_t D, float inf, void* stream) {
+                        float* mbias, int64_t B, int64_t N, int64_t C, int64_t H, int64_t D, float inf, void* stream,
+                        const of3::TrimulOutArgs* before = nullptr) {
   if (!triattn_dims_ok(B, N, C, H, D) || !strides_ok(x_strides) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
   const void* ptrs[] = {x, ln_w, ln_b, w_q, w_k, w_v, w_bias, q, k, vt, tbias, mbias};
   for (const void* p : ptrs)
@@ -415,7 +421,9 @@ static int triattn_proj(int packed, const void* x, const int64_t x_strides[3], c
   args.H = (int)H;
   args.inf = inf;
   args.packed = packed;
-  hipError_t e = of3::triattn_proj_launch(args, (int)C, (int)D, static_cast<hipStream_t>(stream));
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  hipError_t e = before ? of3::trimul_out_triattn_proj_launch(*before, args, (int)C, (int)D, s)
+                        : of3::triattn_proj_launch(args, (int)C, (int)D, s);
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
@@ -483,7 +491,7 @@ static int triattn_fwd(const of3::WeightX3* presplit, int packed, const void* x,
                     const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_bias, const void* w_q, const void* w_k,
                     const void* w_v, const void* w_g, const void* w_o, void* out, int64_t B, int64_t N, int64_t C,
                     int64_t H, int64_t D, float inf, int add_residual, void* workspace, int64_t workspace_bytes,
-                    int dtype, void* stream) {
+                    int dtype, void* stream, const of3::TrimulOutArgs* before = nullptr) {
   if (dtype == OF3_DTYPE_F32) {
     if (!f32_triattn_dims_ok(B, N, C, H, D) || !f32_strides_ok(x_strides) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
     const void* ptrs[] = {x, ln_w, ln_b, w_bias, w_q, w_k, w_v, w_g, w_o, out};
@@ -541,7 +549,7 @@ static int triattn_fwd(const of3::WeightX3* presplit, int packed, const void* x,
   float* mbias = reinterpret_cast<float*>(ws + 3 * qkv + align256(B * H * N * Np * 4));
   void* o = ws + 3 * qkv + align256(B * H * N * Np * 4) + align256(B * N * Np * 4);
   int st = triattn_proj(packed, x, x_strides, mask, mask_strides, ln_w, ln_b, w_q, w_k, w_v, w_bias, q, k, vt, tbias,
-                            mbias, B, N, C, H, D, inf, stream);
+                            mbias, B, N, C, H, D, inf, stream, before);
   if (st != OF3_OK) return st;
   st = of3_triattn_flash(q, k, vt, tbias, mbias, o, B, N, H, D, stream);
   if (st != OF3_OK) return st;
@@ -946,12 +954,19 @@ static int64_t block_split_bytes(int64_t C, int64_t CH, int64_t H, int64_t D, in
   return align256((int64_t)(2 * of3::trimul_wsplit_bytes(C, CH) + 2 * of3::triattn_wsplit_bytes(C, H, D) +
                             (HID ? of3::transition_wsplit_bytes(C, HID) : 0)));
 }
+// Short bf16 sequences: the pass that ends a triangle multiplication and begins the attention after it reads the one's
+// workspace and writes the other's, so they lie side by side.  Whether a call takes that pass depends on the device, the room
+// does not: up to 1024 tiles of 32 positions.
+static bool shared_pass_room(int dtype, int64_t B, int64_t N) {
+  return dtype == OF3_DTYPE_BF16 && N <= 1024 && B <= 1024 && B * N * ((N + 31) / 32) <= 1024;
+}
 static int64_t pair_block_module_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
                                        int64_t HID) {
   int64_t need = of3_trimul_workspace_bytes_for(dtype, B, N, C, CH);
   const int64_t att = of3_triattn_workspace_bytes_for(dtype, B, N, C, H, D);
   if (need < 0 || att < 0) return OF3_EINVAL;
-  if (att > need) need = att;
+  if (shared_pass_room(dtype, B, N)) need += att;
+  else if (att > need) need = att;
   if (HID != 0) {
     if (dtype == OF3_DTYPE_BF16 && (HID < 128 || HID % 32 != 0 || HID > (1 << 16))) return OF3_EINVAL;
     const int64_t tr = of3_transition_workspace_bytes_for(dtype, B, N, C, HID);
@@ -1066,11 +1081,18 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
                           const float* mask, const int64_t mask_strides[3], void* out, int flags, void* workspace,
                           int64_t workspace_bytes, void* stream) {
   const void* src = z;  // the first module reads z, every later one updates out in place
+  bool shared = false;
+  if (!(flags & OF3_BLOCK_ATTENTION_FIRST) && shared_pass_room(d.dtype, d.B, d.N)) {
+    const hipError_t e = of3::trimul_out_triattn_proj_serves((int)d.B, (int)d.N, &shared);
+    if (e != hipSuccess) return fail_hip(e);
+  }
+  const int64_t skip = shared ? of3_trimul_workspace_bytes(d.B, d.N, d.C, d.CH) : 0;
+  of3::TrimulOutArgs between;
   auto trimul = [&](int m) {
     const void* const* w = k.w + 10 * m;
     const int st = trimul_fwd(k.mul ? k.mul + m * of3::kTrimulMatrices : nullptr, k.packed, src, z_strides, mask, mask_strides,
                               w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8], w[9], out, d.B, d.N, d.C, d.CH, m == 0,
-                              1, workspace, workspace_bytes, d.dtype, stream);
+                              1, workspace, workspace_bytes, d.dtype, stream, shared && m == 1 ? &between : nullptr);
     src = out;
     return st;
   };
@@ -1080,8 +1102,9 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
     int64_t mt[3] = {0, 0, 0};
     if (mask) mt[0] = mask_strides[0], mt[1] = mask_strides[m ? 2 : 1], mt[2] = mask_strides[m ? 1 : 2];
     const int st = triattn_fwd(k.att ? k.att + m * of3::kTriattnMatrices : nullptr, k.packed, src, zt, mask, mt, w[0], w[1],
-                               w[2], w[3], w[4], w[5], w[6], w[7], out, d.B, d.N, d.C, d.H, d.D, d.inf, 1, workspace,
-                               workspace_bytes, d.dtype, stream);
+                               w[2], w[3], w[4], w[5], w[6], w[7], out, d.B, d.N, d.C, d.H, d.D, d.inf, 1,
+                               static_cast<char*>(workspace) + skip, workspace_bytes - skip, d.dtype, stream,
+                               shared && m == 0 ? &between : nullptr);
     src = out;
     return st;
   };

@@ -66,3 +66,24 @@ def test_transition_last_round(n_mult, n, batch):
 def test_transition_last_round_packed(monkeypatch):
     """The same inside a block's call (weights in operand order, two short tiles per CU)."""
     blocks.test_pairformer_stack(monkeypatch, torch.bfloat16, 260, 1)
+
+
+@pytest.mark.parametrize("c,d", [(128, 32), (64, 16)])
+@pytest.mark.parametrize("n,batch,masked", [(1, 1, False), (2, 3, True), (31, 2, True), (32, 4, False), (33, 2, True), (64, 2, True),
+                                            (65, 1, False), (86, 1, True)])
+def test_shared_pass(monkeypatch, c, d, n, batch, masked):
+    """A block's call at the lengths where the triangle multiplication ends and the attention begins in one pass (and one
+    beyond): the bits of the modules, for batches, ragged panels, in place and on a transposed tensor."""
+    lib()
+    m = blocks._fill(of3pair.PairStack(c, c, d, 4), n).to("cuda").to(torch.bfloat16).eval()
+    gen = torch.Generator().manual_seed(n)
+    z = torch.randn(batch, n, n, c, generator=gen).to("cuda").to(torch.bfloat16)
+    mask = (torch.rand(batch, n, n, generator=gen) > 0.2).float().to("cuda") if masked else None
+    want = blocks._by_modules(monkeypatch, lambda: m(z, mask))
+    assert torch.isfinite(want.float()).all()
+    assert torch.equal(m(z, mask), want)
+    own = z.clone()
+    m(own, mask, inplace_safe=True)
+    assert torch.equal(own, want)
+    zt = z.transpose(1, 2).contiguous().transpose(1, 2)
+    assert torch.equal(m(zt, mask), want)
