@@ -126,7 +126,7 @@ struct TransitionArgs {
   const bf16_t* operands[3] = {};  // w_a, w_b, w_out in MFMA operand order, where a block's call has made them
 };
 hipError_t transition_launch(const TransitionArgs& args, int C, hipStream_t stream);
-// tiles of 32 or 64 positions (position_tiles 1 or 2), HID a multiple of 128
+// tiles of 32 * position_tiles positions (1 or 2; at C = 128 also 4 or 5), HID a multiple of 128
 // (transition_tiles_bf16.hip)
 hipError_t transition_tiles_launch(const TransitionArgs& args, int C, int position_tiles, hipStream_t stream);
 

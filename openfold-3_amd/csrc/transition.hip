@@ -411,15 +411,20 @@ hipError_t transition_launch(const TransitionArgs& args, int C, hipStream_t stre
   // Short sequences: the hidden dimension shared by a work-group's waves.  256 CUs, C = 128, n = 4, us, tiles of 256 / 64 / 32
   // positions: N = 40 28.1 / 12.9 / 9.3, 64 28.4 / 13.0 / 9.7, 96 29.1 / 13.6 / 15.3, 128 29.6 / 15.0 / 17.4, 160 31.0 / 25.0
   // / 29.1, 200 33.3 / 35.5 / 36.9; C = 64, n = 2, two tensors: N = 64 10.3 / 5.8 / 5.6, 96 10.7 / 8.7 / 10.2, 128 11.6 / 9.7
-  // / 13.3, 160 12.7 / 15.4 / 19.6.  32 positions up to one such tile per CU, 64 up to 3 (or, at 64 channels, 4) times that.
-  // Weights as they are (a module's own call) take longer to read: 18.2 us at N = 64, 23.7 at 128.
+  // / 13.3, 160 12.7 / 15.4 / 19.6.  32 positions up to one such tile per CU, 64 up to 2 (or, at 64 channels, 4) times that.
+  // Then one round of 128 positions up to 4 times, of 160 up to 5 times that (256 / 64 / 128 or 160 positions: N = 128
+  // 29.6 / 16.0 / 22.8, 150 - / 25.2 / 24.0, 157 31.4 / - / 24.1, 181 31.9 / - / 25.3, 190 32.2 / - / 26.7, 202 32.8 / - / 28.1).
+  // Weights as they are (a module's own call) take longer to read: 18.2 us at N = 64, 23.7 at 128, 35 with tiles of 128.
   static int cache[kMaxDevices];
   int cus = 0;
   const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
   if (e != hipSuccess) return e;
   const long panels = (long)args.B * args.R * ((args.N + 31) / 32);
-  const long per_cu = args.operands[0] ? (C == 128 ? 3 : 4) : (C == 128 ? 2 : 1);
-  if (args.HID % 128 == 0 && panels <= per_cu * cus) return transition_tiles_launch(args, C, panels <= cus ? 1 : 2, stream);
+  const long per_cu = args.operands[0] ? (C == 128 ? 5 : 4) : (C == 128 ? 2 : 1);
+  if (args.HID % 128 == 0 && panels <= per_cu * cus) {
+    const int tiles = panels <= cus ? 1 : (panels <= 2l * cus || C == 64 || !args.operands[0]) ? 2 : panels <= 4l * cus ? 4 : 5;
+    return transition_tiles_launch(args, C, tiles, stream);
+  }
   // A last round with few tiles takes as long as a full one (29 us at C = 128, n = 4).  Its positions, where they are the
   // end of one flat batch element, go to the shorter tiles instead if those are done in one go (15 us at two 32-position
   // tiles per CU, 18 at one with the weights as they are).  Two trunk blocks, us: N = 260 728 -> 709, 365 1087 -> 1069,

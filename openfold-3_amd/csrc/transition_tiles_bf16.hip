@@ -1,5 +1,5 @@
-// bf16 pair transition (transition.hip has the operation and its rounding points) on tiles of 32 or 64 positions, for
-// short sequences.
+// bf16 pair transition (transition.hip has the operation and its rounding points) on tiles of 32, 64, 128 or 160
+// positions, for short sequences.
 //
 // transition.hip gives a wave 32 positions and the whole hidden dimension: 256 positions per work-group and about 24 us
 // for one of them, whether a call has seven of them (40 tokens) or one for every CU.  Here the eight waves of a
@@ -8,6 +8,8 @@
 // output.  The sums run over the hidden channels in the same order and groups as there: the results are the same bits.
 // The weights come from L2 for every tile (384 KB at C = 128, n = 4, as long as its products on 64 positions), requested
 // one slice ahead.
+// The longer tiles are for the lengths at which one of them per CU is all there is to do: 24 us for 128 positions, 28 for
+// 160 (their hidden slices are of 128 channels, two or three position tiles to a wave; LDS has no room for more).
 #include "of3_device.h"
 #include "of3_kernels.h"
 #include "of3_launch.h"
@@ -21,7 +23,7 @@ using namespace pass_bf16;
 
 constexpr int kWaves = 8;
 
-// S hidden tiles per slice, P tiles of 32 positions per work-group
+// S hidden tiles per slice, P tiles of 32 positions per work-group (P = 5, S = 4, C = 128: all of the 160 KB)
 template <int C, int S, int P>
 constexpr size_t lds_slots() {
   return (size_t)P * (2 * PanelTile<C, false>::SLOTS + 2 * 32 * 4 * S);
@@ -34,7 +36,8 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
   constexpr int TASKS = P * 32 / LnLane<C>::PPI;        // LayerNorm instructions of a tile
   constexpr int LPW = (TASKS + kWaves - 1) / kWaves;
   // first product: hidden tile of the wave and the position tiles it covers; second: output and position tile
-  constexpr int APT = S == 8 ? P : 1;
+  // (tiles pt_a, pt_a + GA ... and pt_b, pt_b + GB ...; the two waves of a SIMD differ in pt_a and pt_b)
+  constexpr int GA = kWaves / S, GB = kWaves / OT, APT = (P + GA - 1) / GA, BPT = (P + GB - 1) / GB;
   static_assert(S == 8 || S == 4, "");
   extern __shared__ u32x4_t lds[];
   u32x4_t* const xn = lds;                             // [P][XTile::SLOTS] LayerNorm(x)
@@ -42,7 +45,7 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
   u32x4_t* const hid = xr + P * XTile::SLOTS;          // [2][P][32 * HCH]
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int ht = wave % S, pt_a = S == 8 ? 0 : wave / S;
+  const int ht = wave % S, pt_a = wave / S;
   const int ot = wave % OT, pt_b = wave / OT;
   const bool first = pt_a < P, second = pt_b < P;  // wave-uniform
   const int L = p.N, slices = p.HID / (32 * S);
@@ -58,7 +61,9 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
     return (rem - i * tiles_per_row) * 32 * P;
   };
   u32x4_t raw[LPW];
-  float mval = 1.f;
+  float mval[BPT];
+#pragma unroll
+  for (int q = 0; q < BPT; ++q) mval[q] = 1.f;
   auto load_tile = [&](int id) {
     const int ln_chunk = ln.chunk(), ln_pos = ln.pos();
     int b, i;
@@ -72,9 +77,12 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
       raw[u] = *reinterpret_cast<const u32x4_t*>(row + j * p.x_view.stride_k);
     }
     if (p.mask) {
-      int j = j0 + (second ? 32 * pt_b : 0) + lane_here().l32;
-      j = j < L ? j : L - 1;
-      mval = p.mask[b * p.mask_view.stride_b + i * p.mask_view.stride_r + j * p.mask_view.stride_k];
+#pragma unroll
+      for (int q = 0; q < BPT; ++q) {
+        int j = j0 + (second ? 32 * (pt_b + GB * q) : 0) + lane_here().l32;
+        j = j < L ? j : L - 1;
+        mval[q] = p.mask[b * p.mask_view.stride_b + i * p.mask_view.stride_r + j * p.mask_view.stride_k];
+      }
     }
   };
   // operands of hidden tile t of Wa and Wb, and of the output tile's columns of a slice.  The second product's k-step s
@@ -110,9 +118,11 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
         xr[slot] = raw[u];
       }
     }
-    const float mtile = p.mask ? mval : 1.f;
+    float mtile[BPT];
+    f32x16_t oacc[BPT];
+#pragma unroll
+    for (int q = 0; q < BPT; ++q) mtile[q] = mval[q], oacc[q] = zero16();
     __syncthreads();
-    f32x16_t oacc = zero16();
     for (int slice = 0; slice < slices; ++slice) {
       u32x4_t* const h = hid + (slice & 1) * P * 32 * HCH;
       const Lane at = lane_here();
@@ -121,7 +131,9 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
       if (first) {
 #pragma unroll
         for (int q = 0; q < APT; ++q) {
-          const u32x4_t* x = xn + (pt_a + q) * XTile::SLOTS;
+          const int pt = pt_a + GA * q;
+          if (P % GA != 0 && P > GA && pt >= P) break;  // wave-uniform
+          const u32x4_t* x = xn + pt * XTile::SLOTS;
           f32x16_t ca = zero16(), cb = zero16();
 #pragma unroll
           for (int s = 0; s < KS; ++s) {
@@ -132,7 +144,7 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
           float hv[16];
 #pragma unroll
           for (int e = 0; e < 16; ++e) hv[e] = ca[e] * fast_rcp(1.f + fast_exp2(-kLog2e * ca[e])) * cb[e];
-          u32x4_t* dst = h + (pt_a + q) * 32 * HCH;
+          u32x4_t* dst = h + pt * 32 * HCH;
 #pragma unroll
           for (int s = 0; s < 2; ++s) {
             u32x4_t o;
@@ -146,33 +158,43 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
       if (first) load_first(slice + 1 < slices ? slice + 1 : 0);
       if (slice + 1 == slices) load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
       if (second) {
-        const u32x4_t* src = h + pt_b * 32 * HCH;
 #pragma unroll
-        for (int t = 0; t < S; ++t)
+        for (int q = 0; q < BPT; ++q) {
+          const int pt = pt_b + GB * q;
+          if (P % GB != 0 && P > GB && pt >= P) break;  // wave-uniform
+          const u32x4_t* src = h + pt * 32 * HCH;
 #pragma unroll
-          for (int s = 0; s < 2; ++s) oacc = mfma_32x32x16(wo[2 * t + s], src[hid_slot(l32, 4 * t + 2 * lh + s)], oacc);
+          for (int t = 0; t < S; ++t)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) oacc[q] = mfma_32x32x16(wo[2 * t + s], src[hid_slot(l32, 4 * t + 2 * lh + s)], oacc[q]);
+        }
       }
     }
     if (second) {
-      const Lane at = lane_here();
-      const int l32 = at.l32, lh = at.lh, j = j0 + 32 * pt_b + l32;
-      const u32x4_t* res = xr + pt_b * XTile::SLOTS;
-      float r0[8], r1[8];
-      unpack8(res[XTile::slot(l32, 4 * ot + 2 * lh)], r0);
-      unpack8(res[XTile::slot(l32, 4 * ot + 2 * lh + 1)], r1);
-      if (!p.add_residual) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) r0[e] = r1[e] = 0.f;
-      }
+      for (int q = 0; q < BPT; ++q) {
+        const int pt = pt_b + GB * q;
+        if (P % GB != 0 && P > GB && pt >= P) break;  // wave-uniform
+        const Lane at = lane_here();
+        const int l32 = at.l32, lh = at.lh, j = j0 + 32 * pt + l32;
+        const u32x4_t* res = xr + pt * XTile::SLOTS;
+        float r0[8], r1[8];
+        unpack8(res[XTile::slot(l32, 4 * ot + 2 * lh)], r0);
+        unpack8(res[XTile::slot(l32, 4 * ot + 2 * lh + 1)], r1);
+        if (!p.add_residual) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        r0[e] += oacc[e] * mtile;
-        r1[e] += oacc[8 + e] * mtile;
-      }
-      if (j < L) {
-        bf16_t* dst = p.out + b * p.x_view.stride_b + i * p.x_view.stride_r + j * p.x_view.stride_k + 32 * ot + 16 * lh;
-        *reinterpret_cast<u32x4_t*>(dst) = pack8(r0);
-        *reinterpret_cast<u32x4_t*>(dst + 8) = pack8(r1);
+          for (int e = 0; e < 8; ++e) r0[e] = r1[e] = 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          r0[e] += oacc[q][e] * mtile[q];
+          r1[e] += oacc[q][8 + e] * mtile[q];
+        }
+        if (j < L) {
+          bf16_t* dst = p.out + b * p.x_view.stride_b + i * p.x_view.stride_r + j * p.x_view.stride_k + 32 * ot + 16 * lh;
+          *reinterpret_cast<u32x4_t*>(dst) = pack8(r0);
+          *reinterpret_cast<u32x4_t*>(dst + 8) = pack8(r1);
+        }
       }
     }
     __syncthreads();  // both tiles of x are rewritten by the next one
@@ -210,6 +232,10 @@ hipError_t launch(const TransitionArgs& a, hipStream_t stream) {
 }  // namespace
 
 hipError_t transition_tiles_launch(const TransitionArgs& a, int C, int position_tiles, hipStream_t stream) {
+  if (position_tiles > 2) {
+    if (C != 128) return hipErrorInvalidValue;
+    return position_tiles == 4 ? launch<128, 4, 4>(a, stream) : launch<128, 4, 5>(a, stream);
+  }
   const bool one = position_tiles == 1;
   if (a.HID % 256 == 0) {
     if (C == 128) return one ? launch<128, 8, 1>(a, stream) : launch<128, 8, 2>(a, stream);

@@ -87,3 +87,18 @@ def test_shared_pass(monkeypatch, c, d, n, batch, masked):
     assert torch.equal(own, want)
     zt = z.transpose(1, 2).contiguous().transpose(1, 2)
     assert torch.equal(m(zt, mask), want)
+
+
+@pytest.mark.parametrize("n_mult", [1, 4])
+@pytest.mark.parametrize("n,batch", [(129, 1), (150, 1), (104, 2), (181, 1), (182, 1), (202, 1), (203, 1)])
+def test_transition_long_tiles(monkeypatch, n_mult, n, batch):
+    """Inside a block's call: tiles of 128 positions up to four panels of 32 per CU, of 160 up to five, and one beyond
+    (256 CUs; 104: two elements, each with a tile that is not full)."""
+    lib()
+    m = blocks._fill(of3pair.PairBlock(128, 128, 32, 4, transition_n=n_mult), n).to("cuda").to(torch.bfloat16).eval()
+    gen = torch.Generator().manual_seed(n)
+    z = torch.randn(batch, n, n, 128, generator=gen).to("cuda").to(torch.bfloat16)
+    mask = (torch.rand(batch, n, n, generator=gen) > 0.2).float().to("cuda")
+    want = blocks._by_modules(monkeypatch, lambda: m(z, mask))
+    assert torch.isfinite(want.float()).all()
+    assert torch.equal(m(z, mask), want)
