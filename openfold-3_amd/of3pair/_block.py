@@ -192,7 +192,21 @@ def _pairformer_params(q, block, pair_block_type):
     return dims, (c_s, h, hd // h, hid_s, a.inf)
 
 
-_plans = weakref.WeakKeyDictionary()  # block -> (parameters, dimensions), or False where it is not served
+# block -> (parameters, dimensions), False where it is not served, or None: called once
+_plans = weakref.WeakKeyDictionary()
+# Token count from which a block's first call goes module by module and the parameters are looked for in the second: the
+# search takes 100 us or more before the first launch, and from here on issuing the modules keeps ahead of the GPU.
+# First pass of new weights, us, searched first / module by module: two trunk blocks at N = 384 1530 / 1330, four updates at
+# 768 2110 / 2020, one block at 929 4470 / 4260.
+_LATE_FROM = 300
+
+
+def _first_call(block, z):
+    """Whether this is the block's first call and starts without the search for its parameters."""
+    if z.dim() < 3 or z.shape[-2] < _LATE_FROM or block in _plans:
+        return False
+    _plans[block] = None
+    return True
 
 
 def _plan(block, build):
@@ -248,6 +262,8 @@ def _call(fn, what, device, *args):
 
 def run_pair_block(block, z, mask, inplace, attention_first=False, mask_trans=True):
     """z after the block's modules, or None when the single call does not serve it."""
+    if _first_call(block, z):
+        return None
     found = _gather(block, lambda q: _pair_params(q, block), z.dtype)
     args = found and _pair_args(z, mask)
     if not args:
@@ -286,6 +302,8 @@ def _pairformer_args(s, z, single_mask, pair_mask, c, c_s):
 
 def run_pairformer_block(block, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
     """(s, z) after the block, or None when the single call does not serve it."""
+    if _first_call(block, z):
+        return None
     found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
     if not found:
         return None
@@ -330,8 +348,8 @@ def _side_stream(device, stream):
 
 def run_pairformer_stack(blocks, block_type, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
     """(s, z) after all blocks, or None when the single call does not serve them."""
-    if any(block not in _plans for block in blocks):
-        # First call: finding the parameters takes some 100 us per block.  Block by block that passes beside the kernels of
+    if any(_plans.get(block) is None for block in blocks):
+        # First calls: finding the parameters takes some 100 us per block.  Block by block that passes beside the kernels of
         # the blocks before (4 blocks at N = 200: 1350 us in place of 1640).
         return None
     arrays, dims = [], None

@@ -24,3 +24,14 @@ def test_forward_of_a_submodules_own():
         assert not _taken(block)
         del sub.forward
         assert _taken(block)
+
+
+def test_first_call_of_a_long_sequence():
+    """Starts module by module, once; shorter ones do not, and a tensor that no module takes is left to them."""
+    block = of3pair.PairFormerBlock(384, 128, 24, 16, 128, 32, 4).eval()
+    n = _block._LATE_FROM
+    assert not _block._first_call(block, torch.empty(n - 1, n - 1, 1, device="meta"))
+    assert not _block._first_call(block, torch.empty(n))
+    assert _block._first_call(block, torch.empty(1, n, n, 1, device="meta"))
+    assert not _block._first_call(block, torch.empty(1, n, n, 1, device="meta"))
+    assert _taken(block)

@@ -155,3 +155,21 @@ def test_pairformer_stack(monkeypatch, dtype, n, no_blocks):
         got = m(s, z, tok, pair)
         assert torch.equal(got[0], want[0]) and calls[-1] == "of3_pairformer_block_fwd"
         handle.remove()
+
+
+def test_stack_captured_after_one_eager_call():
+    """The first call of a stack goes block by block, the second, under a capture, through the stack's own call."""
+    lib()
+    m = _fill(of3pair.PairFormerStack(384, 128, 24, 16, 128, 32, 4, no_blocks=2), 21).to(DEV).to(torch.bfloat16).eval()
+    gen = torch.Generator().manual_seed(22)
+    s, z = (torch.randn(*shape, generator=gen).to(DEV).to(torch.bfloat16) for shape in ((1, 45, 384), (1, 45, 45, 128)))
+    want = [t.clone() for t in m(s, z, None, None)]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = m(s, z, None, None)
+    for _ in range(3):
+        out[0].zero_(), out[1].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], want[0]) and torch.equal(out[1], want[1])
+        assert all(torch.equal(a, b) for a, b in zip(m(s, z, None, None), want))
