@@ -5,12 +5,12 @@
 //   triangle attention        triangular_attention.py:102-167, attention.py:94-135,265-302
 //   pair transition           transition.py:225-271, activations.py:33-61
 //   pair-bias projection      attention_pair_bias.py:151-161
-// These kernels are written for exactness and generality (any N, C, C_hidden <= 256, head
-// width <= 64) with full-precision expf in the gates (the softmax uses the hardware exp2); they are the precision reference of the library on the
-// GPU, not its fast path (that is the bf16 path).  The linear layers of the position-wise passes
-// run on the fp32 matrix pipe (v_mfma_f32_32x32x2_f32: exact fp32 products, fp32 sums) in
-// work-groups of 32 positions whenever the channel counts are multiples of 8 and the weights are
-// 16-byte aligned; plain FMA kernels of 8 positions serve every other shape.
+// Three forms, by shape: on bf16 matrix instructions with every fp32 operand split into three bf16 terms
+// (of3_split.h; channel counts that are multiples of 16, head widths 32 and 16), on the fp32 matrix instructions
+// (v_mfma_f32_32x32x2_f32: exact products, fp32 sums; channel counts that are multiples of 8 and 16-byte
+// aligned weights), and plain FMA kernels of 8 positions with full-precision expf in the gates for every
+// other shape (any N, C, C_hidden <= 256, head width <= 64).  At 64 and 128 channels the position-wise passes are those of
+// pair_pass_f32.hip, the transition that of transition_f32.hip, pair bias and template tail those of pair_proj_f32.hip.
 //
 // Layouts (workspace, fp32): a, b, x  [B][CH][N][N] with a[b][c][i][k] (k contracted);
 // q, k, v [B][N(i)][H][N(j)][D]; triangle bias [B][H][N][N]; o [B][N][N][H*D].
