@@ -1333,8 +1333,7 @@ __global__ __launch_bounds__(kThreads * PT) void triattn_out_x3_f32(TriattnF32 p
   }
 }
 
-// Attention core on split operands, head width 16 * STEPS (32 or 16; the narrow head leaves half of the
-// O^T tile's rows unused).  Work-group = 4 waves = 2 consecutive rows i x 2
+// Attention core on split operands, head width 16 * STEPS (32 or 16).  Work-group = 4 waves = 2 consecutive rows i x 2
 // halves of one (head, 128-query range); a wave owns 64 queries (two 32-query tiles) of one row.  Two
 // work-groups share a CU, with exactly its 160 KB of LDS: a wave of each on every SIMD, so that the products of
 // one run under the exponentials and splits of the other (the barrier of a key tile holds the waves of a
@@ -1428,6 +1427,13 @@ __global__ __launch_bounds__(128 * kXRows, 2) void triattn_core_x3_f32(TriattnF3
   const __amdgpu_buffer_rsrc_t tb_rsrc = buffer_rsrc(tbp, (size_t)N * Jp * sizeof(float));
   const uint32_t lane_off = lane * 16;
   u32x4_t* kv_row = kv_lds + row * (2 * kXKvSlots);
+  // head width 16: slots of the P V operands below; the zeros lie where head width 32 has the K operands of its second step
+  constexpr int kZeros = 3 * 64;
+  const int narrow = (l32 & 15) + 32 * lh;
+  if constexpr (STEPS == 1) {
+    if (qh == 0 && lane < 2) kv_row[lane * kXKvSlots + kZeros] = u32x4_t{0u, 0u, 0u, 0u};
+    __syncthreads();
+  }
   auto issue_loads = [&](int kt, int buf) {  // buf is a constant at every call site
     u32x4_t* tdst = tb_lds + buf * kXTbSlots + 64 * kTb * wave;
     u32x4_t* kdst = kv_row + buf * kXKvSlots + 6 * 64 * qh;
@@ -1539,6 +1545,19 @@ __global__ __launch_bounds__(128 * kXRows, 2) void triattn_core_x3_f32(TriattnF3
         for (int e = 0; e < 8; ++e) x[e] = s[8 * st + e];
         u32x4_t ph, pm, pl;
         split8(x, ph, pm, pl);
+        if constexpr (STEPS == 1) {
+          // 16 rows of V^T: the upper half of the tile takes the middle terms of the same channels, [vh; vm] p, and is
+          // added at the end; four products instead of six (template branch, us: 3 x 200 1316 -> 1298, 2 x 500 6045 -> 5890;
+          // error against float64 0.98 of what it was)
+          const u32x4_t* kv0 = kv_row + buf * kXKvSlots;
+          const u32x4_t vhm = kv0[(6 + st * 3 + (l32 >> 4)) * 64 + narrow];
+          const u32x4_t vh = kv0[l32 < 16 ? (6 + st * 3) * 64 + narrow : kZeros], vl = kv0[l32 < 16 ? (8 + st * 3) * 64 + narrow : kZeros];
+          oacc[qt] = mfma_32x32x16(vl, ph, oacc[qt]);
+          oacc[qt] = mfma_32x32x16(vh, pl, oacc[qt]);
+          oacc[qt] = mfma_32x32x16(vhm, pm, oacc[qt]);
+          oacc[qt] = mfma_32x32x16(vhm, ph, oacc[qt]);
+          continue;
+        }
         const u32x4_t vh = kvb[(6 + st * 3) * 64], vm = kvb[(7 + st * 3) * 64], vl = kvb[(8 + st * 3) * 64];
         oacc[qt] = mfma_32x32x16(vl, ph, oacc[qt]);
         oacc[qt] = mfma_32x32x16(vh, pl, oacc[qt]);
@@ -1625,6 +1644,10 @@ __global__ __launch_bounds__(128 * kXRows, 2) void triattn_core_x3_f32(TriattnF3
       const int q = q0 + 32 * qt + l32;
       if (q >= N) continue;
       const float inv = 1.0f / l_tot[qt];
+      if constexpr (STEPS == 1) {
+#pragma unroll
+        for (int v = 0; v < 8; ++v) oacc[qt][v] += oacc[qt][v + 8];
+      }
       float* dst = p.o + ((((size_t)b * N + i) * N + q) * H + h) * D + 4 * lh;
 #pragma unroll
       for (int a = 0; a < D / 8; ++a)  // registers 4 a .. 4 a + 3 are head channels 8 a + 4 lh .. + 3
