@@ -13,6 +13,7 @@ module by module.
 from __future__ import annotations
 
 import ctypes
+import math
 import weakref
 
 import torch
@@ -39,7 +40,7 @@ class _Params:
 
     def __init__(self):
         self.links = []    # (children of a module, name, the child they held)
-        self.refs = []     # (parameters of a module, name)
+        self.refs = []     # (parameters of a module, name, number of values)
         self.shapes = []   # what refs must have; None where a parameter may be absent
         self.entries = []  # (index into refs, first row): the pointers handed over
         self.called = []   # submodules that the block calls as modules
@@ -71,7 +72,7 @@ class _Params:
         if name not in module._parameters:
             raise _Refused
         self.entries.append((len(self.refs), 0))
-        self.refs.append((module._parameters, name))
+        self.refs.append((module._parameters, name, math.prod(shape)))
         self.shapes.append((shape, optional))
 
     def norm(self, module, name, c, optional_bias=False):
@@ -82,7 +83,7 @@ class _Params:
     def linears(self, module, names, shape, bias=False):
         """Of several layers of one shape, written out: they are most of a block."""
         children, links, entries, refs, shapes = module._modules, self.links, self.entries, self.refs, self.shapes
-        want = (shape, False)
+        want, count = (shape, False), math.prod(shape)
         for name in names:
             lin = children.get(name)
             if type(lin) is not torch.nn.Linear:
@@ -92,7 +93,7 @@ class _Params:
             if "weight" not in own:
                 raise _Refused
             entries.append((len(refs), 0))
-            refs.append((own, "weight"))
+            refs.append((own, "weight", count))
             shapes.append(want)
             if bias:
                 self.param(lin, "bias", shape[:1])
@@ -100,17 +101,17 @@ class _Params:
     def gather(self, dtype):
         """The pointer array, or None when a parameter is not a plain contiguous tensor of `dtype`."""
         ptrs = []
-        for owner, name in self.refs:
+        for owner, name, count in self.refs:
             p = owner.get(name)
             if p is None:
                 ptrs.append(0)
-            elif p.dtype is dtype and p.is_contiguous():
+            elif p.numel() == count and p.dtype is dtype and p.is_contiguous():
                 ptrs.append(p.data_ptr())
             else:
                 return None
         seen_ptrs, seen_dtype, array = self.last
         if seen_ptrs != ptrs or seen_dtype is not dtype:
-            for (owner, name), (shape, optional) in zip(self.refs, self.shapes):
+            for (owner, name, _), (shape, optional) in zip(self.refs, self.shapes):
                 p = owner.get(name)
                 if not optional if p is None else p.shape != shape:
                     return None

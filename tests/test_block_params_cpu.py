@@ -35,3 +35,16 @@ def test_first_call_of_a_long_sequence():
     assert _block._first_call(block, torch.empty(1, n, n, 1, device="meta"))
     assert not _block._first_call(block, torch.empty(1, n, n, 1, device="meta"))
     assert _taken(block)
+
+
+def test_smaller_parameter_at_the_same_address():
+    """What is kept between calls is the pointers: a parameter replaced by a part of itself has to be seen."""
+    block = of3pair.PairFormerBlock(384, 128, 24, 16, 128, 32, 4).eval()
+    assert _taken(block)
+    for sub in (block.pair_stack.tri_mul_in.linear_z, block.pair_stack.tri_att_end.layer_norm, block.single_transition.linear_out,
+                block.attn_pair_bias.mha.linear_q):
+        whole = sub.weight
+        sub.weight = torch.nn.Parameter(whole.data[: whole.shape[0] // 2])
+        assert sub.weight.data_ptr() == whole.data_ptr() and not _taken(block)
+        sub.weight = whole
+        assert _taken(block)
