@@ -230,9 +230,10 @@ __global__ __launch_bounds__(64 * kLnWaves) void single_proj_x3_f32(SingleAttnF3
 
 // exp(x) for x <= 0 (or -inf) from the hardware's exp2: the part of x * log2(e) that one product rounds away
 // is carried along and put back (e^(r ln 2) = 1 + r ln 2 for |r| far below 1), so the relative error stays at
-// the 1 ulp of the instruction whatever the size of x
+// the 1 ulp of the instruction whatever the size of x.  NaN gives NaN: a compare and a select keep -inf out of the
+// products, where fmaxf would also turn a NaN logit into the weight 0 of a masked key.
 __device__ __forceinline__ float exp_neg(float x) {
-  x = fmaxf(x, -1e30f);
+  x = x < -1e30f ? -1e30f : x;
   const float t = x * kLog2e;
   const float r = fmaf(x, 1.925963033e-8f, fmaf(x, kLog2e, -t));
   const float e = __builtin_amdgcn_exp2f(t);
@@ -351,13 +352,14 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
     float mx = s[0];
 #pragma unroll
     for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
-    const float m_new = fmaxf(m_run, fmaxf(mx, __shfl_xor(mx, 32, 64)));  // finite: every tile holds a key below N
-    const float alpha = exp_neg(m_run - m_new);                           // 0 on the first tile
+    const float m_new = fmaxf(m_run, fmaxf(mx, __shfl_xor(mx, 32, 64)));  // of the logits that are numbers
+    const float ref = m_new == ninf ? 0.f : m_new;  // all of the pair bias so far was -inf: its keys weigh 0, not NaN
+    const float alpha = exp_neg(m_run - ref);       // 0 on the first tile
     m_run = m_new;
     l_run *= alpha;
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      s[v] = exp_neg(s[v] - m_new);
+      s[v] = exp_neg(s[v] - ref);
       l_run += s[v];
       oacc[v] *= alpha;
       osmall[v] *= alpha;
@@ -388,7 +390,7 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
   for (int v = 0; v < 16; ++v) merge[wave][v][lane] = oacc[v] + osmall[v];
   __syncthreads();
   if (wave != 0) return;
-  float m_tot = merge[0][16][lane];  // wave 0 always has tile 0: finite
+  float m_tot = merge[0][16][lane];  // -inf only where no key of the query weighs anything (the row is NaN then)
 #pragma unroll
   for (int w = 1; w < kAttnWaves; ++w) m_tot = fmaxf(m_tot, merge[w][16][lane]);
   float l_tot = 0.f;
