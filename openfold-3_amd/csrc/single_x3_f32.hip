@@ -12,6 +12,10 @@
 // consecutive k-values 16 lh .. + 15 of a block (64 bytes, the two halves complete a 128-byte line) as the
 // operands of two MFMA steps; weights and rows use the same order of k, which is all a sum over k needs.
 // Measured at 64 / 384 / 768 rows, us: see the kernels.
+//
+// The terms of an infinity, and of a value above the largest bf16 (3.39e38), are an infinity and NaN: an output
+// that depends on one comes out as NaN.  Every NaN is therefore computed again with plain fused multiply-adds, in
+// the order of single_f32.hip, which keep an infinity; where an operand is NaN itself they give NaN again.
 #include "of3_device.h"
 #include "of3_kernels.h"
 #include "of3_launch.h"
@@ -83,6 +87,21 @@ __device__ __forceinline__ float4 sum_partials(const float* part, int stride, in
   for (int w = 1; w < NW; ++w) {
     const float4 v = *reinterpret_cast<const float4*>(part + w * stride + row * kPartLd + 4 * c4);
     s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
+  }
+  return s;
+}
+
+__device__ __forceinline__ bool has_nan(const float4& v) { return v.x != v.x || v.y != v.y || v.z != v.z || v.w != v.w; }
+// outputs of four rows of W [..][K] for one row of inputs, x(k): inputs 4 k .. + 3
+template <class Row>
+__device__ __forceinline__ float4 plain_dots(Row&& x, const float* W, int K) {
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto add = [](float acc, const float4& a, const float4& w) { return fmaf(a.w, w.w, fmaf(a.z, w.z, fmaf(a.y, w.y, fmaf(a.x, w.x, acc)))); };
+  auto weights = [&](int row, int k) { return *reinterpret_cast<const float4*>(W + (size_t)row * K + 4 * k); };
+#pragma unroll 1
+  for (int k = 0; k < K / 4; ++k) {
+    const float4 a = x(k);
+    s.x = add(s.x, a, weights(0, k)), s.y = add(s.y, a, weights(1, k)), s.z = add(s.z, a, weights(2, k)), s.w = add(s.w, a, weights(3, k));
   }
   return s;
 }
@@ -173,6 +192,26 @@ __device__ __forceinline__ void ln_products(const float* __restrict__ src, long 
   __syncthreads();
 }
 
+// the outputs of four rows of W for row pos0 + r (a row that exists) without the matrix instructions; red as ln_products
+// has left it
+__device__ __forceinline__ float4 ln_plain_dots(const float* __restrict__ src, long pos0, int r, int C, const float* __restrict__ ln_w,
+                                                const float* __restrict__ ln_b, const float* W, const float* red) {
+  float mean = 0.f, var = 0.f;
+#pragma unroll
+  for (int q = 0; q < kLnWaves; ++q) mean += red[q * 32 + r], var += red[(kLnWaves + q) * 32 + r];
+  mean /= (float)C;
+  const float rstd = 1.0f / sqrtf(var / (float)C + kEps);
+  const float4* x = reinterpret_cast<const float4*>(src + (pos0 + r) * C);
+  const float4 *g = reinterpret_cast<const float4*>(ln_w), *b = reinterpret_cast<const float4*>(ln_b);
+  return plain_dots(
+      [&](int k) {
+        const float4 v = x[k], gk = g[k], bk = b[k];
+        return make_float4((v.x - mean) * rstd * gk.x + bk.x, (v.y - mean) * rstd * gk.y + bk.y, (v.z - mean) * rstd * gk.z + bk.z,
+                           (v.w - mean) * rstd * gk.w + bk.w);
+      },
+      W, C);
+}
+
 // rows pos0 .. + 31 of src [rows][K] times 32 rows of W [..][K] (W points at the first): the partial tile of
 // wave w is left in part[w * kPart].  K a multiple of 32; the next block's operands are in flight meanwhile.
 template <int NW>
@@ -218,6 +257,7 @@ __global__ __launch_bounds__(64 * kLnWaves) void single_proj_x3_f32(SingleAttnF3
   const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
   if (pos0 + r >= rows) return;
   float4 v = sum_partials<kLnWaves>(part, kPart, r, c4);
+  if (has_nan(v)) v = ln_plain_dots(p.a, pos0, r, p.C, p.ln_w, p.ln_b, W[0] + (size_t)4 * c4 * p.C, red);
   if (kind == 0) {
     const float scale = 1.0f / sqrtf((float)p.D);
     const float* bq = p.bq + o0 + 4 * c4;
@@ -404,6 +444,32 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
     for (int v = 0; v < 16; ++v) oacc[v] += merge[w][v][lane] * sc;
   }
   if (!q_valid) return;
+  bool again = l_tot != l_tot;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) again |= oacc[v] != oacc[v];
+  if (again) {  // the query without the matrix instructions: the maximum, then the weighted sum of this lane's channels
+    const float* qr = p.q + (bN + qrow) * HD + h * D;
+    auto logit = [&](int key) {
+      const float* kr = p.k + (bN + key) * HD + h * D;
+      float acc = 0.f;
+      for (int d = 0; d < D; ++d) acc = fmaf(qr[d], kr[d], acc);
+      return acc + p.inf * ((p.mask ? p.mask[bN + key] : 1.f) - 1.f) + pb[key];
+    };
+    m_tot = ninf, l_tot = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) oacc[v] = 0.f;
+#pragma unroll 1
+    for (int key = 0; key < N; ++key) m_tot = fmaxf(m_tot, logit(key));
+#pragma unroll 1
+    for (int key = 0; key < N; ++key) {
+      const float w = exp_neg(logit(key) - m_tot);
+      const float* vr = p.v + (bN + key) * HD + h * D + 4 * lh;
+      l_tot += w;
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (8 * (v >> 2) < D) oacc[v] = fmaf(w, vr[8 * (v >> 2) + (v & 3)], oacc[v]);
+    }
+  }
   const float inv = 1.0f / l_tot;
   const size_t off = (bN + qrow) * HD + h * D + 4 * lh;
 #pragma unroll
@@ -425,6 +491,10 @@ __global__ __launch_bounds__(64 * kOutWaves) void single_out_x3_f32(SingleAttnF3
   const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
   if (pos0 + r >= rows) return;
   float4 v = sum_partials<kOutWaves>(part, kPart, r, c4);
+  if (has_nan(v)) {
+    const float4* x = reinterpret_cast<const float4*>(p.og + (pos0 + r) * HD);
+    v = plain_dots([&](int k) { return x[k]; }, p.wo + (size_t)(o0 + 4 * c4) * HD, HD);
+  }
   const size_t off = (pos0 + r) * p.C + o0 + 4 * c4;
   if (p.add_residual) {
     const float4 x = *reinterpret_cast<const float4*>(p.a + off);
@@ -444,7 +514,9 @@ __global__ __launch_bounds__(64 * kLnWaves) void row_hidden_x3_f32(RowTransition
   ln_products<2>(p.x, pos0, p.rows, p.C, p.ln_w, p.ln_b, W, part, red);
   const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
   if (pos0 + r >= p.rows) return;
-  const float4 a = sum_partials<kLnWaves>(part, 2 * kPart, r, c4), b = sum_partials<kLnWaves>(part + kPart, 2 * kPart, r, c4);
+  float4 a = sum_partials<kLnWaves>(part, 2 * kPart, r, c4), b = sum_partials<kLnWaves>(part + kPart, 2 * kPart, r, c4);
+  if (has_nan(a)) a = ln_plain_dots(p.x, pos0, r, p.C, p.ln_w, p.ln_b, W[0] + (size_t)4 * c4 * p.C, red);
+  if (has_nan(b)) b = ln_plain_dots(p.x, pos0, r, p.C, p.ln_w, p.ln_b, W[1] + (size_t)4 * c4 * p.C, red);
   float4 v;
   v.x = a.x * sigmoid_f32(a.x) * b.x;
   v.y = a.y * sigmoid_f32(a.y) * b.y;
@@ -464,6 +536,10 @@ __global__ __launch_bounds__(64 * kRowOutWaves) void row_out_x3_f32(RowTransitio
   const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
   if (pos0 + r >= p.rows) return;
   float4 v = sum_partials<kRowOutWaves>(part, kPart, r, c4);
+  if (has_nan(v)) {
+    const float4* x = reinterpret_cast<const float4*>(p.hidden + (pos0 + r) * p.HID);
+    v = plain_dots([&](int k) { return x[k]; }, p.wout + (size_t)(o0 + 4 * c4) * p.HID, p.HID);
+  }
   if (p.mask) {
     const float m = p.mask[pos0 + r];
     v.x *= m, v.y *= m, v.z *= m, v.w *= m;

@@ -1,4 +1,5 @@
-"""NaN among the inputs of the fp32 kernels of the single representation: it reaches what depends on it and nothing else."""
+"""NaN, infinities and values above the largest bf16 in the fp32 kernels that split their operands into bf16 terms: they
+reach what depends on them as in plain arithmetic, and nothing else."""
 import pytest
 import torch
 
@@ -66,3 +67,70 @@ def test_keys_at_minus_infinity(n, open_keys):
     scale = max(1.0, float(want.nan_to_num().abs().max()))
     # the bound of the tile tests: 384-term fp32 sums, four of them in a row
     assert float((got.double() - want).nan_to_num().abs().max()) <= 5e-6 * scale
+
+
+def _same(got, want, rtol=5e-5):
+    """got (fp32) against want (64 bits, an infinity from the largest fp32 value on): NaN and infinities at the same
+    places, the rest to rtol: sums of up to 160 terms of which one may be 1e38 times the others."""
+    want = want.float()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got[want.isinf()], want[want.isinf()])
+    fin = want.isfinite()
+    assert torch.allclose(got[fin], want[fin], rtol=rtol, atol=1e-5)
+
+
+INF, HUGE = float("inf"), 3.4e38  # HUGE: above the largest bf16, 3.3895e38
+
+
+@pytest.mark.parametrize("n,name,value", [(33, "wg", INF), (33, "wg", -HUGE), (33, "wo", -INF), (70, "wo", HUGE), (1, "wv", INF), (1, "wv", HUGE),
+                                          (33, "wq", INF), (33, "key", 1e38), (161, "key", 1e38)])
+def test_attention_keeps_infinities(n, name, value):
+    """An infinite or very large weight: infinities, zeros of the gate and left-out keys as plain arithmetic gives them."""
+    lib()
+    c, gen = 32, torch.Generator().manual_seed(6400 + n)
+    w = {k: torch.randn(c, c, generator=gen) / c ** 0.5 for k in ("wq", "wk", "wv", "wg", "wo")}
+    bq = torch.zeros(c)
+    a = torch.randn(1, n, c, generator=gen)
+    if name == "key":
+        # the first channel of key n / 2 is -inf, of every other one 0; that of every query is positive
+        signs = torch.tensor([1.0, -1.0, 1.0, -1.0]).repeat(c // 4)
+        a = signs.repeat(1, n, 1) * torch.tensor([1.0, -1.0])[torch.randint(2, (1, n, 1), generator=gen)]
+        a[0, n // 2, :8] = torch.tensor([1.0, 1.0, 1.0, 1.0, -1.0, -1.0, -1.0, -1.0])
+        w["wk"][0] = 0.0
+        w["wk"][0, :4] = -value
+        w["wq"][0] = 0.0
+        bq[0] = 3.0
+    else:
+        w[name][2, 3] = value
+    one, zero = torch.ones(c), torch.zeros(c)
+    bias = torch.randn(1, 1, n, n, generator=gen)
+    args = [t.to(DEV) for t in (one, zero)] + [None, None, None] + [t.to(DEV) for t in (w["wq"], bq, w["wk"], w["wv"], w["wg"], w["wo"])]
+    got = of3pair.functional.attention_pair_bias(a.to(DEV), None, None, *args, no_heads=1, _bias=bias.to(DEV)).cpu()
+    d = {k: v.double() for k, v in w.items()}
+    an = torch.nn.functional.layer_norm(a.double(), (c,))
+    if name == "key":  # what the logits come to (the zeros of the other keys are exact in 32 bits, not in 64)
+        d["wk"][0] = 0.0
+        bias[..., n // 2] = -INF
+    q, k, v, g = an @ d["wq"].T + bq.double(), an @ d["wk"].T, an @ d["wv"].T, torch.sigmoid(an @ d["wg"].T)
+    o = ((q @ k.transpose(-1, -2) / c ** 0.5 + bias[:, 0].double()).softmax(-1) @ v) * g
+    if n == 1:
+        o = o.float().double()  # what is stored between the kernels is fp32
+    _same(got, o @ d["wo"].T)
+
+
+@pytest.mark.parametrize("name,value", [("wa", INF), ("wa", HUGE), ("wb", INF), ("wb", -HUGE), ("wo", -INF), ("wo", HUGE)])
+def test_row_transition_keeps_infinities(name, value):
+    lib()
+    c, hid, gen = 64, 128, torch.Generator().manual_seed(6500)
+    w = {k: torch.randn(*s, generator=gen) / s[1] ** 0.5 for k, s in (("wa", (hid, c)), ("wb", (hid, c)), ("wo", (c, hid)))}
+    w[name][5, 9] = value
+    x = torch.randn(45, c, generator=gen)
+    got = of3pair.functional.swiglu_transition(x.to(DEV), None, torch.ones(c, device=DEV), torch.zeros(c, device=DEV),
+                                               *[w[k].to(DEV) for k in ("wa", "wb", "wo")]).cpu()
+    d = {k: v.double() for k, v in w.items()}
+    xn = torch.nn.functional.layer_norm(x.double(), (c,))
+    ha, hb = (xn @ d["wa"].T).float(), (xn @ d["wb"].T).float()
+    h = (ha * torch.sigmoid(ha)) * hb
+    # a large hidden channel 5 is the whole sum, to the relative error of its two factors: sums of 64 terms that add up to
+    # 8 in size, 64 * 2^-24 * 8 / 16 = 2e-6 absolute
+    _same(got, h.double() @ d["wo"].T, rtol=5e-5 + 2e-6 / float(ha[:, 5].abs().min()) + 2e-6 / float(hb[:, 5].abs().min()))
