@@ -134,3 +134,23 @@ def test_row_transition_keeps_infinities(name, value):
     # a large hidden channel 5 is the whole sum, to the relative error of its two factors: sums of 64 terms that add up to
     # 8 in size, 64 * 2^-24 * 8 / 16 = 2e-6 absolute
     _same(got, h.double() @ d["wo"].T, rtol=5e-5 + 2e-6 / float(ha[:, 5].abs().min()) + 2e-6 / float(hb[:, 5].abs().min()))
+
+
+@pytest.mark.parametrize("where,value,apply_ln", [("t", INF, False), ("t", HUGE, False), ("t", -INF, False), ("w", INF, True), ("w", -HUGE, True),
+                                                  ("w", INF, False)])
+def test_template_tail_keeps_infinities(where, value, apply_ln):
+    lib()
+    gen = torch.Generator().manual_seed(6600)
+    t, w = torch.randn(2, 3, 7, 7, 64, generator=gen), torch.randn(128, 64, generator=gen)
+    lw, lb = 1.0 + 0.1 * torch.randn(64, generator=gen), 0.1 * torch.randn(64, generator=gen)
+    if where == "t":
+        t[1, 2, 6, 3, 50] = value
+    else:
+        w[77, 13] = value
+    got = of3pair.functional.template_tail(t.to(DEV), lw.to(DEV), lb.to(DEV), w.to(DEV), apply_layer_norm=apply_ln).cpu()
+    u = torch.nn.functional.layer_norm(t.double(), (64,), lw.double(), lb.double()) if apply_ln else t.double()
+    mean = u.sum(1) / 3
+    want = torch.relu(mean) @ w.double().T
+    # an output that a large weight makes is off as its input is: sums of three values up to 4, 3 * 2^-24 * 4, of the smallest
+    small = float(mean[..., 13][mean[..., 13] > 0].min()) if where == "w" else 1.0
+    _same(got, want, rtol=5e-5 + 1e-6 / small)
