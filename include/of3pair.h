@@ -324,6 +324,12 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
                              int64_t HID_s, float inf, float inf_s, int flags, void* workspace, int64_t workspace_bytes,
                              int dtype, void* stream, void* side_stream);
 
+/* A stream of the current device for side_stream above: default priority, not ordered after the default stream.  It is
+ * the caller's, like any other stream; one that is also handed to code that captures graphs on it must not serve
+ * here, a call's events would join that capture.  Destroying it waits for the work it holds. */
+int of3_side_stream_create(void** stream);
+int of3_side_stream_destroy(void* stream);
+
 #ifdef __cplusplus
 }
 #endif

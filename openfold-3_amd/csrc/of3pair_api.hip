@@ -1327,4 +1327,23 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
   return st;
 }
 
+int of3_side_stream_create(void** stream) {
+  if (!stream) return OF3_EINVAL;
+  hipStream_t s = nullptr;
+  const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // the caller goes on with one stream
+    return fail_hip(e);
+  }
+  *stream = s;
+  return OF3_OK;
+}
+
+int of3_side_stream_destroy(void* stream) {
+  if (!stream) return OF3_EINVAL;
+  hipError_t e = hipStreamSynchronize(static_cast<hipStream_t>(stream));
+  if (e == hipSuccess) e = hipStreamDestroy(static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? OF3_OK : fail_hip(e);
+}
+
 }  // extern "C"

@@ -330,23 +330,6 @@ def run_pairformer_block(block, pair_block_type, s, z, single_mask, pair_mask, i
     return s_out, z if inplace else z_out.view(z.shape)
 
 
-_sides = {}  # (device, stream) -> the stream of torch's pool that a stack's single representation runs on
-_MAX_SIDES = 16
-
-
-def _side_stream(device, stream):
-    """A second stream for work that is issued to `stream`; None while a stream is being captured (a graph would draw
-    in a stream that other threads may be using)."""
-    if torch.cuda.is_current_stream_capturing():
-        return None
-    side = _sides.get((device, stream))
-    if side is None:
-        if len(_sides) >= _MAX_SIDES:
-            _sides.clear()
-        side = _sides[(device, stream)] = torch.cuda.Stream(device=device)
-    return side.cuda_stream if side.cuda_stream != stream else None
-
-
 def run_pairformer_stack(blocks, block_type, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
     """(s, z) after all blocks, or None when the single call does not serve them."""
     if any(_plans.get(block) is None for block in blocks):
@@ -384,5 +367,5 @@ def run_pairformer_stack(blocks, block_type, pair_block_type, s, z, single_mask,
           _lib.strides3(z4.stride()[:3]), None if sm is None else sm.data_ptr(), mptr, mstr, s_out.data_ptr(),
           z_out.data_ptr(), B, N, c, ch, h, d, hid, c_s, h_s, d_s, hid_s, float(inf), float(inf_s),
           0 if mask_trans else _lib.OF3_BLOCK_TRANSITION_UNMASKED, ws.data_ptr(), ws.numel(), code, stream,
-          _side_stream(z.device, stream))
+          F3._side_stream(z.device, stream))
     return s_out, z if inplace else z_out.view(z.shape)

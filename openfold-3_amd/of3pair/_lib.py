@@ -71,6 +71,8 @@ SIGNATURES = {
     "of3_pairformer_stack_fwd": (c_int, [ctypes.POINTER(ctypes.POINTER(c_void_p)), c_int64, c_void_p, c_void_p, _I64x3, c_void_p,
                                          c_void_p, _I64x3, c_void_p, c_void_p] + [c_int64] * 11
                                  + [c_float, c_float, c_int, c_void_p, c_int64, c_int, c_void_p, c_void_p]),
+    "of3_side_stream_create": (c_int, [ctypes.POINTER(c_void_p)]),
+    "of3_side_stream_destroy": (c_int, [c_void_p]),
     "of3_template_tail_fwd": (c_int, [c_void_p] * 5 + [c_int64] * 5 + [c_int, c_int, c_void_p]),
 }
 

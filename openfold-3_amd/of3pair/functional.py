@@ -11,6 +11,9 @@ fp32 kernels (slower, the precision path); parameters are converted to the tenso
 """
 from __future__ import annotations
 
+import ctypes
+import threading
+
 import torch
 
 from . import _lib
@@ -45,12 +48,50 @@ def _workspace(device, nbytes: int, stream=None) -> torch.Tensor:
     return buf
 
 
+_MAX_SIDES = 16
+_side_lock = threading.Lock()
+_own_streams: dict = {}  # device -> handles of the library's own streams on it, at most _MAX_SIDES
+_sides: dict = {}  # (device, caller's stream) -> one of them
+
+
+def _side_stream(device, stream):
+    """A second stream for work that is issued to `stream`, one of a few per device that the library makes for itself
+    (torch deals the 32 streams of its pool to everybody, also to a thread that captures a graph on one: the events of
+    a call beside it would run into that capture).  Beyond _MAX_SIDES streams of callers they are shared, which costs
+    them overlap and nothing else.  None while the current stream is captured: the graph stays on that stream."""
+    if torch.cuda.is_current_stream_capturing():
+        return None
+    side = _sides.get((device, stream))
+    if side is None:
+        with _side_lock:
+            own = _own_streams.setdefault(device, [])
+            if len(own) < _MAX_SIDES:
+                made = ctypes.c_void_p()
+                with torch.cuda.device(device):
+                    if _lib.load().of3_side_stream_create(ctypes.byref(made)) == _lib.OF3_OK:
+                        own.append(made.value)
+                        side = made.value
+            if side is None and own:
+                side = own[len(_sides) % len(own)]
+            if len(_sides) >= 16 * _MAX_SIDES:
+                _sides.clear()
+            if side is not None:
+                _sides[(device, stream)] = side
+    return side
+
+
 def release_workspaces():
-    """Drops every scratch buffer, current and outgrown.  Only when no captured graph that used them
-    will be replayed again."""
+    """Drops every scratch buffer, current and outgrown, and the library's own streams.  Only when no call is under way in
+    another thread and no captured graph that used the buffers will be replayed again."""
     _workspaces.clear()
     _in_graph.clear()
     _retired.clear()
+    with _side_lock:
+        _sides.clear()
+        for device, own in _own_streams.items():
+            with torch.cuda.device(device):
+                while own:
+                    _lib.check(_lib.load().of3_side_stream_destroy(own.pop()), "of3_side_stream_destroy")
 
 
 def _require_gpu(t: torch.Tensor, name: str) -> int:
