@@ -6,9 +6,9 @@ queries for each of its seven modules) beside 50 us of launches, more than its k
 tokens.  Here the parameters are gathered in one sweep and the arguments are prepared once per block.
 
 A block is served when it is built of this package's own modules as their constructors left them: anything a
-caller may have changed (a replaced or subclassed submodule, a hook on one, parameters of another dtype than
-the activations, layouts or widths that need a conversion) makes run_* return None, and the block then runs
-module by module.
+caller may have changed (a replaced or subclassed submodule, a hook on one, a method replaced on one or on its class,
+parameters of another dtype than the activations, layouts or widths that need a conversion) makes run_* return None,
+and the block then runs module by module.
 """
 from __future__ import annotations
 
@@ -34,6 +34,34 @@ class _Refused(Exception):
     """The block is not one that the single call serves."""
 
 
+# Everything that a block run module by module calls by name: (class or module, name, what this package put there).
+_written = []
+
+
+def written(owner, *names):
+    _written.extend((owner, name, getattr(owner, name)) for name in names)
+
+
+def _as_written():
+    """Whether a block's modules still do what the single call does in their place: no method replaced on a class (also
+    nn.Module's own __call__, as tracers do), no function of this package replaced by a caller's."""
+    for owner, name, value in _written:
+        if getattr(owner, name, None) is not value:
+            return False
+    return True
+
+
+written(torch.nn.Module, "__call__", "_call_impl", "__getattr__")
+written(F3, "triangle_multiplicative_update", "triangle_attention", "swiglu_transition", "pair_bias", "attention_pair_bias")
+written(layers.SwiGLUTransition, "__call__", "forward")
+written(layers.AttentionPairBias, "__call__", "forward")
+for _mul in _MULS:
+    written(_mul, "_weights")
+# what a pair block calls on itself
+PAIR_METHODS = ("tri_mul_out_in", "tri_att_start_end", "_modules_forward", "_mul", "_att")
+_CALL = frozenset(("forward", "_compiled_call_impl"))
+
+
 class _Params:
     """The parameters of a block in the order of the C ABI, looked up anew in every call: a parameter or a
     submodule that was replaced since, or moved by .to(), is seen."""
@@ -44,6 +72,7 @@ class _Params:
         self.shapes = []   # what refs must have; None where a parameter may be absent
         self.entries = []  # (index into refs, first row): the pointers handed over
         self.called = []   # submodules that the block calls as modules
+        self.methods = []  # (attributes of a module, names it may not have of its own)
         self.attrs = []    # (attributes of a module, name, the value the dimensions were taken from)
         self.last = (None, None, None)  # pointers of refs, dtype and pointer array of the last call
 
@@ -124,12 +153,14 @@ class _Params:
 
 def _pair_params(q, block):
     """Appends what of3_pair_block_fwd takes; returns (C, CH, H, D, HID, inf)."""
+    q.methods.append((block.__dict__.keys(), PAIR_METHODS))
     mul_out, mul_in = q.child(block, "tri_mul_out", _MULS), q.child(block, "tri_mul_in", _MULS)
     c, ch = mul_out.c_z, mul_out.c_hidden
     for m, outgoing in ((mul_out, True), (mul_in, False)):
         if _MULS[type(m)] is not outgoing or m._outgoing is not outgoing or (m.c_z, m.c_hidden) != (c, ch):
             raise _Refused
         q.attr(m, "c_z", "c_hidden", "_outgoing")
+        q.methods.append((m.__dict__.keys(), ("_weights",)))
         q.norm(m, "layer_norm_in", c)
         q.norm(m, "layer_norm_out", ch)
         if isinstance(m, layers.FusedTriangleMultiplicativeUpdate):
@@ -235,8 +266,12 @@ def _gather(block, build, dtype):
     if array is None:
         return None
     for m in q.called:  # modules that the block would call: their hooks, their mode and a forward of their own are theirs
-        if m.training or m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+        if m.training or m._forward_hooks or m._forward_pre_hooks or not _CALL.isdisjoint(m.__dict__):
             return None
+    for own, names in q.methods:
+        for name in names:
+            if name in own:
+                return None
     if _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks:
         return None
     return array, dims
@@ -263,7 +298,7 @@ def _call(fn, what, device, *args):
 
 def run_pair_block(block, z, mask, inplace, attention_first=False, mask_trans=True):
     """z after the block's modules, or None when the single call does not serve it."""
-    if _first_call(block, z):
+    if _first_call(block, z) or not _as_written():
         return None
     found = _gather(block, lambda q: _pair_params(q, block), z.dtype)
     args = found and _pair_args(z, mask)
@@ -303,7 +338,7 @@ def _pairformer_args(s, z, single_mask, pair_mask, c, c_s):
 
 def run_pairformer_block(block, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
     """(s, z) after the block, or None when the single call does not serve it."""
-    if _first_call(block, z):
+    if _first_call(block, z) or not _as_written():
         return None
     found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
     if not found:
@@ -332,13 +367,15 @@ def run_pairformer_block(block, pair_block_type, s, z, single_mask, pair_mask, i
 
 def run_pairformer_stack(blocks, block_type, pair_block_type, s, z, single_mask, pair_mask, inplace, mask_trans=True):
     """(s, z) after all blocks, or None when the single call does not serve them."""
+    if not _as_written():
+        return None
     if any(_plans.get(block) is None for block in blocks):
         # First calls: finding the parameters takes some 100 us per block.  Block by block that passes beside the kernels of
         # the blocks before (4 blocks at N = 200: 1350 us in place of 1640).
         return None
     arrays, dims = [], None
     for block in blocks:
-        if type(block) is not block_type or block.training or block._forward_hooks or block._forward_pre_hooks or "forward" in block.__dict__:
+        if type(block) is not block_type or block.training or block._forward_hooks or block._forward_pre_hooks or not _CALL.isdisjoint(block.__dict__):
             return None
         found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
         if not found or (dims is not None and found[1] != dims):

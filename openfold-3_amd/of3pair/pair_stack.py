@@ -133,3 +133,7 @@ class PairBlock(PairStack):
         z = self._modules_forward(z, pair_mask, inplace_safe)
         # z is owned by this call (or may be overwritten): the transition updates it in place
         return self.pair_transition(z, mask=pair_mask if _mask_trans else None, _add_residual=True, _inplace=True)
+
+
+_block.written(PairStack, *_block.PAIR_METHODS)
+_block.written(PairBlock, "__call__", "forward", *_block.PAIR_METHODS)

@@ -2,7 +2,7 @@
 PairFormerStack (openfold3/core/model/latent/pairformer.py:36-215, :217-470, AF3 Algorithm 17)
 with the same constructor arguments, sub-module names and forward signatures, so that
 `config.architecture.pairformer` constructs the stack and the `pairformer_stack.*` keys of a
-checkpoint load unchanged.  Inference only, bf16.
+checkpoint load unchanged.  Inference only, bf16 and fp32.
 """
 from __future__ import annotations
 
@@ -58,6 +58,9 @@ class PairFormerBlock(nn.Module):
         # s is now a tensor this call owns (or may be overwritten)
         s = self.single_transition(s, mask=single_mask if _mask_trans else None, _add_residual=True, _inplace=True)
         return s, z
+
+
+_block.written(PairFormerBlock, "__call__", "forward")
 
 
 class PairFormerStack(nn.Module):

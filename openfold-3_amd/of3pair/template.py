@@ -47,6 +47,9 @@ class TemplatePairBlock(PairBlock):
         return self.pair_transition(z, mask=mask if _mask_trans else None, _add_residual=True, _inplace=True)
 
 
+_block.written(TemplatePairBlock, *_block.PAIR_METHODS)
+
+
 class TemplatePairStack(nn.Module):
     """template_module.py:200-378: `no_blocks` TemplatePairBlocks and a closing LayerNorm, under
     the reference's sub-module names (blocks.<i>.*, layer_norm.*).  blocks_per_ckpt,

@@ -1,0 +1,78 @@
+"""A method or function that a caller has put in the place of one a block run module by module calls, is called: the block
+does not go through one library call then."""
+import pytest
+import torch
+
+from gpu_util import lib  # noqa: F401
+
+import of3pair
+from of3pair import _block
+from of3pair import functional as F3
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+CLASSES = [(of3pair.PairBlock, "forward"), (of3pair.AttentionPairBias, "forward"), (of3pair.SwiGLUTransition, "forward"),
+           (of3pair.PairFormerBlock, "forward"), (of3pair.PairBlock, "tri_mul_out_in"), (of3pair.PairStack, "tri_att_start_end"),
+           (of3pair.TriangleMultiplicationIncoming, "_weights"), (torch.nn.Module, "__call__"),
+           (F3, "triangle_attention"), (F3, "swiglu_transition"), (F3, "pair_bias")]
+INSTANCES = [("pair_stack", "tri_mul_out_in"), ("pair_stack", "tri_att_start_end"), ("pair_stack", "forward"),
+             ("pair_stack.tri_mul_out", "_weights"), ("pair_stack.pair_transition", "forward"), ("single_transition", "forward"),
+             ("attn_pair_bias", "_compiled_call_impl")]
+
+
+def _setup(monkeypatch, n=21):
+    lib()
+    torch.manual_seed(41)
+    m = of3pair.PairFormerStack(384, 128, 24, 16, 128, 32, 4, no_blocks=2)
+    with torch.no_grad():
+        for p in m.parameters():
+            if p.dim() == 2:
+                p.normal_(std=p.shape[1] ** -0.5)
+    m = m.to(DEV).to(torch.bfloat16).eval()
+    s, z = torch.randn(1, n, 384, device=DEV).to(torch.bfloat16), torch.randn(1, n, n, 128, device=DEV).to(torch.bfloat16)
+    want = m(s, z, None, None)
+    calls = []
+    inner = _block._call
+    monkeypatch.setattr(_block, "_call", lambda fn, what, *a: (calls.append(what), inner(fn, what, *a))[1])
+
+    def run():
+        del calls[:]
+        got = m(s, z, None, None)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        return list(calls)
+
+    assert run() == ["of3_pairformer_stack_fwd"]
+    return m, run
+
+
+def _recording(monkeypatch, owner, name, seen, instance=False):
+    inner = getattr(owner, name)
+    if inner is None:  # a module that torch.compile has not been asked for
+        inner = owner._call_impl
+
+    def put(*args, **kwargs):
+        seen.append(name)
+        return inner(*args, **kwargs)
+
+    monkeypatch.setattr(owner, name, put, raising=not instance)
+
+
+@pytest.mark.parametrize("owner,name", CLASSES, ids=lambda v: getattr(v, "__name__", v))
+def test_replaced_on_the_class(monkeypatch, owner, name):
+    m, run = _setup(monkeypatch)
+    seen = []
+    with monkeypatch.context() as mp:
+        _recording(mp, owner, name, seen)
+        assert run() == [] and seen
+    assert run() == ["of3_pairformer_stack_fwd"]
+
+
+@pytest.mark.parametrize("path,name", INSTANCES)
+def test_replaced_on_an_instance(monkeypatch, path, name):
+    m, run = _setup(monkeypatch)
+    seen = []
+    own = m.blocks[1].get_submodule(path)
+    _recording(monkeypatch, own, name, seen, instance=True)
+    assert "of3_pairformer_stack_fwd" not in run() and len(seen) == 1
+    del own.__dict__[name]
+    assert run() == ["of3_pairformer_stack_fwd"]
