@@ -64,31 +64,41 @@ _CALL = frozenset(("forward", "_compiled_call_impl"))
 
 class _Params:
     """The parameters of a block in the order of the C ABI, looked up anew in every call: a parameter or a
-    submodule that was replaced since, or moved by .to(), is seen."""
+    submodule that was replaced since, or moved by .to(), is seen.  What the search looks at is noted before it is
+    judged, so that a block that was refused is searched again once that has changed."""
 
     def __init__(self):
-        self.links = []    # (children of a module, name, the child they held)
+        self.links = []    # (children or parameters of a module, name, what they held, or None)
         self.refs = []     # (parameters of a module, name, number of values)
         self.shapes = []   # what refs must have; None where a parameter may be absent
         self.entries = []  # (index into refs, first row): the pointers handed over
         self.called = []   # submodules that the block calls as modules
+        self.types = None  # of what links held, where the block was refused
         self.methods = []  # (attributes of a module, names it may not have of its own)
         self.attrs = []    # (attributes of a module, name, the value the dimensions were taken from)
         self.last = (None, None, None)  # pointers of refs, dtype and pointer array of the last call
 
     def child(self, parent, name, kinds=None):
         sub = parent._modules.get(name)
+        self.links.append((parent._modules, name, sub))
         if sub is None or (kinds is not None and type(sub) not in kinds):
             raise _Refused
-        self.links.append((parent._modules, name, sub))
         return sub
 
     def attr(self, module, *names):
         for name in names:
             self.attrs.append((module.__dict__, name, getattr(module, name)))
+        return module
+
+    def refused(self):
+        """Notes the types too: a module may change its own, as one under a parametrization does."""
+        self.types = [type(held) for _, _, held in self.links]
+        return self, None
 
     def current(self):
         """Whether the block still holds the submodules and attributes that it held."""
+        if self.types is not None and any(type(link[2]) is not t for link, t in zip(self.links, self.types)):
+            return False
         for owner, name, sub in self.links:
             if owner.get(name) is not sub:
                 return False
@@ -99,6 +109,7 @@ class _Params:
 
     def param(self, module, name, shape, optional=False):
         if name not in module._parameters:
+            self.links.append((module._parameters, name, None))
             raise _Refused
         self.entries.append((len(self.refs), 0))
         self.refs.append((module._parameters, name, math.prod(shape)))
@@ -115,11 +126,12 @@ class _Params:
         want, count = (shape, False), math.prod(shape)
         for name in names:
             lin = children.get(name)
+            links.append((children, name, lin))
             if type(lin) is not torch.nn.Linear:
                 raise _Refused
-            links.append((children, name, lin))
             own = lin._parameters
             if "weight" not in own:
+                links.append((own, "weight", None))
                 raise _Refused
             entries.append((len(refs), 0))
             refs.append((own, "weight", count))
@@ -157,9 +169,9 @@ def _pair_params(q, block):
     mul_out, mul_in = q.child(block, "tri_mul_out", _MULS), q.child(block, "tri_mul_in", _MULS)
     c, ch = mul_out.c_z, mul_out.c_hidden
     for m, outgoing in ((mul_out, True), (mul_in, False)):
+        q.attr(m, "c_z", "c_hidden", "_outgoing")
         if _MULS[type(m)] is not outgoing or m._outgoing is not outgoing or (m.c_z, m.c_hidden) != (c, ch):
             raise _Refused
-        q.attr(m, "c_z", "c_hidden", "_outgoing")
         q.methods.append((m.__dict__.keys(), ("_weights",)))
         q.norm(m, "layer_norm_in", c)
         q.norm(m, "layer_norm_out", ch)
@@ -175,12 +187,12 @@ def _pair_params(q, block):
         q.linears(m, ("linear_g",), (c, c))
         q.linears(m, ("linear_z",), (c, ch))
     start, end = (q.child(block, n, (layers.TriangleAttention,)) for n in ("tri_att_start", "tri_att_end"))
-    h, d, inf = start.no_heads, start.mha.c_hidden, start.inf
+    h, d, inf = start.no_heads, q.child(start, "mha", (layers._GatedAttentionParams,)).c_hidden, start.inf
     for m in (start, end):
-        mha = q.child(m, "mha", (layers._GatedAttentionParams,))
+        mha = q.attr(q.child(m, "mha", (layers._GatedAttentionParams,)), "c_hidden")
+        q.attr(m, "c_in", "no_heads", "inf")
         if (m.c_in, m.no_heads, mha.c_hidden, m.inf) != (c, h, d, inf):
             raise _Refused
-        q.attr(m, "no_heads", "inf")
         q.norm(m, "layer_norm", c)
         q.linears(m, ("linear_z",), (h, c))
         q.linears(mha, ("linear_q", "linear_k", "linear_v", "linear_g"), (h * d, c))
@@ -192,7 +204,7 @@ def _pair_params(q, block):
 
 
 def _transition_params(q, block, name, c):
-    t = q.child(block, name, (layers.SwiGLUTransition,))
+    t = q.attr(q.child(block, name, (layers.SwiGLUTransition,)), "n")
     q.called.append(t)
     hid = t.n * c
     q.norm(t, "layer_norm", c)
@@ -209,11 +221,14 @@ def _pairformer_params(q, block, pair_block_type):
     a = q.child(block, "attn_pair_bias", (layers.AttentionPairBias,))
     q.called.append(a)
     mha = q.child(a, "mha", (layers._PairBiasAttentionParams,))
+    q.attr(a, "c_q", "c_z", "no_heads", "inf")
     c_s, c_z, h = a.c_q, dims[0], a.no_heads
-    hd = mha.linear_q.weight.shape[0]
-    if a.c_z != c_z or h < 1 or hd % h:
+    lin = q.child(mha, "linear_q", (torch.nn.Linear,))
+    weight = lin._parameters.get("weight")
+    if weight is None or a.c_z != c_z or h < 1 or weight.shape[0] % h:
+        q.links.append((lin._parameters, "weight", weight))
         raise _Refused
-    q.attr(a, "no_heads", "inf")
+    hd = weight.shape[0]
     q.norm(a, "layer_norm_z", c_z, optional_bias=True)
     q.linears(a, ("linear_z",), (h, c_z))
     q.norm(a, "layer_norm_a", c_s)
@@ -224,7 +239,7 @@ def _pairformer_params(q, block, pair_block_type):
     return dims, (c_s, h, hd // h, hid_s, a.inf)
 
 
-# block -> (parameters, dimensions), False where it is not served, or None: called once
+# block -> (parameters, dimensions, or None where the block is not served), or None: called once
 _plans = weakref.WeakKeyDictionary()
 # Token count from which a block's first call goes module by module and the parameters are looked for in the second: the
 # search takes 100 us or more before the first launch, and from here on issuing the modules keeps ahead of the GPU.
@@ -243,25 +258,24 @@ def _first_call(block, z):
 
 def _plan(block, build):
     plan = _plans.get(block)
-    if plan is None:
+    if plan is None or not plan[0].current():
         q = _Params()
         try:
             plan = (q, build(q))
-        except (_Refused, AttributeError, TypeError):
-            plan = False
+        except _Refused:
+            plan = q.refused()
+        except (AttributeError, TypeError):  # not what the search expects of a module of its type: looked at again next time
+            _plans[block] = None
+            return q, None
         _plans[block] = plan
     return plan
 
 
 def _gather(block, build, dtype):
     """(pointer array, dimensions) of the block's parameters, or None."""
-    plan = _plan(block, build)
-    if plan and not plan[0].current():
-        _plans.pop(block, None)
-        plan = _plan(block, build)
-    if not plan:
+    q, dims = _plan(block, build)
+    if dims is None:
         return None
-    q, dims = plan
     array = q.gather(dtype)
     if array is None:
         return None

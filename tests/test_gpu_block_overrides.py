@@ -76,3 +76,53 @@ def test_replaced_on_an_instance(monkeypatch, path, name):
     assert "of3_pairformer_stack_fwd" not in run() and len(seen) == 1
     del own.__dict__[name]
     assert run() == ["of3_pairformer_stack_fwd"]
+
+
+class _Wrapped(torch.nn.Linear):
+    pass
+
+
+def _own_class(m):
+    lin = m.blocks[0].pair_stack.tri_att_end.mha.linear_v
+    lin.__class__ = _Wrapped
+    return lambda: setattr(lin, "__class__", torch.nn.Linear)
+
+
+def _wrapped(m):
+    t = m.blocks[1].single_transition
+    lin = t.linear_out
+    t.linear_out = _Wrapped(lin.in_features, lin.out_features, bias=False).to(lin.weight)
+    t.linear_out.weight = lin.weight
+    return lambda: setattr(t, "linear_out", lin)
+
+
+def _parametrized(m):
+    mul = m.blocks[0].pair_stack.tri_mul_in
+    torch.nn.utils.parametrize.register_parametrization(mul.linear_b_g, "weight", torch.nn.Identity())
+    return lambda: torch.nn.utils.parametrize.remove_parametrizations(mul.linear_b_g, "weight")
+
+
+def _other_inf(m):
+    m.blocks[1].pair_stack.tri_att_start.inf = 2e9
+    return lambda: setattr(m.blocks[1].pair_stack.tri_att_start, "inf", 1e9)
+
+
+def _no_head_width(m):
+    q = m.blocks[0].attn_pair_bias.mha
+    lin = q.linear_q
+    del q.linear_q
+    q.linear_q = torch.nn.Identity()
+    q.linear_q.weight, q.linear_q.bias = lin.weight, lin.bias
+    return lambda: setattr(q, "linear_q", lin)
+
+
+@pytest.mark.parametrize("change", [_own_class, _wrapped, _parametrized, _other_inf, _no_head_width])
+def test_a_refused_block_is_served_once_it_is_restored(monkeypatch, change):
+    m, run = _setup(monkeypatch)
+    _block._plans.clear()
+    restore = change(m)
+    for _ in range(3):
+        assert "of3_pairformer_stack_fwd" not in run()
+    restore()
+    run()
+    assert run() == ["of3_pairformer_stack_fwd"]
