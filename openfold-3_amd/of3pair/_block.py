@@ -339,7 +339,7 @@ def run_pair_block(block, z, mask, inplace, attention_first=False, mask_trans=Tr
 
 def _pairformer_args(s, z, single_mask, pair_mask, c, c_s):
     """The tensors of a block's or a stack's call: (z4, mask arguments, single mask as fp32), or None."""
-    if not s.is_cuda or s.dtype is not z.dtype or not s.is_contiguous():
+    if not s.is_cuda or s.dtype is not z.dtype or not s.is_contiguous() or not F3._is_single(s):
         return None
     args = _pair_args(z, pair_mask)
     if not args or s.shape[:-1] != z.shape[:-2] or args[0].shape[-1] != c or s.shape[-1] != c_s:

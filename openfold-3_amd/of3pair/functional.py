@@ -242,6 +242,11 @@ def triangle_attention(x, mask, norm_weight, norm_bias, bias_weight, q_weight, k
     return _finish(x, x4, out4, lead, inplace)
 
 
+def _is_single(x: torch.Tensor) -> bool:
+    """Whether the transition takes x for the single representation."""
+    return x.shape[-1] == 384 or x.dim() < 3
+
+
 def swiglu_transition(x, mask, norm_weight, norm_bias, a_weight, b_weight, out_weight, add_residual: bool = False,
                       inplace: bool = False):
     """Update of transition.py:256-268 (LayerNorm, SwiGLU, linear_out, mask), or x + update when
@@ -252,7 +257,7 @@ def swiglu_transition(x, mask, norm_weight, norm_bias, a_weight, b_weight, out_w
     A tensor of fewer than three dimensions cannot be a pair tensor and is taken as rows [*, C] too."""
     code = _require_gpu(x, "x")
     lib = _lib.load()
-    if x.shape[-1] == 384 or x.dim() < 3:  # the single representation: position-wise over [*, C] rows
+    if _is_single(x):  # position-wise over [*, C] rows
         return _swiglu_transition_rows(x, mask, norm_weight, norm_bias, a_weight, b_weight, out_weight,
                                        add_residual, inplace, code)
     x4, lead = _flatten_pair(x)

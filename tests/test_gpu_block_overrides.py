@@ -126,3 +126,21 @@ def test_a_refused_block_is_served_once_it_is_restored(monkeypatch, change):
     restore()
     run()
     assert run() == ["of3_pairformer_stack_fwd"]
+
+
+@pytest.mark.parametrize("n", [30, 310])
+def test_widths_of_s_are_refused_as_by_the_modules(n):
+    """A batch of single representations has 384 channels; one without a batch has any.  The first call of a block, the
+    second and a stack's own agree."""
+    lib()
+    m = of3pair.PairFormerStack(64, 64, 16, 4, 64, 16, 4, no_blocks=2).to(DEV).eval()
+    s, z = torch.randn(n, 64, device=DEV), torch.randn(n, n, 64, device=DEV)
+    for _ in range(3):
+        with pytest.raises(ValueError):
+            m(s[None], z[None], None, None)
+    want = m(s, z, None, None)
+    for _ in range(2):
+        got = m(s, z, None, None)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        with pytest.raises(ValueError):
+            m(s[None], z[None], None, None)
