@@ -1246,7 +1246,10 @@ class StreamPair {
 // regions of a stack's workspace
 struct StackSpace {
   int64_t module, prepared, bias, single, total;
-  int64_t buffers;  // pair biases: one per block up to 64 MB of them, at least two
+  // pair biases: one per block up to 64 MB of them.  Above 32 MB it is one, as in the single block's call: the attention that
+  // reads it is over long before the next block's pair updates are (six blocks at N = 1100, bf16, one / two of them:
+  // 32.2 / 32.2 ms, 1357 / 1395 MB; four at N = 1024, fp32: 65.4 / 65.4 ms, 3058 / 3126 MB).
+  int64_t buffers;
 };
 static StackSpace stack_space(const BlockDims& d, int64_t blocks, int64_t C_s, int64_t H_s, int64_t D_s, int64_t HID_s) {
   StackSpace w;
@@ -1259,7 +1262,7 @@ static StackSpace stack_space(const BlockDims& d, int64_t blocks, int64_t C_s, i
   w.prepared = d.prepared_bytes() * (blocks < kPrepared ? blocks : kPrepared);
   w.bias = align256(d.B * H_s * d.N * d.N * (d.wide() ? 4 : 2));
   w.buffers = (64ll << 20) / w.bias;
-  if (w.buffers < 2) w.buffers = 2;
+  if (w.buffers < 1) w.buffers = 1;
   if (w.buffers > blocks) w.buffers = blocks;
   w.single = align256(attn > rows ? attn : rows);
   w.total = w.module + w.prepared + w.buffers * w.bias + w.single;
@@ -1291,6 +1294,8 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
   char* const bias0 = prepared + w.prepared;
   char* const single = bias0 + w.buffers * w.bias;
 
+  // block j overwrites the bias that attention j - buffers reads, and waits for attention j - ahead or the one after it
+  const int64_t ahead = w.buffers < 2 ? w.buffers : 2;
   StreamPair streams(static_cast<hipStream_t>(stream), static_cast<hipStream_t>(side_stream));
   BlockWeights k[kPrepared];
   int st = OF3_OK;
@@ -1320,7 +1325,7 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
     st = last ? streams.join() : streams.order(streams.main, streams.side, StreamPair::kBias);
     const hipStream_t on = last ? streams.main : streams.side;
     if (st != OF3_OK || (st = attention(i ? of3::kSingleAttend : of3::kSingleProject | of3::kSingleAttend, on)) != OF3_OK) break;
-    if (i + 2 < blocks && i + 2 >= w.buffers && (st = streams.record(on, StreamPair::kFree)) != OF3_OK) break;
+    if (i + ahead < blocks && i + ahead >= w.buffers && (st = streams.record(on, StreamPair::kFree)) != OF3_OK) break;
     st = of3_transition_rows_fwd(s_out, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : single_mask, ws_[11], ws_[12],
                                  ws_[13], ws_[14], ws_[15], s_out, B * N, C_s, HID_s, 1, single, w.single, dtype, on);
   }

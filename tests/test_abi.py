@@ -267,3 +267,15 @@ def test_transition_workspace_variant_validates_on_the_host(lib):
     args = (FAKE, xs, None, None, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, 1, 64, 128, 512, 1)
     assert lib.of3_transition_fwd_ws(*args, FAKE, need - 1, L.OF3_DTYPE_F32, None) == L.OF3_ENOSPC
     assert lib.of3_transition_fwd_ws(*args, FAKE + 4, need, L.OF3_DTYPE_F32, None) == L.OF3_EINVAL  # workspace alignment
+
+
+def test_a_stack_holds_one_large_pair_bias(lib):
+    """Pair biases of more than 32 MB are held one at a time, as by the single block's call; up to 64 MB of smaller ones."""
+    def size(dtype, n, blocks):
+        return lib.of3_pairformer_stack_workspace_bytes(dtype, blocks, 1, n, 128, 128, 4, 32, 512, 384, 16, 24, 1536)
+
+    for dtype, itemsize, large in ((1, 2, 2048), (0, 4, 768)):
+        prepared = size(dtype, 64, 4) - size(dtype, 64, 1) - 3 * 16 * 64 * 64 * itemsize  # the weights of three more blocks
+        assert 0 < prepared < 16 << 20
+        assert size(dtype, large, 48) - size(dtype, large, 1) == prepared
+        assert size(dtype, 384, 48) - size(dtype, 384, 1) <= prepared + (64 << 20)
