@@ -267,7 +267,11 @@ hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, 
   p.total = a.B * p.R * p.panels;
   p.HID = a.HID;
   p.add_residual = a.add_residual;
-  const bool large = p.total >= 4 * 256;  // two tiles of 64 positions for every CU
+  static int cache[kMaxDevices];
+  int cus = 0;
+  const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  if (e != hipSuccess) return e;
+  const bool large = p.total >= 4l * cus;  // two tiles of 64 positions for every CU
   if (a.HID % 256 != 0) return a.C == 128 ? launch<128, 4, 2>(p, stream) : launch<64, 4, 2>(p, stream);
   if (a.C == 128) return large ? launch<128, 8, 2>(p, stream) : launch<128, 8, 1>(p, stream);
   return large ? launch<64, 8, 2>(p, stream) : launch<64, 8, 1>(p, stream);
