@@ -1,0 +1,105 @@
+"""Block and stack calls from 300 tokens on, where a module's first call goes module by module: the later ones, which do not,
+against that first one bit for bit, and under a capture."""
+import pytest
+import torch
+
+from gpu_util import lib  # noqa: F401
+
+import of3pair
+from of3pair import _block
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+PAIRFORMER = lambda blocks: of3pair.PairFormerStack(384, 128, 24, 16, 128, 32, 4, no_blocks=blocks)  # noqa: E731
+MODULES = {
+    "pairformer block": lambda: of3pair.PairFormerBlock(384, 128, 24, 16, 128, 32, 4),
+    "pairformer stack": lambda: PAIRFORMER(3),
+    "pair block": lambda: of3pair.PairBlock(128, 128, 32, 4),
+    "pair stack": lambda: of3pair.PairStack(128, 128, 32, 4),
+    "template block": lambda: of3pair.TemplatePairBlock(64, 16, 64, 4),
+}
+
+
+def _setup(kind, dtype, n, padded, monkeypatch):
+    lib()
+    gen = torch.Generator(device=DEV).manual_seed(61)
+    m = MODULES[kind]()
+    with torch.no_grad():
+        for name, p in m.to(DEV).named_parameters():
+            if p.dim() == 2:
+                p.copy_(torch.randn(p.shape, generator=gen, device=DEV) * p.shape[1] ** -0.5)
+            else:
+                p.copy_((1.0 if name.endswith("weight") else 0.0) + 0.1 * torch.randn(p.shape, generator=gen, device=DEV))
+    m = m.to(dtype).eval()
+    c = 64 if kind == "template block" else 128
+    z = torch.randn(1, n, n, c, generator=gen, device=DEV).to(dtype)
+    tok = (torch.arange(n, device=DEV) < n - padded).float()[None]
+    pair = tok[:, :, None] * tok[:, None, :]
+    args = (z, pair)
+    if kind.startswith("pairformer"):
+        args = (torch.randn(1, n, 384, generator=gen, device=DEV).to(dtype), z, tok, pair)
+    calls = []
+    inner = _block._call
+    monkeypatch.setattr(_block, "_call", lambda fn, what, *a: (calls.append(what), inner(fn, what, *a))[1])
+
+    def run():
+        out = m(*args)
+        return out if isinstance(out, tuple) else (out,)
+
+    return run, calls
+
+
+def _equal(a, b):
+    return all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+# around whole tiles of the contraction and of the passes, and the transition's last rounds
+@pytest.mark.parametrize("n,padded", [(300, 0), (321, 40), (384, 38), (513, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("kind", sorted(MODULES))
+def test_later_calls_give_what_the_first_gave(monkeypatch, kind, dtype, n, padded):
+    run, calls = _setup(kind, dtype, n, padded, monkeypatch)
+    want = run()
+    assert calls == []
+    for _ in range(3):
+        assert _equal(run(), want)
+    name = "of3_pairformer_block_fwd" if kind.startswith("pairformer") else "of3_pair_block_fwd"
+    if kind == "pairformer stack":
+        assert calls[:3] == [name] * 3 and calls[3:] == ["of3_pairformer_stack_fwd"] * 2
+    else:
+        assert calls == [name] * 3
+    assert all(bool(torch.isfinite(t).all()) for t in want)
+
+
+@pytest.mark.parametrize("warm", [1, 3])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_capture_after_warm_up_calls(monkeypatch, dtype, warm):
+    run, _ = _setup("pairformer stack", dtype, 310, 20, monkeypatch)
+    for _ in range(warm):
+        want = [t.clone() for t in run()]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+    for _ in range(3):
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _equal(out, want)
+        assert _equal(run(), want)
+
+
+@pytest.mark.parametrize("no_blocks", [2, 5])
+def test_two_streams_at_ordinary_lengths(monkeypatch, no_blocks):
+    """The stack's call on a stream of the caller's own, blocks in place, against one block after the other."""
+    monkeypatch.setitem(MODULES, "pairformer stack", lambda: PAIRFORMER(no_blocks))
+    run, calls = _setup("pairformer stack", torch.bfloat16, 384, 38, monkeypatch)
+    want = run()
+    run()
+    del calls[:]
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(other):
+        got = [run() for _ in range(4)]
+    torch.cuda.current_stream().wait_stream(other)
+    assert all(_equal(g, want) for g in got) and calls == ["of3_pairformer_stack_fwd"] * 4
