@@ -111,35 +111,33 @@ __global__ __launch_bounds__(256, 3) void pair_bias_pass(PairBiasF32Args p, int 
 // plain FMA kernel took 160 us for 3 templates of 200^2 positions, at one dot product per thread
 constexpr int kTailC = 64, kTailOut = 128;
 // 16 outputs of position q from output o0 on with plain fused multiply-adds, for those that are NaN: an infinite or very
-// large weight or input has NaN among its three bf16 terms (single_x3_f32.hip).  ln: weights, then biases
-__device__ __forceinline__ void plain_tail(const TemplateTailF32Args& p, int b, long q, int o0, const float* ln, f32x16_t& out) {
-  constexpr int C = kTailC, K = 2;  // inputs at a time (4: 165 registers, three work-groups per CU)
-  out = zero16();
+// large weight or input has NaN among its three bf16 terms (single_x3_f32.hip).  The sums are kept in the output row, so
+// that the kernel needs no registers for them (with 16 more it ran at four work-groups per CU instead of five, 25 us in
+// place of 19 for three templates of 200^2).  ln: weights, then biases
+__device__ __forceinline__ void plain_tail(const TemplateTailF32Args& p, int b, long q, int o0, const float* ln) {
+  constexpr int C = kTailC;
+  float* out = p.out + ((size_t)b * p.P + q) * kTailOut + o0;
 #pragma unroll 1
-  for (int k0 = 0; k0 < C; k0 += K) {
-    float x[K];
-#pragma unroll
-    for (int e = 0; e < K; ++e) x[e] = 0.f;
+  for (int v = 0; v < 16; ++v) out[v] = 0.f;
+#pragma unroll 1
+  for (int k = 0; k < C; ++k) {
+    float x = 0.f;
 #pragma unroll 1
     for (int t = 0; t < p.T; ++t) {
       const float* row = p.t + (((size_t)b * p.T + t) * p.P + q) * C;
-      float mean = 0.f, var = 0.f;
-      if (p.apply_ln) {
-        for (int c = 0; c < C; ++c) mean += row[c];
-        mean *= 1.f / C;
-        for (int c = 0; c < C; ++c) var += (row[c] - mean) * (row[c] - mean);
+      if (!p.apply_ln) {
+        x += row[k];
+        continue;
       }
-      const float rstd = 1.0f / sqrtf(var * (1.f / C) + kEps);
-#pragma unroll
-      for (int e = 0; e < K; ++e) x[e] += p.apply_ln ? (row[k0 + e] - mean) * rstd * ln[k0 + e] + ln[C + k0 + e] : row[k0 + e];
+      float mean = 0.f, var = 0.f;
+      for (int c = 0; c < C; ++c) mean += row[c];
+      mean *= 1.f / C;
+      for (int c = 0; c < C; ++c) var += (row[c] - mean) * (row[c] - mean);
+      x += (row[k] - mean) * (1.0f / sqrtf(var * (1.f / C) + kEps)) * ln[k] + ln[C + k];
     }
-    const float* w = p.w + (size_t)o0 * C + k0;
-#pragma unroll
-    for (int e = 0; e < K; ++e) {
-      const float u = fmaxf(x[e] / (float)p.T, 0.f);
-#pragma unroll
-      for (int v = 0; v < 16; ++v) out[v] = fmaf(u, w[v * C + e], out[v]);
-    }
+    x = fmaxf(x / (float)p.T, 0.f);
+#pragma unroll 1
+    for (int v = 0; v < 16; ++v) out[v] = fmaf(x, p.w[(size_t)(o0 + v) * C + k], out[v]);
   }
 }
 
@@ -198,7 +196,7 @@ __global__ __launch_bounds__(256, 3) void template_tail_pass(TemplateTailF32Args
                                                                       fmaxf(sum[u].z / T, 0.f), fmaxf(sum[u].w / T, 0.f)));
     }
     __syncthreads();  // the tile is complete
-    f32x16_t acc = unit_product<C, true>(tile, w);
+    const f32x16_t acc = unit_product<C, true>(tile, w);
     __syncthreads();  // everybody has read it
     const Lane at = lane_here();
     const int b = id / tiles_per_b;
@@ -207,8 +205,8 @@ __global__ __launch_bounds__(256, 3) void template_tail_pass(TemplateTailF32Args
     bool again = false;
 #pragma unroll
     for (int v = 0; v < 16; ++v) again |= acc[v] != acc[v];
-    if (again) plain_tail(p, b, q, 32 * wave + 16 * at.lh, ln, acc);
-    store_row16(nullptr, p.out + ((size_t)b * p.P + q) * kTailOut + 32 * wave + 16 * at.lh, acc, false);
+    if (!again) store_row16(nullptr, p.out + ((size_t)b * p.P + q) * kTailOut + 32 * wave + 16 * at.lh, acc, false);
+    else plain_tail(p, b, q, 32 * wave + 16 * at.lh, ln);
   }
 }
 
