@@ -257,7 +257,7 @@ __global__ __launch_bounds__(64 * kLnWaves) void single_proj_x3_f32(SingleAttnF3
   const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
   if (pos0 + r >= rows) return;
   float4 v = sum_partials<kLnWaves>(part, kPart, r, c4);
-  if (has_nan(v)) v = ln_plain_dots(p.a, pos0, r, p.C, p.ln_w, p.ln_b, W[0] + (size_t)4 * c4 * p.C, red);
+  if (__builtin_expect(has_nan(v), 0)) v = ln_plain_dots(p.a, pos0, r, p.C, p.ln_w, p.ln_b, W[0] + (size_t)4 * c4 * p.C, red);
   if (kind == 0) {
     const float scale = 1.0f / sqrtf((float)p.D);
     const float* bq = p.bq + o0 + 4 * c4;
@@ -293,6 +293,9 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
+  // every pointer and size, asked for at once: one trip to the kernel's arguments instead of three or four in a row
+  __asm__ volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.pair_bias), "s"(p.mask), "s"(p.N), "s"(p.H), "s"(p.D), "s"(p.g), "s"(p.og),
+                   "s"(pb_vec));
   const int N = p.N, H = p.H, D = p.D, HD = H * D;
   const int h = blockIdx.y, b = blockIdx.z;
   const int qi = blockIdx.x * 32 + l32;
@@ -318,13 +321,8 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
     for (int e = 0; e < 8; ++e) v[e] = x[8 * s + e];
     split8(v, op[0], op[1], op[2]);
   };
-  u32x4_t qop[2][3];
-  {
-    float x[16];
-    load_row(p.q, qrow, x);
-    split_step(x, 0, qop[0]);
-    split_step(x, 1, qop[1]);
-  }
+  float xq[16];
+  load_row(p.q, qrow, xq);
   const float* pb = p.pair_bias + (((size_t)b * H + h) * N + qrow) * N;
   const float* vcol = p.v + bN * HD + h * D + (l32 < D ? l32 : 0);
   const float vkeep = l32 < D ? 1.f : 0.f;
@@ -358,6 +356,9 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
   const int nkt = (N + 31) / 32;
   Raw cur, nxt;
   if (wave < nkt) load_tile(wave, cur);
+  u32x4_t qop[2][3];  // split behind the first tile's loads, which are under way while the query arrives
+  split_step(xq, 0, qop[0]);
+  split_step(xq, 1, qop[1]);
   for (int kt = wave; kt < nkt; kt += kAttnWaves) {
     if (kt + kAttnWaves < nkt) load_tile(kt + kAttnWaves, nxt);  // in flight under this tile's arithmetic
     const int k0 = 32 * kt;
@@ -424,6 +425,12 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
     cur = nxt;
   }
   // ---- merge the waves: common maximum, rescaled sums and accumulators
+  const size_t off = (bN + qrow) * HD + h * D + 4 * lh;
+  float4 gate[4];
+  if (wave == 0) {  // asked for before the barrier: behind the test for NaN they would be waited for
+#pragma unroll
+    for (int a = 0; a < 4; ++a) gate[a] = *reinterpret_cast<const float4*>(p.g + off + (8 * a < D ? 8 * a : 0));
+  }
   merge[wave][16][lane] = m_run;  // -inf for a wave without tiles
   merge[wave][17][lane] = l_run + __shfl_xor(l_run, 32, 64);
 #pragma unroll
@@ -471,11 +478,10 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
     }
   }
   const float inv = 1.0f / l_tot;
-  const size_t off = (bN + qrow) * HD + h * D + 4 * lh;
 #pragma unroll
   for (int a = 0; a < 4; ++a)
     if (8 * a < D) {  // registers 4 a .. + 3 are head channels 8 a + 4 lh .. + 3
-      const float4 g = *reinterpret_cast<const float4*>(p.g + off + 8 * a);
+      const float4 g = gate[a];
       *reinterpret_cast<float4*>(p.og + off + 8 * a) = make_float4(oacc[4 * a] * inv * g.x, oacc[4 * a + 1] * inv * g.y,
                                                                    oacc[4 * a + 2] * inv * g.z, oacc[4 * a + 3] * inv * g.w);
     }
@@ -491,7 +497,7 @@ __global__ __launch_bounds__(64 * kOutWaves) void single_out_x3_f32(SingleAttnF3
   const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
   if (pos0 + r >= rows) return;
   float4 v = sum_partials<kOutWaves>(part, kPart, r, c4);
-  if (has_nan(v)) {
+  if (__builtin_expect(has_nan(v), 0)) {
     const float4* x = reinterpret_cast<const float4*>(p.og + (pos0 + r) * HD);
     v = plain_dots([&](int k) { return x[k]; }, p.wo + (size_t)(o0 + 4 * c4) * HD, HD);
   }
@@ -515,8 +521,8 @@ __global__ __launch_bounds__(64 * kLnWaves) void row_hidden_x3_f32(RowTransition
   const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
   if (pos0 + r >= p.rows) return;
   float4 a = sum_partials<kLnWaves>(part, 2 * kPart, r, c4), b = sum_partials<kLnWaves>(part + kPart, 2 * kPart, r, c4);
-  if (has_nan(a)) a = ln_plain_dots(p.x, pos0, r, p.C, p.ln_w, p.ln_b, W[0] + (size_t)4 * c4 * p.C, red);
-  if (has_nan(b)) b = ln_plain_dots(p.x, pos0, r, p.C, p.ln_w, p.ln_b, W[1] + (size_t)4 * c4 * p.C, red);
+  if (__builtin_expect(has_nan(a), 0)) a = ln_plain_dots(p.x, pos0, r, p.C, p.ln_w, p.ln_b, W[0] + (size_t)4 * c4 * p.C, red);
+  if (__builtin_expect(has_nan(b), 0)) b = ln_plain_dots(p.x, pos0, r, p.C, p.ln_w, p.ln_b, W[1] + (size_t)4 * c4 * p.C, red);
   float4 v;
   v.x = a.x * sigmoid_f32(a.x) * b.x;
   v.y = a.y * sigmoid_f32(a.y) * b.y;
@@ -536,7 +542,7 @@ __global__ __launch_bounds__(64 * kRowOutWaves) void row_out_x3_f32(RowTransitio
   const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
   if (pos0 + r >= p.rows) return;
   float4 v = sum_partials<kRowOutWaves>(part, kPart, r, c4);
-  if (has_nan(v)) {
+  if (__builtin_expect(has_nan(v), 0)) {
     const float4* x = reinterpret_cast<const float4*>(p.hidden + (pos0 + r) * p.HID);
     v = plain_dots([&](int k) { return x[k]; }, p.wout + (size_t)(o0 + 4 * c4) * p.HID, p.HID);
   }
