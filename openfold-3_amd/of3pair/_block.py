@@ -59,7 +59,7 @@ for _mul in _MULS:
     written(_mul, "_weights")
 # what a pair block calls on itself
 PAIR_METHODS = ("tri_mul_out_in", "tri_att_start_end", "_modules_forward", "_mul", "_att")
-_CALL = frozenset(("forward", "_compiled_call_impl"))
+_CALL = ("forward", "_compiled_call_impl")
 
 
 class _Params:
@@ -73,9 +73,10 @@ class _Params:
         self.shapes = []   # what refs must have; None where a parameter may be absent
         self.entries = []  # (index into refs, first row): the pointers handed over
         self.called = []   # submodules that the block calls as modules
+        self.own = []      # (attributes of a module, a name it may not have of its own)
+        self.attrs = []    # (attributes of a module, name, the value that a call uses)
+        self.noted = []    # the same of values that the search alone looks at
         self.types = None  # of what links held, where the block was refused
-        self.methods = []  # (attributes of a module, names it may not have of its own)
-        self.attrs = []    # (attributes of a module, name, the value the dimensions were taken from)
         self.last = (None, None, None)  # pointers of refs, dtype and pointer array of the last call
 
     def child(self, parent, name, kinds=None):
@@ -88,7 +89,17 @@ class _Params:
     def attr(self, module, *names):
         for name in names:
             self.attrs.append((module.__dict__, name, getattr(module, name)))
-        return module
+
+    def note(self, module, *names):
+        for name in names:
+            self.noted.append((module.__dict__, name, getattr(module, name)))
+
+    def no_own(self, module, names):
+        self.own += [(module.__dict__, name) for name in names]
+
+    def calls(self, module):
+        self.called.append(module)
+        self.no_own(module, _CALL)
 
     def refused(self):
         """Notes the types too: a module may change its own, as one under a parametrization does."""
@@ -97,8 +108,11 @@ class _Params:
 
     def current(self):
         """Whether the block still holds the submodules and attributes that it held."""
-        if self.types is not None and any(type(link[2]) is not t for link, t in zip(self.links, self.types)):
-            return False
+        if self.types is not None:
+            if any(type(link[2]) is not t for link, t in zip(self.links, self.types)):
+                return False
+            if any(owner.get(name) != value for owner, name, value in self.noted):
+                return False
         for owner, name, sub in self.links:
             if owner.get(name) is not sub:
                 return False
@@ -165,14 +179,14 @@ class _Params:
 
 def _pair_params(q, block):
     """Appends what of3_pair_block_fwd takes; returns (C, CH, H, D, HID, inf)."""
-    q.methods.append((block.__dict__.keys(), PAIR_METHODS))
+    q.no_own(block, PAIR_METHODS)
     mul_out, mul_in = q.child(block, "tri_mul_out", _MULS), q.child(block, "tri_mul_in", _MULS)
     c, ch = mul_out.c_z, mul_out.c_hidden
     for m, outgoing in ((mul_out, True), (mul_in, False)):
         q.attr(m, "c_z", "c_hidden", "_outgoing")
         if _MULS[type(m)] is not outgoing or m._outgoing is not outgoing or (m.c_z, m.c_hidden) != (c, ch):
             raise _Refused
-        q.methods.append((m.__dict__.keys(), ("_weights",)))
+        q.no_own(m, ("_weights",))
         q.norm(m, "layer_norm_in", c)
         q.norm(m, "layer_norm_out", ch)
         if isinstance(m, layers.FusedTriangleMultiplicativeUpdate):
@@ -189,8 +203,10 @@ def _pair_params(q, block):
     start, end = (q.child(block, n, (layers.TriangleAttention,)) for n in ("tri_att_start", "tri_att_end"))
     h, d, inf = start.no_heads, q.child(start, "mha", (layers._GatedAttentionParams,)).c_hidden, start.inf
     for m in (start, end):
-        mha = q.attr(q.child(m, "mha", (layers._GatedAttentionParams,)), "c_hidden")
-        q.attr(m, "c_in", "no_heads", "inf")
+        mha = q.child(m, "mha", (layers._GatedAttentionParams,))
+        q.attr(m, "no_heads", "inf")
+        q.note(m, "c_in")
+        q.note(mha, "c_hidden")
         if (m.c_in, m.no_heads, mha.c_hidden, m.inf) != (c, h, d, inf):
             raise _Refused
         q.norm(m, "layer_norm", c)
@@ -204,8 +220,9 @@ def _pair_params(q, block):
 
 
 def _transition_params(q, block, name, c):
-    t = q.attr(q.child(block, name, (layers.SwiGLUTransition,)), "n")
-    q.called.append(t)
+    t = q.child(block, name, (layers.SwiGLUTransition,))
+    q.calls(t)
+    q.note(t, "n")
     hid = t.n * c
     q.norm(t, "layer_norm", c)
     sw = q.child(t, "swiglu", (layers._SwiGLUParams,))
@@ -216,12 +233,13 @@ def _transition_params(q, block, name, c):
 
 def _pairformer_params(q, block, pair_block_type):
     pair = q.child(block, "pair_stack", (pair_block_type,))
-    q.called.append(pair)
+    q.calls(pair)
     dims = _pair_params(q, pair)
     a = q.child(block, "attn_pair_bias", (layers.AttentionPairBias,))
-    q.called.append(a)
+    q.calls(a)
     mha = q.child(a, "mha", (layers._PairBiasAttentionParams,))
-    q.attr(a, "c_q", "c_z", "no_heads", "inf")
+    q.attr(a, "no_heads", "inf")
+    q.note(a, "c_q", "c_z")
     c_s, c_z, h = a.c_q, dims[0], a.no_heads
     lin = q.child(mha, "linear_q", (torch.nn.Linear,))
     weight = lin._parameters.get("weight")
@@ -280,12 +298,11 @@ def _gather(block, build, dtype):
     if array is None:
         return None
     for m in q.called:  # modules that the block would call: their hooks, their mode and a forward of their own are theirs
-        if m.training or m._forward_hooks or m._forward_pre_hooks or not _CALL.isdisjoint(m.__dict__):
+        if m.training or m._forward_hooks or m._forward_pre_hooks:
             return None
-    for own, names in q.methods:
-        for name in names:
-            if name in own:
-                return None
+    for attributes, name in q.own:
+        if name in attributes:
+            return None
     if _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks:
         return None
     return array, dims
@@ -389,7 +406,7 @@ def run_pairformer_stack(blocks, block_type, pair_block_type, s, z, single_mask,
         return None
     arrays, dims = [], None
     for block in blocks:
-        if type(block) is not block_type or block.training or block._forward_hooks or block._forward_pre_hooks or not _CALL.isdisjoint(block.__dict__):
+        if type(block) is not block_type or block.training or block._forward_hooks or block._forward_pre_hooks or any(name in block.__dict__ for name in _CALL):
             return None
         found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
         if not found or (dims is not None and found[1] != dims):
