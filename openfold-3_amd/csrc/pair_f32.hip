@@ -1606,8 +1606,9 @@ __global__ __launch_bounds__(128 * kXRows, 2) void triattn_core_x3_f32(TriattnF3
   // whenever the exponentials neither overflowed nor lost the row's largest terms, which the row sum tells:
   // 2^-60 <= sum <= 2^60 (an overflow leaves +inf, a row of masked keys leaves 0).  A work-group with a query
   // outside that range (its loads and barriers are collective) runs the pass again with running maxima.
-  // A work-group with a row whose sampled keys are all masked goes to the second pass at once, as in the bf16 core: one block at
-  // N = 384, 38 tokens padded, 1850 -> 1825 us, four updates at N = 700, 70 padded, 5813 -> 5740, without padding the same.
+  // A work-group with a row whose sampled keys are all masked goes to the second pass at once, as in the bf16 core: without /
+  // with the samples, us, one block at N = 384, 38 tokens padded, 1734 / 1720, three templates of 200, 20 padded, 1194 / 1179;
+  // without padding the same.
   first_loads();
   const uint64_t masked = __builtin_amdgcn_ballot_w64(sample < -1e8f);
   bool again = false;

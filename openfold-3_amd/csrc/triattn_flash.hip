@@ -420,9 +420,9 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
   // A work-group with a row whose sampled keys (its own token, the first, the middle and the last) are all masked is
   // taken for one with a padded token, which fails that test for certain, and goes to the second pass at once; a wrong
   // guess costs it the offsets' arithmetic and nothing else.  A launch that fits the chip at once lasts as long as its
-  // work-groups with padded rows, of a larger one they are a share: two trunk blocks at N = 384, 38 of them padded,
-  // 1073 -> 1040 us; one at N = 2048, 256 padded, 25.1 -> 23.9 ms; two templates of 187, 12 padded, 391 -> 374 us; without
-  // padding no difference (N = 768).
+  // work-groups with padded rows, of a larger one they are a share: without / with the samples, us, two trunk blocks at
+  // N = 384, 38 of them padded, 1152 / 1126; four at 200, 23 padded, 975 / 946; one at 2048, 256 padded, 25.8 / 24.5 ms; two
+  // templates of 187, 12 padded, 384 / 366; without padding no difference (N = 768).
   first_loads();
   const uint64_t masked = __builtin_amdgcn_ballot_w64(sample < kMaskedBelow);
   bool again = false;
