@@ -99,7 +99,7 @@ __device__ __forceinline__ float4 plain_dots(Row&& x, const float* W, int K) {
   auto add = [](float acc, const float4& a, const float4& w) { return fmaf(a.w, w.w, fmaf(a.z, w.z, fmaf(a.y, w.y, fmaf(a.x, w.x, acc)))); };
   auto weights = [&](int row, int k) { return *reinterpret_cast<const float4*>(W + (size_t)row * K + 4 * k); };
 #pragma unroll 1
-  for (int k = 0; k < K / 4; ++k) {
+  for (int k = 0; k < K / 4 && !(s.x != s.x && s.y != s.y && s.z != s.z && s.w != s.w); ++k) {  // NaN stays NaN
     const float4 a = x(k);
     s.x = add(s.x, a, weights(0, k)), s.y = add(s.y, a, weights(1, k)), s.z = add(s.z, a, weights(2, k)), s.w = add(s.w, a, weights(3, k));
   }
@@ -465,10 +465,15 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
     m_tot = ninf, l_tot = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; ++v) oacc[v] = 0.f;
+    bool lost = false;  // a logit that is NaN, or +inf: so is the whole row
 #pragma unroll 1
-    for (int key = 0; key < N; ++key) m_tot = fmaxf(m_tot, logit(key));
+    for (int key = 0; key < N && !lost; ++key) {
+      const float x = logit(key);
+      lost = !(x < __builtin_inff());
+      m_tot = lost ? x - x : fmaxf(m_tot, x);
+    }
 #pragma unroll 1
-    for (int key = 0; key < N; ++key) {
+    for (int key = 0; key < (lost ? 1 : N); ++key) {
       const float w = exp_neg(logit(key) - m_tot);
       const float* vr = p.v + (bN + key) * HD + h * D + 4 * lh;
       l_tot += w;
