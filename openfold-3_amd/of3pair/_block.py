@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import operator
 import weakref
 
 import torch
@@ -73,10 +74,11 @@ class _Params:
         self.shapes = []   # what refs must have; None where a parameter may be absent
         self.entries = []  # (index into refs, first row): the pointers handed over
         self.called = []   # submodules that the block calls as modules
-        self.own = []      # (attributes of a module, a name it may not have of its own)
+        self.kinds = []    # (a module whose methods the block calls, its type)
+        self.own = []      # (attributes of such a module, a name it may not have of its own)
         self.attrs = []    # (attributes of a module, name, the value that a call uses)
         self.noted = []    # the same of values that the search alone looks at
-        self.types = None  # of what links held, where the block was refused
+        self.held = []     # links and attrs by columns
         self.last = (None, None, None)  # pointers of refs, dtype and pointer array of the last call
 
     def child(self, parent, name, kinds=None):
@@ -95,29 +97,30 @@ class _Params:
             self.noted.append((module.__dict__, name, getattr(module, name)))
 
     def no_own(self, module, names):
+        if (module, type(module)) not in self.kinds:
+            self.kinds.append((module, type(module)))
         self.own += [(module.__dict__, name) for name in names]
 
     def calls(self, module):
         self.called.append(module)
         self.no_own(module, _CALL)
 
-    def refused(self):
-        """Notes the types too: a module may change its own, as one under a parametrization does."""
-        self.types = [type(held) for _, _, held in self.links]
-        return self, None
+    def sealed(self, dims):
+        """The plan of a finished search; dims None: the block is refused, and the types of what was looked at count too (a
+        module may change its own, as one under a parametrization does)."""
+        if dims is None:
+            self.attrs += self.noted
+            self.kinds += [(held, type(held)) for _, _, held in self.links if held is not None]
+        self.held = [tuple(zip(*rows)) or ((), (), ()) for rows in (self.links, self.attrs)]
+        return self, dims
 
     def current(self):
         """Whether the block still holds the submodules and attributes that it held."""
-        if self.types is not None:
-            if any(type(link[2]) is not t for link, t in zip(self.links, self.types)):
-                return False
-            if any(owner.get(name) != value for owner, name, value in self.noted):
-                return False
-        for owner, name, sub in self.links:
-            if owner.get(name) is not sub:
-                return False
-        for owner, name, value in self.attrs:
-            if owner.get(name) != value:
+        (owners, names, subs), (attributes, of, values) = self.held
+        if any(map(operator.is_not, map(dict.get, owners, names), subs)) or tuple(map(dict.get, attributes, of)) != values:
+            return False
+        for m, kind in self.kinds:
+            if type(m) is not kind:
                 return False
         return True
 
@@ -279,9 +282,9 @@ def _plan(block, build):
     if plan is None or not plan[0].current():
         q = _Params()
         try:
-            plan = (q, build(q))
+            plan = q.sealed(build(q))
         except _Refused:
-            plan = q.refused()
+            plan = q.sealed(None)
         except (AttributeError, TypeError):  # not what the search expects of a module of its type: looked at again next time
             _plans[block] = None
             return q, None

@@ -78,6 +78,23 @@ def test_replaced_on_an_instance(monkeypatch, path, name):
     assert run() == ["of3_pairformer_stack_fwd"]
 
 
+@pytest.mark.parametrize("path,name", [("pair_stack", "tri_att_start_end"), ("single_transition", "forward"), ("attn_pair_bias", "forward"),
+                                       ("pair_stack.tri_mul_in", "_weights")])
+def test_another_class_given_to_an_instance(monkeypatch, path, name):
+    m, run = _setup(monkeypatch)
+    own, seen = m.blocks[0].get_submodule(path), []
+    kind = type(own)
+
+    def put(self, *args, **kwargs):
+        seen.append(name)
+        return getattr(kind, name)(self, *args, **kwargs)
+
+    own.__class__ = type("Other", (kind,), {name: put})
+    assert "of3_pairformer_stack_fwd" not in run() and len(seen) == 1
+    own.__class__ = kind
+    assert run() == ["of3_pairformer_stack_fwd"]
+
+
 class _Wrapped(torch.nn.Linear):
     pass
 
@@ -144,3 +161,21 @@ def test_widths_of_s_are_refused_as_by_the_modules(n):
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
         with pytest.raises(ValueError):
             m(s[None], z[None], None, None)
+
+
+def test_a_refused_block_with_another_weight(monkeypatch):
+    """A block refused over a parameter's shape is compared by that parameter, not by its values."""
+    m, run = _setup(monkeypatch)
+    a = m.blocks[0].attn_pair_bias
+    weight, bias, heads = a.mha.linear_q.weight, a.mha.linear_q.bias, a.no_heads
+    a.no_heads = 5  # 384 channels are no five heads
+    with pytest.raises(ValueError):
+        run()
+    a.mha.linear_q.weight = torch.nn.Parameter(weight.detach().clone())
+    with pytest.raises(ValueError):
+        run()
+    a.no_heads = heads
+    run()
+    assert run() == ["of3_pairformer_stack_fwd"]
+    a.mha.linear_q.weight, a.mha.linear_q.bias = weight, bias
+    assert run() == ["of3_pairformer_stack_fwd"]
