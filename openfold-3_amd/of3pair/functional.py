@@ -86,6 +86,8 @@ def release_workspaces():
     _workspaces.clear()
     _in_graph.clear()
     _retired.clear()
+    if not _own_streams or torch.cuda.is_current_stream_capturing():
+        return  # a stream is waited for before it goes, which a capture does not allow: kept until the next release
     with _side_lock:
         _sides.clear()
         for device, own in _own_streams.items():

@@ -96,3 +96,23 @@ def test_many_callers_streams_and_release():
     assert not F3._sides and not any(F3._own_streams.values())
     got = m(s, z, None, None)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def test_release_under_a_capture_keeps_the_streams():
+    lib()
+    m, s, z, want = _stack(33)
+    x = torch.zeros(64, device=DEV)
+    kept = {d: list(own) for d, own in F3._own_streams.items()}
+    assert any(kept.values())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x.add_(1.0)
+        F3.release_workspaces()
+    assert F3._own_streams == kept
+    for _ in range(3):
+        graph.replay()
+        got = m(s, z, None, None)
+        torch.cuda.synchronize()
+    assert float(x[0]) == 3.0 and torch.equal(got[0], want[0])
+    F3.release_workspaces()
+    assert not any(F3._own_streams.values())
