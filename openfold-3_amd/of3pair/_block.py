@@ -69,7 +69,7 @@ class _Params:
     judged, so that a block that was refused is searched again once that has changed."""
 
     def __init__(self):
-        self.links = []    # (children or parameters of a module, name, what they held, or None)
+        self.owners, self.names, self.held = [], [], []  # children or parameters of a module, name, what they held, or None
         self.refs = []     # (parameters of a module, name, number of values)
         self.shapes = []   # what refs must have; None where a parameter may be absent
         self.entries = []  # (index into refs, first row): the pointers handed over
@@ -78,12 +78,17 @@ class _Params:
         self.own = []      # (attributes of such a module, a name it may not have of its own)
         self.attrs = []    # (attributes of a module, name, the value that a call uses)
         self.noted = []    # the same of values that the search alone looks at
-        self.held = []     # links and attrs by columns
         self.last = (None, None, None)  # pointers of refs, dtype and pointer array of the last call
 
+    def link(self, owner, name, held):
+        self.owners.append(owner)
+        self.names.append(name)
+        self.held.append(held)
+
     def child(self, parent, name, kinds=None):
-        sub = parent._modules.get(name)
-        self.links.append((parent._modules, name, sub))
+        children = parent._modules
+        sub = children.get(name)
+        self.link(children, name, sub)
         if sub is None or (kinds is not None and type(sub) not in kinds):
             raise _Refused
         return sub
@@ -97,28 +102,34 @@ class _Params:
             self.noted.append((module.__dict__, name, getattr(module, name)))
 
     def no_own(self, module, names):
-        if (module, type(module)) not in self.kinds:
-            self.kinds.append((module, type(module)))
-        self.own += [(module.__dict__, name) for name in names]
+        attributes = module.__dict__
+        for name in names:
+            self.own.append((attributes, name))
+
+    def uses(self, module, names):
+        """Of a submodule.  Nothing here may hold the block itself: the plans are kept for as long as it lives."""
+        self.kinds.append((module, type(module)))
+        self.no_own(module, names)
 
     def calls(self, module):
         self.called.append(module)
-        self.no_own(module, _CALL)
+        self.uses(module, _CALL)
 
     def sealed(self, dims):
         """The plan of a finished search; dims None: the block is refused, and the types of what was looked at count too (a
         module may change its own, as one under a parametrization does)."""
         if dims is None:
             self.attrs += self.noted
-            self.kinds += [(held, type(held)) for _, _, held in self.links if held is not None]
-        self.held = [tuple(zip(*rows)) or ((), (), ()) for rows in (self.links, self.attrs)]
+            self.kinds += [(held, type(held)) for held in self.held if held is not None]
         return self, dims
 
     def current(self):
         """Whether the block still holds the submodules and attributes that it held."""
-        (owners, names, subs), (attributes, of, values) = self.held
-        if any(map(operator.is_not, map(dict.get, owners, names), subs)) or tuple(map(dict.get, attributes, of)) != values:
+        if any(map(operator.is_not, map(dict.get, self.owners, self.names), self.held)):
             return False
+        for attributes, name, value in self.attrs:
+            if attributes.get(name) != value:
+                return False
         for m, kind in self.kinds:
             if type(m) is not kind:
                 return False
@@ -126,7 +137,7 @@ class _Params:
 
     def param(self, module, name, shape, optional=False):
         if name not in module._parameters:
-            self.links.append((module._parameters, name, None))
+            self.link(module._parameters, name, None)
             raise _Refused
         self.entries.append((len(self.refs), 0))
         self.refs.append((module._parameters, name, math.prod(shape)))
@@ -139,16 +150,18 @@ class _Params:
 
     def linears(self, module, names, shape, bias=False):
         """Of several layers of one shape, written out: they are most of a block."""
-        children, links, entries, refs, shapes = module._modules, self.links, self.entries, self.refs, self.shapes
+        children, entries, refs, shapes = module._modules, self.entries, self.refs, self.shapes
         want, count = (shape, False), math.prod(shape)
-        for name in names:
-            lin = children.get(name)
-            links.append((children, name, lin))
+        found = [children.get(name) for name in names]
+        self.owners += [children] * len(found)
+        self.names += names
+        self.held += found
+        for lin in found:
             if type(lin) is not torch.nn.Linear:
                 raise _Refused
             own = lin._parameters
             if "weight" not in own:
-                links.append((own, "weight", None))
+                self.link(own, "weight", None)
                 raise _Refused
             entries.append((len(refs), 0))
             refs.append((own, "weight", count))
@@ -189,7 +202,7 @@ def _pair_params(q, block):
         q.attr(m, "c_z", "c_hidden", "_outgoing")
         if _MULS[type(m)] is not outgoing or m._outgoing is not outgoing or (m.c_z, m.c_hidden) != (c, ch):
             raise _Refused
-        q.no_own(m, ("_weights",))
+        q.uses(m, ("_weights",))
         q.norm(m, "layer_norm_in", c)
         q.norm(m, "layer_norm_out", ch)
         if isinstance(m, layers.FusedTriangleMultiplicativeUpdate):
@@ -247,7 +260,7 @@ def _pairformer_params(q, block, pair_block_type):
     lin = q.child(mha, "linear_q", (torch.nn.Linear,))
     weight = lin._parameters.get("weight")
     if weight is None or a.c_z != c_z or h < 1 or weight.shape[0] % h:
-        q.links.append((lin._parameters, "weight", weight))
+        q.link(lin._parameters, "weight", weight)
         raise _Refused
     hd = weight.shape[0]
     q.norm(a, "layer_norm_z", c_z, optional_bias=True)
