@@ -11,19 +11,31 @@
 namespace of3 {
 
 // The whole 128-wide pieces of every row come first (full_per_row per row), then the remaining N % 128
-// columns in pieces of 2^tail_shift columns (the smallest power of two >= 2^min_shift that covers them)
-// x (128 >> tail_shift) consecutive rows.
+// columns in pieces of 2^s columns x (128 >> s) consecutive rows, 2^s >= 2^min_shift: one power of two that covers them, or two
+// (72 columns: 64 + 8) where that makes fewer tiles.  tail_shift: s of the first piece + 256 * s of the second, 0 if there is
+// none.  N = 200 takes 313 tiles with two and 400 with one.
 struct RaggedTiles {
   int full_per_row, tail_shift, per_batch;
 };
+OF3_HD inline int tiles_of_columns(int N, int shift) {  // tiles of N rows x 2^shift columns
+  const int rows = 128 >> shift;
+  return (N + rows - 1) / rows;
+}
 inline RaggedTiles ragged_tiles(int N, int min_shift = 3) {
   RaggedTiles t;
   t.full_per_row = N / 128;
   const int r = N % 128;
   t.tail_shift = r ? min_shift : 7;
   while ((1 << t.tail_shift) < r) ++t.tail_shift;
-  const int rows = 128 >> t.tail_shift;
-  t.per_batch = N * t.full_per_row + (r ? (N + rows - 1) / rows : 0);
+  int tail = r ? tiles_of_columns(N, t.tail_shift) : 0;
+  const int s1 = t.tail_shift - 1;
+  if (r && s1 >= min_shift) {
+    int s2 = min_shift;
+    while ((1 << s1) + (1 << s2) < r) ++s2;
+    const int two = tiles_of_columns(N, s1) + tiles_of_columns(N, s2);
+    if (two < tail) tail = two, t.tail_shift = s1 + 256 * s2;
+  }
+  t.per_batch = N * t.full_per_row + tail;
   return t;
 }
 
@@ -33,7 +45,7 @@ struct TilePlace {
   int b, i0, j0, shift;
 };
 // RAGGED = false: whole-row pieces only (full_per_row pieces per row, per_batch = rows * full_per_row).
-// keep_rows_inside: the last piece of the ragged columns is moved up so that it ends at row N - 1 (its rows
+// keep_rows_inside: the last piece of some ragged columns is moved up so that it ends at row N - 1 (its rows
 // all exist, some of them belong to the piece before it as well; needs N >= 128 >> tail_shift); otherwise it
 // runs past the last row and the caller leaves those positions out.
 template <bool RAGGED>
@@ -48,11 +60,18 @@ OF3_HD inline TilePlace tile_place(int tile_id, int N, int full_per_row, int tai
     t.j0 = (rem - t.i0 * full_per_row) * 128;
     t.shift = 7;
   } else {
-    const int rows = 128 >> tail_shift;
-    t.i0 = (rem - main_tiles) * rows;
-    if (keep_rows_inside && t.i0 + rows > N) t.i0 = N - rows;
+    int at = rem - main_tiles;
+    t.shift = tail_shift & 255;
     t.j0 = full_per_row * 128;
-    t.shift = tail_shift;
+    const int first = tiles_of_columns(N, t.shift);
+    if (at >= first) {
+      at -= first;
+      t.j0 += 1 << t.shift;
+      t.shift = tail_shift >> 8;
+    }
+    const int rows = 128 >> t.shift;
+    t.i0 = at * rows;
+    if (keep_rows_inside && t.i0 + rows > N) t.i0 = N - rows;
   }
   return t;
 }
@@ -94,6 +113,40 @@ OF3_HD inline long long flat_offset(const FlatTile& t, int d, int N, long long s
     while (i >= N) i -= N, ++b;
     return b * stride_b + i * stride_r + j * stride_k;
   }
+}
+
+// ---- the last round of a persistent pass ----------------------------------------------------------------
+// `tiles` tiles of 128 positions on `grid` work-groups: the tiles that are left for a last round of their own, if
+// there are no more than half (a quarter) as many as work-groups, go in two (four) pieces of 64 (32) positions each, one
+// piece per work-group: that round then takes as long as its piece, not as a tile.  Items 0 .. whole - 1 are
+// whole tiles, the rest pieces; whole is a multiple of grid where there are pieces.  256 CUs, 128 channels, us per pass, whole
+// tiles / pieces: triangle multiplication in at N = 128 (half a round) 11.2 / 9.0, at 200 (1.37 rounds) 15.8 / 14.5, attention in
+// 12.9 / 11.8 and 17.8 / 16.4, attention out at 200 14.0 / 12.0.  From three rounds on the kernels with pieces, which hold
+// more registers and address their loads at run time, lose what the last round gains: N = 384 (4.5 rounds) the same, 929 167.7 / 171.4.
+struct LastRound {
+  int whole, items, piece;
+};
+inline LastRound last_round(long tiles, int grid) {
+  const int left = (int)(tiles % grid);
+  LastRound r = {(int)tiles, (int)tiles, 128};
+  if (left == 0 || 2 * left > grid || tiles >= 3L * grid) return r;
+  const int split = 4 * left <= grid ? 4 : 2;
+  r.piece = 128 / split;
+  r.whole = (int)(tiles - left);
+  r.items = r.whole + split * left;
+  return r;
+}
+
+// Item of a persistent pass -> its tile, its first position in it, how many positions it has (group_bits: log2 of the
+// groups of eight).  PART: positions per piece, 128: no pieces.
+struct TilePiece {
+  int tile, first, count, group_bits;
+};
+template <int PART>
+OF3_HD inline TilePiece tile_piece(int item, int whole) {
+  if (PART == 128 || item < whole) return {item, 0, 128, 4};
+  const int split = 128 / PART, left = item - whole;
+  return {whole + left / split, left % split * PART, PART, PART == 64 ? 3 : 2};
 }
 
 // ---- order of the attention core's work-groups -----------------------------------------------------------

@@ -15,12 +15,15 @@
 #include "of3_launch.h"
 #include "of3_pass_bf16.h"
 
+#include <type_traits>
+
 namespace of3 {
 
 namespace {
 
-template <int C, int HD, int MODE>
-__global__ __launch_bounds__(512) void triattn_out_kernel(TriattnOutArgs p, uint32_t total_pos, int total_tiles) {
+// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only
+template <int C, int HD, int MODE, int PART>
+__global__ __launch_bounds__(512, C == 64 ? 4 : 2) void triattn_out_kernel(TriattnOutArgs p, uint32_t total_pos, int whole_tiles, int total_items) {
   static_assert(C == HD, "o tile shares the x tile geometry");
   constexpr int NCH = C / 8;
   constexpr int LPP = NCH;
@@ -31,7 +34,7 @@ __global__ __launch_bounds__(512) void triattn_out_kernel(TriattnOutArgs p, uint
   constexpr int KS = C / 16;
   constexpr int NOT = C / 32;
   constexpr int WPG = NW / NOT;
-  constexpr int TPW = 4 / WPG;
+  constexpr int LN_STEP = NW * PPI;      // positions that the waves normalise at a time, PPI consecutive ones each
 
   __shared__ u32x4_t xtile[TP * NCH];  // LayerNorm(x), bf16
   __shared__ u32x4_t otile[TP * NCH];  // o, then o * gate
@@ -51,7 +54,6 @@ __global__ __launch_bounds__(512) void triattn_out_kernel(TriattnOutArgs p, uint
   for (int e = 0; e < 8; ++e) lw[e] *= -kLog2e, lb[e] *= -kLog2e;
 
   const int ot = wave % NOT;
-  const int t0 = (wave / NOT) * TPW;
   u32x4_t wg[KS], wo[KS];
   {
     pass_bf16::load_unit<C>(p.w_g, ot, rowperm16(l32), lh, p.packed, wg);
@@ -70,15 +72,21 @@ __global__ __launch_bounds__(512) void triattn_out_kernel(TriattnOutArgs p, uint
 
   // The loads of a tile are issued one tile ahead (right after the previous tile's values have
   // been consumed by the LayerNorm phase) and travel under that tile's two MFMA phases.
+  // LayerNorm-phase position `it` of this lane, from the item's first one: TP / NW consecutive positions per wave in whole
+  // tiles, in pieces LN_STEP by all waves at a time, so that a piece is the first iterations
+  auto ln_position = [&](bool in_piece, int it) {
+    return in_piece ? it * LN_STEP + wave * PPI + ln_pp : wave * (TP / NW) + it * PPI + ln_pp;
+  };
   u32x4_t xraw[LN_ITERS], oraw[LN_ITERS];
-  auto load_tile = [&](int tile_id) {
-    const Origin t = tile_origin(tile_id);
-    const uint32_t p0 = (uint32_t)tile_id * TP;
+  auto load_tile = [&](int item) {
+    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
+    const Origin t = tile_origin(piece.tile);
+    const uint32_t p0 = (uint32_t)piece.tile * TP;
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      const int d = wave * (TP / NW) + it * PPI + ln_pp;
+      const int d = piece.first + ln_position(piece.count < TP, it);
       u32x4_t vx = {0u, 0u, 0u, 0u}, vo = {0u, 0u, 0u, 0u};
-      if (p0 + d < total_pos) {
+      if ((PART == TP || it * LN_STEP < piece.count) && p0 + d < total_pos) {
         vx = *reinterpret_cast<const u32x4_t*>(p.x + view_offset(t, d) + 8 * ln_chunk);
         vo = *reinterpret_cast<const u32x4_t*>(p.o + (size_t)(p0 + d) * HD + 8 * ln_chunk);  // o is [B][N][N][HD]
       }
@@ -86,28 +94,35 @@ __global__ __launch_bounds__(512) void triattn_out_kernel(TriattnOutArgs p, uint
       oraw[it] = vo;
     }
   };
-  if ((int)blockIdx.x < total_tiles) load_tile(blockIdx.x);
+  if ((int)blockIdx.x < total_items) load_tile(blockIdx.x);
 
-  for (int tile_id = blockIdx.x; tile_id < total_tiles; tile_id += gridDim.x) {
-    const Origin t = tile_origin(tile_id);
-    const uint32_t p0 = (uint32_t)tile_id * TP;
+  auto do_tile = [&](auto positions, int item) {
+    constexpr int P = decltype(positions)::value;
+    constexpr int T = P / 32 >= WPG ? P / 32 / WPG : 1;  // position tiles per wave
+    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
+    const int first = P == TP ? 0 : piece.first;
+    const bool multiplies = P == TP || wave / NOT * T < P / 32;
+    const Origin t = tile_origin(piece.tile);
+    const uint32_t p0 = (uint32_t)piece.tile * TP;
 
     // ---- LayerNorm of this tile's values, then the next tile's loads
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      const int pos = wave * (TP / NW) + it * PPI + ln_pp;
+      const int pos = first + ln_position(P < TP, it);
+      if (P < TP && pos >= first + P) break;
       const int slot = tile_slot<NCH, 0>(pos, ln_chunk);
       xtile[slot] = layer_norm_chunk<C>(xraw[it], lw, lb);
       rtile[slot] = xraw[it];
       otile[slot] = oraw[it];
     }
     __syncthreads();
-    if (tile_id + (int)gridDim.x < total_tiles) load_tile(tile_id + gridDim.x);
+    if (P == TP && item + (int)gridDim.x < total_items) load_tile(item + gridDim.x);
 
     // ---- gate: lane owns gate channels 32*ot + 16*lh + v of position 32*t + l32
 #pragma unroll
-    for (int tt = 0; tt < TPW; ++tt) {
-      const int pos = 32 * (t0 + tt) + l32;
+    for (int tt = 0; tt < T; ++tt) {
+      if (!multiplies) break;
+      const int pos = first + 32 * (wave / NOT * T + tt) + l32;
       f32x16_t acc = zero16();
 #pragma unroll
       for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(wg[s], xtile[tile_slot<NCH, 0>(pos, 2 * s + lh)], acc);
@@ -124,9 +139,10 @@ __global__ __launch_bounds__(512) void triattn_out_kernel(TriattnOutArgs p, uint
     __syncthreads();
 
     // ---- output projection (+ residual)
+    if (!multiplies) return;  // nothing comes after a piece
 #pragma unroll
-    for (int tt = 0; tt < TPW; ++tt) {
-      const int pos = 32 * (t0 + tt) + l32;
+    for (int tt = 0; tt < T; ++tt) {
+      const int pos = first + 32 * (wave / NOT * T + tt) + l32;
       f32x16_t acc = zero16();
 #pragma unroll
       for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(wo[s], otile[tile_slot<NCH, 0>(pos, 2 * s + lh)], acc);
@@ -157,22 +173,30 @@ __global__ __launch_bounds__(512) void triattn_out_kernel(TriattnOutArgs p, uint
         *reinterpret_cast<u32x4_t*>(outrow + off + 8) = o1;
       }
     }
-    __syncthreads();
+    if (P == TP) __syncthreads();
+  };
+  typedef std::integral_constant<int, TP> Whole;
+  int item = blockIdx.x;
+  for (; item < whole_tiles; item += gridDim.x) do_tile(Whole{}, item);
+  if constexpr (PART < TP) {
+    if (item < total_items) do_tile(std::integral_constant<int, PART>{}, item);  // one piece: the last round
   }
 }
 
 template <int C, int HD, int MODE>
 hipError_t launch(const TriattnOutArgs& a, hipStream_t stream) {
-  auto kern = triattn_out_kernel<C, HD, MODE>;
   static int cache[kMaxDevices];
   int grid_cap = 0;
-  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(kern, 512, dev, v); }, &grid_cap);
+  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(triattn_out_kernel<C, HD, MODE, 128>, 512, dev, v); }, &grid_cap);
   if (e != hipSuccess) return e;
   const long positions = (long)a.B * a.N * a.N;
   if (positions <= 0 || positions > 0x7fffffffL) return hipErrorInvalidValue;
-  const long total = (positions + 127) / 128;
-  const int grid = (int)(total < grid_cap ? total : grid_cap);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), 0, stream, a, (uint32_t)positions, (int)total);
+  const LastRound r = last_round((positions + 127) / 128, grid_cap);
+  const int grid = r.items < grid_cap ? r.items : grid_cap;
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(512), 0, stream, a, (uint32_t)positions, r.whole, r.items); };
+  if (r.piece == 32) go(triattn_out_kernel<C, HD, MODE, 32>);
+  else if (r.piece == 64) go(triattn_out_kernel<C, HD, MODE, 64>);
+  else go(triattn_out_kernel<C, HD, MODE, 128>);
   return hipGetLastError();
 }
 

@@ -24,6 +24,8 @@
 #include "of3_launch.h"
 #include "of3_pass_bf16.h"
 
+#include <type_traits>
+
 // Waves per work-group of the C = 128 kernel: 8 (two per SIMD, 248 registers) or 16 (four per SIMD,
 // 118 registers, one matrix per wave).  Measured at N = 768 inside the block: 126 us against 128 us,
 // stand-alone 150 against 158: more waves in flight do not help this pass, the shipped form is 8.
@@ -45,9 +47,10 @@ __device__ __forceinline__ int proj_slot(int pos, int chunk) {
   return pos * NCH + (chunk ^ key);
 }
 
-template <int C, int D, int NW, bool RAGGED>
+// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only
+template <int C, int D, int NW, bool RAGGED, int PART>
 __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p, int full_per_row, int tail_shift,
-                                                               int tiles_per_batch, int total_tiles) {
+                                                               int tiles_per_batch, int whole_tiles, int total_items) {
   constexpr int H = 4;
   constexpr int HD = H * D;
   constexpr int NCH = C / 8;
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
   // else (H*D = 64): waves 0..5 own one (matrix, tile) job, waves 6 and 7 do the bias of two
   //   position tiles each.
   static_assert(!W16 || WIDE, "the sixteen-wave form is built for H*D = 128");
-  constexpr int TPW = 4;               // every wave visits all four position tiles
+  constexpr int LN_STEP = NW * PPI;    // positions that the waves normalise at a time, PPI consecutive ones each
   static_assert(NT == 4 || NT == 2, "H*D must be 128 or 64");
 
   __shared__ u32x4_t tile[2][TP * NCH];
@@ -78,9 +81,9 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
   const int lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int ln_chunk = lane % LPP, ln_pp = lane / LPP;
 
-  float lw[8], lb[8];
-  load_affine8(p.ln_w, ln_chunk, lw);
-  load_affine8(p.ln_b, ln_chunk, lb);
+  // affine parameters of this lane's 8 channels, kept packed (8 registers instead of 16) and unpacked once per tile
+  const u32x4_t lw_pk = *reinterpret_cast<const u32x4_t*>(p.ln_w + 8 * ln_chunk);
+  const u32x4_t lb_pk = *reinterpret_cast<const u32x4_t*>(p.ln_b + 8 * ln_chunk);
 
   if (wave == 0) {
 #pragma unroll
@@ -102,19 +105,25 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
 
   u32x4_t raw[LN_ITERS];
   float mraw[LN_ITERS];  // mask of the same positions (used by the lane with ln_chunk == 0)
-  auto load_tile = [&](int tile_id) {
+  // LayerNorm-phase position `it` of this lane, from the item's first one: TP / NW consecutive positions per wave in whole
+  // tiles, in pieces LN_STEP by all waves at a time, so that a piece is the first iterations
+  auto ln_position = [&](bool in_piece, int it) {
+    return in_piece ? it * LN_STEP + wave * PPI + ln_pp : wave * (TP / NW) + it * PPI + ln_pp;
+  };
+  auto load_tile = [&](int item) {
+    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
     int b, i0, j0, shift_rt;
-    tile_origin(tile_id, b, i0, j0, shift_rt);
+    tile_origin(piece.tile, b, i0, j0, shift_rt);
     const int shift = RAGGED ? shift_rt : 7, jmask = (1 << shift) - 1;
     const bf16_t* xrow = p.x + b * p.x_view.stride_b + i0 * p.x_view.stride_r;  // the tile's first row
     const float* mrow = p.mask ? p.mask + b * p.mask_view.stride_b + i0 * p.mask_view.stride_r : nullptr;
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      const int pos = wave * (TP / NW) + it * PPI + ln_pp;
+      const int in_item = ln_position(piece.count < TP, it), pos = piece.first + in_item;
       const int di = RAGGED ? pos >> shift : 0, j = j0 + (RAGGED ? pos & jmask : pos);  // every row i0 + di exists
       u32x4_t v = {0u, 0u, 0u, 0u};
       float m = 1.f;
-      if (j < N) {
+      if ((PART == TP || in_item < piece.count) && j < N) {
         v = *reinterpret_cast<const u32x4_t*>(xrow + di * p.x_view.stride_r + j * p.x_view.stride_k + 8 * ln_chunk);
         if (mrow && ln_chunk == 0) m = mrow[di * p.mask_view.stride_r + j * p.mask_view.stride_k];
       }
@@ -152,18 +161,29 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
       pass_bf16::load_unit<C>(W, ot, (ROLE == 1) ? l32 : rowperm16(l32), lh, p.packed, wj[jj]);
     }
 
-    auto do_tile = [&](int tile_id, int buf) {
+    auto do_tile = [&](auto positions, int item, int buf) {
+      constexpr int P = decltype(positions)::value;
+      const TilePiece piece = tile_piece<PART>(item, whole_tiles);
+      const int first = P == TP ? 0 : piece.first, tt0 = first / 32;
       int b, i0, j0, shift_rt;
-      tile_origin(tile_id, b, i0, j0, shift_rt);
+      tile_origin(piece.tile, b, i0, j0, shift_rt);
       const int shift = RAGGED ? shift_rt : 7, jmask = (1 << shift) - 1;
       // row and first column of the 32-position tile tt (wave-uniform): one row, one 32-key panel
       auto tile_row = [&](int tt) { return RAGGED ? i0 + ((32 * tt) >> shift) : i0; };
       auto tile_col = [&](int tt) { return RAGGED ? j0 + ((32 * tt) & jmask) : j0 + 32 * tt; };
 
       // ---- LayerNorm phase (+ mask bias, one lane per position)
+      float lw[8], lb[8];
+      {
+        u32x4_t tw = lw_pk, tb = lb_pk;
+        if (WIDE && (RAGGED || PART < TP)) __asm__ volatile("" : "+v"(tw), "+v"(tb));  // keeps the unpacked copies from being hoisted out of the loop
+        unpack8(tw, lw);
+        unpack8(tb, lb);
+      }
 #pragma unroll
       for (int it = 0; it < LN_ITERS; ++it) {
-        const int pos = wave * (TP / NW) + it * PPI + ln_pp;
+        const int pos = first + ln_position(P < TP, it);
+        if (P < TP && pos >= first + P) break;
         tile[buf][proj_slot<NCH>(pos, ln_chunk)] = layer_norm_chunk<C>(raw[it], lw, lb);
         if (ln_chunk == 0) {
           const int i = RAGGED ? i0 + (pos >> shift) : i0, j = j0 + (RAGGED ? pos & jmask : pos);
@@ -172,7 +192,7 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
           p.mbias[((size_t)b * N + i) * Jp + j] = mb;
         }
       }
-      if (tile_id + (int)gridDim.x < total_tiles) load_tile(tile_id + gridDim.x);
+      if (P == TP && item + (int)gridDim.x < total_items) load_tile(item + gridDim.x);
       __syncthreads();  // the only barrier per tile (the LDS tile is double buffered)
 
       // ---- projection phase
@@ -188,17 +208,20 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
           for (int h = 0; h < H; ++h) p.tbias[(((size_t)b * H + h) * N + i) * Jp + j] = (j < N) ? acc[h] * kLog2e : 0.f;
         }
       };
+      auto holds = [&](int tt) { return P == TP || (tt >= tt0 && tt < tt0 + P / 32); };
       if (ROLE == 2) {
         if (W16) {
-          bias_tile(wave - 12);
+          if (holds(wave - 12)) bias_tile(wave - 12);
         } else {
-          bias_tile(2 * (wave - 6));
-          bias_tile(2 * (wave - 6) + 1);
+          if (holds(2 * (wave - 6))) bias_tile(2 * (wave - 6));
+          if (holds(2 * (wave - 6) + 1)) bias_tile(2 * (wave - 6) + 1);
         }
         return;
       }
 #pragma unroll
-      for (int tt = 0; tt < TPW; ++tt) {
+      for (int u = 0; u < P / 32; ++u) {  // every wave visits all position tiles
+        const int tt = tt0 + u;
+        if (!RAGGED && WIDE && PART < TP) __builtin_amdgcn_sched_barrier(0);  // operands of the next position tile held early cost spills
         const size_t bi = (size_t)b * N + tile_row(tt);
         const int jt = tile_col(tt);
 #pragma unroll
@@ -244,18 +267,23 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
           *reinterpret_cast<u32x4_t*>(dst + 8) = o1;
         }
       }
-      if (ROLE == 1 && WIDE && !W16) bias_tile(wave - 4);
+      if (ROLE == 1 && WIDE && !W16 && holds(wave - 4)) bias_tile(wave - 4);
     };
 
-    int tile_id = blockIdx.x;
+    typedef std::integral_constant<int, TP> Whole;
+    int item = blockIdx.x;
     int buf = 0;
-    if (tile_id < total_tiles) {
-      load_tile(tile_id);
-      do_tile(tile_id, buf);
-      tile_id += gridDim.x;
+    if (item >= total_items) return;
+    load_tile(item);
+    if (PART == TP || item < whole_tiles) {
+      do_tile(Whole{}, item, buf);
+      item += gridDim.x;
       buf ^= 1;
     }
-    for (; tile_id < total_tiles; tile_id += gridDim.x, buf ^= 1) do_tile(tile_id, buf);
+    for (; item < whole_tiles; item += gridDim.x, buf ^= 1) do_tile(Whole{}, item, buf);
+    if constexpr (PART < TP) {
+      if (item < total_items) do_tile(std::integral_constant<int, PART>{}, item, buf);  // one piece: the last round
+    }
   };
 
   if (W16) {
@@ -274,17 +302,25 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
 
 template <int C, int D, int NW, bool RAGGED>
 hipError_t launch(const TriattnProjArgs& a, hipStream_t stream) {
-  auto kern = triattn_proj_kernel<C, D, NW, RAGGED>;
   static int cache[kMaxDevices];
   int grid_cap = 0;
-  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(kern, 64 * NW, dev, v); }, &grid_cap);
+  // one work-group per CU at 64 channels too, where some instances would let two share it (4 x 512^2: 121 us against 112)
+  hipError_t e = per_device(
+      cache, [&](int dev, int* v) { return C == 64 ? cu_count(dev, v) : resident_blocks(triattn_proj_kernel<C, D, NW, RAGGED, 128>, 64 * NW, dev, v); },
+      &grid_cap);
   if (e != hipSuccess) return e;
   RaggedTiles t = {a.Jp / 128, 7, a.N * (a.Jp / 128)};  // whole (padded) rows in 128-wide pieces
   if (RAGGED) t = ragged_tiles(a.N, 5);                 // pieces of whole 32-key panels
   const long total = (long)a.B * t.per_batch;
   if (total > 0x7fffffffL) return hipErrorInvalidValue;
-  const int grid = (int)(total < grid_cap ? total : grid_cap);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), 0, stream, a, t.full_per_row, t.tail_shift, t.per_batch, (int)total);
+  const LastRound r = last_round(total, grid_cap);
+  const int grid = r.items < grid_cap ? r.items : grid_cap;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), 0, stream, a, t.full_per_row, t.tail_shift, t.per_batch, r.whole, r.items);
+  };
+  if (r.piece == 32) go(triattn_proj_kernel<C, D, NW, RAGGED, 32>);
+  else if (r.piece == 64) go(triattn_proj_kernel<C, D, NW, RAGGED, 64>);
+  else go(triattn_proj_kernel<C, D, NW, RAGGED, 128>);
   return hipGetLastError();
 }
 

@@ -17,13 +17,16 @@
 #include "of3_launch.h"
 #include "of3_pass_bf16.h"
 
+#include <type_traits>
+
 namespace of3 {
 
 namespace {
 
-template <int C, int CH, bool RAGGED>
+// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only
+template <int C, int CH, bool RAGGED, int PART>
 __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int full_per_row, int tail_shift, int tiles_per_batch,
-                                                           int total_tiles) {
+                                                           int whole_tiles, int total_items) {
   static_assert(C == CH, "position-major x tile shares the z tile geometry");
   constexpr int NCH = C / 8;
   constexpr int LPP = NCH;
@@ -34,7 +37,7 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
   constexpr int KS = C / 16;
   constexpr int NOT = C / 32;            // output-channel tiles
   constexpr int WPG = NW / NOT;          // waves sharing one output tile (2 or 4)
-  constexpr int TPW = 4 / WPG;           // position tiles per wave
+  constexpr int LN_STEP = NW * PPI;      // positions that the waves normalise at a time, PPI consecutive ones each
   constexpr int XROUNDS = (CH / 2) * 16 / 512;  // (channel pair, 8-position group) items per thread
 
   __shared__ u32x4_t ztile[TP * NCH];
@@ -59,7 +62,6 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
   // A operands: logical output channel of A-row r is 32*ot + rowperm16(r), so that a lane
   // ends up with the 16 consecutive channels 32*ot + 16*lh + v
   const int ot = wave % NOT;
-  const int t0 = (wave / NOT) * TPW;
   u32x4_t wz[KS], wgt[KS];
   {
     pass_bf16::load_unit<CH>(p.w_z, ot, rowperm16(l32), lh, p.packed, wz);
@@ -73,30 +75,38 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
     const TilePlace t = tile_place<RAGGED>(tile_id, N, full_per_row, tail_shift, tiles_per_batch, false);
     b = t.b, i0 = t.i0, j0 = t.j0, shift = t.shift;
   };
+  // LayerNorm-phase position `it` of this lane, from the item's first one: TP / NW consecutive positions per wave in whole
+  // tiles, in pieces LN_STEP by all waves at a time, so that a piece is the first iterations
+  auto ln_position = [&](bool in_piece, int it) {
+    return in_piece ? it * LN_STEP + wave * PPI + ln_pp : wave * (TP / NW) + it * PPI + ln_pp;
+  };
   uint32_t* xt32 = reinterpret_cast<uint32_t*>(xtile);
 
   // The loads of a tile (z row-wise for the gate, x channel-major) are issued one tile ahead,
   // right after the previous tile's values have gone into LDS, and travel under its MFMA phase.
   u32x4_t zraw[LN_ITERS];
   u32x4_t xa[XROUNDS], xb[XROUNDS];
-  auto load_tile = [&](int tile_id) {
+  auto load_tile = [&](int item) {
+    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
     int b, i0, j0, shift_rt;
-    tile_origin(tile_id, b, i0, j0, shift_rt);
+    tile_origin(piece.tile, b, i0, j0, shift_rt);
     const int shift = RAGGED ? shift_rt : 7;  // a constant without ragged pieces: di below folds to 0
     const int jmask = (1 << shift) - 1;
     const bf16_t* zrow = p.z + b * p.z_view.stride_b + i0 * p.z_view.stride_r;  // the tile's first row (scalar)
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      const int pos = wave * (TP / NW) + it * PPI + ln_pp;
+      const int pos = piece.first + ln_position(piece.count < TP, it);
       const int di = RAGGED ? pos >> shift : 0, j = j0 + (RAGGED ? pos & jmask : pos);  // di = 0 in the whole-row pieces
       u32x4_t v = {0u, 0u, 0u, 0u};
-      if ((!RAGGED || i0 + di < N) && j < N) v = *reinterpret_cast<const u32x4_t*>(zrow + di * p.z_view.stride_r + j * p.z_view.stride_k + 8 * ln_chunk);
+      if ((PART == TP || it * LN_STEP < piece.count) && (!RAGGED || i0 + di < N) && j < N) v = *reinterpret_cast<const u32x4_t*>(zrow + di * p.z_view.stride_r + j * p.z_view.stride_k + 8 * ln_chunk);
       zraw[it] = v;
     }
 #pragma unroll
     for (int rr = 0; rr < XROUNDS; ++rr) {
       const int item = rr * 512 + tid;
-      const int cp = item >> 4, pg = item & 15;  // channels 2cp, 2cp+1; positions 8pg..8pg+7: one row, as the width is >= 8
+      // channels 2cp, 2cp+1; positions 8pg..8pg+7: one row, as the width is >= 8
+      const int cp = item >> piece.group_bits, pg = (piece.first >> 3) + (item & ((1 << piece.group_bits) - 1));
+      if (PART < TP && cp >= CH / 2) break;
       int i = i0 + (RAGGED ? (8 * pg) >> shift : 0);
       const int j = j0 + (RAGGED ? (8 * pg) & jmask : 8 * pg);  // < Np: the planes are padded to whole 128-wide pieces
       if (RAGGED) i = i < Np ? i : Np - 1;    // rows of a last piece past the end of the plane: any row, never used
@@ -105,20 +115,26 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
       xb[rr] = *reinterpret_cast<const u32x4_t*>(src + (size_t)Np * Np);
     }
   };
-  if ((int)blockIdx.x < total_tiles) load_tile(blockIdx.x);
+  if ((int)blockIdx.x < total_items) load_tile(blockIdx.x);
 
-  for (int tile_id = blockIdx.x; tile_id < total_tiles; tile_id += gridDim.x) {
+  auto do_tile = [&](auto positions, int item) {
+    constexpr int P = decltype(positions)::value;
+    constexpr int GROUPS = P / 8, XR = (CH / 2) * GROUPS > 512 ? (CH / 2) * GROUPS / 512 : 1;
+    constexpr int T = P / 32 >= WPG ? P / 32 / WPG : 1;  // position tiles per wave
+    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
+    const int first = P == TP ? 0 : piece.first;
     int b, i0, j0, shift_rt;
-    tile_origin(tile_id, b, i0, j0, shift_rt);
+    tile_origin(piece.tile, b, i0, j0, shift_rt);
     const int shift = RAGGED ? shift_rt : 7;
     const int jmask = (1 << shift) - 1;
     bf16_t* orow0 = p.out + b * p.z_view.stride_b + i0 * p.z_view.stride_r;  // the tile's first row (scalar)
 
     // x: transpose into xtile[pos][c] with 4-byte (channel pair) writes
 #pragma unroll
-    for (int rr = 0; rr < XROUNDS; ++rr) {
+    for (int rr = 0; rr < XR; ++rr) {
       const int item = rr * 512 + tid;
-      const int cp = item >> 4, pg = item & 15;
+      const int cp = item / GROUPS, pg = (first >> 3) + item % GROUPS;
+      if ((CH / 2) * GROUPS < 512 && cp >= CH / 2) break;
       const int chunk = (2 * cp) >> 3, within = (2 * cp) & 7;  // `within` is even
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -131,27 +147,29 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
     // z: LayerNorm_in -> ztile
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      const int pos = wave * (TP / NW) + it * PPI + ln_pp;
+      const int pos = first + ln_position(P < TP, it);
+      if (P < TP && pos >= first + P) break;
       ztile[tile_slot<NCH, 0>(pos, ln_chunk)] = layer_norm_chunk<C>(zraw[it], iw, ib);
       rtile[tile_slot<NCH, 0>(pos, ln_chunk)] = zraw[it];
     }
     __syncthreads();
-    if (tile_id + (int)gridDim.x < total_tiles) load_tile(tile_id + gridDim.x);
+    if (P == TP && item + (int)gridDim.x < total_items) load_tile(item + gridDim.x);
 
     // x: LayerNorm_out in place (lane owns one 16-byte chunk of one position)
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      const int pos = wave * (TP / NW) + it * PPI + ln_pp;
+      const int pos = first + ln_position(P < TP, it);
+      if (P < TP && pos >= first + P) break;
       const int slot = tile_slot<NCH, 0>(pos, ln_chunk);
       xtile[slot] = layer_norm_chunk<CH>(xtile[slot], ow, ob);
     }
     __syncthreads();
 
     // ---- matrix phase
+    if (P < TP && wave / NOT * T >= P / 32) return;  // nothing comes after a piece
 #pragma unroll
-    for (int tt = 0; tt < TPW; ++tt) {
-      const int t = t0 + tt;
-      const int pos = 32 * t + l32;
+    for (int tt = 0; tt < T; ++tt) {
+      const int pos = first + 32 * (wave / NOT * T + tt) + l32;
       f32x16_t accu = zero16(), accg = zero16();
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
@@ -188,22 +206,33 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
         *reinterpret_cast<u32x4_t*>(orow + off + 8) = o1;
       }
     }
-    __syncthreads();  // both tiles are rewritten by the next iteration
+    if (P == TP) __syncthreads();  // both tiles are rewritten by the next iteration
+  };
+  typedef std::integral_constant<int, TP> Whole;
+  int item = blockIdx.x;
+  for (; item < whole_tiles; item += gridDim.x) do_tile(Whole{}, item);
+  if constexpr (PART < TP) {
+    if (item < total_items) do_tile(std::integral_constant<int, PART>{}, item);  // one piece: the last round
   }
 }
 
 template <int C, int CH, bool RAGGED>
 hipError_t launch(const TrimulOutArgs& a, hipStream_t stream) {
-  auto kern = trimul_out_kernel<C, CH, RAGGED>;
   static int cache[kMaxDevices];
   int grid_cap = 0;
-  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(kern, 512, dev, v); }, &grid_cap);
+  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(trimul_out_kernel<C, CH, RAGGED, 128>, 512, dev, v); }, &grid_cap);
   if (e != hipSuccess) return e;
   const RaggedTiles t = ragged_tiles(a.N);
   const long total = (long)a.B * t.per_batch;
   if (total > 0x7fffffffL) return hipErrorInvalidValue;
-  const int grid = (int)(total < grid_cap ? total : grid_cap);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), 0, stream, a, t.full_per_row, t.tail_shift, t.per_batch, (int)total);
+  const LastRound r = last_round(total, grid_cap);
+  const int grid = r.items < grid_cap ? r.items : grid_cap;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), 0, stream, a, t.full_per_row, t.tail_shift, t.per_batch, r.whole, r.items);
+  };
+  if (r.piece == 32) go(trimul_out_kernel<C, CH, RAGGED, 32>);
+  else if (r.piece == 64) go(trimul_out_kernel<C, CH, RAGGED, 64>);
+  else go(trimul_out_kernel<C, CH, RAGGED, 128>);
   return hipGetLastError();
 }
 

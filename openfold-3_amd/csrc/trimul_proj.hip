@@ -23,12 +23,15 @@
 #include "of3_launch.h"
 #include "of3_pass_bf16.h"
 
+#include <type_traits>
+
 namespace of3 {
 
 namespace {
 
-template <int C, int CH>
-__global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int panels, int total_tiles) {
+// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only
+template <int C, int CH, int PART>
+__global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int panels, int whole_tiles, int total_items) {
   constexpr int NCH = C / 8;        // 16-byte chunks per position
   constexpr int LPP = NCH;          // lanes sharing one position in the LayerNorm phase
   constexpr int PPI = 64 / LPP;     // positions per wave instruction
@@ -36,12 +39,12 @@ __global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int 
   constexpr int TR = TP / 32;
   constexpr int NW = 8;             // waves per work-group (two per SIMD)
   constexpr int LN_ITERS = (TP / NW) / PPI;
+  constexpr int LN_STEP = NW * PPI; // positions that the waves normalise at a time where they share a row
   constexpr int KS = C / 16;        // MFMA k-steps
   constexpr int OT = CH / 32;       // 32-row output tiles per matrix
   constexpr int NJOBS = 2 * OT;     // (a|b, output tile) jobs: 8 or 4
   constexpr int WPJ = NW / NJOBS;   // waves sharing a job: 1 or 2, each takes 4/WPJ position tiles
   constexpr int TPW = 4 / WPJ;      // position tiles per wave: 4 or 2
-  constexpr int KSH = (TPW == 4) ? 2 : 1;  // swizzle key from pos / TPW: distinct for the 8 lanes of a read group
   static_assert(NJOBS == 8 || NJOBS == 4, "CH must be 128 or 64");
 
   // two tiles: LayerNorm of tile n+1 is written while other waves still read tile n
@@ -79,11 +82,13 @@ __global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int 
   const int N = p.N, Np = p.Np;
   const int tiles_per_batch = ((N + TR - 1) / TR) * panels;
 
-  // LayerNorm-phase positions of this lane: wave w takes positions [16w, 16w+16) of the tile,
-  // i.e. 16 consecutive k of row w/2; iteration `it` adds PPI positions.  The lane-dependent
-  // part of the address is computed once, the tile adds a wave-uniform base.
-  const int ln_pos0 = wave * (TP / NW) + ln_pp;
-  const int ln_row = ln_pos0 >> 5, ln_k = ln_pos0 & 31;
+  // LayerNorm-phase position `it` of this lane: a wave takes PPI consecutive ones per instruction.  Whole tiles of 128
+  // channels: TP / NW consecutive positions per wave (N = 768: 112 against 115 us); pieces, and 64 channels (4 x 512^2: 91 against 101): LN_STEP
+  // positions by all waves at a time, so that a piece is the first iterations.
+  constexpr bool RUNS = C == 128;
+  auto ln_first = [&](bool piece, int it) {  // of the wave's PPI positions, which share a row
+    return RUNS && !piece ? wave * (TP / NW) + it * PPI : it * LN_STEP + wave * PPI;
+  };
   // Everything a tile reads from global memory (its z values and this lane's mask values) is
   // requested one tile ahead by a fixed number of unconditional loads (positions past the end
   // are clamped to the last one and zeroed through the mask value), and every tile issues the
@@ -95,49 +100,65 @@ __global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int 
   const float* const mask_base = p.mask ? p.mask : reinterpret_cast<const float*>(p.ln_w);  // dummy when absent
   const int64_t msb = p.mask ? p.mask_view.stride_b : 0, msr = p.mask ? p.mask_view.stride_r : 0,
                 msk = p.mask ? p.mask_view.stride_k : 0;
-  // Positions of the tile are dealt to MFMA columns so that a lane finishes TPW consecutive
-  // positions: position  32*TPW*tgroup + TPW*l32 + tt  is column l32 of this wave's tile tt.
-  const int pos0 = 32 * TPW * tgroup + TPW * l32;
-  auto load_tile = [&](int tile_id) {
-    const int b = tile_id / tiles_per_batch;
-    const int rem = tile_id - b * tiles_per_batch;
-    const int r0 = (rem / panels) * TR;
-    const int k0 = (rem % panels) * 32;
-    int row = r0 + ln_row;
-    row = row < N ? row : N - 1;
-    const bf16_t* base = p.z + b * p.z_view.stride_b + row * p.z_view.stride_r + 8 * ln_chunk;
+  // Positions of a tile, or of a piece of P positions, are dealt to MFMA columns so that a lane finishes
+  // T = min(P / (32 WPJ), 1) consecutive ones: position  32*T*tgroup + T*l32 + tt  is column l32 of this wave's tile tt.
+  struct Place {
+    int b, r0, k0;  // batch element, first row, first k
+  };
+  auto place = [&](int item) {
+    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
+    Place t;
+    t.b = piece.tile / tiles_per_batch;
+    const int rem = piece.tile - t.b * tiles_per_batch, rg = rem / panels;
+    t.r0 = rg * TR + piece.first / 32;
+    t.k0 = (rem - rg * panels) * 32;
+    return t;
+  };
+  auto load_tile = [&](int item) {
+    const Place t = place(item);
+    const bool piece = PART < TP && item >= whole_tiles;
+    // a piece issues the loads of a whole tile, the ones it has no use for from its last row again
+    const int rows = piece ? PART / 32 : TR, per_lane = piece ? (PART / 32 + WPJ - 1) / WPJ : TPW;
+    const int last = t.r0 + rows - 1 < N ? t.r0 + rows - 1 : N - 1;
+    const bf16_t* base = p.z + t.b * p.z_view.stride_b + 8 * ln_chunk;
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      int k = k0 + ln_k + it * PPI;
+      const int pos = ln_first(piece, it);
+      int row = t.r0 + (pos >> 5), k = t.k0 + (pos & 31) + ln_pp;
+      row = row < last ? row : last;
       k = k < N ? k : N - 1;
-      raw[it] = *reinterpret_cast<const u32x4_t*>(base + k * p.z_view.stride_k);
+      raw[it] = *reinterpret_cast<const u32x4_t*>(base + row * p.z_view.stride_r + k * p.z_view.stride_k);
     }
-    int mr = r0 + (pos0 >> 5);
-    mr = mr < N ? mr : N - 1;
-    const float* mrow = mask_base + b * msb + mr * msr;
+    const int pos0 = per_lane * (32 * tgroup + l32);
+    int mr = t.r0 + (pos0 >> 5);
+    mr = mr < last ? mr : last;
+    const float* mrow = mask_base + t.b * msb + mr * msr;
 #pragma unroll
     for (int tt = 0; tt < TPW; ++tt) {
-      int k = k0 + (pos0 & 31) + tt;
-      k = k < N ? k : N - 1;
-      mraw[tt] = mrow[k * msk];
+      int km = t.k0 + (pos0 & 31) + tt;
+      km = km < N ? km : N - 1;
+      mraw[tt] = mrow[km * msk];
     }
   };
 
-  auto do_tile = [&](int tile_id, int buf) {
-    const int b = tile_id / tiles_per_batch;
-    const int rem = tile_id - b * tiles_per_batch;
-    const int r = (rem / panels) * TR + (pos0 >> 5);  // this lane's row and first k
-    const int kfirst = (rem % panels) * 32 + (pos0 & 31);
+  auto do_tile = [&](auto positions, int item, int buf) {
+    constexpr int P = decltype(positions)::value;
+    constexpr int T = P / 32 >= WPJ ? P / 32 / WPJ : 1;  // positions per lane
+    constexpr int KSH = T == 4 ? 2 : T == 2 ? 1 : 0;     // swizzle key from pos / T: distinct for the 8 lanes of a read group
+    const Place t = place(item);
+    const int pos0 = 32 * T * tgroup + T * l32;
+    const int b = t.b, r = t.r0 + (pos0 >> 5);  // this lane's row and first k
+    const int kfirst = t.k0 + (pos0 & 31);
 
-    float mval[TPW];
+    float mval[T];
 #pragma unroll
-    for (int tt = 0; tt < TPW; ++tt) mval[tt] = (kfirst + tt < N && r < N) ? (p.mask ? mraw[tt] : 1.f) : 0.f;
+    for (int tt = 0; tt < T; ++tt) mval[tt] = (kfirst + tt < N && r < N) ? (p.mask ? mraw[tt] : 1.f) : 0.f;
     bool not_one = false;
 #pragma unroll
-    for (int tt = 0; tt < TPW; ++tt) not_one |= mval[tt] != 1.f;
+    for (int tt = 0; tt < T; ++tt) not_one |= mval[tt] != 1.f;
     const bool masked = __builtin_amdgcn_ballot_w64(not_one) != 0;  // wave-uniform
 
-    // ---- LayerNorm phase: wave w normalises positions [16w, 16w+16) of the tile
+    // ---- LayerNorm phase
     float lw[8], lb[8];
     {
       u32x4_t tw = lw_pk, tb = lb_pk;
@@ -147,20 +168,22 @@ __global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int 
     }
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      const int pos = wave * (TP / NW) + it * PPI + ln_pp;
+      const int pos = ln_first(P < TP, it) + ln_pp;
+      if (P < TP && pos >= P) break;
       tile[buf][tile_slot<NCH, KSH>(pos, ln_chunk)] = layer_norm_chunk<C>(raw[it], lw, lb);
     }
     // next tile's z travels while this tile's matrix phase runs
-    if (tile_id + (int)gridDim.x < total_tiles) load_tile(tile_id + gridDim.x);
+    if (P == TP && item + (int)gridDim.x < total_items) load_tile(item + gridDim.x);
     // One barrier per tile: it publishes this tile, and since every wave has finished the
     // previous tile's matrix phase before arriving, the other buffer may be overwritten by
     // the next LayerNorm phase.
     __syncthreads();
+    if (32 * T * tgroup >= P) return;
 
     // ---- projection phase
-    float res[TPW][16];
+    float res[T][16];
 #pragma unroll
-    for (int tt = 0; tt < TPW; ++tt) {
+    for (int tt = 0; tt < T; ++tt) {
       f32x16_t accg = zero16(), accp = zero16();
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
@@ -190,40 +213,52 @@ __global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int 
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         bf16_t* dst = dst0 + (size_t)(8 * (v >> 2) + (v & 3)) * plane;
-        if (TPW == 4) {
+        if constexpr (T == 4) {
           u32x2_t w2 = {pack_bf16(res[0][v], res[1][v]), pack_bf16(res[2][v], res[3][v])};
           *reinterpret_cast<u32x2_t*>(dst) = w2;
-        } else {
+        } else if constexpr (T == 2) {
           *reinterpret_cast<uint32_t*>(dst) = pack_bf16(res[0][v], res[1][v]);
+        } else {
+          *dst = to_bf16(res[0][v]);
         }
       }
     }
   };
 
   // the first tile is peeled: the loop proper is only entered with a tile's stores in flight
-  int tile_id = blockIdx.x;
+  typedef std::integral_constant<int, TP> Whole;
+  int item = blockIdx.x;
   int buf = 0;
-  if (tile_id < total_tiles) {
-    load_tile(tile_id);
-    do_tile(tile_id, buf);
-    tile_id += gridDim.x;
+  if (item >= total_items) return;
+  load_tile(item);
+  if (PART == TP || item < whole_tiles) {
+    do_tile(Whole{}, item, buf);
+    item += gridDim.x;
     buf ^= 1;
   }
-  for (; tile_id < total_tiles; tile_id += gridDim.x, buf ^= 1) do_tile(tile_id, buf);
+  for (; item < whole_tiles; item += gridDim.x, buf ^= 1) do_tile(Whole{}, item, buf);
+  if constexpr (PART < TP) {
+    if (item < total_items) do_tile(std::integral_constant<int, PART>{}, item, buf);  // one piece: the last round
+  }
 }
 
+template <int C, int CH, int PART>
+hipError_t launch(const TrimulProjArgs& a, int panels, const LastRound& r, int grid, hipStream_t stream) {
+  hipLaunchKernelGGL((trimul_proj_kernel<C, CH, PART>), dim3(grid), dim3(512), 0, stream, a, panels, r.whole, r.items);
+  return hipGetLastError();
+}
 template <int C, int CH>
 hipError_t launch(const TrimulProjArgs& a, hipStream_t stream) {
-  auto kern = trimul_proj_kernel<C, CH>;
   static int cache[kMaxDevices];
   int grid_cap = 0;
-  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(kern, 512, dev, v); }, &grid_cap);
+  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(trimul_proj_kernel<C, CH, 128>, 512, dev, v); }, &grid_cap);
   if (e != hipSuccess) return e;
   const int panels = (a.N + 31) / 32;  // the panels that hold a k below N; the contraction reads no others
-  const long total = (long)a.B * ((a.N + 3) / 4) * panels;
-  const int grid = (int)(total < grid_cap ? total : grid_cap);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), 0, stream, a, panels, (int)total);
-  return hipGetLastError();
+  const LastRound r = last_round((long)a.B * ((a.N + 3) / 4) * panels, grid_cap);
+  const int grid = r.items < grid_cap ? r.items : grid_cap;
+  if (r.piece == 32) return launch<C, CH, 32>(a, panels, r, grid, stream);
+  if (r.piece == 64) return launch<C, CH, 64>(a, panels, r, grid, stream);
+  return launch<C, CH, 128>(a, panels, r, grid, stream);
 }
 
 }  // namespace
