@@ -34,7 +34,7 @@ hipError_t trimul_proj_launch(const TrimulProjArgs& args, int C, int CH, hipStre
 // nk: the k-panels that are summed over, ceil(N / 32) (the later ones hold zeros);
 // variant: 1 = 256x192 output tiles, 2 = 256x128, 3 = 256x256, 4 = 384x192 on eight waves
 hipError_t trimul_contract_launch(const bf16_t* a, const bf16_t* b, bf16_t* x, int planes, int Np, int nk, int variant,
-                                  hipStream_t stream);
+                                  bool transposed, hipStream_t stream);
 
 struct TrimulOutArgs {
   const bf16_t* x;  // [B][CH][Np][Np]
@@ -67,10 +67,6 @@ struct TriattnProjArgs {
   int packed = 0;                     // w_q, w_k, w_v in MFMA operand order
 };
 hipError_t triattn_proj_launch(const TriattnProjArgs& args, int C, int D, hipStream_t stream);
-// both in one, the attention on what the output pass writes, in the same orientation (pair_pass_bf16.hip): up to one
-// 32-position tile per CU, where either pass runs on such tiles by itself
-hipError_t trimul_out_triattn_proj_serves(int B, int N, bool* serves);
-hipError_t trimul_out_triattn_proj_launch(const TrimulOutArgs& out, const TriattnProjArgs& proj, int C, int D, hipStream_t stream);
 
 struct TriattnFlashArgs {
   const bf16_t *q, *k, *vt;
@@ -93,6 +89,16 @@ struct TriattnOutArgs {
   int packed = 0;
 };
 hipError_t triattn_out_launch(const TriattnOutArgs& args, int C, int HD, hipStream_t stream);
+
+// The output pass of a module and the input pass of the next in one launch (pair_join_bf16.hip): weights packed, CH = C or
+// H * D = C, four heads, x of a multiplication in the second module's frame.  join_rows: rows of a tile, 0 where the passes
+// run by themselves.
+constexpr int kJoinTokens = 256;
+hipError_t join_rows(int B, int N, int C, int* rows);
+hipError_t trimul_trimul_launch(const TrimulOutArgs& end, const TrimulProjArgs& start, int C, hipStream_t stream);
+hipError_t trimul_triattn_launch(const TrimulOutArgs& end, const TriattnProjArgs& start, int C, hipStream_t stream);
+hipError_t triattn_triattn_launch(const TriattnOutArgs& end, const TriattnProjArgs& start, int C, hipStream_t stream);
+hipError_t triattn_trimul_launch(const TriattnOutArgs& end, const TrimulProjArgs& start, int C, hipStream_t stream);
 
 // the same four passes on tiles of 32 positions (pair_pass_bf16.hip), called by the launchers above for short sequences
 hipError_t trimul_proj_panels_launch(const TrimulProjArgs& args, int C, hipStream_t stream);

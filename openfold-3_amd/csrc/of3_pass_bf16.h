@@ -3,6 +3,7 @@
 #pragma once
 
 #include "of3_device.h"
+#include "of3_kernels.h"
 
 namespace of3 {
 namespace pass_bf16 {
@@ -53,12 +54,12 @@ struct LnLane {
     __asm__ volatile("" : "+v"(lane));
     return lane;
   }
-  // SCALED: the result feeds a gate only, weight and bias carry the factor -log2(e) of its base-2 exponential
+  // Weight and bias unpacked where they are used (16 to 32 instructions) rather than held as 16 floats.  SCALED: the result
+  // feeds a gate only, both carry the factor -log2(e) of its base-2 exponential
   template <bool SCALED>
-  __device__ __forceinline__ u32x4_t normalised(u32x4_t raw) const {
+  __device__ __forceinline__ void unpacked(float (&lw)[8], float (&lb)[8]) const {
     u32x4_t tw = w, tb = b;
-    __asm__ volatile("" : "+v"(tw), "+v"(tb));  // unpacked here rather than held as 16 floats
-    float lw[8], lb[8];
+    __asm__ volatile("" : "+v"(tw), "+v"(tb));
     unpack8(tw, lw);
     unpack8(tb, lb);
     if (SCALED) {
@@ -68,6 +69,11 @@ struct LnLane {
         __asm__("" : "+v"(lb[e]));  // rounded here: the fused multiply-add is the one with the weight, as in the 128-position passes
       }
     }
+  }
+  template <bool SCALED>
+  __device__ __forceinline__ u32x4_t normalised(u32x4_t raw) const {
+    float lw[8], lb[8];
+    unpacked<SCALED>(lw, lb);
     return layer_norm_chunk<C>(raw, lw, lb);
   }
 };
@@ -115,6 +121,70 @@ __device__ __forceinline__ void add16(const bf16_t* src, float (&x)[16]) {
 #pragma unroll
   for (int v = 0; v < 8; ++v) x[8 + v] += r[v];
 }
+
+// ---- triangle attention, projections of one panel: kind 0, 1, 2 a 32-channel tile of q, k or v, 3 the triangle bias (4 rows, the
+// others of its tile zero)
+template <int C>
+__device__ __forceinline__ void load_attention_unit(const TriattnProjArgs& p, int kind, int ot, int lane, u32x4_t (&w)[C / 16]) {
+  constexpr int H = 4;
+  if (kind == 3) {
+#pragma unroll
+    for (int s = 0; s < C / 16; ++s) {
+      w[s] = u32x4_t{0u, 0u, 0u, 0u};
+      if ((lane & 31) < H) w[s] = *reinterpret_cast<const u32x4_t*>(p.w_b + (lane & 31) * C + 16 * s + 8 * (lane >> 5));
+    }
+  } else {
+    load_unit<C>(kind == 0 ? p.w_q : kind == 1 ? p.w_k : p.w_v, ot, kind == 2 ? lane & 31 : rowperm16(lane & 31), lane >> 5, p.packed, w);
+  }
+}
+// products and stores of the wave for the normalised positions j0 .. j0 + 31 of row bi
+template <int C, int D>
+__device__ __forceinline__ void project_panel(const TriattnProjArgs& p, const u32x4_t (&w)[C / 16], const PanelTile<C, true>& tile, int kind,
+                                              int ot, int bi, int j0) {
+  typedef PanelTile<C, true> Tile;
+  constexpr int H = 4, KS = C / 16;
+  const int N = p.N, Jp = p.Jp;
+  const float qscale = kLog2e * __builtin_amdgcn_rsqf((float)D);
+  const Lane at = lane_here();
+  const int l32 = at.l32, lh = at.lh;
+  f32x16_t acc = zero16();
+  float res[16];
+  bf16_t* dst;
+  if (kind == 3) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(w[s], tile.s[Tile::slot(l32, 2 * s + lh)], acc);
+    if (lh == 0) {  // rows 0..3 of the result: registers 0..3 of lanes 0..31
+      const int b = bi / N, i = bi - b * N, j = j0 + l32;
+#pragma unroll
+      for (int h = 0; h < H; ++h) p.tbias[(((size_t)b * H + h) * N + i) * Jp + j] = j < N ? acc[h] * kLog2e : 0.f;
+    }
+    return;
+  }
+  if (kind == 2) {
+    // V^T panel: rows = keys (dealt by rowperm16), columns = channels; lane: channel 32 ot + l32, keys 16 lh + v
+    const int kpos = rowperm16(l32);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(tile.s[Tile::slot(kpos, 2 * s + lh)], w[s], acc);
+    const int ch = 32 * ot + l32, head = ch / D, d = ch % D;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) res[v] = acc[v];
+    dst = p.vt + ((size_t)bi * H + head) * D * Jp + (size_t)(j0 >> 5) * (D * 32) + d * 32 + 16 * lh;
+  } else {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(w[s], tile.s[Tile::slot(l32, 2 * s + lh)], acc);
+    const int ch0 = 32 * ot + 16 * lh, head = ch0 / D, d0 = ch0 % D;
+    const float sc = kind == 0 ? qscale : 1.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) res[v] = acc[v] * sc;
+    dst = (kind == 0 ? p.q : p.k) + (((size_t)bi * H + head) * Jp + j0 + l32) * D + d0;
+  }
+  store16(dst, res);
+}
+// log2(e) times the mask bias of position j of row bi
+__device__ __forceinline__ void store_mask_bias(const TriattnProjArgs& p, int bi, int j, float mask) {
+  p.mbias[(size_t)bi * p.Jp + j] = j < p.N ? kLog2e * (p.inf * (mask - 1.f)) : -__builtin_inff();
+}
+
 
 // logical number of a work-group: consecutive numbers run on one XCD where the grid deals evenly
 __device__ __forceinline__ int grid_slot() {

@@ -191,10 +191,17 @@ int64_t of3_trimul_workspace_bytes_for(int dtype, int64_t B, int64_t N, int64_t 
   return f32_trimul_ab_bytes(B, N, CH) + align256(B * CH * N * N * 4) + align256((int64_t)of3::trimul_wsplit_bytes(C, CH));
 }
 
+// a module's output pass that waits for the next module's input pass (pair_join_bf16.hip)
+struct ModuleEnd {
+  enum { kMul, kAtt } is;
+  of3::TrimulOutArgs mul;
+  of3::TriattnOutArgs att;
+};
+
 static int trimul_proj(int packed, const void* z, const int64_t z_strides[3], const float* mask,
                        const int64_t mask_strides[3], const void* ln_in_w, const void* ln_in_b, const void* w_a_p,
                        const void* w_a_g, const void* w_b_p, const void* w_b_g, void* a, void* b, int64_t B, int64_t N,
-                       int64_t C, int64_t CH, int outgoing, void* stream) {
+                       int64_t C, int64_t CH, int outgoing, void* stream, const ModuleEnd* before = nullptr) {
   if (!trimul_dims_ok(B, N, C, CH) || !strides_ok(z_strides) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
   const void* ptrs[] = {z, ln_in_w, ln_in_b, w_a_p, w_a_g, w_b_p, w_b_g, a, b};
   for (const void* p : ptrs)
@@ -216,7 +223,10 @@ static int trimul_proj(int packed, const void* z, const int64_t z_strides[3], co
   args.N = (int)N;
   args.Np = (int)padded(N);
   args.packed = packed;
-  hipError_t e = of3::trimul_proj_launch(args, (int)C, (int)CH, static_cast<hipStream_t>(stream));
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  hipError_t e = !before                             ? of3::trimul_proj_launch(args, (int)C, (int)CH, s)
+                 : before->is == ModuleEnd::kMul ? of3::trimul_trimul_launch(before->mul, args, (int)C, s)
+                                                 : of3::triattn_trimul_launch(before->att, args, (int)C, s);
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
@@ -228,21 +238,27 @@ int of3_trimul_proj(const void* z, const int64_t z_strides[3], const float* mask
                      C, CH, outgoing, stream);
 }
 
-int of3_trimul_contract(const void* a, const void* b, void* x, int64_t B, int64_t N, int64_t CH, int variant,
-                        void* stream) {
+// transposed: every plane of x as its transpose (variants 2 and 3)
+static int trimul_contract(const void* a, const void* b, void* x, int64_t B, int64_t N, int64_t CH, int variant, bool transposed,
+                           void* stream) {
   if (!positions_ok(B, N) || (CH != 128 && CH != 64) || variant < 0 || variant > 4) return OF3_EINVAL;
   if (!a || !b || !x || !aligned16(a) || !aligned16(b) || !aligned16(x)) return OF3_EINVAL;
   const int64_t Np = padded(N);
   if (variant == 0) variant = contract_variant_auto(B * CH, Np);
   hipError_t e = of3::trimul_contract_launch(bf(a), bf(b), bf(x), (int)(B * CH), (int)Np, (int)((N + 31) / 32), variant,
-                                             static_cast<hipStream_t>(stream));
+                                             transposed, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
+}
+
+int of3_trimul_contract(const void* a, const void* b, void* x, int64_t B, int64_t N, int64_t CH, int variant,
+                        void* stream) {
+  return trimul_contract(a, b, x, B, N, CH, variant, false, stream);
 }
 
 static int trimul_out(int packed, const void* x, const void* z, const int64_t z_strides[3], void* out,
                       const void* ln_in_w, const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
                       const void* w_g, const void* w_z, int64_t B, int64_t N, int64_t C, int64_t CH, int add_residual,
-                      void* stream, of3::TrimulOutArgs* deferred = nullptr) {
+                      void* stream, ModuleEnd* deferred = nullptr) {
   if (!trimul_dims_ok(B, N, C, CH) || !strides_ok(z_strides)) return OF3_EINVAL;
   const void* ptrs[] = {x, z, out, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_g, w_z};
   for (const void* p : ptrs)
@@ -264,7 +280,8 @@ static int trimul_out(int packed, const void* x, const void* z, const int64_t z_
   args.add_residual = add_residual ? 1 : 0;
   args.packed = packed;
   if (deferred) {
-    *deferred = args;
+    deferred->mul = args;
+    deferred->is = ModuleEnd::kMul;
     return OF3_OK;
   }
   hipError_t e = of3::trimul_out_launch(args, (int)C, (int)CH, static_cast<hipStream_t>(stream));
@@ -279,13 +296,15 @@ int of3_trimul_out(const void* x, const void* z, const int64_t z_strides[3], voi
 }
 
 // presplit: the fp32 weights as a block's call has split them, or null; packed: the bf16 weight matrices are copies in
-// MFMA operand order; deferred (bf16): the output pass is not launched but handed on, to the `before` of triattn_fwd
+// MFMA operand order; before (bf16): the end of the module before this one, launched with this one's input pass;
+// deferred (bf16): the output pass is not launched but handed on, to the `before` of the next module, in whose frame
+// (transposed: of the canonical one) x is written
 static int trimul_fwd(const of3::WeightX3* presplit, int packed, const void* z, const int64_t z_strides[3], const float* mask,
                    const int64_t mask_strides[3], const void* ln_in_w, const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
                    const void* w_a_p, const void* w_a_g, const void* w_b_p, const void* w_b_g, const void* w_g,
                    const void* w_z, void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int outgoing,
                    int add_residual, void* workspace, int64_t workspace_bytes, int dtype, void* stream,
-                   of3::TrimulOutArgs* deferred = nullptr) {
+                   const ModuleEnd* before = nullptr, ModuleEnd* deferred = nullptr, bool transposed = false) {
   if (dtype == OF3_DTYPE_F32) {
     if (!f32_trimul_dims_ok(B, N, C, CH) || !f32_strides_ok(z_strides) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
     const void* ptrs[] = {z, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_a_p, w_a_g, w_b_p, w_b_g, w_g, w_z, out};
@@ -339,9 +358,9 @@ static int trimul_fwd(const of3::WeightX3* presplit, int packed, const void* z, 
   void* b = ws + part;
   void* x = ws + 2 * part;
   int st = trimul_proj(packed, z, z_strides, mask, mask_strides, ln_in_w, ln_in_b, w_a_p, w_a_g, w_b_p, w_b_g, a, b, B, N,
-                           C, CH, outgoing, stream);
+                           C, CH, outgoing, stream, before);
   if (st != OF3_OK) return st;
-  st = of3_trimul_contract(a, b, x, B, N, CH, 0, stream);
+  st = trimul_contract(a, b, x, B, N, CH, 0, transposed, stream);
   if (st != OF3_OK) return st;
   return trimul_out(packed, x, z, z_strides, out, ln_in_w, ln_in_b, ln_out_w, ln_out_b, w_g, w_z, B, N, C, CH,
                         add_residual, stream, deferred);
@@ -394,7 +413,7 @@ static int triattn_proj(int packed, const void* x, const int64_t x_strides[3], c
                         const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_q,
                         const void* w_k, const void* w_v, const void* w_bias, void* q, void* k, void* vt, float* tbias,
                         float* mbias, int64_t B, int64_t N, int64_t C, int64_t H, int64_t D, float inf, void* stream,
-                        const of3::TrimulOutArgs* before = nullptr) {
+                        const ModuleEnd* before = nullptr) {
   if (!triattn_dims_ok(B, N, C, H, D) || !strides_ok(x_strides) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
   const void* ptrs[] = {x, ln_w, ln_b, w_q, w_k, w_v, w_bias, q, k, vt, tbias, mbias};
   for (const void* p : ptrs)
@@ -422,8 +441,9 @@ static int triattn_proj(int packed, const void* x, const int64_t x_strides[3], c
   args.inf = inf;
   args.packed = packed;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  hipError_t e = before ? of3::trimul_out_triattn_proj_launch(*before, args, (int)C, (int)D, s)
-                        : of3::triattn_proj_launch(args, (int)C, (int)D, s);
+  hipError_t e = !before                             ? of3::triattn_proj_launch(args, (int)C, (int)D, s)
+                 : before->is == ModuleEnd::kMul ? of3::trimul_triattn_launch(before->mul, args, (int)C, s)
+                                                 : of3::triattn_triattn_launch(before->att, args, (int)C, s);
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
@@ -459,7 +479,7 @@ int of3_triattn_flash(const void* q, const void* k, const void* vt, const float*
 
 static int triattn_out(int packed, const void* o, const void* x, const int64_t x_strides[3], void* out,
                        const void* ln_w, const void* ln_b, const void* w_g, const void* w_o, int64_t B, int64_t N,
-                       int64_t C, int64_t H, int64_t D, int add_residual, void* stream) {
+                       int64_t C, int64_t H, int64_t D, int add_residual, void* stream, ModuleEnd* deferred = nullptr) {
   if (!triattn_dims_ok(B, N, C, H, D) || !strides_ok(x_strides)) return OF3_EINVAL;
   const void* ptrs[] = {o, x, out, ln_w, ln_b, w_g, w_o};
   for (const void* p : ptrs)
@@ -477,6 +497,11 @@ static int triattn_out(int packed, const void* o, const void* x, const int64_t x
   args.N = (int)N;
   args.add_residual = add_residual ? 1 : 0;
   args.packed = packed;
+  if (deferred) {
+    deferred->att = args;
+    deferred->is = ModuleEnd::kAtt;
+    return OF3_OK;
+  }
   hipError_t e = of3::triattn_out_launch(args, (int)C, (int)(H * D), static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
@@ -491,7 +516,7 @@ static int triattn_fwd(const of3::WeightX3* presplit, int packed, const void* x,
                     const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_bias, const void* w_q, const void* w_k,
                     const void* w_v, const void* w_g, const void* w_o, void* out, int64_t B, int64_t N, int64_t C,
                     int64_t H, int64_t D, float inf, int add_residual, void* workspace, int64_t workspace_bytes,
-                    int dtype, void* stream, const of3::TrimulOutArgs* before = nullptr) {
+                    int dtype, void* stream, const ModuleEnd* before = nullptr, ModuleEnd* deferred = nullptr) {
   if (dtype == OF3_DTYPE_F32) {
     if (!f32_triattn_dims_ok(B, N, C, H, D) || !f32_strides_ok(x_strides) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
     const void* ptrs[] = {x, ln_w, ln_b, w_bias, w_q, w_k, w_v, w_g, w_o, out};
@@ -553,7 +578,7 @@ static int triattn_fwd(const of3::WeightX3* presplit, int packed, const void* x,
   if (st != OF3_OK) return st;
   st = of3_triattn_flash(q, k, vt, tbias, mbias, o, B, N, H, D, stream);
   if (st != OF3_OK) return st;
-  return triattn_out(packed, o, x, x_strides, out, ln_w, ln_b, w_g, w_o, B, N, C, H, D, add_residual, stream);
+  return triattn_out(packed, o, x, x_strides, out, ln_w, ln_b, w_g, w_o, B, N, C, H, D, add_residual, stream, deferred);
 }
 
 int of3_triattn_fwd(const void* x, const int64_t x_strides[3], const float* mask, const int64_t mask_strides[3],
@@ -954,18 +979,18 @@ static int64_t block_split_bytes(int64_t C, int64_t CH, int64_t H, int64_t D, in
   return align256((int64_t)(2 * of3::trimul_wsplit_bytes(C, CH) + 2 * of3::triattn_wsplit_bytes(C, H, D) +
                             (HID ? of3::transition_wsplit_bytes(C, HID) : 0)));
 }
-// Short bf16 sequences: the pass that ends a triangle multiplication and begins the attention after it reads the one's
-// workspace and writes the other's, so they lie side by side.  Whether a call takes that pass depends on the device, the room
-// does not: up to 1024 tiles of 32 positions.
-static bool shared_pass_room(int dtype, int64_t B, int64_t N) {
-  return dtype == OF3_DTYPE_BF16 && N <= 1024 && B <= 1024 && B * N * ((N + 31) / 32) <= 1024;
+// Short bf16 sequences: the launch that ends one module and begins the next reads the one's workspace and writes the other's,
+// so a triangle multiplication's and an attention's lie side by side.  Whether a call takes such launches depends on the
+// device (join_rows), the room does not: up to 6144 tiles of 32 positions.
+static bool join_room(int dtype, int64_t B, int64_t N) {
+  return dtype == OF3_DTYPE_BF16 && N <= of3::kJoinTokens && B <= 8192 && B * N * ((N + 31) / 32) <= 6144;
 }
 static int64_t pair_block_module_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
                                        int64_t HID) {
   int64_t need = of3_trimul_workspace_bytes_for(dtype, B, N, C, CH);
   const int64_t att = of3_triattn_workspace_bytes_for(dtype, B, N, C, H, D);
   if (need < 0 || att < 0) return OF3_EINVAL;
-  if (shared_pass_room(dtype, B, N)) need += att;
+  if (join_room(dtype, B, N)) need += att;
   else if (att > need) need = att;
   if (HID != 0) {
     if (dtype == OF3_DTYPE_BF16 && (HID < 128 || HID % 32 != 0 || HID > (1 << 16))) return OF3_EINVAL;
@@ -1081,19 +1106,27 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
                           const float* mask, const int64_t mask_strides[3], void* out, int flags, void* workspace,
                           int64_t workspace_bytes, void* stream) {
   const void* src = z;  // the first module reads z, every later one updates out in place
-  bool shared = false;
-  if (!(flags & OF3_BLOCK_ATTENTION_FIRST) && shared_pass_room(d.dtype, d.B, d.N)) {
-    const hipError_t e = of3::trimul_out_triattn_proj_serves((int)d.B, (int)d.N, &shared);
+  int rows = 0;
+  if (k.packed && d.CH == d.C && d.H == 4 && 4 * d.D == d.C && join_room(d.dtype, d.B, d.N)) {
+    const hipError_t e = of3::join_rows((int)d.B, (int)d.N, (int)d.C, &rows);
     if (e != hipSuccess) return fail_hip(e);
+    const int variant = contract_variant_auto(d.B * d.CH, padded(d.N));
+    if (variant != 2 && variant != 3) rows = 0;  // has no transposed form
   }
-  const int64_t skip = shared ? of3_trimul_workspace_bytes(d.B, d.N, d.C, d.CH) : 0;
-  of3::TrimulOutArgs between;
+  const bool joined = rows > 0, attention_first = flags & OF3_BLOCK_ATTENTION_FIRST;
+  const int64_t skip = joined ? of3_trimul_workspace_bytes(d.B, d.N, d.C, d.CH) : 0;
+  ModuleEnd ends[2];
+  int module = 0;  // of the four
+  // the end of the module before, and where this one leaves its own
+  auto before = [&] { return joined && module > 0 ? &ends[(module - 1) & 1] : nullptr; };
+  auto after = [&] { return joined && module < 3 ? &ends[module & 1] : nullptr; };
   auto trimul = [&](int m) {
     const void* const* w = k.w + 10 * m;
     const int st = trimul_fwd(k.mul ? k.mul + m * of3::kTrimulMatrices : nullptr, k.packed, src, z_strides, mask, mask_strides,
                               w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8], w[9], out, d.B, d.N, d.C, d.CH, m == 0,
-                              1, workspace, workspace_bytes, d.dtype, stream, shared && m == 1 ? &between : nullptr);
+                              1, workspace, workspace_bytes, d.dtype, stream, before(), after(), joined && m == 0);
     src = out;
+    ++module;
     return st;
   };
   auto triattn = [&](int m) {
@@ -1103,15 +1136,15 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
     if (mask) mt[0] = mask_strides[0], mt[1] = mask_strides[m ? 2 : 1], mt[2] = mask_strides[m ? 1 : 2];
     const int st = triattn_fwd(k.att ? k.att + m * of3::kTriattnMatrices : nullptr, k.packed, src, zt, mask, mt, w[0], w[1],
                                w[2], w[3], w[4], w[5], w[6], w[7], out, d.B, d.N, d.C, d.H, d.D, d.inf, 1,
-                               static_cast<char*>(workspace) + skip, workspace_bytes - skip, d.dtype, stream,
-                               shared && m == 0 ? &between : nullptr);
+                               static_cast<char*>(workspace) + skip, workspace_bytes - skip, d.dtype, stream, before(), after());
     src = out;
+    ++module;
     return st;
   };
   int st = OF3_OK;
   for (int part = 0; part < 2; ++part)
     for (int m = 0; m < 2 && st == OF3_OK; ++m)
-      st = (part == 0) == !(flags & OF3_BLOCK_ATTENTION_FIRST) ? trimul(m) : triattn(m);
+      st = (part == 0) == !attention_first ? trimul(m) : triattn(m);
   if (st != OF3_OK || d.HID == 0) return st;
   const void* const* w = k.w + 36;
   return transition_fwd(k.tr, d.wide() ? nullptr : k.tr_operands, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask, mask_strides, w[0], w[1],

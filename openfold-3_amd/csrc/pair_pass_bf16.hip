@@ -201,67 +201,6 @@ __global__ __launch_bounds__(2 * C, 3) void trimul_out_panels(TrimulOutArgs p, i
 // ---- triangle attention, input pass (triattn_proj.hip) -------------------------------------------------------
 // Wave = one 32-channel tile of q, k or v (kind 0, 1, 2), the last wave the triangle bias (4 rows, the others of its tile
 // zero).
-template <int C>
-__device__ __forceinline__ void load_attention_unit(const TriattnProjArgs& p, int kind, int ot, int lane, u32x4_t (&w)[C / 16]) {
-  constexpr int H = 4;
-  if (kind == 3) {
-#pragma unroll
-    for (int s = 0; s < C / 16; ++s) {
-      w[s] = u32x4_t{0u, 0u, 0u, 0u};
-      if ((lane & 31) < H) w[s] = *reinterpret_cast<const u32x4_t*>(p.w_b + (lane & 31) * C + 16 * s + 8 * (lane >> 5));
-    }
-  } else {
-    load_unit<C>(kind == 0 ? p.w_q : kind == 1 ? p.w_k : p.w_v, ot, kind == 2 ? lane & 31 : rowperm16(lane & 31), lane >> 5, p.packed, w);
-  }
-}
-// products and stores of the wave for the normalised positions j0 .. j0 + 31 of row bi
-template <int C, int D>
-__device__ __forceinline__ void project_panel(const TriattnProjArgs& p, const u32x4_t (&w)[C / 16], const PanelTile<C, true>& tile, int kind,
-                                              int ot, int bi, int j0) {
-  typedef PanelTile<C, true> Tile;
-  constexpr int H = 4, KS = C / 16;
-  const int N = p.N, Jp = p.Jp;
-  const float qscale = kLog2e * __builtin_amdgcn_rsqf((float)D);
-  const Lane at = lane_here();
-  const int l32 = at.l32, lh = at.lh;
-  f32x16_t acc = zero16();
-  float res[16];
-  bf16_t* dst;
-  if (kind == 3) {
-#pragma unroll
-    for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(w[s], tile.s[Tile::slot(l32, 2 * s + lh)], acc);
-    if (lh == 0) {  // rows 0..3 of the result: registers 0..3 of lanes 0..31
-      const int b = bi / N, i = bi - b * N, j = j0 + l32;
-#pragma unroll
-      for (int h = 0; h < H; ++h) p.tbias[(((size_t)b * H + h) * N + i) * Jp + j] = j < N ? acc[h] * kLog2e : 0.f;
-    }
-    return;
-  }
-  if (kind == 2) {
-    // V^T panel: rows = keys (dealt by rowperm16), columns = channels; lane: channel 32 ot + l32, keys 16 lh + v
-    const int kpos = rowperm16(l32);
-#pragma unroll
-    for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(tile.s[Tile::slot(kpos, 2 * s + lh)], w[s], acc);
-    const int ch = 32 * ot + l32, head = ch / D, d = ch % D;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) res[v] = acc[v];
-    dst = p.vt + ((size_t)bi * H + head) * D * Jp + (size_t)(j0 >> 5) * (D * 32) + d * 32 + 16 * lh;
-  } else {
-#pragma unroll
-    for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(w[s], tile.s[Tile::slot(l32, 2 * s + lh)], acc);
-    const int ch0 = 32 * ot + 16 * lh, head = ch0 / D, d0 = ch0 % D;
-    const float sc = kind == 0 ? qscale : 1.f;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) res[v] = acc[v] * sc;
-    dst = (kind == 0 ? p.q : p.k) + (((size_t)bi * H + head) * Jp + j0 + l32) * D + d0;
-  }
-  store16(dst, res);
-}
-// log2(e) times the mask bias of position j of row bi
-__device__ __forceinline__ void store_mask_bias(const TriattnProjArgs& p, int bi, int j, float mask) {
-  p.mbias[(size_t)bi * p.Jp + j] = j < p.N ? kLog2e * (p.inf * (mask - 1.f)) : -__builtin_inff();
-}
-
 template <int C, int D>
 __global__ __launch_bounds__(6 * C + 64) void triattn_proj_panels(TriattnProjArgs p, int panels, int total) {
   typedef PanelTile<C, true> Tile;
@@ -301,107 +240,6 @@ __global__ __launch_bounds__(6 * C + 64) void triattn_proj_panels(TriattnProjArg
     __syncthreads();  // the tile is complete, everybody has finished with the other one
     project_panel<C, D>(p, w, tile, kind, ot, bi, j0);
   }
-}
-
-// ---- the two passes between a triangle multiplication and the triangle attention after it, in one ------------
-// One tile per work-group: the output pass of the multiplication (trimul_out_panels) by the first C / 32 waves, its
-// result rounded to bf16, stored, and normalised again from LDS for the projections of the attention
-// (triattn_proj_panels).  Bound, as both passes are at these sizes, by the chain of loads, LayerNorms and barriers
-// (5.5 and 5.4 us at N = 40); what goes is a launch with its drain and start (2 us), a trip to memory for z, and the
-// wait for the attention's weights, which most waves request at the start.  us per call: four updates at N = 80 91.5 -> 87,
-// at N = 50 80 -> 78; two blocks of a template at N = 64 192 -> 184; 4 trunk blocks at N = 40 478 -> 467 (bound by the host).
-// p.out (= a.x) has a.x_view's addressing.
-template <int C, int D>
-__global__ __launch_bounds__(6 * C + 64) void trimul_out_triattn_proj_panels(TrimulOutArgs p, TriattnProjArgs a, int panels) {
-  typedef PanelTile<C, false> OTile;
-  typedef PanelTile<C, true> PTile;
-  typedef LnLane<C> Ln;
-  constexpr int KS = C / 16, OT = C / 32, NTASK = 32 / Ln::PPI;
-  static_assert(NTASK <= 3 * OT + 1, "");
-  __shared__ u32x4_t zt[OTile::SLOTS], xt[OTile::SLOTS], ut[OTile::SLOTS], nt[PTile::SLOTS];
-  const OTile zn = {zt}, xn = {xt}, upd = {ut};
-  const PTile tile = {nt};
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int N = p.N, Np = p.Np;
-  const int kind = wave / OT, ot = wave % OT;
-  const bool first = wave < OT;
-  const int id = grid_slot(), bi = id / panels, j0 = 32 * (id - bi * panels), b = bi / N, i = bi - b * N;
-  const bf16_t* const zrow = p.z + b * p.z_view.stride_b + i * p.z_view.stride_r;
-
-  u32x4_t w[KS], wz[KS], raw;
-  uint32_t xraw[8];
-  float mraw = 1.f;
-  const int ln_chunk = lane % Ln::NCH, pos = wave * Ln::PPI + lane / Ln::NCH;  // LayerNorm: waves below NTASK
-  const int j_ln = j0 + pos < N ? j0 + pos : N - 1;
-  if (wave < NTASK) {
-    raw = *reinterpret_cast<const u32x4_t*>(zrow + j_ln * p.z_view.stride_k + 8 * ln_chunk);
-    if (a.mask) mraw = a.mask[b * a.mask_view.stride_b + i * a.mask_view.stride_r + j_ln * a.mask_view.stride_k];
-  }
-  const int xp = tid & 15, xc = tid >> 4;  // position pair and chunk of x, threads of the first waves
-  if (first) {
-    const bf16_t* x = p.x + (((size_t)b * C + 8 * xc) * Np + i) * Np + j0 + 2 * xp;  // planes are padded: always inside
-#pragma unroll
-    for (int e = 0; e < 8; ++e) xraw[e] = *reinterpret_cast<const uint32_t*>(x + (size_t)e * Np * Np);
-    load_unit<C>(p.w_g, wave, rowperm16(lane & 31), lane >> 5, p.packed, w);
-    load_unit<C>(p.w_z, wave, rowperm16(lane & 31), lane >> 5, p.packed, wz);
-  } else {
-    load_attention_unit<C>(a, kind, ot, lane, w);
-  }
-  const Ln lz = ln_lane<C>(p.ln_in_w, p.ln_in_b, lane), lx = ln_lane<C>(p.ln_out_w, p.ln_out_b, lane),
-           la = ln_lane<C>(a.ln_w, a.ln_b, lane);
-  if (wave < NTASK) zn.s[OTile::slot(pos, ln_chunk)] = lz.template normalised<true>(raw);
-  if (first) {  // x as it is into position-major order: a thread holds one chunk of two positions
-    u32x4_t lo, hi;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      lo[q] = __builtin_amdgcn_perm(xraw[2 * q + 1], xraw[2 * q], 0x05040100u);
-      hi[q] = __builtin_amdgcn_perm(xraw[2 * q + 1], xraw[2 * q], 0x07060302u);
-    }
-    xn.s[OTile::slot(2 * xp, xc)] = lo;
-    xn.s[OTile::slot(2 * xp + 1, xc)] = hi;
-  }
-  __syncthreads();
-  if (wave < NTASK) {  // LayerNorm in place
-    u32x4_t& x = xn.s[OTile::slot(pos, ln_chunk)];
-    x = lx.template normalised<false>(x);
-  }
-  __syncthreads();
-  if (first) {
-    const Lane at = lane_here();
-    const int l32 = at.l32, lh = at.lh;
-    f32x16_t ag = zero16(), az = zero16();
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const int slot = OTile::slot(l32, 2 * s + lh);
-      az = mfma_32x32x16(wz[s], xn.s[slot], az);
-      ag = mfma_32x32x16(w[s], zn.s[slot], ag);
-    }
-    load_attention_unit<C>(a, kind, ot, lane, w);  // kind 0: under the rest of this pass
-    // lane (position l32, half lh): channels 32 wave + 16 lh + v
-    if (j0 + l32 < N) {
-      const int64_t off = (j0 + l32) * p.z_view.stride_k + 32 * wave + 16 * lh;
-      float res[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) res[e] = az[e] * sigmoid_from_scaled(ag[e]);
-      if (p.add_residual) add16(zrow + off, res);
-      u32x4_t o[2];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) o[0][q] = pack_bf16(res[2 * q], res[2 * q + 1]), o[1][q] = pack_bf16(res[8 + 2 * q], res[8 + 2 * q + 1]);
-      bf16_t* dst = p.out + b * p.z_view.stride_b + i * p.z_view.stride_r + off;
-      *reinterpret_cast<u32x4_t*>(dst) = o[0];
-      *reinterpret_cast<u32x4_t*>(dst + 8) = o[1];
-#pragma unroll
-      for (int half = 0; half < 2; ++half) upd.s[OTile::slot(l32, 4 * wave + 2 * lh + half)] = o[half];
-    }
-  }
-  __syncthreads();
-  if (wave < NTASK) {  // positions past the end are copies of the last one, as in triattn_proj_panels
-    tile.s[PTile::slot(pos, ln_chunk)] = la.template normalised<false>(upd.s[OTile::slot(j_ln - j0, ln_chunk)]);
-    if (ln_chunk == 0) store_mask_bias(a, bi, j0 + pos, mraw);
-  }
-  __syncthreads();
-  project_panel<C, D>(a, w, tile, kind, ot, bi, j0);
 }
 
 // ---- triangle attention, output pass (triattn_out.hip) -------------------------------------------------------
@@ -522,12 +360,6 @@ hipError_t launch_triattn_proj(const TriattnProjArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL((triattn_proj_panels<C, D>), dim3(grid), dim3(6 * C + 64), 0, stream, a, panels, (int)total);
   return hipGetLastError();
 }
-template <int C, int D>
-hipError_t launch_out_proj(const TrimulOutArgs& o, const TriattnProjArgs& a, hipStream_t stream) {
-  const int panels = (o.N + 31) / 32;
-  hipLaunchKernelGGL((trimul_out_triattn_proj_panels<C, D>), dim3((unsigned)(o.B * o.N * panels)), dim3(6 * C + 64), 0, stream, o, a, panels);
-  return hipGetLastError();
-}
 template <int C>
 hipError_t launch_triattn_out(const TriattnOutArgs& a, hipStream_t stream) {
   const int panels = (a.N + 31) / 32;
@@ -550,15 +382,6 @@ hipError_t trimul_out_panels_launch(const TrimulOutArgs& a, int C, hipStream_t s
 hipError_t triattn_proj_panels_launch(const TriattnProjArgs& a, int C, hipStream_t stream) {
   return C == 128 ? launch_triattn_proj<128, 32>(a, stream) : launch_triattn_proj<64, 16>(a, stream);
 }
-hipError_t trimul_out_triattn_proj_launch(const TrimulOutArgs& o, const TriattnProjArgs& a, int C, int D, hipStream_t stream) {
-  if (o.B != a.B || o.N != a.N || a.H != 4 || 4 * D != C || (C != 128 && C != 64)) return hipErrorInvalidValue;
-  bool small = false;
-  const hipError_t e = trimul_out_triattn_proj_serves(o.B, o.N, &small);
-  if (e != hipSuccess) return e;
-  if (!small) return hipErrorInvalidValue;
-  return C == 128 ? launch_out_proj<128, 32>(o, a, stream) : launch_out_proj<64, 16>(o, a, stream);
-}
-hipError_t trimul_out_triattn_proj_serves(int B, int N, bool* serves) { return small_pass(B, N, 1, serves); }
 hipError_t triattn_out_panels_launch(const TriattnOutArgs& a, int C, hipStream_t stream) {
   return C == 128 ? launch_triattn_out<128>(a, stream) : launch_triattn_out<64>(a, stream);
 }

@@ -61,7 +61,9 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | 0x70 | 0xF00 | ((N >> 4) << 14));
 }
 
-template <int BN, int kNS>
+// TRANSPOSED: every plane of x is written as its transpose, for a reader that walks columns (pair_join_bf16.hip).  The products
+// take their operands the other way round: the same sums, with a lane's values along i.
+template <int BN, int kNS, bool TRANSPOSED>
 __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restrict__ pm,  // j side planes (b)
                                                           const bf16_t* __restrict__ pn,  // i side planes (a)
                                                           bf16_t* __restrict__ x, int Np, int nk, int tiles_m,
@@ -181,11 +183,12 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
   for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
     for (int nt = 0; nt < TN; ++nt) acc[mt][nt] = zero16();
+  auto product = [&](u32x4_t af, u32x4_t bfr, f32x16_t c) { return TRANSPOSED ? mfma_32x32x16(bfr, af, c) : mfma_32x32x16(af, bfr, c); };
   auto mma = [&](const u32x4_t (&af)[TM], const u32x4_t (&bfr)[TN]) {
 #pragma unroll
     for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < TN; ++nt) acc[mt][nt] = mfma_32x32x16(af[mt], bfr[nt], acc[mt][nt]);
+      for (int nt = 0; nt < TN; ++nt) acc[mt][nt] = product(af[mt], bfr[nt], acc[mt][nt]);
   };
   // the same, with the refill's loads issued in between
   auto mma_and_issue = [&](const u32x4_t (&af)[TM], const u32x4_t (&bfr)[TN]) {
@@ -194,7 +197,7 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
     for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
       for (int nt = 0; nt < TN; ++nt) {
-        acc[mt][nt] = mfma_32x32x16(af[mt], bfr[nt], acc[mt][nt]);
+        acc[mt][nt] = product(af[mt], bfr[nt], acc[mt][nt]);
         if (n < IPW) issue_one(n++);
       }
     issue_advance();
@@ -225,7 +228,7 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
       // carries the wait for a0/b0 (with direct-to-LDS loads in flight every LDS wait the
       // compiler emits is a wait for all outstanding reads), so the new reads travel under the
       // remaining MFMAs instead of being waited for at once.
-      acc[0][0] = mfma_32x32x16(a0[0], b0[0], acc[0][0]);
+      acc[0][0] = product(a0[0], b0[0], acc[0][0]);
       __builtin_amdgcn_sched_barrier(0);
       fetch(cur, 1, a1, b1);
       __builtin_amdgcn_sched_barrier(0);
@@ -233,7 +236,7 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
       for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
         for (int nt = 0; nt < TN; ++nt)
-          if (mt + nt > 0) acc[mt][nt] = mfma_32x32x16(a0[mt], b0[nt], acc[mt][nt]);
+          if (mt + nt > 0) acc[mt][nt] = product(a0[mt], b0[nt], acc[mt][nt]);
       __builtin_amdgcn_sched_barrier(0);
 
       // This wave holds all of stage s in registers.  Stages s+1..s+3 are in flight and
@@ -268,6 +271,41 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
     u32x4_t* epi = lds + kNS * STAGE + wave * 512;
     const int jbase = tm * BM + wm0;
     int n_stores = 0;
+    if constexpr (TRANSPOSED) {
+      // 32 columns j at a time: staged as rows of WN i's (8-byte pieces: a lane holds runs of four), out as row segments
+      constexpr int CHR = WN / 8;
+      static_assert(CHR == 8 || CHR == 16, "the swizzle permutes chunks in groups of eight");
+      auto key = [](int row) { return row & 7; };
+      const int i0 = tn * BN + wn0, Nr = 32 * nk;
+      const bool whole = i0 + WN <= Nr && jbase + WM <= Nr;
+      u32x2_t* const epi2 = reinterpret_cast<u32x2_t*>(epi);
+#pragma unroll
+      for (int mt = 0; mt < TM; ++mt) {
+#pragma unroll
+        for (int nt = 0; nt < TN; ++nt) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {  // registers 4g..4g+3: i-local = 32*nt + 8*g + 4*lh + (0..3)
+            const u32x2_t v = {pack_bf16(acc[mt][nt][4 * g], acc[mt][nt][4 * g + 1]),
+                               pack_bf16(acc[mt][nt][4 * g + 2], acc[mt][nt][4 * g + 3])};
+            epi2[(l32 * CHR + ((4 * nt + g) ^ key(l32))) * 2 + lh] = v;
+          }
+          acc[mt][nt] = zero16();
+        }
+#pragma unroll
+        for (int rr = 0; rr < CHR / 2; ++rr) {
+          const int idx = 64 * rr + lane, row = idx / CHR, chunk = idx % CHR;
+          const u32x4_t v = epi[row * CHR + (chunk ^ key(row))];
+          // operand row `row` of the tile: j-local as in am_slot
+          const int j = jbase + 16 * TM * ((row >> 2) & 1) + 16 * mt + 4 * (row >> 3) + (row & 3), i = i0 + 8 * chunk;
+          if (whole || (j < Nr && i < Nr)) *reinterpret_cast<u32x4_t*>(xo + (size_t)j * Np + i) = v;
+        }
+        if (whole) n_stores += CHR / 2;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      static_assert(TM * (CHR / 2) == 8 * TN, "as many stores as the other form");
+      stores_pending = n_stores == 8 * TN;
+      continue;
+    }
 #pragma unroll
     for (int nt = 0; nt < TN; ++nt) {
 #pragma unroll
@@ -313,10 +351,10 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
   wait_vmcnt<0>();  // loads issued past the end must not outlive the work-group's LDS
 }
 
-template <int BN, int kNS>
+template <int BN, int kNS, bool TRANSPOSED>
 hipError_t launch_contract(const bf16_t* a, const bf16_t* b, bf16_t* x, int planes, int Np, int nk, hipStream_t stream) {
   constexpr int BM = 256;
-  auto kern = contract_kernel<BN, kNS>;
+  auto kern = contract_kernel<BN, kNS, TRANSPOSED>;
   const size_t smem = ((size_t)kNS * (BM + BN) * 4 + 4 * 512) * sizeof(u32x4_t);  // ring + epilogue staging
   static int cache[kMaxDevices];
   int cus = 0;
@@ -594,18 +632,22 @@ hipError_t launch_contract8(const bf16_t* a, const bf16_t* b, bf16_t* x, int pla
 }  // namespace
 
 hipError_t trimul_contract_launch(const bf16_t* a, const bf16_t* b, bf16_t* x, int planes, int Np, int nk, int variant,
-                                  hipStream_t stream) {
+                                  bool transposed, hipStream_t stream) {
   if (nk < 1 || nk > Np / kBK) return hipErrorInvalidValue;
-  switch (variant) {
+  switch (transposed ? variant + 8 : variant) {
     case 1:
-      return launch_contract<192, 4>(a, b, x, planes, Np, nk, stream);
+      return launch_contract<192, 4, false>(a, b, x, planes, Np, nk, stream);
     case 2:
-      return launch_contract<128, 4>(a, b, x, planes, Np, nk, stream);
+      return launch_contract<128, 4, false>(a, b, x, planes, Np, nk, stream);
     case 3:
-      return launch_contract<256, 4>(a, b, x, planes, Np, nk, stream);
+      return launch_contract<256, 4, false>(a, b, x, planes, Np, nk, stream);
     case 4:
       return launch_contract8<3>(a, b, x, planes, Np, nk, stream);
-    default:
+    case 10:
+      return launch_contract<128, 4, true>(a, b, x, planes, Np, nk, stream);
+    case 11:
+      return launch_contract<256, 4, true>(a, b, x, planes, Np, nk, stream);
+    default:  // 192-wide tiles have no transposed form: up to 256 tokens they are never the choice
       return hipErrorInvalidValue;
   }
 }

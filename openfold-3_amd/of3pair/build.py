@@ -40,7 +40,7 @@ SOURCES = [
     "transition_f32.hip",
     "weight_split.hip",
     "weight_pack.hip",
-    "pair_pass_bf16.hip", "transition_tiles_bf16.hip",
+    "pair_pass_bf16.hip", "pair_join_bf16.hip", "transition_tiles_bf16.hip",
     "single_f32.hip",
     "single_x3_f32.hip",
 ]
