@@ -7,10 +7,10 @@
 // With head width 16 or 32 the kernel is bound by the softmax's vector instructions (a SIMD spends
 // matrix time plus vector time), so the organisation removes vector work and keeps four waves per
 // SIMD to cover each other's waits:
-//  * work-group = 8 waves = 4 consecutive rows i x 2 halves of one (head, 128-query range); a wave
-//    owns 64 queries (two 32-query tiles) of one row; two work-groups share a CU (64 KB of LDS and
-//    128 registers per lane each).  The triangle bias of the query range does not depend on i:
-//    each 32-key slice of it is brought into LDS once per work-group and every wave reads it
+//  * work-group = 4 consecutive rows i x one (head, query range); a wave owns two (four) 32-query tiles of one row.  Long
+//    launches with heads of 32: 8 waves, 128 queries, two work-groups per CU (64 KB of LDS and 128 registers per lane
+//    each); otherwise 4 waves, 64 or 128 queries, three or four work-groups per CU.  The triangle bias of the query range
+//    does not depend on i: each 32-key slice of it is brought into LDS once per work-group and every wave reads it
 //    straight into the MFMA accumulator, which adds it for free.
 //  * everything a key tile needs (the work-group's bias slice, each row's K tile and V^T tile,
 //    loaded by one wave of the row each) travels global -> LDS with direct-to-LDS buffer loads, one
@@ -47,14 +47,6 @@
 
 #include <type_traits>
 
-// Token count from which the 16-wave form (256 queries per work-group, one work-group per CU) is used.
-// Measured against the 8-wave form (two work-groups per CU): N = 768 395 vs 375 us, N = 2048 7.57 vs
-// 6.95 ms, 4 x 512 with head width 16 474 vs 400 us: the K / V^T loads it saves cost less than the second
-// independent work-group hides, so the default is never.
-#ifndef OF3_FLASH_WIDE_FROM
-#define OF3_FLASH_WIDE_FROM (1 << 30)
-#endif
-
 namespace of3 {
 
 namespace {
@@ -77,14 +69,7 @@ __device__ __forceinline__ int key2(int row) { return (row >> 4) & 1; }  // 2 ch
 // Every iteration of the tile loop issues the same loads (indices past the end are clamped, their
 // data is never read), so that the compiler can count the loads in flight and its own waits do not
 // drain the ring.
-// 32-query tiles per wave: 2 (the shipped form) or 1 (half the accumulators, so that six waves per SIMD fit:
-// measured slower, head width 16 at 4 x 512^2 443 vs 392 us with 76 registers and no spills, head width 32
-// does not fit 80 registers; a K / V^T tile read from LDS then serves half as many logits)
-#ifndef OF3_FLASH_RQ
-#define OF3_FLASH_RQ 2
-#endif
-constexpr int kRows = 4, kRQ = OF3_FLASH_RQ, kStages = 2;
-constexpr int kQW = 32 * kRQ;  // queries per wave
+constexpr int kRows = 4, kStages = 2;
 #ifndef OF3_FLASH_RG_BLOCK
 #define OF3_FLASH_RG_BLOCK 8
 #endif
@@ -99,13 +84,16 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   return r;
 }
 
-// QW = waves per row: 2 (work-group = 8 waves = 4 rows x 128 queries, two work-groups per CU) or 4 (16 waves
-// = 4 rows x 256 queries, one work-group per CU: a row's K and V^T tiles, the loads that miss L2, are brought
-// in for twice as many queries).
-template <int D, int QW>
-__global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_flash_kernel(TriattnFlashArgs p, int n_qc, int n_rg,
-                                                                             int total, int per_xcd) {
+// QW = waves per row, RQ = 32-query tiles per wave: a work-group is 4 rows x 32 QW RQ queries.  Two waves (128 queries, two
+// work-groups of 8 waves per CU) move the fewest K and V^T bytes into LDS; one wave (64 or 128 queries, four or three work-groups
+// of 4 waves per CU) needs one K / V^T stage in place of two, and its smaller work-groups fill a short launch better.  Which
+// is taken where: triattn_flash_launch.  (Four waves, one work-group per CU, were slower everywhere: N = 768 395 against 375 us;
+// one 32-query tile per wave, too: 4 x 512 with head width 16 443 against 392 us.)
+template <int D, int QW, int RQ>
+__global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flash_kernel(TriattnFlashArgs p, int n_qc, int n_rg, int total,
+                                                                                        int per_xcd) {
   constexpr int kWaves = kRows * QW;
+  constexpr int kRQ = RQ, kQW = 32 * RQ;  // queries per wave
   constexpr int QWG = kQW * QW;  // queries per work-group
   constexpr int H = 4;
   constexpr int HD = H * D;
@@ -117,15 +105,17 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
   constexpr int KI = KSLOTS / 64, VI = VSLOTS / 64;
   static_assert(KI == VI, "a row's K and V^T tiles take the same number of load instructions");
   constexpr int KVI = KI + VI;                       // 1-KB load instructions per row and tile: K0, (K1), V0, (V1)
-  constexpr int SPW = KVI / QW > 0 ? KVI / QW : 1;   // of which a wave issues this many (waves beyond KVI: none)
+  constexpr int SPW = KVI / QW;                      // of which a wave issues this many
+  static_assert(QW == 1 || QW == 2, "one wave brings a row's K and V^T tiles, or two one each");
+  // K and V^T stages: a row's only wave (QW = 1) requests the next tile when it holds this one's operands in registers
+  constexpr int KVST = QW == 1 ? 1 : kStages;
   constexpr int TBS = QWG * 8;  // [QWG q][32 k] fp32 in 16-byte slots
   constexpr int TBI = kRQ;  // bias instructions per wave and tile
   static_assert(TBI * 64 * kWaves == TBS, "the waves share the bias slice evenly");
-  constexpr int LPT = TBI + KI;
 
   extern __shared__ u32x4_t lds[];
   u32x4_t* tb_lds = lds;                         // [kStages][TBS]
-  u32x4_t* kv_lds = lds + kStages * TBS;        // [kRows][kStages][KVS]
+  u32x4_t* kv_lds = lds + kStages * TBS;        // [kRows][KVST][KVS]
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -177,7 +167,8 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
 
   // bias slice: instruction n of wave w fills slots 64*(TBI*w+n)..+63; slot t holds chunk
   // (t & 7) ^ ((q >> 1) & 7) of query q = t >> 3 of the work-group's range
-  uint32_t tb_off[TBI];
+  uint32_t tb_off[4];  // TBI of them: with the dependent size clang leaves the kernel out of the host code
+  static_assert(TBI <= 4, "");
 #pragma unroll
   for (int n = 0; n < TBI; ++n) {
     const int t = 64 * (TBI * wave + n) + lane;
@@ -186,41 +177,44 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
     qrow = qrow < N ? qrow : N - 1;
     tb_off[n] = (uint32_t)(((size_t)qrow * Jp + 4 * chunk) * sizeof(float));
   }
-  // the wave's share of its row's stage: SPW of the row's KVI load instructions, all of the K tile or all
-  // of the V^T tile (the second instruction of a tile takes rows 16 further on, which flips bit 1 of
-  // key4: its offset is (first ^ 32) + 1024)
+  // The wave's share of its row's stage, all of the K tile, all of the V^T tile, or (QW = 1) both.  The second instruction
+  // of a tile takes rows 16 further on, which flips bit 1 of key4: its offset is (first ^ 32) + 1024
   static_assert(KI == 1 || (KI == 2 && QCH == 4), "offset rule of the second instruction");
-  const int slot0 = qq * SPW;               // first instruction slot of this wave
-  const bool has_kv = slot0 < KVI;          // wave-uniform
-  const bool is_v = slot0 >= KI;
-  const int idx0 = is_v ? slot0 - KI : slot0;
-  uint32_t kv_off;
-  if (!is_v) {
+  const bool is_v = QW == 2 && qq == 1;  // what the first SPW / 2 (QW = 1) or all of its instructions bring
+  auto k_offset = [&] {
     const int r = lane / QCH, chunk = (lane % QCH) ^ (QCH == 4 ? key4(r) : key2(r));
-    kv_off = (uint32_t)((r * D + 8 * chunk) * sizeof(bf16_t));
-  } else {
+    return (uint32_t)((r * D + 8 * chunk) * sizeof(bf16_t));
+  };
+  auto v_offset = [&] {
     const int r = lane >> 2, chunk = (lane & 3) ^ key4(r);
-    kv_off = (uint32_t)((r * 32 + 8 * chunk) * sizeof(bf16_t));
-  }
-  if (idx0 == 1) kv_off = (kv_off ^ 32u) + 1024u;
-  u32x4_t* kv_row = kv_lds + row * (kStages * KVS);
+    return (uint32_t)((r * 32 + 8 * chunk) * sizeof(bf16_t));
+  };
+  const uint32_t kv_off = is_v ? v_offset() : k_offset(), v_off = QW == 1 ? v_offset() : 0u;
+  u32x4_t* kv_row = kv_lds + row * (KVST * KVS);
   // Loads go through buffer descriptors (scalar base, 32-bit lane offset, scalar tile offset): the
   // addresses cost one register per stream, and a load beyond its range would return zeros.
   const __amdgpu_buffer_rsrc_t tb_rsrc = buffer_rsrc(tb, (size_t)N * Jp * sizeof(float));
   const __amdgpu_buffer_rsrc_t kv_rsrc = buffer_rsrc(is_v ? Vt : K, (size_t)Jp * D * sizeof(bf16_t));
+  const __amdgpu_buffer_rsrc_t v_rsrc = buffer_rsrc(Vt, (size_t)Jp * D * sizeof(bf16_t));  // QW = 1
   const __amdgpu_buffer_rsrc_t mb_rsrc = buffer_rsrc(mb, (size_t)Jp * sizeof(float));
-  auto issue_loads = [&](int kt, int buf) {  // buf is a constant at every call site
+  auto issue_bias = [&](int kt, int buf) {  // buf is a constant at every call site
     u32x4_t* tdst = tb_lds + buf * TBS + 64 * TBI * wave;
-    u32x4_t* kdst = kv_row + buf * KVS + (is_v ? KSLOTS : 0) + 64 * idx0;
 #pragma unroll
     for (int n = 0; n < TBI; ++n)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(tb_rsrc, (void OF3_LDS_AS*)(tdst + 64 * n), 16, tb_off[n],
                                                kt * (32 * (int)sizeof(float)), 0, 0);
+  };
+  auto issue_kv = [&](int kt, int buf) {
+    u32x4_t* kdst = kv_row + (KVST == 1 ? 0 : buf) * KVS + (is_v ? KSLOTS : 0);
     const int kv_tile = kt * (32 * D * (int)sizeof(bf16_t));
-    if (has_kv) {  // wave-uniform and the same in every tile: the number of loads per tile stays a constant of the wave
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(kv_rsrc, (void OF3_LDS_AS*)kdst, 16, kv_off, kv_tile, 0, 0);
-      if (SPW == 2)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(kv_rsrc, (void OF3_LDS_AS*)(kdst + 64), 16, (kv_off ^ 32u) + 1024u,
+#pragma unroll
+    for (int n = 0; n < KI; ++n)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(kv_rsrc, (void OF3_LDS_AS*)(kdst + 64 * n), 16, n ? (kv_off ^ 32u) + 1024u : kv_off, kv_tile,
+                                               0, 0);
+    if (QW == 1) {
+#pragma unroll
+      for (int n = 0; n < VI; ++n)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rsrc, (void OF3_LDS_AS*)(kdst + KSLOTS + 64 * n), 16, n ? (v_off ^ 32u) + 1024u : v_off,
                                                  kv_tile, 0, 0);
     }
   };
@@ -279,7 +273,26 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
   // still takes part in the loads and barriers of its work-group but leaves the arithmetic out; so does
   // a 32-query tile past the end.  All of these are wave-uniform.
   const bool wave_has_work = row_valid && q0 < N;
-  auto tile = [&](auto track, int buf, float mb_cur) {
+  // operands of a tile
+  struct Operands {
+    u32x4_t k[KSQ], v[2];
+  };
+  auto read_operands = [&](int buf) {
+    const u32x4_t* kvb = kv_row + (KVST == 1 ? 0 : buf) * KVS;
+    Operands o;
+#pragma unroll
+    for (int ks = 0; ks < KSQ; ++ks) o.k[ks] = kvb[k_rd[ks]];
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      const u32x4_t v = kvb[v_rd[s2]];
+      // head width 16: rows 16..31 of the operand are free; row 16 is ones (the row sum), the rest zeros
+      const uint32_t fill = (krow == 16) ? 0x3F803F80u : 0u;
+      const u32x4_t z = {fill, fill, fill, fill};
+      o.v[s2] = (D == 32 || vvalid) ? v : z;
+    }
+    return o;
+  };
+  auto tile = [&](auto track, int buf, float mb_cur, const Operands& given) {
     constexpr bool kTrack = decltype(track)::value;
     if (!wave_has_work) return;
     // first pass: a tile whose keys are all masked or padded adds exp2(-1.44e9 + logit) = 0 exactly to
@@ -288,18 +301,7 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
     if (!kTrack && __builtin_amdgcn_ballot_w64(mb_cur > kMaskedBelow) == 0) return;
     const bool has_mb = __builtin_amdgcn_ballot_w64(mb_cur != 0.f) != 0;
     const u32x4_t* tbuf = tb_lds + buf * TBS + tb_row;
-    const u32x4_t* kvb = kv_row + buf * KVS;
-    u32x4_t kc[KSQ], vc[2];
-#pragma unroll
-    for (int ks = 0; ks < KSQ; ++ks) kc[ks] = kvb[k_rd[ks]];
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      const u32x4_t v = kvb[v_rd[s2]];
-      // head width 16: rows 16..31 of the operand are free; row 16 is ones (the row sum), the rest zeros
-      const uint32_t fill = (krow == 16) ? 0x3F803F80u : 0u;
-      const u32x4_t z = {fill, fill, fill, fill};
-      vc[s2] = (D == 32 || vvalid) ? v : z;
-    }
+    const Operands op = KVST == 1 ? given : read_operands(buf);
 #pragma unroll
     for (int rq = 0; rq < kRQ; ++rq) {
       if (rq > 0 && q0 + 32 * rq >= N) continue;
@@ -312,7 +314,7 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
       }
       if (has_mb) s = mask_step(mb_cur, s);
 #pragma unroll
-      for (int ks = 0; ks < KSQ; ++ks) s = mfma_32x32x16(kc[ks], qop[rq][ks], s);
+      for (int ks = 0; ks < KSQ; ++ks) s = mfma_32x32x16(op.k[ks], qop[rq][ks], s);
 
       if constexpr (kTrack) {
         float mx = max3(s[0], s[1], s[2]);
@@ -350,7 +352,7 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
         }
         pop0[w] = pack_bf16(e0, e1);
       }
-      oacc[rq] = mfma_32x32x16(vc[0], pop0, oacc[rq]);
+      oacc[rq] = mfma_32x32x16(op.v[0], pop0, oacc[rq]);
       if (D == 32 && !kTrack) lsum[rq] = mfma_16x16x32(ones_a, pop0, lsum[rq]);
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
@@ -361,7 +363,7 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
         }
         pop1[w] = pack_bf16(e0, e1);
       }
-      oacc[rq] = mfma_32x32x16(vc[1], pop1, oacc[rq]);
+      oacc[rq] = mfma_32x32x16(op.v[1], pop1, oacc[rq]);
       if (D == 32 && !kTrack) lsum[rq] = mfma_16x16x32(ones_a, pop1, lsum[rq]);
       l_run[rq] = rs;
     }
@@ -371,7 +373,8 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
   float mb_next;
   auto first_loads = [&]() {
     mb_next = __uint_as_float(load_mb(0, mb_off));
-    issue_loads(0, 0);
+    issue_bias(0, 0);
+    issue_kv(0, 0);
   };
   auto pass = [&](auto track) {
 #pragma unroll
@@ -388,8 +391,15 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
       const float mb_cur = mb_next;
       const int ktn = kt + 1 < nkt ? kt + 1 : nkt - 1;
       mb_next = __uint_as_float(load_mb(ktn, mb_off));
-      issue_loads(ktn, buf ^ 1);
-      tile(track, buf, mb_cur);
+      issue_bias(ktn, buf ^ 1);
+      Operands op;
+      if (KVST == 1) {
+        op = read_operands(buf);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): they have arrived, their place in LDS is free
+        compiler_fence();
+      }
+      issue_kv(ktn, buf ^ 1);
+      tile(track, buf, mb_cur, op);
       compiler_fence();
     };
     for (int kt = 0; kt < nkt; kt += 2) {
@@ -461,30 +471,20 @@ __global__ __launch_bounds__(64 * kRows * QW, kRQ == 1 ? 6 : 4) void triattn_fla
 }
 
 
-template <int D, int QW>
+template <int D, int QW, int RQ>
 constexpr int lds_bytes() {
-  return (kStages * kQW * QW * 8 + kRows * kStages * (32 * (D / 8) + D * 4)) * 16;
+  return (kStages * 32 * RQ * QW * 8 + kRows * (QW == 1 ? 1 : kStages) * (32 * (D / 8) + D * 4)) * 16;
 }
 
-template <int D, int QW>
+template <int D, int QW, int RQ>
 hipError_t launch(const TriattnFlashArgs& a, hipStream_t stream) {
-  static int cache[kMaxDevices];
-  int configured = 0;
-  hipError_t e = per_device(
-      cache,
-      [&](int, int* v) {
-        *v = 1;
-        return hipFuncSetAttribute(reinterpret_cast<const void*>(&triattn_flash_kernel<D, QW>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (lds_bytes<D, QW>()));
-      },
-      &configured);
+  constexpr int kLds = lds_bytes<D, QW, RQ>();
+  const hipError_t e = allow_dynamic_lds<triattn_flash_kernel<D, QW, RQ>>(kLds);
   if (e != hipSuccess) return e;
-  const int n_qc = (a.N + kQW * QW - 1) / (kQW * QW), n_rg = (a.N + kRows - 1) / kRows;
+  const int n_qc = (a.N + 32 * RQ * QW - 1) / (32 * RQ * QW), n_rg = (a.N + kRows - 1) / kRows;
   const long total = (long)n_qc * n_rg * a.B * a.H;
   const int per_xcd = (int)((total + 7) / 8);
-  constexpr int kLds = lds_bytes<D, QW>();
-  triattn_flash_kernel<D, QW><<<dim3(per_xcd * 8), dim3(64 * kRows * QW), kLds, stream>>>(a, n_qc, n_rg, (int)total,
-                                                                                          per_xcd);
+  triattn_flash_kernel<D, QW, RQ><<<dim3(per_xcd * 8), dim3(64 * kRows * QW), kLds, stream>>>(a, n_qc, n_rg, (int)total, per_xcd);
   return hipGetLastError();
 }
 
@@ -492,9 +492,24 @@ hipError_t launch(const TriattnFlashArgs& a, hipStream_t stream) {
 
 hipError_t triattn_flash_launch(const TriattnFlashArgs& args, int D, hipStream_t stream) {
   if (args.H != 4) return hipErrorInvalidValue;
-  const bool wide = args.N >= OF3_FLASH_WIDE_FROM;
-  if (D == 32) return wide ? launch<32, 4>(args, stream) : launch<32, 2>(args, stream);
-  if (D == 16) return wide ? launch<16, 4>(args, stream) : launch<16, 2>(args, stream);
+  static int cache[kMaxDevices];
+  int cus = 0;
+  const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  if (e != hipSuccess) return e;
+  // work-groups that launches of 128 queries each have
+  const long ranges = (args.N + 127) / 128, wide = ranges * ((args.N + kRows - 1) / kRows) * args.B * args.H;
+  if (D == 32) {
+    // Head width 32, 64 against 128 queries, us (256 CUs): N = 128 6.3 / 8.0, 160 9.0 / 12.7, 192 13.1 / 15.3, 300 32 / 39, 384 53 / 58,
+    // 450 94 / 96, 512 115 / 114, 768 365 / 343, 1280 1652 / 1544: up to three rounds of the latter.  Not where those are
+    // between one and two per CU and nearly full (N = 200 16.9 / 16.6, 230 19.2 / 18.6, 256 20.6 / 19.9).
+    const bool full = wide > cus && wide <= 2L * cus && (args.N + 63) / 64 == 2 * ranges;
+    return wide <= 6L * cus && !full ? launch<32, 1, 2>(args, stream) : launch<32, 2, 2>(args, stream);
+  }
+  if (D == 16) {
+    // Head width 16, one wave per row: 64 / 128 queries, and 128 with two waves: 2 x 187 15.6 / 16.9 / 18.2, 3 x 256 38.8 / 40.2 / 41.6,
+    // 2 x 400 (28 % of the 128-query ranges empty) 92 / 105 / 112, 1 x 512 84.8 / 83.1 / 88.3, 4 x 512 370 / 339 / 367.
+    return wide >= 12L * cus && 128 * ranges * 100 <= 115L * args.N ? launch<16, 1, 4>(args, stream) : launch<16, 1, 2>(args, stream);
+  }
   return hipErrorInvalidValue;
 }
 

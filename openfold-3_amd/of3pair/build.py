@@ -56,7 +56,7 @@ HIPCC_FLAGS = [
 
 
 def _flags():
-    """The compiler flags, plus what OF3_HIPCC_EXTRA adds (e.g. -DOF3_FLASH_WIDE_FROM=1 to run the tests on a
+    """The compiler flags, plus what OF3_HIPCC_EXTRA adds (e.g. -DOF3_TP_WAVES=16 to run the tests on a
     kernel variant that the default thresholds would not pick at the tests' sizes)."""
     return HIPCC_FLAGS + os.environ.get("OF3_HIPCC_EXTRA", "").split()
 
