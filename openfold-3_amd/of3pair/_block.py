@@ -16,12 +16,15 @@ import ctypes
 import math
 import operator
 import weakref
+from array import array as _array
 
 import torch
 from torch.nn.modules import module as _nn_module
 
 from . import _lib, layers
 from . import functional as F3
+
+_scan = _lib.load_scan()
 
 _TRI_MUL = ("linear_a_p", "linear_a_g", "linear_b_p", "linear_b_g")
 _NORM = (torch.nn.LayerNorm,)
@@ -78,7 +81,8 @@ class _Params:
         self.own = []      # (attributes of such a module, a name it may not have of its own)
         self.attrs = []    # (attributes of a module, name, the value that a call uses)
         self.noted = []    # the same of values that the search alone looks at
-        self.last = (None, None, None)  # pointers of refs, dtype and pointer array of the last call
+        self.last = (b"", None, None)  # pointers of refs, dtype and pointer array of the last call
+        self.lists = None  # refs as _native.scan takes them
 
     def link(self, owner, name, held):
         self.owners.append(owner)
@@ -171,17 +175,16 @@ class _Params:
 
     def gather(self, dtype):
         """The pointer array, or None when a parameter is not a plain contiguous tensor of `dtype`."""
-        ptrs = []
-        for owner, name, count in self.refs:
-            p = owner.get(name)
-            if p is None:
-                ptrs.append(0)
-            elif p.numel() == count and p.dtype is dtype and p.is_contiguous():
-                ptrs.append(p.data_ptr())
-            else:
-                return None
-        seen_ptrs, seen_dtype, array = self.last
-        if seen_ptrs != ptrs or seen_dtype is not dtype:
+        seen, seen_dtype, array = self.last
+        if self.lists is None:
+            self.lists = ([ref[0] for ref in self.refs], [ref[1] for ref in self.refs], _array("q", [ref[2] for ref in self.refs]))
+        found = _scan(*self.lists, dtype, seen) if _scan is not None else None
+        if found is None:
+            found = self._scan_in_python(dtype)
+        if found is False:
+            return None
+        if (found is not True and found != seen) or seen_dtype is not dtype:
+            ptrs = _array("Q", seen if found is True else found)
             for (owner, name, _), (shape, optional) in zip(self.refs, self.shapes):
                 p = owner.get(name)
                 if not optional if p is None else p.shape != shape:
@@ -189,8 +192,21 @@ class _Params:
             size = dtype.itemsize
             at = [ptrs[ref] + (row * self.shapes[ref][0][1] * size if row else 0) or None for ref, row in self.entries]
             array = (ctypes.c_void_p * len(at))(*at)
-            self.last = (ptrs, dtype, array)
+            self.last = (ptrs.tobytes(), dtype, array)
         return array
+
+    def _scan_in_python(self, dtype):
+        """What csrc/host_params.cpp does, for parameters of other types and where it is not built."""
+        ptrs = _array("Q")
+        for owner, name, count in self.refs:
+            p = owner.get(name)
+            if p is None:
+                ptrs.append(0)
+            elif p.numel() == count and p.dtype is dtype and p.is_contiguous():
+                ptrs.append(p.data_ptr())
+            else:
+                return False
+        return ptrs.tobytes()
 
 
 def _pair_params(q, block):

@@ -6,6 +6,7 @@ status, the caller gets an exception.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 
@@ -96,6 +97,19 @@ def load() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+def load_scan():
+    """csrc/host_params.cpp's scan, or None where it is not built or was built for another torch."""
+    if not os.path.exists(_build.HOST_PATH):
+        return None
+    spec = importlib.util.spec_from_file_location("_of3host", _build.HOST_PATH)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except ImportError:
+        return None
+    return module.scan
 
 
 def strides3(values):

@@ -45,6 +45,10 @@ SOURCES = [
     "single_x3_f32.hip",
 ]
 
+# host code against torch's headers, a Python extension of its own (the library above has a plain C interface)
+HOST_SOURCE = "host_params.cpp"
+HOST_PATH = os.path.join(LIB_DIR, "_of3host.so")
+
 # packed fp32 VALU ops are disabled on purpose (device code only)
 HIPCC_FLAGS = [
     "-O3",
@@ -78,7 +82,7 @@ def source_digest() -> str:
     """sha256 over everything the library is compiled from: the kernel sources and headers, the public
     header and the compiler flags."""
     h = hashlib.sha256(" ".join(_flags()).encode())
-    files = [os.path.join(CSRC, f) for f in SOURCES]
+    files = [os.path.join(CSRC, f) for f in SOURCES + [HOST_SOURCE]]
     files += [os.path.join(CSRC, f) for f in sorted(os.listdir(CSRC)) if f.endswith(".h")]
     if os.path.isdir(INCLUDE_DIR):
         files += [os.path.join(INCLUDE_DIR, f) for f in sorted(os.listdir(INCLUDE_DIR)) if f.endswith(".h")]
@@ -87,6 +91,20 @@ def source_digest() -> str:
         with open(path, "rb") as fh:
             h.update(fh.read())
     return h.hexdigest()
+
+
+def _build_host():
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+           *["-isystem" + d for d in cpp_extension.include_paths()], "-I" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, HOST_SOURCE), "-o", HOST_PATH,
+           *["-L" + d for d in cpp_extension.library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    _run(cmd)
 
 
 def build(verbose: bool = False, jobs: int = 4) -> str:
@@ -104,7 +122,9 @@ def build(verbose: bool = False, jobs: int = 4) -> str:
         return obj
 
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_build_host)
         objs = list(ex.map(compile_one, SOURCES))
+        host.result()
     _run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs])
     with open(STAMP_PATH, "w") as fh:
         fh.write(digest + "\n")
