@@ -169,6 +169,11 @@ __device__ __forceinline__ void wait_vmcnt() {  // vmcnt(N) only (gfx9 encoding,
   static_assert(N >= 0 && N < 16, "low field only");
   __builtin_amdgcn_s_waitcnt(0x0F70 | N);
 }
+// what this wave asked of LDS has arrived: nothing of it is read after the next barrier
+__device__ __forceinline__ void wait_lds_reads() {
+  compiler_fence();
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0) only
+}
 
 // XCD-aware block index: hardware deals consecutive workgroup ids round-robin to the 8
 // XCDs; this returns a logical id such that ids [x*per, (x+1)*per) all run on XCD x, so

@@ -722,19 +722,30 @@ __global__ __launch_bounds__(kThreads * PT) void trimul_proj_x3_f32(TrimulF32 p,
 }
 
 // Contraction on split operands: x[b][c][i][j] = sum_k a[b][c][i][k] b[b][c][j][k] in fp32, six bf16
-// products per k-step.  Work-group = 8 waves (4 x 2) = a 256 x 128 tile of one channel, a wave owns
-// 64 x 64 (2 x 2 MFMA tiles).  Per 32-wide k-panel the three terms of the tile's a rows and b rows
-// travel global -> LDS with direct-to-LDS buffer loads, one panel ahead, into double buffers; one
-// vmcnt(0) + barrier per panel.  A row of a panel is 64 bytes = 4 chunks of 16 bytes; chunk c of row
+// products per k-step.  Work-group = WM x 2 waves = one tile of one channel, a wave owns T x T MFMA tiles of 32 x 32.
+// Per 32-wide k-panel the three terms of the tile's a rows and b rows
+// travel global -> LDS with direct-to-LDS buffer loads.  A row of a panel is 64 bytes = 4 chunks of 16 bytes; chunk c of row
 // r is stored at position c ^ ((r >> 2) & 3), so that the 8 lanes of an operand read (8 rows, same
-// chunk) fall into different banks; the swizzle is applied on the global side.
-constexpr int kCtM = 256, kCtN = 128;
-constexpr int kCtASlots = kCtM * 4, kCtBSlots = kCtN * 4;      // per term and stage, in 16-byte slots
-constexpr int kCtStage = 3 * (kCtASlots + kCtBSlots);
-constexpr size_t kContractX3Lds = (size_t)2 * kCtStage * 16;
+// chunk) fall into different banks; the swizzle is applied on the global side.  Parts of a tile past the last panel row are
+// neither loaded nor multiplied.
+// The matrix pipes bound it from 300 tokens on (1.25 PFLOP/s of bf16 products at N = 768), the 12 bytes per element of a and b
+// around 200 (4 TB/s), one work-group's chain load -> products -> store below that.  Four forms, summing in the same order:
+//   <4, 2, 2>  256 x 128, two stages of LDS, alone on its CU: the next panel's loads run beside a panel's products.
+//   <4, 2, 1>  256 x 128, one stage (72 KB), two work-groups on a CU.
+//   <2, 2, 1>  128 x 128, one stage (48 KB): three work-groups on a CU, one's products beside another's loads, first panel and stores.
+//   <2, 1, 1>  64 x 64, one stage (24 KB).
+template <int WM, int T, int STAGES>
+struct CtX3 {
+  static constexpr int kWaves = 2 * WM, kM = 32 * T * WM, kN = 64 * T;
+  static constexpr int kA = kM * 4, kB = kN * 4;  // per term and stage, in 16-byte slots
+  static constexpr int kStage = 3 * (kA + kB);
+  static constexpr size_t kLds = (size_t)STAGES * kStage * 16;
+  static constexpr int kAI = kM / 16 / kWaves, kBI = kN / 16 / kWaves;  // loads of a wave per term, 16 rows each
+};
 
-__global__ __launch_bounds__(512) void trimul_contract_x3_f32(TrimulF32 p, int tiles_m, int tiles_n, int total,
-                                                               int per_xcd) {
+template <int WM, int T, int STAGES>
+__global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, int tiles_m, int tiles_n, int total, int per_xcd) {
+  typedef CtX3<WM, T, STAGES> K;
   extern __shared__ u32x4_t lds4[];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -744,7 +755,7 @@ __global__ __launch_bounds__(512) void trimul_contract_x3_f32(TrimulF32 p, int t
   const int logical = xcd_logical_block(blockIdx.x, per_xcd);
   if (logical >= total) return;  // the whole work-group leaves together
   const int tn = logical % tiles_n, tm = (logical / tiles_n) % tiles_m, bc = logical / (tiles_n * tiles_m);
-  const int i0 = tm * kCtM, j0 = tn * kCtN;
+  const int i0 = tm * K::kM, j0 = tn * K::kN;
   const size_t chan = (size_t)Np * Np;
   // one descriptor per term and side over the channel's plane
   __amdgpu_buffer_rsrc_t a_rsrc[3], b_rsrc[3];
@@ -753,57 +764,62 @@ __global__ __launch_bounds__(512) void trimul_contract_x3_f32(TrimulF32 p, int t
     a_rsrc[pl] = buffer_rsrc(p.as + pl * p.ab_plane + bc * chan, chan * sizeof(bf16_t));
     b_rsrc[pl] = buffer_rsrc(p.bs + pl * p.ab_plane + bc * chan, chan * sizeof(bf16_t));
   }
-  // slot t of a stage's a (b) part holds chunk (t & 3) ^ ((row >> 2) & 3) of tile row t >> 2; wave w
-  // fills a slots 128 w .. + 127 (two instructions) and b slots 64 w .. + 63 of each term
-  uint32_t a_off[2], b_off;
+  // slot t of a term's a (b) part holds chunk (t & 3) ^ ((row >> 2) & 3) of tile row t >> 2; wave w fills the a rows
+  // 16 kAI w .. and the b rows 16 kBI w ..
+  uint32_t a_off[2], b_off[2];  // kAI and kBI of them (of constant size: the compiler's host side loses the kernel otherwise)
+  static_assert(K::kAI >= 1 && K::kAI <= 2 && K::kBI >= 1 && K::kBI <= 2, "");
   const int rot = panel_rotation(bc % p.CH, Np);
-  auto rotated = [&](int r) { return panel_row(r < Np ? r : Np - 1, rot, Np); };  // rows past the end: computed, not stored
+  auto offset = [&](int first, int t) {
+    const int row = t >> 2, c = (t & 3) ^ ((row >> 2) & 3), r = first + row;
+    return (uint32_t)((panel_row(r < Np ? r : Np - 1, rot, Np) * 32 + 8 * c) * sizeof(bf16_t));
+  };
 #pragma unroll
-  for (int n = 0; n < 2; ++n) {
-    const int t = 128 * wave + 64 * n + lane, row = t >> 2, c = (t & 3) ^ ((row >> 2) & 3);
-    a_off[n] = (uint32_t)((rotated(i0 + row) * 32 + 8 * c) * sizeof(bf16_t));
-  }
-  {
-    const int t = 64 * wave + lane, row = t >> 2, c = (t & 3) ^ ((row >> 2) & 3);
-    b_off = (uint32_t)((rotated(j0 + row) * 32 + 8 * c) * sizeof(bf16_t));
-  }
+  for (int n = 0; n < K::kAI; ++n) a_off[n] = offset(i0, 64 * (K::kAI * wave + n) + lane);
+#pragma unroll
+  for (int n = 0; n < K::kBI; ++n) b_off[n] = offset(j0, 64 * (K::kBI * wave + n) + lane);
   auto issue_loads = [&](int panel, int buf) {  // buf is a constant at every call site
-    u32x4_t* st = lds4 + buf * kCtStage;
+    u32x4_t* st = lds4 + buf * K::kStage;
     const int soff = panel * Np * 32 * (int)sizeof(bf16_t);
 #pragma unroll
     for (int pl = 0; pl < 3; ++pl) {
 #pragma unroll
-      for (int n = 0; n < 2; ++n)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc[pl], (void OF3_LDS_AS*)(st + pl * kCtASlots + 128 * wave + 64 * n), 16,
-                                                 a_off[n], soff, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc[pl], (void OF3_LDS_AS*)(st + 3 * kCtASlots + pl * kCtBSlots + 64 * wave),
-                                               16, b_off, soff, 0, 0);
+      for (int n = 0; n < K::kAI; ++n)
+        if (i0 + 16 * (K::kAI * wave + n) < Np)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc[pl], (void OF3_LDS_AS*)(st + pl * K::kA + 64 * (K::kAI * wave + n)), 16,
+                                                   a_off[n], soff, 0, 0);
+#pragma unroll
+      for (int n = 0; n < K::kBI; ++n)
+        if (j0 + 16 * (K::kBI * wave + n) < Np)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc[pl],
+                                                   (void OF3_LDS_AS*)(st + 3 * K::kA + pl * K::kB + 64 * (K::kBI * wave + n)), 16,
+                                                   b_off[n], soff, 0, 0);
     }
   };
-  f32x16_t acc[2][2];
+  const int im = i0 + 32 * T * wm, jn = j0 + 32 * T * wn;  // this wave's part of the tile
+  const bool busy = im < N && jn < N;
+  f32x16_t acc[T][T];
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
+  for (int mi = 0; mi < T; ++mi)
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = zero16();
+    for (int ni = 0; ni < T; ++ni) acc[mi][ni] = zero16();
   const int key = (l32 >> 2) & 3;
   auto panel_products = [&](int buf) {
-    const u32x4_t* sa = lds4 + buf * kCtStage + (64 * wm + l32) * 4;
-    const u32x4_t* sb = lds4 + buf * kCtStage + 3 * kCtASlots + (64 * wn + l32) * 4;
+    const u32x4_t* sa = lds4 + buf * K::kStage + (32 * T * wm + l32) * 4;
+    const u32x4_t* sb = lds4 + buf * K::kStage + 3 * K::kA + (32 * T * wn + l32) * 4;
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       const int c = (2 * st + lh) ^ key;
-      u32x4_t ao[2][3], bo[2][3];
+      u32x4_t ao[T][3], bo[T][3];
 #pragma unroll
-      for (int pl = 0; pl < 3; ++pl) {
+      for (int pl = 0; pl < 3; ++pl)
 #pragma unroll
-        for (int mi = 0; mi < 2; ++mi) ao[mi][pl] = sa[pl * kCtASlots + mi * 128 + c];
+        for (int n = 0; n < T; ++n) ao[n][pl] = sa[pl * K::kA + n * 128 + c], bo[n][pl] = sb[pl * K::kB + n * 128 + c];
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni) bo[ni][pl] = sb[pl * kCtBSlots + ni * 128 + c];
-      }
+      for (int mi = 0; mi < T; ++mi)
 #pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {  // smallest terms first
+        for (int ni = 0; ni < T; ++ni) {
+          if ((mi > 0 && im + 32 * mi >= N) || (ni > 0 && jn + 32 * ni >= N)) continue;
+          // smallest terms first
           acc[mi][ni] = mfma_32x32x16(ao[mi][2], bo[ni][0], acc[mi][ni]);
           acc[mi][ni] = mfma_32x32x16(ao[mi][0], bo[ni][2], acc[mi][ni]);
           acc[mi][ni] = mfma_32x32x16(ao[mi][1], bo[ni][1], acc[mi][ni]);
@@ -816,25 +832,36 @@ __global__ __launch_bounds__(512) void trimul_contract_x3_f32(TrimulF32 p, int t
   issue_loads(0, 0);
   auto step = [&](int panel, int buf) {
     wait_vmcnt<0>();               // this wave's loads of the panel have landed ...
-    __builtin_amdgcn_s_barrier();  // ... and everybody's; nobody reads the previous panel's buffers any more
+    wait_lds_reads();
+    __builtin_amdgcn_s_barrier();  // ... and everybody's; nobody reads the other stage any more
     compiler_fence();
-    issue_loads(panel + 1 < panels ? panel + 1 : panels - 1, buf ^ 1);
-    panel_products(buf);
+    if (STAGES == 2) issue_loads(panel + 1 < panels ? panel + 1 : panels - 1, buf ^ 1);
+    if (busy) panel_products(buf);
     compiler_fence();
+    if (STAGES == 1 && panel + 1 < panels) {
+      wait_lds_reads();
+      __builtin_amdgcn_s_barrier();  // everybody has read the panel: its operands are in registers
+      compiler_fence();
+      issue_loads(panel + 1, 0);
+    }
   };
-  for (int panel = 0; panel < panels; panel += 2) {
-    step(panel, 0);
-    if (panel + 1 < panels) step(panel + 1, 1);
+  if (STAGES == 2) {
+    for (int panel = 0; panel < panels; panel += 2) {
+      step(panel, 0);
+      if (panel + 1 < panels) step(panel + 1, 1);
+    }
+    wait_vmcnt<0>();  // the loads issued past the end must not outlive the work-group's LDS
+  } else {
+    for (int panel = 0; panel < panels; ++panel) step(panel, 0);
   }
-  wait_vmcnt<0>();  // the loads issued past the end must not outlive the work-group's LDS
 
   float* xc = p.x + (size_t)bc * N * N;
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
+  for (int mi = 0; mi < T; ++mi)
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni) {
-      const int ib = i0 + 64 * wm + 32 * mi, j = j0 + 64 * wn + 32 * ni + l32;
-      if (ib + 32 <= N && j0 + 64 * wn + 32 * ni + 32 <= N) {
+    for (int ni = 0; ni < T; ++ni) {
+      const int ib = im + 32 * mi, j = jn + 32 * ni + l32;
+      if (ib + 32 <= N && jn + 32 * ni + 32 <= N) {
         float* lp = xc + (size_t)(ib + 4 * lh) * N + j;
 #pragma unroll
         for (int v = 0; v < 16; ++v) lp[(size_t)(8 * (v >> 2) + (v & 3)) * N] = acc[mi][ni][v];
@@ -846,6 +873,44 @@ __global__ __launch_bounds__(512) void trimul_contract_x3_f32(TrimulF32 p, int t
         }
       }
     }
+}
+
+template <int WM, int T, int STAGES>
+hipError_t launch_contract_x3(const TrimulF32& p, int cus, hipStream_t stream) {
+  typedef CtX3<WM, T, STAGES> K;
+  constexpr size_t kAlone = 100 * 1024;  // more than half of a CU's
+  const hipError_t e = allow_dynamic_lds<trimul_contract_x3_f32<WM, T, STAGES>>(K::kLds > kAlone ? K::kLds : kAlone);
+  if (e != hipSuccess) return e;
+  const int tiles_m = (p.N + K::kM - 1) / K::kM, tiles_n = (p.N + K::kN - 1) / K::kN;
+  const long total = (long)p.B * p.CH * tiles_m * tiles_n;
+  if (total > 0x7fffffffL - 8) return hipErrorInvalidValue;
+  const int per_xcd = (int)((total + 7) / 8);
+  // No more tiles than CUs: LDS enough for one work-group per CU, or the scheduler puts several on one beside another stream's
+  // kernels (four blocks with their single representations on a second stream, 64 / 48 / 30 tokens: 639 / 628 / 577 us, so
+  // 614 / 601 / 556).
+  const size_t lds = total <= cus && K::kLds < kAlone ? kAlone : K::kLds;
+  hipLaunchKernelGGL((trimul_contract_x3_f32<WM, T, STAGES>), dim3(per_xcd * 8), dim3(128 * WM), lds, stream, p, tiles_m, tiles_n,
+                     (int)total, per_xcd);
+  return hipGetLastError();
+}
+
+// Whole passes, us, with tiles of 256 x 128 multiplied in full (all there was before) | 256 x 128 | 128 | 64:
+//   pair stack, 128 channels: N = 64 123 | 117 | 117 | 114, 128 191 | 186 | 189 | 183, 163 314 | 301 | 301 | 322, 200 426 | 418 | 416 | 436,
+//     256 549 | 544 | 546 | 562, 300 920 | 888 | 871 | 869, 384 1379 | 1361 | 1351 | 1374, 600 4093 | 3965 | 3938 | 4064
+//   templates of 64 channels (3 x 162, 3 x 200: 845, 1233 with one stage, which pays from two rounds on: 163 and 200 above 307, 429):
+//     4 x 64 260 | 252 | 254 | 247, 4 x 128 646 | 618 | 620 | 613, 3 x 162 888 | 853 | 870 | 900,
+//     3 x 200 1271 | 1247 | 1286 | 1273, 2 x 400 3903 | 3822 | 3818 | 3897, 4 x 512 12120 | 12129 | 12090 | 12401
+// Alone and with a and b in cache the smaller tiles do better yet (3 x 200: 30 us against 38); under power they move more
+// bytes into LDS per product and slow the kernels around them.
+hipError_t contract_x3_launch(const TrimulF32& p, hipStream_t stream) {
+  static int cache[kMaxDevices];
+  int cus = 0;
+  const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  if (e != hipSuccess) return e;
+  if (p.N <= 128) return launch_contract_x3<2, 1, 1>(p, cus, stream);
+  if (p.N > 256) return launch_contract_x3<2, 2, 1>(p, cus, stream);
+  // two tiles per channel
+  return 2l * p.B * p.CH <= cus ? launch_contract_x3<4, 2, 2>(p, cus, stream) : launch_contract_x3<4, 2, 1>(p, cus, stream);
 }
 
 // Output pass.  The gate is computed first and kept in registers, so that LayerNorm(x) can take the
@@ -2307,7 +2372,6 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
   const bool pass = split_ab && trimul_pass_serves(p);
   if (pass) {
     if (hipError_t ep = trimul_proj_pass_f32(p, stream); ep != hipSuccess) return ep;
-    if (hipError_t ep = allow_lds<trimul_contract_x3_f32>(kLdsLimit); ep != hipSuccess) return ep;
   } else if (x3) {
     auto proj = split_ab ? (fast ? trimul_proj_x3_f32<kXT, kPT, true, true> : trimul_proj_x3_f32<kXT, kPT, false, true>)
                          : (fast ? trimul_proj_x3_f32<kXT, kPT, true, false> : trimul_proj_x3_f32<kXT, kPT, false, false>);
@@ -2319,7 +2383,6 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
     if (e == hipSuccess) e = allow_lds<trimul_out_x3_f32<kXT, kPT, true, false>>(kLdsLimit);
     if (e == hipSuccess) e = allow_lds<trimul_out_x3_f32<kXT, kPT, false, true>>(kLdsLimit);
     if (e == hipSuccess) e = allow_lds<trimul_out_x3_f32<kXT, kPT, true, true>>(kLdsLimit);
-    if (e == hipSuccess) e = allow_lds<trimul_contract_x3_f32>(kLdsLimit);
     if (e != hipSuccess) return e;
     const size_t lds = tile_bytes_x3(a.C, 32 * kXT * kPT) + 32 * kXT * kPT * sizeof(float);
     const int kgroups = (a.N + 32 * kXT - 1) / (32 * kXT), row_groups = (a.N + kPT - 1) / kPT;
@@ -2336,12 +2399,7 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
   // the contraction has no shape or alignment condition of its own; the FMA kernel stays with the
   // FMA passes so that odd shapes run one family of kernels
   if (split_ab) {
-    const int tiles_m = (a.N + kCtM - 1) / kCtM, tiles_n = (a.N + kCtN - 1) / kCtN;
-    const long total = (long)a.B * a.CH * tiles_m * tiles_n;
-    if (total > 0x7fffffffL - 8) return hipErrorInvalidValue;
-    const int per_xcd = (int)((total + 7) / 8);
-    hipLaunchKernelGGL(trimul_contract_x3_f32, dim3(per_xcd * 8), dim3(512), kContractX3Lds, stream, p, tiles_m, tiles_n,
-                       (int)total, per_xcd);
+    if (hipError_t ec = contract_x3_launch(p, stream); ec != hipSuccess) return ec;
   } else if (mm || x3) {
     const unsigned t = (unsigned)((a.N + 127) / 128);
     hipLaunchKernelGGL(trimul_contract_mm_f32, dim3(t, t, (unsigned)(a.B * a.CH)), dim3(kThreads), 0, stream, p.a, p.b,
