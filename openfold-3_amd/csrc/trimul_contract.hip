@@ -61,9 +61,7 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | 0x70 | 0xF00 | ((N >> 4) << 14));
 }
 
-// TRANSPOSED: every plane of x is written as its transpose, for a reader that walks columns (pair_join_bf16.hip).  The products
-// take their operands the other way round: the same sums, with a lane's values along i.
-template <int BN, int kNS, bool TRANSPOSED>
+template <int BN, int kNS>
 __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restrict__ pm,  // j side planes (b)
                                                           const bf16_t* __restrict__ pn,  // i side planes (a)
                                                           bf16_t* __restrict__ x, int Np, int nk, int tiles_m,
@@ -183,12 +181,11 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
   for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
     for (int nt = 0; nt < TN; ++nt) acc[mt][nt] = zero16();
-  auto product = [&](u32x4_t af, u32x4_t bfr, f32x16_t c) { return TRANSPOSED ? mfma_32x32x16(bfr, af, c) : mfma_32x32x16(af, bfr, c); };
   auto mma = [&](const u32x4_t (&af)[TM], const u32x4_t (&bfr)[TN]) {
 #pragma unroll
     for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < TN; ++nt) acc[mt][nt] = product(af[mt], bfr[nt], acc[mt][nt]);
+      for (int nt = 0; nt < TN; ++nt) acc[mt][nt] = mfma_32x32x16(af[mt], bfr[nt], acc[mt][nt]);
   };
   // the same, with the refill's loads issued in between
   auto mma_and_issue = [&](const u32x4_t (&af)[TM], const u32x4_t (&bfr)[TN]) {
@@ -197,7 +194,7 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
     for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
       for (int nt = 0; nt < TN; ++nt) {
-        acc[mt][nt] = product(af[mt], bfr[nt], acc[mt][nt]);
+        acc[mt][nt] = mfma_32x32x16(af[mt], bfr[nt], acc[mt][nt]);
         if (n < IPW) issue_one(n++);
       }
     issue_advance();
@@ -228,7 +225,7 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
       // carries the wait for a0/b0 (with direct-to-LDS loads in flight every LDS wait the
       // compiler emits is a wait for all outstanding reads), so the new reads travel under the
       // remaining MFMAs instead of being waited for at once.
-      acc[0][0] = product(a0[0], b0[0], acc[0][0]);
+      acc[0][0] = mfma_32x32x16(a0[0], b0[0], acc[0][0]);
       __builtin_amdgcn_sched_barrier(0);
       fetch(cur, 1, a1, b1);
       __builtin_amdgcn_sched_barrier(0);
@@ -236,7 +233,7 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
       for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
         for (int nt = 0; nt < TN; ++nt)
-          if (mt + nt > 0) acc[mt][nt] = product(a0[mt], b0[nt], acc[mt][nt]);
+          if (mt + nt > 0) acc[mt][nt] = mfma_32x32x16(a0[mt], b0[nt], acc[mt][nt]);
       __builtin_amdgcn_sched_barrier(0);
 
       // This wave holds all of stage s in registers.  Stages s+1..s+3 are in flight and
@@ -271,41 +268,6 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
     u32x4_t* epi = lds + kNS * STAGE + wave * 512;
     const int jbase = tm * BM + wm0;
     int n_stores = 0;
-    if constexpr (TRANSPOSED) {
-      // 32 columns j at a time: staged as rows of WN i's (8-byte pieces: a lane holds runs of four), out as row segments
-      constexpr int CHR = WN / 8;
-      static_assert(CHR == 8 || CHR == 16, "the swizzle permutes chunks in groups of eight");
-      auto key = [](int row) { return row & 7; };
-      const int i0 = tn * BN + wn0, Nr = 32 * nk;
-      const bool whole = i0 + WN <= Nr && jbase + WM <= Nr;
-      u32x2_t* const epi2 = reinterpret_cast<u32x2_t*>(epi);
-#pragma unroll
-      for (int mt = 0; mt < TM; ++mt) {
-#pragma unroll
-        for (int nt = 0; nt < TN; ++nt) {
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {  // registers 4g..4g+3: i-local = 32*nt + 8*g + 4*lh + (0..3)
-            const u32x2_t v = {pack_bf16(acc[mt][nt][4 * g], acc[mt][nt][4 * g + 1]),
-                               pack_bf16(acc[mt][nt][4 * g + 2], acc[mt][nt][4 * g + 3])};
-            epi2[(l32 * CHR + ((4 * nt + g) ^ key(l32))) * 2 + lh] = v;
-          }
-          acc[mt][nt] = zero16();
-        }
-#pragma unroll
-        for (int rr = 0; rr < CHR / 2; ++rr) {
-          const int idx = 64 * rr + lane, row = idx / CHR, chunk = idx % CHR;
-          const u32x4_t v = epi[row * CHR + (chunk ^ key(row))];
-          // operand row `row` of the tile: j-local as in am_slot
-          const int j = jbase + 16 * TM * ((row >> 2) & 1) + 16 * mt + 4 * (row >> 3) + (row & 3), i = i0 + 8 * chunk;
-          if (whole || (j < Nr && i < Nr)) *reinterpret_cast<u32x4_t*>(xo + (size_t)j * Np + i) = v;
-        }
-        if (whole) n_stores += CHR / 2;
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      static_assert(TM * (CHR / 2) == 8 * TN, "as many stores as the other form");
-      stores_pending = n_stores == 8 * TN;
-      continue;
-    }
 #pragma unroll
     for (int nt = 0; nt < TN; ++nt) {
 #pragma unroll
@@ -351,10 +313,10 @@ __global__ __launch_bounds__(256, 1) void contract_kernel(const bf16_t* __restri
   wait_vmcnt<0>();  // loads issued past the end must not outlive the work-group's LDS
 }
 
-template <int BN, int kNS, bool TRANSPOSED>
+template <int BN, int kNS>
 hipError_t launch_contract(const bf16_t* a, const bf16_t* b, bf16_t* x, int planes, int Np, int nk, hipStream_t stream) {
   constexpr int BM = 256;
-  auto kern = contract_kernel<BN, kNS, TRANSPOSED>;
+  auto kern = contract_kernel<BN, kNS>;
   const size_t smem = ((size_t)kNS * (BM + BN) * 4 + 4 * 512) * sizeof(u32x4_t);  // ring + epilogue staging
   static int cache[kMaxDevices];
   int cus = 0;
@@ -629,25 +591,139 @@ hipError_t launch_contract8(const bf16_t* a, const bf16_t* b, bf16_t* x, int pla
   return hipGetLastError();
 }
 
+// ---- up to 256 tokens -------------------------------------------------------------------------------------
+// A round or two of work-groups, so what bounds it is one work-group's chain: first panel from L2, products, stores.  Tiles of
+// 64 x 64 of one plane, four waves of 32 x 32 each, five work-groups to a CU: one's stores run beside another's loads.  A ring of
+// four panels (32 KB of LDS), three of them requested ahead, one barrier per panel: behind it everybody has read the panel
+// before, whose place the next request takes.
+// `pm` holds the operand along the rows of the output in memory, `pn` the other: x[n][m] = sum_k pm[m][k] pn[n][k], so
+// the transposed planes, for a reader that walks columns (pair_join_bf16.hip), are the operands' roles exchanged (M_IS_I).  The
+// panels are visited in the order of contract_kernel's tiles (its sums, bit for bit).
+// Whole passes, us, with contract_kernel / this: pair stack 60 tokens 62 / 56, 110 91 / 87; pairformer, 4 blocks, 40 364 / 343, 85 434 / 412,
+// 150 646 / 626, 190 780 / 754, 225 1019 / 1011; templates 4 x 60 154 / 150, 4 x 120 257 / 248, 3 x 187 406 / 389.  With tiles of 128:
+// 59, 90, 394, 426, 637, 773, 1023, 153, 252, 407.
+constexpr int kShortTile = 64, kShortRing = 4;
+constexpr int kShortSide = kShortTile * 4;  // u32x4 slots of one side of a panel
+constexpr size_t kShortLds = (size_t)kShortRing * 2 * kShortSide * 16;
+
+template <bool M_IS_I>
+__global__ __launch_bounds__(256) void contract_short_kernel(const bf16_t* __restrict__ pm, const bf16_t* __restrict__ pn,
+                                                             bf16_t* __restrict__ x, int Np, int nk, int bn_order, int tiles, int total,
+                                                             int per_xcd) {
+  extern __shared__ u32x4_t lds[];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
+  const int logical = xcd_logical_block(blockIdx.x, per_xcd);
+  if (logical >= total) return;  // the whole work-group leaves together
+  const int plane = logical / (tiles * tiles), rem = logical - plane * (tiles * tiles);
+  const int tn = rem / tiles, tm = rem - tn * tiles;
+  const int m0 = tm * kShortTile, n0 = tn * kShortTile, Nr = 32 * nk;
+  const int wm0 = 32 * (wave >> 1), wn0 = 32 * (wave & 1);
+  const size_t plane_bytes = (size_t)plane * Np * Np * 2, panel_bytes = (size_t)Np * kBK * 2;
+  // The m side's rows are read in the order 0..3, 16..19, 4..7, 20..23, ...: a lane ends with 16 consecutive m's of one n.
+  // (row % 4, key) differs within each group of 16 lanes, there and in the n side's natural order.
+  auto m_key = [](int row) { return ((row >> 2) & 1) | (((row >> 4) & 1) << 1); };
+  auto n_key = [](int row) { return (row >> 2) & 3; };
+
+  // this wave's loads, 16 rows of each side: lane l fills slot l, row l / 4, with chunk (l % 4) ^ key(row)
+  const int rb = 16 * wave, within = lane >> 2, row = rb + within;
+  const char* src_m = reinterpret_cast<const char*>(pm) + plane_bytes + (size_t)(contract_rows_first(m0, rb, Nr) + within) * 64 +
+                      16 * ((lane & 3) ^ m_key(row));
+  const char* src_n = reinterpret_cast<const char*>(pn) + plane_bytes + (size_t)(contract_rows_first(n0, rb, Nr) + within) * 64 +
+                      16 * ((lane & 3) ^ n_key(row));
+  // the panel that contract_kernel begins this output with: tiles of 256 j's and bn_order i's
+  int next = (M_IS_I ? m0 / bn_order + n0 / 256 : n0 / bn_order + m0 / 256) % 4 % nk;
+  auto issue = [&](int buf) {
+    u32x4_t* st = lds + buf * (2 * kShortSide) + 64 * wave;
+    const size_t at = next * panel_bytes;
+    __builtin_amdgcn_global_load_lds((const void OF3_GLOBAL_AS*)(src_m + at), (void OF3_LDS_AS*)st, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((const void OF3_GLOBAL_AS*)(src_n + at), (void OF3_LDS_AS*)(st + kShortSide), 16, 0, 0);
+    next = next + 1 == nk ? 0 : next + 1;
+  };
+
+  const int mr = wm0 + 16 * ((l32 >> 2) & 1) + 4 * (l32 >> 3) + (l32 & 3), nr = wn0 + l32;
+  const int m_slot = mr * 4 + (lh ^ m_key(mr)), n_slot = kShortSide + nr * 4 + (lh ^ n_key(nr));
+  f32x16_t acc = zero16();
+  const bool busy = m0 + wm0 < Nr && n0 + wn0 < Nr;
+  const int ahead = nk < kShortRing - 1 ? nk : kShortRing - 1;
+  for (int q = 0; q < ahead; ++q) issue(q);
+  for (int p = 0; p < nk; ++p) {
+    const int newer = nk - 1 - p;  // panels requested after this one: up to two, two loads each
+    if (newer >= 2) wait_vmcnt<4>();
+    else if (newer == 1) wait_vmcnt<2>();
+    else wait_vmcnt<0>();
+    wait_lds_reads();  // of the panel before
+    __builtin_amdgcn_s_barrier();
+    compiler_fence();
+    const u32x4_t* st = lds + p % kShortRing * (2 * kShortSide);
+    if (p + 3 < nk) issue((p + 3) % kShortRing);
+    if (!busy) continue;
+    const u32x4_t a0 = st[m_slot], b0 = st[n_slot], a1 = st[m_slot ^ 2], b1 = st[n_slot ^ 2];
+    acc = mfma_32x32x16(a0, b0, acc);
+    acc = mfma_32x32x16(a1, b1, acc);
+  }
+  wait_lds_reads();
+  __builtin_amdgcn_s_barrier();  // everybody has read the last panel
+  compiler_fence();
+
+  // through LDS, the wave's own 32 rows of four chunks, so that a store writes 64 consecutive bytes of a row
+  u32x4_t* epi = lds + wave * 128;
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    u32x4_t v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = pack_bf16(acc[8 * hf + 2 * q], acc[8 * hf + 2 * q + 1]);
+    epi[l32 * 4 + ((2 * lh + hf) ^ (l32 & 3))] = v;
+  }
+  bf16_t* xo = x + (size_t)plane * Np * Np;
+#pragma unroll
+  for (int rr = 0; rr < 2; ++rr) {
+    const int idx = 64 * rr + lane, r = idx >> 2, chunk = idx & 3;
+    const u32x4_t v = epi[r * 4 + (chunk ^ (r & 3))];
+    const int n = n0 + wn0 + r, m = m0 + wm0 + 8 * chunk;
+    if (n < Nr && m < Nr) *reinterpret_cast<u32x4_t*>(xo + (size_t)n * Np + m) = v;
+  }
+}
+
+hipError_t launch_contract_short(const bf16_t* a, const bf16_t* b, bf16_t* x, int planes, int Np, int nk, int bn_order, bool transposed,
+                                 hipStream_t stream) {
+  const int tiles = (32 * nk + kShortTile - 1) / kShortTile, total = planes * tiles * tiles, per_xcd = (total + 7) / 8;
+  if (transposed)
+    hipLaunchKernelGGL(contract_short_kernel<true>, dim3(per_xcd * 8), dim3(256), kShortLds, stream, a, b, x, Np, nk, bn_order, tiles,
+                       total, per_xcd);
+  else
+    hipLaunchKernelGGL(contract_short_kernel<false>, dim3(per_xcd * 8), dim3(256), kShortLds, stream, b, a, x, Np, nk, bn_order, tiles,
+                       total, per_xcd);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t trimul_contract_launch(const bf16_t* a, const bf16_t* b, bf16_t* x, int planes, int Np, int nk, int variant,
                                   bool transposed, hipStream_t stream) {
   if (nk < 1 || nk > Np / kBK) return hipErrorInvalidValue;
-  switch (transposed ? variant + 8 : variant) {
+  if ((variant == 2 || variant == 3) && Np <= 256) {
+    static int cache[kMaxDevices];
+    int cus = 0;
+    const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+    if (e != hipSuccess) return e;
+    // Above 192 tokens only while the 256-wide tiles are one round: 4 blocks at 225 / 256 tokens, 128 planes, 1019 / 1049 us with those,
+    // 1011 / 1044 with these; 256 planes, 4 x 256 templates, 747 and 762.
+    if (transposed || nk <= 6 || 2l * planes <= cus)
+      return launch_contract_short(a, b, x, planes, Np, nk, variant == 2 ? 128 : 256, transposed, stream);
+  }
+  if (transposed) return hipErrorInvalidValue;  // the larger tiles have no such form
+  switch (variant) {
     case 1:
-      return launch_contract<192, 4, false>(a, b, x, planes, Np, nk, stream);
+      return launch_contract<192, 4>(a, b, x, planes, Np, nk, stream);
     case 2:
-      return launch_contract<128, 4, false>(a, b, x, planes, Np, nk, stream);
+      return launch_contract<128, 4>(a, b, x, planes, Np, nk, stream);
     case 3:
-      return launch_contract<256, 4, false>(a, b, x, planes, Np, nk, stream);
+      return launch_contract<256, 4>(a, b, x, planes, Np, nk, stream);
     case 4:
       return launch_contract8<3>(a, b, x, planes, Np, nk, stream);
-    case 10:
-      return launch_contract<128, 4, true>(a, b, x, planes, Np, nk, stream);
-    case 11:
-      return launch_contract<256, 4, true>(a, b, x, planes, Np, nk, stream);
-    default:  // 192-wide tiles have no transposed form: up to 256 tokens they are never the choice
+    default:
       return hipErrorInvalidValue;
   }
 }
