@@ -338,21 +338,26 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
 // Wave = one 32-channel tile of q, k or v (12 waves at 128 channels, three per SIMD).  Tile = one 32-position panel;
 // double buffered, one barrier per tile (three panels per barrier: 417 against 385 us at N = 768).  The H rows of the
 // triangle bias are dot products taken on the normalised rows while they are in registers.
+// PARTS work-groups share a tile, each with every output tile's PARTS-th and as many of the bias rows, where there are CUs left:
+// what bounds a launch of one tile per CU is the 288 KB of weights through the CU's L1 (3 us) and the products of three waves
+// per SIMD.
 template <int C>
 struct AttProjLds {
   static constexpr size_t kBytes = (size_t)2 * PassTile<C>::SLOTS * 16 + (2 * C + 8 * C) * sizeof(float);
 };
 
-template <int C>
-__global__ __launch_bounds__(6 * C) void triattn_proj_pass(TriattnF32 p, int panels, int total) {
+template <int C, int PARTS>
+__global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p, int panels, int total) {
   typedef PassTile<C> Tile;
-  constexpr int OT = C / 32, NW = 3 * OT, KS = C / 16, TASKS = (8 + NW - 1) / NW;
+  constexpr int OT = C / 32 / PARTS, NW = 3 * OT, KS = C / 16, TASKS = (8 + NW - 1) / NW;
   extern __shared__ u32x4_t lds[];
   float* ln = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS);  // [2][C]
   float* wb = ln + 2 * C;                                       // [H][C], H <= 8
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int N = p.N, H = p.H, kind = wave / OT, ot = wave % OT;
+  const int slot = grid_slot(), part = slot % PARTS;
+  const int N = p.N, H = p.H, kind = wave / OT, ot = part * OT + wave % OT;
+  const int h0 = H * part / PARTS, h1 = H * (part + 1) / PARTS;  // this work-group's heads of the bias
   const bool narrow = p.D == 16;
   for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c], ln[C + c] = p.ln_b[c];
   for (int c = tid; c < H * C; c += 64 * NW) wb[c] = p.w_b[c];
@@ -413,9 +418,10 @@ __global__ __launch_bounds__(6 * C) void triattn_proj_pass(TriattnF32 p, int pan
     d4[2 * plane8] = lo;
   };
 
-  int pn = grid_slot(), buf = 0;
+  const int step = (int)gridDim.x / PARTS;
+  int pn = slot / PARTS, buf = 0;
   if (pn < total) load_tile(pn);
-  for (; pn < total; pn += gridDim.x, buf ^= 1) {
+  for (; pn < total; pn += step, buf ^= 1) {
     const Tile xn = {lds + buf * Tile::SLOTS};
     const Lane here = lane_here();
     int j0;
@@ -429,7 +435,7 @@ __global__ __launch_bounds__(6 * C) void triattn_proj_pass(TriattnF32 p, int pan
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) xn.store4(pos, li + 16 * e, y[e]);
       float bias = 0.f;  // of head li
-      for (int h = 0; h < H; ++h) {
+      for (int h = h0; h < h1; ++h) {
         float d = 0.f;
 #pragma unroll
         for (int e = 0; e < C / 64; ++e) {
@@ -439,12 +445,12 @@ __global__ __launch_bounds__(6 * C) void triattn_proj_pass(TriattnF32 p, int pan
         d = group_sum<16>(d);
         bias = li == h ? d : bias;
       }
-      if (li < H) {  // rows padded to whole panels: zero rows store zeros
+      if (li >= h0 && li < h1) {  // rows padded to whole panels: zero rows store zeros
         const int b = bi / N, i = bi - b * N;
         p.tb[(((size_t)b * H + li) * N + i) * p.Jp + j0 + pos] = bias;
       }
     }
-    load_tile(pn + (int)gridDim.x < total ? pn + gridDim.x : pn);
+    load_tile(pn + step < total ? pn + step : pn);
     __syncthreads();  // this tile is complete, and everybody has finished with the other buffer
     const Lane out = lane_here();
     const int l32 = out.l32, lh = out.lh, lane = l32 + 32 * lh, nt = p.Jp / 32, jt = j0 / 32;
@@ -586,16 +592,29 @@ hipError_t launch_trimul_out(const TrimulF32& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <int C, int PARTS>
+hipError_t launch_triattn_proj(const TriattnF32& p, int panels, long total, hipStream_t stream) {
+  unsigned grid = 0;
+  hipError_t e = resident_grid<triattn_proj_pass<C, PARTS>>(6 * C / PARTS, AttProjLds<C>::kBytes, PARTS * total, &grid);
+  if (e != hipSuccess) return e;
+  grid -= grid % PARTS;
+  hipLaunchKernelGGL((triattn_proj_pass<C, PARTS>), dim3(grid), dim3(6 * C / PARTS), AttProjLds<C>::kBytes, stream, p, panels,
+                     (int)total);
+  return hipGetLastError();
+}
 template <int C>
 hipError_t launch_triattn_proj(const TriattnF32& p, hipStream_t stream) {
   const int panels = p.Jp / 32;
   const long total = (long)p.B * p.N * panels;
   if (total > 0x3fffffffL) return hipErrorInvalidValue;
-  unsigned grid = 0;
-  hipError_t e = resident_grid<triattn_proj_pass<C>>(6 * C, AttProjLds<C>::kBytes, total, &grid);
+  static int cache[kMaxDevices];
+  int cus = 0;
+  const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(triattn_proj_pass<C>, dim3(grid), dim3(6 * C), AttProjLds<C>::kBytes, stream, p, panels, (int)total);
-  return hipGetLastError();
+  // One / two / four work-groups per tile, us: four trunk blocks at N = 64 615 / 612 / 624, 45 599 / 591 / 599, 30 558 / 546 / 551, a pair stack
+  // at 64 112 / 110 / 111, and with more tiles than half of the CUs, at 80, 137 / 142 / 143.
+  if (C == 128 && 2 * total <= cus) return launch_triattn_proj<C, C == 128 ? 2 : 1>(p, panels, total, stream);
+  return launch_triattn_proj<C, 1>(p, panels, total, stream);
 }
 
 template <int C>
