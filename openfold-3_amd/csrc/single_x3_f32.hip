@@ -80,12 +80,12 @@ __device__ __forceinline__ void store_partial(float* part, const f32x16_t& acc, 
   }
 }
 // outputs 4 c4 .. 4 c4 + 3 of row `row`, summed over the NW waves' partial tiles (stride: floats between them)
-template <int NW>
+template <int NW, int LD = kPartLd>
 __device__ __forceinline__ float4 sum_partials(const float* part, int stride, int row, int c4) {
-  float4 s = *reinterpret_cast<const float4*>(part + row * kPartLd + 4 * c4);
+  float4 s = *reinterpret_cast<const float4*>(part + row * LD + 4 * c4);
 #pragma unroll
   for (int w = 1; w < NW; ++w) {
-    const float4 v = *reinterpret_cast<const float4*>(part + w * stride + row * kPartLd + 4 * c4);
+    const float4 v = *reinterpret_cast<const float4*>(part + w * stride + row * LD + 4 * c4);
     s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
   }
   return s;
@@ -239,6 +239,44 @@ __device__ __forceinline__ void plain_products(const float* __restrict__ src, lo
     for (int e = 0; e < 16; ++e) x[e] = xn[e], w[0][e] = wn[e];
   }
   store_partial(part + wave * kPart, acc[0], small[0], l32, lh);
+  __syncthreads();
+}
+
+// The same for a tile of 16 rows x 16 outputs: lane (row l16, quarter lq) reads the 8 consecutive k-values 8 lq .. + 7 of a block, the
+// operand of one MFMA step, and ends with outputs 4 lq .. + 3 of row l16.
+constexpr int kPart16Ld = 20, kPart16 = 16 * kPart16Ld;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
+__device__ __forceinline__ f32x4_t mfma_16x16x32(u32x4_t a, u32x4_t b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+template <int NW>
+__device__ __forceinline__ void plain_products16(const float* __restrict__ src, long pos0, long n_rows, int K,
+                                                 const float* __restrict__ W, float* part) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+  const int blocks = K / 32;
+  const long row = pos0 + l16 < n_rows ? pos0 + l16 : n_rows - 1;
+  const float4* xp = reinterpret_cast<const float4*>(src + row * K + 8 * lq);
+  const float4* wp = reinterpret_cast<const float4*>(W + (long)l16 * K + 8 * lq);
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f}, small = acc;
+  float4 x[2], w[2];
+  auto load = [&](int kb) { x[0] = xp[8 * kb], x[1] = xp[8 * kb + 1], w[0] = wp[8 * kb], w[1] = wp[8 * kb + 1]; };
+  if (wave < blocks) load(wave);
+  for (int kb = wave; kb < blocks; kb += NW) {
+    u32x4_t xo[3], wo[3];
+    const float xv[8] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w};
+    const float wv[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
+    load(kb + NW < blocks ? kb + NW : kb);  // the last one is read again: no load under a condition
+    split8(xv, xo[0], xo[1], xo[2]);
+    split8(wv, wo[0], wo[1], wo[2]);
+    small = mfma_16x16x32(wo[2], xo[0], small);
+    acc = mfma_16x16x32(wo[1], xo[0], acc);
+    small = mfma_16x16x32(wo[0], xo[2], small);
+    acc = mfma_16x16x32(wo[0], xo[1], acc);
+    small = mfma_16x16x32(wo[1], xo[1], small);
+    acc = mfma_16x16x32(wo[0], xo[0], acc);
+  }
+  *reinterpret_cast<float4*>(part + wave * kPart16 + l16 * kPart16Ld + 4 * lq) =
+      make_float4(acc[0] + small[0], acc[1] + small[1], acc[2] + small[2], acc[3] + small[3]);
   __syncthreads();
 }
 
@@ -492,20 +530,33 @@ __global__ __launch_bounds__(64 * kAttnWaves) void single_attn_x3_f32(SingleAttn
     }
 }
 
-// out = [a +] og Wo^T (plain FMA kernel 41 / 45 / 49 us at 64 / 384 / 768 rows)
-constexpr int kOutWaves = 4;
-__global__ __launch_bounds__(64 * kOutWaves) void single_out_x3_f32(SingleAttnF32Args p) {
-  __shared__ __align__(16) float part[kOutWaves * kPart];
-  const long rows = (long)p.B * p.N, pos0 = (long)blockIdx.x * 32;
-  const int HD = p.H * p.D, o0 = 32 * blockIdx.y;
-  plain_products<kOutWaves>(p.og, pos0, rows, HD, p.wo + (size_t)o0 * HD, part);
-  const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
-  if (pos0 + r >= rows) return;
-  float4 v = sum_partials<kOutWaves>(part, kPart, r, c4);
+// outputs 4 c4 .. + 3 of row r of a tile of T x T, for the threads that have one
+template <int T, int NW>
+__device__ __forceinline__ bool tile_products(const float* src, long pos0, long n_rows, int K, const float* W, float* part, int& r, int& c4,
+                                              float4& v) {
+  if (T == 32) plain_products<NW>(src, pos0, n_rows, K, W, part);
+  else plain_products16<NW>(src, pos0, n_rows, K, W, part);
+  r = threadIdx.x / (T / 4), c4 = threadIdx.x % (T / 4);
+  if (threadIdx.x >= T * T / 4 || pos0 + r >= n_rows) return false;
+  v = sum_partials<NW, T == 32 ? kPartLd : kPart16Ld>(part, T == 32 ? kPart : kPart16, r, c4);
   if (__builtin_expect(has_nan(v), 0)) {
-    const float4* x = reinterpret_cast<const float4*>(p.og + (pos0 + r) * HD);
-    v = plain_dots([&](int k) { return x[k]; }, p.wo + (size_t)(o0 + 4 * c4) * HD, HD);
+    const float4* x = reinterpret_cast<const float4*>(src + (pos0 + r) * K);
+    v = plain_dots([&](int k) { return x[k]; }, W + (size_t)4 * c4 * K, K);
   }
+  return true;
+}
+
+// out = [a +] og Wo^T (plain FMA kernel 41 / 45 / 49 us at 64 / 384 / 768 rows)
+template <int T>
+constexpr int kOutWaves = T == 32 ? 4 : 8;
+template <int T>  // rows and outputs of a tile, 32 or 16
+__global__ __launch_bounds__(64 * kOutWaves<T>) void single_out_x3_f32(SingleAttnF32Args p) {
+  __shared__ __align__(16) float part[kOutWaves<T> * (T == 32 ? kPart : kPart16)];
+  const long rows = (long)p.B * p.N, pos0 = (long)blockIdx.x * T;
+  const int HD = p.H * p.D, o0 = T * blockIdx.y;
+  int r, c4;
+  float4 v;
+  if (!tile_products<T, kOutWaves<T>>(p.og, pos0, rows, HD, p.wo + (size_t)o0 * HD, part, r, c4, v)) return;
   const size_t off = (pos0 + r) * p.C + o0 + 4 * c4;
   if (p.add_residual) {
     const float4 x = *reinterpret_cast<const float4*>(p.a + off);
@@ -538,19 +589,14 @@ __global__ __launch_bounds__(64 * kLnWaves) void row_hidden_x3_f32(RowTransition
 
 // out = [x +] (h Wout^T) * mask; the sum over up to 2048 hidden channels is dealt to 16 waves
 constexpr int kRowOutWaves = 16;
+template <int T>  // rows and outputs of a tile, 32 or 16
 __global__ __launch_bounds__(64 * kRowOutWaves) void row_out_x3_f32(RowTransitionF32Args p) {
-  extern __shared__ float part[];  // [kRowOutWaves][kPart]
-  const long pos0 = (long)blockIdx.x * 32;
-  const int o0 = 32 * blockIdx.y;
-  plain_products<kRowOutWaves>(p.hidden, pos0, p.rows, p.HID, p.wout + (size_t)o0 * p.HID, part);
-  if (threadIdx.x >= 256) return;
-  const int r = threadIdx.x >> 3, c4 = threadIdx.x & 7;
-  if (pos0 + r >= p.rows) return;
-  float4 v = sum_partials<kRowOutWaves>(part, kPart, r, c4);
-  if (__builtin_expect(has_nan(v), 0)) {
-    const float4* x = reinterpret_cast<const float4*>(p.hidden + (pos0 + r) * p.HID);
-    v = plain_dots([&](int k) { return x[k]; }, p.wout + (size_t)(o0 + 4 * c4) * p.HID, p.HID);
-  }
+  extern __shared__ __align__(16) float part[];  // [kRowOutWaves][kPart or kPart16]
+  const long pos0 = (long)blockIdx.x * T;
+  const int o0 = T * blockIdx.y;
+  int r, c4;
+  float4 v;
+  if (!tile_products<T, kRowOutWaves>(p.hidden, pos0, p.rows, p.HID, p.wout + (size_t)o0 * p.HID, part, r, c4, v)) return;
   if (p.mask) {
     const float m = p.mask[pos0 + r];
     v.x *= m, v.y *= m, v.z *= m, v.w *= m;
@@ -561,6 +607,18 @@ __global__ __launch_bounds__(64 * kRowOutWaves) void row_out_x3_f32(RowTransitio
     v.x = x.x + v.x, v.y = x.y + v.y, v.z = x.z + v.z, v.w = x.w + v.w;
   }
   *reinterpret_cast<float4*>(p.out + off) = v;
+}
+
+// The output products in tiles of 16 x 16 where all of these run at once, two to a CU: a tile of 32 x 32 splits and multiplies for twice as
+// long and reads twice as much through its CU's L1, on a quarter of the CUs.  Tiles of 32 / 16, us, at 24 / 64 / 150 / 256 / 300 | 384 / 640
+// rows: the transition's two kernels 24.6 / 26.2 / 28.5 / 33.3 / 33.0 | 39.6 / 46.4, 17.4 / 17.7 / 20.5 / 30.0 / 30.1 | 41.6 / 53.8; the attention's
+// three, 22.7 / 24.2 / 31.3 / 41.6 / 46.1 | 59.2 and 19.6 / 20.8 / 28.2 / 39.8 / 44.3 | 58.3 (512 rows 74.5, 75.7).
+hipError_t small_tiles(long rows, int C, bool* small) {
+  static int cache[kMaxDevices];
+  int cus = 0;
+  const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  *small = (rows + 15) / 16 * (C / 16) <= 2l * cus;
+  return e;
 }
 
 bool aligned16(std::initializer_list<const void*> ptrs) {
@@ -591,9 +649,15 @@ hipError_t single_attn_x3_fwd_f32(const SingleAttnF32Args& a, hipStream_t stream
   if (!(a.phases & kSingleAttend)) return hipSuccess;
   const int pb_vec = a.N % 4 == 0 && aligned16({a.pair_bias}) ? 1 : 0;
   hipLaunchKernelGGL(single_attn_x3_f32, dim3((a.N + 31) / 32, a.H, a.B), dim3(64 * kAttnWaves), 0, stream, a, pb_vec);
-  const hipError_t e = hipGetLastError();
+  hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(single_out_x3_f32, dim3((unsigned)row_tiles, a.C / 32), dim3(64 * kOutWaves), 0, stream, a);
+  bool small = false;
+  e = small_tiles(rows, a.C, &small);
+  if (e != hipSuccess) return e;
+  if (small)
+    hipLaunchKernelGGL(single_out_x3_f32<16>, dim3((unsigned)((rows + 15) / 16), a.C / 16), dim3(64 * kOutWaves<16>), 0, stream, a);
+  else
+    hipLaunchKernelGGL(single_out_x3_f32<32>, dim3((unsigned)row_tiles, a.C / 32), dim3(64 * kOutWaves<32>), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -606,12 +670,19 @@ hipError_t row_transition_x3_fwd_f32(const RowTransitionF32Args& a, hipStream_t 
   const long row_tiles = (a.rows + 31) / 32;
   if (row_tiles > 0x7fffffffl) return hipErrorInvalidValue;
   constexpr size_t lds = (size_t)kRowOutWaves * kPart * sizeof(float);
-  hipError_t e = allow_dynamic_lds<row_out_x3_f32>(lds);
+  hipError_t e = allow_dynamic_lds<row_out_x3_f32<32>>(lds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(row_hidden_x3_f32, dim3((unsigned)row_tiles, a.HID / 32), dim3(64 * kLnWaves), 0, stream, a);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(row_out_x3_f32, dim3((unsigned)row_tiles, a.C / 32), dim3(64 * kRowOutWaves), lds, stream, a);
+  bool small = false;
+  e = small_tiles(a.rows, a.C, &small);
+  if (e != hipSuccess) return e;
+  if (small)
+    hipLaunchKernelGGL(row_out_x3_f32<16>, dim3((unsigned)((a.rows + 15) / 16), a.C / 16), dim3(64 * kRowOutWaves),
+                       kRowOutWaves * kPart16 * sizeof(float), stream, a);
+  else
+    hipLaunchKernelGGL(row_out_x3_f32<32>, dim3((unsigned)row_tiles, a.C / 32), dim3(64 * kRowOutWaves), lds, stream, a);
   return hipGetLastError();
 }
 
