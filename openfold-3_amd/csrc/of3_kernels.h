@@ -132,6 +132,11 @@ struct TransitionArgs {
   const bf16_t* operands[3] = {};  // w_a, w_b, w_out in MFMA operand order, where a block's call has made them
 };
 hipError_t transition_launch(const TransitionArgs& args, int C, hipStream_t stream);
+// The output pass of the ending node's triangle attention and the transition after it in one launch, where the transition is one
+// of transition_tiles (transition_after_attention; contiguous rows: args.R == 1, weights packed)
+hipError_t transition_after_attention(const TransitionArgs& args, int C, bool* yes);
+hipError_t triattn_transition_launch(const TriattnOutArgs& end, const TransitionArgs& args, int C, hipStream_t stream);
+hipError_t triattn_transition_tiles_launch(const TriattnOutArgs& end, const TransitionArgs& args, int C, int position_tiles, hipStream_t stream);
 // tiles of 32 * position_tiles positions (1 or 2; at C = 128 also 4 or 5), HID a multiple of 128
 // (transition_tiles_bf16.hip)
 hipError_t transition_tiles_launch(const TransitionArgs& args, int C, int position_tiles, hipStream_t stream);

@@ -186,6 +186,14 @@ __device__ __forceinline__ void store_mask_bias(const TriattnProjArgs& p, int bi
 }
 
 
+// n / d for n * d < 2^32 by a multiplication
+struct Division {
+  int d;
+  unsigned inverse;  // 2^32 / d rounded up, 0 for d = 1
+  static Division by(int d) { return {d, d == 1 ? 0u : (unsigned)(((1ull << 32) + d - 1) / d)}; }
+  __device__ __forceinline__ int quotient(int n) const { return inverse ? (int)__umulhi((unsigned)n, inverse) : n; }
+};
+
 // logical number of a work-group: consecutive numbers run on one XCD where the grid deals evenly
 __device__ __forceinline__ int grid_slot() {
   return gridDim.x % 8 == 0 ? xcd_logical_block(blockIdx.x, gridDim.x / 8) : blockIdx.x;

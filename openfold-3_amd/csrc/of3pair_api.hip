@@ -604,11 +604,13 @@ int of3_transition_fwd(const void* x, const int64_t x_strides[3], const float* m
                                add_residual, nullptr, 0, dtype, stream);
 }
 
-// presplit as above; operands: w_a, w_b, w_out in MFMA operand order (bf16), or null
+// presplit as above; operands: w_a, w_b, w_out in MFMA operand order (bf16), or null.  before: the attention whose output pass the
+// launch begins with; takes_end: says whether it could, and launches nothing
 static int transition_fwd(const of3::WeightX3* presplit, const void* const* operands, const void* x, const int64_t x_strides[3], const float* mask,
                           const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_a, const void* w_b, const void* w_out,
                           void* out, int64_t B, int64_t N, int64_t C, int64_t HID, int add_residual, void* workspace,
-                          int64_t workspace_bytes, int dtype, void* stream) {
+                          int64_t workspace_bytes, int dtype, void* stream, const ModuleEnd* before = nullptr, bool* takes_end = nullptr) {
+  if (takes_end) *takes_end = false;
   const void* ptrs[] = {x, ln_w, ln_b, w_a, w_b, w_out, out};
   if (!positions_ok(B, N) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
   if (dtype == OF3_DTYPE_F32) {
@@ -678,7 +680,12 @@ static int transition_fwd(const of3::WeightX3* presplit, const void* const* oper
   args.HID = (int)HID;
   args.add_residual = add_residual ? 1 : 0;
   for (int i = 0; i < 3 && operands; ++i) args.operands[i] = bf(operands[i]);
-  hipError_t e = of3::transition_launch(args, (int)C, static_cast<hipStream_t>(stream));
+  if (takes_end) {
+    const hipError_t e = operands && rows == 1 ? of3::transition_after_attention(args, (int)C, takes_end) : hipSuccess;
+    return e == hipSuccess ? OF3_OK : fail_hip(e);
+  }
+  hipError_t e = before ? of3::triattn_transition_launch(before->att, args, (int)C, static_cast<hipStream_t>(stream))
+                        : of3::transition_launch(args, (int)C, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
@@ -1119,7 +1126,8 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
   int module = 0;  // of the four
   // the end of the module before, and where this one leaves its own
   auto before = [&] { return joined && module > 0 ? &ends[(module - 1) & 1] : nullptr; };
-  auto after = [&] { return joined && module < 3 ? &ends[module & 1] : nullptr; };
+  bool last_joined = false;  // the last module with the transition
+  auto after = [&] { return joined && (module < 3 || last_joined) ? &ends[module & 1] : nullptr; };
   auto trimul = [&](int m) {
     const void* const* w = k.w + 10 * m;
     const int st = trimul_fwd(k.mul ? k.mul + m * of3::kTrimulMatrices : nullptr, k.packed, src, z_strides, mask, mask_strides,
@@ -1141,15 +1149,19 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
     ++module;
     return st;
   };
+  auto transition = [&](const ModuleEnd* end, bool* takes_end) {
+    const void* const* w = k.w + 36;
+    return transition_fwd(k.tr, d.wide() ? nullptr : k.tr_operands, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask,
+                          mask_strides, w[0], w[1], w[2], w[3], w[4], out, d.B, d.N, d.C, d.HID, 1, d.wide() ? workspace : nullptr,
+                          d.wide() ? workspace_bytes : 0, d.dtype, stream, end, takes_end);
+  };
   int st = OF3_OK;
+  if (joined && !attention_first && d.HID != 0) st = transition(nullptr, &last_joined);
   for (int part = 0; part < 2; ++part)
     for (int m = 0; m < 2 && st == OF3_OK; ++m)
       st = (part == 0) == !attention_first ? trimul(m) : triattn(m);
   if (st != OF3_OK || d.HID == 0) return st;
-  const void* const* w = k.w + 36;
-  return transition_fwd(k.tr, d.wide() ? nullptr : k.tr_operands, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask, mask_strides, w[0], w[1],
-                        w[2], w[3], w[4], out, d.B, d.N, d.C, d.HID, 1, d.wide() ? workspace : nullptr,
-                        d.wide() ? workspace_bytes : 0, d.dtype, stream);
+  return transition(last_joined ? &ends[3 & 1] : nullptr, nullptr);
 }
 
 // what a block's call checks before its first launch: a block is updated in place, half of one is of no use

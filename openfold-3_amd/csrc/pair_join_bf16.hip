@@ -47,14 +47,6 @@ __device__ __forceinline__ int plain_slot(int panel, int pos, int chunk) {
   return panel * PanelTile<C, false>::SLOTS + PanelTile<C, false>::slot(pos, chunk);
 }
 
-// n / d for n * d < 2^32 by a multiplication
-struct Division {
-  int d;
-  unsigned inverse;  // 2^32 / d rounded up, 0 for d = 1
-  static Division by(int d) { return {d, d == 1 ? 0u : (unsigned)(((1ull << 32) + d - 1) / d)}; }
-  __device__ __forceinline__ int quotient(int n) const { return inverse ? (int)__umulhi((unsigned)n, inverse) : n; }
-};
-
 struct JoinTile {
   int b, r0, k0;        // batch element, first row, first column, in the frame of the second half
   int64_t sb, sr, sk;   // of z in that frame

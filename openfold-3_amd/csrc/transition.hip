@@ -404,7 +404,29 @@ hipError_t launch(const TransitionArgs& a, long limit, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// 32-position tiles per work-group of transition_tiles, 0: not there
+int position_tiles(const TransitionArgs& args, int C, int cus) {
+  const long panels = (long)args.B * args.R * ((args.N + 31) / 32);
+  const long per_cu = args.operands[0] ? (C == 128 ? 5 : 4) : (C == 128 ? 2 : 1);
+  if (args.HID % 128 != 0 || panels > per_cu * cus) return 0;
+  return panels <= cus ? 1 : (panels <= 2l * cus || C == 64 || !args.operands[0]) ? 2 : panels <= 4l * cus ? 4 : 5;
+}
+
 }  // namespace
+
+hipError_t transition_after_attention(const TransitionArgs& args, int C, bool* yes) {
+  static int cache[kMaxDevices];
+  int cus = 0;
+  const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  *yes = e == hipSuccess && position_tiles(args, C, cus) > 0;
+  return e;
+}
+hipError_t triattn_transition_launch(const TriattnOutArgs& end, const TransitionArgs& args, int C, hipStream_t stream) {
+  static int cache[kMaxDevices];
+  int cus = 0;
+  const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  return e == hipSuccess ? triattn_transition_tiles_launch(end, args, C, position_tiles(args, C, cus), stream) : e;
+}
 
 hipError_t transition_launch(const TransitionArgs& args, int C, hipStream_t stream) {
   if (args.HID % 32 != 0 || args.HID < 128) return hipErrorInvalidValue;  // at least four hidden tiles
@@ -419,12 +441,8 @@ hipError_t transition_launch(const TransitionArgs& args, int C, hipStream_t stre
   int cus = 0;
   const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
   if (e != hipSuccess) return e;
-  const long panels = (long)args.B * args.R * ((args.N + 31) / 32);
-  const long per_cu = args.operands[0] ? (C == 128 ? 5 : 4) : (C == 128 ? 2 : 1);
-  if (args.HID % 128 == 0 && panels <= per_cu * cus) {
-    const int tiles = panels <= cus ? 1 : (panels <= 2l * cus || C == 64 || !args.operands[0]) ? 2 : panels <= 4l * cus ? 4 : 5;
-    return transition_tiles_launch(args, C, tiles, stream);
-  }
+  const int tiles = position_tiles(args, C, cus);
+  if (tiles > 0) return transition_tiles_launch(args, C, tiles, stream);
   // A last round with few tiles takes as long as a full one (29 us at C = 128, n = 4).  Its positions, where they are the
   // end of one flat batch element, go to the shorter tiles instead if those are done in one go (15 us at two 32-position
   // tiles per CU, 18 at one with the weights as they are).  Two trunk blocks, us: N = 260 728 -> 709, 365 1087 -> 1069,

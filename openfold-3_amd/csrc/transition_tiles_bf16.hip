@@ -29,8 +29,13 @@ constexpr size_t lds_slots() {
   return (size_t)P * (2 * PanelTile<C, false>::SLOTS + 2 * 32 * 4 * S);
 }
 
-template <int C, int S, int P>
-__global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p, int packed, int tiles_per_row, int total) {
+// AFTER: the tile begins with the output pass of the triangle attention before it (the ending node's: its frame is the transposed one),
+// whose result goes from LDS to LDS; one tile per work-group, weights packed.  Saves a launch, the tile's trip to memory and back and the wait for the
+// first tile: four trunk blocks at N = 40 / 85 / 128 / 150 / 200 353 / 410 / 491 / 617 / 881 us, so 324 / 395 / 477 / 603 / 855; templates 4 x 60 152 /
+// 134, 2 x 90 166 / 160, 1 x 180 223 / 219.
+template <int C, int S, int P, bool AFTER>
+__global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p, int packed, int tiles_per_row, int total, TriattnOutArgs e,
+                                                                Division by_n) {
   typedef PanelTile<C, false> XTile;
   constexpr int KS = C / 16, OT = C / 32, HCH = 4 * S;  // 16-byte chunks of a position's hidden slice
   constexpr int TASKS = P * 32 / LnLane<C>::PPI;        // LayerNorm instructions of a tile
@@ -102,21 +107,94 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
       for (int s = 0; s < 2; ++s) wo[2 * t + s] = *reinterpret_cast<const u32x4_t*>(base + (slice * S + t) * step_t + s * step_s);
   };
 
-  int id = blockIdx.x;
+  int id = AFTER ? grid_slot() : blockIdx.x;
   if (id >= total) return;
   load_tile(id);
-  if (first) load_first(0);
+  if (!AFTER && first) load_first(0);
   for (; id < total; id += gridDim.x) {
     int b, i;
     const int j0 = place(id, b, i);
+    auto ln_slot = [&](int u) {
+      const int pos = (wave + kWaves * u) * ln.PPI + ln.pos();
+      return (pos >> 5) * XTile::SLOTS + XTile::slot(pos & 31, ln.chunk());
+    };
+    if constexpr (AFTER) {
+      // the same steps and rounding points as triattn_out.hip
+      constexpr int MINE = (P + GB - 1) / GB;
+      u32x4_t o[MINE][2], wg[KS], wz[KS];
+      const LnLane<C> lz = ln_lane<C>(e.ln_w, e.ln_b, lane);
 #pragma unroll
-    for (int u = 0; u < LPW; ++u) {
-      const int task = wave + kWaves * u;
-      if (task < TASKS) {
-        const int pos = task * ln.PPI + ln.pos(), slot = (pos >> 5) * XTile::SLOTS + XTile::slot(pos & 31, ln.chunk());
-        xn[slot] = ln.template normalised<false>(raw[u]);
+      for (int q = 0; q < MINE; ++q) {
+        const int pos = j0 + 32 * (pt_b + GB * q) + (lane & 31), f = pos < L ? pos : L - 1;
+        const int r = by_n.quotient(f), k = f - r * by_n.d;
+        const bf16_t* src = e.o + (((int64_t)b * by_n.d + k) * by_n.d + r) * C + 32 * ot + 16 * half;
+        o[q][0] = *reinterpret_cast<const u32x4_t*>(src);
+        o[q][1] = *reinterpret_cast<const u32x4_t*>(src + 8);
+      }
+      if (second) {
+        load_unit<C>(e.w_g, ot, arow, half, 1, wg);
+        load_unit<C>(e.w_o, ot, arow, half, 1, wz);
+      }
+#pragma unroll
+      for (int u = 0; u < LPW; ++u) {
+        if (wave + kWaves * u >= TASKS) continue;
+        const int slot = ln_slot(u);
+        xn[slot] = lz.template normalised<true>(raw[u]);
         xr[slot] = raw[u];
       }
+      __syncthreads();
+      if (second) {
+#pragma unroll
+        for (int q = 0; q < MINE; ++q) {  // the attention's output times its gate
+          const int pt = pt_b + GB * q;
+          if (P % GB != 0 && pt >= P) break;
+          const Lane at = lane_here();
+          f32x16_t acc = zero16();
+#pragma unroll
+          for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(wg[s], xn[pt * XTile::SLOTS + XTile::slot(at.l32, 2 * s + at.lh)], acc);
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {
+            float ov[8];
+            unpack8(o[q][hf], ov);
+#pragma unroll
+            for (int v = 0; v < 8; ++v) ov[v] *= sigmoid_from_scaled(acc[8 * hf + v]);
+            hid[pt * XTile::SLOTS + XTile::slot(at.l32, 4 * ot + 2 * at.lh + hf)] = pack8(ov);
+          }
+        }
+      }
+      __syncthreads();
+      if (first) load_first(0);
+      if (second) {
+#pragma unroll
+        for (int q = 0; q < MINE; ++q) {
+          const int pt = pt_b + GB * q;
+          if (P % GB != 0 && pt >= P) break;
+          const Lane at = lane_here();
+          f32x16_t acc = zero16();
+#pragma unroll
+          for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(wz[s], hid[pt * XTile::SLOTS + XTile::slot(at.l32, 2 * s + at.lh)], acc);
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {
+            u32x4_t* const s = xr + pt * XTile::SLOTS + XTile::slot(at.l32, 4 * ot + 2 * at.lh + hf);
+            float r[8];
+            unpack8(*s, r);
+#pragma unroll
+            for (int v = 0; v < 8; ++v) r[v] = acc[8 * hf + v] + r[v];
+            *s = pack8(r);
+          }
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < LPW; ++u)
+        if (wave + kWaves * u < TASKS) raw[u] = xr[ln_slot(u)];
+    }
+#pragma unroll
+    for (int u = 0; u < LPW; ++u) {
+      if (wave + kWaves * u >= TASKS) continue;
+      const int slot = ln_slot(u);
+      xn[slot] = ln.template normalised<false>(raw[u]);
+      if (!AFTER) xr[slot] = raw[u];
     }
     float mtile[BPT];
     f32x16_t oacc[BPT];
@@ -156,7 +234,7 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
       }
       __syncthreads();  // the slice is complete, and nobody reads the one before any more
       if (first) load_first(slice + 1 < slices ? slice + 1 : 0);
-      if (slice + 1 == slices) load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
+      if (!AFTER && slice + 1 == slices) load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
       if (second) {
 #pragma unroll
         for (int q = 0; q < BPT; ++q) {
@@ -197,23 +275,25 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
         }
       }
     }
+    if (AFTER) return;
     __syncthreads();  // both tiles of x are rewritten by the next one
   }
 }
 
-template <int C, int S, int P>
-hipError_t launch(const TransitionArgs& a, hipStream_t stream) {
+template <int C, int S, int P, bool AFTER = false>
+hipError_t launch(const TransitionArgs& a, hipStream_t stream, const TriattnOutArgs& end = {}) {
   constexpr size_t lds = lds_slots<C, S, P>() * 16;
+  constexpr auto kernel = transition_tiles<C, S, P, AFTER>;
   static int cache[kMaxDevices];
   int fit = 0;
-  hipError_t e = allow_dynamic_lds<transition_tiles<C, S, P>>(lds);
+  hipError_t e = allow_dynamic_lds<kernel>(lds);
   if (e == hipSuccess)
     e = per_device(
         cache,
         [&](int dev, int* v) {
           int cus = 0, per_cu = 0;
           hipError_t s = cu_count(dev, &cus);
-          if (s == hipSuccess) s = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, transition_tiles<C, S, P>, 64 * kWaves, lds);
+          if (s == hipSuccess) s = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * kWaves, lds);
           *v = cus * (per_cu > 0 ? per_cu : 1);
           return s;
         },
@@ -224,12 +304,28 @@ hipError_t launch(const TransitionArgs& a, hipStream_t stream) {
   TransitionArgs k = a;
   const int packed = a.operands[0] ? 1 : 0;
   if (packed) k.w_a = a.operands[0], k.w_b = a.operands[1], k.w_out = a.operands[2];
-  hipLaunchKernelGGL((transition_tiles<C, S, P>), dim3((unsigned)(total < fit ? total : fit)), dim3(64 * kWaves), lds, stream, k,
-                     packed, tiles_per_row, (int)total);
+  if (AFTER && (!packed || a.R != 1 || a.N != end.N * end.N || a.B != end.B)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(AFTER || total < fit ? total : fit)), dim3(64 * kWaves), lds, stream, k, packed, tiles_per_row, (int)total,
+                     end, Division::by(AFTER ? end.N : 1));
   return hipGetLastError();
 }
 
 }  // namespace
+
+hipError_t triattn_transition_tiles_launch(const TriattnOutArgs& end, const TransitionArgs& a, int C, int position_tiles, hipStream_t stream) {
+  const bool wide = a.HID % 256 == 0;
+  if (C == 64) {
+    if (position_tiles == 1) return wide ? launch<64, 8, 1, true>(a, stream, end) : launch<64, 4, 1, true>(a, stream, end);
+    return wide ? launch<64, 8, 2, true>(a, stream, end) : launch<64, 4, 2, true>(a, stream, end);
+  }
+  switch (position_tiles) {
+    case 1: return wide ? launch<128, 8, 1, true>(a, stream, end) : launch<128, 4, 1, true>(a, stream, end);
+    case 2: return wide ? launch<128, 8, 2, true>(a, stream, end) : launch<128, 4, 2, true>(a, stream, end);
+    case 4: return launch<128, 4, 4, true>(a, stream, end);
+    case 5: return launch<128, 4, 5, true>(a, stream, end);
+  }
+  return hipErrorInvalidValue;
+}
 
 hipError_t transition_tiles_launch(const TransitionArgs& a, int C, int position_tiles, hipStream_t stream) {
   if (position_tiles > 2) {
