@@ -157,6 +157,36 @@ __device__ __forceinline__ int tile_slot(int pos, int chunk) {
 // ---- global -> LDS loads without registers ------------------------------------------------------
 #define OF3_LDS_AS __attribute__((address_space(3)))
 
+// the first `left` (up to all) of 16 values as bf16; vec_ok: dst is 16-byte aligned
+__device__ __forceinline__ void store_run16(bf16_t* dst, const f32x16_t& acc, int left, bool vec_ok) {
+  if (vec_ok && left >= 16) {
+    u32x4_t o0, o1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      o0[q] = pack_bf16(acc[2 * q], acc[2 * q + 1]);
+      o1[q] = pack_bf16(acc[8 + 2 * q], acc[8 + 2 * q + 1]);
+    }
+    *reinterpret_cast<u32x4_t*>(dst) = o0;
+    *reinterpret_cast<u32x4_t*>(dst + 8) = o1;
+  } else if (left >= 16) {
+    // rows of a length that is no multiple of 8 start at any even byte: pairs of positions from the
+    // first 4-byte boundary on (8 stores, or 1 + 7 + 1) instead of 16 single ones
+    const bool odd = (reinterpret_cast<uintptr_t>(dst) & 2) != 0;
+    if (odd) {
+      dst[0] = to_bf16(acc[0]);
+      dst[15] = to_bf16(acc[15]);
+    }
+    uint32_t* d32 = reinterpret_cast<uint32_t*>(dst + (odd ? 1 : 0));
+#pragma unroll
+    for (int q = 0; q < 7; ++q) d32[q] = odd ? pack_bf16(acc[2 * q + 1], acc[2 * q + 2]) : pack_bf16(acc[2 * q], acc[2 * q + 1]);
+    if (!odd) d32[7] = pack_bf16(acc[14], acc[15]);
+  } else {
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      if (v < left) dst[v] = to_bf16(acc[v]);
+  }
+}
+
 // raw buffer descriptor over [base, base + bytes): 32-bit offsets, no swizzling; reads beyond the
 // range return zeros
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, size_t bytes) {

@@ -135,8 +135,11 @@ hipError_t transition_launch(const TransitionArgs& args, int C, hipStream_t stre
 // The output pass of the ending node's triangle attention and the transition after it in one launch, where the transition is one
 // of transition_tiles (transition_after_attention; contiguous rows: args.R == 1, weights packed)
 hipError_t transition_after_attention(const TransitionArgs& args, int C, bool* yes);
-hipError_t triattn_transition_launch(const TriattnOutArgs& end, const TransitionArgs& args, int C, hipStream_t stream);
-hipError_t triattn_transition_tiles_launch(const TriattnOutArgs& end, const TransitionArgs& args, int C, int position_tiles, hipStream_t stream);
+// bias: a pair bias of the result to go with it (128 channels), or null
+struct PairBiasArgs;
+hipError_t triattn_transition_launch(const TriattnOutArgs& end, const TransitionArgs& args, const PairBiasArgs* bias, int C, hipStream_t stream);
+hipError_t triattn_transition_tiles_launch(const TriattnOutArgs& end, const TransitionArgs& args, const PairBiasArgs* bias, int C,
+                                           int position_tiles, hipStream_t stream);
 // tiles of 32 * position_tiles positions (1 or 2; at C = 128 also 4 or 5), HID a multiple of 128
 // (transition_tiles_bf16.hip)
 hipError_t transition_tiles_launch(const TransitionArgs& args, int C, int position_tiles, hipStream_t stream);

@@ -605,11 +605,12 @@ int of3_transition_fwd(const void* x, const int64_t x_strides[3], const float* m
 }
 
 // presplit as above; operands: w_a, w_b, w_out in MFMA operand order (bf16), or null.  before: the attention whose output pass the
-// launch begins with; takes_end: says whether it could, and launches nothing
+// launch begins with; takes_end: says whether it could, and launches nothing; bias: a pair bias of the result that goes with `before`
 static int transition_fwd(const of3::WeightX3* presplit, const void* const* operands, const void* x, const int64_t x_strides[3], const float* mask,
                           const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_a, const void* w_b, const void* w_out,
                           void* out, int64_t B, int64_t N, int64_t C, int64_t HID, int add_residual, void* workspace,
-                          int64_t workspace_bytes, int dtype, void* stream, const ModuleEnd* before = nullptr, bool* takes_end = nullptr) {
+                          int64_t workspace_bytes, int dtype, void* stream, const ModuleEnd* before = nullptr, bool* takes_end = nullptr,
+                          const of3::PairBiasArgs* bias = nullptr) {
   if (takes_end) *takes_end = false;
   const void* ptrs[] = {x, ln_w, ln_b, w_a, w_b, w_out, out};
   if (!positions_ok(B, N) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
@@ -684,7 +685,7 @@ static int transition_fwd(const of3::WeightX3* presplit, const void* const* oper
     const hipError_t e = operands && rows == 1 ? of3::transition_after_attention(args, (int)C, takes_end) : hipSuccess;
     return e == hipSuccess ? OF3_OK : fail_hip(e);
   }
-  hipError_t e = before ? of3::triattn_transition_launch(before->att, args, (int)C, static_cast<hipStream_t>(stream))
+  hipError_t e = before ? of3::triattn_transition_launch(before->att, args, bias, (int)C, static_cast<hipStream_t>(stream))
                         : of3::transition_launch(args, (int)C, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
@@ -1109,9 +1110,11 @@ static hipError_t prepare_blocks(const void* const* const* weights, int n, const
   return of3::pack_weights_launch(jobs, stream);
 }
 
+// bias: where the launches allow it, the pair bias of the result goes with the last of them (*bias_done).  Its output may be the beginning of
+// the workspace, as large as a triangle multiplication's: nothing of that is read by then.
 static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void* z, const int64_t z_strides[3],
                           const float* mask, const int64_t mask_strides[3], void* out, int flags, void* workspace,
-                          int64_t workspace_bytes, void* stream) {
+                          int64_t workspace_bytes, void* stream, const of3::PairBiasArgs* bias = nullptr, bool* bias_done = nullptr) {
   const void* src = z;  // the first module reads z, every later one updates out in place
   int rows = 0;
   if (k.packed && d.CH == d.C && d.H == 4 && 4 * d.D == d.C && join_room(d.dtype, d.B, d.N)) {
@@ -1153,7 +1156,7 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
     const void* const* w = k.w + 36;
     return transition_fwd(k.tr, d.wide() ? nullptr : k.tr_operands, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask,
                           mask_strides, w[0], w[1], w[2], w[3], w[4], out, d.B, d.N, d.C, d.HID, 1, d.wide() ? workspace : nullptr,
-                          d.wide() ? workspace_bytes : 0, d.dtype, stream, end, takes_end);
+                          d.wide() ? workspace_bytes : 0, d.dtype, stream, end, takes_end, end ? bias : nullptr);
   };
   int st = OF3_OK;
   if (joined && !attention_first && d.HID != 0) st = transition(nullptr, &last_joined);
@@ -1161,6 +1164,7 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
     for (int m = 0; m < 2 && st == OF3_OK; ++m)
       st = (part == 0) == !attention_first ? trimul(m) : triattn(m);
   if (st != OF3_OK || d.HID == 0) return st;
+  if (bias_done) *bias_done = bias && last_joined;
   return transition(last_joined ? &ends[3 & 1] : nullptr, nullptr);
 }
 
@@ -1182,10 +1186,10 @@ int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t 
   return need < 0 ? need : need + d.prepared_bytes();
 }
 
-int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t z_strides[3], const float* mask,
-                       const int64_t mask_strides[3], void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H,
-                       int64_t D, int64_t HID, float inf, int flags, void* workspace, int64_t workspace_bytes, int dtype,
-                       void* stream) {
+static int pair_block_fwd(const void* const* weights, const void* z, const int64_t z_strides[3], const float* mask,
+                          const int64_t mask_strides[3], void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H,
+                          int64_t D, int64_t HID, float inf, int flags, void* workspace, int64_t workspace_bytes, int dtype,
+                          void* stream, const of3::PairBiasArgs* bias = nullptr, bool* bias_done = nullptr) {
   const int64_t need = of3_pair_block_workspace_bytes(dtype, B, N, C, CH, H, D, HID);
   const BlockDims d = {dtype, B, N, C, CH, H, D, HID, inf};
   if (need < 0 || !pair_block_args_ok(d, weights, z, z_strides, mask, mask_strides, out, workspace)) return OF3_EINVAL;
@@ -1194,7 +1198,14 @@ int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t 
   const hipError_t e = prepare_blocks(&weights, 1, d, static_cast<char*>(workspace) + need - d.prepared_bytes(), &k,
                                       static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail_hip(e);
-  return run_pair_block(k, d, z, z_strides, mask, mask_strides, out, flags, workspace, workspace_bytes, stream);
+  return run_pair_block(k, d, z, z_strides, mask, mask_strides, out, flags, workspace, workspace_bytes, stream, bias, bias_done);
+}
+int of3_pair_block_fwd(const void* const* weights, const void* z, const int64_t z_strides[3], const float* mask,
+                       const int64_t mask_strides[3], void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H,
+                       int64_t D, int64_t HID, float inf, int flags, void* workspace, int64_t workspace_bytes, int dtype,
+                       void* stream) {
+  return pair_block_fwd(weights, z, z_strides, mask, mask_strides, out, B, N, C, CH, H, D, HID, inf, flags, workspace, workspace_bytes, dtype,
+                        stream);
 }
 
 int64_t of3_pairformer_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
@@ -1206,6 +1217,21 @@ int64_t of3_pairformer_block_workspace_bytes(int dtype, int64_t B, int64_t N, in
   const int64_t single = align256(B * H_s * N * N * (dtype == OF3_DTYPE_BF16 ? 2 : 4)) + attn;  // the pair bias, then its consumer's
   if (single > need) need = single;
   return rows > need ? rows : need;
+}
+
+// A block's pair bias, to go with its last pair launch; what of3_pair_bias_fwd would refuse, or the launch cannot take, is left to that call
+static bool block_bias_args(const BlockDims& d, const void* const* ws_, int64_t H_s, void* out, of3::PairBiasArgs* a) {
+  if (d.dtype != OF3_DTYPE_BF16 || d.C != 128 || H_s < 1 || H_s > 32 || !ws_[0] || !ws_[2] || !out) return false;
+  if (!aligned16(ws_[0]) || !aligned16(ws_[1]) || !aligned16(ws_[2]) || !aligned16(out)) return false;
+  a->z = nullptr;  // the launch's own result
+  a->ln_w = bf(ws_[0]);
+  a->ln_b = bf(ws_[1]);
+  a->w = bf(ws_[2]);
+  a->out = bf(out);
+  a->B = (int)d.B;
+  a->N = (int)d.N;
+  a->H = (int)H_s;
+  return true;
 }
 
 static bool single_args_ok(const BlockDims& d, const void* const* w, const void* s, const void* s_out, const float* single_mask) {
@@ -1226,11 +1252,14 @@ int of3_pairformer_block_fwd(const void* const* weights, const void* s, const vo
   const void* const* ws_ = weights + OF3_PAIR_BLOCK_WEIGHTS;
   if (!single_args_ok(d, ws_, s, s_out, single_mask)) return OF3_EINVAL;
   if (workspace_bytes < need) return OF3_ENOSPC;
-  int st = of3_pair_block_fwd(weights, z, z_strides, pair_mask, mask_strides, z_out, B, N, C, CH, H, D, HID, inf, flags,
-                              workspace, workspace_bytes, dtype, stream);
+  of3::PairBiasArgs bias;
+  bool bias_done = false;
+  const bool with_bias = block_bias_args(d, ws_, H_s, workspace, &bias);
+  int st = pair_block_fwd(weights, z, z_strides, pair_mask, mask_strides, z_out, B, N, C, CH, H, D, HID, inf, flags,
+                          workspace, workspace_bytes, dtype, stream, with_bias ? &bias : nullptr, &bias_done);
   if (st != OF3_OK) return st;
   const int64_t bias_bytes = align256(B * H_s * N * N * (d.wide() ? 4 : 2));
-  st = of3_pair_bias_fwd(z_out, z_strides, ws_[0], ws_[1], ws_[2], workspace, B, N, C, H_s, dtype, stream);
+  if (!bias_done) st = of3_pair_bias_fwd(z_out, z_strides, ws_[0], ws_[1], ws_[2], workspace, B, N, C, H_s, dtype, stream);
   if (st != OF3_OK) return st;
   st = of3_attn_pair_bias_fwd(s, workspace, single_mask, ws_[3], ws_[4], ws_[5], ws_[6], ws_[7], ws_[8], ws_[9], ws_[10],
                               s_out, B, N, C_s, H_s, D_s, inf_s, 1, static_cast<char*>(workspace) + bias_bytes,
@@ -1354,17 +1383,21 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
     }
     const void* const* ws_ = weights[i] + OF3_PAIR_BLOCK_WEIGHTS;
     void* const bias = bias0 + (i % w.buffers) * w.bias;
+    of3::PairBiasArgs bias_args;
+    bool bias_done = false;
+    const bool with_bias = i < w.buffers && block_bias_args(d, ws_, H_s, bias, &bias_args);  // else its buffer has to be waited for
     auto attention = [&](int phases, hipStream_t on) {
       return attn_pair_bias(phases, i ? s_out : s, bias, single_mask, ws_[3], ws_[4], ws_[5], ws_[6], ws_[7], ws_[8], ws_[9],
                             ws_[10], s_out, B, N, C_s, H_s, D_s, inf_s, 1, single, w.single, dtype, on);
     };
     // the projections of s need no pair bias; those of the first block have nothing to wait behind on the side stream
     if (i > 0 && (st = attention(of3::kSingleProject, streams.side)) != OF3_OK) break;
-    st = run_pair_block(k[q], d, i ? z_out : z, z_strides, pair_mask, mask_strides, z_out, flags, workspace, w.module, streams.main);
+    st = run_pair_block(k[q], d, i ? z_out : z, z_strides, pair_mask, mask_strides, z_out, flags, workspace, w.module, streams.main,
+                        with_bias ? &bias_args : nullptr, &bias_done);
     if (st != OF3_OK) break;
     // a buffer is used again: the attentions issued so far have read theirs
     if (i >= w.buffers && (st = streams.wait(streams.main, StreamPair::kFree)) != OF3_OK) break;
-    st = of3_pair_bias_fwd(z_out, z_strides, ws_[0], ws_[1], ws_[2], bias, B, N, C, H_s, dtype, streams.main);
+    if (!bias_done) st = of3_pair_bias_fwd(z_out, z_strides, ws_[0], ws_[1], ws_[2], bias, B, N, C, H_s, dtype, streams.main);
     if (st != OF3_OK) break;
     // the last block has nothing beside it: it goes on where its bias was written
     st = last ? streams.join() : streams.order(streams.main, streams.side, StreamPair::kBias);

@@ -421,11 +421,11 @@ hipError_t transition_after_attention(const TransitionArgs& args, int C, bool* y
   *yes = e == hipSuccess && position_tiles(args, C, cus) > 0;
   return e;
 }
-hipError_t triattn_transition_launch(const TriattnOutArgs& end, const TransitionArgs& args, int C, hipStream_t stream) {
+hipError_t triattn_transition_launch(const TriattnOutArgs& end, const TransitionArgs& args, const PairBiasArgs* bias, int C, hipStream_t stream) {
   static int cache[kMaxDevices];
   int cus = 0;
   const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
-  return e == hipSuccess ? triattn_transition_tiles_launch(end, args, C, position_tiles(args, C, cus), stream) : e;
+  return e == hipSuccess ? triattn_transition_tiles_launch(end, args, bias, C, position_tiles(args, C, cus), stream) : e;
 }
 
 hipError_t transition_launch(const TransitionArgs& args, int C, hipStream_t stream) {

@@ -29,13 +29,16 @@ constexpr size_t lds_slots() {
   return (size_t)P * (2 * PanelTile<C, false>::SLOTS + 2 * 32 * 4 * S);
 }
 
+// BIAS: and ends with the pair bias of the block's attention over s (pair_bias.hip), from the rows that it has just finished; the positions
+// of a tile are as contiguous there as in z.  Four trunk blocks at N = 40 / 85 / 128 / 151 / 200 364 / 397 / 476 / 610 / 865 us, so 347 / 375 / 457 /
+// 592 / 847 (a launch, and z read once more from memory).
 // AFTER: the tile begins with the output pass of the triangle attention before it (the ending node's: its frame is the transposed one),
 // whose result goes from LDS to LDS; one tile per work-group, weights packed.  Saves a launch, the tile's trip to memory and back and the wait for the
 // first tile: four trunk blocks at N = 40 / 85 / 128 / 150 / 200 353 / 410 / 491 / 617 / 881 us, so 324 / 395 / 477 / 603 / 855; templates 4 x 60 152 /
 // 134, 2 x 90 166 / 160, 1 x 180 223 / 219.
-template <int C, int S, int P, bool AFTER>
+template <int C, int S, int P, bool AFTER, bool BIAS>
 __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p, int packed, int tiles_per_row, int total, TriattnOutArgs e,
-                                                                Division by_n) {
+                                                                Division by_n, PairBiasArgs pb) {
   typedef PanelTile<C, false> XTile;
   constexpr int KS = C / 16, OT = C / 32, HCH = 4 * S;  // 16-byte chunks of a position's hidden slice
   constexpr int TASKS = P * 32 / LnLane<C>::PPI;        // LayerNorm instructions of a tile
@@ -255,10 +258,11 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
         if (P % GB != 0 && P > GB && pt >= P) break;  // wave-uniform
         const Lane at = lane_here();
         const int l32 = at.l32, lh = at.lh, j = j0 + 32 * pt + l32;
-        const u32x4_t* res = xr + pt * XTile::SLOTS;
+        u32x4_t* const s0 = xr + pt * XTile::SLOTS + XTile::slot(l32, 4 * ot + 2 * lh);
+        u32x4_t* const s1 = xr + pt * XTile::SLOTS + XTile::slot(l32, 4 * ot + 2 * lh + 1);
         float r0[8], r1[8];
-        unpack8(res[XTile::slot(l32, 4 * ot + 2 * lh)], r0);
-        unpack8(res[XTile::slot(l32, 4 * ot + 2 * lh + 1)], r1);
+        unpack8(*s0, r0);
+        unpack8(*s1, r1);
         if (!p.add_residual) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) r0[e] = r1[e] = 0.f;
@@ -268,11 +272,45 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
           r0[e] += oacc[q][e] * mtile[q];
           r1[e] += oacc[q][8 + e] * mtile[q];
         }
+        const u32x4_t o0 = pack8(r0), o1 = pack8(r1);
+        if (BIAS) *s0 = o0, *s1 = o1;
         if (j < L) {
           bf16_t* dst = p.out + b * p.x_view.stride_b + i * p.x_view.stride_r + j * p.x_view.stride_k + 32 * ot + 16 * lh;
-          *reinterpret_cast<u32x4_t*>(dst) = pack8(r0);
-          *reinterpret_cast<u32x4_t*>(dst + 8) = pack8(r1);
+          *reinterpret_cast<u32x4_t*>(dst) = o0;
+          *reinterpret_cast<u32x4_t*>(dst + 8) = o1;
         }
+      }
+    }
+    if constexpr (BIAS) {
+      LnLane<C> lb;
+      const int chunk = lane % LnLane<C>::NCH;
+      lb.w = *reinterpret_cast<const u32x4_t*>(pb.ln_w + 8 * chunk);
+      lb.b = u32x4_t{0u, 0u, 0u, 0u};
+      if (pb.ln_b) lb.b = *reinterpret_cast<const u32x4_t*>(pb.ln_b + 8 * chunk);
+      u32x4_t wh[KS];
+      const int head = lane & 31;
+      if (wave < P) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          wh[s] = u32x4_t{0u, 0u, 0u, 0u};
+          if (head < pb.H) wh[s] = *reinterpret_cast<const u32x4_t*>(pb.w + head * C + 16 * s + 8 * half);
+        }
+      }
+      __syncthreads();  // the tile's rows are complete
+#pragma unroll
+      for (int u = 0; u < LPW; ++u) {
+        if (wave + kWaves * u >= TASKS) continue;
+        const int slot = ln_slot(u);
+        xn[slot] = lb.template normalised<false>(xr[slot]);
+      }
+      __syncthreads();
+      if (wave < P) {
+        f32x16_t acc = zero16();
+#pragma unroll
+        for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(xn[wave * XTile::SLOTS + XTile::slot(arow, 2 * s + half)], wh[s], acc);
+        // lane (head, half): 16 positions
+        const int f = j0 + 32 * wave + 16 * half;
+        if (head < pb.H && f < L) store_run16(pb.out + ((int64_t)b * pb.H + head) * L + f, acc, L - f, L % 8 == 0);
       }
     }
     if (AFTER) return;
@@ -280,10 +318,10 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
   }
 }
 
-template <int C, int S, int P, bool AFTER = false>
-hipError_t launch(const TransitionArgs& a, hipStream_t stream, const TriattnOutArgs& end = {}) {
+template <int C, int S, int P, bool AFTER = false, bool BIAS = false>
+hipError_t launch(const TransitionArgs& a, hipStream_t stream, const TriattnOutArgs& end = {}, const PairBiasArgs& bias = {}) {
   constexpr size_t lds = lds_slots<C, S, P>() * 16;
-  constexpr auto kernel = transition_tiles<C, S, P, AFTER>;
+  constexpr auto kernel = transition_tiles<C, S, P, AFTER, BIAS>;
   static int cache[kMaxDevices];
   int fit = 0;
   hipError_t e = allow_dynamic_lds<kernel>(lds);
@@ -306,25 +344,30 @@ hipError_t launch(const TransitionArgs& a, hipStream_t stream, const TriattnOutA
   if (packed) k.w_a = a.operands[0], k.w_b = a.operands[1], k.w_out = a.operands[2];
   if (AFTER && (!packed || a.R != 1 || a.N != end.N * end.N || a.B != end.B)) return hipErrorInvalidValue;
   hipLaunchKernelGGL(kernel, dim3((unsigned)(AFTER || total < fit ? total : fit)), dim3(64 * kWaves), lds, stream, k, packed, tiles_per_row, (int)total,
-                     end, Division::by(AFTER ? end.N : 1));
+                     end, Division::by(AFTER ? end.N : 1), bias);
   return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t triattn_transition_tiles_launch(const TriattnOutArgs& end, const TransitionArgs& a, int C, int position_tiles, hipStream_t stream) {
+template <int C, bool BIAS>
+static hipError_t launch_after(const TriattnOutArgs& end, const TransitionArgs& a, const PairBiasArgs& bias, int position_tiles, hipStream_t stream) {
   const bool wide = a.HID % 256 == 0;
-  if (C == 64) {
-    if (position_tiles == 1) return wide ? launch<64, 8, 1, true>(a, stream, end) : launch<64, 4, 1, true>(a, stream, end);
-    return wide ? launch<64, 8, 2, true>(a, stream, end) : launch<64, 4, 2, true>(a, stream, end);
-  }
-  switch (position_tiles) {
-    case 1: return wide ? launch<128, 8, 1, true>(a, stream, end) : launch<128, 4, 1, true>(a, stream, end);
-    case 2: return wide ? launch<128, 8, 2, true>(a, stream, end) : launch<128, 4, 2, true>(a, stream, end);
-    case 4: return launch<128, 4, 4, true>(a, stream, end);
-    case 5: return launch<128, 4, 5, true>(a, stream, end);
+  if (position_tiles == 1)
+    return wide ? launch<C, 8, 1, true, BIAS>(a, stream, end, bias) : launch<C, 4, 1, true, BIAS>(a, stream, end, bias);
+  if (position_tiles == 2)
+    return wide ? launch<C, 8, 2, true, BIAS>(a, stream, end, bias) : launch<C, 4, 2, true, BIAS>(a, stream, end, bias);
+  if constexpr (C == 128) {
+    if (position_tiles == 4) return launch<128, 4, 4, true, BIAS>(a, stream, end, bias);
+    if (position_tiles == 5) return launch<128, 4, 5, true, BIAS>(a, stream, end, bias);
   }
   return hipErrorInvalidValue;
+}
+hipError_t triattn_transition_tiles_launch(const TriattnOutArgs& end, const TransitionArgs& a, const PairBiasArgs* bias, int C,
+                                           int position_tiles, hipStream_t stream) {
+  if (bias && (bias->B != a.B || bias->N * bias->N != a.N || bias->H > 32 || C != 128)) return hipErrorInvalidValue;
+  if (C == 64) return launch_after<64, false>(end, a, {}, position_tiles, stream);
+  return bias ? launch_after<128, true>(end, a, *bias, position_tiles, stream) : launch_after<128, false>(end, a, {}, position_tiles, stream);
 }
 
 hipError_t transition_tiles_launch(const TransitionArgs& a, int C, int position_tiles, hipStream_t stream) {

@@ -46,3 +46,17 @@ def test_template_tiles(monkeypatch, n_mult, n, batch):
     want = blocks._by_modules(monkeypatch, lambda: m(t, mask))
     assert torch.isfinite(want.float()).all()
     assert torch.equal(m(t, mask), want)
+
+
+@pytest.mark.parametrize("n,batch", [(1, 2), (16, 1), (45, 3), (90, 1), (91, 1), (128, 1), (61, 4), (131, 1), (179, 1), (202, 1), (203, 1)])
+def test_with_pair_bias(monkeypatch, n, batch):
+    """The pair bias of the attention over s as the end of the same launch: every alignment of a head's runs, ragged ends, one length beyond."""
+    m = blocks._fill(of3pair.PairFormerBlock(384, 128, 24, 16, 128, 32, 4), n).to("cuda").to(torch.bfloat16).eval()
+    gen = torch.Generator().manual_seed(n)
+    s = torch.randn(batch, n, 384, generator=gen).to("cuda").to(torch.bfloat16)
+    z = torch.randn(batch, n, n, 128, generator=gen).to("cuda").to(torch.bfloat16)
+    tok = (torch.rand(batch, n, generator=gen) > 0.2).float().to("cuda")
+    pair = tok[:, :, None] * tok[:, None, :]
+    want = blocks._by_modules(monkeypatch, lambda: m(s, z, tok, pair))
+    got = m(s, z, tok, pair)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
