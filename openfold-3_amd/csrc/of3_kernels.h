@@ -272,6 +272,7 @@ inline size_t trimul_wsplit_bytes(long C, long CH) {
   return (size_t)6 * (4 * wsplit_elems(CH, C) + wsplit_elems(C, C) + wsplit_elems(C, CH));
 }
 
+struct TriattnF32;  // of3_pair_f32.h
 struct TriattnF32Args {
   const float* x;
   const float* mask;                 // may be null
@@ -287,6 +288,8 @@ struct TriattnF32Args {
   float* out;
   int B, N, C, H, D, add_residual;
   float inf;
+  // where not null and the output pass is triattn_out_pass_f32's, its arguments, and it is left to the caller (o stays null otherwise)
+  TriattnF32* deferred = nullptr;
 };
 hipError_t triattn_fwd_f32(const TriattnF32Args& args, hipStream_t stream);
 inline size_t triattn_wsplit_bytes(long C, long H, long D) {
@@ -307,6 +310,8 @@ struct TransitionF32Args {
   const WeightX3* presplit = nullptr;
   float* out;
   int B, N, C, HID, add_residual;
+  // the deferred output pass of the ending node's attention on x, to be done first (in place: x is its result), or null
+  const TriattnF32* end = nullptr;
 };
 // the three weight matrices split into three bf16 terms each, rows padded to multiples of 32
 inline size_t transition_wsplit_bytes(long C, long HID) {

@@ -70,6 +70,7 @@ hipError_t triattn_proj_pass_f32(const TriattnF32& p, hipStream_t stream);
 hipError_t triattn_out_pass_f32(const TriattnF32& p, hipStream_t stream);
 // the pair transition likewise (transition_f32.hip)
 bool transition_pass_serves(const TransitionF32Args& a);
+bool transition_pass_takes(const TransitionF32Args& a);  // a.end, as the beginning of its launch
 hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, const WeightX3& s_b, const WeightX3& s_out,
                                hipStream_t stream);
 

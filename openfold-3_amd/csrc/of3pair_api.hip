@@ -196,6 +196,7 @@ struct ModuleEnd {
   enum { kMul, kAtt } is;
   of3::TrimulOutArgs mul;
   of3::TriattnOutArgs att;
+  of3::TriattnF32 att_f32;  // fp32: o is null where the pass has not been deferred
 };
 
 static int trimul_proj(int packed, const void* z, const int64_t z_strides[3], const float* mask,
@@ -557,6 +558,10 @@ static int triattn_fwd(const of3::WeightX3* presplit, int packed, const void* x,
     a.D = (int)D;
     a.add_residual = add_residual ? 1 : 0;
     a.inf = inf;
+    if (deferred) {
+      deferred->att_f32.o = nullptr;
+      a.deferred = &deferred->att_f32;
+    }
     hipError_t e = of3::triattn_fwd_f32(a, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? OF3_OK : (e == hipErrorInvalidValue ? (int)OF3_EINVAL : fail_hip(e));
   }
@@ -643,6 +648,8 @@ static int transition_fwd(const of3::WeightX3* presplit, const void* const* oper
     a.C = (int)C;
     a.HID = (int)HID;
     a.add_residual = add_residual ? 1 : 0;
+    if (before && before->att_f32.o) a.end = &before->att_f32;
+    if (takes_end) return OF3_OK;
     hipError_t e = of3::transition_fwd_f32(a, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? OF3_OK : fail_hip(e);
   }
@@ -1130,7 +1137,7 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
   // the end of the module before, and where this one leaves its own
   auto before = [&] { return joined && module > 0 ? &ends[(module - 1) & 1] : nullptr; };
   bool last_joined = false;  // the last module with the transition
-  auto after = [&] { return joined && (module < 3 || last_joined) ? &ends[module & 1] : nullptr; };
+  auto after = [&] { return (joined && module < 3) || (last_joined && module == 3) ? &ends[module & 1] : nullptr; };
   auto trimul = [&](int m) {
     const void* const* w = k.w + 10 * m;
     const int st = trimul_fwd(k.mul ? k.mul + m * of3::kTrimulMatrices : nullptr, k.packed, src, z_strides, mask, mask_strides,
@@ -1160,11 +1167,12 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
   };
   int st = OF3_OK;
   if (joined && !attention_first && d.HID != 0) st = transition(nullptr, &last_joined);
+  if (d.wide() && k.tr && !attention_first && d.HID != 0) last_joined = true;  // if both can; else transition_fwd_f32 takes them one by one
   for (int part = 0; part < 2; ++part)
     for (int m = 0; m < 2 && st == OF3_OK; ++m)
       st = (part == 0) == !attention_first ? trimul(m) : triattn(m);
   if (st != OF3_OK || d.HID == 0) return st;
-  if (bias_done) *bias_done = bias && last_joined;
+  if (bias_done) *bias_done = bias && last_joined && !d.wide();
   return transition(last_joined ? &ends[3 & 1] : nullptr, nullptr);
 }
 

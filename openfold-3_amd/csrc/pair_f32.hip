@@ -2540,6 +2540,10 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
     }
     hipLaunchKernelGGL(core, dim3((unsigned)cblocks), dim3(kThreads), 0, stream, p, qgroups);
   }
+  if (pass && a.deferred) {
+    *a.deferred = p;
+    return hipGetLastError();
+  }
   if (pass) return triattn_out_pass_f32(p, stream);
   if (x3) {
     const int HD = a.H * a.D;
@@ -2557,8 +2561,13 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-hipError_t transition_fwd_f32(const TransitionF32Args& a, hipStream_t stream) {
+hipError_t transition_fwd_f32(const TransitionF32Args& args, hipStream_t stream) {
+  TransitionF32Args a = args;
   if (a.C > kMaxC || a.HID > kMaxHid) return hipErrorInvalidValue;
+  if (a.end && !(a.presplit && transition_split_widths(a.C, a.HID) && transition_pass_serves(a) && transition_pass_takes(a))) {
+    if (hipError_t e = triattn_out_pass_f32(*a.end, stream); e != hipSuccess) return e;
+    a.end = nullptr;
+  }
   TransitionF32 p;
   p.x = a.x;
   p.mask = a.mask;

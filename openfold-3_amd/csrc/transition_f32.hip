@@ -29,15 +29,24 @@ struct TransitionPass {
   int panels;   // 32-position panels per row
   int total;    // panels in all
   int HID, add_residual;
+  // the attention before it (AFTER)
+  const float *att_o, *att_ln_w, *att_ln_b;
+  WeightX3 att_g, att_out;
+  int N;
 };
 
-template <int C, int S, int NPT>
+constexpr int kRowLd = 4;  // floats between the rows of the updated tile, beside their channels
+template <int C, int S, int NPT, bool AFTER>
 constexpr size_t transition_lds() {
-  return (size_t)NPT * (PassTile<C>::SLOTS + PassTile<32 * S>::SLOTS) * 16 + 2 * C * sizeof(float);
+  return (size_t)NPT * (PassTile<C>::SLOTS + PassTile<32 * S>::SLOTS) * 16 + 2 * C * sizeof(float) +
+         (AFTER ? (2 * C + 32 * (C + kRowLd)) * sizeof(float) : 0);
 }
 
-template <int C, int S, int NPT>
+// AFTER: the tile begins with the output pass of the ending node's triangle attention (triattn_out_pass: same steps, same bits), its gates in
+// the first four waves and its output projection in the others; the updated rows stay in LDS.
+template <int C, int S, int NPT, bool AFTER>
 __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
+  static_assert(!AFTER || (C == 128 && NPT == 1), "eight waves: a gate and an output tile for each 32 channels");
   static_assert(S == 8 || (S == 4 && NPT == 2), "eight waves share the hidden tiles of a slice");
   typedef PassTile<C> XTile;
   typedef PassTile<32 * S> HTile;
@@ -97,8 +106,79 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
   const int tiles = (p.total + NPT - 1) / NPT;
   int tile = grid_slot();
   if (tile < tiles) load_tile(tile);
+  float* const att_ln = ln + 2 * C;         // [2][C]
+  float* const rows = att_ln + 2 * C;       // [32][C + kRowLd]
+  if (AFTER)
+    for (int c = tid; c < C; c += 64 * NW) att_ln[c] = p.att_ln_w[c], att_ln[C + c] = p.att_ln_b[c];
   __syncthreads();
   for (; tile < tiles; tile += gridDim.x) {
+    if constexpr (AFTER) {
+      const XTile xn = {lds}, gated = {hid};
+      u32x4_t w[KS][3];
+      load_unit<C, 3>(kh == 0 ? p.att_g : p.att_out, ot, src_lane, w);
+      int j0;
+      const int b = row_of(tile, j0);  // one row per batch element
+      const Lane here = lane_here();
+      float4 o[4];
+      if (kh == 0) {
+        const int f = j0 + here.l32 < L ? j0 + here.l32 : L - 1, r = f / p.N, k = f - r * p.N;
+        const float* src = p.att_o + (((size_t)b * p.N + k) * p.N + r) * C + 32 * ot + 16 * here.lh;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) o[a] = *reinterpret_cast<const float4*>(src + 4 * a);
+      }
+      // the operands of a step are read one step ahead, no further: all of them do not fit the registers
+      auto product = [&](const XTile& t) {
+        f32x16_t acc = zero16();
+        u32x4_t nxt[3];
+        const Lane at = lane_here();
+        auto read = [&](int s) {
+          const u32x4_t* x = t.s + XTile::slot(at.l32, 2 * s + at.lh);
+          nxt[0] = x[0], nxt[1] = x[XTile::PLANE], nxt[2] = x[2 * XTile::PLANE];
+        };
+        read(0);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const u32x4_t op[3] = {nxt[0], nxt[1], nxt[2]};
+          if (s + 1 < KS) read(s + 1);
+          __builtin_amdgcn_sched_barrier(0);
+          acc = step6<true>(w[s], op, acc);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        return acc;
+      };
+      const int pos = 4 * wave + here.lg;
+      float4 y[C / 64];
+      norm_row<C>(raw[0], j0 + pos < L, att_ln, here.li, y);
+#pragma unroll
+      for (int e = 0; e < C / 64; ++e) {
+        xn.store4(pos, here.li + 16 * e, y[e]);
+        *reinterpret_cast<float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li) = raw[0].v[e];
+      }
+      __syncthreads();
+      if (kh == 0) {
+        const f32x16_t gate = product(xn);
+        const Lane mid = lane_here();
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+          const float4 o0 = o[2 * hf], o1 = o[2 * hf + 1];
+          const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
+          float g[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) g[e] = ov[e] * sigmoid_hw_f32(gate[8 * hf + e]);
+          gated.store8(mid.l32, 4 * ot + 2 * mid.lh + hf, g);
+        }
+      }
+      __syncthreads();
+      if (kh > 0) {
+        const f32x16_t acc = product(gated);
+        const Lane mid = lane_here();
+        float* row = rows + mid.l32 * (C + kRowLd) + 32 * ot + 16 * mid.lh;
+        store_row16(row, row, acc, 1);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < C / 64; ++e) raw[0].v[e] = *reinterpret_cast<const float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li);
+    }
     {
       const Lane here = lane_here();
 #pragma unroll
@@ -188,8 +268,9 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
           if (s + 1 < OSTEPS) read_h(s + 1);
           if (s + DO < OSTEPS) fetch_o(slice, s + DO);
           if (s + DO == OSTEPS) {  // after the last weights: loads return in order
-            if (last) load_tile(tile + (int)gridDim.x < tiles ? tile + gridDim.x : tile);
-            else
+            if (last) {
+              if (!AFTER) load_tile(tile + (int)gridDim.x < tiles ? tile + gridDim.x : tile);
+            } else
 #pragma unroll
               for (int q = 0; q < DA; ++q) fetch_ab(slice + 1, q);
           }
@@ -224,19 +305,29 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) oacc[v] *= m;
       }
-      store_row16(p.x + off, p.out + off, oacc, p.add_residual);
+      store_row16(AFTER ? rows + at.l32 * (C + kRowLd) + 32 * ot + 16 * at.lh : p.x + off, p.out + off, oacc, p.add_residual);
     }
+    if (AFTER) return;
   }
 }
 
-template <int C, int S, int NPT>
+template <int C, int S, int NPT, bool AFTER = false>
 hipError_t launch(const TransitionPass& p, hipStream_t stream) {
-  constexpr size_t lds = transition_lds<C, S, NPT>();
+  constexpr size_t lds = transition_lds<C, S, NPT, AFTER>();
   unsigned grid = 0;
-  hipError_t e = resident_grid<transition_pass<C, S, NPT>>(512, lds, (p.total + NPT - 1) / NPT, &grid);
+  hipError_t e = resident_grid<transition_pass<C, S, NPT, AFTER>>(512, lds, (p.total + NPT - 1) / NPT, &grid);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((transition_pass<C, S, NPT>), dim3(grid), dim3(512), lds, stream, p);
+  if (AFTER) grid = (unsigned)p.total;  // a tile each
+  hipLaunchKernelGGL((transition_pass<C, S, NPT, AFTER>), dim3(grid), dim3(512), lds, stream, p);
   return hipGetLastError();
+}
+
+hipError_t device_cus(int* cus) {
+  static int cache[kMaxDevices];
+  return per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, cus);
+}
+bool flat_rows(const TransitionF32Args& a) {
+  return a.x_view.stride_r == a.N * a.x_view.stride_k && (!a.mask || a.mask_view.stride_r == a.N * a.mask_view.stride_k);
 }
 
 }  // namespace
@@ -244,6 +335,15 @@ hipError_t launch(const TransitionPass& p, hipStream_t stream) {
 bool transition_pass_serves(const TransitionF32Args& a) {
   return (a.C == 64 || a.C == 128) && a.HID % 128 == 0 && rows_aligned(a.x, a.x_view) && rows_aligned(a.out, a.x_view) &&
          (long)a.B * a.N * ((a.N + 31) / 32) <= 0x3fffffffL;
+}
+
+// Up to one tile of 32 positions per CU: the launch, z's way to memory and back and the wait for the first tile that it saves.  Four
+// trunk blocks at N = 45 / 64 / 80 / 90 586 / 597 / 705 / 780 us, so 578 / 588 / 696 / 758; with more tiles, 110 / 128, 940 / 975 and 945 / 975.
+bool transition_pass_takes(const TransitionF32Args& a) {
+  int cus = 0;
+  return device_cus(&cus) == hipSuccess && a.C == 128 && a.HID % 256 == 0 && flat_rows(a) && a.end->C == 128 && a.end->N == a.N &&
+         a.end->B == a.B && a.end->add_residual && a.end->out == a.x && a.x == a.out && a.add_residual &&
+         (long)a.B * (((long)a.N * a.N + 31) / 32) <= cus;
 }
 
 hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, const WeightX3& s_b, const WeightX3& s_out,
@@ -260,17 +360,25 @@ hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, 
   p.s_out = s_out;
   p.out = a.out;
   // a tensor (and mask) whose rows follow one another without gaps is one row of N * N positions
-  const bool flat = a.x_view.stride_r == a.N * a.x_view.stride_k && (!a.mask || a.mask_view.stride_r == a.N * a.mask_view.stride_k);
+  const bool flat = flat_rows(a);
   p.R = flat ? 1 : a.N;
   p.L = flat ? a.N * a.N : a.N;
   p.panels = (p.L + 31) / 32;
   p.total = a.B * p.R * p.panels;
   p.HID = a.HID;
   p.add_residual = a.add_residual;
-  static int cache[kMaxDevices];
   int cus = 0;
-  const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  const hipError_t e = device_cus(&cus);
   if (e != hipSuccess) return e;
+  if (a.end) {  // transition_pass_takes
+    p.att_o = a.end->o;
+    p.att_ln_w = a.end->ln_w;
+    p.att_ln_b = a.end->ln_b;
+    p.att_g = a.end->s_g;
+    p.att_out = a.end->s_o;
+    p.N = a.N;
+    return launch<128, 8, 1, true>(p, stream);
+  }
   const bool large = p.total >= 4l * cus;  // two tiles of 64 positions for every CU
   if (a.HID % 256 != 0) return a.C == 128 ? launch<128, 4, 2>(p, stream) : launch<64, 4, 2>(p, stream);
   if (a.C == 128) return large ? launch<128, 8, 2>(p, stream) : launch<128, 8, 1>(p, stream);

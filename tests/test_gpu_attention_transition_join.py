@@ -60,3 +60,21 @@ def test_with_pair_bias(monkeypatch, n, batch):
     want = blocks._by_modules(monkeypatch, lambda: m(s, z, tok, pair))
     got = m(s, z, tok, pair)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("n_mult", [1, 2, 4, 6])
+@pytest.mark.parametrize("n,batch", [(1, 1), (31, 2), (45, 1), (64, 2), (90, 1), (91, 1)])
+def test_fp32(monkeypatch, n_mult, n, batch):
+    """transition_pass, AFTER, up to a tile of 32 positions per CU, and beyond; hidden slices of 256 (n_mult 1: slices of 128, apart)."""
+    m = blocks._fill(of3pair.PairBlock(128, 128, 32, 4, transition_n=n_mult), n).to("cuda").eval()
+    gen = torch.Generator().manual_seed(n)
+    z = torch.randn(batch, n, n, 128, generator=gen).to("cuda")
+    mask = (torch.rand(batch, n, n, generator=gen) > 0.2).float().to("cuda")
+    wide = torch.zeros(batch, n, n + 3, 128, device="cuda")
+    wide[:, :, :n] = z
+    for x, mk, mask_trans in ((z, mask, True), (z, None, True), (z, mask, False), (wide[:, :, :n], mask, True)):
+        want = blocks._by_modules(monkeypatch, lambda: m(x, mk, _mask_trans=mask_trans))
+        assert torch.equal(m(x, mk, _mask_trans=mask_trans), want)
+    own = z.clone()
+    m(own, mask, inplace_safe=True)
+    assert torch.equal(own, blocks._by_modules(monkeypatch, lambda: m(z, mask)))
