@@ -1280,7 +1280,7 @@ int of3_pairformer_block_fwd(const void* const* weights, const void* s, const vo
 
 // ---- a stack of PairFormerBlocks in one call --------------------------------------------------
 // The pair representation of block i + 1 needs nothing of block i's single representation: with a second stream the
-// attention and transition of s (44 us per block at 40 tokens, of 148) run beside the next block's pair updates, which
+// attention and transition of s (33 us per block at 40 tokens, of 102) run beside the next block's pair updates, which
 // do not fill the chip at the lengths where that time counts.
 
 // Two streams of one call and the order between them; without a second stream nothing to order.  An event waited for on
