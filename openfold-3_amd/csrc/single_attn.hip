@@ -25,7 +25,7 @@
 //     operands requested before the current tile's arithmetic, running
 //     maximum and sum in fp32, O^T = V^T P^T with P^T taken from the S^T registers; the result
 //     is divided by the sum, multiplied by the gate and written as [B][N][H*D].
-//  3. single_out: the same tiling as 1 without the LayerNorm: out = [a +] og Wo^T.
+//  3. single_out: a wave per 32 x 32 tile, no LayerNorm, no LDS: out = [a +] og Wo^T.
 #include "of3_device.h"
 #include "of3_kernels.h"
 #include "of3_rowtile.h"
@@ -242,44 +242,38 @@ __global__ __launch_bounds__(64 * kSplit) void single_attn_kernel(SingleAttnArgs
 }
 
 // ---- 3. output projection ----------------------------------------------------------------
-__global__ __launch_bounds__(256) void single_out_kernel(SingleAttnArgs p) {
-  __shared__ u32x4_t act[32 * kChunks];
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
-  const int N = p.N;
-  const int b = blockIdx.z;
-  const long pos0 = (long)blockIdx.x * 32;
-  fill_tile<false>(act, p.og + (size_t)b * N * kK, kK, pos0, N, nullptr, nullptr, wave, lane);
-  __syncthreads();
-  const long pos = pos0 + l32;
-  for (int tile = blockIdx.y * 4 + wave; tile < kK / 32; tile += gridDim.y * 4) {
-    const f32x16_t acc = tile_product<true>(act, p.wo + (size_t)(32 * tile + rowperm16(l32)) * kK, l32, lh);
-    if (pos < N) {
-      const size_t off = ((size_t)b * N + pos) * kK + 32 * tile + 16 * lh;
-      float f[16];
+// One wave per 32 rows x 32 outputs, both operands straight from memory.  With the rows in an LDS tile for four waves of one output tile each,
+// 21 work-groups at 200 rows, the fill, the barrier and then the weights' trip were in a row: the attention's three kernels at 24 / 64 / 200 / 384 /
+// 768 rows 22.3 / 22.0 / 26.4 / 33.7 / 55.5 us, so 19.8 / 19.6 / 23.7 / 30.8 / 54.1.
+__global__ __launch_bounds__(64) void single_out_kernel(SingleAttnArgs p) {
+  const int lane = threadIdx.x, l32 = lane & 31, lh = lane >> 5;
+  const int N = p.N, b = blockIdx.z, tile = blockIdx.y;
+  const long pos = (long)blockIdx.x * 32 + l32;
+  const bf16_t* x_row = p.og + ((size_t)b * N + (pos < N ? pos : N - 1)) * kK;
+  const f32x16_t acc = row_product(x_row, p.wo + (size_t)(32 * tile + rowperm16(l32)) * kK, lh, zero16());
+  if (pos >= N) return;
+  const size_t off = ((size_t)b * N + pos) * kK + 32 * tile + 16 * lh;
+  float f[16];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) f[v] = acc[v];
-      if (p.add_residual) {
-        // the reference adds the module's bf16 output to s: round before the add
-        u32x4_t r[2];
-        load16_raw(p.a + off, 0, 16, true, r);
+  for (int v = 0; v < 16; ++v) f[v] = acc[v];
+  if (p.add_residual) {
+    // the reference adds the module's bf16 output to s: round before the add
+    u32x4_t r[2];
+    load16_raw(p.a + off, 0, 16, true, r);
 #pragma unroll
-        for (int w = 0; w < 8; ++w) {
-          f[2 * w] = bf16_to_f32(to_bf16(f[2 * w])) + bf16_lo(r[w >> 2][w & 3]);
-          f[2 * w + 1] = bf16_to_f32(to_bf16(f[2 * w + 1])) + bf16_hi(r[w >> 2][w & 3]);
-        }
-      }
-      u32x4_t o0, o1;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        o0[w] = pack_bf16(f[2 * w], f[2 * w + 1]);
-        o1[w] = pack_bf16(f[8 + 2 * w], f[8 + 2 * w + 1]);
-      }
-      *reinterpret_cast<u32x4_t*>(p.out + off) = o0;
-      *reinterpret_cast<u32x4_t*>(p.out + off + 8) = o1;
+    for (int w = 0; w < 8; ++w) {
+      f[2 * w] = bf16_to_f32(to_bf16(f[2 * w])) + bf16_lo(r[w >> 2][w & 3]);
+      f[2 * w + 1] = bf16_to_f32(to_bf16(f[2 * w + 1])) + bf16_hi(r[w >> 2][w & 3]);
     }
   }
+  u32x4_t o0, o1;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    o0[w] = pack_bf16(f[2 * w], f[2 * w + 1]);
+    o1[w] = pack_bf16(f[8 + 2 * w], f[8 + 2 * w + 1]);
+  }
+  *reinterpret_cast<u32x4_t*>(p.out + off) = o0;
+  *reinterpret_cast<u32x4_t*>(p.out + off + 8) = o1;
 }
 
 }  // namespace
@@ -298,7 +292,7 @@ hipError_t single_attn_launch(const SingleAttnArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL(single_attn_kernel, dim3(row_blocks, a.H, a.B), dim3(64 * kSplit), 0, stream, a, row_blocks);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(single_out_kernel, dim3(row_blocks, 3, a.B), dim3(256), 0, stream, a);
+  hipLaunchKernelGGL(single_out_kernel, dim3(row_blocks, kK / 32, a.B), dim3(64), 0, stream, a);
   return hipGetLastError();
 }
 
