@@ -47,6 +47,9 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
   // (tiles pt_a, pt_a + GA ... and pt_b, pt_b + GB ...; the two waves of a SIMD differ in pt_a and pt_b)
   constexpr int GA = kWaves / S, GB = kWaves / OT, APT = (P + GA - 1) / GA, BPT = (P + GB - 1) / GB;
   static_assert(S == 8 || S == 4, "");
+  // The next slice's first weights requested before the slice's barrier, where the registers are there (one tile per work-group): four trunk blocks
+  // at N = 140 / 160 / 180 569 / 601 / 675 us, so 561 / 593 / 666; 128 and 200 451 and 801, 449 and 799; with one position tile no difference.
+  constexpr bool EARLY = AFTER && P > 1;
   extern __shared__ u32x4_t lds[];
   u32x4_t* const xn = lds;                             // [P][XTile::SLOTS] LayerNorm(x)
   u32x4_t* const xr = xn + P * XTile::SLOTS;           // x as loaded: the residual
@@ -235,8 +238,9 @@ __global__ __launch_bounds__(64 * kWaves) void transition_tiles(TransitionArgs p
           }
         }
       }
+      if (EARLY && first && slice + 1 < slices) load_first(slice + 1);
       __syncthreads();  // the slice is complete, and nobody reads the one before any more
-      if (first) load_first(slice + 1 < slices ? slice + 1 : 0);
+      if (!EARLY && first) load_first(slice + 1 < slices ? slice + 1 : 0);
       if (!AFTER && slice + 1 == slices) load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
       if (second) {
 #pragma unroll
