@@ -312,6 +312,9 @@ struct TransitionF32Args {
   int B, N, C, HID, add_residual;
   // the deferred output pass of the ending node's attention on x, to be done first (in place: x is its result), or null
   const TriattnF32* end = nullptr;
+  // where `end` is, a pair bias of the result to go with the launch if it can: *bias_done says whether it did
+  const struct PairBiasF32Args* bias = nullptr;
+  bool* bias_done = nullptr;
 };
 // the three weight matrices split into three bf16 terms each, rows padded to multiples of 32
 inline size_t transition_wsplit_bytes(long C, long HID) {

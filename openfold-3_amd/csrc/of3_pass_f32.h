@@ -118,6 +118,16 @@ __device__ __forceinline__ void load_unit(const WeightX3& W, int t, int lane_src
     for (int pl = 0; pl < TERMS; ++pl) w[s][pl] = src[pl * (W.plane / 8) + 64 * s];
 }
 
+// rows of a fp32 weight matrix as split MFMA operands: k-values 16 s + 8 lh .. + 7 of `row`
+__device__ __forceinline__ void split_operand(const float* row, int s, int lh, u32x4_t (&w)[3]) {
+  const float4 u = *reinterpret_cast<const float4*>(row + 16 * s + 8 * lh);
+  const float4 v = *reinterpret_cast<const float4*>(row + 16 * s + 8 * lh + 4);
+  const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+  split8(x, w[0], w[1], w[2]);
+}
+
+constexpr int kBiasLd = 36;  // floats per head row of the pair bias's partial tiles
+
 // one k-step: six products, smallest terms first (one chain of dependent MFMAs: two alternating chains were no
 // faster, their second accumulator is what some of the kernels spill for).  W_ROWS: the outputs are the MFMA rows,
 // otherwise the positions

@@ -611,11 +611,17 @@ int of3_transition_fwd(const void* x, const int64_t x_strides[3], const float* m
 
 // presplit as above; operands: w_a, w_b, w_out in MFMA operand order (bf16), or null.  before: the attention whose output pass the
 // launch begins with; takes_end: says whether it could, and launches nothing; bias: a pair bias of the result that goes with `before`
+// A block's pair bias of the attention over s, to go with its last pair launch
+struct BlockBias {
+  of3::PairBiasArgs bf16;
+  of3::PairBiasF32Args f32;
+};
+
 static int transition_fwd(const of3::WeightX3* presplit, const void* const* operands, const void* x, const int64_t x_strides[3], const float* mask,
                           const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_a, const void* w_b, const void* w_out,
                           void* out, int64_t B, int64_t N, int64_t C, int64_t HID, int add_residual, void* workspace,
                           int64_t workspace_bytes, int dtype, void* stream, const ModuleEnd* before = nullptr, bool* takes_end = nullptr,
-                          const of3::PairBiasArgs* bias = nullptr) {
+                          const BlockBias* bias = nullptr, bool* bias_done = nullptr) {
   if (takes_end) *takes_end = false;
   const void* ptrs[] = {x, ln_w, ln_b, w_a, w_b, w_out, out};
   if (!positions_ok(B, N) || !mask_ok(mask, mask_strides)) return OF3_EINVAL;
@@ -650,6 +656,7 @@ static int transition_fwd(const of3::WeightX3* presplit, const void* const* oper
     a.add_residual = add_residual ? 1 : 0;
     if (before && before->att_f32.o) a.end = &before->att_f32;
     if (takes_end) return OF3_OK;
+    if (a.end && bias) a.bias = &bias->f32, a.bias_done = bias_done;
     hipError_t e = of3::transition_fwd_f32(a, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? OF3_OK : fail_hip(e);
   }
@@ -692,8 +699,9 @@ static int transition_fwd(const of3::WeightX3* presplit, const void* const* oper
     const hipError_t e = operands && rows == 1 ? of3::transition_after_attention(args, (int)C, takes_end) : hipSuccess;
     return e == hipSuccess ? OF3_OK : fail_hip(e);
   }
-  hipError_t e = before ? of3::triattn_transition_launch(before->att, args, bias, (int)C, static_cast<hipStream_t>(stream))
+  hipError_t e = before ? of3::triattn_transition_launch(before->att, args, bias ? &bias->bf16 : nullptr, (int)C, static_cast<hipStream_t>(stream))
                         : of3::transition_launch(args, (int)C, static_cast<hipStream_t>(stream));
+  if (before && bias) *bias_done = true;
   return e == hipSuccess ? OF3_OK : fail_hip(e);
 }
 
@@ -1118,10 +1126,10 @@ static hipError_t prepare_blocks(const void* const* const* weights, int n, const
 }
 
 // bias: where the launches allow it, the pair bias of the result goes with the last of them (*bias_done).  Its output may be the beginning of
-// the workspace, as large as a triangle multiplication's: nothing of that is read by then.
+// the workspace, no larger than a triangle multiplication's planes (bf16) or an attention's q, k and v (fp32): none of these is read by then.
 static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void* z, const int64_t z_strides[3],
                           const float* mask, const int64_t mask_strides[3], void* out, int flags, void* workspace,
-                          int64_t workspace_bytes, void* stream, const of3::PairBiasArgs* bias = nullptr, bool* bias_done = nullptr) {
+                          int64_t workspace_bytes, void* stream, const BlockBias* bias = nullptr, bool* bias_done = nullptr) {
   const void* src = z;  // the first module reads z, every later one updates out in place
   int rows = 0;
   if (k.packed && d.CH == d.C && d.H == 4 && 4 * d.D == d.C && join_room(d.dtype, d.B, d.N)) {
@@ -1163,7 +1171,7 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
     const void* const* w = k.w + 36;
     return transition_fwd(k.tr, d.wide() ? nullptr : k.tr_operands, out, z_strides, flags & OF3_BLOCK_TRANSITION_UNMASKED ? nullptr : mask,
                           mask_strides, w[0], w[1], w[2], w[3], w[4], out, d.B, d.N, d.C, d.HID, 1, d.wide() ? workspace : nullptr,
-                          d.wide() ? workspace_bytes : 0, d.dtype, stream, end, takes_end, end ? bias : nullptr);
+                          d.wide() ? workspace_bytes : 0, d.dtype, stream, end, takes_end, end ? bias : nullptr, bias_done);
   };
   int st = OF3_OK;
   if (joined && !attention_first && d.HID != 0) st = transition(nullptr, &last_joined);
@@ -1172,7 +1180,6 @@ static int run_pair_block(const BlockWeights& k, const BlockDims& d, const void*
     for (int m = 0; m < 2 && st == OF3_OK; ++m)
       st = (part == 0) == !attention_first ? trimul(m) : triattn(m);
   if (st != OF3_OK || d.HID == 0) return st;
-  if (bias_done) *bias_done = bias && last_joined && !d.wide();
   return transition(last_joined ? &ends[3 & 1] : nullptr, nullptr);
 }
 
@@ -1197,7 +1204,7 @@ int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t 
 static int pair_block_fwd(const void* const* weights, const void* z, const int64_t z_strides[3], const float* mask,
                           const int64_t mask_strides[3], void* out, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H,
                           int64_t D, int64_t HID, float inf, int flags, void* workspace, int64_t workspace_bytes, int dtype,
-                          void* stream, const of3::PairBiasArgs* bias = nullptr, bool* bias_done = nullptr) {
+                          void* stream, const BlockBias* bias = nullptr, bool* bias_done = nullptr) {
   const int64_t need = of3_pair_block_workspace_bytes(dtype, B, N, C, CH, H, D, HID);
   const BlockDims d = {dtype, B, N, C, CH, H, D, HID, inf};
   if (need < 0 || !pair_block_args_ok(d, weights, z, z_strides, mask, mask_strides, out, workspace)) return OF3_EINVAL;
@@ -1228,9 +1235,25 @@ int64_t of3_pairformer_block_workspace_bytes(int dtype, int64_t B, int64_t N, in
 }
 
 // A block's pair bias, to go with its last pair launch; what of3_pair_bias_fwd would refuse, or the launch cannot take, is left to that call
-static bool block_bias_args(const BlockDims& d, const void* const* ws_, int64_t H_s, void* out, of3::PairBiasArgs* a) {
-  if (d.dtype != OF3_DTYPE_BF16 || d.C != 128 || H_s < 1 || H_s > 32 || !ws_[0] || !ws_[2] || !out) return false;
+static bool block_bias_args(const BlockDims& d, const void* const* ws_, int64_t H_s, const void* z, const int64_t z_strides[3], void* out,
+                            BlockBias* bias) {
+  if (d.C != 128 || H_s < 1 || H_s > 32 || !ws_[0] || !ws_[2] || !out) return false;
   if (!aligned16(ws_[0]) || !aligned16(ws_[1]) || !aligned16(ws_[2]) || !aligned16(out)) return false;
+  if (d.wide()) {
+    of3::PairBiasF32Args* a = &bias->f32;
+    a->z = static_cast<const float*>(z);
+    a->z_view = view(z_strides, false);
+    a->ln_w = static_cast<const float*>(ws_[0]);
+    a->ln_b = static_cast<const float*>(ws_[1]);
+    a->w = static_cast<const float*>(ws_[2]);
+    a->out = static_cast<float*>(out);
+    a->B = (int)d.B;
+    a->N = (int)d.N;
+    a->C = (int)d.C;
+    a->H = (int)H_s;
+    return true;
+  }
+  of3::PairBiasArgs* a = &bias->bf16;
   a->z = nullptr;  // the launch's own result
   a->ln_w = bf(ws_[0]);
   a->ln_b = bf(ws_[1]);
@@ -1260,9 +1283,9 @@ int of3_pairformer_block_fwd(const void* const* weights, const void* s, const vo
   const void* const* ws_ = weights + OF3_PAIR_BLOCK_WEIGHTS;
   if (!single_args_ok(d, ws_, s, s_out, single_mask)) return OF3_EINVAL;
   if (workspace_bytes < need) return OF3_ENOSPC;
-  of3::PairBiasArgs bias;
+  BlockBias bias;
   bool bias_done = false;
-  const bool with_bias = block_bias_args(d, ws_, H_s, workspace, &bias);
+  const bool with_bias = block_bias_args(d, ws_, H_s, z_out, z_strides, workspace, &bias);
   int st = pair_block_fwd(weights, z, z_strides, pair_mask, mask_strides, z_out, B, N, C, CH, H, D, HID, inf, flags,
                           workspace, workspace_bytes, dtype, stream, with_bias ? &bias : nullptr, &bias_done);
   if (st != OF3_OK) return st;
@@ -1391,9 +1414,9 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
     }
     const void* const* ws_ = weights[i] + OF3_PAIR_BLOCK_WEIGHTS;
     void* const bias = bias0 + (i % w.buffers) * w.bias;
-    of3::PairBiasArgs bias_args;
+    BlockBias bias_args;
     bool bias_done = false;
-    const bool with_bias = i < w.buffers && block_bias_args(d, ws_, H_s, bias, &bias_args);  // else its buffer has to be waited for
+    const bool with_bias = i < w.buffers && block_bias_args(d, ws_, H_s, z_out, z_strides, bias, &bias_args);  // else its buffer has to be waited for
     auto attention = [&](int phases, hipStream_t on) {
       return attn_pair_bias(phases, i ? s_out : s, bias, single_mask, ws_[3], ws_[4], ws_[5], ws_[6], ws_[7], ws_[8], ws_[9],
                             ws_[10], s_out, B, N, C_s, H_s, D_s, inf_s, 1, single, w.single, dtype, on);

@@ -2567,6 +2567,7 @@ hipError_t transition_fwd_f32(const TransitionF32Args& args, hipStream_t stream)
   if (a.end && !(a.presplit && transition_split_widths(a.C, a.HID) && transition_pass_serves(a) && transition_pass_takes(a))) {
     if (hipError_t e = triattn_out_pass_f32(*a.end, stream); e != hipSuccess) return e;
     a.end = nullptr;
+    a.bias = nullptr;
   }
   TransitionF32 p;
   p.x = a.x;

@@ -13,18 +13,9 @@ namespace {
 
 using namespace pass_f32;
 
-// rows of a fp32 weight matrix as split MFMA operands: k-values 16 s + 8 lh .. + 7 of `row`
-__device__ __forceinline__ void split_operand(const float* row, int s, int lh, u32x4_t (&w)[3]) {
-  const float4 u = *reinterpret_cast<const float4*>(row + 16 * s + 8 * lh);
-  const float4 v = *reinterpret_cast<const float4*>(row + 16 * s + 8 * lh + 4);
-  const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-  split8(x, w[0], w[1], w[2]);
-}
-
 // ---- out[b][h][i][j] = LN(z[b,i,j,:]) . w[h,:], H <= 32: head h is row h of one accumulator tile whose sum over the
 // channels is dealt to the four waves and meets in LDS, so that a head's 32 positions leave as one 128-byte store.
 // One wave per tile with its LayerNorm in 16 dependent steps (pair_f32.hip): 17 / 62 / 255 us at N = 64 / 384 / 768.
-constexpr int kBiasLd = 36;  // floats per head row of a partial tile
 template <int C>
 constexpr size_t pair_bias_lds() {
   return (size_t)PassTile<C>::SLOTS * 16 + (4 * 32 * kBiasLd + 2 * C) * sizeof(float);

@@ -33,6 +33,10 @@ struct TransitionPass {
   const float *att_o, *att_ln_w, *att_ln_b;
   WeightX3 att_g, att_out;
   int N;
+  // the pair bias of the result (BIAS)
+  const float *pb_w, *pb_ln_w, *pb_ln_b;
+  float* pb_out;
+  int pb_H;
 };
 
 constexpr int kRowLd = 4;  // floats between the rows of the updated tile, beside their channels
@@ -44,8 +48,11 @@ constexpr size_t transition_lds() {
 
 // AFTER: the tile begins with the output pass of the ending node's triangle attention (triattn_out_pass: same steps, same bits), its gates in
 // the first four waves and its output projection in the others; the updated rows stay in LDS.
-template <int C, int S, int NPT, bool AFTER>
+// BIAS: and ends with the pair bias of the block's attention over s (pair_bias_pass: same steps, same bits), from the rows that it has just finished. Four
+// trunk blocks at N = 24 / 45 / 64 / 80 / 90 527 / 579 / 587 / 696 / 758 us, so 502 / 554 / 565 / 671 / 736 (a launch, and z read once more).
+template <int C, int S, int NPT, bool AFTER, bool BIAS>
 __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
+  static_assert(AFTER || !BIAS, "one tile per work-group");
   static_assert(!AFTER || (C == 128 && NPT == 1), "eight waves: a gate and an output tile for each 32 channels");
   static_assert(S == 8 || (S == 4 && NPT == 2), "eight waves share the hidden tiles of a slice");
   typedef PassTile<C> XTile;
@@ -289,15 +296,77 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
         for (int v = 0; v < 16; ++v) red[(kh - 1) * (OT * NPT * 1024) + 64 * v] = oacc[v];
       }
       __syncthreads();
-      if (kh > 0) continue;
+      if (AFTER && !BIAS && kh > 0) return;
+      if (!BIAS && kh > 0) continue;
+      if (!BIAS || kh == 0) {
 #pragma unroll
-      for (int q = 0; q < KSPLIT - 1; ++q)
+        for (int q = 0; q < KSPLIT - 1; ++q)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) oacc[v] += red[q * (OT * NPT * 1024) + 64 * v];
+          for (int v = 0; v < 16; ++v) oacc[v] += red[q * (OT * NPT * 1024) + 64 * v];
+      }
     }
     int j0;
     const int pn = NPT * tile + pt_b;
     const int r = row_of(pn, j0), bb = r / p.R, i = r - bb * p.R, j = j0 + at.l32;
+    if constexpr (BIAS) {
+      float* row = rows + at.l32 * (C + kRowLd) + 32 * ot + 16 * at.lh;
+      if (kh == 0) {
+        if (p.mask) {
+          const float m = j < L ? p.mask[bb * p.mv.stride_b + i * p.mv.stride_r + (int64_t)j * p.mv.stride_k] : 0.f;
+#pragma unroll
+          for (int v = 0; v < 16; ++v) oacc[v] *= m;
+        }
+        store_row16(row, row, oacc, 1);
+        if (j < L) {
+          float4* dst = reinterpret_cast<float4*>(p.out + bb * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j * p.xv.stride_k + 32 * ot + 16 * at.lh);
+#pragma unroll
+          for (int a = 0; a < 4; ++a) dst[a] = *reinterpret_cast<const float4*>(row + 4 * a);
+        }
+      }
+      for (int c = tid; c < C; c += 64 * NW) att_ln[c] = p.pb_ln_w[c], att_ln[C + c] = p.pb_ln_b ? p.pb_ln_b[c] : 0.f;
+      constexpr int SPW = KS / 4;  // four waves share the sum over the channels
+      u32x4_t w[SPW][3];
+      if (wave < 4) {
+        const int head = at.l32 < p.pb_H ? at.l32 : p.pb_H - 1;  // the rows from H on are dropped
+#pragma unroll
+        for (int s = 0; s < SPW; ++s) split_operand(p.pb_w + (size_t)head * C, SPW * wave + s, at.lh, w[s]);
+      }
+      __syncthreads();  // the rows are complete, and everybody has read the partial sums
+      const XTile xn = {lds};
+      {
+        const Lane here = lane_here();
+        const int pos = 4 * wave + here.lg;
+        float4 y[C / 64];
+#pragma unroll
+        for (int e = 0; e < C / 64; ++e) raw[0].v[e] = *reinterpret_cast<const float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li);
+        norm_row<C>(raw[0], true, att_ln, here.li, y);
+#pragma unroll
+        for (int e = 0; e < C / 64; ++e) xn.store4(pos, here.li + 16 * e, y[e]);
+      }
+      __syncthreads();
+      float* part = reinterpret_cast<float*>(hid);  // [4][32 heads][kBiasLd]
+      if (wave < 4) {
+        f32x16_t acc = zero16();
+#pragma unroll
+        for (int s = 0; s < SPW; ++s) {
+          const u32x4_t* x = lds + XTile::slot(at.l32, 2 * (SPW * wave + s) + at.lh);
+          const u32x4_t op[3] = {x[0], x[XTile::PLANE], x[2 * XTile::PLANE]};
+          acc = step6<true>(w[s], op, acc);
+        }
+        float* mine = part + wave * (32 * kBiasLd) + at.l32;
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          if (8 * (v >> 2) < p.pb_H) mine[acc_row(v, at.lh) * kBiasLd] = acc[v];
+      }
+      __syncthreads();
+      for (int h = tid >> 5; h < p.pb_H; h += 2 * NW) {
+        const float* q = part + h * kBiasLd + (tid & 31);
+        const float v = (q[0] + q[32 * kBiasLd]) + (q[2 * 32 * kBiasLd] + q[3 * 32 * kBiasLd]);
+        const int f = j0 + (tid & 31);
+        if (f < L) p.pb_out[((size_t)bb * p.pb_H + h) * L + f] = v;
+      }
+      return;
+    }
     if (pn < p.total && j < L) {
       const int64_t off = bb * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j * p.xv.stride_k + 32 * ot + 16 * at.lh;
       if (p.mask) {
@@ -311,14 +380,14 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
   }
 }
 
-template <int C, int S, int NPT, bool AFTER = false>
+template <int C, int S, int NPT, bool AFTER = false, bool BIAS = false>
 hipError_t launch(const TransitionPass& p, hipStream_t stream) {
   constexpr size_t lds = transition_lds<C, S, NPT, AFTER>();
   unsigned grid = 0;
-  hipError_t e = resident_grid<transition_pass<C, S, NPT, AFTER>>(512, lds, (p.total + NPT - 1) / NPT, &grid);
+  hipError_t e = resident_grid<transition_pass<C, S, NPT, AFTER, BIAS>>(512, lds, (p.total + NPT - 1) / NPT, &grid);
   if (e != hipSuccess) return e;
   if (AFTER) grid = (unsigned)p.total;  // a tile each
-  hipLaunchKernelGGL((transition_pass<C, S, NPT, AFTER>), dim3(grid), dim3(512), lds, stream, p);
+  hipLaunchKernelGGL((transition_pass<C, S, NPT, AFTER, BIAS>), dim3(grid), dim3(512), lds, stream, p);
   return hipGetLastError();
 }
 
@@ -377,6 +446,15 @@ hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, 
     p.att_g = a.end->s_g;
     p.att_out = a.end->s_o;
     p.N = a.N;
+    if (a.bias && pair_bias_pass_serves(*a.bias) && a.bias->C == 128 && a.bias->N == a.N && a.bias->B == a.B) {
+      p.pb_w = a.bias->w;
+      p.pb_ln_w = a.bias->ln_w;
+      p.pb_ln_b = a.bias->ln_b;
+      p.pb_out = a.bias->out;
+      p.pb_H = a.bias->H;
+      *a.bias_done = true;
+      return launch<128, 8, 1, true, true>(p, stream);
+    }
     return launch<128, 8, 1, true>(p, stream);
   }
   const bool large = p.total >= 4l * cus;  // two tiles of 64 positions for every CU

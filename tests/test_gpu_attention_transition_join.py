@@ -78,3 +78,16 @@ def test_fp32(monkeypatch, n_mult, n, batch):
     own = z.clone()
     m(own, mask, inplace_safe=True)
     assert torch.equal(own, blocks._by_modules(monkeypatch, lambda: m(z, mask)))
+
+
+@pytest.mark.parametrize("masked", [True, False])
+@pytest.mark.parametrize("n,batch", [(1, 1), (31, 2), (45, 1), (64, 2), (90, 1), (91, 1)])
+def test_fp32_with_pair_bias(monkeypatch, n, batch, masked):
+    m = blocks._fill(of3pair.PairFormerBlock(384, 128, 24, 16, 128, 32, 4), n).to("cuda").eval()
+    gen = torch.Generator().manual_seed(n)
+    s, z = torch.randn(batch, n, 384, generator=gen).to("cuda"), torch.randn(batch, n, n, 128, generator=gen).to("cuda")
+    tok = (torch.rand(batch, n, generator=gen) > 0.2).float().to("cuda") if masked else torch.ones(batch, n, device="cuda")
+    pair = tok[:, :, None] * tok[:, None, :]
+    want = blocks._by_modules(monkeypatch, lambda: m(s, z, tok, pair, _mask_trans=masked))
+    got = m(s, z, tok, pair, _mask_trans=masked)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
