@@ -406,13 +406,14 @@ bool transition_pass_serves(const TransitionF32Args& a) {
          (long)a.B * a.N * ((a.N + 31) / 32) <= 0x3fffffffL;
 }
 
-// Up to one tile of 32 positions per CU: the launch, z's way to memory and back and the wait for the first tile that it saves.  Four
-// trunk blocks at N = 45 / 64 / 80 / 90 586 / 597 / 705 / 780 us, so 578 / 588 / 696 / 758; with more tiles, 110 / 128, 940 / 975 and 945 / 975.
+// Wherever the transition by itself takes tiles of 32 positions (below four per CU).  Saves the launches, z's way to memory and back and the wait for
+// the first tile: with the attention's output pass and the pair bias apart / in one, four trunk blocks at N = 64 / 80 / 90 / 128 / 180
+// 597 / 705 / 780 / 1009 / 1913 us, so 565 / 671 / 736 / 977 / 1875, two at 140 744 / 728.
 bool transition_pass_takes(const TransitionF32Args& a) {
   int cus = 0;
   return device_cus(&cus) == hipSuccess && a.C == 128 && a.HID % 256 == 0 && flat_rows(a) && a.end->C == 128 && a.end->N == a.N &&
          a.end->B == a.B && a.end->add_residual && a.end->out == a.x && a.x == a.out && a.add_residual &&
-         (long)a.B * (((long)a.N * a.N + 31) / 32) <= cus;
+         (long)a.B * (((long)a.N * a.N + 31) / 32) < 4l * cus;
 }
 
 hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, const WeightX3& s_b, const WeightX3& s_out,

@@ -63,9 +63,9 @@ def test_with_pair_bias(monkeypatch, n, batch):
 
 
 @pytest.mark.parametrize("n_mult", [1, 2, 4, 6])
-@pytest.mark.parametrize("n,batch", [(1, 1), (31, 2), (45, 1), (64, 2), (90, 1), (91, 1)])
+@pytest.mark.parametrize("n,batch", [(1, 1), (31, 2), (45, 1), (64, 2), (91, 1), (180, 1), (181, 1)])
 def test_fp32(monkeypatch, n_mult, n, batch):
-    """transition_pass, AFTER, up to a tile of 32 positions per CU, and beyond; hidden slices of 256 (n_mult 1: slices of 128, apart)."""
+    """transition_pass, AFTER, below four tiles of 32 positions per CU, and beyond; hidden slices of 256 (n_mult 1: slices of 128, apart)."""
     m = blocks._fill(of3pair.PairBlock(128, 128, 32, 4, transition_n=n_mult), n).to("cuda").eval()
     gen = torch.Generator().manual_seed(n)
     z = torch.randn(batch, n, n, 128, generator=gen).to("cuda")
@@ -81,7 +81,7 @@ def test_fp32(monkeypatch, n_mult, n, batch):
 
 
 @pytest.mark.parametrize("masked", [True, False])
-@pytest.mark.parametrize("n,batch", [(1, 1), (31, 2), (45, 1), (64, 2), (90, 1), (91, 1)])
+@pytest.mark.parametrize("n,batch", [(1, 1), (31, 2), (45, 1), (64, 2), (91, 1), (180, 1), (181, 1)])
 def test_fp32_with_pair_bias(monkeypatch, n, batch, masked):
     m = blocks._fill(of3pair.PairFormerBlock(384, 128, 24, 16, 128, 32, 4), n).to("cuda").eval()
     gen = torch.Generator().manual_seed(n)
