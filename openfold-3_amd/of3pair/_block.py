@@ -82,7 +82,7 @@ class _Params:
         self.attrs = []    # (attributes of a module, name, the value that a call uses)
         self.noted = []    # the same of values that the search alone looks at
         self.last = (b"", None, None)  # pointers of refs, dtype and pointer array of the last call
-        self.lists = None  # refs as _native.scan takes them
+        self.lists = None  # refs as _scan takes them
 
     def link(self, owner, name, held):
         self.owners.append(owner)

@@ -8,7 +8,10 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import warnings
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
+
+import torch
 
 from . import build as _build
 from .build import LIB_PATH
@@ -100,16 +103,25 @@ def load() -> ctypes.CDLL:
 
 
 def load_scan():
-    """csrc/host_params.cpp's scan, or None where it is not built or was built for another torch."""
-    if not os.path.exists(_build.HOST_PATH):
-        return None
-    spec = importlib.util.spec_from_file_location("_of3host", _build.HOST_PATH)
+    """csrc/host_params.cpp's scan, or None where it is not built for this torch and Python or is older than its source."""
     try:
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-    except ImportError:
+        if not os.path.exists(LIB_PATH) or _build.is_stale():
+            return None  # load() says so
+    except OSError:  # a stamp, and no sources to compare it with: neither does load() take the library
         return None
-    return module.scan
+    why = "it is not built for torch %s" % torch.__version__
+    path = _build.host_path()
+    if os.path.exists(path):
+        spec = importlib.util.spec_from_file_location("_of3host", path)
+        try:
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            return module.scan
+        except ImportError as e:
+            why = e
+    warnings.warn("calls of blocks look at their parameters in Python, which takes some 25 us of host time per block; "
+                  "`python -m of3pair.build` builds %s: %s" % (_build.HOST_SOURCE, why))
+    return None
 
 
 def strides3(values):

@@ -48,7 +48,7 @@ SOURCES = [
 
 # host code against torch's headers, a Python extension of its own (the library above has a plain C interface)
 HOST_SOURCE = "host_params.cpp"
-HOST_PATH = os.path.join(LIB_DIR, "_of3host.so")
+HOST_STEM = "_of3host."
 
 # packed fp32 VALU ops are disabled on purpose (device code only)
 HIPCC_FLAGS = [
@@ -94,6 +94,18 @@ def source_digest() -> str:
     return h.hexdigest()
 
 
+def host_path() -> str:
+    """Where the host extension for this torch and this Python lies: it reads their objects through the layouts of their
+    headers, which the same symbols do not vouch for, so its name says what it was compiled against."""
+    import sysconfig
+
+    import torch
+
+    built_for = (torch.__version__, torch.version.git_version, torch.version.debug, torch._C._GLIBCXX_USE_CXX11_ABI,
+                 sysconfig.get_config_var("SOABI"))
+    return os.path.join(LIB_DIR, HOST_STEM + hashlib.sha256(repr(built_for).encode()).hexdigest()[:16] + ".so")
+
+
 def _build_host():
     """Needs a C++ compiler, Python.h and torch's headers, which the library does without, and only spares host time."""
     import sysconfig
@@ -104,7 +116,7 @@ def _build_host():
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
            *["-isystem" + d for d in cpp_extension.include_paths()], "-I" + sysconfig.get_paths()["include"],
-           os.path.join(CSRC, HOST_SOURCE), "-o", HOST_PATH,
+           os.path.join(CSRC, HOST_SOURCE), "-o", host_path(),
            *["-L" + d for d in cpp_extension.library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10"]
     _run(cmd)
 
@@ -112,9 +124,9 @@ def _build_host():
 def build(verbose: bool = False, jobs: int = 4) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     digest = source_digest()
-    for path in (STAMP_PATH, HOST_PATH):  # no stamp while the objects are in flux, no extension of an earlier build
-        if os.path.exists(path):
-            os.remove(path)
+    for name in os.listdir(LIB_DIR):  # no stamp while the objects are in flux, no extension of an earlier build
+        if name == os.path.basename(STAMP_PATH) or (name.startswith(HOST_STEM) and name.endswith(".so")):
+            os.remove(os.path.join(LIB_DIR, name))
     objs = []
 
     def compile_one(src):
@@ -130,7 +142,7 @@ def build(verbose: bool = False, jobs: int = 4) -> str:
         try:
             host.result()
         except (ImportError, OSError, RuntimeError) as e:
-            warnings.warn("%s is not built, calls of blocks look at their parameters in Python: %s" % (os.path.basename(HOST_PATH), e))
+            warnings.warn("%s is not built, calls of blocks look at their parameters in Python: %s" % (HOST_SOURCE, e))
     _run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs])
     with open(STAMP_PATH, "w") as fh:
         fh.write(digest + "\n")
