@@ -609,14 +609,14 @@ int of3_transition_fwd(const void* x, const int64_t x_strides[3], const float* m
                                add_residual, nullptr, 0, dtype, stream);
 }
 
-// presplit as above; operands: w_a, w_b, w_out in MFMA operand order (bf16), or null.  before: the attention whose output pass the
-// launch begins with; takes_end: says whether it could, and launches nothing; bias: a pair bias of the result that goes with `before`
 // A block's pair bias of the attention over s, to go with its last pair launch
 struct BlockBias {
   of3::PairBiasArgs bf16;
   of3::PairBiasF32Args f32;
 };
 
+// presplit as above; operands: w_a, w_b, w_out in MFMA operand order (bf16), or null.  before: the attention whose output pass the
+// launch begins with; takes_end: says whether it could, and launches nothing; bias: a pair bias of the result that goes with `before`
 static int transition_fwd(const of3::WeightX3* presplit, const void* const* operands, const void* x, const int64_t x_strides[3], const float* mask,
                           const int64_t mask_strides[3], const void* ln_w, const void* ln_b, const void* w_a, const void* w_b, const void* w_out,
                           void* out, int64_t B, int64_t N, int64_t C, int64_t HID, int add_residual, void* workspace,

@@ -458,8 +458,10 @@ hipError_t join_rows(int B, int N, int C, int* rows) {
   // The fewest rows with which all tiles run at once (one work-group per CU at 128 channels, two at 64).  Three joins against
   // their six passes, us, 256 CUs, packed weights; 128 channels: N = 40 24 / 30, 80 32 / 38, 128 45 / 56, 160 62 / 70, 200 (six
   // rows) 82 / 86; 64 channels: 2 x 100 39 / 46, 2 x 187 57 / 72, 2 x 205 66 / 87, 1 x 256 50 / 78.  At 64 channels, where two
-  // work-groups cover each other's waits, four rows stay the better up to three rounds (3 x 220 100 / 118, 4 x 187 96 / 110;
-  // four rounds, 4 x 256, 157 / 164); at 128 a second round costs what the join saves.
+  // work-groups cover each other's waits, four rows stay the better up to three rounds (3 x 220 100 / 118, 4 x 187 96 / 110), which
+  // is also what the workspace has room for (join_room).  At four, 4 x 256, the launches are level (168 / 169 in a trace) and the
+  // contraction that writes x transposed takes 27 us in place of 21: two blocks 788 / 782; in between, 4 x 225 (3.6 rounds), they would
+  // still gain, 712 / 742.  At 128 a second round costs what the join saves.
   const long slots = (C == 128 ? 1 : 2) * (long)cus, panels = (N + 31) / 32;
   auto tiles = [&](int r) { return B * (long)((N + r - 1) / r) * panels; };
   for (int r = 1; r <= 6 && *rows == 0; ++r)
@@ -476,6 +478,9 @@ hipError_t trimul_triattn_launch(const TrimulOutArgs& e, const TriattnProjArgs& 
 hipError_t triattn_triattn_launch(const TriattnOutArgs& e, const TriattnProjArgs& s, int C, hipStream_t stream) {
   return C == 128 ? launch<128, TriattnEnd, TriattnStart>(e, s, stream) : launch<64, TriattnEnd, TriattnStart>(e, s, stream);
 }
+// Only blocks whose attentions come first have this boundary.  Such blocks, us, with this launch / its two passes / no join at all: 64
+// channels 64 57.2 / 60.2 / 65.0, 2 x 100 86.6 / 88.5 / 99.8, 2 x 187 161.1 / 164.4 / 170.8, 4 x 187 245.5 / 250.0 / 257.8; 128 channels
+// 64 64.1 / 67.5 / 74.7, 160 138.1 / 140.8 / 145.1, 200 188.1 / 190.9 / 193.4.
 hipError_t triattn_trimul_launch(const TriattnOutArgs& e, const TrimulProjArgs& s, int C, hipStream_t stream) {
   return C == 128 ? launch<128, TriattnEnd, TrimulStart>(e, s, stream) : launch<64, TriattnEnd, TrimulStart>(e, s, stream);
 }
