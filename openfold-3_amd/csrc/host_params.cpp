@@ -1,10 +1,10 @@
 // What a block's call looks at in its parameters, for all of them at once (of3pair/_block.py): 57 parameters take 27 us per block
 // in Python, a third of the host time of a block of 40 tokens, and 2 us here.
 //
-// scan(owners, names, counts, dtype, seen)
+// scan(owners, names, counts, dtype, seen, gpu = -1)
 //   owners[i][names[i]] is parameter i (a dict and a string), counts the number of values each has to have (int64 buffer), dtype
-//   what all of them have to be, seen the pointers that this returned before (bytes).
-//   True: all are contiguous tensors of that dtype and size, where `seen` says; bytes: they are, elsewhere, and these are their
+//   what all of them have to be, seen the pointers that this returned before (bytes), gpu the device they have to be on (-1: any, or none).
+//   True: all are contiguous tensors of that dtype and size, on that device, where `seen` says; bytes: they are, elsewhere, and these are their
 //   addresses (uint64, 0 for one that is None); False: one is not; None: one is of a type whose methods may be its own (a tensor
 //   subclass) or has no address, to be asked in Python.
 // Nothing is kept between calls and nothing is written to, so threads may share what they pass.
@@ -30,10 +30,12 @@ struct Buffer {
 PyObject* parameter_type = nullptr;
 
 PyObject* scan(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
-  if (n_args != 5 || !PyList_Check(args[0]) || !PyList_Check(args[1]) || !THPDtype_Check(args[3]) || !PyBytes_Check(args[4])) {
-    PyErr_SetString(PyExc_TypeError, "scan(list of dicts, list of names, int64 counts, dtype, bytes)");
+  if (n_args < 5 || n_args > 6 || !PyList_Check(args[0]) || !PyList_Check(args[1]) || !THPDtype_Check(args[3]) || !PyBytes_Check(args[4])) {
+    PyErr_SetString(PyExc_TypeError, "scan(list of dicts, list of names, int64 counts, dtype, bytes, gpu = -1)");
     return nullptr;
   }
+  const long gpu = n_args == 6 ? PyLong_AsLong(args[5]) : -1;
+  if (gpu == -1 && PyErr_Occurred()) return nullptr;
   const Py_ssize_t n = PyList_GET_SIZE(args[0]);
   const Buffer counts(args[2]);
   if (!counts.ok) return nullptr;
@@ -56,6 +58,7 @@ PyObject* scan(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
       const at::Tensor& v = THPVariable_Unpack(p);
       if (!v.has_storage()) Py_RETURN_NONE;
       if (v.numel() != count[i] || v.scalar_type() != type || !v.is_contiguous()) Py_RETURN_FALSE;
+      if (gpu >= 0 && !(v.is_cuda() && v.get_device() == gpu)) Py_RETURN_FALSE;
       found[i] = reinterpret_cast<uint64_t>(v.data_ptr());
     }
     const Py_ssize_t bytes = n * 8;

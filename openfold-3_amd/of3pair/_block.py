@@ -173,14 +173,15 @@ class _Params:
             if bias:
                 self.param(lin, "bias", shape[:1])
 
-    def gather(self, dtype):
-        """The pointer array, or None when a parameter is not a plain contiguous tensor of `dtype`."""
+    def gather(self, dtype, device=None):
+        """The pointer array, or None when a parameter is not a plain contiguous tensor of `dtype` on the GPU `device` (None: anywhere)."""
         seen, seen_dtype, array = self.last
         if self.lists is None:
             self.lists = ([ref[0] for ref in self.refs], [ref[1] for ref in self.refs], _array("q", [ref[2] for ref in self.refs]))
-        found = _scan(*self.lists, dtype, seen) if _scan is not None else None
+        gpu = -1 if device is None or device.index is None else device.index  # of activations on the host _pair_args has its say
+        found = _scan(*self.lists, dtype, seen, gpu) if _scan is not None else None
         if found is None:
-            found = self._scan_in_python(dtype)
+            found = self._scan_in_python(dtype, device)
         if found is False:
             return None
         if (found is not True and found != seen) or seen_dtype is not dtype:
@@ -195,14 +196,14 @@ class _Params:
             self.last = (ptrs.tobytes(), dtype, array)
         return array
 
-    def _scan_in_python(self, dtype):
+    def _scan_in_python(self, dtype, device):
         """What csrc/host_params.cpp does, for parameters of other types and where it is not built."""
         ptrs = _array("Q")
         for owner, name, count in self.refs:
             p = owner.get(name)
             if p is None:
                 ptrs.append(0)
-            elif p.numel() == count and p.dtype is dtype and p.is_contiguous():
+            elif p.numel() == count and p.dtype is dtype and p.is_contiguous() and (device is None or p.device == device):
                 ptrs.append(p.data_ptr())
             else:
                 return False
@@ -321,12 +322,12 @@ def _plan(block, build):
     return plan
 
 
-def _gather(block, build, dtype):
+def _gather(block, build, dtype, device=None):
     """(pointer array, dimensions) of the block's parameters, or None."""
     q, dims = _plan(block, build)
     if dims is None:
         return None
-    array = q.gather(dtype)
+    array = q.gather(dtype, device)
     if array is None:
         return None
     for m in q.called:  # modules that the block would call: their hooks, their mode and a forward of their own are theirs
@@ -363,7 +364,7 @@ def run_pair_block(block, z, mask, inplace, attention_first=False, mask_trans=Tr
     """z after the block's modules, or None when the single call does not serve it."""
     if _first_call(block, z) or not _as_written():
         return None
-    found = _gather(block, lambda q: _pair_params(q, block), z.dtype)
+    found = _gather(block, lambda q: _pair_params(q, block), z.dtype, z.device)
     args = found and _pair_args(z, mask)
     if not args:
         return None
@@ -388,13 +389,14 @@ def run_pair_block(block, z, mask, inplace, attention_first=False, mask_trans=Tr
 
 def _pairformer_args(s, z, single_mask, pair_mask, c, c_s):
     """The tensors of a block's or a stack's call: (z4, mask arguments, single mask as fp32), or None."""
-    if not s.is_cuda or s.dtype is not z.dtype or not s.is_contiguous() or not F3._is_single(s):
+    if s.device != z.device or s.dtype is not z.dtype or not s.is_contiguous() or not F3._is_single(s):
         return None
     args = _pair_args(z, pair_mask)
     if not args or s.shape[:-1] != z.shape[:-2] or args[0].shape[-1] != c or s.shape[-1] != c_s:
         return None
     sm = None
     if single_mask is not None:
+        F3._require_device(single_mask, s.device, "single_mask")
         sm = single_mask.to(torch.float32).expand(s.shape[:-1]).contiguous()
     return args + (sm,)
 
@@ -403,7 +405,7 @@ def run_pairformer_block(block, pair_block_type, s, z, single_mask, pair_mask, i
     """(s, z) after the block, or None when the single call does not serve it."""
     if _first_call(block, z) or not _as_written():
         return None
-    found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
+    found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype, z.device)
     if not found:
         return None
     array, ((c, ch, h, d, hid, inf), (c_s, h_s, d_s, hid_s, inf_s)) = found
@@ -440,7 +442,7 @@ def run_pairformer_stack(blocks, block_type, pair_block_type, s, z, single_mask,
     for block in blocks:
         if type(block) is not block_type or block.training or block._forward_hooks or block._forward_pre_hooks or any(name in block.__dict__ for name in _CALL):
             return None
-        found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype)
+        found = _gather(block, lambda q: _pairformer_params(q, block, pair_block_type), z.dtype, z.device)
         if not found or (dims is not None and found[1] != dims):
             return None
         arrays.append(found[0])

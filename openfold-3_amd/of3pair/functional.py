@@ -150,6 +150,7 @@ def _mask_arg(mask, lead, B, N, device):
     m = mask
     if m.shape[-2:] != (N, N):
         raise ValueError("mask must be [*, N, N]")
+    _require_device(m, device, "mask")
     if m.dtype != torch.float32:
         m = m.to(torch.float32)
     m = m.expand(*lead, N, N) if len(lead) else m
@@ -157,11 +158,20 @@ def _mask_arg(mask, lead, B, N, device):
     return m3, m3.data_ptr(), _lib.strides3(m3.stride())
 
 
-def _w(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
-    """Parameter as a contiguous device tensor of the activations' dtype (what a module cast
+def _require_device(t: torch.Tensor, device, name: str):
+    """The kernels follow a pointer wherever it leads: memory of the host or of another GPU is refused here."""
+    if t.device != device:
+        raise RuntimeError("%s must live on %s as the activations do, not on %s" % (name, device, t.device))
+
+
+def _w(t: torch.Tensor, x: torch.Tensor, count: int) -> torch.Tensor:
+    """Parameter of `count` values as a contiguous tensor of the activations' dtype (what a module cast
     with .to(dtype) already holds; otherwise converted once per call)."""
-    if t.dtype != dtype or not t.is_contiguous():
-        t = t.detach().to(dtype).contiguous()
+    _require_device(t, x.device, "parameter")
+    if t.numel() != count:
+        raise ValueError("a parameter of shape %s does not fit activations of %d channels" % (tuple(t.shape), x.shape[-1]))
+    if t.dtype != x.dtype or not t.is_contiguous():
+        t = t.detach().to(x.dtype).contiguous()
     return t
 
 
@@ -200,8 +210,9 @@ def triangle_multiplicative_update(z, mask, norm_in_weight, norm_in_bias, norm_o
     if nbytes < 0:
         raise ValueError("triangle multiplication: bf16 supports (c_z, c_hidden) = (128,128) or (64,64), fp32 any "
                          "widths up to 256; got (%d,%d) in %s" % (C, CH, z.dtype))
-    keep = [_w(t, z.dtype) for t in (norm_in_weight, norm_in_bias, norm_out_weight, norm_out_bias, a_p_weight, a_g_weight,
-                            b_p_weight, b_g_weight, g_out_weight, p_out_weight)]
+    keep = [_w(t, z, n) for t, n in ((norm_in_weight, C), (norm_in_bias, C), (norm_out_weight, CH), (norm_out_bias, CH),
+                                     (a_p_weight, CH * C), (a_g_weight, CH * C), (b_p_weight, CH * C), (b_g_weight, CH * C),
+                                     (g_out_weight, C * C), (p_out_weight, C * CH))]
     m3, mptr, mstr = _mask_arg(mask, lead, B, N, z.device)
     out4 = z4 if inplace else _out_like(z4)
     ws = _workspace(z.device, nbytes)
@@ -232,7 +243,8 @@ def triangle_attention(x, mask, norm_weight, norm_bias, bias_weight, q_weight, k
     if nbytes < 0:
         raise ValueError("triangle attention: bf16 supports 4 heads with (c_in, c_head) = (128,32) or (64,16), fp32 "
                          "c_in <= 256, head widths up to 64 and heads * c_head <= 256; got c_in=%d heads=%d c_head=%d in %s" % (C, H, D, x.dtype))
-    keep = [_w(t, x.dtype) for t in (norm_weight, norm_bias, bias_weight, q_weight, k_weight, v_weight, g_weight, o_weight)]
+    keep = [_w(t, x, n) for t, n in ((norm_weight, C), (norm_bias, C), (bias_weight, H * C), (q_weight, H * D * C), (k_weight, H * D * C),
+                                     (v_weight, H * D * C), (g_weight, H * D * C), (o_weight, C * H * D))]
     m3, mptr, mstr = _mask_arg(mask, lead, B, N, x.device)
     out4 = x4 if inplace else _out_like(x4)
     ws = _workspace(x.device, nbytes)
@@ -275,7 +287,7 @@ def swiglu_transition(x, mask, norm_weight, norm_bias, a_weight, b_weight, out_w
         return _through_fp32(swiglu_transition, x, inplace, mask, norm_weight, norm_bias, a_weight, b_weight, out_weight,
                              add_residual=add_residual)
     served = bf16_widths if code == _lib.OF3_DTYPE_BF16 else fp32_widths
-    keep = [_w(t, x.dtype) for t in (norm_weight, norm_bias, a_weight, b_weight, out_weight)]
+    keep = [_w(t, x, n) for t, n in ((norm_weight, C), (norm_bias, C), (a_weight, HID * C), (b_weight, HID * C), (out_weight, C * HID))]
     m3, mptr, mstr = _mask_arg(mask, lead, B, N, x.device)
     out4 = x4 if inplace else _out_like(x4)
     need = lib.of3_transition_workspace_bytes_for(code, B, N, C, HID)  # fp32: room for the split weights
@@ -307,6 +319,7 @@ def _swiglu_transition_rows(x, mask, norm_weight, norm_bias, a_weight, b_weight,
     out = xc if (inplace and xc is x) else torch.empty_like(xc)
     m = None
     if mask is not None:
+        _require_device(mask, x.device, "mask")
         if tuple(mask.shape) != tuple(x.shape[:-1]):
             mask = mask.expand(*x.shape[:-1])
         m = mask.to(torch.float32).contiguous()
@@ -323,7 +336,7 @@ def _swiglu_transition_rows(x, mask, norm_weight, norm_bias, a_weight, b_weight,
         raise ValueError("single transition: bf16 supports c_in = 384 with a hidden width that is a multiple of 384, "
                          "fp32 c_in <= 512 and hidden <= 2048; got hidden=%d in %s" % (HID, x.dtype))
     ws = _workspace(x.device, max(need, 256))
-    keep = [_w(t, x.dtype) for t in (norm_weight, norm_bias, a_weight, b_weight, out_weight)]
+    keep = [_w(t, x, n) for t, n in ((norm_weight, C), (norm_bias, C), (a_weight, HID * C), (b_weight, HID * C), (out_weight, C * HID))]
     with torch.cuda.device(x.device):
         st = lib.of3_transition_rows_fwd(xc.data_ptr(), None if m is None else m.data_ptr(),
                                          *[k.data_ptr() for k in keep], out.data_ptr(), rows, C, HID,
@@ -352,8 +365,8 @@ def pair_bias(z, norm_weight, norm_bias, weight):
         # widths the bf16 kernel does not serve: the fp32 kernel on widened activations, rounded once at the end
         return pair_bias(z.float(), norm_weight, norm_bias, weight).to(torch.bfloat16)
     served = bf16_widths if code == _lib.OF3_DTYPE_BF16 else fp32_widths
-    nw, w = _w(norm_weight, z.dtype), _w(weight, z.dtype)
-    nb = None if norm_bias is None else _w(norm_bias, z.dtype)
+    nw, w = _w(norm_weight, z, C), _w(weight, z, H * C)
+    nb = None if norm_bias is None else _w(norm_bias, z, C)
     out = torch.empty(B, H, N, N, dtype=z.dtype, device=z.device)
     with torch.cuda.device(z.device):
         st = lib.of3_pair_bias_fwd(z4.data_ptr(), _lib.strides3(z4.stride()[:3]), nw.data_ptr(),
@@ -379,7 +392,7 @@ def layer_norm(x, weight, bias):
     xc = x.contiguous()
     rows = xc.numel() // C
     out = torch.empty_like(xc)
-    w, b = _w(weight, x.dtype), _w(bias, x.dtype)
+    w, b = _w(weight, x, C), _w(bias, x, C)
     with torch.cuda.device(x.device):
         st = lib.of3_layer_norm_fwd(xc.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), rows, C, code,
                                     _stream(x))
@@ -414,9 +427,9 @@ def template_tail(t, norm_weight, norm_bias, linear_t_weight, apply_layer_norm: 
         # the fp32 kernel on widened activations, rounded once at the end
         return template_tail(t.float(), norm_weight, norm_bias, linear_t_weight, apply_layer_norm).to(torch.bfloat16)
     served = bf16_widths if code == _lib.OF3_DTYPE_BF16 else fp32_widths
-    w = _w(linear_t_weight, t.dtype)
-    nw = _w(norm_weight, t.dtype) if apply_layer_norm else None
-    nb = _w(norm_bias, t.dtype) if apply_layer_norm else None
+    w = _w(linear_t_weight, t, CZ * CT)
+    nw = _w(norm_weight, t, CT) if apply_layer_norm else None
+    nb = _w(norm_bias, t, CT) if apply_layer_norm else None
     out = torch.empty(*lead, N, N, CZ, dtype=t.dtype, device=t.device)
     with torch.cuda.device(t.device):
         st = lib.of3_template_tail_fwd(tc.data_ptr(), None if nw is None else nw.data_ptr(),
@@ -439,6 +452,7 @@ def attention_pair_bias(a, z, mask, norm_a_weight, norm_a_bias, norm_z_weight, n
     code = _require_gpu(a, "a")
     lib = _lib.load()
     bias = _bias if _bias is not None else pair_bias(z, norm_z_weight, norm_z_bias, z_weight)  # [*, H, N, N]
+    _require_device(bias, a.device, "z")
     if bias.dtype != a.dtype:
         bias = bias.to(a.dtype)
     lead = a.shape[:-2]
@@ -457,6 +471,7 @@ def attention_pair_bias(a, z, mask, norm_a_weight, norm_a_bias, norm_z_weight, n
     out = ac if (inplace and ac is a) else torch.empty_like(ac)
     m = None
     if mask is not None:
+        _require_device(mask, a.device, "mask")
         m = mask.to(torch.float32).expand(*lead, N).contiguous()
     need = lib.of3_attn_pair_bias_workspace_bytes_for(code, B, N, CS, H, D)
     if need < 0 and code == _lib.OF3_DTYPE_BF16 and lib.of3_attn_pair_bias_workspace_bytes_for(_lib.OF3_DTYPE_F32, B, N, CS, H, D) >= 0:
@@ -472,7 +487,8 @@ def attention_pair_bias(a, z, mask, norm_a_weight, norm_a_bias, norm_z_weight, n
         raise ValueError("attention_pair_bias: bf16 supports C_s = no_heads * c = 384 with c a multiple of 8 up to "
                          "24, fp32 C_s <= 512 and c <= 64; got C_s=%d heads=%d c=%d in %s" % (CS, H, D, a.dtype))
     ws = _workspace(a.device, need)
-    w = [_w(t, a.dtype) for t in (norm_a_weight, norm_a_bias, q_weight, q_bias, k_weight, v_weight, g_weight, o_weight)]
+    w = [_w(t, a, n) for t, n in ((norm_a_weight, CS), (norm_a_bias, CS), (q_weight, HD * CS), (q_bias, HD), (k_weight, HD * CS),
+                                  (v_weight, HD * CS), (g_weight, HD * CS), (o_weight, CS * HD))]
     with torch.cuda.device(a.device):
         st = lib.of3_attn_pair_bias_fwd(ac.data_ptr(), bias.data_ptr(), None if m is None else m.data_ptr(),
                                         *[t.data_ptr() for t in w], out.data_ptr(), B, N, CS, H, D, float(inf),
