@@ -119,9 +119,23 @@ def _through_fp32(fn, x, inplace, *args, **kwargs):
     return out
 
 
+def _overlaps(z4: torch.Tensor) -> bool:
+    """Whether two positions of [B, N, N, C] may share memory, as those of an expanded tensor do.  Kernels write their results
+    in z's own strides and update them in place, one position beside another."""
+    if z4.is_contiguous():
+        return False
+    end = z4.shape[3]  # of what the smaller strides span
+    for stride, size in sorted(zip(z4.stride()[:3], z4.shape[:3])):
+        if size > 1:
+            if stride < end:
+                return True
+            end += stride * (size - 1)
+    return False
+
+
 def _flatten_pair(z: torch.Tensor):
     """[*, N, N, C] -> a 4-D view [B, N, N, C] with unit channel stride, no copy when the
-    leading dimensions can be merged."""
+    leading dimensions can be merged and no two positions share memory."""
     if z.dim() < 3:
         raise ValueError("pair tensor must be [*, N, N, C]")
     n1, n2, c = z.shape[-3:]
@@ -139,7 +153,7 @@ def _flatten_pair(z: torch.Tensor):
             z4 = z.view(-1, n1, n2, c)
         except RuntimeError:
             z4 = z.reshape(-1, n1, n2, c)
-    if z.dtype == torch.bfloat16 and (any(s % 8 for s in z4.stride()[:3]) or z4.data_ptr() % 16):
+    if (z.dtype == torch.bfloat16 and (any(s % 8 for s in z4.stride()[:3]) or z4.data_ptr() % 16)) or _overlaps(z4):
         z4 = z4.contiguous()
     return z4, lead
 
