@@ -6,10 +6,19 @@
 
 namespace of3 {
 
-// split, operand-ordered copy of a weight matrix [rows][K]: three planes of ceil(rows / 32) * 32 * K bf16
+// split, operand-ordered copy of a weight matrix [rows][K]: planes of ceil(rows / 32) * 32 * K values, three of bf16 or
+// two of fp16 (of3_split.h); behind the fp16 planes, the scales of each 32 rows
+struct WeightScales {
+  float unscale;    // 1 / (the weights' scale times `input`): from the accumulator to the layer's output
+  float input;      // the scale of the inputs where these come from a LayerNorm (the same for all rows), else 1
+  float output;     // the scale that the rows' outputs take as fp16 terms (0: not used as such)
+  float inv_bound;  // a power of two, 1 / it is a bound on the rows' outputs (inputs from a LayerNorm)
+};
 struct WeightX3 {
   const bf16_t* h;
   long plane;
+  int terms;
+  __device__ __forceinline__ const WeightScales* scales() const { return reinterpret_cast<const WeightScales*>(h + 2 * plane); }
 };
 __host__ __device__ constexpr long packed_elems(long rows, long K) { return (rows + 31) / 32 * 32 * K; }
 
@@ -32,9 +41,10 @@ struct TrimulF32 {
   const float *w_ap, *w_ag, *w_bp, *w_bg, *w_g, *w_z;
   WeightX3 s_ap, s_ag, s_bp, s_bg, s_g, s_z;  // split copies (the *_x3 kernels only)
   float *a, *b, *x, *out;
-  // a and b split into three bf16 terms in the k-panel layout (the split-operand contraction only):
+  // a and b as terms (three bf16, or two fp16 of the values times the scale of w_ap's and w_bp's outputs) in the k-panel
+  // layout (the split-operand contraction only):
   // element (b, c, r, k) of a term sits at ((((b CH + c) Np / 32 + k / 32) Np + panel_row(r, c)) 32 + k % 32,
-  // the three terms ab_plane elements apart; Np = N rounded up to whole 32-wide panels
+  // the terms ab_plane elements apart; Np = N rounded up to whole 32-wide panels
   bf16_t *as, *bs;
   long ab_plane;
   int Np;
@@ -48,11 +58,14 @@ struct TriattnF32 {
   const float *ln_w, *ln_b, *w_q, *w_k, *w_v, *w_b, *w_g, *w_o;
   WeightX3 s_q, s_k, s_v, s_g, s_o;  // split copies (the *_x3 kernels only)
   float *q, *k, *v, *tb, *o, *out;
-  // q, k and v^T split into three bf16 terms and stored as MFMA operands (the split-operand core only):
+  // q, k and v^T as terms (three bf16, or two fp16 of the values times the scale of their weights' outputs) stored as MFMA
+  // operands (the split-operand cores only):
   // the 16 bytes of lane l for step s of 32-position tile t of (b, i, h) are slot
   // (((b N + i) H + h) * Jp / 32 + t) * steps + s) * 64 + l of a plane.  q and k have D / 16 steps (16
   // head channels each) and planes of qk_plane elements; v^T always has two steps (16 keys each) of 32
-  // rows, the rows from D on being zero, and planes of v_plane elements
+  // rows, the rows from D on being zero, and planes of v_plane elements.  As fp16 terms at D = 16, v^T is one plane: the
+  // rows 0 .. 15 of an operand are the first terms, 16 .. 31 the second ones of the same channels.  With fp16 terms tb
+  // holds the bias times the scales of q and k.
   bf16_t *qs, *ks, *vs;
   long qk_plane, v_plane;
   int Jp;  // N rounded up to whole 32-position tiles
@@ -67,6 +80,7 @@ hipError_t trimul_proj_pass_f32(const TrimulF32& p, hipStream_t stream);
 hipError_t trimul_out_pass_f32(const TrimulF32& p, hipStream_t stream);
 bool triattn_pass_serves(const TriattnF32& p);
 hipError_t triattn_proj_pass_f32(const TriattnF32& p, hipStream_t stream);
+hipError_t triattn_core_h2_f32_launch(const TriattnF32& p, hipStream_t stream);  // triattn_core_f32.hip
 hipError_t triattn_out_pass_f32(const TriattnF32& p, hipStream_t stream);
 // the pair transition likewise (transition_f32.hip)
 bool transition_pass_serves(const TransitionF32Args& a);

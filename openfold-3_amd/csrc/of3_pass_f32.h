@@ -1,5 +1,6 @@
-// Building blocks of the fp32 position-wise passes on split operands (pair_pass_f32.hip, transition_f32.hip): LDS tiles
-// of 32 positions in three bf16 planes, LayerNorm of rows spread over 16 lanes, six-product MFMA steps.
+// Building blocks of the fp32 position-wise passes on split operands (pair_pass_f32.hip, transition_f32.hip,
+// pair_proj_f32.hip): LDS tiles of 32 positions in planes of terms, LayerNorm of rows spread over 16 lanes, MFMA steps of
+// three (two fp16 terms) or six (three bf16 terms) products.
 #pragma once
 
 #include "of3_device.h"
@@ -14,6 +15,11 @@ constexpr float kEps = 1e-5f;
 constexpr float kLog2eF32 = 1.4426950408889634f;
 __device__ __forceinline__ float sigmoid_hw_f32(float x) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * kLog2eF32));
+}
+
+// of a value still multiplied by 1 / unscale, a power of two
+__device__ __forceinline__ float sigmoid_hw_f32(float x, float unscale) {
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * (-kLog2eF32 * unscale)));
 }
 
 // four values as the halves of three MFMA operand chunks
@@ -57,6 +63,30 @@ struct PassTile {
     d[0] = h;
     d[PLANE] = m;
     d[2 * PLANE] = l;
+  }
+};
+
+// The same in two planes of fp16 terms, of values already scaled
+template <int C>
+struct HalfTile {
+  static constexpr int NCH = C / 8, PLANE = 32 * NCH, SLOTS = 2 * PLANE;
+  u32x4_t* s;
+  __device__ __forceinline__ static int slot(int pos, int chunk) { return PassTile<C>::slot(pos, chunk); }
+  __device__ __forceinline__ void store4(int pos, int c4, const float4& y) const {
+    u32x2_t h, l;
+    uint32_t a, b;
+    split2h(y.x, y.y, a, b), h[0] = a, l[0] = b;
+    split2h(y.z, y.w, a, b), h[1] = a, l[1] = b;
+    u32x2_t* d = reinterpret_cast<u32x2_t*>(s) + 2 * slot(pos, c4 >> 1) + (c4 & 1);
+    d[0] = h;
+    d[2 * PLANE] = l;
+  }
+  __device__ __forceinline__ void store8(int pos, int chunk, const float (&y)[8]) const {
+    u32x4_t h, l;
+    split8h(y, h, l);
+    u32x4_t* d = s + slot(pos, chunk);
+    d[0] = h;
+    d[PLANE] = l;
   }
 };
 
@@ -118,6 +148,15 @@ __device__ __forceinline__ void load_unit(const WeightX3& W, int t, int lane_src
     for (int pl = 0; pl < TERMS; ++pl) w[s][pl] = src[pl * (W.plane / 8) + 64 * s];
 }
 
+// the scale of a gated attention output over C channels: a weighted mean of v, so no larger than v's bound
+template <int C>
+__device__ __forceinline__ float attention_scale(const WeightX3& Wv) {
+  float s = Wv.scales()[0].output;
+#pragma unroll
+  for (int t = 1; t < C / 32; ++t) s = fminf(s, Wv.scales()[t].output);
+  return s;
+}
+
 // rows of a fp32 weight matrix as split MFMA operands: k-values 16 s + 8 lh .. + 7 of `row`
 __device__ __forceinline__ void split_operand(const float* row, int s, int lh, u32x4_t (&w)[3]) {
   const float4 u = *reinterpret_cast<const float4*>(row + 16 * s + 8 * lh);
@@ -144,6 +183,38 @@ __device__ __forceinline__ f32x16_t step6(const u32x4_t (&w)[3], const u32x4_t (
   acc = mm<W_ROWS>(w[0], x[1], acc);
   return mm<W_ROWS>(w[0], x[0], acc);
 }
+// Sum of a product over C channels in fp16 terms, k-step by k-step.  At 64 channels the products with a second term are
+// summed apart and added at the end: rounded to the size of their own sum they leave 0.86 of the error (9.8 against 11.3 in
+// 1e-8, three bf16 terms 10.9); at 128 channels one sum is below the three terms' error already.
+template <bool W_ROWS>
+__device__ __forceinline__ f32x16_t mm_f16(u32x4_t w, u32x4_t x, f32x16_t acc) {
+  return W_ROWS ? mfma_32x32x16_f16(w, x, acc) : mfma_32x32x16_f16(x, w, acc);
+}
+template <int C, bool W_ROWS>
+struct HalfSum {
+  static constexpr bool kApart = C == 64;
+  f32x16_t acc = zero16(), low = zero16();
+  __device__ __forceinline__ void step(const u32x4_t (&w)[2], const u32x4_t (&x)[2]) {
+    f32x16_t& l = kApart ? low : acc;
+    l = mm_f16<W_ROWS>(w[1], x[0], l);
+    l = mm_f16<W_ROWS>(w[0], x[1], l);
+    acc = mm_f16<W_ROWS>(w[0], x[0], acc);
+  }
+  __device__ __forceinline__ f32x16_t total() const { return kApart ? acc + low : acc; }
+};
+template <int C, bool W_ROWS>
+__device__ __forceinline__ f32x16_t unit_product(const HalfTile<C>& t, const u32x4_t (&w)[C / 16][2]) {
+  HalfSum<C, W_ROWS> sum;
+  const Lane at = lane_here();
+#pragma unroll
+  for (int s = 0; s < C / 16; ++s) {
+    const u32x4_t* x = t.s + HalfTile<C>::slot(at.l32, 2 * s + at.lh);
+    const u32x4_t op[2] = {x[0], x[HalfTile<C>::PLANE]};
+    sum.step(w[s], op);
+  }
+  return sum.total();
+}
+
 template <int C, bool W_ROWS>
 __device__ __forceinline__ f32x16_t unit_product(const PassTile<C>& t, const u32x4_t (&w)[C / 16][3]) {
   f32x16_t acc = zero16();

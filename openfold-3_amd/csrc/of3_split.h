@@ -37,6 +37,42 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4_t& h, u32x4_t&
   }
 }
 
+// ---- two fp16 terms -----------------------------------------------------------------------------
+// x s = h + l with h = fp16(x s), l = fp16(x s - h) and s a power of two: 22 to 23 significant bits, and three products
+//     x w = (l wh + h wl + h wh) / (sx sw)        (l wl is below 2^-22 |x w| and left out)
+// instead of six, four bytes per value instead of six.  A rounded operand adds about 2^-24.6 of its value; what fp32
+// accumulation adds grows with the number of products summed and is the larger part of either form's error.  Measured
+// against float64 on normal operands, relative 2-norm in 1e-8, three bf16 terms | two fp16 terms | plain fp32 fused
+// multiply-adds: 32 values summed 6.8 | 9.3 | 10.4, 64 10.9 | 11.3 | 14.3, 128 16.3 | 14.2 | 20.5, 256 23.4 | 19.0 | 28.6, 768 42 | 31 | 50.
+// fp16 ends at 65504, so every operand is scaled by a power of two (exact) that a bound on its values allows: of3_weight_split.h.
+// Values far below that bound lose relative precision only where they are 2^-13 or less after scaling; an operand
+// bounded by 2^14 is held to 2^-39 of the bound.
+typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
+typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2_t;
+__device__ __forceinline__ f32x16_t mfma_32x32x16_f16(u32x4_t a, u32x4_t b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+// two values (scaled) as the halves of a word of each term, round to nearest even
+__device__ __forceinline__ void split2h(float a, float b, uint32_t& h, uint32_t& l) {
+  const f32x2_t x = {a, b};
+  const f16x2_t hi = __builtin_convertvector(x, f16x2_t);
+  h = __builtin_bit_cast(uint32_t, hi);
+  f32x2_t r;  // a - hi[0], b - hi[1], exact (the compiler makes a conversion and a subtraction of it, two instructions each)
+  float ra, rb;
+  __asm__("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(ra) : "v"(h), "v"(a));
+  __asm__("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb) : "v"(h), "v"(b));
+  r[0] = ra, r[1] = rb;
+  l = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2_t));
+}
+__device__ __forceinline__ void split8h(const float (&x)[8], u32x4_t& h, u32x4_t& l) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    uint32_t a, b;
+    split2h(x[2 * w], x[2 * w + 1], a, b);
+    h[w] = a, l[w] = b;
+  }
+}
+
 // row of accumulator register v in lane half lh of a 32 x 32 MFMA result (the lane's column is lane & 31)
 __device__ __forceinline__ int acc_row(int v, int lh) { return 8 * (v >> 2) + 4 * lh + (v & 3); }
 

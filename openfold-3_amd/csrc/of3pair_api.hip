@@ -1030,6 +1030,7 @@ struct BlockDims {
   int dtype;
   int64_t B, N, C, CH, H, D, HID;
   float inf;
+  bool rows16 = false;  // fp32: z and the result have their rows on 16-byte boundaries
   bool wide() const { return dtype == OF3_DTYPE_F32; }
   int weights() const { return OF3_PAIR_BLOCK_WEIGHTS - (HID == 0 ? 5 : 0); }
   int64_t prepared_bytes() const {
@@ -1066,9 +1067,10 @@ static hipError_t prepare_blocks(const void* const* const* weights, int n, const
         for (int d = 0; d < 2; ++d, next += of3::kTrimulMatrices) {
           const void* const* w = o.w + 10 * d;
           of3::TrimulF32Args a;
+          a.ln_in_w = f(w[0]), a.ln_in_b = f(w[1]), a.ln_out_w = f(w[2]), a.ln_out_b = f(w[3]);
           a.w_ap = f(w[4]), a.w_ag = f(w[5]), a.w_bp = f(w[6]), a.w_bg = f(w[7]), a.w_g = f(w[8]), a.w_z = f(w[9]);
           a.C = (int)C, a.CH = (int)CH;
-          of3::trimul_split_jobs(splitter, a, next);
+          of3::trimul_split_jobs(splitter, a, k.rows16 && of3::trimul_half_shapes(k.B, k.N, C, CH), next);
         }
       }
       if (of3::triattn_split_widths(C, k.H, k.D)) {
@@ -1076,17 +1078,19 @@ static hipError_t prepare_blocks(const void* const* const* weights, int n, const
         for (int d = 0; d < 2; ++d, next += of3::kTriattnMatrices) {
           const void* const* w = o.w + 20 + 8 * d;
           of3::TriattnF32Args a;
+          a.ln_w = f(w[0]), a.ln_b = f(w[1]);
           a.w_q = f(w[3]), a.w_k = f(w[4]), a.w_v = f(w[5]), a.w_g = f(w[6]), a.w_o = f(w[7]);
           a.C = (int)C, a.H = (int)k.H, a.D = (int)k.D;
-          of3::triattn_split_jobs(splitter, a, next);
+          of3::triattn_split_jobs(splitter, a, k.rows16 && of3::triattn_half_shapes(k.B, k.N, C, k.H, k.D), next);
         }
       }
       if (k.HID && of3::transition_split_widths(C, k.HID)) {
         o.tr = next;
         of3::TransitionF32Args a;
+        a.ln_w = f(o.w[36]), a.ln_b = f(o.w[37]);
         a.w_a = f(o.w[38]), a.w_b = f(o.w[39]), a.w_out = f(o.w[40]);
         a.C = (int)C, a.HID = (int)k.HID;
-        of3::transition_split_jobs(splitter, a, next);
+        of3::transition_split_jobs(splitter, a, k.rows16 && of3::transition_half_shapes(k.B, k.N, C, k.HID), next);
       }
     }
     return splitter.j.n > 0 ? splitter.launch(stream) : hipSuccess;
@@ -1194,6 +1198,10 @@ static bool pair_block_args_ok(const BlockDims& d, const void* const* weights, c
   return d.wide() ? aligned4(z) && aligned4(out) : aligned16(z) && aligned16(out);
 }
 
+static bool rows16(const void* z, const void* out, const int64_t z_strides[3]) {
+  return aligned16(z) && aligned16(out) && ((z_strides[0] | z_strides[1] | z_strides[2]) & 3) == 0;
+}
+
 int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,
                                        int64_t HID) {
   const int64_t need = pair_block_module_bytes(dtype, B, N, C, CH, H, D, HID);
@@ -1206,9 +1214,10 @@ static int pair_block_fwd(const void* const* weights, const void* z, const int64
                           int64_t D, int64_t HID, float inf, int flags, void* workspace, int64_t workspace_bytes, int dtype,
                           void* stream, const BlockBias* bias = nullptr, bool* bias_done = nullptr) {
   const int64_t need = of3_pair_block_workspace_bytes(dtype, B, N, C, CH, H, D, HID);
-  const BlockDims d = {dtype, B, N, C, CH, H, D, HID, inf};
+  BlockDims d = {dtype, B, N, C, CH, H, D, HID, inf};
   if (need < 0 || !pair_block_args_ok(d, weights, z, z_strides, mask, mask_strides, out, workspace)) return OF3_EINVAL;
   if (workspace_bytes < need) return OF3_ENOSPC;
+  d.rows16 = rows16(z, out, z_strides);
   BlockWeights k;
   const hipError_t e = prepare_blocks(&weights, 1, d, static_cast<char*>(workspace) + need - d.prepared_bytes(), &k,
                                       static_cast<hipStream_t>(stream));
@@ -1387,7 +1396,7 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
                              int64_t CH, int64_t H, int64_t D, int64_t HID, int64_t C_s, int64_t H_s, int64_t D_s,
                              int64_t HID_s, float inf, float inf_s, int flags, void* workspace, int64_t workspace_bytes,
                              int dtype, void* stream, void* side_stream) {
-  const BlockDims d = {dtype, B, N, C, CH, H, D, HID, inf};
+  BlockDims d = {dtype, B, N, C, CH, H, D, HID, inf};
   const StackSpace w = stack_space(d, blocks, C_s, H_s, D_s, HID_s);
   if (w.total < 0 || B > 65535 || N > (1 << 16) || !weights) return OF3_EINVAL;
   for (int64_t i = 0; i < blocks; ++i)
@@ -1395,6 +1404,7 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
         !single_args_ok(d, weights[i] + OF3_PAIR_BLOCK_WEIGHTS, s, s_out, single_mask))
       return OF3_EINVAL;
   if (workspace_bytes < w.total) return OF3_ENOSPC;
+  d.rows16 = rows16(z, z_out, z_strides);
   char* const prepared = static_cast<char*>(workspace) + w.module;
   char* const bias0 = prepared + w.prepared;
   char* const single = bias0 + w.buffers * w.bias;

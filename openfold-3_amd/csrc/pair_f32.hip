@@ -10,7 +10,8 @@
 // (v_mfma_f32_32x32x2_f32: exact products, fp32 sums; channel counts that are multiples of 8 and 16-byte
 // aligned weights), and plain FMA kernels of 8 positions with full-precision expf in the gates for every
 // other shape (any N, C, C_hidden <= 256, head width <= 64).  At 64 and 128 channels the position-wise passes are those of
-// pair_pass_f32.hip, the transition that of transition_f32.hip, pair bias and template tail those of pair_proj_f32.hip.
+// pair_pass_f32.hip and the attention core that of triattn_core_f32.hip, the transition that of transition_f32.hip (all on two fp16
+// terms, as is then the contraction here), pair bias and template tail those of pair_proj_f32.hip.
 //
 // Layouts (workspace, fp32): a, b, x  [B][CH][N][N] with a[b][c][i][k] (k contracted);
 // q, k, v [B][N(i)][H][N(j)][D]; triangle bias [B][H][N][N]; o [B][N][N][H*D].
@@ -734,18 +735,18 @@ __global__ __launch_bounds__(kThreads * PT) void trimul_proj_x3_f32(TrimulF32 p,
 //   <4, 2, 1>  256 x 128, one stage (72 KB), two work-groups on a CU.
 //   <2, 2, 1>  128 x 128, one stage (48 KB): three work-groups on a CU, one's products beside another's loads, first panel and stores.
 //   <2, 1, 1>  64 x 64, one stage (24 KB).
-template <int WM, int T, int STAGES>
+template <int WM, int T, int STAGES, int TERMS>
 struct CtX3 {
   static constexpr int kWaves = 2 * WM, kM = 32 * T * WM, kN = 64 * T;
   static constexpr int kA = kM * 4, kB = kN * 4;  // per term and stage, in 16-byte slots
-  static constexpr int kStage = 3 * (kA + kB);
+  static constexpr int kStage = TERMS * (kA + kB);
   static constexpr size_t kLds = (size_t)STAGES * kStage * 16;
   static constexpr int kAI = kM / 16 / kWaves, kBI = kN / 16 / kWaves;  // loads of a wave per term, 16 rows each
 };
 
-template <int WM, int T, int STAGES>
+template <int WM, int T, int STAGES, int TERMS>
 __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, int tiles_m, int tiles_n, int total, int per_xcd) {
-  typedef CtX3<WM, T, STAGES> K;
+  typedef CtX3<WM, T, STAGES, TERMS> K;
   extern __shared__ u32x4_t lds4[];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -758,9 +759,9 @@ __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, 
   const int i0 = tm * K::kM, j0 = tn * K::kN;
   const size_t chan = (size_t)Np * Np;
   // one descriptor per term and side over the channel's plane
-  __amdgpu_buffer_rsrc_t a_rsrc[3], b_rsrc[3];
+  __amdgpu_buffer_rsrc_t a_rsrc[3], b_rsrc[3];  // TERMS of them (of constant size, as the offsets below)
 #pragma unroll
-  for (int pl = 0; pl < 3; ++pl) {
+  for (int pl = 0; pl < TERMS; ++pl) {
     a_rsrc[pl] = buffer_rsrc(p.as + pl * p.ab_plane + bc * chan, chan * sizeof(bf16_t));
     b_rsrc[pl] = buffer_rsrc(p.bs + pl * p.ab_plane + bc * chan, chan * sizeof(bf16_t));
   }
@@ -781,7 +782,7 @@ __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, 
     u32x4_t* st = lds4 + buf * K::kStage;
     const int soff = panel * Np * 32 * (int)sizeof(bf16_t);
 #pragma unroll
-    for (int pl = 0; pl < 3; ++pl) {
+    for (int pl = 0; pl < TERMS; ++pl) {
 #pragma unroll
       for (int n = 0; n < K::kAI; ++n)
         if (i0 + 16 * (K::kAI * wave + n) < Np)
@@ -791,7 +792,7 @@ __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, 
       for (int n = 0; n < K::kBI; ++n)
         if (j0 + 16 * (K::kBI * wave + n) < Np)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc[pl],
-                                                   (void OF3_LDS_AS*)(st + 3 * K::kA + pl * K::kB + 64 * (K::kBI * wave + n)), 16,
+                                                   (void OF3_LDS_AS*)(st + TERMS * K::kA + pl * K::kB + 64 * (K::kBI * wave + n)), 16,
                                                    b_off[n], soff, 0, 0);
     }
   };
@@ -805,13 +806,13 @@ __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, 
   const int key = (l32 >> 2) & 3;
   auto panel_products = [&](int buf) {
     const u32x4_t* sa = lds4 + buf * K::kStage + (32 * T * wm + l32) * 4;
-    const u32x4_t* sb = lds4 + buf * K::kStage + 3 * K::kA + (32 * T * wn + l32) * 4;
+    const u32x4_t* sb = lds4 + buf * K::kStage + TERMS * K::kA + (32 * T * wn + l32) * 4;
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       const int c = (2 * st + lh) ^ key;
-      u32x4_t ao[T][3], bo[T][3];
+      u32x4_t ao[T][TERMS], bo[T][TERMS];
 #pragma unroll
-      for (int pl = 0; pl < 3; ++pl)
+      for (int pl = 0; pl < TERMS; ++pl)
 #pragma unroll
         for (int n = 0; n < T; ++n) ao[n][pl] = sa[pl * K::kA + n * 128 + c], bo[n][pl] = sb[pl * K::kB + n * 128 + c];
 #pragma unroll
@@ -820,6 +821,12 @@ __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, 
         for (int ni = 0; ni < T; ++ni) {
           if ((mi > 0 && im + 32 * mi >= N) || (ni > 0 && jn + 32 * ni >= N)) continue;
           // smallest terms first
+          if constexpr (TERMS == 2) {
+            acc[mi][ni] = mfma_32x32x16_f16(ao[mi][1], bo[ni][0], acc[mi][ni]);
+            acc[mi][ni] = mfma_32x32x16_f16(ao[mi][0], bo[ni][1], acc[mi][ni]);
+            acc[mi][ni] = mfma_32x32x16_f16(ao[mi][0], bo[ni][0], acc[mi][ni]);
+            continue;
+          }
           acc[mi][ni] = mfma_32x32x16(ao[mi][2], bo[ni][0], acc[mi][ni]);
           acc[mi][ni] = mfma_32x32x16(ao[mi][0], bo[ni][2], acc[mi][ni]);
           acc[mi][ni] = mfma_32x32x16(ao[mi][1], bo[ni][1], acc[mi][ni]);
@@ -855,6 +862,16 @@ __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, 
     for (int panel = 0; panel < panels; ++panel) step(panel, 0);
   }
 
+  if constexpr (TERMS == 2) {
+    const int ct = bc % p.CH / 32;
+    const float unscale = 1.f / (p.s_ap.scales()[ct].output * p.s_bp.scales()[ct].output);
+#pragma unroll
+    for (int mi = 0; mi < T; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < T; ++ni)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[mi][ni][v] *= unscale;
+  }
   float* xc = p.x + (size_t)bc * N * N;
 #pragma unroll
   for (int mi = 0; mi < T; ++mi)
@@ -875,11 +892,11 @@ __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, 
     }
 }
 
-template <int WM, int T, int STAGES>
+template <int WM, int T, int STAGES, int TERMS>
 hipError_t launch_contract_x3(const TrimulF32& p, int cus, hipStream_t stream) {
-  typedef CtX3<WM, T, STAGES> K;
+  typedef CtX3<WM, T, STAGES, TERMS> K;
   constexpr size_t kAlone = 100 * 1024;  // more than half of a CU's
-  const hipError_t e = allow_dynamic_lds<trimul_contract_x3_f32<WM, T, STAGES>>(K::kLds > kAlone ? K::kLds : kAlone);
+  const hipError_t e = allow_dynamic_lds<trimul_contract_x3_f32<WM, T, STAGES, TERMS>>(K::kLds > kAlone ? K::kLds : kAlone);
   if (e != hipSuccess) return e;
   const int tiles_m = (p.N + K::kM - 1) / K::kM, tiles_n = (p.N + K::kN - 1) / K::kN;
   const long total = (long)p.B * p.CH * tiles_m * tiles_n;
@@ -889,7 +906,7 @@ hipError_t launch_contract_x3(const TrimulF32& p, int cus, hipStream_t stream) {
   // kernels (four blocks with their single representations on a second stream, 64 / 48 / 30 tokens: 639 / 628 / 577 us, so
   // 614 / 601 / 556).
   const size_t lds = total <= cus && K::kLds < kAlone ? kAlone : K::kLds;
-  hipLaunchKernelGGL((trimul_contract_x3_f32<WM, T, STAGES>), dim3(per_xcd * 8), dim3(128 * WM), lds, stream, p, tiles_m, tiles_n,
+  hipLaunchKernelGGL((trimul_contract_x3_f32<WM, T, STAGES, TERMS>), dim3(per_xcd * 8), dim3(128 * WM), lds, stream, p, tiles_m, tiles_n,
                      (int)total, per_xcd);
   return hipGetLastError();
 }
@@ -902,15 +919,16 @@ hipError_t launch_contract_x3(const TrimulF32& p, int cus, hipStream_t stream) {
 //     3 x 200 1271 | 1247 | 1286 | 1273, 2 x 400 3903 | 3822 | 3818 | 3897, 4 x 512 12120 | 12129 | 12090 | 12401
 // Alone and with a and b in cache the smaller tiles do better yet (3 x 200: 30 us against 38); under power they move more
 // bytes into LDS per product and slow the kernels around them.
+template <int TERMS>
 hipError_t contract_x3_launch(const TrimulF32& p, hipStream_t stream) {
   static int cache[kMaxDevices];
   int cus = 0;
   const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
   if (e != hipSuccess) return e;
-  if (p.N <= 128) return launch_contract_x3<2, 1, 1>(p, cus, stream);
-  if (p.N > 256) return launch_contract_x3<2, 2, 1>(p, cus, stream);
+  if (p.N <= 128) return launch_contract_x3<2, 1, 1, TERMS>(p, cus, stream);
+  if (p.N > 256) return launch_contract_x3<2, 2, 1, TERMS>(p, cus, stream);
   // two tiles per channel
-  return 2l * p.B * p.CH <= cus ? launch_contract_x3<4, 2, 2>(p, cus, stream) : launch_contract_x3<4, 2, 1>(p, cus, stream);
+  return 2l * p.B * p.CH <= cus ? launch_contract_x3<4, 2, 2, TERMS>(p, cus, stream) : launch_contract_x3<4, 2, 1, TERMS>(p, cus, stream);
 }
 
 // Output pass.  The gate is computed first and kept in registers, so that LayerNorm(x) can take the
@@ -2354,7 +2372,6 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
   p.Np = (a.N + 31) / 32 * 32;
   p.ab_plane = (long)a.B * a.CH * p.Np * p.Np;
   p.as = static_cast<bf16_t*>(a.ab_split);
-  p.bs = p.as + 3 * p.ab_plane;
   const bool split_ab = x3 && a.ab_split && aligned16({a.ab_split}) && (long)p.Np * p.Np * 2 <= 0x7fffffffL;
   const int xgroups = (a.N + 32 * kXT * kPT - 1) / (32 * kXT * kPT);
   const unsigned xblocks = (unsigned)((long)a.B * a.N * xgroups);
@@ -2364,12 +2381,14 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
       for (int i = 0; i < kTrimulMatrices; ++i) w[i] = a.presplit[i];
     } else {
       WeightSplitter splitter(a.wsplit);
-      trimul_split_jobs(splitter, a, w);
+      trimul_split_jobs(splitter, a, split_ab && trimul_pass_serves(p), w);
       if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
     }
     p.s_ap = w[0], p.s_ag = w[1], p.s_bp = w[2], p.s_bg = w[3], p.s_g = w[4], p.s_z = w[5];
   }
-  const bool pass = split_ab && trimul_pass_serves(p);
+  const bool pass = x3 && p.s_ap.terms == 2;
+  if (pass && !(split_ab && trimul_pass_serves(p))) return hipErrorInvalidValue;
+  p.bs = p.as + (pass ? 2 : 3) * p.ab_plane;
   if (pass) {
     if (hipError_t ep = trimul_proj_pass_f32(p, stream); ep != hipSuccess) return ep;
   } else if (x3) {
@@ -2399,7 +2418,7 @@ hipError_t trimul_fwd_f32(const TrimulF32Args& a, hipStream_t stream) {
   // the contraction has no shape or alignment condition of its own; the FMA kernel stays with the
   // FMA passes so that odd shapes run one family of kernels
   if (split_ab) {
-    if (hipError_t ec = contract_x3_launch(p, stream); ec != hipSuccess) return ec;
+    if (hipError_t ec = pass ? contract_x3_launch<2>(p, stream) : contract_x3_launch<3>(p, stream); ec != hipSuccess) return ec;
   } else if (mm || x3) {
     const unsigned t = (unsigned)((a.N + 127) / 128);
     hipLaunchKernelGGL(trimul_contract_mm_f32, dim3(t, t, (unsigned)(a.B * a.CH)), dim3(kThreads), 0, stream, p.a, p.b,
@@ -2472,8 +2491,6 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
   p.qk_plane = (long)a.B * a.N * a.H * p.Jp * a.D;
   p.v_plane = (long)a.B * a.N * a.H * p.Jp * 32;
   p.qs = static_cast<bf16_t*>(a.qkv_split);
-  p.ks = p.qs + 3 * p.qk_plane;
-  p.vs = p.qs + 6 * p.qk_plane;
   const int xgroups = (a.N + 32 * kXT * kPT - 1) / (32 * kXT * kPT);
   const unsigned xblocks = (unsigned)((long)a.B * a.N * xgroups);
   if (x3) {
@@ -2482,16 +2499,17 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
       for (int i = 0; i < kTriattnMatrices; ++i) w[i] = a.presplit[i];
     } else {
       WeightSplitter splitter(a.wsplit);
-      triattn_split_jobs(splitter, a, w);
+      triattn_split_jobs(splitter, a, core_x3 && triattn_pass_serves(p), w);
       if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
     }
     p.s_q = w[0], p.s_k = w[1], p.s_v = w[2], p.s_g = w[3], p.s_o = w[4];
   }
-  const bool pass = core_x3 && triattn_pass_serves(p);
+  const bool pass = x3 && p.s_q.terms == 2;
+  if (pass && !(core_x3 && triattn_pass_serves(p))) return hipErrorInvalidValue;
+  p.ks = p.qs + (pass ? 2 : 3) * p.qk_plane;
+  p.vs = p.ks + (pass ? 2 : 3) * p.qk_plane;
   if (pass) {
     if (hipError_t ep = triattn_proj_pass_f32(p, stream); ep != hipSuccess) return ep;
-    if (hipError_t ep = allow_lds<triattn_core_x3_f32<1>>(kCoreX3Lds); ep != hipSuccess) return ep;
-    if (hipError_t ep = allow_lds<triattn_core_x3_f32<2>>(kCoreX3Lds); ep != hipSuccess) return ep;
   } else if (x3) {
     auto proj = core_x3 ? (fast ? triattn_proj_x3_f32<kXT, kPT, true, true> : triattn_proj_x3_f32<kXT, kPT, true, false>)
                         : (fast ? triattn_proj_x3_f32<kXT, kPT, false, true> : triattn_proj_x3_f32<kXT, kPT, false, false>);
@@ -2517,7 +2535,9 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
   } else {
     hipLaunchKernelGGL(triattn_proj_f32, dim3((unsigned)blocks), dim3(kThreads), 0, stream, p, groups);
   }
-  if (core_x3) {
+  if (pass) {
+    if (hipError_t ep = triattn_core_h2_f32_launch(p, stream); ep != hipSuccess) return ep;
+  } else if (core_x3) {
     const int n_qc = (a.N + 127) / 128, n_rg = (a.N + kXRows - 1) / kXRows;
     const long total = (long)n_qc * n_rg * a.B * a.H;
     if (total > 0x7fffffffL - 8) return hipErrorInvalidValue;
@@ -2564,7 +2584,7 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& a, hipStream_t stream) {
 hipError_t transition_fwd_f32(const TransitionF32Args& args, hipStream_t stream) {
   TransitionF32Args a = args;
   if (a.C > kMaxC || a.HID > kMaxHid) return hipErrorInvalidValue;
-  if (a.end && !(a.presplit && transition_split_widths(a.C, a.HID) && transition_pass_serves(a) && transition_pass_takes(a))) {
+  if (a.end && !(a.presplit && a.presplit[0].terms == 2 && transition_pass_serves(a) && transition_pass_takes(a))) {
     if (hipError_t e = triattn_out_pass_f32(*a.end, stream); e != hipSuccess) return e;
     a.end = nullptr;
     a.bias = nullptr;
@@ -2591,11 +2611,12 @@ hipError_t transition_fwd_f32(const TransitionF32Args& args, hipStream_t stream)
       for (int i = 0; i < kTransitionMatrices; ++i) w[i] = a.presplit[i];
     } else {
       WeightSplitter splitter(a.wsplit);
-      transition_split_jobs(splitter, a, w);
+      transition_split_jobs(splitter, a, transition_pass_serves(a), w);
       if (hipError_t es = splitter.launch(stream); es != hipSuccess) return es;  // no kernel may read unsplit weights
     }
     p.s_a = w[0], p.s_b = w[1], p.s_out = w[2];
-    if (transition_pass_serves(a)) return transition_pass_f32(a, p.s_a, p.s_b, p.s_out, stream);
+    if (p.s_a.terms == 2)
+      return transition_pass_serves(a) ? transition_pass_f32(a, p.s_a, p.s_b, p.s_out, stream) : hipErrorInvalidValue;
     const bool fast = a.C % 64 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 7u) == 0 && even_strides(a.x_view);
     const bool wide = a.C > 128;
     auto kern = wide ? (fast ? transition_x3_f32<true, true> : transition_x3_f32<true, false>)

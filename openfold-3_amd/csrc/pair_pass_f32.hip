@@ -1,13 +1,13 @@
 // Position-wise passes of the two fp32 triangle modules at 64 and 128 channels (c_z = c_hidden = heads x width:
-// the template stack's and the trunk's), products on the bf16 matrix instructions with operands split into three
-// bf16 terms (of3_split.h).  pair_f32.hip has the passes for every other shape.
+// the template stack's and the trunk's), products on the fp16 matrix instructions with operands split into two
+// fp16 terms (of3_split.h).  pair_f32.hip has the passes for every other shape.
 //
 // What bounded the passes of pair_f32.hip at these widths: every group of 32 positions read all split weights
 // again from L2 (6 KB per k-step of a wave against 12 MFMAs, 64 bytes per clock and compute unit: the rate of the
 // L1), and LayerNorm, products and epilogue ran one after the other.  Here the weights stay on the chip:
 // persistent work-groups whose waves each own one 32-output tile of one or two matrices and keep its split
-// operands in registers (96 registers per matrix at 128 channels, 48 at 64) for all the tiles they process; a tile
-// of 32 positions goes through LDS once (three bf16 planes, 16-byte chunks XOR-swizzled by the position), read by
+// operands in registers (64 registers per matrix at 128 channels, 32 at 64) for all the tiles they process; a tile
+// of 32 positions goes through LDS once (two fp16 planes, 16-byte chunks XOR-swizzled by the position), read by
 // all waves.  The next tile's rows are in flight meanwhile, in registers.  At small N the weights are a
 // one-time 3 us instead of a latency in every k-step.
 #include <type_traits>
@@ -18,6 +18,7 @@
 #include "of3_pair_f32.h"
 #include "of3_pass_f32.h"
 #include "of3_split.h"
+#include "of3_weight_split.h"
 
 namespace of3 {
 
@@ -31,44 +32,36 @@ __device__ __forceinline__ uint32_t swap_adjacent(uint32_t v) {
 }
 
 // ---- triangle multiplication, input pass: a, b = mask * sigmoid(LN(z) Wg^T) * (LN(z) Wp^T) ------------------
-// Wave = gate and projection of one 32-channel tile of a or b: two matrices, 192 registers of split operands at 128
-// channels, of which the gate's third terms (used by one product of six) sit in LDS.  A work-group has four waves: at
+// Wave = gate and projection of one 32-channel tile of a or b: two matrices, 128 registers of split operands at 128
+// channels.  A work-group has four waves: at
 // 64 channels a and b, at 128 one of the two, so that two work-groups share a CU and the products of one run beside
 // the LayerNorm and the stores of the other (one work-group of eight waves in step: 468 against 462 us at N = 768).  Tile = 32 columns k of one row; four
 // consecutive rows of a panel are consecutive tiles of one XCD, so that the 64-byte pieces a tile writes per channel
 // and term meet in L2 as whole lines.
 template <int C>
 struct ProjLds {
-  static constexpr bool kThirdInLds = C == 128;
-  static constexpr int kWl = kThirdInLds ? 4 * (C / 16) * 64 : 0;  // slots
-  static constexpr size_t kBytes = (size_t)(PassTile<C>::SLOTS + kWl) * 16 + (2 * C + 64) * sizeof(float);
+  static constexpr size_t kBytes = (size_t)HalfTile<C>::SLOTS * 16 + (2 * C + 64) * sizeof(float);
 };
 
 template <int C>
 __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int panels, int row_groups, int total) {
-  typedef PassTile<C> Tile;
+  typedef HalfTile<C> Tile;
   constexpr int NW = 4, KS = C / 16, OT = C / 32, TASKS = 8 / NW;
   constexpr bool kOneSide = OT == NW;  // a and b in work-groups of their own
-  constexpr bool TL = ProjLds<C>::kThirdInLds;
-  constexpr int GTERMS = TL ? 2 : 3;
   extern __shared__ u32x4_t lds[];
   const Tile xn = {lds};
   const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
-  u32x4_t* wl = lds + Tile::SLOTS + wave * (KS * 64) + lane;
-  float* ln = reinterpret_cast<float*>(lds + Tile::SLOTS + ProjLds<C>::kWl);  // [2][C]
-  float* msk = ln + 2 * C;                                                   // [2][32]
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  float* ln = reinterpret_cast<float*>(lds + Tile::SLOTS);  // [2][C], times the scale of the activations
+  float* msk = ln + 2 * C;                                 // [2][32]
   const int slot = grid_slot(), N = p.N, pair = kOneSide ? slot & 1 : wave / OT, ot = wave % OT;
-  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_in_w[c], ln[C + c] = p.ln_in_b[c];
   const WeightX3 Wg = pair ? p.s_bg : p.s_ag, Wp = pair ? p.s_bp : p.s_ap;
-  u32x4_t wg[KS][GTERMS], wp[KS][3];
-  load_unit<C, GTERMS>(Wg, ot, lane, wg);
-  load_unit<C, 3>(Wp, ot, lane, wp);
-  if (TL) {
-    const u32x4_t* g = reinterpret_cast<const u32x4_t*>(Wg.h) + 2 * (Wg.plane / 8) + (size_t)ot * KS * 64 + lane;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) wl[64 * s] = g[64 * s];
-  }
+  const WeightScales sg = Wg.scales()[ot], sp = Wp.scales()[ot];
+  u32x4_t wg[KS][2], wp[KS][2];
+  load_unit<C, 2>(Wg, ot, lane, wg);
+  load_unit<C, 2>(Wp, ot, lane, wp);
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_in_w[c] * sg.input, ln[C + c] = p.ln_in_b[c] * sg.input;
+  const float out_scale = sp.unscale * sp.output;
   __syncthreads();
 
   struct Place {
@@ -119,16 +112,16 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
     if (tid < 32) msk[32 * buf + tid] = mraw;
     load_tile(id + step < total ? id + step : id);
     __syncthreads();  // the tile is complete
-    f32x16_t ag = zero16(), ap = zero16();
+    HalfSum<C, false> sum_g, sum_p;
     const Lane at = lane_here();
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const u32x4_t* x = xn.s + Tile::slot(at.l32, 2 * s + at.lh);
-      const u32x4_t op[3] = {x[0], x[Tile::PLANE], x[2 * Tile::PLANE]};
-      const u32x4_t g[3] = {wg[s][0], wg[s][1], TL ? wl[64 * s] : wg[s][GTERMS - 1]};
-      ag = step6<false>(g, op, ag);
-      ap = step6<false>(wp[s], op, ap);
+      const u32x4_t op[2] = {x[0], x[Tile::PLANE]};
+      sum_g.step(wg[s], op);
+      sum_p.step(wp[s], op);
     }
+    const f32x16_t ag = sum_g.total(), ap = sum_p.total();
     __syncthreads();  // everybody has read it
     // channels in the lanes, positions in the registers: registers 8 st .. + 7 are the k-values 16 st + 8 (e >> 2)
     // + 4 lh + (e & 3), stored as the 8 consecutive columns 16 st + 8 lh .. of the panel row (a and b in the same
@@ -138,7 +131,7 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
       const int l32 = out.l32, lh = out.lh;
       const bool odd = l32 & 1;
       const int rot0 = panel_rotation(32 * ot + (l32 & ~1), p.Np), rot1 = panel_rotation(32 * ot + (l32 | 1), p.Np);
-      u32x4_t op[2][3];
+      u32x4_t op[2][2];
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
         float x[8];
@@ -149,10 +142,10 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int v = 8 * st + 4 * a + e;
-            x[4 * a + e] = m[e] * sigmoid_hw_f32(ag[v]) * ap[v];
+            x[4 * a + e] = m[e] * sigmoid_hw_f32(ag[v], sg.unscale) * (ap[v] * out_scale);
           }
         }
-        split8(x, op[st][0], op[st][1], op[st][2]);
+        split8h(x, op[st][0], op[st][1]);
       }
       // The lanes of an even and an odd channel exchange a chunk, so that one store writes the 64 bytes of the even
       // channels and the next those of the odd ones (32-byte pieces of every channel otherwise: twice the requests).
@@ -161,7 +154,7 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
       bf16_t* lp0 = lp + (pn + panel_row(t.r, rot0, p.Np)) * 32;
       bf16_t* lp1 = lp + chan + (pn + panel_row(t.r, rot1, p.Np)) * 32;
 #pragma unroll
-      for (int pl = 0; pl < 3; ++pl) {
+      for (int pl = 0; pl < 2; ++pl) {
         u32x4_t first, second;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
@@ -178,49 +171,26 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
 }
 
 // ---- output passes ------------------------------------------------------------------------------------------
-// Wave = one 32-channel tile of the gate and the same tile of the output projection (weights as in the input pass of
-// the multiplication: the gate's third terms in LDS at 128 channels).  The LDS tile holds LayerNorm(z) for the gates,
+// Wave = one 32-channel tile of the gate and the same tile of the output projection, weights in registers as in the input
+// passes.  The LDS tile holds LayerNorm(z) for the gates,
 // then LayerNorm(x) or the gated attention output in its place.  Four waves per work-group at 128 channels, two
 // work-groups per CU; two waves at 64.
 template <int C>
 struct OutLds {
-  static constexpr int NW = C / 32, KS = C / 16;
-  static constexpr bool kThirdInLds = C == 128;
-  static constexpr int kWl = kThirdInLds ? NW * KS * 64 : 0;  // slots
-  static constexpr size_t kTrimul = (size_t)(PassTile<C>::SLOTS + kWl) * 16 + (2 * 32 * 2 * NW + 4 * C) * sizeof(float);
-  static constexpr size_t kTriattn = (size_t)(PassTile<C>::SLOTS + kWl) * 16 + 2 * C * sizeof(float);
+  static constexpr int NW = C / 32;
+  static constexpr size_t kTrimul = (size_t)HalfTile<C>::SLOTS * 16 + (2 * 32 * 2 * NW + 4 * C) * sizeof(float);
+  static constexpr size_t kTriattn = (size_t)HalfTile<C>::SLOTS * 16 + 2 * C * sizeof(float);
 };
 // the two matrices of an output wave, outputs dealt by rowperm16: lane (position l32, half lh) ends with the outputs
 // 32 ot + 16 lh + v
 template <int C>
 struct OutWeights {
   static constexpr int KS = C / 16;
-  static constexpr bool TL = OutLds<C>::kThirdInLds;
-  static constexpr int GTERMS = TL ? 2 : 3;
-  u32x4_t g[KS][GTERMS], o[KS][3];
-  u32x4_t* wl;
-  __device__ __forceinline__ void load(const WeightX3& Wg, const WeightX3& Wo, int ot, int l32, int lh, u32x4_t* lds_wave) {
+  u32x4_t g[KS][2], o[KS][2];
+  __device__ __forceinline__ void load(const WeightX3& Wg, const WeightX3& Wo, int ot, int l32, int lh) {
     const int src = rowperm16(l32) + 32 * lh;
-    load_unit<C, GTERMS>(Wg, ot, src, g);
-    load_unit<C, 3>(Wo, ot, src, o);
-    wl = lds_wave + l32 + 32 * lh;
-    if (TL) {
-      const u32x4_t* t = reinterpret_cast<const u32x4_t*>(Wg.h) + 2 * (Wg.plane / 8) + (size_t)ot * KS * 64 + src;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) wl[64 * s] = t[64 * s];
-    }
-  }
-  __device__ __forceinline__ f32x16_t gate(const PassTile<C>& t) const {
-    f32x16_t acc = zero16();
-    const Lane at = lane_here();
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const u32x4_t* x = t.s + PassTile<C>::slot(at.l32, 2 * s + at.lh);
-      const u32x4_t op[3] = {x[0], x[PassTile<C>::PLANE], x[2 * PassTile<C>::PLANE]};
-      const u32x4_t w[3] = {g[s][0], g[s][1], TL ? wl[64 * s] : g[s][GTERMS - 1]};
-      acc = step6<true>(w, op, acc);
-    }
-    return acc;
+    load_unit<C, 2>(Wg, ot, src, g);
+    load_unit<C, 2>(Wo, ot, src, o);
   }
 };
 // ---- triangle multiplication, output pass: out = [z +] (LN(x) Wz^T) * sigmoid(LN(z) Wg^T)
@@ -228,19 +198,22 @@ struct OutWeights {
 // combined from the groups' means and squared deviations (one exchange).
 template <int C>
 __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int panels, int total) {
-  typedef PassTile<C> Tile;
-  constexpr int NW = C / 32, KS = C / 16, TASKS = 8 / NW, NG = 2 * NW;
+  typedef HalfTile<C> Tile;
+  constexpr int NW = C / 32, TASKS = 8 / NW, NG = 2 * NW;
   extern __shared__ u32x4_t lds[];
   const Tile tile = {lds};
-  float* red = reinterpret_cast<float*>(lds + Tile::SLOTS + OutLds<C>::kWl);  // [NG][32] means, [NG][32] squared deviations
-  float* ln = red + 2 * 32 * NG;                                             // LayerNorm of z [2][C], of x [2][C]
+  float* red = reinterpret_cast<float*>(lds + Tile::SLOTS);  // [NG][32] means, [NG][32] squared deviations
+  float* ln = red + 2 * 32 * NG;                             // LayerNorm of z [2][C], of x [2][C], times the activations' scales
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int N = p.N;
-  for (int c = tid; c < C; c += 64 * NW)
-    ln[c] = p.ln_in_w[c], ln[C + c] = p.ln_in_b[c], ln[2 * C + c] = p.ln_out_w[c], ln[3 * C + c] = p.ln_out_b[c];
+  const WeightScales sg = p.s_g.scales()[wave], sz = p.s_z.scales()[wave];
   OutWeights<C> w;
-  w.load(p.s_g, p.s_z, wave, l32, lh, lds + Tile::SLOTS + wave * (KS * 64));
+  w.load(p.s_g, p.s_z, wave, l32, lh);
+  for (int c = tid; c < C; c += 64 * NW) {
+    ln[c] = p.ln_in_w[c] * sg.input, ln[C + c] = p.ln_in_b[c] * sg.input;
+    ln[2 * C + c] = p.ln_out_w[c] * sz.input, ln[3 * C + c] = p.ln_out_b[c] * sz.input;
+  }
   __syncthreads();
 
   struct Place {
@@ -300,7 +273,7 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
       red[(NG + xg) * 32 + xpos] = q;
     }
     __syncthreads();  // LayerNorm(z) is complete
-    f32x16_t gate = w.gate(tile);
+    const f32x16_t gate = unit_product<C, true>(tile, w.g);
     __syncthreads();  // everybody has read it
     {
       // mean of the groups' means; squared deviations = within the groups + 16 x those of the groups' means
@@ -328,7 +301,7 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
     if (t.j0 + out.l32 < N) {
       const int64_t off = t.b * p.zc.stride_b + t.i * p.zc.stride_r + (t.j0 + out.l32) * p.zc.stride_k + 32 * wave + 16 * out.lh;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[v] *= sigmoid_hw_f32(gate[v]);
+      for (int v = 0; v < 16; ++v) acc[v] = acc[v] * sz.unscale * sigmoid_hw_f32(gate[v], sg.unscale);
       store_row16(p.z + off, p.out + off, acc, p.add_residual);
     }
   }
@@ -339,32 +312,38 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
 // double buffered, one barrier per tile (three panels per barrier: 417 against 385 us at N = 768).  The H rows of the
 // triangle bias are dot products taken on the normalised rows while they are in registers.
 // PARTS work-groups share a tile, each with every output tile's PARTS-th and as many of the bias rows, where there are CUs left:
-// what bounds a launch of one tile per CU is the 288 KB of weights through the CU's L1 (3 us) and the products of three waves
+// what bounds a launch of one tile per CU is the 192 KB of weights through the CU's L1 (3 us) and the products of three waves
 // per SIMD.
 template <int C>
 struct AttProjLds {
-  static constexpr size_t kBytes = (size_t)2 * PassTile<C>::SLOTS * 16 + (2 * C + 8 * C) * sizeof(float);
+  static constexpr size_t kBytes = (size_t)2 * HalfTile<C>::SLOTS * 16 + (2 * C + 8 * C) * sizeof(float);
 };
 
 template <int C, int PARTS>
 __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p, int panels, int total) {
-  typedef PassTile<C> Tile;
+  typedef HalfTile<C> Tile;
   constexpr int OT = C / 32 / PARTS, NW = 3 * OT, KS = C / 16, TASKS = (8 + NW - 1) / NW;
   extern __shared__ u32x4_t lds[];
-  float* ln = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS);  // [2][C]
-  float* wb = ln + 2 * C;                                       // [H][C], H <= 8
+  float* ln = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS);  // [2][C], times the scale of the activations
+  float* wb = ln + 2 * C;                                       // [H][C], H <= 8, times the scale of the logits over that of the activations
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int slot = grid_slot(), part = slot % PARTS;
   const int N = p.N, H = p.H, kind = wave / OT, ot = part * OT + wave % OT;
   const int h0 = H * part / PARTS, h1 = H * (part + 1) / PARTS;  // this work-group's heads of the bias
   const bool narrow = p.D == 16;
-  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c], ln[C + c] = p.ln_b[c];
-  for (int c = tid; c < H * C; c += 64 * NW) wb[c] = p.w_b[c];
-  u32x4_t w[KS][3];
-  load_unit<C, 3>(kind == 0 ? p.s_q : kind == 1 ? p.s_k : p.s_v, ot, tid & 63, w);
+  const WeightX3 W = kind == 0 ? p.s_q : kind == 1 ? p.s_k : p.s_v;
+  const WeightScales sc = W.scales()[ot];
+  u32x4_t w[KS][2];
+  load_unit<C, 2>(W, ot, tid & 63, w);
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * sc.input, ln[C + c] = p.ln_b[c] * sc.input;
+  for (int c = tid; c < H * C; c += 64 * NW) {
+    const int t = c / C * p.D / 32;  // the head's tile of q and k
+    wb[c] = p.w_b[c] * (p.s_q.scales()[t].output * p.s_k.scales()[t].output / sc.input);
+  }
   __syncthreads();
-  const float scale = 1.0f / sqrtf((float)p.D);
+  // q / sqrt(c) after the projection (attention.py:283-284)
+  const float out_scale = sc.unscale * sc.output * (kind == 0 ? 1.0f / sqrtf((float)p.D) : 1.f);
 
   // panel -> its row (b N + i) and first position
   auto row_of = [&](int pn, int& j0) {
@@ -388,34 +367,33 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
   // the operands of a step are read one step ahead, no further: read as early as the compiler would have it, they do
   // not fit the registers of three waves per SIMD
   auto product = [&](auto w_rows, const Tile& t) {
-    f32x16_t acc = zero16();
-    u32x4_t nxt[3];
+    HalfSum<C, decltype(w_rows)::value> sum;
+    u32x4_t nxt[2];
     const Lane at = lane_here();
     auto read = [&](int s) {
       const u32x4_t* x = t.s + Tile::slot(at.l32, 2 * s + at.lh);
-      nxt[0] = x[0], nxt[1] = x[Tile::PLANE], nxt[2] = x[2 * Tile::PLANE];
+      nxt[0] = x[0], nxt[1] = x[Tile::PLANE];
     };
     read(0);
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      const u32x4_t op[3] = {nxt[0], nxt[1], nxt[2]};
+      const u32x4_t op[2] = {nxt[0], nxt[1]};
       if (s + 1 < KS) read(s + 1);
       __builtin_amdgcn_sched_barrier(0);
-      acc = step6<decltype(w_rows)::value>(w[s], op, acc);
+      sum.step(w[s], op);
       __builtin_amdgcn_sched_barrier(0);
     }
-    return acc;
+    return sum.total();
   };
-  auto split_store = [&](bf16_t* dst, long plane8, size_t slot, const f32x16_t& acc, int st, float mul) {
+  auto split_store = [&](bf16_t* dst, long second, size_t slot, const f32x16_t& acc, int st) {
     float x[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = acc[8 * st + e] * mul;
-    u32x4_t h, m, lo;
-    split8(x, h, m, lo);
+    for (int e = 0; e < 8; ++e) x[e] = acc[8 * st + e] * out_scale;
+    u32x4_t h, lo;
+    split8h(x, h, lo);
     u32x4_t* d4 = reinterpret_cast<u32x4_t*>(dst) + slot;
     d4[0] = h;
-    d4[plane8] = m;
-    d4[2 * plane8] = lo;
+    d4[second] = lo;
   };
 
   const int step = (int)gridDim.x / PARTS;
@@ -458,30 +436,20 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
     // A 32-column tile of the projections is one head, or two of width 16.  q and k: head channels in the
     // registers, positions in the lanes; v the other way round.  Registers 8 st .. + 7 of a lane are its operand
     // for step st (narrow heads: q, k have one step, that of head 2 ot + st; lane l32 of the v tile is row
-    // l32 % 16 of head 2 ot + l32 / 16, whose rows 16 .. 31 are written as zeros).
+    // l32 % 16 of head 2 ot + l32 / 16, its second term row 16 + l32 % 16).
     if (kind < 2) {
       const f32x16_t acc = product(std::true_type{}, xn);
-      const float mul = kind == 0 ? scale : 1.f;  // q / sqrt(c) after the projection (attention.py:283-284)
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
         const size_t slot = narrow ? ((row * H + 2 * ot + st) * nt + jt) * 64 + lane : (((row * H + ot) * nt + jt) * 2 + st) * 64 + lane;
-        split_store(kind == 0 ? p.qs : p.ks, p.qk_plane / 8, slot, acc, st, mul);
+        split_store(kind == 0 ? p.qs : p.ks, p.qk_plane / 8, slot, acc, st);
       }
     } else {
       const f32x16_t acc = product(std::false_type{}, xn);
       const int head = narrow ? 2 * ot + (l32 >> 4) : ot, vrow = narrow ? (l32 & 15) : l32;
 #pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        const size_t slot = (((row * H + head) * nt + jt) * 2 + st) * 64 + vrow + 32 * lh;
-        split_store(p.vs, p.v_plane / 8, slot, acc, st, 1.f);
-        if (narrow) {
-          const u32x4_t zero = {0u, 0u, 0u, 0u};
-          u32x4_t* d4 = reinterpret_cast<u32x4_t*>(p.vs) + slot + 16;
-          d4[0] = zero;
-          d4[p.v_plane / 8] = zero;
-          d4[2 * (p.v_plane / 8)] = zero;
-        }
-      }
+      for (int st = 0; st < 2; ++st)
+        split_store(p.vs, narrow ? 16 : p.v_plane / 8, (((row * H + head) * nt + jt) * 2 + st) * 64 + vrow + 32 * lh, acc, st);
     }
   }
 }
@@ -490,17 +458,20 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
 // A wave's 16 channels of a position are consecutive: 64 bytes of o, and two chunks of the second product's operand.
 template <int C>
 __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int panels, int total) {
-  typedef PassTile<C> Tile;
-  constexpr int NW = C / 32, KS = C / 16, TASKS = 8 / NW;
+  typedef HalfTile<C> Tile;
+  constexpr int NW = C / 32, TASKS = 8 / NW;
   extern __shared__ u32x4_t lds[];
   const Tile tile = {lds};
-  float* ln = reinterpret_cast<float*>(lds + Tile::SLOTS + OutLds<C>::kWl);  // [2][C]
+  float* ln = reinterpret_cast<float*>(lds + Tile::SLOTS);  // [2][C], times the scale of the activations
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int N = p.N;
-  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c], ln[C + c] = p.ln_b[c];
+  const WeightScales sg = p.s_g.scales()[wave];
+  const float o_scale = attention_scale<C>(p.s_v);
+  const float unscale = p.s_o.scales()[wave].unscale / o_scale;
   OutWeights<C> w;
-  w.load(p.s_g, p.s_o, wave, l32, lh, lds + Tile::SLOTS + wave * (KS * 64));
+  w.load(p.s_g, p.s_o, wave, l32, lh);
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * sg.input, ln[C + c] = p.ln_b[c] * sg.input;
   __syncthreads();
 
   auto place = [&](int id, int& b, int& i) {  // returns the first position
@@ -543,7 +514,7 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
       for (int e = 0; e < C / 64; ++e) tile.store4(pos, li + 16 * e, y[e]);
     }
     __syncthreads();  // LayerNorm(x) is complete
-    const f32x16_t gate = w.gate(tile);
+    const f32x16_t gate = unit_product<C, true>(tile, w.g);
     __syncthreads();  // everybody has read it
     const Lane mid = lane_here();
 #pragma unroll
@@ -552,15 +523,17 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
       const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
       float y[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = ov[e] * sigmoid_hw_f32(gate[8 * hf + e]);
+      for (int e = 0; e < 8; ++e) y[e] = ov[e] * o_scale * sigmoid_hw_f32(gate[8 * hf + e], sg.unscale);
       tile.store8(mid.l32, 4 * wave + 2 * mid.lh + hf, y);
     }
     load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
     __syncthreads();  // the gated output is complete
-    const f32x16_t acc = unit_product<C, true>(tile, w.o);
+    f32x16_t acc = unit_product<C, true>(tile, w.o);
     __syncthreads();  // everybody has read it
     const Lane out = lane_here();
     if (j0 + out.l32 < N) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[v] *= unscale;
       const int64_t off = b * p.xv.stride_b + i * p.xv.stride_r + (j0 + out.l32) * p.xv.stride_k + 32 * wave + 16 * out.lh;
       store_row16(p.x + off, p.out + off, acc, p.add_residual);
     }
@@ -632,8 +605,7 @@ hipError_t launch_triattn_out(const TriattnF32& p, hipStream_t stream) {
 }  // namespace
 
 bool trimul_pass_serves(const TrimulF32& p) {
-  return p.C == p.CH && (p.C == 64 || p.C == 128) && rows_aligned(p.z, p.zv) && rows_aligned(p.out, p.zc) &&
-         (long)p.B * (p.N + 3) * (p.Np / 32) <= 0x3fffffffL;
+  return trimul_half_shapes(p.B, p.N, p.C, p.CH) && rows_aligned(p.z, p.zv) && rows_aligned(p.out, p.zc);
 }
 hipError_t trimul_proj_pass_f32(const TrimulF32& p, hipStream_t stream) {
   return p.C == 128 ? launch_trimul_proj<128>(p, stream) : launch_trimul_proj<64>(p, stream);
@@ -643,8 +615,7 @@ hipError_t trimul_out_pass_f32(const TrimulF32& p, hipStream_t stream) {
 }
 
 bool triattn_pass_serves(const TriattnF32& p) {
-  return p.H * p.D == p.C && (p.C == 64 || p.C == 128) && p.H <= 8 && rows_aligned(p.x, p.xv) && rows_aligned(p.out, p.xv) &&
-         (long)p.B * p.N * (p.Jp / 32) <= 0x3fffffffL;
+  return triattn_half_shapes(p.B, p.N, p.C, p.H, p.D) && rows_aligned(p.x, p.xv) && rows_aligned(p.out, p.xv);
 }
 hipError_t triattn_proj_pass_f32(const TriattnF32& p, hipStream_t stream) {
   return p.C == 128 ? launch_triattn_proj<128>(p, stream) : launch_triattn_proj<64>(p, stream);

@@ -1,10 +1,10 @@
 // fp32 pair transition (transition.py:225-271, activations.py:33-61) at 64 and 128 channels with a hidden width in
-// multiples of 128, products on the bf16 matrix instructions with operands split into three bf16 terms:
+// multiples of 128, products on the fp16 matrix instructions with operands split into two fp16 terms:
 //     out = [x +] ((silu(LN(x) Wa^T) * (LN(x) Wb^T)) Wout^T) * mask
 // pair_f32.hip has the kernels for every other shape.
 //
-// 36 flops per channel and hidden channel in bf16 products: 1.4 Tflop for N = 768 at n = 4, 730 us of the matrix
-// pipes at the rate they sustain.  The split weights (590 KB at C = 128, n = 4) do not fit a CU and stream from L2.
+// 18 flops per channel and hidden channel in fp16 products: 0.7 Tflop for N = 768 at n = 4, 365 us of the matrix
+// pipes at the rate they sustain.  The split weights (393 KB at C = 128, n = 4) do not fit a CU and stream from L2.
 // One wave per tile of 32 hidden channels and all of the tile's positions: a work-group of eight waves takes the
 // hidden dimension in slices of 32 S channels (S = 8, or 4 with a wave per position tile), so that an operand of Wa
 // and Wb is read once for 64 positions and a slice of 256 hidden channels costs two barriers, against 32 positions
@@ -12,6 +12,7 @@
 // the other product before the barrier between them.  Below two tiles of 64 positions per CU, tiles of 32 positions (two
 // waves then share the sum of the second product).
 #include "of3_pass_f32.h"
+#include "of3_weight_split.h"
 
 namespace of3 {
 
@@ -31,7 +32,7 @@ struct TransitionPass {
   int HID, add_residual;
   // the attention before it (AFTER)
   const float *att_o, *att_ln_w, *att_ln_b;
-  WeightX3 att_g, att_out;
+  WeightX3 att_g, att_out, att_v;
   int N;
   // the pair bias of the result (BIAS)
   const float *pb_w, *pb_ln_w, *pb_ln_b;
@@ -40,10 +41,18 @@ struct TransitionPass {
 };
 
 constexpr int kRowLd = 4;  // floats between the rows of the updated tile, beside their channels
-template <int C, int S, int NPT, bool AFTER>
+template <int C, int S, int NPT, bool AFTER, bool BIAS>
 constexpr size_t transition_lds() {
-  return (size_t)NPT * (PassTile<C>::SLOTS + PassTile<32 * S>::SLOTS) * 16 + 2 * C * sizeof(float) +
-         (AFTER ? (2 * C + 32 * (C + kRowLd)) * sizeof(float) : 0);
+  return (size_t)NPT * (HalfTile<C>::SLOTS + HalfTile<32 * S>::SLOTS) * 16 + 2 * C * sizeof(float) +
+         (AFTER ? (2 * C + 32 * (C + kRowLd)) * sizeof(float) : 0) + (BIAS ? PassTile<C>::SLOTS * 16 : 0);
+}
+// the smallest of a value over the first n <= 32 tiles of a weight matrix
+__device__ __forceinline__ float smallest_inv_bound(const WeightX3& W, int n) {
+  const int lane = threadIdx.x & 31;
+  float v = W.scales()[lane < n ? lane : n - 1].inv_bound;
+#pragma unroll
+  for (int d = 16; d > 0; d >>= 1) v = fminf(v, __shfl_xor(v, d, 32));
+  return v;
 }
 
 // AFTER: the tile begins with the output pass of the ending node's triangle attention (triattn_out_pass: same steps, same bits), its gates in
@@ -55,8 +64,8 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
   static_assert(AFTER || !BIAS, "one tile per work-group");
   static_assert(!AFTER || (C == 128 && NPT == 1), "eight waves: a gate and an output tile for each 32 channels");
   static_assert(S == 8 || (S == 4 && NPT == 2), "eight waves share the hidden tiles of a slice");
-  typedef PassTile<C> XTile;
-  typedef PassTile<32 * S> HTile;
+  typedef HalfTile<C> XTile;
+  typedef HalfTile<32 * S> HTile;
   constexpr int NW = 8, KS = C / 16, OT = C / 32;
   constexpr int XT = S == 8 ? NPT : 1;             // position tiles of a wave in the first product
   constexpr int KSPLIT = NW / (OT * NPT);          // waves sharing an output tile's sum in the second
@@ -72,7 +81,11 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
   const int ht = S == 8 ? wave : wave & 3, pt_a = S == 8 ? 0 : wave >> 2;
   const int ot = wave % OT, pt_b = (wave / OT) % NPT, kh = wave / (OT * NPT);
   const int L = p.L, slices = p.HID / (32 * S);
-  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c], ln[C + c] = p.ln_b[c];
+  // The activations' scale is in ln, the hidden ones take the largest that the bounds of their two factors allow
+  const float x_scale = p.s_a.scales()[0].input;
+  const float h_scale = fminf(0x1p14f * smallest_inv_bound(p.s_a, p.HID / 32) * smallest_inv_bound(p.s_b, p.HID / 32), 0x1p40f);
+  const float unscale = p.s_out.scales()[ot].unscale / h_scale;
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * x_scale, ln[C + c] = p.ln_b[c] * x_scale;
 
   const int lane0 = tid & 63, src_lane = rowperm16(lane0 & 31) + (lane0 & 32);  // outputs dealt by rowperm16
   const u32x4_t* wa = reinterpret_cast<const u32x4_t*>(p.s_a.h) + src_lane;
@@ -98,16 +111,16 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       load_row<C>(p.x + b * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j * p.xv.stride_k, here.li, raw[t]);
     }
   };
-  u32x4_t na[DA][3], nb[DA][3], no[DO][3];  // operands of the next steps
+  u32x4_t na[DA][2], nb[DA][2], no[DO][2];  // operands of the next steps
   auto fetch_ab = [&](int slice, int s) {
     const size_t at = ((size_t)(slice * S + ht) * KS + s) * 64;
 #pragma unroll
-    for (int pl = 0; pl < 3; ++pl) na[s % DA][pl] = wa[pl * pa + at], nb[s % DA][pl] = wb[pl * pa + at];
+    for (int pl = 0; pl < 2; ++pl) na[s % DA][pl] = wa[pl * pa + at], nb[s % DA][pl] = wb[pl * pa + at];
   };
   auto fetch_o = [&](int slice, int s) {
     const size_t at = (size_t)(slice * 2 * S + s) * 64;
 #pragma unroll
-    for (int pl = 0; pl < 3; ++pl) no[s % DO][pl] = wo[pl * po + at];
+    for (int pl = 0; pl < 2; ++pl) no[s % DO][pl] = wo[pl * po + at];
   };
 
   const int tiles = (p.total + NPT - 1) / NPT;
@@ -116,13 +129,18 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
   float* const att_ln = ln + 2 * C;         // [2][C]
   float* const rows = att_ln + 2 * C;       // [32][C + kRowLd]
   if (AFTER)
-    for (int c = tid; c < C; c += 64 * NW) att_ln[c] = p.att_ln_w[c], att_ln[C + c] = p.att_ln_b[c];
+    for (int c = tid; c < C; c += 64 * NW) {
+      const float s = p.att_g.scales()[0].input;
+      att_ln[c] = p.att_ln_w[c] * s, att_ln[C + c] = p.att_ln_b[c] * s;
+    }
   __syncthreads();
   for (; tile < tiles; tile += gridDim.x) {
     if constexpr (AFTER) {
       const XTile xn = {lds}, gated = {hid};
-      u32x4_t w[KS][3];
-      load_unit<C, 3>(kh == 0 ? p.att_g : p.att_out, ot, src_lane, w);
+      u32x4_t w[KS][2];
+      load_unit<C, 2>(kh == 0 ? p.att_g : p.att_out, ot, src_lane, w);
+      const float o_scale = attention_scale<C>(p.att_v);
+      const float att_unscale = kh == 0 ? p.att_g.scales()[ot].unscale : p.att_out.scales()[ot].unscale / o_scale;
       int j0;
       const int b = row_of(tile, j0);  // one row per batch element
       const Lane here = lane_here();
@@ -135,23 +153,23 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       }
       // the operands of a step are read one step ahead, no further: all of them do not fit the registers
       auto product = [&](const XTile& t) {
-        f32x16_t acc = zero16();
-        u32x4_t nxt[3];
+        HalfSum<C, true> sum;
+        u32x4_t nxt[2];
         const Lane at = lane_here();
         auto read = [&](int s) {
           const u32x4_t* x = t.s + XTile::slot(at.l32, 2 * s + at.lh);
-          nxt[0] = x[0], nxt[1] = x[XTile::PLANE], nxt[2] = x[2 * XTile::PLANE];
+          nxt[0] = x[0], nxt[1] = x[XTile::PLANE];
         };
         read(0);
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-          const u32x4_t op[3] = {nxt[0], nxt[1], nxt[2]};
+          const u32x4_t op[2] = {nxt[0], nxt[1]};
           if (s + 1 < KS) read(s + 1);
           __builtin_amdgcn_sched_barrier(0);
-          acc = step6<true>(w[s], op, acc);
+          sum.step(w[s], op);
           __builtin_amdgcn_sched_barrier(0);
         }
-        return acc;
+        return sum.total();
       };
       const int pos = 4 * wave + here.lg;
       float4 y[C / 64];
@@ -171,13 +189,15 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
           const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
           float g[8];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) g[e] = ov[e] * sigmoid_hw_f32(gate[8 * hf + e]);
+          for (int e = 0; e < 8; ++e) g[e] = ov[e] * o_scale * sigmoid_hw_f32(gate[8 * hf + e], att_unscale);
           gated.store8(mid.l32, 4 * ot + 2 * mid.lh + hf, g);
         }
       }
       __syncthreads();
       if (kh > 0) {
-        const f32x16_t acc = product(gated);
+        f32x16_t acc = product(gated);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] *= att_unscale;
         const Lane mid = lane_here();
         float* row = rows + mid.l32 * (C + kRowLd) + 32 * ot + 16 * mid.lh;
         store_row16(row, row, acc, 1);
@@ -203,28 +223,27 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
     }
 #pragma unroll
     for (int s = 0; s < DA; ++s) fetch_ab(0, s);
-    f32x16_t oacc = zero16();
+    HalfSum<128, true> osum;
     for (int slice = 0; slice < slices; ++slice) {
       __syncthreads();  // the activations (first slice), or: everybody has read the slice before
       f32x16_t a[XT], b[XT];
-#pragma unroll
-      for (int t = 0; t < XT; ++t) a[t] = b[t] = zero16();
+      HalfSum<C, true> sum_a[XT], sum_b[XT];
       {
         const Lane at = lane_here();
-        u32x4_t nx[XT][3];
+        u32x4_t nx[XT][2];
         auto read_x = [&](int s) {
 #pragma unroll
           for (int t = 0; t < XT; ++t) {
             const u32x4_t* x = lds + (pt_a + t) * XTile::SLOTS + XTile::slot(at.l32, 2 * s + at.lh);
-            nx[t][0] = x[0], nx[t][1] = x[XTile::PLANE], nx[t][2] = x[2 * XTile::PLANE];
+            nx[t][0] = x[0], nx[t][1] = x[XTile::PLANE];
           }
         };
         read_x(0);
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-          u32x4_t x[XT][3], ca[3], cb[3];
+          u32x4_t x[XT][2], ca[2], cb[2];
 #pragma unroll
-          for (int pl = 0; pl < 3; ++pl) {
+          for (int pl = 0; pl < 2; ++pl) {
             ca[pl] = na[s % DA][pl], cb[pl] = nb[s % DA][pl];
 #pragma unroll
             for (int t = 0; t < XT; ++t) x[t][pl] = nx[t][pl];
@@ -238,14 +257,19 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int t = 0; t < XT; ++t) {
-            a[t] = step6<true>(ca, x[t], a[t]);
-            b[t] = step6<true>(cb, x[t], b[t]);
+            sum_a[t].step(ca, x[t]);
+            sum_b[t].step(cb, x[t]);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int t = 0; t < XT; ++t) a[t] = sum_a[t].total(), b[t] = sum_b[t].total();
       }
       {
         const Lane at = lane_here();
+        const WeightScales* ta = p.s_a.scales() + slice * S + ht;
+        const WeightScales* tb = p.s_b.scales() + slice * S + ht;
+        const float ua = ta->unscale, ub = ua * tb->unscale * h_scale;
 #pragma unroll
         for (int t = 0; t < XT; ++t) {
           const HTile h = {hid + (pt_a + t) * HTile::SLOTS};
@@ -253,7 +277,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
           for (int hf = 0; hf < 2; ++hf) {  // lane (position, half lh): hidden channels 32 ht + 16 lh + 8 hf + e
             float y[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) y[e] = (a[t][8 * hf + e] * sigmoid_hw_f32(a[t][8 * hf + e])) * b[t][8 * hf + e];
+            for (int e = 0; e < 8; ++e) y[e] = (a[t][8 * hf + e] * sigmoid_hw_f32(a[t][8 * hf + e], ua)) * (b[t][8 * hf + e] * ub);
             h.store8(at.l32, 4 * ht + 2 * at.lh + hf, y);
           }
         }
@@ -263,15 +287,15 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       {
         const Lane at = lane_here();
         const u32x4_t* ht0 = hid + pt_b * HTile::SLOTS;
-        u32x4_t nx[3];
+        u32x4_t nx[2];
         auto read_h = [&](int s) {
           const u32x4_t* x = ht0 + HTile::slot(at.l32, 2 * (kh * OSTEPS + s) + at.lh);
-          nx[0] = x[0], nx[1] = x[HTile::PLANE], nx[2] = x[2 * HTile::PLANE];
+          nx[0] = x[0], nx[1] = x[HTile::PLANE];
         };
         read_h(0);
 #pragma unroll
         for (int s = 0; s < OSTEPS; ++s) {
-          const u32x4_t x[3] = {nx[0], nx[1], nx[2]}, co[3] = {no[s % DO][0], no[s % DO][1], no[s % DO][2]};
+          const u32x4_t x[2] = {nx[0], nx[1]}, co[2] = {no[s % DO][0], no[s % DO][1]};
           if (s + 1 < OSTEPS) read_h(s + 1);
           if (s + DO < OSTEPS) fetch_o(slice, s + DO);
           if (s + DO == OSTEPS) {  // after the last weights: loads return in order
@@ -282,11 +306,12 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
               for (int q = 0; q < DA; ++q) fetch_ab(slice + 1, q);
           }
           __builtin_amdgcn_sched_barrier(0);
-          oacc = step6<true>(co, x, oacc);
+          osum.step(co, x);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
+    f32x16_t oacc = osum.total();
     const Lane at = lane_here();
     if (KSPLIT > 1) {  // the waves of an output tile add up through the hidden tile's memory
       __syncthreads();
@@ -305,6 +330,8 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
           for (int v = 0; v < 16; ++v) oacc[v] += red[q * (OT * NPT * 1024) + 64 * v];
       }
     }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) oacc[v] *= unscale;
     int j0;
     const int pn = NPT * tile + pt_b;
     const int r = row_of(pn, j0), bb = r / p.R, i = r - bb * p.R, j = j0 + at.l32;
@@ -332,7 +359,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
         for (int s = 0; s < SPW; ++s) split_operand(p.pb_w + (size_t)head * C, SPW * wave + s, at.lh, w[s]);
       }
       __syncthreads();  // the rows are complete, and everybody has read the partial sums
-      const XTile xn = {lds};
+      const PassTile<C> xn = {reinterpret_cast<u32x4_t*>(rows + 32 * (C + kRowLd))};
       {
         const Lane here = lane_here();
         const int pos = 4 * wave + here.lg;
@@ -349,8 +376,8 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
         f32x16_t acc = zero16();
 #pragma unroll
         for (int s = 0; s < SPW; ++s) {
-          const u32x4_t* x = lds + XTile::slot(at.l32, 2 * (SPW * wave + s) + at.lh);
-          const u32x4_t op[3] = {x[0], x[XTile::PLANE], x[2 * XTile::PLANE]};
+          const u32x4_t* x = xn.s + PassTile<C>::slot(at.l32, 2 * (SPW * wave + s) + at.lh);
+          const u32x4_t op[3] = {x[0], x[PassTile<C>::PLANE], x[2 * PassTile<C>::PLANE]};
           acc = step6<true>(w[s], op, acc);
         }
         float* mine = part + wave * (32 * kBiasLd) + at.l32;
@@ -382,7 +409,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
 
 template <int C, int S, int NPT, bool AFTER = false, bool BIAS = false>
 hipError_t launch(const TransitionPass& p, hipStream_t stream) {
-  constexpr size_t lds = transition_lds<C, S, NPT, AFTER>();
+  constexpr size_t lds = transition_lds<C, S, NPT, AFTER, BIAS>();
   unsigned grid = 0;
   hipError_t e = resident_grid<transition_pass<C, S, NPT, AFTER, BIAS>>(512, lds, (p.total + NPT - 1) / NPT, &grid);
   if (e != hipSuccess) return e;
@@ -402,8 +429,7 @@ bool flat_rows(const TransitionF32Args& a) {
 }  // namespace
 
 bool transition_pass_serves(const TransitionF32Args& a) {
-  return (a.C == 64 || a.C == 128) && a.HID % 128 == 0 && rows_aligned(a.x, a.x_view) && rows_aligned(a.out, a.x_view) &&
-         (long)a.B * a.N * ((a.N + 31) / 32) <= 0x3fffffffL;
+  return transition_half_shapes(a.B, a.N, a.C, a.HID) && rows_aligned(a.x, a.x_view) && rows_aligned(a.out, a.x_view);
 }
 
 // Wherever the transition by itself takes tiles of 32 positions (below four per CU).  Saves the launches, z's way to memory and back and the wait for
@@ -411,7 +437,7 @@ bool transition_pass_serves(const TransitionF32Args& a) {
 // 597 / 705 / 780 / 1009 / 1913 us, so 565 / 671 / 736 / 977 / 1875, two at 140 744 / 728.
 bool transition_pass_takes(const TransitionF32Args& a) {
   int cus = 0;
-  return device_cus(&cus) == hipSuccess && a.C == 128 && a.HID % 256 == 0 && flat_rows(a) && a.end->C == 128 && a.end->N == a.N &&
+  return device_cus(&cus) == hipSuccess && a.C == 128 && a.HID % 256 == 0 && flat_rows(a) && a.end->C == 128 && a.end->s_o.terms == 2 && a.end->N == a.N &&
          a.end->B == a.B && a.end->add_residual && a.end->out == a.x && a.x == a.out && a.add_residual &&
          (long)a.B * (((long)a.N * a.N + 31) / 32) < 4l * cus;
 }
@@ -446,6 +472,7 @@ hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, 
     p.att_ln_b = a.end->ln_b;
     p.att_g = a.end->s_g;
     p.att_out = a.end->s_o;
+    p.att_v = a.end->s_v;
     p.N = a.N;
     if (a.bias && pair_bias_pass_serves(*a.bias) && a.bias->C == 128 && a.bias->N == a.N && a.bias->B == a.B) {
       p.pb_w = a.bias->w;

@@ -37,6 +37,7 @@ SOURCES = [
     "single_transition.hip",
     "pair_f32.hip",
     "pair_pass_f32.hip",
+    "triattn_core_f32.hip",
     "pair_proj_f32.hip",
     "transition_f32.hip",
     "weight_split.hip",
