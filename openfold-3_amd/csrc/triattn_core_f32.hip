@@ -46,11 +46,12 @@ constexpr int kTbI = kTb / (64 * 2 * kRows);    // load instructions of a wave f
 template <int STEPS>
 struct CoreH2 {
   static constexpr int kKv = 2 * STEPS * 64;    // K (steps x terms), and as many of V^T (two steps x terms, or x 1 at width 16)
-  static constexpr size_t kLds = (size_t)(2 * kTb + kRows * 2 * 2 * kKv) * 16;
+  static constexpr int kStages = STEPS == 2 ? 1 : 2;  // of K and V^T
+  static constexpr size_t kLds = (size_t)(2 * kTb + kRows * kStages * 2 * kKv) * 16;
 };
 
 template <int STEPS>
-__global__ __launch_bounds__(128 * kRows, 2) void triattn_core_h2_f32(TriattnF32 p, int n_qc, int n_rg, int total, int per_xcd) {
+__global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32 p, int n_qc, int n_rg, int total, int per_xcd) {
   typedef CoreH2<STEPS> L;
   constexpr int QT = 2, D = 16 * STEPS;
   extern __shared__ u32x4_t lds4[];
@@ -119,14 +120,16 @@ __global__ __launch_bounds__(128 * kRows, 2) void triattn_core_h2_f32(TriattnF32
                                              buffer_rsrc(kvp + kv_plane, STEPS == 1 && qh ? kv_bytes - 1024 : kv_bytes)};
   const __amdgpu_buffer_rsrc_t tb_rsrc = buffer_rsrc(tbp, (size_t)N * Jp * sizeof(float));
   const uint32_t lane_off = lane * 16;
-  u32x4_t* kv_row = kv_lds + row * (2 * 2 * L::kKv);
-  auto issue_loads = [&](int kt, int buf) {  // buf is a constant at every call site
+  u32x4_t* kv_row = kv_lds + row * (L::kStages * 2 * L::kKv);
+  auto issue_bias = [&](int kt, int buf) {  // buf is a constant at every call site
     u32x4_t* tdst = tb_lds + buf * kTb + 64 * kTbI * wave;
-    u32x4_t* kdst = kv_row + (2 * buf + qh) * L::kKv;
 #pragma unroll
     for (int n = 0; n < kTbI; ++n)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(tb_rsrc, (void OF3_LDS_AS*)(tdst + 64 * n), 16, tb_off[n],
                                                kt * (32 * (int)sizeof(float)), 0, 0);
+  };
+  auto issue_kv = [&](int kt, int buf) {
+    u32x4_t* kdst = kv_row + (2 * (L::kStages == 2 ? buf : 0) + qh) * L::kKv;
 #pragma unroll
     for (int n = 0; n < 2 * STEPS; ++n)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(kv_rsrc[n & 1], (void OF3_LDS_AS*)(kdst + 64 * n), 16, lane_off,
@@ -168,19 +171,30 @@ __global__ __launch_bounds__(128 * kRows, 2) void triattn_core_h2_f32(TriattnF32
     for (int v = 1; v < 16; ++v) m = fmaxf(m, s[v]);
     return fmaxf(m, __shfl_xor(m, 32, 64));
   };
-  auto tile = [&](auto track, int buf, float mb) {
+  struct Operands {
+    u32x4_t k[STEPS][2], v[2][STEPS];
+  };
+  auto read_operands = [&](int buf) {
+    const u32x4_t* kvb = kv_row + (L::kStages == 2 ? buf : 0) * (2 * L::kKv) + lane;
+    Operands o;
+#pragma unroll
+    for (int st = 0; st < STEPS; ++st)
+#pragma unroll
+      for (int pl = 0; pl < 2; ++pl) o.k[st][pl] = kvb[(st * 2 + pl) * 64];
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int pl = 0; pl < STEPS; ++pl) o.v[st][pl] = kvb[L::kKv + (st * STEPS + pl) * 64];
+    return o;
+  };
+  auto tile = [&](auto track, int buf, float mb, const Operands& given) {
     constexpr bool kTrack = decltype(track)::value;
     if (!wave_has_work) return;
     // first pass: a tile whose keys are all masked or padded adds exp(-1e9 + logit) = 0 exactly to every sum
     if (!kTrack && __builtin_amdgcn_ballot_w64(mb > -1e8f) == 0) return;
     const bool has_mb = __builtin_amdgcn_ballot_w64(mb != 0.f) != 0;
-    const u32x4_t* kvb = kv_row + buf * (2 * L::kKv) + lane;
     const u32x4_t* tbuf = tb_lds + buf * kTb + (64 * qh + l32) * 8;
-    u32x4_t kop[STEPS][2];
-#pragma unroll
-    for (int st = 0; st < STEPS; ++st)
-#pragma unroll
-      for (int pl = 0; pl < 2; ++pl) kop[st][pl] = kvb[(st * 2 + pl) * 64];
+    const Operands op = L::kStages == 1 ? given : read_operands(buf);
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       if (qt > 0 && q0 + 32 * qt >= N) continue;
@@ -194,9 +208,9 @@ __global__ __launch_bounds__(128 * kRows, 2) void triattn_core_h2_f32(TriattnF32
       if (has_mb) s = mask_step(mb * logit_scale, s);
 #pragma unroll
       for (int st = 0; st < STEPS; ++st) {  // smallest terms first
-        s = mfma_32x32x16_f16(kop[st][1], qop[qt][st][0], s);
-        s = mfma_32x32x16_f16(kop[st][0], qop[qt][st][1], s);
-        s = mfma_32x32x16_f16(kop[st][0], qop[qt][st][0], s);
+        s = mfma_32x32x16_f16(op.k[st][1], qop[qt][st][0], s);
+        s = mfma_32x32x16_f16(op.k[st][0], qop[qt][st][1], s);
+        s = mfma_32x32x16_f16(op.k[st][0], qop[qt][st][0], s);
       }
       float lsum = 0.f;
       if constexpr (kTrack) {
@@ -237,14 +251,12 @@ __global__ __launch_bounds__(128 * kRows, 2) void triattn_core_h2_f32(TriattnF32
         u32x4_t ph, pl;
         split8h(x, ph, pl);
         if constexpr (STEPS == 1) {
-          const u32x4_t v = kvb[L::kKv + st * 64];
-          oacc[qt] = mfma_32x32x16_f16(v, pl, oacc[qt]);
-          oacc[qt] = mfma_32x32x16_f16(v, ph, oacc[qt]);
+          oacc[qt] = mfma_32x32x16_f16(op.v[st][0], pl, oacc[qt]);
+          oacc[qt] = mfma_32x32x16_f16(op.v[st][0], ph, oacc[qt]);
         } else {
-          const u32x4_t vh = kvb[L::kKv + (st * 2) * 64], vl = kvb[L::kKv + (st * 2 + 1) * 64];
-          oacc[qt] = mfma_32x32x16_f16(vl, ph, oacc[qt]);
-          oacc[qt] = mfma_32x32x16_f16(vh, pl, oacc[qt]);
-          oacc[qt] = mfma_32x32x16_f16(vh, ph, oacc[qt]);
+          oacc[qt] = mfma_32x32x16_f16(op.v[st][STEPS - 1], ph, oacc[qt]);
+          oacc[qt] = mfma_32x32x16_f16(op.v[st][0], pl, oacc[qt]);
+          oacc[qt] = mfma_32x32x16_f16(op.v[st][0], ph, oacc[qt]);
         }
       }
     }
@@ -254,7 +266,8 @@ __global__ __launch_bounds__(128 * kRows, 2) void triattn_core_h2_f32(TriattnF32
   float mv_next;
   auto first_loads = [&]() {
     mv_next = load_mask(0);
-    issue_loads(0, 0);
+    issue_bias(0, 0);
+    issue_kv(0, 0);
   };
   auto pass = [&](auto track) {
 #pragma unroll
@@ -270,8 +283,16 @@ __global__ __launch_bounds__(128 * kRows, 2) void triattn_core_h2_f32(TriattnF32
       const float mb = mask_bias(kt, mv_next);
       const int ktn = kt + 1 < nkt ? kt + 1 : nkt - 1;
       mv_next = load_mask(ktn);
-      issue_loads(ktn, buf ^ 1);
-      tile(track, buf, mb);
+      issue_bias(ktn, buf ^ 1);
+      Operands op;
+      if (L::kStages == 1) {
+        op = read_operands(buf);
+        wait_lds_reads();
+        __builtin_amdgcn_s_barrier();  // both waves of the row hold the operands in registers: their place is free
+        compiler_fence();
+      }
+      issue_kv(ktn, buf ^ 1);
+      tile(track, buf, mb, op);
       compiler_fence();
     };
     for (int kt = 0; kt < nkt; kt += 2) {
