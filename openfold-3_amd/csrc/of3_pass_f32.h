@@ -7,6 +7,7 @@
 #include "of3_launch.h"
 #include "of3_pair_f32.h"
 #include "of3_split.h"
+#include "of3_weight_split.h"
 
 namespace of3 {
 namespace pass_f32 {
@@ -228,6 +229,39 @@ __device__ __forceinline__ f32x16_t unit_product(const PassTile<C>& t, const u32
   return acc;
 }
 
+// Residual and result rows of a tile of 32 positions, 16 channels to a lane, through buffer descriptors: a lane whose position
+// lies past the end has an offset past the range, its loads return zeros and its stores are dropped, and without a
+// residual so does every load.  No branch lies around them, so the compiler counts what is in flight: a wait for the
+// residual leaves the next tile's rows, requested after it, in flight, and a wait for those the stores.
+struct Row16 {
+  u32x4_t v[4];
+};
+struct RowTile {
+  __amdgpu_buffer_rsrc_t z, out;
+  __device__ __forceinline__ RowTile(const float* zp, float* op, int64_t first, bool add_residual)
+      : z(buffer_rsrc(zp + first, add_residual ? 0x7fffffff : 0)), out(buffer_rsrc(op + first, 0x7fffffff)) {}
+  // of the lane's position and 16 channels from c0 + 16 (lane half) on; a position's distance to the first one fits 31 bits: rows_aligned
+  __device__ __forceinline__ uint32_t offset(int j0, int N, int64_t stride_k, int c0) const {
+    const Lane at = lane_here();
+    return j0 + at.l32 < N ? (uint32_t)(((uint32_t)at.l32 * (uint32_t)stride_k + c0 + 16 * at.lh) * sizeof(float)) : 0x80000000u;
+  }
+  __device__ __forceinline__ Row16 load(uint32_t off) const {
+    Row16 r;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) r.v[a] = __builtin_amdgcn_raw_buffer_load_b128(z, off + 16 * a, 0, 0);
+    return r;
+  }
+  __device__ __forceinline__ void store(uint32_t off, const f32x16_t& v, const Row16& res) const {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      u32x4_t r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = __float_as_uint(__uint_as_float(res.v[a][e]) + v[4 * a + e]);
+      __builtin_amdgcn_raw_buffer_store_b128(r, out, off + 16 * a, 0, 0);
+    }
+  }
+};
+
 // out row (16 channels from op on) = [residual +] v * g
 __device__ __forceinline__ void store_row16(const float* zp, float* op, const f32x16_t& v, bool add_residual) {
   float4 z[4];
@@ -249,7 +283,7 @@ __device__ __forceinline__ int grid_slot() {
 }
 
 inline bool rows_aligned(const float* p, const PairView& v) {
-  return (reinterpret_cast<uintptr_t>(p) & 15u) == 0 && ((v.stride_b | v.stride_r | v.stride_k) & 3) == 0;
+  return (reinterpret_cast<uintptr_t>(p) & 15u) == 0 && ((v.stride_b | v.stride_r | v.stride_k) & 3) == 0 && near_rows(v.stride_r, v.stride_k);
 }
 
 // persistent grid: what fits the device at once, at most one work-group per tile

@@ -76,7 +76,9 @@ inline bool trimul_split_widths(long C, long CH) { return C % 16 == 0 && CH % 16
 inline bool triattn_split_widths(long C, long H, long D) { return C % 16 == 0 && (H * D) % 16 == 0; }
 inline bool transition_split_widths(long C, long HID) { return C % 16 == 0 && HID % 128 == 0; }
 
-// the shapes whose passes hold fp16 terms (pair_pass_f32.hip, transition_f32.hip); the tensors' rows have to be on 16-byte boundaries too
+// the shapes whose passes hold fp16 terms (pair_pass_f32.hip, transition_f32.hip); the tensors' rows have to be on 16-byte boundaries too,
+// and 32 positions of a row or of a column within the 31 bits of a buffer offset
+inline bool near_rows(int64_t stride_r, int64_t stride_k) { return stride_r < (1 << 24) && stride_k < (1 << 24); }
 inline bool trimul_half_shapes(long B, long N, long C, long CH) {
   const long Np = (N + 31) / 32 * 32;
   return C == CH && (C == 64 || C == 128) && Np * Np * 2 <= 0x7fffffffL && B * (N + 3) * (Np / 32) <= 0x3fffffffL;

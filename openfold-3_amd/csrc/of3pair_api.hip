@@ -1030,7 +1030,7 @@ struct BlockDims {
   int dtype;
   int64_t B, N, C, CH, H, D, HID;
   float inf;
-  bool rows16 = false;  // fp32: z and the result have their rows on 16-byte boundaries
+  bool rows16 = false;  // fp32: z and the result have their rows on 16-byte boundaries, and near each other
   bool wide() const { return dtype == OF3_DTYPE_F32; }
   int weights() const { return OF3_PAIR_BLOCK_WEIGHTS - (HID == 0 ? 5 : 0); }
   int64_t prepared_bytes() const {
@@ -1199,7 +1199,8 @@ static bool pair_block_args_ok(const BlockDims& d, const void* const* weights, c
 }
 
 static bool rows16(const void* z, const void* out, const int64_t z_strides[3]) {
-  return aligned16(z) && aligned16(out) && ((z_strides[0] | z_strides[1] | z_strides[2]) & 3) == 0;
+  return aligned16(z) && aligned16(out) && ((z_strides[0] | z_strides[1] | z_strides[2]) & 3) == 0 &&
+         of3::near_rows(z_strides[1], z_strides[2]);
 }
 
 int64_t of3_pair_block_workspace_bytes(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH, int64_t H, int64_t D,

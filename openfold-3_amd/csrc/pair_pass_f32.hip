@@ -33,27 +33,31 @@ __device__ __forceinline__ uint32_t swap_adjacent(uint32_t v) {
 
 // ---- triangle multiplication, input pass: a, b = mask * sigmoid(LN(z) Wg^T) * (LN(z) Wp^T) ------------------
 // Wave = gate and projection of one 32-channel tile of a or b: two matrices, 128 registers of split operands at 128
-// channels.  A work-group has four waves: at
-// 64 channels a and b, at 128 one of the two, so that two work-groups share a CU and the products of one run beside
-// the LayerNorm and the stores of the other (one work-group of eight waves in step: 468 against 462 us at N = 768).  Tile = 32 columns k of one row; four
+// channels.  At 64 channels a work-group of four waves has a and b.  At 128 it has a and b in eight waves, so that a tile is read
+// and normalised once, as long as there is more than a tile per CU; below that four waves of one of the two, which
+// spread over all CUs (us, four / eight waves: pair stack N = 80 116.8 / 117.9, 200 310.0 / 309.3, 768 4590 / 4465, trunk 384 1260 / 1204).
+// Bytes per tile: 16 KB read, 32 KB written; N = 768 359 us with two barriers per tile and every tile read by two work-groups,
+// 324 now (212 without the products, 267 without the stores: matrix and vector time and the transfers still add up, at the clock
+// that they allow together).
+// Tile = 32 columns k of one row; four
 // consecutive rows of a panel are consecutive tiles of one XCD, so that the 64-byte pieces a tile writes per channel
 // and term meet in L2 as whole lines.
 template <int C>
 struct ProjLds {
-  static constexpr size_t kBytes = (size_t)HalfTile<C>::SLOTS * 16 + (2 * C + 64) * sizeof(float);
+  static constexpr size_t kBytes = (size_t)2 * HalfTile<C>::SLOTS * 16 + (2 * C + 128) * sizeof(float);
 };
 
-template <int C>
-__global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int panels, int row_groups, int total) {
+template <int C, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int panels, int row_groups, int total) {
   typedef HalfTile<C> Tile;
-  constexpr int NW = 4, KS = C / 16, OT = C / 32, TASKS = 8 / NW;
+  constexpr int KS = C / 16, OT = C / 32, TASKS = 8 / NW;
   constexpr bool kOneSide = OT == NW;  // a and b in work-groups of their own
+  constexpr bool kStagger = NW == 8;
   extern __shared__ u32x4_t lds[];
-  const Tile xn = {lds};
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  float* ln = reinterpret_cast<float*>(lds + Tile::SLOTS);  // [2][C], times the scale of the activations
-  float* msk = ln + 2 * C;                                 // [2][32]
+  float* ln = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS);  // [2][C], times the scale of the activations
+  float* msk = ln + 2 * C;                                 // [4][32]
   const int slot = grid_slot(), N = p.N, pair = kOneSide ? slot & 1 : wave / OT, ot = wave % OT;
   const WeightX3 Wg = pair ? p.s_bg : p.s_ag, Wp = pair ? p.s_bp : p.s_ap;
   const WeightScales sg = Wg.scales()[ot], sp = Wp.scales()[ot];
@@ -62,6 +66,7 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
   load_unit<C, 2>(Wp, ot, lane, wp);
   for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_in_w[c] * sg.input, ln[C + c] = p.ln_in_b[c] * sg.input;
   const float out_scale = sp.unscale * sp.output;
+  wait_vmcnt<0>();  // the weights have landed: no wait for them, and with it for the rows in flight, inside the loop
   __syncthreads();
 
   struct Place {
@@ -95,10 +100,11 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
     if (p.mask) mraw = p.mask[t.b * p.mv.stride_b + r * p.mv.stride_r + k * p.mv.stride_k];
   };
 
-  const int step = kOneSide ? gridDim.x / 2 : gridDim.x;
-  int id = kOneSide ? slot >> 1 : slot, buf = 0;
-  if (id < total) load_tile(id);
-  for (; id < total; id += step, buf ^= 1) {
+  const int step = kOneSide ? gridDim.x / 2 : gridDim.x, first_id = kOneSide ? slot >> 1 : slot;
+  // rows of the n-th tile of this work-group, in registers, to its LDS tile; requests those of the next one
+  auto normalise = [&](int n) {
+    const int id = first_id + n * step;
+    const Tile xn = {lds + (n & 1) * Tile::SLOTS};
     const Place t = place(id);
     const Lane here = lane_here();
 #pragma unroll
@@ -109,9 +115,22 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) xn.store4(pos, li + 16 * e, y[e]);
     }
-    if (tid < 32) msk[32 * buf + tid] = mraw;
+    if (tid < 32) msk[32 * (n & 3) + tid] = mraw;
     load_tile(id + step < total ? id + step : id);
-    __syncthreads();  // the tile is complete
+  };
+  if (first_id >= total) return;  // the whole work-group
+  const int count = (total - first_id + step - 1) / step;
+  // Interval n lies between the barrier that completes tile n and the next one.  In it the early half of a work-group of eight waves
+  // finishes tile n - 1, normalises tile n + 1 and takes the products of tile n, the late half takes the products first, so that
+  // of the two waves of a SIMD (w and w + 4) one has vector work while the other has matrix work: 4500 -> 4470 us per pair stack N = 768.
+  const bool early = kStagger && wave < NW / 2;
+  load_tile(first_id);
+  normalise(0);
+  __syncthreads();
+  if (early && count > 1) normalise(1);
+  for (int n = 0; n < count; ++n) {
+    const Tile xn = {lds + (n & 1) * Tile::SLOTS};
+    const Place t = place(first_id + n * step);
     HalfSum<C, false> sum_g, sum_p;
     const Lane at = lane_here();
 #pragma unroll
@@ -122,7 +141,8 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
       sum_p.step(wp[s], op);
     }
     const f32x16_t ag = sum_g.total(), ap = sum_p.total();
-    __syncthreads();  // everybody has read it
+    if (early && n + 1 < count) __syncthreads();
+    wait_vmcnt<0>();  // the rows in flight since a product ago, ahead of the stores, so that nobody waits for these
     // channels in the lanes, positions in the registers: registers 8 st .. + 7 are the k-values 16 st + 8 (e >> 2)
     // + 4 lh + (e & 3), stored as the 8 consecutive columns 16 st + 8 lh .. of the panel row (a and b in the same
     // order, which is all a sum over k needs); positions past N are zero rows and store the panel's padding
@@ -137,7 +157,7 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
         float x[8];
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
-          const float4 m4 = *reinterpret_cast<const float4*>(msk + 32 * buf + 16 * st + 8 * a + 4 * lh);
+          const float4 m4 = *reinterpret_cast<const float4*>(msk + 32 * (n & 3) + 16 * st + 8 * a + 4 * lh);
           const float m[4] = {m4.x, m4.y, m4.z, m4.w};
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -167,19 +187,22 @@ __global__ __launch_bounds__(256, 2) void trimul_proj_pass(TrimulF32 p, int pane
         *reinterpret_cast<u32x4_t*>(lp1 + pl * p.ab_plane) = second;
       }
     }
+    if (n + (early ? 2 : 1) < count) normalise(n + (early ? 2 : 1));
+    if (!early && n + 1 < count) __syncthreads();
   }
 }
 
 // ---- output passes ------------------------------------------------------------------------------------------
 // Wave = one 32-channel tile of the gate and the same tile of the output projection, weights in registers as in the input
-// passes.  The LDS tile holds LayerNorm(z) for the gates,
-// then LayerNorm(x) or the gated attention output in its place.  Four waves per work-group at 128 channels, two
+// passes.  One LDS tile holds LayerNorm(z) for the gates, another LayerNorm(x) or the gated attention output: two barriers per tile.
+// Every load of a tile is requested before the product ahead of its use, residual rows before the next tile's, and nothing waits
+// for a store (N = 768, 268 -> 251 and 256 -> 239 us).  Four waves per work-group at 128 channels, two
 // work-groups per CU; two waves at 64.
 template <int C>
 struct OutLds {
   static constexpr int NW = C / 32;
-  static constexpr size_t kTrimul = (size_t)HalfTile<C>::SLOTS * 16 + (2 * 32 * 2 * NW + 4 * C) * sizeof(float);
-  static constexpr size_t kTriattn = (size_t)HalfTile<C>::SLOTS * 16 + 2 * C * sizeof(float);
+  static constexpr size_t kTrimul = (size_t)2 * HalfTile<C>::SLOTS * 16 + (2 * 32 * 2 * NW + 4 * C) * sizeof(float);
+  static constexpr size_t kTriattn = (size_t)2 * HalfTile<C>::SLOTS * 16 + 2 * C * sizeof(float);
 };
 // the two matrices of an output wave, outputs dealt by rowperm16: lane (position l32, half lh) ends with the outputs
 // 32 ot + 16 lh + v
@@ -201,8 +224,8 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
   typedef HalfTile<C> Tile;
   constexpr int NW = C / 32, TASKS = 8 / NW, NG = 2 * NW;
   extern __shared__ u32x4_t lds[];
-  const Tile tile = {lds};
-  float* red = reinterpret_cast<float*>(lds + Tile::SLOTS);  // [NG][32] means, [NG][32] squared deviations
+  const Tile tile = {lds}, second = {lds + Tile::SLOTS};
+  float* red = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS);  // [NG][32] means, [NG][32] squared deviations
   float* ln = red + 2 * 32 * NG;                             // LayerNorm of z [2][C], of x [2][C], times the activations' scales
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
@@ -214,6 +237,7 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
     ln[c] = p.ln_in_w[c] * sg.input, ln[C + c] = p.ln_in_b[c] * sg.input;
     ln[2 * C + c] = p.ln_out_w[c] * sz.input, ln[3 * C + c] = p.ln_out_b[c] * sz.input;
   }
+  wait_vmcnt<0>();  // the weights
   __syncthreads();
 
   struct Place {
@@ -231,7 +255,7 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
   RowRegs<C> zraw[TASKS];
   float xraw[16];  // channels 8 xg .. + 7 and C / 2 + 8 xg .. + 7
   const size_t NN = (size_t)N * N;
-  auto load_tile = [&](int id) {
+  auto load_z = [&](int id) {
     const Lane here = lane_here();
     const int li = here.li, lg = here.lg;
     const Place t = place(id);
@@ -242,6 +266,9 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
       j = j < N ? j : N - 1;
       load_row<C>(base + j * p.zc.stride_k, li, zraw[u]);
     }
+  };
+  auto load_x = [&](int id) {
+    const Place t = place(id);
     int j = t.j0 + xpos;
     j = j < N ? j : N - 1;
     const float* xp = p.x + (((size_t)t.b * C + 8 * xg) * N + t.i) * N + j;
@@ -250,9 +277,10 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
   };
 
   int id = grid_slot();
-  if (id < total) load_tile(id);
+  if (id < total) load_z(id), load_x(id);
   for (; id < total; id += gridDim.x) {
     const Place t = place(id);
+    const int next = id + (int)gridDim.x < total ? id + (int)gridDim.x : id;
     const Lane here = lane_here();
 #pragma unroll
     for (int u = 0; u < TASKS; ++u) {
@@ -262,6 +290,7 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) tile.store4(pos, li + 16 * e, y[e]);
     }
+    load_z(next);
     {
       float s = 0.f, q = 0.f;
 #pragma unroll
@@ -272,9 +301,8 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
       red[xg * 32 + xpos] = s;
       red[(NG + xg) * 32 + xpos] = q;
     }
-    __syncthreads();  // LayerNorm(z) is complete
+    __syncthreads();  // LayerNorm(z) is complete, and everybody has finished with the second tile
     const f32x16_t gate = unit_product<C, true>(tile, w.g);
-    __syncthreads();  // everybody has read it
     {
       // mean of the groups' means; squared deviations = within the groups + 16 x those of the groups' means
       float mg[NG], mean = 0.f, q = 0.f;
@@ -290,20 +318,18 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
         float y[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) y[e] = (xraw[8 * hf + e] - mean) * rstd * wv[e] + wv[C + e];
-        tile.store8(xpos, hf * (C / 16) + xg, y);
+        second.store8(xpos, hf * (C / 16) + xg, y);
       }
     }
-    load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
-    __syncthreads();  // LayerNorm(x) is complete
-    f32x16_t acc = unit_product<C, true>(tile, w.o);
-    __syncthreads();  // everybody has read it
-    const Lane out = lane_here();
-    if (t.j0 + out.l32 < N) {
-      const int64_t off = t.b * p.zc.stride_b + t.i * p.zc.stride_r + (t.j0 + out.l32) * p.zc.stride_k + 32 * wave + 16 * out.lh;
+    const RowTile rows(p.z, p.out, t.b * p.zc.stride_b + t.i * p.zc.stride_r + t.j0 * p.zc.stride_k, p.add_residual);
+    const uint32_t off = rows.offset(t.j0, N, p.zc.stride_k, 32 * wave);
+    const Row16 res = rows.load(off);
+    load_x(next);
+    __syncthreads();  // LayerNorm(x) is complete, and everybody has finished with the first tile
+    f32x16_t acc = unit_product<C, true>(second, w.o);
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[v] = acc[v] * sz.unscale * sigmoid_hw_f32(gate[v], sg.unscale);
-      store_row16(p.z + off, p.out + off, acc, p.add_residual);
-    }
+    for (int v = 0; v < 16; ++v) acc[v] = acc[v] * sz.unscale * sigmoid_hw_f32(gate[v], sg.unscale);
+    rows.store(off, acc, res);
   }
 }
 
@@ -341,6 +367,7 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
     const int t = c / C * p.D / 32;  // the head's tile of q and k
     wb[c] = p.w_b[c] * (p.s_q.scales()[t].output * p.s_k.scales()[t].output / sc.input);
   }
+  wait_vmcnt<0>();  // the weights
   __syncthreads();
   // q / sqrt(c) after the projection (attention.py:283-284)
   const float out_scale = sc.unscale * sc.output * (kind == 0 ? 1.0f / sqrtf((float)p.D) : 1.f);
@@ -439,6 +466,7 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
     // l32 % 16 of head 2 ot + l32 / 16, its second term row 16 + l32 % 16).
     if (kind < 2) {
       const f32x16_t acc = product(std::true_type{}, xn);
+      wait_vmcnt<0>();  // the rows in flight, ahead of the stores
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
         const size_t slot = narrow ? ((row * H + 2 * ot + st) * nt + jt) * 64 + lane : (((row * H + ot) * nt + jt) * 2 + st) * 64 + lane;
@@ -446,6 +474,7 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
       }
     } else {
       const f32x16_t acc = product(std::false_type{}, xn);
+      wait_vmcnt<0>();
       const int head = narrow ? 2 * ot + (l32 >> 4) : ot, vrow = narrow ? (l32 & 15) : l32;
 #pragma unroll
       for (int st = 0; st < 2; ++st)
@@ -461,8 +490,8 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
   typedef HalfTile<C> Tile;
   constexpr int NW = C / 32, TASKS = 8 / NW;
   extern __shared__ u32x4_t lds[];
-  const Tile tile = {lds};
-  float* ln = reinterpret_cast<float*>(lds + Tile::SLOTS);  // [2][C], times the scale of the activations
+  const Tile tile = {lds}, second = {lds + Tile::SLOTS};
+  float* ln = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS);  // [2][C], times the scale of the activations
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int N = p.N;
@@ -472,6 +501,7 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
   OutWeights<C> w;
   w.load(p.s_g, p.s_o, wave, l32, lh);
   for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * sg.input, ln[C + c] = p.ln_b[c] * sg.input;
+  wait_vmcnt<0>();  // the weights
   __syncthreads();
 
   auto place = [&](int id, int& b, int& i) {  // returns the first position
@@ -482,7 +512,7 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
   };
   RowRegs<C> raw[TASKS];
   float4 oraw[4];
-  auto load_tile = [&](int id) {
+  auto load_rows = [&](int id) {
     const Lane here = lane_here();
     const int li = here.li, lg = here.lg;
     int b, i;
@@ -493,6 +523,11 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
       j = j < N ? j : N - 1;
       load_row<C>(p.x + b * p.xv.stride_b + i * p.xv.stride_r + j * p.xv.stride_k, li, raw[u]);
     }
+  };
+  auto load_o = [&](int id) {
+    const Lane here = lane_here();
+    int b, i;
+    const int j0 = place(id, b, i);
     const int j = j0 + here.l32 < N ? j0 + here.l32 : N - 1;
     const float* op = p.o + (((size_t)b * N + i) * N + j) * C + 32 * wave + 16 * here.lh;
 #pragma unroll
@@ -500,8 +535,9 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
   };
 
   int id = grid_slot();
-  if (id < total) load_tile(id);
+  if (id < total) load_rows(id), load_o(id);
   for (; id < total; id += gridDim.x) {
+    const int next = id + (int)gridDim.x < total ? id + (int)gridDim.x : id;
     int b, i;
     const int j0 = place(id, b, i);
     const Lane here = lane_here();
@@ -513,9 +549,9 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) tile.store4(pos, li + 16 * e, y[e]);
     }
-    __syncthreads();  // LayerNorm(x) is complete
+    load_rows(next);
+    __syncthreads();  // LayerNorm(x) is complete, and everybody has finished with the second tile
     const f32x16_t gate = unit_product<C, true>(tile, w.g);
-    __syncthreads();  // everybody has read it
     const Lane mid = lane_here();
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
@@ -524,33 +560,43 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
       float y[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) y[e] = ov[e] * o_scale * sigmoid_hw_f32(gate[8 * hf + e], sg.unscale);
-      tile.store8(mid.l32, 4 * wave + 2 * mid.lh + hf, y);
+      second.store8(mid.l32, 4 * wave + 2 * mid.lh + hf, y);
     }
-    load_tile(id + (int)gridDim.x < total ? id + gridDim.x : id);
-    __syncthreads();  // the gated output is complete
-    f32x16_t acc = unit_product<C, true>(tile, w.o);
-    __syncthreads();  // everybody has read it
-    const Lane out = lane_here();
-    if (j0 + out.l32 < N) {
+    const RowTile rows(p.x, p.out, b * p.xv.stride_b + i * p.xv.stride_r + j0 * p.xv.stride_k, p.add_residual);
+    const uint32_t off = rows.offset(j0, N, p.xv.stride_k, 32 * wave);
+    const Row16 res = rows.load(off);
+    load_o(next);
+    __syncthreads();  // the gated output is complete, and everybody has finished with the first tile
+    f32x16_t acc = unit_product<C, true>(second, w.o);
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[v] *= unscale;
-      const int64_t off = b * p.xv.stride_b + i * p.xv.stride_r + (j0 + out.l32) * p.xv.stride_k + 32 * wave + 16 * out.lh;
-      store_row16(p.x + off, p.out + off, acc, p.add_residual);
-    }
+    for (int v = 0; v < 16; ++v) acc[v] *= unscale;
+    rows.store(off, acc, res);
   }
 }
 
+template <int C, int NW>
+hipError_t launch_trimul_proj(const TrimulF32& p, int panels, int row_groups, long total, hipStream_t stream) {
+  constexpr bool kOneSide = C / 32 == NW;
+  unsigned grid = 0;
+  hipError_t e = resident_grid<trimul_proj_pass<C, NW>>(64 * NW, ProjLds<C>::kBytes, kOneSide ? 2 * total : total, &grid);
+  if (e != hipSuccess) return e;
+  if (kOneSide) grid &= ~1u;  // a and b
+  hipLaunchKernelGGL((trimul_proj_pass<C, NW>), dim3(grid), dim3(64 * NW), ProjLds<C>::kBytes, stream, p, panels, row_groups, (int)total);
+  return hipGetLastError();
+}
 template <int C>
 hipError_t launch_trimul_proj(const TrimulF32& p, hipStream_t stream) {
   const int panels = p.Np / 32, row_groups = (p.N + 3) / 4;
   const long total = (long)p.B * row_groups * panels * 4;
   if (total > 0x3fffffffL) return hipErrorInvalidValue;
-  unsigned grid = 0;
-  hipError_t e = resident_grid<trimul_proj_pass<C>>(256, ProjLds<C>::kBytes, C == 128 ? 2 * total : total, &grid);
-  if (e != hipSuccess) return e;
-  if (C == 128) grid &= ~1u;  // a and b
-  hipLaunchKernelGGL(trimul_proj_pass<C>, dim3(grid), dim3(256), ProjLds<C>::kBytes, stream, p, panels, row_groups, (int)total);
-  return hipGetLastError();
+  if constexpr (C == 128) {
+    static int cache[kMaxDevices];
+    int cus = 0;
+    const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+    if (e != hipSuccess) return e;
+    if (total > cus) return launch_trimul_proj<C, 8>(p, panels, row_groups, total, stream);
+  }
+  return launch_trimul_proj<C, 4>(p, panels, row_groups, total, stream);
 }
 
 template <int C>

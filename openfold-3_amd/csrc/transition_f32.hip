@@ -59,7 +59,9 @@ __device__ __forceinline__ float smallest_inv_bound(const WeightX3& W, int n) {
 // the first four waves and its output projection in the others; the updated rows stay in LDS.
 // BIAS: and ends with the pair bias of the block's attention over s (pair_bias_pass: same steps, same bits), from the rows that it has just finished. Four
 // trunk blocks at N = 24 / 45 / 64 / 80 / 90 527 / 579 / 587 / 696 / 758 us, so 502 / 554 / 565 / 671 / 736 (a launch, and z read once more).
-template <int C, int S, int NPT, bool AFTER, bool BIAS>
+// KEEP: the hidden dimension is one slice, a wave's operands of all three matrices stay in registers (96 of 208).  Three templates of 200, 64
+// channels, n = 2, two transitions of 2100 tiles: the operands fetched again for every tile 107 us, so 90.
+template <int C, int S, int NPT, bool AFTER, bool BIAS, bool KEEP>
 __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
   static_assert(AFTER || !BIAS, "one tile per work-group");
   static_assert(!AFTER || (C == 128 && NPT == 1), "eight waves: a gate and an output tile for each 32 channels");
@@ -71,8 +73,10 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
   constexpr int KSPLIT = NW / (OT * NPT);          // waves sharing an output tile's sum in the second
   constexpr int OSTEPS = 2 * S / KSPLIT;           // its k-steps per slice and wave
   // steps that an operand is requested ahead: an L2 read takes about as long as 24 MFMAs of two waves per SIMD
-  constexpr int DA = XT == 1 ? 2 : 1, DO = 4;
+  constexpr int DA = KEEP ? KS : XT == 1 ? 2 : 1, DO = KEEP ? OSTEPS : 4;
   static_assert(OSTEPS >= DO && KS >= DA, "");
+  // the residual before the next tile's rows and a slice's scales before its operands; there they would spill
+  constexpr bool kEarly = !(C == 64 && S == 8 && NPT == 2);
   extern __shared__ u32x4_t lds[];
   u32x4_t* const hid = lds + NPT * XTile::SLOTS;
   float* ln = reinterpret_cast<float*>(hid + NPT * HTile::SLOTS);  // [2][C]
@@ -123,6 +127,13 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
     for (int pl = 0; pl < 2; ++pl) no[s % DO][pl] = wo[pl * po + at];
   };
 
+  if constexpr (KEEP) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) fetch_ab(0, s);
+#pragma unroll
+    for (int s = 0; s < OSTEPS; ++s) fetch_o(0, s);
+    wait_vmcnt<0>();  // no wait for them, and with it for the rows in flight, inside the loop
+  }
   const int tiles = (p.total + NPT - 1) / NPT;
   int tile = grid_slot();
   if (tile < tiles) load_tile(tile);
@@ -221,10 +232,31 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
         for (int e = 0; e < C / 64; ++e) xn.store4(pos, here.li + 16 * e, y[e]);
       }
     }
+    // this wave's rows of the result
+    const int pn = NPT * tile + pt_b;
+    int j0;
+    const int r = row_of(pn < p.total ? pn : p.total - 1, j0), bb = r / p.R, i = r - bb * p.R;
+    const int64_t row0 = bb * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j0 * p.xv.stride_k;
+    Row16 res;
+    float m = 1.f;
+    const RowTile out_rows(p.x, p.out, AFTER ? 0 : row0, p.add_residual && kh == 0);
+    const uint32_t off = out_rows.offset(j0, pn < p.total && kh == 0 ? L : 0, p.xv.stride_k, 32 * ot);
+    // before the next tile's rows, so that a wait for these leaves those in flight
+    auto load_residual = [&] {
+      const int j = j0 + lane_here().l32 < L ? j0 + lane_here().l32 : L - 1;
+      if (p.mask) m = p.mask[bb * p.mv.stride_b + i * p.mv.stride_r + (int64_t)j * p.mv.stride_k];
+      if (!AFTER) res = out_rows.load(off);
+    };
+    if constexpr (!KEEP) {
 #pragma unroll
-    for (int s = 0; s < DA; ++s) fetch_ab(0, s);
+      for (int s = 0; s < DA; ++s) fetch_ab(0, s);
+    }
     HalfSum<128, true> osum;
     for (int slice = 0; slice < slices; ++slice) {
+      // requested ahead of the operands (where the registers allow it): behind them they wait for every operand in flight
+      float ua, ub;
+      auto load_scales = [&] { ua = p.s_a.scales()[slice * S + ht].unscale, ub = ua * p.s_b.scales()[slice * S + ht].unscale * h_scale; };
+      if (kEarly) load_scales();
       __syncthreads();  // the activations (first slice), or: everybody has read the slice before
       f32x16_t a[XT], b[XT];
       HalfSum<C, true> sum_a[XT], sum_b[XT];
@@ -250,7 +282,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
           }
           if (s + 1 < KS) read_x(s + 1);
           if (s + DA < KS) fetch_ab(slice, s + DA);
-          if (s + 1 == KS) {
+          if (!KEEP && s + 1 == KS) {
 #pragma unroll
             for (int q = 0; q < DO; ++q) fetch_o(slice, q);
           }
@@ -265,11 +297,9 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
 #pragma unroll
         for (int t = 0; t < XT; ++t) a[t] = sum_a[t].total(), b[t] = sum_b[t].total();
       }
+      if (!kEarly) load_scales();
       {
         const Lane at = lane_here();
-        const WeightScales* ta = p.s_a.scales() + slice * S + ht;
-        const WeightScales* tb = p.s_b.scales() + slice * S + ht;
-        const float ua = ta->unscale, ub = ua * tb->unscale * h_scale;
 #pragma unroll
         for (int t = 0; t < XT; ++t) {
           const HTile h = {hid + (pt_a + t) * HTile::SLOTS};
@@ -299,7 +329,8 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
           if (s + 1 < OSTEPS) read_h(s + 1);
           if (s + DO < OSTEPS) fetch_o(slice, s + DO);
           if (s + DO == OSTEPS) {  // after the last weights: loads return in order
-            if (last) {
+            if (KEEP || last) {
+              if (kEarly) load_residual();
               if (!AFTER) load_tile(tile + (int)gridDim.x < tiles ? tile + gridDim.x : tile);
             } else
 #pragma unroll
@@ -312,6 +343,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       }
     }
     f32x16_t oacc = osum.total();
+    if (!kEarly) load_residual();
     const Lane at = lane_here();
     if (KSPLIT > 1) {  // the waves of an output tile add up through the hidden tile's memory
       __syncthreads();
@@ -332,17 +364,14 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
     }
 #pragma unroll
     for (int v = 0; v < 16; ++v) oacc[v] *= unscale;
-    int j0;
-    const int pn = NPT * tile + pt_b;
-    const int r = row_of(pn, j0), bb = r / p.R, i = r - bb * p.R, j = j0 + at.l32;
+    const int j = j0 + at.l32;
+    if (p.mask) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) oacc[v] *= m;
+    }
     if constexpr (BIAS) {
       float* row = rows + at.l32 * (C + kRowLd) + 32 * ot + 16 * at.lh;
       if (kh == 0) {
-        if (p.mask) {
-          const float m = j < L ? p.mask[bb * p.mv.stride_b + i * p.mv.stride_r + (int64_t)j * p.mv.stride_k] : 0.f;
-#pragma unroll
-          for (int v = 0; v < 16; ++v) oacc[v] *= m;
-        }
         store_row16(row, row, oacc, 1);
         if (j < L) {
           float4* dst = reinterpret_cast<float4*>(p.out + bb * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j * p.xv.stride_k + 32 * ot + 16 * at.lh);
@@ -394,27 +423,23 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       }
       return;
     }
-    if (pn < p.total && j < L) {
-      const int64_t off = bb * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j * p.xv.stride_k + 32 * ot + 16 * at.lh;
-      if (p.mask) {
-        const float m = p.mask[bb * p.mv.stride_b + i * p.mv.stride_r + (int64_t)j * p.mv.stride_k];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) oacc[v] *= m;
-      }
-      store_row16(AFTER ? rows + at.l32 * (C + kRowLd) + 32 * ot + 16 * at.lh : p.x + off, p.out + off, oacc, p.add_residual);
+    if constexpr (AFTER) {
+      if (j < L) store_row16(rows + at.l32 * (C + kRowLd) + 32 * ot + 16 * at.lh, p.out + row0 + (int64_t)at.l32 * p.xv.stride_k + 32 * ot + 16 * at.lh, oacc, p.add_residual);
+      return;
+    } else {
+      out_rows.store(off, oacc, res);
     }
-    if (AFTER) return;
   }
 }
 
-template <int C, int S, int NPT, bool AFTER = false, bool BIAS = false>
+template <int C, int S, int NPT, bool AFTER = false, bool BIAS = false, bool KEEP = false>
 hipError_t launch(const TransitionPass& p, hipStream_t stream) {
   constexpr size_t lds = transition_lds<C, S, NPT, AFTER, BIAS>();
   unsigned grid = 0;
-  hipError_t e = resident_grid<transition_pass<C, S, NPT, AFTER, BIAS>>(512, lds, (p.total + NPT - 1) / NPT, &grid);
+  hipError_t e = resident_grid<transition_pass<C, S, NPT, AFTER, BIAS, KEEP>>(512, lds, (p.total + NPT - 1) / NPT, &grid);
   if (e != hipSuccess) return e;
   if (AFTER) grid = (unsigned)p.total;  // a tile each
-  hipLaunchKernelGGL((transition_pass<C, S, NPT, AFTER, BIAS>), dim3(grid), dim3(512), lds, stream, p);
+  hipLaunchKernelGGL((transition_pass<C, S, NPT, AFTER, BIAS, KEEP>), dim3(grid), dim3(512), lds, stream, p);
   return hipGetLastError();
 }
 
@@ -486,7 +511,10 @@ hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, 
     return launch<128, 8, 1, true>(p, stream);
   }
   const bool large = p.total >= 4l * cus;  // two tiles of 64 positions for every CU
-  if (a.HID % 256 != 0) return a.C == 128 ? launch<128, 4, 2>(p, stream) : launch<64, 4, 2>(p, stream);
+  if (a.HID % 256 != 0) {
+    if (a.C == 128) return launch<128, 4, 2>(p, stream);
+    return a.HID == 128 ? launch<64, 4, 2, false, false, true>(p, stream) : launch<64, 4, 2>(p, stream);
+  }
   if (a.C == 128) return large ? launch<128, 8, 2>(p, stream) : launch<128, 8, 1>(p, stream);
   return large ? launch<64, 8, 2>(p, stream) : launch<64, 8, 1>(p, stream);
 }

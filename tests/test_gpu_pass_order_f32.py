@@ -1,0 +1,48 @@
+"""fp32 passes: the two halves of a work-group that take a tile's vector and matrix work in opposite order, at one tile per
+work-group, some with two, and several; and rows too far apart for a buffer offset, which the general kernels serve."""
+import pytest
+import torch
+
+from gpu_util import lib, report  # noqa: F401
+from oracle import pairstack_oracle as orc
+
+import of3pair
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+REL = 1e-5  # of the largest value: some 100 roundings of it, as the other fp32 tests of these modules
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("n", [84, 85, 131, 181])  # 252, 264, 660 and 1104 tiles of 32 positions on 256 CUs
+def test_trimul_tiles_per_work_group(n, masked):
+    lib()
+    c = 128
+    gen = torch.Generator().manual_seed(8600 + n)
+    z = orc.make_pair_input(8601, (1,), n, c)
+    mask = (torch.rand(1, n, n, generator=gen) > 0.2).float() if masked else None
+    p = orc.make_trimul_params(gen, c, c)
+    m = of3pair.TriangleMultiplicationOutgoing(c, c)
+    m.load_state_dict(p, strict=True)
+    print("trimul", n, masked, flush=True)
+    ones = torch.ones(1, n, n) if mask is None else mask
+    want = orc.trimul_update(z.double(), ones.double(), {k: v.double() for k, v in p.items()}, True)
+    got = m.to(DEV).eval()(z.to(DEV), None if mask is None else mask.to(DEV)).cpu()
+    report("update", got, want, atol=REL * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("c", [64, 128])
+def test_rows_far_apart(c):
+    lib()
+    n, heads, far = 5, 4, 1 << 24
+    p = orc.make_block_params(8602, c, c, c // heads, heads)
+    m = of3pair.PairStack(c, c, c // heads, heads)
+    m.load_state_dict(p, strict=True)
+    m = m.to(DEV).eval()
+    z = torch.randn(1, n, n, c, generator=torch.Generator().manual_seed(8603)).to(DEV)
+    apart = torch.zeros(n * far, device=DEV).as_strided((1, n, n, c), (n * far, far, c, 1))
+    apart.copy_(z)
+    mask = torch.ones(1, n, n, device=DEV)
+    print("rows far apart", c, flush=True)
+    want = m(z, mask)
+    report("block", m(apart, mask), want, atol=REL * float(want.abs().max()))
