@@ -236,9 +236,9 @@ __device__ __forceinline__ f32x16_t unit_product(const PassTile<C>& t, const u32
 struct Row16 {
   u32x4_t v[4];
 };
-struct RowTile {
+struct GlobalRows {
   __amdgpu_buffer_rsrc_t z, out;
-  __device__ __forceinline__ RowTile(const float* zp, float* op, int64_t first, bool add_residual)
+  __device__ __forceinline__ GlobalRows(const float* zp, float* op, int64_t first, bool add_residual)
       : z(buffer_rsrc(zp + first, add_residual ? 0x7fffffff : 0)), out(buffer_rsrc(op + first, 0x7fffffff)) {}
   // of the lane's position and 16 channels from c0 + 16 (lane half) on; a position's distance to the first one fits 31 bits: rows_aligned
   __device__ __forceinline__ uint32_t offset(int j0, int N, int64_t stride_k, int c0) const {
@@ -276,6 +276,38 @@ __device__ __forceinline__ void store_row16(const float* zp, float* op, const f3
     *reinterpret_cast<float4*>(op + 4 * a) = r;
   }
 }
+
+// 32 fp32 rows in LDS on their way from a tile's residual to its result: put as they were loaded (16 lanes a row), added to by the waves
+// that own 32 of their channels each, and stored whole, so that a store instruction writes four rows (256 bytes of each) in
+// the place of 16 bytes of 64.  16-byte slots, XOR-swizzled by the position.
+template <int C>
+struct RowTile {
+  static constexpr int ROW = C / 4, SLOTS = 32 * ROW;
+  float4* s;
+  __device__ __forceinline__ float4& at(int pos, int c4) const { return s[pos * ROW + (c4 ^ (pos & (ROW - 1)))]; }
+  __device__ __forceinline__ void put(int pos, int li, const RowRegs<C>& r) const {
+#pragma unroll
+    for (int e = 0; e < C / 64; ++e) at(pos, 16 * e + li) = r.v[e];
+  }
+  // the lane's position and 16 channels from 32 ot + 16 (lane half) on
+  __device__ __forceinline__ void add(int ot, const f32x16_t& v, bool to_residual) const {
+    const Lane here = lane_here();
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      float4& place = at(here.l32, 8 * ot + 4 * here.lh + a);
+      float4 r = make_float4(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);
+      if (to_residual) {
+        const float4 z = place;
+        r.x = z.x + r.x, r.y = z.y + r.y, r.z = z.z + r.z, r.w = z.w + r.w;
+      }
+      place = r;
+    }
+  }
+  __device__ __forceinline__ void store(float* row, int pos, int li) const {
+#pragma unroll
+    for (int e = 0; e < C / 64; ++e) *reinterpret_cast<float4*>(row + 64 * e + 4 * li) = at(pos, 16 * e + li);
+  }
+};
 
 // logical number of a work-group: consecutive numbers run on one XCD where the grid deals evenly
 __device__ __forceinline__ int grid_slot() {

@@ -195,14 +195,16 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
 // ---- output passes ------------------------------------------------------------------------------------------
 // Wave = one 32-channel tile of the gate and the same tile of the output projection, weights in registers as in the input
 // passes.  One LDS tile holds LayerNorm(z) for the gates, another LayerNorm(x) or the gated attention output: two barriers per tile.
-// Every load of a tile is requested before the product ahead of its use, residual rows before the next tile's, and nothing waits
-// for a store (N = 768, 268 -> 251 and 256 -> 239 us).  Four waves per work-group at 128 channels, two
+// Every load of a tile is requested before the product ahead of its use and nothing waits for a store (N = 768, 268 -> 251 and
+// 256 -> 239 us); the rows leave whole, by way of the residual's place in LDS, after the next tile's first barrier (RowTile: -> 235 and 221; lanes
+// that load and store 64 bytes of their own row each kept the address unit busy for 54 and 64 % of the time).
+// Four waves per work-group at 128 channels, two
 // work-groups per CU; two waves at 64.
 template <int C>
 struct OutLds {
   static constexpr int NW = C / 32;
-  static constexpr size_t kTrimul = (size_t)2 * HalfTile<C>::SLOTS * 16 + (2 * 32 * 2 * NW + 4 * C) * sizeof(float);
-  static constexpr size_t kTriattn = (size_t)2 * HalfTile<C>::SLOTS * 16 + 2 * C * sizeof(float);
+  static constexpr size_t kTrimul = (size_t)(2 * HalfTile<C>::SLOTS + RowTile<C>::SLOTS) * 16 + (2 * 32 * 2 * NW + 4 * C) * sizeof(float);
+  static constexpr size_t kTriattn = (size_t)(2 * HalfTile<C>::SLOTS + RowTile<C>::SLOTS) * 16 + 2 * C * sizeof(float);
 };
 // the two matrices of an output wave, outputs dealt by rowperm16: lane (position l32, half lh) ends with the outputs
 // 32 ot + 16 lh + v
@@ -225,7 +227,8 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
   constexpr int NW = C / 32, TASKS = 8 / NW, NG = 2 * NW;
   extern __shared__ u32x4_t lds[];
   const Tile tile = {lds}, second = {lds + Tile::SLOTS};
-  float* red = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS);  // [NG][32] means, [NG][32] squared deviations
+  const RowTile<C> rows = {reinterpret_cast<float4*>(lds + 2 * Tile::SLOTS)};
+  float* red = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS + RowTile<C>::SLOTS);  // [NG][32] means, [NG][32] squared deviations
   float* ln = red + 2 * 32 * NG;                             // LayerNorm of z [2][C], of x [2][C], times the activations' scales
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
@@ -276,7 +279,19 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
     for (int e = 0; e < 8; ++e) xraw[e] = xp[e * NN], xraw[8 + e] = xp[(C / 2 + e) * NN];
   };
 
+  // result rows of a tile, as the threads have normalised them
+  auto store_rows = [&](const Place& t) {
+    const Lane here = lane_here();
+    float* base = p.out + t.b * p.zc.stride_b + t.i * p.zc.stride_r;
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      const int pos = 4 * (wave + NW * u) + here.lg;
+      if (t.j0 + pos < N) rows.store(base + (t.j0 + pos) * p.zc.stride_k, pos, here.li);
+    }
+  };
   int id = grid_slot();
+  bool first = true;
+  Place before = {};
   if (id < total) load_z(id), load_x(id);
   for (; id < total; id += gridDim.x) {
     const Place t = place(id);
@@ -290,7 +305,6 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) tile.store4(pos, li + 16 * e, y[e]);
     }
-    load_z(next);
     {
       float s = 0.f, q = 0.f;
 #pragma unroll
@@ -301,7 +315,14 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
       red[xg * 32 + xpos] = s;
       red[(NG + xg) * 32 + xpos] = q;
     }
-    __syncthreads();  // LayerNorm(z) is complete, and everybody has finished with the second tile
+    __syncthreads();  // LayerNorm(z) and the rows of the tile before are complete, and everybody has finished with the second tile
+    if (!first) store_rows(before);
+    if (p.add_residual) {
+      const Lane at = lane_here();
+#pragma unroll
+      for (int u = 0; u < TASKS; ++u) rows.put(4 * (wave + NW * u) + at.lg, at.li, zraw[u]);
+    }
+    load_z(next);
     const f32x16_t gate = unit_product<C, true>(tile, w.g);
     {
       // mean of the groups' means; squared deviations = within the groups + 16 x those of the groups' means
@@ -321,16 +342,18 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
         second.store8(xpos, hf * (C / 16) + xg, y);
       }
     }
-    const RowTile rows(p.z, p.out, t.b * p.zc.stride_b + t.i * p.zc.stride_r + t.j0 * p.zc.stride_k, p.add_residual);
-    const uint32_t off = rows.offset(t.j0, N, p.zc.stride_k, 32 * wave);
-    const Row16 res = rows.load(off);
     load_x(next);
     __syncthreads();  // LayerNorm(x) is complete, and everybody has finished with the first tile
     f32x16_t acc = unit_product<C, true>(second, w.o);
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] = acc[v] * sz.unscale * sigmoid_hw_f32(gate[v], sg.unscale);
-    rows.store(off, acc, res);
+    rows.add(wave, acc, p.add_residual);
+    before = t;
+    first = false;
   }
+  if (first) return;  // the whole work-group
+  __syncthreads();
+  store_rows(before);
 }
 
 // ---- triangle attention, input pass: q / sqrt(D), k, v^T as split operands of the core, triangle bias --------
@@ -491,7 +514,8 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
   constexpr int NW = C / 32, TASKS = 8 / NW;
   extern __shared__ u32x4_t lds[];
   const Tile tile = {lds}, second = {lds + Tile::SLOTS};
-  float* ln = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS);  // [2][C], times the scale of the activations
+  const RowTile<C> rows = {reinterpret_cast<float4*>(lds + 2 * Tile::SLOTS)};
+  float* ln = reinterpret_cast<float*>(lds + 2 * Tile::SLOTS + RowTile<C>::SLOTS);  // [2][C], times the scale of the activations
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int N = p.N;
@@ -534,7 +558,19 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
     for (int a = 0; a < 4; ++a) oraw[a] = *reinterpret_cast<const float4*>(op + 4 * a);
   };
 
+  auto store_rows = [&](int id) {
+    const Lane here = lane_here();
+    int b, i;
+    const int j0 = place(id, b, i);
+    float* base = p.out + b * p.xv.stride_b + i * p.xv.stride_r;
+#pragma unroll
+    for (int u = 0; u < TASKS; ++u) {
+      const int pos = 4 * (wave + NW * u) + here.lg;
+      if (j0 + pos < N) rows.store(base + (j0 + pos) * p.xv.stride_k, pos, here.li);
+    }
+  };
   int id = grid_slot();
+  const int first = id;
   if (id < total) load_rows(id), load_o(id);
   for (; id < total; id += gridDim.x) {
     const int next = id + (int)gridDim.x < total ? id + (int)gridDim.x : id;
@@ -549,8 +585,14 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) tile.store4(pos, li + 16 * e, y[e]);
     }
+    __syncthreads();  // LayerNorm(x) and the rows of the tile before are complete, and everybody has finished with the second tile
+    if (id != first) store_rows(id - gridDim.x);
+    if (p.add_residual) {
+      const Lane at = lane_here();
+#pragma unroll
+      for (int u = 0; u < TASKS; ++u) rows.put(4 * (wave + NW * u) + at.lg, at.li, raw[u]);
+    }
     load_rows(next);
-    __syncthreads();  // LayerNorm(x) is complete, and everybody has finished with the second tile
     const f32x16_t gate = unit_product<C, true>(tile, w.g);
     const Lane mid = lane_here();
 #pragma unroll
@@ -562,16 +604,16 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
       for (int e = 0; e < 8; ++e) y[e] = ov[e] * o_scale * sigmoid_hw_f32(gate[8 * hf + e], sg.unscale);
       second.store8(mid.l32, 4 * wave + 2 * mid.lh + hf, y);
     }
-    const RowTile rows(p.x, p.out, b * p.xv.stride_b + i * p.xv.stride_r + j0 * p.xv.stride_k, p.add_residual);
-    const uint32_t off = rows.offset(j0, N, p.xv.stride_k, 32 * wave);
-    const Row16 res = rows.load(off);
     load_o(next);
     __syncthreads();  // the gated output is complete, and everybody has finished with the first tile
     f32x16_t acc = unit_product<C, true>(second, w.o);
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] *= unscale;
-    rows.store(off, acc, res);
+    rows.add(wave, acc, p.add_residual);
   }
+  if (first >= total) return;  // the whole work-group
+  __syncthreads();
+  store_rows(id - gridDim.x);
 }
 
 template <int C, int NW>

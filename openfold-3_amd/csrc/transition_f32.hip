@@ -239,7 +239,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
     const int64_t row0 = bb * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j0 * p.xv.stride_k;
     Row16 res;
     float m = 1.f;
-    const RowTile out_rows(p.x, p.out, AFTER ? 0 : row0, p.add_residual && kh == 0);
+    const GlobalRows out_rows(p.x, p.out, AFTER ? 0 : row0, p.add_residual && kh == 0);
     const uint32_t off = out_rows.offset(j0, pn < p.total && kh == 0 ? L : 0, p.xv.stride_k, 32 * ot);
     // before the next tile's rows, so that a wait for these leaves those in flight
     auto load_residual = [&] {

@@ -46,3 +46,31 @@ def test_rows_far_apart(c):
     print("rows far apart", c, flush=True)
     want = m(z, mask)
     report("block", m(apart, mask), want, atol=REL * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("inplace", [False, True])
+@pytest.mark.parametrize("c", [64, 128])
+@pytest.mark.parametrize("n", [1, 33, 97, 150])  # a work-group's only tile, and rows on their way through LDS beside the next tile's
+def test_result_rows(n, c, inplace):
+    """Output passes, with the residual (blocks) and without it (a module's update alone)."""
+    lib()
+    heads = 4
+    p = orc.make_block_params(8604, c, c, c // heads, heads)
+    m = of3pair.PairStack(c, c, c // heads, heads)
+    m.load_state_dict(p, strict=True)
+    m = m.to(DEV).eval()
+    z = orc.make_pair_input(8605, (1,), n, c)
+    mask = torch.rand(1, n, n, generator=torch.Generator().manual_seed(8606)) > 0.2
+    mask[..., 0] = True  # in 64 bits -1e9 does not absorb the logits of a row without a real key
+    mask = mask.float()
+    p64 = {k: v.double() for k, v in p.items()}
+    print("rows", n, c, inplace, flush=True)
+    want = orc.pair_stack_block(z.double(), mask.double(), p64, heads)
+    got = m(z.to(DEV), mask.to(DEV), inplace_safe=inplace).cpu()
+    report("block", got, want, atol=2 * REL * float(want.abs().max()))
+    if not inplace:
+        for module, prefix, oracle in ((m.tri_mul_in, "tri_mul_in.", lambda x, k, q: orc.trimul_update(x, k, q, False)),
+                                       (m.tri_att_start, "tri_att_start.", lambda x, k, q: orc.triattn_update(x, k, q, heads))):
+            q = {k[len(prefix):]: v for k, v in p64.items() if k.startswith(prefix)}
+            want = oracle(z.double(), mask.double(), q)
+            report(prefix, module(z.to(DEV), mask.to(DEV)).cpu(), want, atol=2 * REL * float(want.abs().max()))
