@@ -78,11 +78,9 @@ constexpr float kRaise = 64.0f;  // the offset of a query is raised only when a 
 constexpr float kSnap = 32.0f;   // ... and an offset within +-32 is replaced by 0
 constexpr float kMaskedBelow = -1e8f;  // a mask bias below this sends exp2 of any sane logit to exactly 0
 
-__device__ __forceinline__ float max3(float a, float b, float c) {
-  float r;
-  __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
+// v_max3_f32, but not as inline assembly: the compiler does not put the wait states between a matrix product and its first
+// reader there, and the maximum then is that of the logits before their last k-step
+__device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
 // QW = waves per row, RQ = 32-query tiles per wave: a work-group is 4 rows x 32 QW RQ queries.  Two waves (128 queries, two
 // work-groups of 8 waves per CU) move the fewest K and V^T bytes into LDS; one wave (64 or 128 queries, four or three work-groups
