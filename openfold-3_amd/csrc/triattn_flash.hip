@@ -319,7 +319,8 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
 #pragma unroll
         for (int v = 3; v < 15; v += 2) mx = max3(mx, s[v], s[v + 1]);
         mx = fmaxf(mx, s[15]);
-        if (__builtin_amdgcn_ballot_w64(mx > m_run[rq] + kRaise) != 0) {
+        // a difference: at a masked key's -1.44e9 the logits are 128 apart, and the offset + 64 would round to the next one
+        if (__builtin_amdgcn_ballot_w64(mx - m_run[rq] > kRaise) != 0) {
           // both halves of a query's lane pair take the same new offset; an offset of moderate size is
           // replaced by 0 (any offset gives the same softmax, and 0 needs no subtraction below)
           float m_new = fmaxf(m_run[rq], fmaxf(mx, xhalf(mx)));
