@@ -41,6 +41,7 @@ namespace {
 constexpr int kRows = 2;
 constexpr float kLift = 4.f, kHigh = 0x1p15f;
 constexpr float kFloor = -3e38f;  // in place of -infinity as an offset
+enum { kFirst, kTracked, kLevelled };  // what a pass over the keys does
 constexpr int kTb = 128 * 8;                    // bias slice [128 queries][32 keys] fp32 in 16-byte slots
 constexpr int kTbI = kTb / (64 * 2 * kRows);    // load instructions of a wave for it
 template <int STEPS>
@@ -187,11 +188,13 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
       for (int pl = 0; pl < STEPS; ++pl) o.v[st][pl] = kvb[L::kKv + (st * STEPS + pl) * 64];
     return o;
   };
-  auto tile = [&](auto track, int buf, float mb, const Operands& given) {
-    constexpr bool kTrack = decltype(track)::value;
+  uint32_t uneven[QT];  // level pass: bits in which a logit of the lane's query differed from level_at's
+  uint32_t level_at = 0u;
+  auto tile = [&](auto kind, int buf, float mb, const Operands& given, int keys_left) {
+    constexpr bool kTrack = decltype(kind)::value == kTracked, kLevel = decltype(kind)::value == kLevelled;
     if (!wave_has_work) return;
     // first pass: a tile whose keys are all masked or padded adds exp(-1e9 + logit) = 0 exactly to every sum
-    if (!kTrack && __builtin_amdgcn_ballot_w64(mb > -1e8f) == 0) return;
+    if (!kTrack && !kLevel && __builtin_amdgcn_ballot_w64(mb > -1e8f) == 0) return;
     const bool has_mb = __builtin_amdgcn_ballot_w64(mb != 0.f) != 0;
     const u32x4_t* tbuf = tb_lds + buf * kTb + (64 * qh + l32) * 8;
     const Operands op = L::kStages == 1 ? given : read_operands(buf);
@@ -211,6 +214,29 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
         s = mfma_32x32x16_f16(op.k[st][1], qop[qt][st][0], s);
         s = mfma_32x32x16_f16(op.k[st][0], qop[qt][st][1], s);
         s = mfma_32x32x16_f16(op.k[st][0], qop[qt][st][0], s);
+      }
+      if constexpr (kLevel) {
+        // register v holds key 8 (v >> 2) + 4 lh + (v & 3) of the tile, and so do the weights' operands: all 2^kLift, of keys below N
+        constexpr uint32_t kOne = 0x4C00u;
+        static_assert(kLift == 4.f, "fp16(16)");
+        const int left = keys_left - 4 * lh;
+        if (keys_left >= 32) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) uneven[qt] |= __float_as_uint(s[v]) ^ level_at;  // NaN too
+        } else {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) uneven[qt] |= acc_row(v, 0) < left ? __float_as_uint(s[v]) ^ level_at : 0u;
+        }
+        if (qt > 0) continue;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          u32x4_t ph;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) ph[w] = (acc_row(8 * st + 2 * w, 0) < left ? kOne : 0u) | (acc_row(8 * st + 2 * w + 1, 0) < left ? kOne << 16 : 0u);
+          if constexpr (STEPS == 2) oacc[0] = mfma_32x32x16_f16(op.v[st][STEPS - 1], ph, oacc[0]);
+          oacc[0] = mfma_32x32x16_f16(op.v[st][0], ph, oacc[0]);
+        }
+        continue;
       }
       float lsum = 0.f;
       if constexpr (kTrack) {
@@ -260,7 +286,7 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
         }
       }
     }
-    if (!kTrack) fresh = false;
+    if (!kTrack && !kLevel) fresh = false;
   };
 
   float mv_next;
@@ -269,18 +295,21 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
     issue_bias(0, 0);
     issue_kv(0, 0);
   };
-  auto pass = [&](auto track) {
+  auto pass = [&](auto kind) {
+    constexpr bool kLevel = decltype(kind)::value == kLevelled;
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       oacc[qt] = zero16();
       m_run[qt] = kFloor;
       l_run[qt] = 0.f;
+      uneven[qt] = 0u;
     }
     auto step = [&](int kt, int buf) {  // buf is a constant at both call sites: LDS addresses are immediates
       wait_vmcnt<0>();               // this wave's loads of tile kt (and its mask values) have landed ...
       __builtin_amdgcn_s_barrier();  // ... and everybody's; nobody reads tile kt - 1's buffers any more
       compiler_fence();
       const float mb = mask_bias(kt, mv_next);
+      if (kLevel && kt == 0) level_at = __builtin_amdgcn_readfirstlane(__float_as_uint(mb * logit_scale));
       const int ktn = kt + 1 < nkt ? kt + 1 : nkt - 1;
       mv_next = load_mask(ktn);
       issue_bias(ktn, buf ^ 1);
@@ -292,7 +321,7 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
         compiler_fence();
       }
       issue_kv(ktn, buf ^ 1);
-      tile(track, buf, mb, op);
+      tile(kind, buf, mb, op, N - 32 * kt);
       compiler_fence();
     };
     for (int kt = 0; kt < nkt; kt += 2) {
@@ -301,24 +330,27 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
     }
     wait_vmcnt<0>();  // the loads issued past the end must not outlive the pass (or the work-group's LDS)
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) l_tot[qt] = l_run[qt] + __shfl_xor(l_run[qt], 32, 64);
+    for (int qt = 0; qt < QT; ++qt) {
+      if (kLevel && qt > 0) oacc[qt] = oacc[0];
+      l_tot[qt] = kLevel ? (float)N * 16.f : l_run[qt] + __shfl_xor(l_run[qt], 32, 64);
+    }
   };
 
   // A work-group with a row whose sampled keys are all masked goes to the second pass at once, as in the bf16 core.
   first_loads();
   const uint64_t masked = __builtin_amdgcn_ballot_w64(sample < -1e8f);
-  bool again = false;
+  // Where all of its rows look so, a pass that sees whether all logits are the mask bias itself, which takes those of an ordinary size up: the
+  // weights are then equal, their sum N and the result the mean of v, the same for every query (three templates of 200, 20 tokens padded, 868 / 858
+  // us, a trunk block at 600, 100 padded, 3170 / 3114).
+  bool again = false, level = true;  // the same in every wave of the work-group
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) again |= ((masked >> (4 * r)) & 15u) == 15u;  // the same in every wave of the work-group
-  if (!again) {
-    pass(std::false_type{});
-    bool bad = false;
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-      const bool in_range = l_tot[qt] > 0.f && l_tot[qt] <= 0x1p60f;  // false for NaN and +inf (a logit 80 above the first tile's) too
-      bad |= row_valid && (q0 + 32 * qt + l32 < N) && !in_range;
-    }
-    // the vote goes through the bias buffers
+  for (int r = 0; r < kRows; ++r) {
+    const bool all = ((masked >> (4 * r)) & 15u) == 15u;
+    again |= all;
+    level &= all || rg * kRows + r >= N;
+  }
+  level &= again;
+  auto any_wave = [&](bool bad) {  // the vote goes through the bias buffers
     uint32_t* votes = reinterpret_cast<uint32_t*>(lds4);
     __syncthreads();
     const uint32_t wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
@@ -327,13 +359,30 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
     uint32_t any = 0;
 #pragma unroll
     for (int w = 0; w < 2 * kRows; ++w) any |= votes[w];
-    again = __builtin_amdgcn_readfirstlane(any) != 0;
-    if (again) {
+    const bool result = __builtin_amdgcn_readfirstlane(any) != 0;
+    if (result) {
       __syncthreads();  // every wave has read the votes before loads land on them
       first_loads();
     }
+    return result;
+  };
+  if (level) {
+    pass(std::integral_constant<int, kLevelled>{});
+    bool bad = false;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) bad |= row_valid && q0 + 32 * qt + l32 < N && uneven[qt] != 0;
+    again = any_wave(bad);
+  } else if (!again) {
+    pass(std::integral_constant<int, kFirst>{});
+    bool bad = false;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const bool in_range = l_tot[qt] > 0.f && l_tot[qt] <= 0x1p60f;  // false for NaN and +inf (a logit 80 above the first tile's) too
+      bad |= row_valid && (q0 + 32 * qt + l32 < N) && !in_range;
+    }
+    again = any_wave(bad);
   }
-  if (again) pass(std::true_type{});
+  if (again) pass(std::integral_constant<int, kTracked>{});
 
   if (row_valid) {
 #pragma unroll

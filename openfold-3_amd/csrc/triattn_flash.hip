@@ -76,6 +76,8 @@ constexpr int kRows = 4, kStages = 2;
 constexpr int kRgBlock = OF3_FLASH_RG_BLOCK, kQcBlock = 8;  // row groups x query ranges per block of the work-group order
 constexpr float kRaise = 64.0f;  // the offset of a query is raised only when a logit exceeds it by 2^64 ...
 constexpr float kSnap = 32.0f;   // ... and an offset within +-32 is replaced by 0
+// What a pass over the keys does: first pass, with running maxima, or (rows of masked keys) see that all logits are level
+enum { kFirst, kTracked, kLevelled };
 constexpr float kMaskedBelow = -1e8f;  // a mask bias below this sends exp2 of any sane logit to exactly 0
 
 // v_max3_f32, but not as inline assembly: the compiler does not put the wait states between a matrix product and its first
@@ -290,13 +292,15 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
     }
     return o;
   };
-  auto tile = [&](auto track, int buf, float mb_cur, const Operands& given) {
-    constexpr bool kTrack = decltype(track)::value;
+  uint32_t uneven[kRQ];  // level pass: bits in which a logit of the lane's query differed from level_at's
+  uint32_t level_at = 0u;
+  auto tile = [&](auto kind, int buf, float mb_cur, const Operands& given, int keys_left) {
+    constexpr bool kTrack = decltype(kind)::value == kTracked, kLevel = decltype(kind)::value == kLevelled;
     if (!wave_has_work) return;
     // first pass: a tile whose keys are all masked or padded adds exp2(-1.44e9 + logit) = 0 exactly to
     // every sum and is left out (a row without any unmasked key thus does nothing here, ends with the
     // row sum 0 and takes the second pass, as it has to anyway)
-    if (!kTrack && __builtin_amdgcn_ballot_w64(mb_cur > kMaskedBelow) == 0) return;
+    if (!kTrack && !kLevel && __builtin_amdgcn_ballot_w64(mb_cur > kMaskedBelow) == 0) return;
     const bool has_mb = __builtin_amdgcn_ballot_w64(mb_cur != 0.f) != 0;
     const u32x4_t* tbuf = tb_lds + buf * TBS + tb_row;
     const Operands op = KVST == 1 ? given : read_operands(buf);
@@ -314,6 +318,26 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
 #pragma unroll
       for (int ks = 0; ks < KSQ; ++ks) s = mfma_32x32x16(op.k[ks], qop[rq][ks], s);
 
+      if constexpr (kLevel) {
+        const int left = keys_left - 16 * lh;  // of this lane's 16 keys
+        if (keys_left >= 32) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) uneven[rq] |= __float_as_uint(s[v]) ^ level_at;
+        } else {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) uneven[rq] |= v < left ? __float_as_uint(s[v]) ^ level_at : 0u;
+        }
+        if (rq > 0) continue;
+        u32x4_t one0, one1;  // the weights, all 1, in the order of the other passes: the same sums
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          one0[w] = (2 * w < left ? 0x3F80u : 0u) | (2 * w + 1 < left ? 0x3F800000u : 0u);
+          one1[w] = (8 + 2 * w < left ? 0x3F80u : 0u) | (9 + 2 * w < left ? 0x3F800000u : 0u);
+        }
+        oacc[0] = mfma_32x32x16(op.v[0], one0, oacc[0]);
+        oacc[0] = mfma_32x32x16(op.v[1], one1, oacc[0]);
+        continue;
+      }
       if constexpr (kTrack) {
         float mx = max3(s[0], s[1], s[2]);
 #pragma unroll
@@ -375,10 +399,12 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
     issue_bias(0, 0);
     issue_kv(0, 0);
   };
-  auto pass = [&](auto track) {
+  auto pass = [&](auto kind) {
+    constexpr bool kTrack = decltype(kind)::value == kTracked, kLevel = decltype(kind)::value == kLevelled;
 #pragma unroll
     for (int rq = 0; rq < kRQ; ++rq) {
-      m_run[rq] = decltype(track)::value ? -__builtin_inff() : 0.f;
+      m_run[rq] = kTrack ? -__builtin_inff() : 0.f;
+      uneven[rq] = 0u;
       l_run[rq] = 0.f;
       oacc[rq] = zero16();
       lsum[rq] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -388,6 +414,8 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
       __builtin_amdgcn_s_barrier();  // ... and everybody's; nobody reads tile kt-1's buffers any more
       compiler_fence();
       const float mb_cur = mb_next;
+      if (kLevel && kt == 0)  // the first key's mask bias as the k-step adds it
+        level_at = __builtin_amdgcn_readfirstlane(pack_bf16(mb_cur, 0.f) << 16);
       const int ktn = kt + 1 < nkt ? kt + 1 : nkt - 1;
       mb_next = __uint_as_float(load_mb(ktn, mb_off));
       issue_bias(ktn, buf ^ 1);
@@ -398,7 +426,7 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
         compiler_fence();
       }
       issue_kv(ktn, buf ^ 1);
-      tile(track, buf, mb_cur, op);
+      tile(kind, buf, mb_cur, op, N - 32 * kt);
       compiler_fence();
     };
     for (int kt = 0; kt < nkt; kt += 2) {
@@ -408,7 +436,10 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
     wait_vmcnt<0>();  // the loads issued past the end must not outlive the pass (or the work-group's LDS)
 #pragma unroll
     for (int rq = 0; rq < kRQ; ++rq) {
-      if (D == 32 && decltype(track)::value) {
+      if (kLevel && rq > 0) oacc[rq] = oacc[0];
+      if (D == 32 && kLevel) {
+        l_tot[rq] = (float)N;
+      } else if (D == 32 && kTrack) {
         l_tot[rq] = l_run[rq] + xhalf(l_run[rq]);
       } else if (D == 32) {
         const float lo = __shfl(lsum[rq][0], l32 & 15, 64), hi = __shfl(lsum[rq][1], l32 & 15, 64);
@@ -426,6 +457,12 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
   // row sum itself tells: 2^-60 <= sum <= 2^60 (an overflow leaves +inf in the sum, a row of masked
   // keys leaves 0).  If any query of the work-group fails that test, the whole work-group (its
   // loads and barriers are collective) runs the pass again with running maxima.
+  // Where all rows of a work-group look so, the pass only sees whether every logit is the mask bias itself, which takes logits of an
+  // ordinary size up (128 are between it and its neighbours).  The weights then are equal and the result is the mean of v, the same
+  // for every query: no exponentials, no maxima, no sums, and P V for one of the query tiles; the bits are those of the pass with
+  // running maxima, which comes after it where a logit is another.  Launches, us: N = 2048, 256 tokens padded, 6389 / 5922, 384, 38
+  // padded, 56.5 / 53.9; whole passes 24.4 / 23.4 ms and 1087 / 1077, one block at 929, 40 padded, 3735 / 3711, four templates of 512, 51
+  // padded, 3558 / 3522.
   // A work-group with a row whose sampled keys (its own token, the first, the middle and the last) are all masked is
   // taken for one with a padded token, which fails that test for certain, and goes to the second pass at once; a wrong
   // guess costs it the offsets' arithmetic and nothing else.  A launch that fits the chip at once lasts as long as its
@@ -434,11 +471,23 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
   // templates of 187, 12 padded, 384 / 366; without padding no difference (N = 768).
   first_loads();
   const uint64_t masked = __builtin_amdgcn_ballot_w64(sample < kMaskedBelow);
-  bool again = false;
+  bool again = false, level = true;  // the same in every wave of the work-group
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) again |= ((masked >> (4 * r)) & 15u) == 15u;  // the same in every wave of the work-group
-  if (!again) {
-    pass(std::false_type{});
+  for (int r = 0; r < kRows; ++r) {
+    const bool all = ((masked >> (4 * r)) & 15u) == 15u;
+    again |= all;
+    level &= all || rg * kRows + r >= N;
+  }
+  level &= again;
+  if (level) {
+    pass(std::integral_constant<int, kLevelled>{});
+    bool bad = false;
+#pragma unroll
+    for (int rq = 0; rq < kRQ; ++rq) bad |= row_valid && q0 + 32 * rq + l32 < N && uneven[rq] != 0;
+    level = !__syncthreads_or(bad);
+    if (!level) first_loads();
+  } else if (!again) {
+    pass(std::integral_constant<int, kFirst>{});
     bool bad = false;
 #pragma unroll
     for (int rq = 0; rq < kRQ; ++rq) {
@@ -448,7 +497,7 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
     again = __syncthreads_or(bad);
     if (again) first_loads();
   }
-  if (again) pass(std::true_type{});
+  if (again && !level) pass(std::integral_constant<int, kTracked>{});
 
   if (row_valid && 16 * lh < D) {
 #pragma unroll
