@@ -195,11 +195,14 @@ template <int C, bool W_ROWS>
 struct HalfSum {
   static constexpr bool kApart = C == 64;
   f32x16_t acc = zero16(), low = zero16();
+  // one of a k-step's three products, in this order
+  __device__ __forceinline__ void term(int i, const u32x4_t (&w)[2], const u32x4_t (&x)[2]) {
+    f32x16_t& sum = kApart && i < 2 ? low : acc;
+    sum = mm_f16<W_ROWS>(w[i == 0], x[i == 1], sum);
+  }
   __device__ __forceinline__ void step(const u32x4_t (&w)[2], const u32x4_t (&x)[2]) {
-    f32x16_t& l = kApart ? low : acc;
-    l = mm_f16<W_ROWS>(w[1], x[0], l);
-    l = mm_f16<W_ROWS>(w[0], x[1], l);
-    acc = mm_f16<W_ROWS>(w[0], x[0], acc);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) term(i, w, x);
   }
   __device__ __forceinline__ f32x16_t total() const { return kApart ? acc + low : acc; }
 };

@@ -8,7 +8,7 @@
 // One wave per tile of 32 hidden channels and all of the tile's positions: a work-group of eight waves takes the
 // hidden dimension in slices of 32 S channels (S = 8, or 4 with a wave per position tile), so that an operand of Wa
 // and Wb is read once for 64 positions and a slice of 256 hidden channels costs two barriers, against 32 positions
-// and slices of 128 in pair_f32.hip's kernel.  The operands of a k-step are requested one to four steps ahead, those of
+// and slices of 128 in pair_f32.hip's kernel.  Many tiles: work-groups of four waves with slices of 128, two to a CU (NW).  The operands of a k-step are requested one to four steps ahead, those of
 // the other product before the barrier between them.  Below two tiles of 64 positions per CU, tiles of 32 positions (two
 // waves then share the sum of the second product).
 #include "of3_pass_f32.h"
@@ -61,29 +61,35 @@ __device__ __forceinline__ float smallest_inv_bound(const WeightX3& W, int n) {
 // trunk blocks at N = 24 / 45 / 64 / 80 / 90 527 / 579 / 587 / 696 / 758 us, so 502 / 554 / 565 / 671 / 736 (a launch, and z read once more).
 // KEEP: the hidden dimension is one slice, a wave's operands of all three matrices stay in registers (96 of 208).  Three templates of 200, 64
 // channels, n = 2, two transitions of 2100 tiles: the operands fetched again for every tile 107 us, so 90.
-template <int C, int S, int NPT, bool AFTER, bool BIAS, bool KEEP>
-__global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
+// NW: waves of the work-group.  With four, each has a hidden tile and an output tile for all of the tile's positions, and two work-groups share a
+// CU: their barriers, LayerNorms and SiLUs do not coincide, and at 128 channels an operand of Wout serves both position tiles.  One of eight waves /
+// two of four, us: 128 channels, n = 4, N = 384 211.5 / 207.5 (matrix pipe 43 % busy, vector pipe 32 %; 196 with every weight in
+// the L1, so no wait for those), 64 channels, KEEP, 44.2 / 40.6.  Same bits.
+template <int C, int S, int NPT, bool AFTER, bool BIAS, bool KEEP, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) {
   static_assert(AFTER || !BIAS, "one tile per work-group");
   static_assert(!AFTER || (C == 128 && NPT == 1), "eight waves: a gate and an output tile for each 32 channels");
-  static_assert(S == 8 || (S == 4 && NPT == 2), "eight waves share the hidden tiles of a slice");
+  static_assert(S == NW || (S == 4 && NW == 8 && NPT == 2), "the waves share the hidden tiles of a slice");
   typedef HalfTile<C> XTile;
   typedef HalfTile<32 * S> HTile;
-  constexpr int NW = 8, KS = C / 16, OT = C / 32;
-  constexpr int XT = S == 8 ? NPT : 1;             // position tiles of a wave in the first product
-  constexpr int KSPLIT = NW / (OT * NPT);          // waves sharing an output tile's sum in the second
+  constexpr int KS = C / 16, OT = C / 32, RG = 8 / NW;  // RG: rows of a position tile that a lane has a part of
+  constexpr int XT = S == NW ? NPT : 1;                 // position tiles of a wave in the first product
+  constexpr int OP = OT * NPT > NW ? OT * NPT / NW : 1;  // ... in the second
+  constexpr int KSPLIT = NW * OP / (OT * NPT);          // waves sharing an output tile's sum in the second
+  static_assert(OP == 1 || OP == NPT, "");
   constexpr int OSTEPS = 2 * S / KSPLIT;           // its k-steps per slice and wave
   // steps that an operand is requested ahead: an L2 read takes about as long as 24 MFMAs of two waves per SIMD
-  constexpr int DA = KEEP ? KS : XT == 1 ? 2 : 1, DO = KEEP ? OSTEPS : 4;
+  constexpr int DA = KEEP ? KS : XT == 1 ? 2 : 1, DO = KEEP ? OSTEPS : 4 / OP;
   static_assert(OSTEPS >= DO && KS >= DA, "");
   // the residual before the next tile's rows and a slice's scales before its operands; there they would spill
-  constexpr bool kEarly = !(C == 64 && S == 8 && NPT == 2);
+  constexpr bool kEarly = !(C == 64 && S == 8 && NPT == 2), kEarlyRes = kEarly && OP == 1;
   extern __shared__ u32x4_t lds[];
   u32x4_t* const hid = lds + NPT * XTile::SLOTS;
   float* ln = reinterpret_cast<float*>(hid + NPT * HTile::SLOTS);  // [2][C]
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ht = S == 8 ? wave : wave & 3, pt_a = S == 8 ? 0 : wave >> 2;
-  const int ot = wave % OT, pt_b = (wave / OT) % NPT, kh = wave / (OT * NPT);
+  const int ht = S == NW ? wave : wave & 3, pt_a = S == NW ? 0 : wave >> 2;
+  const int ot = wave % OT, pt_b = OP > 1 ? 0 : (wave / OT) % NPT, kh = wave / (OT * NPT);
   const int L = p.L, slices = p.HID / (32 * S);
   // The activations' scale is in ln, the hidden ones take the largest that the bounds of their two factors allow
   const float x_scale = p.s_a.scales()[0].input;
@@ -102,7 +108,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
     j0 = 32 * (pn - r * p.panels);
     return r;
   };
-  RowRegs<C> raw[NPT];
+  RowRegs<C> raw[NPT][RG];
   auto load_tile = [&](int tile) {
     const Lane here = lane_here();
 #pragma unroll
@@ -110,9 +116,12 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       int pn = NPT * tile + t, j0;
       pn = pn < p.total ? pn : p.total - 1;
       const int r = row_of(pn, j0), b = r / p.R, i = r - b * p.R;
-      int j = j0 + 4 * wave + here.lg;
-      j = j < L ? j : L - 1;
-      load_row<C>(p.x + b * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j * p.xv.stride_k, here.li, raw[t]);
+#pragma unroll
+      for (int g = 0; g < RG; ++g) {
+        int j = j0 + 4 * (NW * g + wave) + here.lg;
+        j = j < L ? j : L - 1;
+        load_row<C>(p.x + b * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j * p.xv.stride_k, here.li, raw[t][g]);
+      }
     }
   };
   u32x4_t na[DA][2], nb[DA][2], no[DO][2];  // operands of the next steps
@@ -184,11 +193,11 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       };
       const int pos = 4 * wave + here.lg;
       float4 y[C / 64];
-      norm_row<C>(raw[0], j0 + pos < L, att_ln, here.li, y);
+      norm_row<C>(raw[0][0], j0 + pos < L, att_ln, here.li, y);
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) {
         xn.store4(pos, here.li + 16 * e, y[e]);
-        *reinterpret_cast<float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li) = raw[0].v[e];
+        *reinterpret_cast<float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li) = raw[0][0].v[e];
       }
       __syncthreads();
       if (kh == 0) {
@@ -215,7 +224,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       }
       __syncthreads();
 #pragma unroll
-      for (int e = 0; e < C / 64; ++e) raw[0].v[e] = *reinterpret_cast<const float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li);
+      for (int e = 0; e < C / 64; ++e) raw[0][0].v[e] = *reinterpret_cast<const float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li);
     }
     {
       const Lane here = lane_here();
@@ -224,34 +233,50 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
         int j0;
         const int pn = NPT * tile + t;
         row_of(pn, j0);
-        const int pos = 4 * wave + here.lg;
-        float4 y[C / 64];
-        norm_row<C>(raw[t], pn < p.total && j0 + pos < L, ln, here.li, y);
         const XTile xn = {lds + t * XTile::SLOTS};
 #pragma unroll
-        for (int e = 0; e < C / 64; ++e) xn.store4(pos, here.li + 16 * e, y[e]);
+        for (int g = 0; g < RG; ++g) {
+          const int pos = 4 * (NW * g + wave) + here.lg;
+          float4 y[C / 64];
+          norm_row<C>(raw[t][g], pn < p.total && j0 + pos < L, ln, here.li, y);
+#pragma unroll
+          for (int e = 0; e < C / 64; ++e) xn.store4(pos, here.li + 16 * e, y[e]);
+        }
       }
     }
-    // this wave's rows of the result
-    const int pn = NPT * tile + pt_b;
-    int j0;
-    const int r = row_of(pn < p.total ? pn : p.total - 1, j0), bb = r / p.R, i = r - bb * p.R;
-    const int64_t row0 = bb * p.xv.stride_b + i * p.xv.stride_r + (int64_t)j0 * p.xv.stride_k;
-    Row16 res;
-    float m = 1.f;
-    const GlobalRows out_rows(p.x, p.out, AFTER ? 0 : row0, p.add_residual && kh == 0);
-    const uint32_t off = out_rows.offset(j0, pn < p.total && kh == 0 ? L : 0, p.xv.stride_k, 32 * ot);
+    // this wave's rows of the result, of one position tile or of all
+    struct Rows {
+      int r, bb, i, j0;
+      int64_t row0;
+    };
+    auto rows_of = [&](int o) {
+      const int pn = NPT * tile + pt_b + o;
+      Rows w;
+      w.r = row_of(pn < p.total ? pn : p.total - 1, w.j0), w.bb = w.r / p.R, w.i = w.r - w.bb * p.R;
+      w.row0 = w.bb * p.xv.stride_b + w.i * p.xv.stride_r + (int64_t)w.j0 * p.xv.stride_k;
+      return w;
+    };
+    Row16 res[OP];
+    float m[OP];
+    auto global_rows = [&](const Rows& w) { return GlobalRows(p.x, p.out, AFTER ? 0 : w.row0, p.add_residual && kh == 0); };
+    auto offset_of = [&](int o, const Rows& w) {
+      return global_rows(w).offset(w.j0, NPT * tile + pt_b + o < p.total && kh == 0 ? L : 0, p.xv.stride_k, 32 * ot);
+    };
     // before the next tile's rows, so that a wait for these leaves those in flight
     auto load_residual = [&] {
-      const int j = j0 + lane_here().l32 < L ? j0 + lane_here().l32 : L - 1;
-      if (p.mask) m = p.mask[bb * p.mv.stride_b + i * p.mv.stride_r + (int64_t)j * p.mv.stride_k];
-      if (!AFTER) res = out_rows.load(off);
+#pragma unroll
+      for (int o = 0; o < OP; ++o) {
+        const Rows w = rows_of(o);
+        const int j = w.j0 + lane_here().l32 < L ? w.j0 + lane_here().l32 : L - 1;
+        m[o] = p.mask ? p.mask[w.bb * p.mv.stride_b + w.i * p.mv.stride_r + (int64_t)j * p.mv.stride_k] : 1.f;
+        if (!AFTER) res[o] = global_rows(w).load(offset_of(o, w));
+      }
     };
     if constexpr (!KEEP) {
 #pragma unroll
       for (int s = 0; s < DA; ++s) fetch_ab(0, s);
     }
-    HalfSum<128, true> osum;
+    HalfSum<128, true> osum[OP];
     for (int slice = 0; slice < slices; ++slice) {
       // requested ahead of the operands (where the registers allow it): behind them they wait for every operand in flight
       float ua, ub;
@@ -288,9 +313,9 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
           }
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int t = 0; t < XT; ++t) {
-            sum_a[t].step(ca, x[t]);
-            sum_b[t].step(cb, x[t]);
+          for (int term = 0; term < 3; ++term) {  // chains of dependent products in turn (211 / 207.5 us at N = 384)
+#pragma unroll
+            for (int t = 0; t < XT; ++t) sum_a[t].term(term, ca, x[t]), sum_b[t].term(term, cb, x[t]);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -317,33 +342,60 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       {
         const Lane at = lane_here();
         const u32x4_t* ht0 = hid + pt_b * HTile::SLOTS;
-        u32x4_t nx[2];
+        u32x4_t nx[OP][2];
         auto read_h = [&](int s) {
-          const u32x4_t* x = ht0 + HTile::slot(at.l32, 2 * (kh * OSTEPS + s) + at.lh);
-          nx[0] = x[0], nx[1] = x[HTile::PLANE];
+#pragma unroll
+          for (int o = 0; o < OP; ++o) {
+            const u32x4_t* x = ht0 + o * HTile::SLOTS + HTile::slot(at.l32, 2 * (kh * OSTEPS + s) + at.lh);
+            nx[o][0] = x[0], nx[o][1] = x[HTile::PLANE];
+          }
         };
         read_h(0);
 #pragma unroll
         for (int s = 0; s < OSTEPS; ++s) {
-          const u32x4_t x[2] = {nx[0], nx[1]}, co[2] = {no[s % DO][0], no[s % DO][1]};
+          const u32x4_t co[2] = {no[s % DO][0], no[s % DO][1]};
+          u32x4_t x[OP][2];
+#pragma unroll
+          for (int o = 0; o < OP; ++o) x[o][0] = nx[o][0], x[o][1] = nx[o][1];
           if (s + 1 < OSTEPS) read_h(s + 1);
           if (s + DO < OSTEPS) fetch_o(slice, s + DO);
           if (s + DO == OSTEPS) {  // after the last weights: loads return in order
             if (KEEP || last) {
-              if (kEarly) load_residual();
+              if (kEarlyRes) load_residual();
               if (!AFTER) load_tile(tile + (int)gridDim.x < tiles ? tile + gridDim.x : tile);
             } else
 #pragma unroll
               for (int q = 0; q < DA; ++q) fetch_ab(slice + 1, q);
           }
           __builtin_amdgcn_sched_barrier(0);
-          osum.step(co, x);
+#pragma unroll
+          for (int term = 0; term < 3; ++term) {
+#pragma unroll
+            for (int o = 0; o < OP; ++o) osum[o].term(term, co, x[o]);
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
-    f32x16_t oacc = osum.total();
-    if (!kEarly) load_residual();
+    if (!kEarlyRes) load_residual();
+    if constexpr (OP > 1) {
+#pragma unroll
+      for (int o = 0; o < OP; ++o) {
+        const Rows w = rows_of(o);
+        f32x16_t v = osum[o].total();
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] *= unscale;
+        if (p.mask) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) v[e] *= m[o];
+        }
+        global_rows(w).store(offset_of(o, w), v, res[o]);
+      }
+      continue;
+    }
+    f32x16_t oacc = osum[0].total();
+    const Rows w = rows_of(0);
+    const int j0 = w.j0, i = w.i, bb = w.bb;
     const Lane at = lane_here();
     if (KSPLIT > 1) {  // the waves of an output tile add up through the hidden tile's memory
       __syncthreads();
@@ -367,7 +419,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
     const int j = j0 + at.l32;
     if (p.mask) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) oacc[v] *= m;
+      for (int v = 0; v < 16; ++v) oacc[v] *= m[0];
     }
     if constexpr (BIAS) {
       float* row = rows + at.l32 * (C + kRowLd) + 32 * ot + 16 * at.lh;
@@ -381,11 +433,11 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       }
       for (int c = tid; c < C; c += 64 * NW) att_ln[c] = p.pb_ln_w[c], att_ln[C + c] = p.pb_ln_b ? p.pb_ln_b[c] : 0.f;
       constexpr int SPW = KS / 4;  // four waves share the sum over the channels
-      u32x4_t w[SPW][3];
+      u32x4_t wp[SPW][3];
       if (wave < 4) {
         const int head = at.l32 < p.pb_H ? at.l32 : p.pb_H - 1;  // the rows from H on are dropped
 #pragma unroll
-        for (int s = 0; s < SPW; ++s) split_operand(p.pb_w + (size_t)head * C, SPW * wave + s, at.lh, w[s]);
+        for (int s = 0; s < SPW; ++s) split_operand(p.pb_w + (size_t)head * C, SPW * wave + s, at.lh, wp[s]);
       }
       __syncthreads();  // the rows are complete, and everybody has read the partial sums
       const PassTile<C> xn = {reinterpret_cast<u32x4_t*>(rows + 32 * (C + kRowLd))};
@@ -394,8 +446,8 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
         const int pos = 4 * wave + here.lg;
         float4 y[C / 64];
 #pragma unroll
-        for (int e = 0; e < C / 64; ++e) raw[0].v[e] = *reinterpret_cast<const float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li);
-        norm_row<C>(raw[0], true, att_ln, here.li, y);
+        for (int e = 0; e < C / 64; ++e) raw[0][0].v[e] = *reinterpret_cast<const float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li);
+        norm_row<C>(raw[0][0], true, att_ln, here.li, y);
 #pragma unroll
         for (int e = 0; e < C / 64; ++e) xn.store4(pos, here.li + 16 * e, y[e]);
       }
@@ -407,7 +459,7 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
         for (int s = 0; s < SPW; ++s) {
           const u32x4_t* x = xn.s + PassTile<C>::slot(at.l32, 2 * (SPW * wave + s) + at.lh);
           const u32x4_t op[3] = {x[0], x[PassTile<C>::PLANE], x[2 * PassTile<C>::PLANE]};
-          acc = step6<true>(w[s], op, acc);
+          acc = step6<true>(wp[s], op, acc);
         }
         float* mine = part + wave * (32 * kBiasLd) + at.l32;
 #pragma unroll
@@ -424,22 +476,22 @@ __global__ __launch_bounds__(512) void transition_pass(TransitionPass p) {
       return;
     }
     if constexpr (AFTER) {
-      if (j < L) store_row16(rows + at.l32 * (C + kRowLd) + 32 * ot + 16 * at.lh, p.out + row0 + (int64_t)at.l32 * p.xv.stride_k + 32 * ot + 16 * at.lh, oacc, p.add_residual);
+      if (j < L) store_row16(rows + at.l32 * (C + kRowLd) + 32 * ot + 16 * at.lh, p.out + w.row0 + (int64_t)at.l32 * p.xv.stride_k + 32 * ot + 16 * at.lh, oacc, p.add_residual);
       return;
     } else {
-      out_rows.store(off, oacc, res);
+      global_rows(w).store(offset_of(0, w), oacc, res[0]);
     }
   }
 }
 
-template <int C, int S, int NPT, bool AFTER = false, bool BIAS = false, bool KEEP = false>
+template <int C, int S, int NPT, bool AFTER = false, bool BIAS = false, bool KEEP = false, int NW = 8>
 hipError_t launch(const TransitionPass& p, hipStream_t stream) {
   constexpr size_t lds = transition_lds<C, S, NPT, AFTER, BIAS>();
   unsigned grid = 0;
-  hipError_t e = resident_grid<transition_pass<C, S, NPT, AFTER, BIAS, KEEP>>(512, lds, (p.total + NPT - 1) / NPT, &grid);
+  hipError_t e = resident_grid<transition_pass<C, S, NPT, AFTER, BIAS, KEEP, NW>>(64 * NW, lds, (p.total + NPT - 1) / NPT, &grid);
   if (e != hipSuccess) return e;
   if (AFTER) grid = (unsigned)p.total;  // a tile each
-  hipLaunchKernelGGL((transition_pass<C, S, NPT, AFTER, BIAS, KEEP>), dim3(grid), dim3(512), lds, stream, p);
+  hipLaunchKernelGGL((transition_pass<C, S, NPT, AFTER, BIAS, KEEP, NW>), dim3(grid), dim3(64 * NW), lds, stream, p);
   return hipGetLastError();
 }
 
@@ -513,9 +565,9 @@ hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, 
   const bool large = p.total >= 4l * cus;  // two tiles of 64 positions for every CU
   if (a.HID % 256 != 0) {
     if (a.C == 128) return launch<128, 4, 2>(p, stream);
-    return a.HID == 128 ? launch<64, 4, 2, false, false, true>(p, stream) : launch<64, 4, 2>(p, stream);
+    return a.HID == 128 ? launch<64, 4, 1, false, false, true, 4>(p, stream) : launch<64, 4, 2>(p, stream);
   }
-  if (a.C == 128) return large ? launch<128, 8, 2>(p, stream) : launch<128, 8, 1>(p, stream);
+  if (a.C == 128) return large ? launch<128, 4, 2, false, false, false, 4>(p, stream) : launch<128, 8, 1>(p, stream);
   return large ? launch<64, 8, 2>(p, stream) : launch<64, 8, 1>(p, stream);
 }
 

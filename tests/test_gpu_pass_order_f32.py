@@ -74,3 +74,25 @@ def test_result_rows(n, c, inplace):
             q = {k[len(prefix):]: v for k, v in p64.items() if k.startswith(prefix)}
             want = oracle(z.double(), mask.double(), q)
             report(prefix, module(z.to(DEV), mask.to(DEV)).cpu(), want, atol=2 * REL * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("view", ["flat", "rows"])
+@pytest.mark.parametrize("c,n_mult,n", [(64, 2, 1), (64, 2, 31), (64, 2, 129), (64, 2, 187), (128, 4, 182), (128, 4, 183)])
+def test_transition_work_groups_of_four_waves(c, n_mult, n, view):
+    """One tile, a few and several per work-group; rows that follow one another and rows with a gap (ragged tiles at
+    their ends, and at 128 channels an odd number of 32-position tiles in pairs: 183 rows of 6)."""
+    lib()
+    gen = torch.Generator().manual_seed(8610 + n)
+    z = orc.make_pair_input(8611, (1,), n, c)
+    mask = (torch.rand(1, n, n, generator=gen) > 0.2).float()
+    p = orc.make_transition_params(gen, c, n_mult)
+    m = of3pair.SwiGLUTransition(c, n_mult)
+    m.load_state_dict(p, strict=True)
+    x = z.to(DEV)
+    if view == "rows":
+        x = torch.zeros(1, n, n + 3, c, device=DEV)[:, :, :n]
+        x.copy_(z)
+    print("transition", c, n_mult, n, view, flush=True)
+    want = orc.transition_update(z.double(), mask.double(), {k: v.double() for k, v in p.items()})
+    got = m.to(DEV).eval()(x, mask.to(DEV)).cpu()
+    report("update", got, want, atol=REL * float(want.abs().max()))
