@@ -57,3 +57,25 @@ def test_pair_biases_take_turns(monkeypatch, dtype, n, no_blocks, heads, batch, 
     m(a, b, tok, pair, inplace_safe=True)
     assert torch.equal(a, want[0]) and torch.equal(b, want[1])
     assert calls == ["of3_pairformer_stack_fwd"] * 4
+
+
+# room for every bias: s of two blocks goes together, of the last two each by itself
+@pytest.mark.parametrize("dtype,n", [(torch.bfloat16, 24), (torch.bfloat16, 131), (torch.float32, 40)])
+@pytest.mark.parametrize("no_blocks", [1, 2, 3, 4, 5, 6, 9])
+def test_single_representation_of_two_blocks_together(monkeypatch, dtype, n, no_blocks):
+    lib()
+    calls = _recorded(monkeypatch)
+    m, s, z, tok, pair = _stack(dtype, n, no_blocks)
+    print("stack", dtype, n, no_blocks, flush=True)
+    want = (s, z)
+    for blk in m.blocks:
+        want = blk(*want, tok, pair)
+    m(s, z, tok, pair)
+    del calls[:]
+    for _ in range(3):
+        got = m(s, z, tok, pair)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    a, b = s.clone(), z.clone()
+    m(a, b, tok, pair, inplace_safe=True)
+    assert torch.equal(a, want[0]) and torch.equal(b, want[1])
+    assert calls == ["of3_pairformer_stack_fwd"] * 4
