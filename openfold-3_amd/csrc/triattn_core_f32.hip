@@ -3,8 +3,9 @@
 // (pair_pass_f32.hip); pair_f32.hip has the cores for every other shape.
 //
 // Work-group = 4 waves = 2 consecutive rows i x 2 halves of one (head, 128-query range); a wave owns 64 queries (two
-// 32-query tiles) of one row.  Two work-groups share a CU, so that the products of one run under the exponentials and
-// splits of the other.
+// 32-query tiles) of one row.  Three work-groups share a CU, so that the products of one run under the exponentials and
+// splits of the others.  Bound by matrix and vector time at the clock that both leave (N = 768, heads of 32: 901 us a launch, matrix
+// pipe 48 %, vector pipe 63 %, 1.67 GHz; three bf16 terms 1446; heads of 16, three templates of 200: 54 us, 22 and 59 %; 88).
 //   S^T = K Q^T  (rows = keys, columns = queries), three products per k-step, started from the triangle bias (the
 //                accumulator is loaded with it).  Logits are in natural units times the scales of q and k, a power of
 //                two that the bias and the mask bias carry too, and not pre-multiplied by log2(e): a row of masked keys
@@ -17,8 +18,9 @@
 //                all four of the terms.
 // Per 32-key tile the work-group brings in the bias slice of its query range (it does not depend on i: shared by its
 // rows) and each row's K and V^T operands (shared by the row's two waves) with direct-to-LDS buffer loads, one tile
-// ahead, into double buffers: no registers are held for data in flight, and the only wait is one vmcnt(0) + barrier per
-// key tile, a whole tile of arithmetic after the loads were issued.  The bias slice is XOR-swizzled on the global side
+// ahead, the bias and (width 16) the operands into double buffers: no registers are held for data in flight, and the only wait for
+// loads is one vmcnt(0) + barrier per key tile, a whole tile of arithmetic after they were issued.  At width 32 the operands
+// have one place, which a second barrier frees once they are in registers: with two, only two work-groups fit (N = 768 4744 / 4596 us a pass).  The bias slice is XOR-swizzled on the global side
 // (a lane picks which 16-byte chunk it fetches for its fixed LDS slot).
 //
 // Softmax weights as fp16 terms have to lie between 2^-13 (below it their second terms lose bits) and 2^16.  The first
@@ -57,7 +59,7 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
   constexpr int QT = 2, D = 16 * STEPS;
   extern __shared__ u32x4_t lds4[];
   u32x4_t* tb_lds = lds4;                 // [2][kTb]
-  u32x4_t* kv_lds = lds4 + 2 * kTb;    // [kRows][2][K, V^T]
+  u32x4_t* kv_lds = lds4 + 2 * kTb;    // [kRows][kStages][K, V^T]
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row = wave >> 1, qh = wave & 1;
