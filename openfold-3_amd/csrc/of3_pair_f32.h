@@ -9,10 +9,12 @@ namespace of3 {
 // split, operand-ordered copy of a weight matrix [rows][K]: planes of ceil(rows / 32) * 32 * K values, three of bf16 or
 // two of fp16 (of3_split.h); behind the fp16 planes, the scales of each 32 rows
 struct WeightScales {
-  float unscale;    // 1 / (the weights' scale times `input`): from the accumulator to the layer's output
-  float input;      // the scale of the inputs where these come from a LayerNorm (the same for all rows), else 1
-  float output;     // the scale that the rows' outputs take as fp16 terms (0: not used as such)
-  float inv_bound;  // a power of two, 1 / it is a bound on the rows' outputs (inputs from a LayerNorm)
+  float unscale;   // from the accumulator to the layer's output, where its rows have one scale (not kUseProduct, kUseValues, kUseHidden);
+                   // without a LayerNorm before the layer a tile is 32 columns, and this what its products have to be multiplied with
+  float input;     // the scale of the inputs where these come from a LayerNorm (the same for all rows), else 1
+  float store;     // from the accumulator to the values that the outputs take as fp16 terms (0: not used as such)
+  float output;    // the scale of these, where the rows have one
+  float rows[32];  // ... of each row, where they have their own
 };
 struct WeightX3 {
   const bf16_t* h;
@@ -41,7 +43,7 @@ struct TrimulF32 {
   const float *w_ap, *w_ag, *w_bp, *w_bg, *w_g, *w_z;
   WeightX3 s_ap, s_ag, s_bp, s_bg, s_g, s_z;  // split copies (the *_x3 kernels only)
   float *a, *b, *x, *out;
-  // a and b as terms (three bf16, or two fp16 of the values times the scale of w_ap's and w_bp's outputs) in the k-panel
+  // a and b as terms (three bf16, or two fp16 of the values times the scales of w_ap's and w_bp's rows) in the k-panel
   // layout (the split-operand contraction only):
   // element (b, c, r, k) of a term sits at ((((b CH + c) Np / 32 + k / 32) Np + panel_row(r, c)) 32 + k % 32,
   // the terms ab_plane elements apart; Np = N rounded up to whole 32-wide panels
@@ -65,7 +67,7 @@ struct TriattnF32 {
   // head channels each) and planes of qk_plane elements; v^T always has two steps (16 keys each) of 32
   // rows, the rows from D on being zero, and planes of v_plane elements.  As fp16 terms at D = 16, v^T is one plane: the
   // rows 0 .. 15 of an operand are the first terms, 16 .. 31 the second ones of the same channels.  With fp16 terms tb
-  // holds the bias times the scales of q and k.
+  // holds the bias times the scales of q and k, and o is at the scales of v's channels.
   bf16_t *qs, *ks, *vs;
   long qk_plane, v_plane;
   int Jp;  // N rounded up to whole 32-position tiles

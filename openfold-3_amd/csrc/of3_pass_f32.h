@@ -149,14 +149,21 @@ __device__ __forceinline__ void load_unit(const WeightX3& W, int t, int lane_src
     for (int pl = 0; pl < TERMS; ++pl) w[s][pl] = src[pl * (W.plane / 8) + 64 * s];
 }
 
-// the scale of a gated attention output over C channels: a weighted mean of v, so no larger than v's bound
-template <int C>
-__device__ __forceinline__ float attention_scale(const WeightX3& Wv) {
-  float s = Wv.scales()[0].output;
+// Layers without a LayerNorm before them (fp16 terms): `total` leads from the accumulator to the output, where the inputs of column
+// tile t, at the scales of their channels, are multiplied with at(t) <= 1
+struct ColumnScales {
+  const WeightScales* s;
+  float total, inverse;
+  __device__ __forceinline__ ColumnScales(const WeightX3& W, int tiles) : s(W.scales()) {  // at most 32 tiles
+    const int l32 = threadIdx.x & 31;
+    float v = s[l32 < tiles ? l32 : tiles - 1].unscale;
 #pragma unroll
-  for (int t = 1; t < C / 32; ++t) s = fminf(s, Wv.scales()[t].output);
-  return s;
-}
+    for (int d = 16; d > 0; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 32));
+    total = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+    inverse = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(1.f / v)));
+  }
+  __device__ __forceinline__ float at(int t) const { return s[t].unscale * inverse; }
+};
 
 // rows of a fp32 weight matrix as split MFMA operands: k-values 16 s + 8 lh .. + 7 of `row`
 __device__ __forceinline__ void split_operand(const float* row, int s, int lh, u32x4_t (&w)[3]) {

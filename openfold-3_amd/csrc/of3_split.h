@@ -45,8 +45,8 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4_t& h, u32x4_t&
 // against float64 on normal operands, relative 2-norm in 1e-8, three bf16 terms | two fp16 terms | plain fp32 fused
 // multiply-adds: 32 values summed 6.8 | 9.3 | 10.4, 64 10.9 | 11.3 | 14.3, 128 16.3 | 14.2 | 20.5, 256 23.4 | 19.0 | 28.6, 768 42 | 31 | 50.
 // fp16 ends at 65504, so every operand is scaled by a power of two (exact) that a bound on its values allows: of3_weight_split.h.
-// Values far below that bound lose relative precision only where they are 2^-13 or less after scaling; an operand
-// bounded by 2^14 is held to 2^-39 of the bound.
+// Below 2^-3 after scaling the second term is one of fp16's subnormal numbers, 2^-24 apart, and has one bit less for every power
+// of two: an operand bounded by 2^14 is held to 2^-39 of the bound, 2^17 of them with all bits.
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
 typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2_t;
 __device__ __forceinline__ f32x16_t mfma_32x32x16_f16(u32x4_t a, u32x4_t b, f32x16_t c) {

@@ -863,8 +863,8 @@ __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, 
   }
 
   if constexpr (TERMS == 2) {
-    const int ct = bc % p.CH / 32;
-    const float unscale = 1.f / (p.s_ap.scales()[ct].output * p.s_bp.scales()[ct].output);
+    const int c = bc % p.CH;
+    const float unscale = 1.f / (p.s_ap.scales()[c / 32].rows[c % 32] * p.s_bp.scales()[c / 32].rows[c % 32]);
 #pragma unroll
     for (int mi = 0; mi < T; ++mi)
 #pragma unroll

@@ -60,12 +60,12 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
   float* msk = ln + 2 * C;                                 // [4][32]
   const int slot = grid_slot(), N = p.N, pair = kOneSide ? slot & 1 : wave / OT, ot = wave % OT;
   const WeightX3 Wg = pair ? p.s_bg : p.s_ag, Wp = pair ? p.s_bp : p.s_ap;
-  const WeightScales sg = Wg.scales()[ot], sp = Wp.scales()[ot];
+  const WeightScales &sg = Wg.scales()[ot], &sp = Wp.scales()[ot];
+  const float in_scale = sg.input, g_unscale = sg.unscale, out_scale = sp.store;
   u32x4_t wg[KS][2], wp[KS][2];
   load_unit<C, 2>(Wg, ot, lane, wg);
   load_unit<C, 2>(Wp, ot, lane, wp);
-  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_in_w[c] * sg.input, ln[C + c] = p.ln_in_b[c] * sg.input;
-  const float out_scale = sp.unscale * sp.output;
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_in_w[c] * in_scale, ln[C + c] = p.ln_in_b[c] * in_scale;
   wait_vmcnt<0>();  // the weights have landed: no wait for them, and with it for the rows in flight, inside the loop
   __syncthreads();
 
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int v = 8 * st + 4 * a + e;
-            x[4 * a + e] = m[e] * sigmoid_hw_f32(ag[v], sg.unscale) * (ap[v] * out_scale);
+            x[4 * a + e] = m[e] * sigmoid_hw_f32(ag[v], g_unscale) * (ap[v] * out_scale);
           }
         }
         split8h(x, op[st][0], op[st][1]);
@@ -233,12 +233,13 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int N = p.N;
-  const WeightScales sg = p.s_g.scales()[wave], sz = p.s_z.scales()[wave];
+  const WeightScales &sg = p.s_g.scales()[wave], &sz = p.s_z.scales()[wave];
+  const float g_in = sg.input, g_unscale = sg.unscale, z_in = sz.input, z_unscale = sz.unscale;
   OutWeights<C> w;
   w.load(p.s_g, p.s_z, wave, l32, lh);
   for (int c = tid; c < C; c += 64 * NW) {
-    ln[c] = p.ln_in_w[c] * sg.input, ln[C + c] = p.ln_in_b[c] * sg.input;
-    ln[2 * C + c] = p.ln_out_w[c] * sz.input, ln[3 * C + c] = p.ln_out_b[c] * sz.input;
+    ln[c] = p.ln_in_w[c] * g_in, ln[C + c] = p.ln_in_b[c] * g_in;
+    ln[2 * C + c] = p.ln_out_w[c] * z_in, ln[3 * C + c] = p.ln_out_b[c] * z_in;
   }
   wait_vmcnt<0>();  // the weights
   __syncthreads();
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
     __syncthreads();  // LayerNorm(x) is complete, and everybody has finished with the first tile
     f32x16_t acc = unit_product<C, true>(second, w.o);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = acc[v] * sz.unscale * sigmoid_hw_f32(gate[v], sg.unscale);
+    for (int v = 0; v < 16; ++v) acc[v] = acc[v] * z_unscale * sigmoid_hw_f32(gate[v], g_unscale);
     rows.add(wave, acc, p.add_residual);
     before = t;
     first = false;
@@ -382,18 +383,19 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
   const int h0 = H * part / PARTS, h1 = H * (part + 1) / PARTS;  // this work-group's heads of the bias
   const bool narrow = p.D == 16;
   const WeightX3 W = kind == 0 ? p.s_q : kind == 1 ? p.s_k : p.s_v;
-  const WeightScales sc = W.scales()[ot];
+  const WeightScales& sc = W.scales()[ot];
+  const float in_scale = sc.input;
+  // q / sqrt(c) after the projection (attention.py:283-284)
+  const float out_scale = sc.store * (kind == 0 ? 1.0f / sqrtf((float)p.D) : 1.f);
   u32x4_t w[KS][2];
   load_unit<C, 2>(W, ot, tid & 63, w);
-  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * sc.input, ln[C + c] = p.ln_b[c] * sc.input;
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * in_scale, ln[C + c] = p.ln_b[c] * in_scale;
   for (int c = tid; c < H * C; c += 64 * NW) {
     const int t = c / C * p.D / 32;  // the head's tile of q and k
-    wb[c] = p.w_b[c] * (p.s_q.scales()[t].output * p.s_k.scales()[t].output / sc.input);
+    wb[c] = p.w_b[c] * (p.s_q.scales()[t].output * p.s_k.scales()[t].output / in_scale);
   }
   wait_vmcnt<0>();  // the weights
   __syncthreads();
-  // q / sqrt(c) after the projection (attention.py:283-284)
-  const float out_scale = sc.unscale * sc.output * (kind == 0 ? 1.0f / sqrtf((float)p.D) : 1.f);
 
   // panel -> its row (b N + i) and first position
   auto row_of = [&](int pn, int& j0) {
@@ -519,12 +521,12 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int N = p.N;
-  const WeightScales sg = p.s_g.scales()[wave];
-  const float o_scale = attention_scale<C>(p.s_v);
-  const float unscale = p.s_o.scales()[wave].unscale / o_scale;
+  const WeightScales& sg = p.s_g.scales()[wave];
+  const ColumnScales so(p.s_o, NW);
+  const float g_in = sg.input, g_unscale = sg.unscale, o_scale = so.at(wave), unscale = so.total;
   OutWeights<C> w;
   w.load(p.s_g, p.s_o, wave, l32, lh);
-  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * sg.input, ln[C + c] = p.ln_b[c] * sg.input;
+  for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * g_in, ln[C + c] = p.ln_b[c] * g_in;
   wait_vmcnt<0>();  // the weights
   __syncthreads();
 
@@ -601,7 +603,7 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
       const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
       float y[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = ov[e] * o_scale * sigmoid_hw_f32(gate[8 * hf + e], sg.unscale);
+      for (int e = 0; e < 8; ++e) y[e] = ov[e] * o_scale * sigmoid_hw_f32(gate[8 * hf + e], g_unscale);
       second.store8(mid.l32, 4 * wave + 2 * mid.lh + hf, y);
     }
     load_o(next);

@@ -32,7 +32,7 @@ struct TransitionPass {
   int HID, add_residual;
   // the attention before it (AFTER)
   const float *att_o, *att_ln_w, *att_ln_b;
-  WeightX3 att_g, att_out, att_v;
+  WeightX3 att_g, att_out;
   int N;
   // the pair bias of the result (BIAS)
   const float *pb_w, *pb_ln_w, *pb_ln_b;
@@ -45,14 +45,6 @@ template <int C, int S, int NPT, bool AFTER, bool BIAS>
 constexpr size_t transition_lds() {
   return (size_t)NPT * (HalfTile<C>::SLOTS + HalfTile<32 * S>::SLOTS) * 16 + 2 * C * sizeof(float) +
          (AFTER ? (2 * C + 32 * (C + kRowLd)) * sizeof(float) : 0) + (BIAS ? PassTile<C>::SLOTS * 16 : 0);
-}
-// the smallest of a value over the first n <= 32 tiles of a weight matrix
-__device__ __forceinline__ float smallest_inv_bound(const WeightX3& W, int n) {
-  const int lane = threadIdx.x & 31;
-  float v = W.scales()[lane < n ? lane : n - 1].inv_bound;
-#pragma unroll
-  for (int d = 16; d > 0; d >>= 1) v = fminf(v, __shfl_xor(v, d, 32));
-  return v;
 }
 
 // AFTER: the tile begins with the output pass of the ending node's triangle attention (triattn_out_pass: same steps, same bits), its gates in
@@ -91,10 +83,9 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
   const int ht = S == NW ? wave : wave & 3, pt_a = S == NW ? 0 : wave >> 2;
   const int ot = wave % OT, pt_b = OP > 1 ? 0 : (wave / OT) % NPT, kh = wave / (OT * NPT);
   const int L = p.L, slices = p.HID / (32 * S);
-  // The activations' scale is in ln, the hidden ones take the largest that the bounds of their two factors allow
+  // The activations' scale is in ln, those of the hidden channels are in the rows of Wb, their inverses in the columns of Wout
   const float x_scale = p.s_a.scales()[0].input;
-  const float h_scale = fminf(0x1p14f * smallest_inv_bound(p.s_a, p.HID / 32) * smallest_inv_bound(p.s_b, p.HID / 32), 0x1p40f);
-  const float unscale = p.s_out.scales()[ot].unscale / h_scale;
+  const ColumnScales so(p.s_out, p.HID / 32);
   for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * x_scale, ln[C + c] = p.ln_b[c] * x_scale;
 
   const int lane0 = tid & 63, src_lane = rowperm16(lane0 & 31) + (lane0 & 32);  // outputs dealt by rowperm16
@@ -159,8 +150,8 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
       const XTile xn = {lds}, gated = {hid};
       u32x4_t w[KS][2];
       load_unit<C, 2>(kh == 0 ? p.att_g : p.att_out, ot, src_lane, w);
-      const float o_scale = attention_scale<C>(p.att_v);
-      const float att_unscale = kh == 0 ? p.att_g.scales()[ot].unscale : p.att_out.scales()[ot].unscale / o_scale;
+      const ColumnScales att_so(p.att_out, OT);
+      const float o_scale = att_so.at(ot), att_unscale = kh == 0 ? p.att_g.scales()[ot].unscale : att_so.total;
       int j0;
       const int b = row_of(tile, j0);  // one row per batch element
       const Lane here = lane_here();
@@ -280,7 +271,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
     for (int slice = 0; slice < slices; ++slice) {
       // requested ahead of the operands (where the registers allow it): behind them they wait for every operand in flight
       float ua, ub;
-      auto load_scales = [&] { ua = p.s_a.scales()[slice * S + ht].unscale, ub = ua * p.s_b.scales()[slice * S + ht].unscale * h_scale; };
+      auto load_scales = [&] { ua = p.s_a.scales()[slice * S + ht].unscale, ub = ua * p.s_b.scales()[slice * S + ht].store * so.at(slice * S + ht); };
       if (kEarly) load_scales();
       __syncthreads();  // the activations (first slice), or: everybody has read the slice before
       f32x16_t a[XT], b[XT];
@@ -384,7 +375,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
         const Rows w = rows_of(o);
         f32x16_t v = osum[o].total();
 #pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] *= unscale;
+        for (int e = 0; e < 16; ++e) v[e] *= so.total;
         if (p.mask) {
 #pragma unroll
           for (int e = 0; e < 16; ++e) v[e] *= m[o];
@@ -415,7 +406,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
       }
     }
 #pragma unroll
-    for (int v = 0; v < 16; ++v) oacc[v] *= unscale;
+    for (int v = 0; v < 16; ++v) oacc[v] *= so.total;
     const int j = j0 + at.l32;
     if (p.mask) {
 #pragma unroll
@@ -549,7 +540,6 @@ hipError_t transition_pass_f32(const TransitionF32Args& a, const WeightX3& s_a, 
     p.att_ln_b = a.end->ln_b;
     p.att_g = a.end->s_g;
     p.att_out = a.end->s_o;
-    p.att_v = a.end->s_v;
     p.N = a.N;
     if (a.bias && pair_bias_pass_serves(*a.bias) && a.bias->C == 128 && a.bias->N == a.N && a.bias->B == a.B) {
       p.pb_w = a.bias->w;

@@ -89,7 +89,6 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
   const int wt = h * D / 32;  // the head's tile of 32 rows of its weights
   const float logit_scale = p.s_q.scales()[wt].output * p.s_k.scales()[wt].output;
   const float to_exp2 = 1.4426950408889634f / logit_scale;
-  const float v_unscale = 1.f / p.s_v.scales()[wt].output;
 
   u32x4_t qop[QT][STEPS][2];
 #pragma unroll
@@ -391,7 +390,7 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
     for (int qt = 0; qt < QT; ++qt) {
       const int q = q0 + 32 * qt + l32;
       if (q >= N) continue;
-      const float inv = 1.0f / l_tot[qt] * v_unscale;
+      const float inv = 1.0f / l_tot[qt];  // o keeps the scales of v's channels, w_o has their inverses
       if constexpr (STEPS == 1) {
 #pragma unroll
         for (int v = 0; v < 8; ++v) oacc[qt][v] += oacc[qt][v + 8];
