@@ -112,6 +112,17 @@ __device__ __forceinline__ float group_sum(float v) {
   if (LPP == 16) v += dpp_move<0x140>(v);  // row_mirror
   return v;
 }
+// the same moves: the largest of a wave's 64 values
+__device__ __forceinline__ int wave_max(int v) {
+  auto larger = [](int a, int b) { return a > b ? a : b; };
+  auto bits = [](int i) { return __int_as_float(i); };
+  v = larger(v, __float_as_int(dpp_move<0xB1>(bits(v))));
+  v = larger(v, __float_as_int(dpp_move<0x4E>(bits(v))));
+  v = larger(v, __float_as_int(dpp_move<0x141>(bits(v))));
+  v = larger(v, __float_as_int(dpp_move<0x140>(bits(v))));
+  return larger(larger(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+                larger(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
 
 // ---- LayerNorm of one position spread over C/8 lanes -------------------------------------
 // raw: the lane's 8 channels (bf16 packed); w, b: affine parameters of those 8 channels.

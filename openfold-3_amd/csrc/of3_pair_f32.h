@@ -22,6 +22,22 @@ struct WeightX3 {
   int terms;
   __device__ __forceinline__ const WeightScales* scales() const { return reinterpret_cast<const WeightScales*>(h + 2 * plane); }
 };
+// The largest absolute value of a pair mask, as the triangle multiplication's fp16 terms need it: a and b are those of mask 2^-exponent, at
+// most 1.  Behind the scales of w_ap: partial maxima from the launch that splits the weights, and the exponent from trimul_proj_pass
+// for the contraction.
+struct MaskTop {
+  static constexpr int kParts = 64;
+  int exponent;
+  float parts[kParts];
+  // work-groups that take them: 1024 values each, four to a thread, until there are 64
+  __host__ __device__ static int count(const float* mask, int B, int N) {
+    const long n = mask ? ((long)B * N * N + 1023) / 1024 : 0;
+    return n < kParts ? (int)n : kParts;
+  }
+  __host__ __device__ static MaskTop* of(const WeightX3& w_ap) {  // the third plane, of at least 64 x 64 values
+    return reinterpret_cast<MaskTop*>(const_cast<bf16_t*>(w_ap.h) + 2 * w_ap.plane + 2048);
+  }
+};
 __host__ __device__ constexpr long packed_elems(long rows, long K) { return (rows + 31) / 32 * 32 * K; }
 
 // Row of a k-panel that holds row r of channel c: the rows of a channel's panels are rotated by 4 c.  A store of the

@@ -149,20 +149,35 @@ __device__ __forceinline__ void load_unit(const WeightX3& W, int t, int lane_src
     for (int pl = 0; pl < TERMS; ++pl) w[s][pl] = src[pl * (W.plane / 8) + 64 * s];
 }
 
+// the least e with |mask| <= 2^e, of the whole mask: its loads first, what follows from them behind other loads
+struct MaskExponent {
+  uint32_t part;  // of a non-negative number: ordered as the bits
+  int count;
+  __device__ __forceinline__ void load(const TrimulF32& p) {
+    const int lane = threadIdx.x & 63;
+    count = MaskTop::count(p.mask, p.B, p.N);
+    part = __float_as_uint(MaskTop::of(p.s_ap)->parts[lane < count ? lane : 0]);
+  }
+  __device__ __forceinline__ int of_wave() const {
+    const int top = count ? wave_max((int)part) : 0;
+    return top == 0 ? 0 : __builtin_amdgcn_frexp_expf(__uint_as_float(top - 1));
+  }
+};
+
 // Layers without a LayerNorm before them (fp16 terms): `total` leads from the accumulator to the output, where the inputs of column
 // tile t, at the scales of their channels, are multiplied with at(t) <= 1
 struct ColumnScales {
   const WeightScales* s;
-  float total, inverse;
-  __device__ __forceinline__ ColumnScales(const WeightX3& W, int tiles) : s(W.scales()) {  // at most 32 tiles
+  float total;
+  // at most 32 tiles; the load first, what follows from it behind other loads
+  __device__ __forceinline__ ColumnScales(const WeightX3& W, int tiles) : s(W.scales()) {
     const int l32 = threadIdx.x & 31;
-    float v = s[l32 < tiles ? l32 : tiles - 1].unscale;
-#pragma unroll
-    for (int d = 16; d > 0; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 32));
-    total = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
-    inverse = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(1.f / v)));
+    total = s[l32 < tiles ? l32 : tiles - 1].unscale;
   }
-  __device__ __forceinline__ float at(int t) const { return s[t].unscale * inverse; }
+  __device__ __forceinline__ void finish() { total = __int_as_float(wave_max(__float_as_int(total))); }  // positive: ordered as the bits
+  __device__ __forceinline__ float at(int t) const {
+    return s[t].unscale * __uint_as_float(0x7f000000u - __float_as_uint(total));  // 1 / total, a power of two
+  }
 };
 
 // rows of a fp32 weight matrix as split MFMA operands: k-values 16 s + 8 lh .. + 7 of `row`

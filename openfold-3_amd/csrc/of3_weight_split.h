@@ -39,12 +39,17 @@ struct SplitJobs {
   // norm: the LayerNorm that the inputs come from; with: kUseHidden: the matrix whose outputs are multiplied with this one's, without a
   // LayerNorm: the matrix whose outputs (times something of at most 1) are the inputs
   uint8_t terms[kMax], norm[kMax], use[kMax], with[kMax];
+  // a mask [B][N][N] whose largest value is taken by work-groups behind those of the tiles
+  const float* mask;
+  PairView mask_view;
+  int B, N, mask_parts, masked;
+  MaskTop* mask_top[kMax / kBlock * 2];
 };
 constexpr uint8_t kNone = 255;
 // What becomes of a layer's outputs, which decides the scale that they take (fp16 terms only)
 enum LayerUse : uint8_t {
   kUsePlain,      // nothing is multiplied with them as terms
-  kUseProduct,    // a and b of the triangle multiplication, times the mask: bound at 2^8, which leaves masks up to 255
+  kUseProduct,    // a and b of the triangle multiplication, times a mask of at most 1 (MaskTop)
   kUseLogits,     // q and k: scale at most 2^24 (a logit and its biases are scaled by both: 2^48, where a mask bias of
                   // -1e9 and far beyond is finite)
   kUseValues,     // v
@@ -81,6 +86,15 @@ struct WeightSplitter {
     w += 3 * dst.plane;  // room for either form: the scales of two planes lie in the third's
     return j.n++;
   }
+  // of a triangle multiplication; all of a launch have the same mask
+  void take_mask(const TrimulF32Args& a, const WeightX3& w_ap) {
+    j.mask = a.mask;
+    j.mask_view = a.mask_view;
+    j.B = a.B;
+    j.N = a.N;
+    j.mask_parts = MaskTop::count(a.mask, a.B, a.N);
+    j.mask_top[j.masked++] = MaskTop::of(w_ap);
+  }
   hipError_t launch(hipStream_t stream) const { return split_weights_launch(j, stream); }
 };
 
@@ -110,6 +124,7 @@ inline void trimul_split_jobs(WeightSplitter& s, const TrimulF32Args& a, bool ha
   s.terms = half ? 2 : 3;
   s.input(a.ln_in_w, a.ln_in_b);
   s.add(a.w_ap, a.CH, a.C, w[0], kUseProduct);
+  if (half) s.take_mask(a, w[0]);
   s.add(a.w_ag, a.CH, a.C, w[1]);
   s.add(a.w_bp, a.CH, a.C, w[2], kUseProduct);
   s.add(a.w_bg, a.CH, a.C, w[3]);

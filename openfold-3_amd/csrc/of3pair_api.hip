@@ -1049,8 +1049,8 @@ struct BlockWeights {
 // Prepares the matrices of n <= kPrepared blocks at dst by one launch (4 to 5 us however many they are)
 constexpr int kPrepared = of3::PackJobs::kMax / of3::PackJobs::kBlock;
 static_assert(kPrepared * of3::SplitJobs::kBlock <= of3::SplitJobs::kMax, "");
-static hipError_t prepare_blocks(const void* const* const* weights, int n, const BlockDims& k, void* dst, BlockWeights* out,
-                                 hipStream_t stream) {
+static hipError_t prepare_blocks(const void* const* const* weights, int n, const BlockDims& k, const float* mask, const int64_t mask_strides[3],
+                                 void* dst, BlockWeights* out, hipStream_t stream) {
   const int64_t C = k.C, CH = k.CH, HD = k.H * k.D;
   if (k.wide()) {
     of3::WeightSplitter splitter(dst);
@@ -1069,7 +1069,9 @@ static hipError_t prepare_blocks(const void* const* const* weights, int n, const
           of3::TrimulF32Args a;
           a.ln_in_w = f(w[0]), a.ln_in_b = f(w[1]), a.ln_out_w = f(w[2]), a.ln_out_b = f(w[3]);
           a.w_ap = f(w[4]), a.w_ag = f(w[5]), a.w_bp = f(w[6]), a.w_bg = f(w[7]), a.w_g = f(w[8]), a.w_z = f(w[9]);
-          a.C = (int)C, a.CH = (int)CH;
+          a.C = (int)C, a.CH = (int)CH, a.B = (int)k.B, a.N = (int)k.N;
+          a.mask = mask;
+          a.mask_view = mask_view(mask, mask_strides, false);
           of3::trimul_split_jobs(splitter, a, k.rows16 && of3::trimul_half_shapes(k.B, k.N, C, CH), next);
         }
       }
@@ -1220,7 +1222,7 @@ static int pair_block_fwd(const void* const* weights, const void* z, const int64
   if (workspace_bytes < need) return OF3_ENOSPC;
   d.rows16 = rows16(z, out, z_strides);
   BlockWeights k;
-  const hipError_t e = prepare_blocks(&weights, 1, d, static_cast<char*>(workspace) + need - d.prepared_bytes(), &k,
+  const hipError_t e = prepare_blocks(&weights, 1, d, mask, mask_strides, static_cast<char*>(workspace) + need - d.prepared_bytes(), &k,
                                       static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail_hip(e);
   return run_pair_block(k, d, z, z_strides, mask, mask_strides, out, flags, workspace, workspace_bytes, stream, bias, bias_done);
@@ -1437,7 +1439,7 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
     const bool last = i + 1 == blocks;
     if (q == 0) {
       const int n = (int)(blocks - i < kPrepared ? blocks - i : kPrepared);
-      const hipError_t e = prepare_blocks(weights + i, n, d, prepared, k, streams.main);
+      const hipError_t e = prepare_blocks(weights + i, n, d, pair_mask, mask_strides, prepared, k, streams.main);
       if (e != hipSuccess) return fail_hip(e);
     }
     const void* const* ws_ = weights[i] + OF3_PAIR_BLOCK_WEIGHTS;

@@ -865,12 +865,13 @@ __global__ __launch_bounds__(128 * WM) void trimul_contract_x3_f32(TrimulF32 p, 
   if constexpr (TERMS == 2) {
     const int c = bc % p.CH;
     const float unscale = 1.f / (p.s_ap.scales()[c / 32].rows[c % 32] * p.s_bp.scales()[c / 32].rows[c % 32]);
+    const int mask_e = 2 * MaskTop::of(p.s_ap)->exponent;
 #pragma unroll
     for (int mi = 0; mi < T; ++mi)
 #pragma unroll
       for (int ni = 0; ni < T; ++ni)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[mi][ni][v] *= unscale;
+        for (int v = 0; v < 16; ++v) acc[mi][ni][v] = __builtin_ldexpf(acc[mi][ni][v] * unscale, mask_e);
   }
   float* xc = p.x + (size_t)bc * N * N;
 #pragma unroll

@@ -62,11 +62,14 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
   const WeightX3 Wg = pair ? p.s_bg : p.s_ag, Wp = pair ? p.s_bp : p.s_ap;
   const WeightScales &sg = Wg.scales()[ot], &sp = Wp.scales()[ot];
   const float in_scale = sg.input, g_unscale = sg.unscale, out_scale = sp.store;
+  MaskExponent mask_top;
   u32x4_t wg[KS][2], wp[KS][2];
   load_unit<C, 2>(Wg, ot, lane, wg);
   load_unit<C, 2>(Wp, ot, lane, wp);
+  mask_top.load(p);
   for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_in_w[c] * in_scale, ln[C + c] = p.ln_in_b[c] * in_scale;
   wait_vmcnt<0>();  // the weights have landed: no wait for them, and with it for the rows in flight, inside the loop
+  const int mask_e = mask_top.of_wave();
   __syncthreads();
 
   struct Place {
@@ -115,7 +118,7 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) xn.store4(pos, li + 16 * e, y[e]);
     }
-    if (tid < 32) msk[32 * (n & 3) + tid] = mraw;
+    if (tid < 32) msk[32 * (n & 3) + tid] = __builtin_ldexpf(mraw, -mask_e);
     load_tile(id + step < total ? id + step : id);
   };
   if (first_id >= total) return;  // the whole work-group
@@ -190,6 +193,8 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
     if (n + (early ? 2 : 1) < count) normalise(n + (early ? 2 : 1));
     if (!early && n + 1 < count) __syncthreads();
   }
+  // block 0 has a tile.  Not ahead of the rows, whose wait would be for this store too (0.5 us of 8 at one tile per work-group)
+  if (blockIdx.x == 0 && tid == 0) MaskTop::of(p.s_ap)->exponent = mask_e;
 }
 
 // ---- output passes ------------------------------------------------------------------------------------------
@@ -522,12 +527,14 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int N = p.N;
   const WeightScales& sg = p.s_g.scales()[wave];
-  const ColumnScales so(p.s_o, NW);
-  const float g_in = sg.input, g_unscale = sg.unscale, o_scale = so.at(wave), unscale = so.total;
+  const float g_in = sg.input, g_unscale = sg.unscale;
   OutWeights<C> w;
   w.load(p.s_g, p.s_o, wave, l32, lh);
+  ColumnScales so(p.s_o, NW);
   for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * g_in, ln[C + c] = p.ln_b[c] * g_in;
   wait_vmcnt<0>();  // the weights
+  so.finish();
+  const float o_scale = so.at(wave), unscale = so.total;
   __syncthreads();
 
   auto place = [&](int id, int& b, int& i) {  // returns the first position

@@ -85,7 +85,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
   const int L = p.L, slices = p.HID / (32 * S);
   // The activations' scale is in ln, those of the hidden channels are in the rows of Wb, their inverses in the columns of Wout
   const float x_scale = p.s_a.scales()[0].input;
-  const ColumnScales so(p.s_out, p.HID / 32);
+  ColumnScales so(p.s_out, p.HID / 32);
   for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * x_scale, ln[C + c] = p.ln_b[c] * x_scale;
 
   const int lane0 = tid & 63, src_lane = rowperm16(lane0 & 31) + (lane0 & 32);  // outputs dealt by rowperm16
@@ -144,14 +144,14 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
       const float s = p.att_g.scales()[0].input;
       att_ln[c] = p.att_ln_w[c] * s, att_ln[C + c] = p.att_ln_b[c] * s;
     }
+  so.finish();
   __syncthreads();
   for (; tile < tiles; tile += gridDim.x) {
     if constexpr (AFTER) {
       const XTile xn = {lds}, gated = {hid};
       u32x4_t w[KS][2];
       load_unit<C, 2>(kh == 0 ? p.att_g : p.att_out, ot, src_lane, w);
-      const ColumnScales att_so(p.att_out, OT);
-      const float o_scale = att_so.at(ot), att_unscale = kh == 0 ? p.att_g.scales()[ot].unscale : att_so.total;
+      ColumnScales att_so(p.att_out, OT);
       int j0;
       const int b = row_of(tile, j0);  // one row per batch element
       const Lane here = lane_here();
@@ -190,6 +190,8 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
         xn.store4(pos, here.li + 16 * e, y[e]);
         *reinterpret_cast<float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li) = raw[0][0].v[e];
       }
+      att_so.finish();
+      const float o_scale = att_so.at(ot), att_unscale = kh == 0 ? p.att_g.scales()[ot].unscale : att_so.total;
       __syncthreads();
       if (kh == 0) {
         const f32x16_t gate = product(xn);

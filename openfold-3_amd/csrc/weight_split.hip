@@ -16,15 +16,6 @@ __device__ __forceinline__ int clamp(int e, int low, int high) { return e < low 
 __device__ __forceinline__ int exponent(float v) {
   return v != 0.f && __builtin_fabsf(v) < __builtin_inff() ? __builtin_amdgcn_frexp_expf(v) : kAbsent;
 }
-__device__ __forceinline__ int wave_max(int v) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    const int o = __shfl_xor(v, d, 64);
-    v = v > o ? v : o;
-  }
-  return v;
-}
-
 __device__ __forceinline__ bool aligned16(const float* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 template <int n>
 __device__ __forceinline__ void load(const float* p, bool aligned, float* x) {
@@ -69,15 +60,14 @@ __device__ __forceinline__ Row row_of(const SplitJobs& j, int q, int item) {
       top_w = fmaxf(top_w, __builtin_fabsf(w[e])), top_b = fmaxf(top_b, __builtin_fabsf(b[e]));
     }
   }
+  static_assert(kRowLanes == 4, "a quad of lanes");
   auto row_max = [](float v) {
-#pragma unroll
-    for (int d = 1; d < kRowLanes; d *= 2) v = fmaxf(v, __shfl_xor(v, d, 64));
-    return v;
+    v = fmaxf(v, dpp_move<0xB1>(v));
+    return fmaxf(v, dpp_move<0x4E>(v));
   };
   auto row_sum = [](float v) {
-#pragma unroll
-    for (int d = 1; d < kRowLanes; d *= 2) v += __shfl_xor(v, d, 64);
-    return v;
+    v += dpp_move<0xB1>(v);
+    return v + dpp_move<0x4E>(v);
   };
   top = row_max(top), top_w = row_max(top_w), top_b = row_max(top_b);
   const float root = sqrtf((float)K);
@@ -118,13 +108,13 @@ __device__ __forceinline__ TileScale shared_scale(const Row& row, bool logits) {
   s.store = s.output - s.weight - row.input;
   return s;
 }
-// Or one each: outputs at 2^limit, weights as far below 2^14 as that takes with one `store` for all (a wave's rows are in its
+// Or one each: outputs at 2^14, weights as far below 2^14 as that takes with one `store` for all (a wave's rows are in its
 // registers: one number in place of 16).  A row that would put the others' weights more than 2^8 lower keeps its own
 // and its outputs are lower.
-__device__ __forceinline__ TileScale own_scale(const Row& row, int bound, int limit) {
+__device__ __forceinline__ TileScale own_scale(const Row& row, int bound) {
   TileScale s;
   const bool live = bound != kAbsent;
-  const int want = clamp(limit - bound, -60, 60), lead = want - row.weight - row.input;
+  const int want = clamp(14 - bound, -60, 60), lead = want - row.weight - row.input;
   const int most = wave_max(live ? lead : kAbsent), least = -wave_max(live ? -lead : kAbsent);
   s.store = most == kAbsent ? 0 : most < least + 8 ? most : least + 8;
   s.weight = live && want - row.input - s.store < row.weight ? want - row.input - s.store : row.weight;
@@ -136,11 +126,35 @@ __device__ __forceinline__ TileScale own_scale(const Row& row, int bound, int li
 // of tile t of matrix q, `with`: that of the matrix that its outputs are multiplied with (kUseHidden)
 __device__ __forceinline__ TileScale tile_scale(int use, const Row& row, const Row& with) {
   switch (use) {
-    case kUseProduct: return own_scale(row, row.bound, 8);
-    case kUseValues: return own_scale(row, row.bound, 14);
-    case kUseHidden: return own_scale(row, row.bound == kAbsent || with.bound == kAbsent ? kAbsent : row.bound + with.bound, 14);
+    case kUseProduct:
+    case kUseValues: return own_scale(row, row.bound);
+    case kUseHidden: return own_scale(row, row.bound == kAbsent || with.bound == kAbsent ? kAbsent : row.bound + with.bound);
     default: return shared_scale(row, use == kUseLogits);
   }
+}
+
+// of work-group `part`: what is no finite number makes its own products no finite numbers and is left out
+__device__ void mask_top(const SplitJobs& j, int part) {
+  __shared__ float tops[kWaves];
+  const long values = (long)j.B * j.N * j.N;
+  float top = 0.f;
+  auto take = [&](auto number) {
+    typedef decltype(number) Index;
+    const Index N = j.N, all = values, step = j.mask_parts * kThreads;
+#pragma unroll 4
+    for (Index at = part * kThreads + threadIdx.x; at < all; at += step) {
+      const Index row = at / N, k = at - row * N, b = row / N, r = row - b * N;
+      const float v = __builtin_fabsf(j.mask[(long)b * j.mask_view.stride_b + (long)r * j.mask_view.stride_r + (long)k * j.mask_view.stride_k]);
+      top = v < __builtin_inff() ? fmaxf(top, v) : top;
+    }
+  };
+  if (values < 1l << 31) take(0u);  // divisions of 64 bits cost as much as the loads
+  else take(0ul);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) top = fmaxf(top, __shfl_xor(top, d, 64));
+  if (threadIdx.x % 64 == 0) tops[threadIdx.x / 64] = top;
+  __syncthreads();
+  if ((int)threadIdx.x < j.masked) j.mask_top[threadIdx.x]->parts[part] = fmaxf(fmaxf(tops[0], tops[1]), fmaxf(tops[2], tops[3]));
 }
 
 // A work-group per tile of 32 rows, or of 32 columns without a LayerNorm before them (fp16 terms), a thread per (row tile,
@@ -152,6 +166,7 @@ __global__ __launch_bounds__(kThreads) void split_weights_f32(SplitJobs j) {
   __shared__ int columns[32];
   __shared__ int tops[kWaves];
   const int tile = blockIdx.x, tid = threadIdx.x;
+  if (tile >= j.first[j.n]) return mask_top(j, tile - j.first[j.n]);
   int q = 0, end = j.n;  // the matrix that holds the tile
   while (end - q > 1) {
     const int mid = (q + end) / 2;
@@ -252,7 +267,7 @@ __global__ __launch_bounds__(kThreads) void split_weights_f32(SplitJobs j) {
 }  // namespace
 
 hipError_t split_weights_launch(const SplitJobs& jobs, hipStream_t stream) {
-  hipLaunchKernelGGL(split_weights_f32, dim3((unsigned)jobs.first[jobs.n]), dim3(kThreads), 0, stream, jobs);
+  hipLaunchKernelGGL(split_weights_f32, dim3((unsigned)(jobs.first[jobs.n] + jobs.mask_parts)), dim3(kThreads), 0, stream, jobs);
   return hipGetLastError();
 }
 

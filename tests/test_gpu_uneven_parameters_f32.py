@@ -37,7 +37,7 @@ def _norm_channel(p, norm, behind, s, channel=3):
         p[_name(p, name)][:, channel] /= s
 
 
-def _check(what, module, args, oracle, p):
+def _check(what, module, args, oracle, p, beyond=0.0):
     want = oracle(*[a.double() for a in args], {k: v.double() for k, v in p.items()})
     plain = oracle(*args, p)
     module.load_state_dict(p, strict=True)
@@ -48,7 +48,7 @@ def _check(what, module, args, oracle, p):
 
     print("%s: relative 2-norm %.3e, plain fp32 %.3e" % (what, error(got), error(plain)), flush=True)
     assert got.isfinite().all()
-    assert error(got) <= error(plain)
+    assert error(got) <= error(plain) + beyond
 
 
 @pytest.mark.parametrize("c,n_mult", [(64, 2), (64, 4), (128, 4)])
