@@ -37,6 +37,11 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4_t& h, u32x4_t&
   }
 }
 
+// A mask bias as the matrix instructions can add logits to it: with an even mantissa.  What is negative and far below half of the
+// accumulator's last bit is rounded as that half, to the even neighbour: an odd bias of -1e10 lost a last bit, 1024, to every negative logit
+// and to no other, and a row of masked keys averaged those that had lost none.
+__device__ __forceinline__ float even_bias(float v) { return __uint_as_float(__float_as_uint(v) & ~1u); }
+
 // ---- two fp16 terms -----------------------------------------------------------------------------
 // x s = h + l with h = fp16(x s), l = fp16(x s - h) and s a power of two: 22 to 23 significant bits, and three products
 //     x w = (l wh + h wl + h wh) / (sx sw)        (l wl is below 2^-22 |x w| and left out)

@@ -145,7 +145,7 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
     return mrow[k * mstep];
   };
   auto mask_bias = [&](int kt, float mv) {
-    return kt * 32 + l32 < N ? (p.mask ? p.inf * (mv - 1.f) : 0.f) : -__builtin_inff();
+    return kt * 32 + l32 < N ? (p.mask ? even_bias(p.inf * (mv - 1.f)) : 0.f) : -__builtin_inff();
   };
   // the mask-bias k-step on the 8-deep MFMA (two registers per operand): lanes 0..31 hold k = 0..3
   auto mask_step = [&](float mb, f32x16_t acc) {
