@@ -20,6 +20,8 @@
 // 18, 71, 18200 | 3.2.
 #pragma once
 
+#include <cmath>
+
 #include "of3_kernels.h"
 #include "of3_pair_f32.h"
 
@@ -44,14 +46,15 @@ struct SplitJobs {
   PairView mask_view;
   int B, N, mask_parts, masked;
   MaskTop* mask_top[kMax / kBlock * 2];
+  int logit_limit;  // largest exponent of the scale of q and of k
 };
 constexpr uint8_t kNone = 255;
 // What becomes of a layer's outputs, which decides the scale that they take (fp16 terms only)
 enum LayerUse : uint8_t {
   kUsePlain,      // nothing is multiplied with them as terms
   kUseProduct,    // a and b of the triangle multiplication, times a mask of at most 1 (MaskTop)
-  kUseLogits,     // q and k: scale at most 2^24 (a logit and its biases are scaled by both: 2^48, where a mask bias of
-                  // -1e9 and far beyond is finite)
+  kUseLogits,     // q and k: a logit and its biases are scaled by both, so their scale is at most 2^24, less for mask biases beyond
+                  // 1e22 (logit_limit)
   kUseValues,     // v
   kUseHidden,     // times silu of the outputs of `with`
 };
@@ -136,6 +139,8 @@ inline void triattn_split_jobs(WeightSplitter& s, const TriattnF32Args& a, bool 
   const int HD = a.H * a.D;
   s.terms = half ? 2 : 3;
   s.input(a.ln_w, a.ln_b);
+  // inf (mask - 1) times both scales is finite: for masks up to 16 with an inf near fp32's largest number, 2^50 at 1e9
+  s.j.logit_limit = (int)std::fmin(24.f, std::floor((122.f - std::log2(std::fmax(a.inf, 1.f))) / 2.f));
   s.add(a.w_q, HD, a.C, w[0], kUseLogits);
   s.add(a.w_k, HD, a.C, w[1], kUseLogits);
   const int v = s.add(a.w_v, HD, a.C, w[2], kUseValues);

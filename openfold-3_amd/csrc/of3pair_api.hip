@@ -1082,7 +1082,7 @@ static hipError_t prepare_blocks(const void* const* const* weights, int n, const
           of3::TriattnF32Args a;
           a.ln_w = f(w[0]), a.ln_b = f(w[1]);
           a.w_q = f(w[3]), a.w_k = f(w[4]), a.w_v = f(w[5]), a.w_g = f(w[6]), a.w_o = f(w[7]);
-          a.C = (int)C, a.H = (int)k.H, a.D = (int)k.D;
+          a.C = (int)C, a.H = (int)k.H, a.D = (int)k.D, a.inf = k.inf;
           of3::triattn_split_jobs(splitter, a, k.rows16 && of3::triattn_half_shapes(k.B, k.N, C, k.H, k.D), next);
         }
       }

@@ -100,11 +100,11 @@ struct TileScale {
   int weight, output, store;
 };
 // the rows have one scale
-__device__ __forceinline__ TileScale shared_scale(const Row& row, bool logits) {
+__device__ __forceinline__ TileScale shared_scale(const Row& row, bool logits, int logit_limit) {
   TileScale s;
   s.weight = -wave_max(-row.weight);
   const int bound = wave_max(row.bound);
-  s.output = logits && bound != kAbsent ? clamp(14 - bound, -110, 24) : 0;
+  s.output = logits && bound != kAbsent ? clamp(14 - bound, -110, logit_limit) : 0;
   s.store = s.output - s.weight - row.input;
   return s;
 }
@@ -124,12 +124,12 @@ __device__ __forceinline__ TileScale own_scale(const Row& row, int bound) {
   return s;
 }
 // of tile t of matrix q, `with`: that of the matrix that its outputs are multiplied with (kUseHidden)
-__device__ __forceinline__ TileScale tile_scale(int use, const Row& row, const Row& with) {
+__device__ __forceinline__ TileScale tile_scale(int use, int logit_limit, const Row& row, const Row& with) {
   switch (use) {
     case kUseProduct:
     case kUseValues: return own_scale(row, row.bound);
     case kUseHidden: return own_scale(row, row.bound == kAbsent || with.bound == kAbsent ? kAbsent : row.bound + with.bound);
-    default: return shared_scale(row, use == kUseLogits);
+    default: return shared_scale(row, use == kUseLogits, logit_limit);
   }
 }
 
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(kThreads) void split_weights_f32(SplitJobs j) {
       if (lane % kRowLanes == 0) bounds[kItemRows * wave + lane / kRowLanes] = r;
     }
     __syncthreads();
-    const TileScale scale = tile_scale(j.use[one], bounds[l32], bounds[(other != one) * 32 + l32]);
+    const TileScale scale = tile_scale(j.use[one], j.logit_limit, bounds[l32], bounds[(other != one) * 32 + l32]);
     if (normed) {
       const float ws = power_of_two(scale.weight);
       for (int s = wave; s < steps; s += kWaves) {

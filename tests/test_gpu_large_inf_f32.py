@@ -1,5 +1,6 @@
-"""fp32 triangle attention with other mask biases than -1e9: with odd mantissas, to which the matrix instructions do not add a
-small logit as it should be (64 and 128 channels: two fp16 terms, 96: three bf16 terms, 40: no matrix instructions)."""
+"""fp32 triangle attention with other mask biases than -1e9: near fp32's largest numbers, where they are multiplied with the scales of q
+and k (two fp16 terms: 64 and 128 channels), and with odd mantissas, to which the matrix instructions do not add a small logit as it
+should be (all biases but 1e9 here; 96 channels: three bf16 terms, 40: no matrix instructions)."""
 import pytest
 import torch
 
@@ -14,7 +15,7 @@ DEV = "cuda"
 
 @pytest.mark.parametrize("c,d", [(64, 16), (128, 32), (96, 32), (40, 8)])
 @pytest.mark.parametrize("size", [1e-3, 1.0])  # of the weights: the smaller they are the larger the scales
-@pytest.mark.parametrize("inf", [1e9, 1e10, 1e15])
+@pytest.mark.parametrize("inf", [1e9, 1e10, 1e15, 1e25, 1e33, 1e38])
 def test_large_inf(inf, size, c, d):
     lib()
     n = 45
