@@ -392,6 +392,12 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
     }
   };
 
+  auto any_uneven = [&]() {  // the same answer in every wave; nobody reads a buffer of the tiles before it any more
+    bool bad = false;
+#pragma unroll
+    for (int rq = 0; rq < kRQ; ++rq) bad |= row_valid && q0 + 32 * rq + l32 < N && uneven[rq] != 0;
+    return __syncthreads_or(bad) != 0;
+  };
   const uint32_t mb_off = krow * sizeof(float);
   float mb_next;
   auto first_loads = [&]() {
@@ -429,9 +435,15 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
       tile(kind, buf, mb_cur, op, N - 32 * kt);
       compiler_fence();
     };
-    for (int kt = 0; kt < nkt; kt += 2) {
-      step(kt, 0);
-      if (kt + 1 < nkt) step(kt + 1, 1);
+    // The level pass looks whether it is of any use after 2, 8, 32 ... tiles: one that is not has then taken a small part of the second
+    // pass's time (at its end / so, q times 24, a fifth of the tokens padded, us: pair stack N = 384 531 / 518, 768 2591 / 2527; where the logits are
+    // level no difference: 1842 / 1845)
+    for (int kt = 0, stop = kLevel ? 2 : nkt;; stop *= 4) {
+      for (; kt < nkt && kt < stop; kt += 2) {
+        step(kt, 0);
+        if (kt + 1 < nkt) step(kt + 1, 1);
+      }
+      if (!kLevel || kt >= nkt || any_uneven()) break;
     }
     wait_vmcnt<0>();  // the loads issued past the end must not outlive the pass (or the work-group's LDS)
 #pragma unroll
@@ -481,10 +493,7 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
   level &= again;
   if (level) {
     pass(std::integral_constant<int, kLevelled>{});
-    bool bad = false;
-#pragma unroll
-    for (int rq = 0; rq < kRQ; ++rq) bad |= row_valid && q0 + 32 * rq + l32 < N && uneven[rq] != 0;
-    level = !__syncthreads_or(bad);
+    level = !any_uneven();
     if (!level) first_loads();
   } else if (!again) {
     pass(std::integral_constant<int, kFirst>{});

@@ -45,3 +45,32 @@ def test_level_rows(what, n, c, d, dtype):
     assert torch.equal(torch.isnan(out[0]), torch.isnan(out[1]))
     assert torch.equal(torch.nan_to_num(out[0].float()), torch.nan_to_num(out[1].float()))
     assert bool(torch.isnan(out[0]).any()) == (what == "nan")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("c,d", [(64, 16), (128, 32)])
+# keys on both sides of the tiles after which the core looks: 2, 8 of 32 keys, the last
+@pytest.mark.parametrize("n,key", [(65, 0), (65, 40), (65, 64), (451, 31), (451, 63), (451, 64), (451, 250), (451, 256), (451, 450)])
+def test_one_logit_is_not_level(n, key, c, d, dtype):
+    """The triangle bias of one query and key alone is too large for the mask bias to take up."""
+    lib()
+    gen = torch.Generator().manual_seed(8720 + c)
+    p = orc.make_triattn_params(gen, c, d, c // d)
+    name = [k for k in p if p[k].dim() == 2 and p[k].shape[0] == c // d][0]
+    p[name][:, 0] = 100.0
+    p["layer_norm.bias"][0] = 0.0
+    z = orc.make_pair_input(8721, (1,), n, c)
+    z = z - z.mean(-1, keepdim=True)
+    z[..., 0] = 0.0
+    query = n - 2
+    z[0, query, key, 0] = 1e3
+    m = of3pair.TriangleAttention(c, d, c // d)
+    m.load_state_dict(p, strict=True)
+    m = m.to(DEV).to(dtype).eval()
+    print("one logit", key, n, c, dtype, flush=True)
+    out = []
+    for rows in (range(4, 8), (5,)):
+        mask = torch.ones(1, n, n)
+        mask[:, list(rows)] = 0.0
+        out.append(m(z.to(DEV).to(dtype), mask.to(DEV))[0, 5].cpu())
+    assert torch.equal(out[0], out[1]) and bool(torch.isfinite(out[0]).all())
