@@ -73,7 +73,8 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
   // steps that an operand is requested ahead: an L2 read takes about as long as 24 MFMAs of two waves per SIMD
   constexpr int DA = KEEP ? KS : XT == 1 ? 2 : 1, DO = KEEP ? OSTEPS : 4 / OP;
   static_assert(OSTEPS >= DO && KS >= DA, "");
-  // the residual before the next tile's rows and a slice's scales before its operands; there they would spill
+  // the residual before the next tile's rows, a slice's scales before its operands and Wout's first operands before the hidden values; there
+  // they would spill (four templates of 200, 64 channels, n = 4: with 4 registers spilled 1242 us a pass, so 1238; two of 300 1453, 1446)
   constexpr bool kEarly = !(C == 64 && S == 8 && NPT == 2), kEarlyRes = kEarly && OP == 1;
   extern __shared__ u32x4_t lds[];
   u32x4_t* const hid = lds + NPT * XTile::SLOTS;
@@ -300,7 +301,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
           }
           if (s + 1 < KS) read_x(s + 1);
           if (s + DA < KS) fetch_ab(slice, s + DA);
-          if (!KEEP && s + 1 == KS) {
+          if (!KEEP && kEarly && s + 1 == KS) {
 #pragma unroll
             for (int q = 0; q < DO; ++q) fetch_o(slice, q);
           }
@@ -315,7 +316,11 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
 #pragma unroll
         for (int t = 0; t < XT; ++t) a[t] = sum_a[t].total(), b[t] = sum_b[t].total();
       }
-      if (!kEarly) load_scales();
+      if (!kEarly) {
+        load_scales();
+#pragma unroll
+        for (int q = 0; q < DO; ++q) fetch_o(slice, q);
+      }
       {
         const Lane at = lane_here();
 #pragma unroll
