@@ -1415,10 +1415,11 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
   // block j overwrites the bias that attention j - buffers reads, and waits for attention j - ahead or the one after it
   const int64_t ahead = w.buffers < 2 ? w.buffers : 2;
   StreamPair streams(static_cast<hipStream_t>(stream), static_cast<hipStream_t>(side_stream));
-  // Where every block has a bias of its own, s of two blocks goes to the side stream together, behind one wait in place of two.  Of the last
-  // two blocks each goes by itself: the one beside the last pair updates, the other after them.  s of two blocks takes less than the pair updates
-  // of one (66 us of 68 at 40 tokens), so nothing ends later.  Four blocks, one wait a block / for two, us: N = 40 bf16, where the host sets the
-  // pace, 375 / 332, N = 64 fp32 493 / 487, N = 200 bf16 825 / 822.
+  // Where every block has a bias of its own, s of two blocks goes to the side stream together, behind one wait in place of two, as long as two more pair
+  // updates follow: beside one alone it may end later (three blocks, waited for, one wait a block / for two, us: N = 40 310 / 329, 200 678 / 696).  Pair
+  // updates take longer than s of their block (68 us against 33 at 40 tokens), so behind two of them nothing is left over.  One wait a block / for two, us, calls one after
+  // the other, bf16, where the host sets the pace: four blocks N = 16 343 / 331, 40 349 / 331, 64 350 / 332, eight at 40 657 / 614; further up no difference
+  // (four at 130 557 / 558, at 200 802 / 804); fp32, four blocks, 16 437 / 434, 24 445 / 440.
   const bool pairs = streams.main != streams.side && w.buffers >= blocks;
   auto attention = [&](int64_t j, int phases, hipStream_t on) {
     const void* const* ws_ = weights[j] + OF3_PAIR_BLOCK_WEIGHTS;
@@ -1435,7 +1436,7 @@ int of3_pairformer_stack_fwd(const void* const* const* weights, int64_t blocks, 
   int st = OF3_OK;
   for (int64_t i = 0; i < blocks && st == OF3_OK; ++i) {
     const int q = (int)(i % kPrepared);
-    const bool hold = pairs && i % 2 == 0 && i + 2 < blocks;  // s goes with the next block's
+    const bool hold = pairs && i % 2 == 0 && i + 3 < blocks;  // s goes with the next block's
     const bool last = i + 1 == blocks;
     if (q == 0) {
       const int n = (int)(blocks - i < kPrepared ? blocks - i : kPrepared);

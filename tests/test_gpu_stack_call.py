@@ -59,7 +59,7 @@ def test_pair_biases_take_turns(monkeypatch, dtype, n, no_blocks, heads, batch, 
     assert calls == ["of3_pairformer_stack_fwd"] * 4
 
 
-# room for every bias: s of two blocks goes together, of the last two each by itself
+# room for every bias: s of two blocks goes together as long as two more follow, of the last two or three each by itself
 @pytest.mark.parametrize("dtype,n", [(torch.bfloat16, 24), (torch.bfloat16, 131), (torch.float32, 40)])
 @pytest.mark.parametrize("no_blocks", [1, 2, 3, 4, 5, 6, 9])
 def test_single_representation_of_two_blocks_together(monkeypatch, dtype, n, no_blocks):
