@@ -60,11 +60,13 @@
  * every tensor and parameter is fp32, pointers 4-byte aligned, strides any positive
  * element counts, any N, C and CH <= 256, H*D <= 256 with D <= 64; fp32-grade
  * arithmetic in the reference's order of operations.  With channel counts in multiples of
- * 16 the two triangle modules compute every fp32 product from three bf16 terms per operand
- * on the bf16 matrix instructions (six exact products, summed in fp32; the workspace holds
- * the split weights and intermediates); channel counts in multiples of 8 and the pair
- * transition use the fp32 matrix instructions, every other shape plain FMA kernels.  The
- * stage entry points are bf16 only.
+ * 16 the two triangle modules compute every fp32 product from split operands on the 16-bit
+ * matrix instructions (the workspace holds the split weights and intermediates): at
+ * C = CH (H*D) = 64 or 128 with rows on 16-byte boundaries two fp16 terms per operand and three
+ * products, else three bf16 terms and six, summed in fp32; a pair mask may then have any finite
+ * values, and keeps full precision in those within 2^10 of the largest.  Channel counts in
+ * multiples of 8 and the pair transition without a workspace use the fp32 matrix instructions,
+ * every other shape plain FMA kernels.  The stage entry points are bf16 only.
  */
 #ifndef OF3PAIR_H
 #define OF3PAIR_H
@@ -202,8 +204,8 @@ int of3_transition_fwd(const void* x, const int64_t x_strides[3], const float* m
                        void* stream);
 
 /* The same with a workspace (same reference lines): in fp32, with
- * of3_transition_workspace_bytes_for(dtype, B, N, C, HID) bytes (256-byte aligned) for the weights
- * split into three bf16 terms, C a multiple of 16 and HID a multiple of 128 run on the bf16 matrix
+ * of3_transition_workspace_bytes_for(dtype, B, N, C, HID) bytes (256-byte aligned) for the split
+ * weights, C a multiple of 16 and HID a multiple of 128 run on the 16-bit matrix
  * instructions with fp32-grade products, as the triangle modules do; other shapes, a null workspace
  * and bf16 (which needs none: 0 bytes) behave exactly like of3_transition_fwd. */
 int64_t of3_transition_workspace_bytes_for(int dtype, int64_t B, int64_t N, int64_t C, int64_t HID);

@@ -260,13 +260,14 @@ struct TrimulF32Args {
   float* out;
   int B, N, C, CH, add_residual;
 };
-// a and b in three bf16 terms each, rows and k padded to whole 32-wide panels
+// a and b in three bf16 terms each, rows and k padded to whole 32-wide panels.  Here and below: two fp16 terms take two thirds
+// of it, but which form a call takes depends on its tensors' alignment too, which a workspace is sized without.
 inline size_t trimul_ab_split_bytes(long B, long N, long CH) {
   const long Np = (N + 31) / 32 * 32;
   return (size_t)12 * B * CH * Np * Np;
 }
 hipError_t trimul_fwd_f32(const TrimulF32Args& args, hipStream_t stream);
-// room for the six weight matrices split into three bf16 terms each, rows padded to multiples of 32
+// room for the six weight matrices split into terms (three bf16, or two fp16 and their scales), rows padded to multiples of 32
 inline long wsplit_elems(long rows, long K) { return (rows + 31) / 32 * 32 * K; }
 inline size_t trimul_wsplit_bytes(long C, long CH) {
   return (size_t)6 * (4 * wsplit_elems(CH, C) + wsplit_elems(C, C) + wsplit_elems(C, CH));
@@ -295,7 +296,7 @@ hipError_t triattn_fwd_f32(const TriattnF32Args& args, hipStream_t stream);
 inline size_t triattn_wsplit_bytes(long C, long H, long D) {
   return (size_t)6 * (4 * wsplit_elems(H * D, C) + wsplit_elems(C, H * D));
 }
-// q, k and v^T in three bf16 terms each, rows padded to whole 32-position tiles; v^T operands always
+// q, k and v^T in three bf16 terms each (two fp16 take less), rows padded to whole 32-position tiles; v^T operands always
 // have 32 rows (head widths below 32 leave the rest zero)
 inline size_t triattn_qkv_split_bytes(long B, long N, long H, long D) {
   return (size_t)6 * B * N * H * ((N + 31) / 32 * 32) * (2 * D + (D > 32 ? D : 32));
@@ -316,7 +317,7 @@ struct TransitionF32Args {
   const struct PairBiasF32Args* bias = nullptr;
   bool* bias_done = nullptr;
 };
-// the three weight matrices split into three bf16 terms each, rows padded to multiples of 32
+// the three weight matrices split into terms (three bf16, or two fp16 and their scales), rows padded to multiples of 32
 inline size_t transition_wsplit_bytes(long C, long HID) {
   return (size_t)6 * (2 * wsplit_elems(HID, C) + wsplit_elems(C, HID));
 }

@@ -187,7 +187,7 @@ int64_t of3_trimul_workspace_bytes(int64_t B, int64_t N, int64_t C, int64_t CH) 
 int64_t of3_trimul_workspace_bytes_for(int dtype, int64_t B, int64_t N, int64_t C, int64_t CH) {
   if (dtype == OF3_DTYPE_BF16) return of3_trimul_workspace_bytes(B, N, C, CH);
   if (dtype != OF3_DTYPE_F32 || !f32_trimul_dims_ok(B, N, C, CH)) return OF3_EINVAL;
-  // a, b (fp32, or split into three bf16 terms in whole 32-wide panels), x and the weights split into three bf16 terms
+  // a, b (fp32, or split into terms in whole 32-wide panels: room for three bf16 ones), x and the weights split likewise
   return f32_trimul_ab_bytes(B, N, CH) + align256(B * CH * N * N * 4) + align256((int64_t)of3::trimul_wsplit_bytes(C, CH));
 }
 
@@ -404,8 +404,8 @@ int64_t of3_triattn_workspace_bytes(int64_t B, int64_t N, int64_t C, int64_t H, 
 int64_t of3_triattn_workspace_bytes_for(int dtype, int64_t B, int64_t N, int64_t C, int64_t H, int64_t D) {
   if (dtype == OF3_DTYPE_BF16) return of3_triattn_workspace_bytes(B, N, C, H, D);
   if (dtype != OF3_DTYPE_F32 || !f32_triattn_dims_ok(B, N, C, H, D)) return OF3_EINVAL;
-  // q, k, v (fp32, or split into three bf16 terms in whole 32-position tiles), o, the triangle bias
-  // and the weights split into three bf16 terms
+  // q, k, v (fp32, or split into terms in whole 32-position tiles: room for three bf16 ones), o, the triangle bias
+  // and the weights split likewise
   return f32_triattn_qkv_bytes(B, N, H, D) + align256(B * N * N * H * D * 4) + f32_triattn_tb_bytes(B, N, H) +
          align256((int64_t)of3::triattn_wsplit_bytes(C, H, D));
 }
@@ -598,7 +598,7 @@ int of3_triattn_fwd(const void* x, const int64_t x_strides[3], const float* mask
 int64_t of3_transition_workspace_bytes_for(int dtype, int64_t B, int64_t N, int64_t C, int64_t HID) {
   if (dtype == OF3_DTYPE_BF16) return (B >= 1 && N >= 1) ? 0 : (int64_t)OF3_EINVAL;
   if (dtype != OF3_DTYPE_F32 || B < 1 || N < 1 || C < 1 || C > 256 || HID < 1 || HID > 1024) return OF3_EINVAL;
-  return align256((int64_t)of3::transition_wsplit_bytes(C, HID));  // the weights split into three bf16 terms
+  return align256((int64_t)of3::transition_wsplit_bytes(C, HID));  // the weights split into terms
 }
 
 int of3_transition_fwd(const void* x, const int64_t x_strides[3], const float* mask, const int64_t mask_strides[3],

@@ -722,19 +722,20 @@ __global__ __launch_bounds__(kThreads * PT) void trimul_proj_x3_f32(TrimulF32 p,
   }
 }
 
-// Contraction on split operands: x[b][c][i][j] = sum_k a[b][c][i][k] b[b][c][j][k] in fp32, six bf16
-// products per k-step.  Work-group = WM x 2 waves = one tile of one channel, a wave owns T x T MFMA tiles of 32 x 32.
-// Per 32-wide k-panel the three terms of the tile's a rows and b rows
+// Contraction on split operands: x[b][c][i][j] = sum_k a[b][c][i][k] b[b][c][j][k] in fp32, per k-step six products
+// (TERMS = 3, bf16) or three (TERMS = 2, fp16: 64 and 128 channels).  Work-group = WM x 2 waves = one tile of one channel, a wave owns T x T MFMA tiles of 32 x 32.
+// Per 32-wide k-panel the terms of the tile's a rows and b rows
 // travel global -> LDS with direct-to-LDS buffer loads.  A row of a panel is 64 bytes = 4 chunks of 16 bytes; chunk c of row
 // r is stored at position c ^ ((r >> 2) & 3), so that the 8 lanes of an operand read (8 rows, same
 // chunk) fall into different banks; the swizzle is applied on the global side.  Parts of a tile past the last panel row are
 // neither loaded nor multiplied.
-// The matrix pipes bound it from 300 tokens on (1.25 PFLOP/s of bf16 products at N = 768), the 12 bytes per element of a and b
-// around 200 (4 TB/s), one work-group's chain load -> products -> store below that.  Four forms, summing in the same order:
-//   <4, 2, 2>  256 x 128, two stages of LDS, alone on its CU: the next panel's loads run beside a panel's products.
-//   <4, 2, 1>  256 x 128, one stage (72 KB), two work-groups on a CU.
-//   <2, 2, 1>  128 x 128, one stage (48 KB): three work-groups on a CU, one's products beside another's loads, first panel and stores.
-//   <2, 1, 1>  64 x 64, one stage (24 KB).
+// Two | three terms: the matrix pipes bound it from 300 tokens on (N = 768: 355 us, 0.98 PFLOP/s of products, the pipes 57 % busy | 1.25 PFLOP/s),
+// the 8 | 12 bytes per element of a and b around 200 (4 TB/s), one work-group's chain load -> products -> store below that.  Four
+// forms, summing in the same order, with the LDS of two | three terms:
+//   <4, 2, 2>  256 x 128, two stages (96 | 144 KB), alone on its CU: the next panel's loads run beside a panel's products.
+//   <4, 2, 1>  256 x 128, one stage (48 | 72 KB), two work-groups on a CU.
+//   <2, 2, 1>  128 x 128, one stage (32 | 48 KB): three work-groups on a CU, one's products beside another's loads, first panel and stores.
+//   <2, 1, 1>  64 x 64, one stage (16 | 24 KB).
 template <int WM, int T, int STAGES, int TERMS>
 struct CtX3 {
   static constexpr int kWaves = 2 * WM, kM = 32 * T * WM, kN = 64 * T;
@@ -912,7 +913,12 @@ hipError_t launch_contract_x3(const TrimulF32& p, int cus, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Whole passes, us, with tiles of 256 x 128 multiplied in full (all there was before) | 256 x 128 | 128 | 64:
+// Whole passes on two terms, us, two stages of 256 x 128 | one | 128 | 64 (rounds of all four in turn, medians of 7; two runs of one differ by 1 %):
+//   pair stack: N = 48 97 | 98 | 97 | 94, 100 149 | 150 | 151 | 144, 128 153 | 155 | 154 | 149, 140 202 | 205 | 201 | 200, 163 227 | 233 | 232 | 238,
+//     200 309 | 314 | 308 | 316, 256 395 | 393 | 391 | 397, 300 593 | 596 | 591 | 599, 384 915 | 915 | 900 | 917, 768 4600 | 4561 | 4591 | 4781
+//   templates of 64 channels: 4 x 128 502 | 508 | 507 | 498, 2 x 150 429 | 435 | 428 | 433, 3 x 162 656 | 647 | 665 | 687, 3 x 200
+//     913 | 888 | 934 | 926, 2 x 300 1321 | 1320 | 1338 | 1364, 2 x 400 2630 | 2586 | 2597 | 2649, 4 x 512 8321 | 8183 | 8268 | 8438
+// On three terms, where the lines were found, with tiles of 256 x 128 multiplied in full (all there was before) | 256 x 128 | 128 | 64:
 //   pair stack, 128 channels: N = 64 123 | 117 | 117 | 114, 128 191 | 186 | 189 | 183, 163 314 | 301 | 301 | 322, 200 426 | 418 | 416 | 436,
 //     256 549 | 544 | 546 | 562, 300 920 | 888 | 871 | 869, 384 1379 | 1361 | 1351 | 1374, 600 4093 | 3965 | 3938 | 4064
 //   templates of 64 channels (3 x 162, 3 x 200: 845, 1233 with one stage, which pays from two rounds on: 163 and 200 above 307, 429):

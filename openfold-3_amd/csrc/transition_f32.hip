@@ -3,8 +3,8 @@
 //     out = [x +] ((silu(LN(x) Wa^T) * (LN(x) Wb^T)) Wout^T) * mask
 // pair_f32.hip has the kernels for every other shape.
 //
-// 18 flops per channel and hidden channel in fp16 products: 0.7 Tflop for N = 768 at n = 4, 365 us of the matrix
-// pipes at the rate they sustain.  The split weights (393 KB at C = 128, n = 4) do not fit a CU and stream from L2.
+// 18 flops per channel and hidden channel in fp16 products: 0.17 Tflop for N = 384 at n = 4, 145 us at the 1.2 PFLOP/s of a large bf16
+// product, 207.5 taken (0.84).  The split weights (393 KB at C = 128, n = 4) do not fit a CU and stream from L2.
 // One wave per tile of 32 hidden channels and all of the tile's positions: a work-group of eight waves takes the
 // hidden dimension in slices of 32 S channels (S = 8, or 4 with a wave per position tile), so that an operand of Wa
 // and Wb is read once for 64 positions and a slice of 256 hidden channels costs two barriers, against 32 positions

@@ -473,8 +473,8 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
   // ordinary size up (128 are between it and its neighbours).  The weights then are equal and the result is the mean of v, the same
   // for every query: no exponentials, no maxima, no sums, and P V for one of the query tiles; the bits are those of the pass with
   // running maxima, which comes after it where a logit is another.  Launches, us: N = 2048, 256 tokens padded, 6389 / 5922, 384, 38
-  // padded, 56.5 / 53.9; whole passes 24.4 / 23.4 ms and 1087 / 1077, one block at 929, 40 padded, 3735 / 3711, four templates of 512, 51
-  // padded, 3558 / 3522.
+  // padded, 56.5 / 53.9; whole passes 24.4 / 23.4 ms, four templates of 512, 51 padded, 3558 / 3522; with 10 % of 384 or 4 % of 929
+  // padded no more than two runs differ.
   // A work-group with a row whose sampled keys (its own token, the first, the middle and the last) are all masked is
   // taken for one with a padded token, which fails that test for certain, and goes to the second pass at once; a wrong
   // guess costs it the offsets' arithmetic and nothing else.  A launch that fits the chip at once lasts as long as its
