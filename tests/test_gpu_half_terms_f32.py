@@ -37,6 +37,15 @@ def _f64(p):
     return {k: v.double() for k, v in p.items()}
 
 
+def _no_worse_than_fp32(got, want, plain):
+    """The whole result (REL alone is some 70 times the kernels' error): no further off than fp32 arithmetic on the same values."""
+    def error(x):
+        return float((x.double() - want).norm() / want.norm())
+
+    print("relative 2-norm %.3e, plain fp32 %.3e" % (error(got), error(plain)), flush=True)
+    assert error(got) <= error(plain)
+
+
 SCALES = [(1.0, 1.0, 30.0), (1e-4, 1.0, 1.0), (30.0, 0.1, 1.0), (0.02, 50.0, 1.0), (1e12, 1e-12, 1.0)]
 
 
@@ -52,6 +61,7 @@ def test_trimul_scales(c, weights, norms, spread):
     want = orc.trimul_update(z.double(), mask.double(), _f64(p), True)
     got = _module(of3pair.TriangleMultiplicationOutgoing, p, c, c)(z.to(DEV), mask.to(DEV)).cpu()
     report("update", got, want, atol=REL * float(want.abs().max()))
+    _no_worse_than_fp32(got, want, orc.trimul_update(z, mask, p, True))
 
 
 @pytest.mark.parametrize("c,d", [(64, 16), (128, 32)])
@@ -68,6 +78,7 @@ def test_triattn_scales(c, d, weights, norms, spread):
     want = orc.triattn_update(z.double(), mask.double(), _f64(p), c // d)
     got = _module(of3pair.TriangleAttention, p, c, d, c // d)(z.to(DEV), mask.to(DEV)).cpu()
     report("update", got, want, atol=4 * REL * float(want.abs().max()))
+    _no_worse_than_fp32(got, want, orc.triattn_update(z, mask, p, c // d))
 
 
 @pytest.mark.parametrize("c,n_mult", [(64, 2), (128, 4)])
@@ -81,6 +92,7 @@ def test_transition_scales(c, n_mult, weights, norms, spread):
     want = orc.transition_update(z.double(), None, _f64(p))
     got = _module(of3pair.SwiGLUTransition, p, c, n_mult)(z.to(DEV)).cpu()
     report("update", got, want, atol=REL * float(want.abs().max()))
+    _no_worse_than_fp32(got, want, orc.transition_update(z, None, p))
 
 
 @pytest.mark.parametrize("c,d", [(64, 16), (128, 32)])
