@@ -38,7 +38,7 @@ def test_trimul_masks(what, n, c):
                spread)
 
 
-@pytest.mark.parametrize("view", ["transposed", "one row", "batch"])
+@pytest.mark.parametrize("view", ["plain", "transposed", "one row", "batch", "off 16 bytes"])
 def test_trimul_mask_views(view):
     lib()
     c, n, b = 128, 37, 3
@@ -53,12 +53,32 @@ def test_trimul_mask_views(view):
         mask = mask.to(DEV).transpose(-1, -2)
     elif view == "one row":
         mask = mask[:, n - 1:].to(DEV).expand(b, n, n)
+    elif view == "plain":
+        mask = mask.to(DEV)
+    elif view == "off 16 bytes":
+        mask = torch.empty(mask.numel() + 1, device=DEV)[1:].view(mask.shape).copy_(mask)
     else:
         mask = mask[b - 1:].to(DEV).expand(b, n, n)
     print("mask view", view, flush=True)
     want = orc.trimul_update(z.double(), mask.cpu().double(), {k: v.double() for k, v in p.items()}, True)
     got = m.to(DEV).eval()(z.to(DEV), mask).cpu()
     report("update", got, want, atol=1e-5 * float(want.abs().max()))
+
+
+def test_one_large_value():
+    """Wherever it lies: a value left out of the maximum would make a or b infinite (64 work-groups take 524288 values a round)."""
+    lib()
+    c, n = 64, 740
+    gen = torch.Generator().manual_seed(8915)
+    m = of3pair.TriangleMultiplicationOutgoing(c, c)
+    m.load_state_dict(orc.make_trimul_params(gen, c, c), strict=True)
+    m = m.to(DEV).eval()
+    z = orc.make_pair_input(8916, (1,), n, c).to(DEV)
+    for at in (0, 3, 1023, 65535, 131072, 262143, 524287, 524288, 540000, n * n - 4, n * n - 1):
+        mask = torch.ones(1, n, n, device=DEV)
+        mask.view(-1)[at] = 1e6
+        print("large value at", at, flush=True)
+        assert m(z, mask).isfinite().all() and m(z, mask.transpose(-1, -2)).isfinite().all()
 
 
 def test_value_that_is_no_number():
