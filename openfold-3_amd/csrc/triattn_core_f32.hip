@@ -50,8 +50,7 @@ template <int STEPS>
 struct CoreH2 {
   static constexpr int kKv = 2 * STEPS * 64;    // K (steps x terms), and as many of V^T (two steps x terms, or x 1 at width 16)
   static constexpr int kStages = STEPS == 2 ? 1 : 2;  // of K and V^T
-  static constexpr int kSlots = 2 * kTb + kRows * kStages * 2 * kKv;
-  static constexpr size_t kLds = kSlots * 16 + 2 * kRows * sizeof(uint32_t);  // and a vote for each wave
+  static constexpr size_t kLds = (size_t)(2 * kTb + kRows * kStages * 2 * kKv) * 16;
 };
 
 template <int STEPS>
@@ -291,23 +290,6 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
     if (!kTrack && !kLevel) fresh = false;
   };
 
-  auto any_wave = [&](bool bad) {  // the same answer in every wave; nobody reads a buffer of the tiles before it any more
-    uint32_t* votes = reinterpret_cast<uint32_t*>(lds4 + L::kSlots);
-    __syncthreads();
-    const uint32_t wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
-    if (lane == 0) votes[wave] = wave_bad;
-    __syncthreads();
-    uint32_t any = 0;
-#pragma unroll
-    for (int w = 0; w < 2 * kRows; ++w) any |= votes[w];
-    return __builtin_amdgcn_readfirstlane(any) != 0;
-  };
-  auto any_uneven = [&]() {
-    bool bad = false;
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) bad |= row_valid && q0 + 32 * qt + l32 < N && uneven[qt] != 0;
-    return any_wave(bad);
-  };
   float mv_next;
   auto first_loads = [&]() {
     mv_next = load_mask(0);
@@ -343,15 +325,9 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
       tile(kind, buf, mb, op, N - 32 * kt);
       compiler_fence();
     };
-    // The level pass looks whether it is of any use after 2, 8, 32 ... tiles: one that is not has then taken a small part of the second
-    // pass's time (at its end / so, q times 12, a fifth of the tokens padded, us: pair stack N = 384 951 / 925, 768 4673 / 4369, three templates of 200
-    // 925 / 899; where the logits are level no difference: 4136 / 4135, 850 / 849)
-    for (int kt = 0, stop = kLevel ? 2 : nkt;; stop *= 4) {
-      for (; kt < nkt && kt < stop; kt += 2) {
-        step(kt, 0);
-        if (kt + 1 < nkt) step(kt + 1, 1);
-      }
-      if (!kLevel || kt >= nkt || any_uneven()) break;
+    for (int kt = 0; kt < nkt; kt += 2) {
+      step(kt, 0);
+      if (kt + 1 < nkt) step(kt + 1, 1);
     }
     wait_vmcnt<0>();  // the loads issued past the end must not outlive the pass (or the work-group's LDS)
 #pragma unroll
@@ -375,10 +351,28 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
     level &= all || rg * kRows + r >= N;
   }
   level &= again;
-  const bool tried = level || !again;
+  auto any_wave = [&](bool bad) {  // the vote goes through the bias buffers
+    uint32_t* votes = reinterpret_cast<uint32_t*>(lds4);
+    __syncthreads();
+    const uint32_t wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+    if (lane == 0) votes[wave] = wave_bad;
+    __syncthreads();
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < 2 * kRows; ++w) any |= votes[w];
+    const bool result = __builtin_amdgcn_readfirstlane(any) != 0;
+    if (result) {
+      __syncthreads();  // every wave has read the votes before loads land on them
+      first_loads();
+    }
+    return result;
+  };
   if (level) {
     pass(std::integral_constant<int, kLevelled>{});
-    again = any_uneven();
+    bool bad = false;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) bad |= row_valid && q0 + 32 * qt + l32 < N && uneven[qt] != 0;
+    again = any_wave(bad);
   } else if (!again) {
     pass(std::integral_constant<int, kFirst>{});
     bool bad = false;
@@ -389,10 +383,7 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
     }
     again = any_wave(bad);
   }
-  if (again) {
-    if (tried) first_loads();
-    pass(std::integral_constant<int, kTracked>{});
-  }
+  if (again) pass(std::integral_constant<int, kTracked>{});
 
   if (row_valid) {
 #pragma unroll

@@ -392,12 +392,6 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
     }
   };
 
-  auto any_uneven = [&]() {  // the same answer in every wave; nobody reads a buffer of the tiles before it any more
-    bool bad = false;
-#pragma unroll
-    for (int rq = 0; rq < kRQ; ++rq) bad |= row_valid && q0 + 32 * rq + l32 < N && uneven[rq] != 0;
-    return __syncthreads_or(bad) != 0;
-  };
   const uint32_t mb_off = krow * sizeof(float);
   float mb_next;
   auto first_loads = [&]() {
@@ -435,15 +429,9 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
       tile(kind, buf, mb_cur, op, N - 32 * kt);
       compiler_fence();
     };
-    // The level pass looks whether it is of any use after 2, 8, 32 ... tiles: one that is not has then taken a small part of the second
-    // pass's time (at its end / so, q times 24, a fifth of the tokens padded, us: pair stack N = 384 531 / 518, 768 2591 / 2527; where the logits are
-    // level no difference: 1842 / 1845)
-    for (int kt = 0, stop = kLevel ? 2 : nkt;; stop *= 4) {
-      for (; kt < nkt && kt < stop; kt += 2) {
-        step(kt, 0);
-        if (kt + 1 < nkt) step(kt + 1, 1);
-      }
-      if (!kLevel || kt >= nkt || any_uneven()) break;
+    for (int kt = 0; kt < nkt; kt += 2) {
+      step(kt, 0);
+      if (kt + 1 < nkt) step(kt + 1, 1);
     }
     wait_vmcnt<0>();  // the loads issued past the end must not outlive the pass (or the work-group's LDS)
 #pragma unroll
@@ -472,7 +460,8 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
   // Where all rows of a work-group look so, the pass only sees whether every logit is the mask bias itself, which takes logits of an
   // ordinary size up (128 are between it and its neighbours).  The weights then are equal and the result is the mean of v, the same
   // for every query: no exponentials, no maxima, no sums, and P V for one of the query tiles; the bits are those of the pass with
-  // running maxima, which comes after it where a logit is another.  Launches, us: N = 2048, 256 tokens padded, 6389 / 5922, 384, 38
+  // running maxima, which comes after it where a logit is another (pair stack, a fifth of the tokens padded, q times 24: 2.5 % of the
+  // pass at 384 and 768 tokens).  Launches, us: N = 2048, 256 tokens padded, 6389 / 5922, 384, 38
   // padded, 56.5 / 53.9; whole passes 24.4 / 23.4 ms, four templates of 512, 51 padded, 3558 / 3522; with 10 % of 384 or 4 % of 929
   // padded no more than two runs differ.
   // A work-group with a row whose sampled keys (its own token, the first, the middle and the last) are all masked is
@@ -493,7 +482,10 @@ __global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flas
   level &= again;
   if (level) {
     pass(std::integral_constant<int, kLevelled>{});
-    level = !any_uneven();
+    bool bad = false;
+#pragma unroll
+    for (int rq = 0; rq < kRQ; ++rq) bad |= row_valid && q0 + 32 * rq + l32 < N && uneven[rq] != 0;
+    level = !__syncthreads_or(bad);
     if (!level) first_loads();
   } else if (!again) {
     pass(std::integral_constant<int, kFirst>{});
