@@ -175,9 +175,10 @@ struct ColumnScales {
     total = s[l32 < tiles ? l32 : tiles - 1].unscale;
   }
   __device__ __forceinline__ void finish() { total = __int_as_float(wave_max(__float_as_int(total))); }  // positive: ordered as the bits
-  __device__ __forceinline__ float at(int t) const {
-    return s[t].unscale * __uint_as_float(0x7f000000u - __float_as_uint(total));  // 1 / total, a power of two
+  __device__ __forceinline__ float of(float unscale) const {  // of a tile, read before any wait: behind one it is a trip to L2 by itself
+    return unscale * __uint_as_float(0x7f000000u - __float_as_uint(total));  // 1 / total, a power of two
   }
+  __device__ __forceinline__ float at(int t) const { return of(s[t].unscale); }
 };
 
 // rows of a fp32 weight matrix as split MFMA operands: k-values 16 s + 8 lh .. + 7 of `row`

@@ -527,14 +527,12 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int N = p.N;
   const WeightScales& sg = p.s_g.scales()[wave];
-  const float g_in = sg.input, g_unscale = sg.unscale;
+  const float g_in = sg.input, g_unscale = sg.unscale, tile_unscale = p.s_o.scales()[wave].unscale;
   OutWeights<C> w;
   w.load(p.s_g, p.s_o, wave, l32, lh);
   ColumnScales so(p.s_o, NW);
   for (int c = tid; c < C; c += 64 * NW) ln[c] = p.ln_w[c] * g_in, ln[C + c] = p.ln_b[c] * g_in;
   wait_vmcnt<0>();  // the weights
-  so.finish();
-  const float o_scale = so.at(wave), unscale = so.total;
   __syncthreads();
 
   auto place = [&](int id, int& b, int& i) {  // returns the first position
@@ -581,6 +579,8 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
   int id = grid_slot();
   const int first = id;
   if (id < total) load_rows(id), load_o(id);
+  so.finish();  // beside the first tile's loads
+  const float o_scale = so.of(tile_unscale), unscale = so.total;
   for (; id < total; id += gridDim.x) {
     const int next = id + (int)gridDim.x < total ? id + (int)gridDim.x : id;
     int b, i;

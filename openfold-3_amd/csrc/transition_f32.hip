@@ -153,6 +153,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
       u32x4_t w[KS][2];
       load_unit<C, 2>(kh == 0 ? p.att_g : p.att_out, ot, src_lane, w);
       ColumnScales att_so(p.att_out, OT);
+      const float att_tile = p.att_out.scales()[ot].unscale, att_g_unscale = p.att_g.scales()[ot].unscale;
       int j0;
       const int b = row_of(tile, j0);  // one row per batch element
       const Lane here = lane_here();
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
         *reinterpret_cast<float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li) = raw[0][0].v[e];
       }
       att_so.finish();
-      const float o_scale = att_so.at(ot), att_unscale = kh == 0 ? p.att_g.scales()[ot].unscale : att_so.total;
+      const float o_scale = att_so.of(att_tile), att_unscale = kh == 0 ? att_g_unscale : att_so.total;
       __syncthreads();
       if (kh == 0) {
         const f32x16_t gate = product(xn);
