@@ -1,4 +1,4 @@
-// Tiling of the N x N positions of a batch element into 128-position tiles for the position-wise passes.
+// Tiling of the N x N positions of a batch element into tiles of TP (128, or 64) positions for the position-wise passes.
 // Plain C++ (no HIP types): the kernels and the host-side test of the scheme compile the same functions.
 #pragma once
 
@@ -10,45 +10,47 @@
 
 namespace of3 {
 
-// The whole 128-wide pieces of every row come first (full_per_row per row), then the remaining N % 128
-// columns in pieces of 2^s columns x (128 >> s) consecutive rows, 2^s >= 2^min_shift: one power of two that covers them, or two
+// The whole TP-wide pieces of every row come first (full_per_row per row), then the remaining N % TP
+// columns in pieces of 2^s columns x (TP >> s) consecutive rows, 2^s >= 2^min_shift: one power of two that covers them, or two
 // (72 columns: 64 + 8) where that makes fewer tiles.  tail_shift: s of the first piece + 256 * s of the second, 0 if there is
-// none.  N = 200 takes 313 tiles with two and 400 with one.
+// none.  N = 200 takes 313 tiles of 128 with two and 400 with one.
 struct RaggedTiles {
   int full_per_row, tail_shift, per_batch;
 };
+template <int TP = 128>
 OF3_HD inline int tiles_of_columns(int N, int shift) {  // tiles of N rows x 2^shift columns
-  const int rows = 128 >> shift;
+  const int rows = TP >> shift;
   return (N + rows - 1) / rows;
 }
+template <int TP = 128>
 inline RaggedTiles ragged_tiles(int N, int min_shift = 3) {
   RaggedTiles t;
-  t.full_per_row = N / 128;
-  const int r = N % 128;
-  t.tail_shift = r ? min_shift : 7;
+  t.full_per_row = N / TP;
+  const int r = N % TP;
+  t.tail_shift = r ? min_shift : TP == 128 ? 7 : 6;
   while ((1 << t.tail_shift) < r) ++t.tail_shift;
-  int tail = r ? tiles_of_columns(N, t.tail_shift) : 0;
+  int tail = r ? tiles_of_columns<TP>(N, t.tail_shift) : 0;
   const int s1 = t.tail_shift - 1;
   if (r && s1 >= min_shift) {
     int s2 = min_shift;
     while ((1 << s1) + (1 << s2) < r) ++s2;
-    const int two = tiles_of_columns(N, s1) + tiles_of_columns(N, s2);
+    const int two = tiles_of_columns<TP>(N, s1) + tiles_of_columns<TP>(N, s2);
     if (two < tail) tail = two, t.tail_shift = s1 + 256 * s2;
   }
   t.per_batch = N * t.full_per_row + tail;
   return t;
 }
 
-// Where a tile lies: batch element, first row, first column, log2 of its width.  Position pos (0..127) of
+// Where a tile lies: batch element, first row, first column, log2 of its width.  Position pos (0..TP - 1) of
 // the tile is row i0 + (pos >> shift), column j0 + (pos & ((1 << shift) - 1)).
 struct TilePlace {
   int b, i0, j0, shift;
 };
 // RAGGED = false: whole-row pieces only (full_per_row pieces per row, per_batch = rows * full_per_row).
 // keep_rows_inside: the last piece of some ragged columns is moved up so that it ends at row N - 1 (its rows
-// all exist, some of them belong to the piece before it as well; needs N >= 128 >> tail_shift); otherwise it
+// all exist, some of them belong to the piece before it as well; needs N >= TP >> tail_shift); otherwise it
 // runs past the last row and the caller leaves those positions out.
-template <bool RAGGED>
+template <bool RAGGED, int TP = 128>
 OF3_HD inline TilePlace tile_place(int tile_id, int N, int full_per_row, int tail_shift, int per_batch,
                                    bool keep_rows_inside) {
   TilePlace t;
@@ -57,36 +59,37 @@ OF3_HD inline TilePlace tile_place(int tile_id, int N, int full_per_row, int tai
   const int main_tiles = N * full_per_row;
   if (!RAGGED || rem < main_tiles) {
     t.i0 = rem / full_per_row;
-    t.j0 = (rem - t.i0 * full_per_row) * 128;
-    t.shift = 7;
+    t.j0 = (rem - t.i0 * full_per_row) * TP;
+    t.shift = TP == 128 ? 7 : 6;
   } else {
     int at = rem - main_tiles;
     t.shift = tail_shift & 255;
-    t.j0 = full_per_row * 128;
-    const int first = tiles_of_columns(N, t.shift);
+    t.j0 = full_per_row * TP;
+    const int first = tiles_of_columns<TP>(N, t.shift);
     if (at >= first) {
       at -= first;
       t.j0 += 1 << t.shift;
       t.shift = tail_shift >> 8;
     }
-    const int rows = 128 >> t.shift;
+    const int rows = TP >> t.shift;
     t.i0 = at * rows;
     if (keep_rows_inside && t.i0 + rows > N) t.i0 = N - rows;
   }
   return t;
 }
 
-// ---- tiles of 128 consecutive positions of the flattened [B][N][N] index space (triattn_out) -----------
-// A tile starts at position p0 = 128 * tile_id = (b0, i0, j0).  MODE 0: N is a multiple of 128, a tile lies
-// inside one row; 1: N >= 128, at most two rows, whose element offsets in the strided view are row0 and row1;
+// ---- tiles of TP consecutive positions of the flattened [B][N][N] index space (triattn_out) ------------
+// A tile starts at position p0 = TP * tile_id = (b0, i0, j0).  MODE 0: N is a multiple of TP, a tile lies
+// inside one row; 1: N >= TP, at most two rows, whose element offsets in the strided view are row0 and row1;
 // 2: any N, the general walk.
 struct FlatTile {
   int b0, i0, j0;
   long long row0, row1;
 };
+template <int TP = 128>
 OF3_HD inline FlatTile flat_tile(int tile_id, int N, long long stride_b, long long stride_r) {
   FlatTile t;
-  const unsigned p0 = (unsigned)tile_id * 128u, nn = (unsigned)N * (unsigned)N;
+  const unsigned p0 = (unsigned)tile_id * (unsigned)TP, nn = (unsigned)N * (unsigned)N;
   t.b0 = (int)(p0 / nn);
   const unsigned rem = p0 - (unsigned)t.b0 * nn;
   t.i0 = (int)(rem / (unsigned)N);
@@ -96,7 +99,7 @@ OF3_HD inline FlatTile flat_tile(int tile_id, int N, long long stride_b, long lo
   t.row1 = (t.b0 + (last ? 1 : 0)) * stride_b + (last ? 0 : t.i0 + 1) * stride_r;
   return t;
 }
-// element offset of position d (0..127) of the tile in the view; the position must exist
+// element offset of position d (0..TP - 1) of the tile in the view; the position must exist
 template <int MODE>
 OF3_HD inline long long flat_offset(const FlatTile& t, int d, int N, long long stride_b, long long stride_r,
                                     long long stride_k) {
@@ -109,15 +112,15 @@ OF3_HD inline long long flat_offset(const FlatTile& t, int d, int N, long long s
     return (wrapped ? t.row1 : t.row0) + j * stride_k;
   } else {
     int b = t.b0, i = t.i0;
-    while (j >= N) j -= N, ++i;  // at most once when N >= 128
+    while (j >= N) j -= N, ++i;  // at most once when N >= TP
     while (i >= N) i -= N, ++b;
     return b * stride_b + i * stride_r + j * stride_k;
   }
 }
 
 // ---- the last round of a persistent pass ----------------------------------------------------------------
-// `tiles` tiles of 128 positions on `grid` work-groups: the tiles that are left for a last round of their own, if
-// there are no more than half (a quarter) as many as work-groups, go in two (four) pieces of 64 (32) positions each, one
+// `tiles` tiles of TP = 128 positions on `grid` work-groups: the tiles that are left for a last round of their own, if
+// there are no more than half (a quarter) as many as work-groups, go in two (four) pieces of 64 (32) positions each (tiles of 64 in halves only), one
 // piece per work-group: that round then takes as long as its piece, not as a tile.  Items 0 .. whole - 1 are
 // whole tiles, the rest pieces; whole is a multiple of grid where there are pieces.  256 CUs, 128 channels, us per pass, whole
 // tiles / pieces: triangle multiplication in at N = 128 (half a round) 11.2 / 9.0, at 200 (1.37 rounds) 15.8 / 14.5, attention in
@@ -126,26 +129,40 @@ OF3_HD inline long long flat_offset(const FlatTile& t, int d, int N, long long s
 struct LastRound {
   int whole, items, piece;
 };
+template <int TP = 128>
 inline LastRound last_round(long tiles, int grid) {
   const int left = (int)(tiles % grid);
-  LastRound r = {(int)tiles, (int)tiles, 128};
+  LastRound r = {(int)tiles, (int)tiles, TP};
   if (left == 0 || 2 * left > grid || tiles >= 3L * grid) return r;
-  const int split = 4 * left <= grid ? 4 : 2;
-  r.piece = 128 / split;
+  const int split = TP == 128 && 4 * left <= grid ? 4 : 2;
+  r.piece = TP / split;
   r.whole = (int)(tiles - left);
   r.items = r.whole + split * left;
   return r;
 }
 
+// Positions of a tile of the triangle multiplication's output pass (planes: it reads x, channel by channel) and of the attention's: tiles of
+// 64 on work-groups of four waves, or of 128 on eight.  A wave does the same either way; where the smaller work-groups share a CU (two at
+// 128 channels, three at 64 in the multiplication's pass) their barriers, three a tile, do not coincide.  128 / 64 positions, us a launch of
+// the multiplication's pass at 128 channels: N = 300 24.7 / 22.9, 384 35.0 / 32.0, 451 52.8 / 47.8, 768 118 / 116, 850 157 / 148, 1100 236 / 226, 1700
+// 546 / 536; at 64, three templates of 300 30.8 / 25.8, four of 512 95.0 / 86.9.  Of the attention's at 128: N = 300 21.5 / 21.4, 384 31.9 /
+// 28.5, 640 79.8 / 75.1, 896 148 / 143, 1280 275 / 269, and at 64, where two work-groups of eight waves share a CU, 42.4 / 42.7 for two of 512.
+// Beyond 1536 tokens they lose (attention 1536 401 / 402, 1792 528 / 546, 2048 708 / 742: more rows open in memory at once), and so does x at whole
+// multiples of 1024, where the 128-byte pieces of a tile's planes are a power of two apart (929 170 / 173, 1024 203 / 211, 2048 779 / 814).
+inline int out_tile_positions(int C, int N, bool planes) {
+  if (N > 1536 || (C == 64 && !planes)) return 128;
+  return planes && (N + 127) / 128 % 8 == 0 ? 128 : 64;
+}
+
 // Item of a persistent pass -> its tile, its first position in it, how many positions it has (group_bits: log2 of the
-// groups of eight).  PART: positions per piece, 128: no pieces.
+// groups of eight).  PART: positions per piece, TP: no pieces.
 struct TilePiece {
   int tile, first, count, group_bits;
 };
-template <int PART>
+template <int PART, int TP = 128>
 OF3_HD inline TilePiece tile_piece(int item, int whole) {
-  if (PART == 128 || item < whole) return {item, 0, 128, 4};
-  const int split = 128 / PART, left = item - whole;
+  if (PART == TP || item < whole) return {item, 0, TP, TP == 128 ? 4 : 3};
+  const int split = TP / PART, left = item - whole;
   return {whole + left / split, left % split * PART, PART, PART == 64 ? 3 : 2};
 }
 

@@ -5,9 +5,9 @@
 // through the PairView (transposed for the ending node).  The gate is recomputed from x
 // rather than stored by the input pass (one z-sized write and read less).
 //
-// HBM bound: reads o and x once, writes out once.  Two MFMA passes per 128-position tile:
+// HBM bound: reads o and x once, writes out once.  Two MFMA passes per tile of 128 or 64 positions:
 // gate tile -> multiplied into the o tile in LDS in place -> output projection.
-// A tile is 128 consecutive positions of the flattened [B][N][N] index space of the module frame, so it
+// A tile is consecutive positions of the flattened [B][N][N] index space of the module frame, so it
 // may run over the end of a row (or of a batch element): a token count off the multiples of 128 costs
 // no partly filled tile per row, only one at the very end.
 #include "of3_device.h"
@@ -21,15 +21,15 @@ namespace of3 {
 
 namespace {
 
-// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only
-template <int C, int HD, int MODE, int PART>
-__global__ __launch_bounds__(512, C == 64 ? 4 : 2) void triattn_out_kernel(TriattnOutArgs p, uint32_t total_pos, int whole_tiles, int total_items) {
+// TP: positions of a tile (out_tile_positions in of3_tiles.h); PART: of the pieces that the tiles of the last round are dealt in (last_round), TP:
+// whole tiles only
+template <int C, int HD, int MODE, int PART, int TP>
+__global__ __launch_bounds__(4 * TP, C == 64 ? 4 : 2) void triattn_out_kernel(TriattnOutArgs p, uint32_t total_pos, int whole_tiles, int total_items) {
   static_assert(C == HD, "o tile shares the x tile geometry");
   constexpr int NCH = C / 8;
   constexpr int LPP = NCH;
   constexpr int PPI = 64 / LPP;
-  constexpr int TP = 128;
-  constexpr int NW = 8;                  // waves per work-group (two per SIMD)
+  constexpr int NW = TP / 16;            // waves per work-group
   constexpr int LN_ITERS = (TP / NW) / PPI;
   constexpr int KS = C / 16;
   constexpr int NOT = C / 32;
@@ -61,11 +61,11 @@ __global__ __launch_bounds__(512, C == 64 ? 4 : 2) void triattn_out_kernel(Triat
   }
 
   const int N = p.N;
-  // A tile starts at position p0 = (b0, i0, j0) (wave-uniform: scalar divisions); with N >= 128 it holds
+  // A tile starts at position p0 = (b0, i0, j0) (wave-uniform: scalar divisions); with N >= TP it holds
   // positions of at most two rows, whose offsets in the view are scalars, and position d of the tile costs a
   // compare and two selects (of3_tiles.h).
   typedef FlatTile Origin;
-  auto tile_origin = [&](int tile_id) { return flat_tile(tile_id, N, p.x_view.stride_b, p.x_view.stride_r); };
+  auto tile_origin = [&](int tile_id) { return flat_tile<TP>(tile_id, N, p.x_view.stride_b, p.x_view.stride_r); };
   auto view_offset = [&](const Origin& t, int d) -> int64_t {
     return flat_offset<MODE>(t, d, N, p.x_view.stride_b, p.x_view.stride_r, p.x_view.stride_k);
   };
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(512, C == 64 ? 4 : 2) void triattn_out_kernel(Triat
   };
   u32x4_t xraw[LN_ITERS], oraw[LN_ITERS];
   auto load_tile = [&](int item) {
-    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
+    const TilePiece piece = tile_piece<PART, TP>(item, whole_tiles);
     const Origin t = tile_origin(piece.tile);
     const uint32_t p0 = (uint32_t)piece.tile * TP;
 #pragma unroll
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(512, C == 64 ? 4 : 2) void triattn_out_kernel(Triat
   auto do_tile = [&](auto positions, int item) {
     constexpr int P = decltype(positions)::value;
     constexpr int T = P / 32 >= WPG ? P / 32 / WPG : 1;  // position tiles per wave
-    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
+    const TilePiece piece = tile_piece<PART, TP>(item, whole_tiles);
     const int first = P == TP ? 0 : piece.first;
     const bool multiplies = P == TP || wave / NOT * T < P / 32;
     const Origin t = tile_origin(piece.tile);
@@ -183,21 +183,40 @@ __global__ __launch_bounds__(512, C == 64 ? 4 : 2) void triattn_out_kernel(Triat
   }
 }
 
-template <int C, int HD, int MODE>
+template <int C, int HD, int MODE, int TP>
 hipError_t launch(const TriattnOutArgs& a, hipStream_t stream) {
   static int cache[kMaxDevices];
   int grid_cap = 0;
-  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(triattn_out_kernel<C, HD, MODE, 128>, 512, dev, v); }, &grid_cap);
+  hipError_t e =
+      per_device(cache, [&](int dev, int* v) { return resident_blocks(triattn_out_kernel<C, HD, MODE, TP, TP>, 4 * TP, dev, v); }, &grid_cap);
   if (e != hipSuccess) return e;
   const long positions = (long)a.B * a.N * a.N;
   if (positions <= 0 || positions > 0x7fffffffL) return hipErrorInvalidValue;
-  const LastRound r = last_round((positions + 127) / 128, grid_cap);
+  const int tiles = (int)((positions + TP - 1) / TP);
+  constexpr bool kManyRounds = C == 128 && TP == 128;
+  const LastRound r = kManyRounds ? LastRound{tiles, tiles, TP} : last_round<TP>(tiles, grid_cap);
   const int grid = r.items < grid_cap ? r.items : grid_cap;
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(512), 0, stream, a, (uint32_t)positions, r.whole, r.items); };
-  if (r.piece == 32) go(triattn_out_kernel<C, HD, MODE, 32>);
-  else if (r.piece == 64) go(triattn_out_kernel<C, HD, MODE, 64>);
-  else go(triattn_out_kernel<C, HD, MODE, 128>);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(4 * TP), 0, stream, a, (uint32_t)positions, r.whole, r.items); };
+  if constexpr (!kManyRounds) {
+    if (r.piece == 32) {
+      go(triattn_out_kernel<C, HD, MODE, 32, TP>);
+      return hipGetLastError();
+    }
+    if (r.piece != TP) {
+      go(triattn_out_kernel<C, HD, MODE, 64, TP>);
+      return hipGetLastError();
+    }
+  }
+  go(triattn_out_kernel<C, HD, MODE, TP, TP>);
   return hipGetLastError();
+}
+// a tile lies in one row (N a multiple of its positions), in at most two (N no less), or anywhere
+template <int C, int TP>
+hipError_t launch_tiles(const TriattnOutArgs& a, hipStream_t stream) {
+  if (a.N % TP == 0) return launch<C, C, 0, TP>(a, stream);
+  if (a.N >= TP) return launch<C, C, 1, TP>(a, stream);
+  if constexpr (C == 64 || TP == 64) return launch<C, C, 2, TP>(a, stream);
+  return hipErrorInvalidValue;  // tiles of 128 at 128 channels are for long sequences only
 }
 
 }  // namespace
@@ -210,11 +229,8 @@ hipError_t triattn_out_launch(const TriattnOutArgs& args, int C, int HD, hipStre
   const hipError_t e = small_pass(args.B, args.N, C == 128 ? 2 : 1, &small);
   if (e != hipSuccess) return e;
   if (small) return triattn_out_panels_launch(args, C, stream);
-  // a 128-position tile lies in one row (N a multiple of 128), in at most two (N >= 128), or anywhere
-  const int mode = args.N % 128 == 0 ? 0 : (args.N >= 128 ? 1 : 2);
-  if (C == 128)
-    return mode == 0 ? launch<128, 128, 0>(args, stream) : (mode == 1 ? launch<128, 128, 1>(args, stream) : launch<128, 128, 2>(args, stream));
-  return mode == 0 ? launch<64, 64, 0>(args, stream) : (mode == 1 ? launch<64, 64, 1>(args, stream) : launch<64, 64, 2>(args, stream));
+  if (C == 64) return launch_tiles<64, 128>(args, stream);
+  return out_tile_positions(C, args.N, false) == 64 ? launch_tiles<128, 64>(args, stream) : launch_tiles<128, 128>(args, stream);
 }
 
 }  // namespace of3

@@ -8,8 +8,8 @@
 //
 // HBM bound: reads x and z once, writes out once.
 //
-// Tiles are 128 positions: the whole 128-wide pieces of every row first, then, when N is not a multiple
-// of 128, the remaining columns in pieces of 2^s columns x 128 / 2^s consecutive rows (2^s the smallest
+// Tiles are TP = 128 or 64 positions: the whole TP-wide pieces of every row first, then, when N is not a multiple
+// of TP, the remaining columns in pieces of 2^s columns x TP / 2^s consecutive rows (2^s the smallest
 // power of two >= 8 that covers them), so that the ragged end of the rows costs a few tiles per batch
 // element rather than one more tile per row.
 #include "of3_device.h"
@@ -23,22 +23,23 @@ namespace of3 {
 
 namespace {
 
-// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only
-template <int C, int CH, bool RAGGED, int PART>
-__global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int full_per_row, int tail_shift, int tiles_per_batch,
+// TP: positions of a tile (out_tile_positions in of3_tiles.h); PART: of the pieces that the tiles of the last round are dealt in (last_round), TP:
+// whole tiles only
+template <int C, int CH, bool RAGGED, int PART, int TP>
+__global__ __launch_bounds__(4 * TP, C == 64 && TP == 64 ? 3 : 2) void trimul_out_kernel(TrimulOutArgs p, int full_per_row, int tail_shift, int tiles_per_batch,
                                                            int whole_tiles, int total_items) {
   static_assert(C == CH, "position-major x tile shares the z tile geometry");
   constexpr int NCH = C / 8;
   constexpr int LPP = NCH;
   constexpr int PPI = 64 / LPP;
-  constexpr int TP = 128;
-  constexpr int NW = 8;                  // waves per work-group (two per SIMD)
+  constexpr int WHOLE = TP == 128 ? 7 : 6;  // log2 of its width where it lies in one row
+  constexpr int NW = TP / 16, NTH = 64 * NW;  // waves and threads per work-group
   constexpr int LN_ITERS = (TP / NW) / PPI;
   constexpr int KS = C / 16;
   constexpr int NOT = C / 32;            // output-channel tiles
   constexpr int WPG = NW / NOT;          // waves sharing one output tile (2 or 4)
   constexpr int LN_STEP = NW * PPI;      // positions that the waves normalise at a time, PPI consecutive ones each
-  constexpr int XROUNDS = (CH / 2) * 16 / 512;  // (channel pair, 8-position group) items per thread
+  constexpr int XROUNDS = (CH / 2) * (TP / 8) / NTH;  // (channel pair, 8-position group) items per thread
 
   __shared__ u32x4_t ztile[TP * NCH];
   __shared__ u32x4_t xtile[TP * NCH];
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
   // tile -> batch element, first row, first column, log2 of its width (all wave-uniform); the last ragged
   // piece may run past the last row: those positions are left out below
   auto tile_origin = [&](int tile_id, int& b, int& i0, int& j0, int& shift) {
-    const TilePlace t = tile_place<RAGGED>(tile_id, N, full_per_row, tail_shift, tiles_per_batch, false);
+    const TilePlace t = tile_place<RAGGED, TP>(tile_id, N, full_per_row, tail_shift, tiles_per_batch, false);
     b = t.b, i0 = t.i0, j0 = t.j0, shift = t.shift;
   };
   // LayerNorm-phase position `it` of this lane, from the item's first one: TP / NW consecutive positions per wave in whole
@@ -87,10 +88,10 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
   u32x4_t zraw[LN_ITERS];
   u32x4_t xa[XROUNDS], xb[XROUNDS];
   auto load_tile = [&](int item) {
-    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
+    const TilePiece piece = tile_piece<PART, TP>(item, whole_tiles);
     int b, i0, j0, shift_rt;
     tile_origin(piece.tile, b, i0, j0, shift_rt);
-    const int shift = RAGGED ? shift_rt : 7;  // a constant without ragged pieces: di below folds to 0
+    const int shift = RAGGED ? shift_rt : WHOLE;  // a constant without ragged pieces: di below folds to 0
     const int jmask = (1 << shift) - 1;
     const bf16_t* zrow = p.z + b * p.z_view.stride_b + i0 * p.z_view.stride_r;  // the tile's first row (scalar)
 #pragma unroll
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
     }
 #pragma unroll
     for (int rr = 0; rr < XROUNDS; ++rr) {
-      const int item = rr * 512 + tid;
+      const int item = rr * NTH + tid;
       // channels 2cp, 2cp+1; positions 8pg..8pg+7: one row, as the width is >= 8
       const int cp = item >> piece.group_bits, pg = (piece.first >> 3) + (item & ((1 << piece.group_bits) - 1));
       if (PART < TP && cp >= CH / 2) break;
@@ -119,22 +120,22 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
 
   auto do_tile = [&](auto positions, int item) {
     constexpr int P = decltype(positions)::value;
-    constexpr int GROUPS = P / 8, XR = (CH / 2) * GROUPS > 512 ? (CH / 2) * GROUPS / 512 : 1;
+    constexpr int GROUPS = P / 8, XR = (CH / 2) * GROUPS > NTH ? (CH / 2) * GROUPS / NTH : 1;
     constexpr int T = P / 32 >= WPG ? P / 32 / WPG : 1;  // position tiles per wave
-    const TilePiece piece = tile_piece<PART>(item, whole_tiles);
+    const TilePiece piece = tile_piece<PART, TP>(item, whole_tiles);
     const int first = P == TP ? 0 : piece.first;
     int b, i0, j0, shift_rt;
     tile_origin(piece.tile, b, i0, j0, shift_rt);
-    const int shift = RAGGED ? shift_rt : 7;
+    const int shift = RAGGED ? shift_rt : WHOLE;
     const int jmask = (1 << shift) - 1;
     bf16_t* orow0 = p.out + b * p.z_view.stride_b + i0 * p.z_view.stride_r;  // the tile's first row (scalar)
 
     // x: transpose into xtile[pos][c] with 4-byte (channel pair) writes
 #pragma unroll
     for (int rr = 0; rr < XR; ++rr) {
-      const int item = rr * 512 + tid;
+      const int item = rr * NTH + tid;
       const int cp = item / GROUPS, pg = (first >> 3) + item % GROUPS;
-      if ((CH / 2) * GROUPS < 512 && cp >= CH / 2) break;
+      if ((CH / 2) * GROUPS < NTH && cp >= CH / 2) break;
       const int chunk = (2 * cp) >> 3, within = (2 * cp) & 7;  // `within` is even
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -216,24 +217,29 @@ __global__ __launch_bounds__(512) void trimul_out_kernel(TrimulOutArgs p, int fu
   }
 }
 
-template <int C, int CH, bool RAGGED>
+template <int C, int CH, bool RAGGED, int TP>
 hipError_t launch(const TrimulOutArgs& a, hipStream_t stream) {
   static int cache[kMaxDevices];
   int grid_cap = 0;
-  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(trimul_out_kernel<C, CH, RAGGED, 128>, 512, dev, v); }, &grid_cap);
+  hipError_t e =
+      per_device(cache, [&](int dev, int* v) { return resident_blocks(trimul_out_kernel<C, CH, RAGGED, TP, TP>, 4 * TP, dev, v); }, &grid_cap);
   if (e != hipSuccess) return e;
-  const RaggedTiles t = ragged_tiles(a.N);
+  const RaggedTiles t = ragged_tiles<TP>(a.N);
   const long total = (long)a.B * t.per_batch;
   if (total > 0x7fffffffL) return hipErrorInvalidValue;
-  const LastRound r = last_round(total, grid_cap);
+  LastRound r = {(int)total, (int)total, TP};
+  if (TP == 64) r = last_round<TP>(total, grid_cap);  // tiles of 128: dozens of rounds
   const int grid = r.items < grid_cap ? r.items : grid_cap;
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), 0, stream, a, t.full_per_row, t.tail_shift, t.per_batch, r.whole, r.items);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(4 * TP), 0, stream, a, t.full_per_row, t.tail_shift, t.per_batch, r.whole, r.items);
   };
-  if (r.piece == 32) go(trimul_out_kernel<C, CH, RAGGED, 32>);
-  else if (r.piece == 64) go(trimul_out_kernel<C, CH, RAGGED, 64>);
-  else go(trimul_out_kernel<C, CH, RAGGED, 128>);
+  if (r.piece == TP) go(trimul_out_kernel<C, CH, RAGGED, TP, TP>);
+  else if constexpr (TP == 64) go(trimul_out_kernel<C, CH, RAGGED, 32, TP>);
   return hipGetLastError();
+}
+template <int C, int TP>
+hipError_t launch_tiles(const TrimulOutArgs& a, hipStream_t stream) {
+  return a.N % TP != 0 ? launch<C, C, true, TP>(a, stream) : launch<C, C, false, TP>(a, stream);
 }
 
 }  // namespace
@@ -247,9 +253,9 @@ hipError_t trimul_out_launch(const TrimulOutArgs& args, int C, int CH, hipStream
   const hipError_t e = small_pass(args.B, args.N, C == 128 ? 2 : 1, &small);
   if (e != hipSuccess) return e;
   if (small) return trimul_out_panels_launch(args, C, stream);
-  const bool ragged = args.N % 128 != 0;
-  if (C == 128) return ragged ? launch<128, 128, true>(args, stream) : launch<128, 128, false>(args, stream);
-  return ragged ? launch<64, 64, true>(args, stream) : launch<64, 64, false>(args, stream);
+  const bool half = out_tile_positions(C, args.N, true) == 64;
+  if (C == 128) return half ? launch_tiles<128, 64>(args, stream) : launch_tiles<128, 128>(args, stream);
+  return half ? launch_tiles<64, 64>(args, stream) : launch_tiles<64, 128>(args, stream);
 }
 
 }  // namespace of3
