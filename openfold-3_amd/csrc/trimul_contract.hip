@@ -648,7 +648,7 @@ __global__ __launch_bounds__(256) void contract_short_kernel(const bf16_t* __res
   const bool busy = m0 + wm0 < Nr && n0 + wn0 < Nr;
   const int ahead = nk < kShortRing - 1 ? nk : kShortRing - 1;
   for (int q = 0; q < ahead; ++q) issue(q);
-  for (int p = 0; p < nk; ++p) {
+  auto panel_ready = [&](int p) {
     const int newer = nk - 1 - p;  // panels requested after this one: up to two, two loads each
     if (newer >= 2) wait_vmcnt<4>();
     else if (newer == 1) wait_vmcnt<2>();
@@ -656,12 +656,21 @@ __global__ __launch_bounds__(256) void contract_short_kernel(const bf16_t* __res
     wait_lds_reads();  // of the panel before
     __builtin_amdgcn_s_barrier();
     compiler_fence();
-    const u32x4_t* st = lds + p % kShortRing * (2 * kShortSide);
     if (p + 3 < nk) issue((p + 3) % kShortRing);
-    if (!busy) continue;
-    const u32x4_t a0 = st[m_slot], b0 = st[n_slot], a1 = st[m_slot ^ 2], b1 = st[n_slot ^ 2];
-    acc = mfma_32x32x16(a0, b0, acc);
-    acc = mfma_32x32x16(a1, b1, acc);
+  };
+  // A loop of its own for the waves that lie past the last row or column: with the products under a condition inside one loop the
+  // accumulator was copied from one register file to the other and back for every panel, 32 instructions beside two products (N = 200
+  // 13.3 / 11.9 us a launch, two templates of 187 10.2 / 8.9)
+  if (busy) {
+    for (int p = 0; p < nk; ++p) {
+      panel_ready(p);
+      const u32x4_t* st = lds + p % kShortRing * (2 * kShortSide);
+      const u32x4_t a0 = st[m_slot], b0 = st[n_slot], a1 = st[m_slot ^ 2], b1 = st[n_slot ^ 2];
+      acc = mfma_32x32x16(a0, b0, acc);
+      acc = mfma_32x32x16(a1, b1, acc);
+    }
+  } else {
+    for (int p = 0; p < nk; ++p) panel_ready(p);
   }
   wait_lds_reads();
   __builtin_amdgcn_s_barrier();  // everybody has read the last panel
