@@ -593,33 +593,40 @@ hipError_t launch_contract8(const bf16_t* a, const bf16_t* b, bf16_t* x, int pla
 
 // ---- up to 256 tokens -------------------------------------------------------------------------------------
 // A round or two of work-groups, so what bounds it is one work-group's chain: first panel from L2, products, stores.  Tiles of
-// 64 x 64 of one plane, four waves of 32 x 32 each, five work-groups to a CU: one's stores run beside another's loads.  A ring of
-// four panels (32 KB of LDS), three of them requested ahead, one barrier per panel: behind it everybody has read the panel
+// 64 x TN of one plane, four waves, several work-groups to a CU: one's stores run beside another's loads.  A ring of
+// panels, all but one of them requested ahead, one barrier per panel: behind it everybody has read the panel
 // before, whose place the next request takes.
 // `pm` holds the operand along the rows of the output in memory, `pn` the other: x[n][m] = sum_k pm[m][k] pn[n][k], so
 // the transposed planes, for a reader that walks columns (pair_join_bf16.hip), are the operands' roles exchanged (M_IS_I).  The
 // panels are visited in the order of contract_kernel's tiles (its sums, bit for bit).
-// Whole passes, us, with contract_kernel / this: pair stack 60 tokens 62 / 56, 110 91 / 87; pairformer, 4 blocks, 40 364 / 343, 85 434 / 412,
+// Whole passes, us, with contract_kernel / this on tiles of 64 x 64 with a ring of four: pair stack 60 tokens 62 / 56, 110 91 / 87; pairformer, 4 blocks, 40 364 / 343, 85 434 / 412,
 // 150 646 / 626, 190 780 / 754, 225 1019 / 1011; templates 4 x 60 154 / 150, 4 x 120 257 / 248, 3 x 187 406 / 389.  With tiles of 128:
 // 59, 90, 394, 426, 637, 773, 1023, 153, 252, 407.
-constexpr int kShortTile = 64, kShortRing = 4;
-constexpr int kShortSide = kShortTile * 4;  // u32x4 slots of one side of a panel
-constexpr size_t kShortLds = (size_t)kShortRing * 2 * kShortSide * 16;
+// A ring of three panels, so that six work-groups fit a CU, and from 193 tokens on tiles of 64 x 128, two of 32 x 32 to a wave (three
+// quarters of the bytes through the CU's L1, and 1024 work-groups for 128 planes, all of them at once): us a launch, tiles of 64 x 64 with four
+// panels / with three / 64 x 128: N = 200 11.7 / 11.3 / 10.5, 170 8.9 / 8.2 / 8.3, two templates of 187 8.9 / 8.4 / 8.3, 128 5.1 / 5.1 / 5.4.
+constexpr int kShortM = 64, kShortRing = 3;
+constexpr int kShortSide = kShortM * 4;  // u32x4 slots of the m side of a panel
+constexpr int short_panel(int tn) { return (kShortM + tn) * 4; }
+constexpr size_t short_lds(int tn) { return (size_t)kShortRing * short_panel(tn) * 16; }
+inline int short_tile_n(int nk) { return nk > 6 ? 128 : 64; }
 
-template <bool M_IS_I>
+template <bool M_IS_I, int TN>
 __global__ __launch_bounds__(256) void contract_short_kernel(const bf16_t* __restrict__ pm, const bf16_t* __restrict__ pn,
                                                              bf16_t* __restrict__ x, int Np, int nk, int bn_order, int tiles, int total,
                                                              int per_xcd) {
+  constexpr int NT = TN / 64, PANEL = short_panel(TN);
   extern __shared__ u32x4_t lds[];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int logical = xcd_logical_block(blockIdx.x, per_xcd);
   if (logical >= total) return;  // the whole work-group leaves together
-  const int plane = logical / (tiles * tiles), rem = logical - plane * (tiles * tiles);
+  const int Nr = 32 * nk, tiles_n = (Nr + TN - 1) / TN;
+  const int plane = logical / (tiles * tiles_n), rem = logical - plane * (tiles * tiles_n);
   const int tn = rem / tiles, tm = rem - tn * tiles;
-  const int m0 = tm * kShortTile, n0 = tn * kShortTile, Nr = 32 * nk;
-  const int wm0 = 32 * (wave >> 1), wn0 = 32 * (wave & 1);
+  const int m0 = tm * kShortM, n0 = tn * TN;
+  const int wm0 = 32 * (wave >> 1), wn0 = 32 * NT * (wave & 1);
   const size_t plane_bytes = (size_t)plane * Np * Np * 2, panel_bytes = (size_t)Np * kBK * 2;
   // The m side's rows are read in the order 0..3, 16..19, 4..7, 20..23, ...: a lane ends with 16 consecutive m's of one n.
   // (row % 4, key) differs within each group of 16 lanes, there and in the n side's natural order.
@@ -630,33 +637,40 @@ __global__ __launch_bounds__(256) void contract_short_kernel(const bf16_t* __res
   const int rb = 16 * wave, within = lane >> 2, row = rb + within;
   const char* src_m = reinterpret_cast<const char*>(pm) + plane_bytes + (size_t)(contract_rows_first(m0, rb, Nr) + within) * 64 +
                       16 * ((lane & 3) ^ m_key(row));
-  const char* src_n = reinterpret_cast<const char*>(pn) + plane_bytes + (size_t)(contract_rows_first(n0, rb, Nr) + within) * 64 +
-                      16 * ((lane & 3) ^ n_key(row));
+  const char* src_n[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    src_n[t] = reinterpret_cast<const char*>(pn) + plane_bytes + (size_t)(contract_rows_first(n0, rb + 64 * t, Nr) + within) * 64 +
+               16 * ((lane & 3) ^ n_key(row));
   // the panel that contract_kernel begins this output with: tiles of 256 j's and bn_order i's
   int next = (M_IS_I ? m0 / bn_order + n0 / 256 : n0 / bn_order + m0 / 256) % 4 % nk;
   auto issue = [&](int buf) {
-    u32x4_t* st = lds + buf * (2 * kShortSide) + 64 * wave;
+    u32x4_t* st = lds + buf * PANEL + 64 * wave;
     const size_t at = next * panel_bytes;
     __builtin_amdgcn_global_load_lds((const void OF3_GLOBAL_AS*)(src_m + at), (void OF3_LDS_AS*)st, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((const void OF3_GLOBAL_AS*)(src_n + at), (void OF3_LDS_AS*)(st + kShortSide), 16, 0, 0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      __builtin_amdgcn_global_load_lds((const void OF3_GLOBAL_AS*)(src_n[t] + at), (void OF3_LDS_AS*)(st + kShortSide + 256 * t), 16, 0, 0);
     next = next + 1 == nk ? 0 : next + 1;
   };
 
   const int mr = wm0 + 16 * ((l32 >> 2) & 1) + 4 * (l32 >> 3) + (l32 & 3), nr = wn0 + l32;
   const int m_slot = mr * 4 + (lh ^ m_key(mr)), n_slot = kShortSide + nr * 4 + (lh ^ n_key(nr));
-  f32x16_t acc = zero16();
+  f32x16_t acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = zero16();
   const bool busy = m0 + wm0 < Nr && n0 + wn0 < Nr;
   const int ahead = nk < kShortRing - 1 ? nk : kShortRing - 1;
   for (int q = 0; q < ahead; ++q) issue(q);
   auto panel_ready = [&](int p) {
     const int newer = nk - 1 - p;  // panels requested after this one: up to two, two loads each
-    if (newer >= 2) wait_vmcnt<4>();
-    else if (newer == 1) wait_vmcnt<2>();
+    if (newer >= kShortRing - 2) wait_vmcnt<(kShortRing - 2) * (1 + NT)>();
+    else if (newer == 1) wait_vmcnt<1 + NT>();
     else wait_vmcnt<0>();
     wait_lds_reads();  // of the panel before
     __builtin_amdgcn_s_barrier();
     compiler_fence();
-    if (p + 3 < nk) issue((p + 3) % kShortRing);
+    if (p + kShortRing - 1 < nk) issue((p + kShortRing - 1) % kShortRing);
   };
   // A loop of its own for the waves that lie past the last row or column: with the products under a condition inside one loop the
   // accumulator was copied from one register file to the other and back for every panel, 32 instructions beside two products (N = 200
@@ -664,10 +678,15 @@ __global__ __launch_bounds__(256) void contract_short_kernel(const bf16_t* __res
   if (busy) {
     for (int p = 0; p < nk; ++p) {
       panel_ready(p);
-      const u32x4_t* st = lds + p % kShortRing * (2 * kShortSide);
-      const u32x4_t a0 = st[m_slot], b0 = st[n_slot], a1 = st[m_slot ^ 2], b1 = st[n_slot ^ 2];
-      acc = mfma_32x32x16(a0, b0, acc);
-      acc = mfma_32x32x16(a1, b1, acc);
+      const u32x4_t* st = lds + p % kShortRing * PANEL;
+      const u32x4_t a0 = st[m_slot], a1 = st[m_slot ^ 2];
+      u32x4_t b0[NT], b1[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) b0[t] = st[n_slot + 128 * t], b1[t] = st[(n_slot ^ 2) + 128 * t];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = mfma_32x32x16(a0, b0[t], acc[t]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = mfma_32x32x16(a1, b1[t], acc[t]);
     }
   } else {
     for (int p = 0; p < nk; ++p) panel_ready(p);
@@ -678,32 +697,35 @@ __global__ __launch_bounds__(256) void contract_short_kernel(const bf16_t* __res
 
   // through LDS, the wave's own 32 rows of four chunks, so that a store writes 64 consecutive bytes of a row
   u32x4_t* epi = lds + wave * 128;
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    u32x4_t v;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = pack_bf16(acc[8 * hf + 2 * q], acc[8 * hf + 2 * q + 1]);
-    epi[l32 * 4 + ((2 * lh + hf) ^ (l32 & 3))] = v;
-  }
   bf16_t* xo = x + (size_t)plane * Np * Np;
 #pragma unroll
-  for (int rr = 0; rr < 2; ++rr) {
-    const int idx = 64 * rr + lane, r = idx >> 2, chunk = idx & 3;
-    const u32x4_t v = epi[r * 4 + (chunk ^ (r & 3))];
-    const int n = n0 + wn0 + r, m = m0 + wm0 + 8 * chunk;
-    if (n < Nr && m < Nr) *reinterpret_cast<u32x4_t*>(xo + (size_t)n * Np + m) = v;
+  for (int t = 0; t < NT; ++t) {
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      u32x4_t v;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = pack_bf16(acc[t][8 * hf + 2 * q], acc[t][8 * hf + 2 * q + 1]);
+      epi[l32 * 4 + ((2 * lh + hf) ^ (l32 & 3))] = v;
+    }
+#pragma unroll
+    for (int rr = 0; rr < 2; ++rr) {
+      const int idx = 64 * rr + lane, r = idx >> 2, chunk = idx & 3;
+      const u32x4_t v = epi[r * 4 + (chunk ^ (r & 3))];
+      const int n = n0 + wn0 + 32 * t + r, m = m0 + wm0 + 8 * chunk;
+      if (n < Nr && m < Nr) *reinterpret_cast<u32x4_t*>(xo + (size_t)n * Np + m) = v;
+    }
   }
 }
 
+template <int TN>
 hipError_t launch_contract_short(const bf16_t* a, const bf16_t* b, bf16_t* x, int planes, int Np, int nk, int bn_order, bool transposed,
                                  hipStream_t stream) {
-  const int tiles = (32 * nk + kShortTile - 1) / kShortTile, total = planes * tiles * tiles, per_xcd = (total + 7) / 8;
-  if (transposed)
-    hipLaunchKernelGGL(contract_short_kernel<true>, dim3(per_xcd * 8), dim3(256), kShortLds, stream, a, b, x, Np, nk, bn_order, tiles,
-                       total, per_xcd);
-  else
-    hipLaunchKernelGGL(contract_short_kernel<false>, dim3(per_xcd * 8), dim3(256), kShortLds, stream, b, a, x, Np, nk, bn_order, tiles,
-                       total, per_xcd);
+  const int tiles = (32 * nk + kShortM - 1) / kShortM, total = planes * tiles * ((32 * nk + TN - 1) / TN), per_xcd = (total + 7) / 8;
+  auto go = [&](auto kern, const bf16_t* pm, const bf16_t* pn) {
+    hipLaunchKernelGGL(kern, dim3(per_xcd * 8), dim3(256), short_lds(TN), stream, pm, pn, x, Np, nk, bn_order, tiles, total, per_xcd);
+  };
+  if (transposed) go(contract_short_kernel<true, TN>, a, b);
+  else go(contract_short_kernel<false, TN>, b, a);
   return hipGetLastError();
 }
 
@@ -719,8 +741,11 @@ hipError_t trimul_contract_launch(const bf16_t* a, const bf16_t* b, bf16_t* x, i
     if (e != hipSuccess) return e;
     // Above 192 tokens only while the 256-wide tiles are one round: 4 blocks at 225 / 256 tokens, 128 planes, 1019 / 1049 us with those,
     // 1011 / 1044 with these; 256 planes, 4 x 256 templates, 747 and 762.
-    if (transposed || nk <= 6 || 2l * planes <= cus)
-      return launch_contract_short(a, b, x, planes, Np, nk, variant == 2 ? 128 : 256, transposed, stream);
+    if (transposed || nk <= 6 || 2l * planes <= cus) {
+      const int order = variant == 2 ? 128 : 256;
+      return short_tile_n(nk) == 128 ? launch_contract_short<128>(a, b, x, planes, Np, nk, order, transposed, stream)
+                                     : launch_contract_short<64>(a, b, x, planes, Np, nk, order, transposed, stream);
+    }
   }
   if (transposed) return hipErrorInvalidValue;  // the larger tiles have no such form
   switch (variant) {
