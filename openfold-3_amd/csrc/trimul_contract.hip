@@ -739,9 +739,9 @@ hipError_t trimul_contract_launch(const bf16_t* a, const bf16_t* b, bf16_t* x, i
     int cus = 0;
     const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
     if (e != hipSuccess) return e;
-    // Above 192 tokens only while the 256-wide tiles are one round: 4 blocks at 225 / 256 tokens, 128 planes, 1019 / 1049 us with those,
-    // 1011 / 1044 with these; 256 planes, 4 x 256 templates, 747 and 762.
-    if (transposed || nk <= 6 || 2l * planes <= cus) {
+    // Above 192 tokens while the 256-wide tiles are up to two rounds, us a launch with those / with these: 128 planes, 256 tokens 14.2 / 11.4 (these on
+    // tiles of 64 x 64: already level), 192, three templates of 230 18.9 / 15.7, 256, four of 240 20.9 / 19.9.
+    if (transposed || nk <= 6 || planes <= cus) {
       const int order = variant == 2 ? 128 : 256;
       return short_tile_n(nk) == 128 ? launch_contract_short<128>(a, b, x, planes, Np, nk, order, transposed, stream)
                                      : launch_contract_short<64>(a, b, x, planes, Np, nk, order, transposed, stream);

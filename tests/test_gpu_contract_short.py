@@ -18,11 +18,11 @@ def test_short(variant, n):
 
 @pytest.mark.parametrize("variant", [2, 3])
 @pytest.mark.parametrize("n", [193, 225, 256])
-@pytest.mark.parametrize("batch", [2, 3])
+@pytest.mark.parametrize("batch", [2, 3, 5])
 def test_many_planes(variant, n, batch):
     """Against fp32 products: one rounding to bf16 (2^-9 of the value, doubled) beside two fp32 sums of kk products in different
-    orders (each within kk 2^-24 of the sum of magnitudes, which is below kk).  192 planes take the large tiles (several of them per persistent
-    work-group) on any device of at most 383 CUs, 128 the small ones from 256 CUs on.  Panels past the end are never read (NaN)."""
+    orders (each within kk 2^-24 of the sum of magnitudes, which is below kk).  320 planes take the large tiles (several of them per persistent
+    work-group) on any device of at most 319 CUs, 128 and 192 the small ones from 256 CUs on.  Panels past the end are never read (NaN)."""
     L = lib()
     gen = torch.Generator(device="cuda").manual_seed(n + variant + batch)
     CH = 64
