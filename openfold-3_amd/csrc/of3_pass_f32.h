@@ -113,9 +113,18 @@ __device__ __forceinline__ void load_row(const float* row, int li, RowRegs<C>& r
 #pragma unroll
   for (int e = 0; e < C / 64; ++e) r.v[e] = *reinterpret_cast<const float4*>(row + 64 * e + 4 * li);
 }
-// LayerNorm of the row (two-pass statistics); ln: LDS, weights [C] then biases [C]
+// 1 / sqrt(v), v a variance plus eps: the hardware's (1 ulp) and one Newton step, in the place of a correctly rounded root and a correctly rounded
+// division, 22 instructions for every row.  Infinity gives 0, NaN NaN.  Error against float64 over 2^-17 ... 2^20,
+// rms and largest in 1e-8: 2.8 and 7.4, of the two 3.6 and 8.9.
+__device__ __forceinline__ float rsqrt_f32(float v) {
+  const float r = __builtin_amdgcn_rsqf(v);
+  const float vh = fminf(v, 3.402823466e38f) * (0.5f * r);
+  return __builtin_fmaf(r, __builtin_fmaf(-vh, r, 0.5f), r);
+}
+// LayerNorm of the row (two-pass statistics); ln: LDS, weights [C] then biases [C].  Rows past the end are some real row's or zeros: whoever sums over
+// positions leaves them out.
 template <int C>
-__device__ __forceinline__ void norm_row(const RowRegs<C>& r, bool has, const float* ln, int li, float4 (&y)[C / 64]) {
+__device__ __forceinline__ void norm_row(const RowRegs<C>& r, const float* ln, int li, float4 (&y)[C / 64]) {
   float s = 0.f;
 #pragma unroll
   for (int e = 0; e < C / 64; ++e) s += (r.v[e].x + r.v[e].y) + (r.v[e].z + r.v[e].w);
@@ -126,15 +135,15 @@ __device__ __forceinline__ void norm_row(const RowRegs<C>& r, bool has, const fl
     y[e].x = r.v[e].x - mean, y[e].y = r.v[e].y - mean, y[e].z = r.v[e].z - mean, y[e].w = r.v[e].w - mean;
     q += y[e].x * y[e].x + y[e].y * y[e].y + y[e].z * y[e].z + y[e].w * y[e].w;
   }
-  const float rstd = 1.0f / sqrtf(group_sum<16>(q) * (1.f / C) + kEps);
+  const float rstd = rsqrt_f32(group_sum<16>(q) * (1.f / C) + kEps);
 #pragma unroll
   for (int e = 0; e < C / 64; ++e) {
     const float4 w = *reinterpret_cast<const float4*>(ln + 64 * e + 4 * li);
     const float4 b = *reinterpret_cast<const float4*>(ln + C + 64 * e + 4 * li);
-    y[e].x = has ? y[e].x * rstd * w.x + b.x : 0.f;
-    y[e].y = has ? y[e].y * rstd * w.y + b.y : 0.f;
-    y[e].z = has ? y[e].z * rstd * w.z + b.z : 0.f;
-    y[e].w = has ? y[e].w * rstd * w.w + b.w : 0.f;
+    y[e].x = y[e].x * rstd * w.x + b.x;
+    y[e].y = y[e].y * rstd * w.y + b.y;
+    y[e].z = y[e].z * rstd * w.z + b.z;
+    y[e].w = y[e].w * rstd * w.w + b.w;
   }
 }
 

@@ -26,9 +26,10 @@ namespace {
 
 using namespace pass_f32;
 
-// the value of the lane with the lowest bit flipped (quad_perm [1,0,3,2])
-__device__ __forceinline__ uint32_t swap_adjacent(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);
+// the odd rows of 16 lanes of `even` change places with the even rows of `odd`
+__device__ __forceinline__ void swap_rows(uint32_t& even, uint32_t& odd) {
+  const u32x2_t r = __builtin_amdgcn_permlane16_swap(even, odd, false, false);
+  even = r[0], odd = r[1];
 }
 
 // ---- triangle multiplication, input pass: a, b = mask * sigmoid(LN(z) Wg^T) * (LN(z) Wp^T) ------------------
@@ -114,11 +115,12 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
     for (int u = 0; u < TASKS; ++u) {
       const int li = here.li, pos = 4 * (wave + NW * u) + here.lg;
       float4 y[C / 64];
-      norm_row<C>(raw[u], t.k0 + pos < N && t.r < N, ln, li, y);
+      norm_row<C>(raw[u], ln, li, y);
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) xn.store4(pos, li + 16 * e, y[e]);
     }
-    if (tid < 32) msk[32 * (n & 3) + tid] = __builtin_ldexpf(mraw, -mask_e);
+    // the panel's padding holds zeros
+    if (tid < 32) msk[32 * (n & 3) + tid] = t.k0 + tid < N ? __builtin_ldexpf(mraw, -mask_e) : 0.f;
     load_tile(id + step < total ? id + step : id);
   };
   if (first_id >= total) return;  // the whole work-group
@@ -152,8 +154,8 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
     if (t.r < N) {
       const Lane out = lane_here();
       const int l32 = out.l32, lh = out.lh;
-      const bool odd = l32 & 1;
-      const int rot0 = panel_rotation(32 * ot + (l32 & ~1), p.Np), rot1 = panel_rotation(32 * ot + (l32 | 1), p.Np);
+      const int l16 = l32 & 15;
+      const int rot0 = panel_rotation(32 * ot + l16, p.Np), rot1 = panel_rotation(32 * ot + 16 + l16, p.Np);
       u32x4_t op[2][2];
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
@@ -170,24 +172,25 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
         }
         split8h(x, op[st][0], op[st][1]);
       }
-      // The lanes of an even and an odd channel exchange a chunk, so that one store writes the 64 bytes of the even
-      // channels and the next those of the odd ones (32-byte pieces of every channel otherwise: twice the requests).
-      const size_t chan = (size_t)p.Np * p.Np, pn = (size_t)(t.k0 >> 5) * p.Np;
-      bf16_t* lp = (pair ? p.bs : p.as) + ((size_t)t.b * C + 32 * ot + (l32 & ~1)) * chan + 8 * lh + (odd ? 16 : 0);
-      bf16_t* lp0 = lp + (pn + panel_row(t.r, rot0, p.Np)) * 32;
-      bf16_t* lp1 = lp + chan + (pn + panel_row(t.r, rot1, p.Np)) * 32;
+      // Lane l32, half lh has the chunks lh and 2 + lh of channel l32.  Rows of 16 lanes exchange one, so that one store writes the 64 bytes of
+      // channels 0..15 and the next those of 16..31 (32-byte pieces of every channel otherwise: twice the requests).  Eight instructions in the place
+      // of the 32 of an exchange between neighbouring lanes, which selected by lane before and after.
 #pragma unroll
-      for (int pl = 0; pl < 2; ++pl) {
-        u32x4_t first, second;
+      for (int pl = 0; pl < 2; ++pl)
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-          const uint32_t mine = odd ? op[1][pl][w] : op[0][pl][w];
-          const uint32_t got = swap_adjacent(odd ? op[0][pl][w] : op[1][pl][w]);
-          first[w] = odd ? got : mine;
-          second[w] = odd ? mine : got;
+          uint32_t a = op[0][pl][w], b = op[1][pl][w];
+          swap_rows(a, b);
+          op[0][pl][w] = a, op[1][pl][w] = b;
         }
-        *reinterpret_cast<u32x4_t*>(lp0 + pl * p.ab_plane) = first;
-        *reinterpret_cast<u32x4_t*>(lp1 + pl * p.ab_plane) = second;
+      const size_t chan = (size_t)p.Np * p.Np, pn = (size_t)(t.k0 >> 5) * p.Np;
+      bf16_t* lp = (pair ? p.bs : p.as) + ((size_t)t.b * C + 32 * ot + l16) * chan + 8 * lh + (l32 & 16);
+      bf16_t* lp0 = lp + (pn + panel_row(t.r, rot0, p.Np)) * 32;
+      bf16_t* lp1 = lp + 16 * chan + (pn + panel_row(t.r, rot1, p.Np)) * 32;
+#pragma unroll
+      for (int pl = 0; pl < 2; ++pl) {
+        *reinterpret_cast<u32x4_t*>(lp0 + pl * p.ab_plane) = op[0][pl];
+        *reinterpret_cast<u32x4_t*>(lp1 + pl * p.ab_plane) = op[1][pl];
       }
     }
     if (n + (early ? 2 : 1) < count) normalise(n + (early ? 2 : 1));
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
     for (int u = 0; u < TASKS; ++u) {
       const int li = here.li, pos = 4 * (wave + NW * u) + here.lg;
       float4 y[C / 64];
-      norm_row<C>(zraw[u], t.j0 + pos < N, ln, li, y);
+      norm_row<C>(zraw[u], ln, li, y);
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) tile.store4(pos, li + 16 * e, y[e]);
     }
@@ -338,7 +341,7 @@ __global__ __launch_bounds__(2 * C, 2) void trimul_out_pass(TrimulF32 p, int pan
       mean *= 1.f / NG;
 #pragma unroll
       for (int g = 0; g < NG; ++g) q += red[(NG + g) * 32 + xpos] + 16.f * ((mg[g] - mean) * (mg[g] - mean));
-      const float rstd = 1.0f / sqrtf(q * (1.f / C) + kEps);
+      const float rstd = rsqrt_f32(q * (1.f / C) + kEps);
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
         const float* wv = ln + 2 * C + hf * (C / 2) + 8 * xg;
@@ -466,7 +469,7 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
       if (wave + NW * u >= 8) continue;
       const int li = here.li, pos = 4 * (wave + NW * u) + here.lg;
       float4 y[C / 64];
-      norm_row<C>(raw[u], j0 + pos < N, ln, li, y);
+      norm_row<C>(raw[u], ln, li, y);
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) xn.store4(pos, li + 16 * e, y[e]);
       float bias = 0.f;  // of head li
@@ -480,9 +483,9 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
         d = group_sum<16>(d);
         bias = li == h ? d : bias;
       }
-      if (li >= h0 && li < h1) {  // rows padded to whole panels: zero rows store zeros
+      if (li >= h0 && li < h1) {  // rows padded to whole panels with zeros
         const int b = bi / N, i = bi - b * N;
-        p.tb[(((size_t)b * H + li) * N + i) * p.Jp + j0 + pos] = bias;
+        p.tb[(((size_t)b * H + li) * N + i) * p.Jp + j0 + pos] = j0 + pos < N ? bias : 0.f;
       }
     }
     load_tile(pn + step < total ? pn + step : pn);
@@ -590,7 +593,7 @@ __global__ __launch_bounds__(2 * C, 2) void triattn_out_pass(TriattnF32 p, int p
     for (int u = 0; u < TASKS; ++u) {
       const int li = here.li, pos = 4 * (wave + NW * u) + here.lg;
       float4 y[C / 64];
-      norm_row<C>(raw[u], j0 + pos < N, ln, li, y);
+      norm_row<C>(raw[u], ln, li, y);
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) tile.store4(pos, li + 16 * e, y[e]);
     }

@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256, 3) void pair_bias_pass(PairBiasF32Args p, int 
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         float4 y[C / 64];
-        norm_row<C>(raw[u], true, ln, here.li, y);
+        norm_row<C>(raw[u], ln, here.li, y);
 #pragma unroll
         for (int e = 0; e < C / 64; ++e) tile.store4(4 * (wave + NW * u) + here.lg, here.li + 16 * e, y[e]);
       }
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(256, 3) void template_tail_pass(TemplateTailF32Args
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         float4 y[1] = {now[u].v[0]};
-        if (p.apply_ln) norm_row<C>(now[u], true, ln, here.li, y);
+        if (p.apply_ln) norm_row<C>(now[u], ln, here.li, y);
         sum[u].x += y[0].x, sum[u].y += y[0].y, sum[u].z += y[0].z, sum[u].w += y[0].w;
       }
     }

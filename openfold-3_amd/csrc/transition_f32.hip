@@ -186,7 +186,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
       };
       const int pos = 4 * wave + here.lg;
       float4 y[C / 64];
-      norm_row<C>(raw[0][0], j0 + pos < L, att_ln, here.li, y);
+      norm_row<C>(raw[0][0], att_ln, here.li, y);
 #pragma unroll
       for (int e = 0; e < C / 64; ++e) {
         xn.store4(pos, here.li + 16 * e, y[e]);
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
         for (int g = 0; g < RG; ++g) {
           const int pos = 4 * (NW * g + wave) + here.lg;
           float4 y[C / 64];
-          norm_row<C>(raw[t][g], pn < p.total && j0 + pos < L, ln, here.li, y);
+          norm_row<C>(raw[t][g], ln, here.li, y);
 #pragma unroll
           for (int e = 0; e < C / 64; ++e) xn.store4(pos, here.li + 16 * e, y[e]);
         }
@@ -446,7 +446,7 @@ __global__ __launch_bounds__(64 * NW, 2) void transition_pass(TransitionPass p) 
         float4 y[C / 64];
 #pragma unroll
         for (int e = 0; e < C / 64; ++e) raw[0][0].v[e] = *reinterpret_cast<const float4*>(rows + pos * (C + kRowLd) + 64 * e + 4 * here.li);
-        norm_row<C>(raw[0][0], true, att_ln, here.li, y);
+        norm_row<C>(raw[0][0], att_ln, here.li, y);
 #pragma unroll
         for (int e = 0; e < C / 64; ++e) xn.store4(pos, here.li + 16 * e, y[e]);
       }
