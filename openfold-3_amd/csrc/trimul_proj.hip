@@ -6,8 +6,8 @@
 // makes (r, k) = (i, k) for the outgoing update and (r, k) = (i, k) of the transposed tensor
 // for the incoming one.
 //
-// HBM bound (reads z once, writes a and b once).  Persistent work-groups of 8 waves (two
-// per SIMD, so one wave's MFMAs overlap the other's VALU work) keep the four weight
+// Persistent work-groups of 8 waves (at 64 channels also of 4), two per SIMD, so that
+// one wave's MFMAs overlap the other's VALU work, keep the four weight
 // matrices in registers as MFMA A operands, one 32-row slice pair per wave; each tile of
 // 128 positions is normalised in registers (statistics by DPP lane permutations), staged
 // once in LDS as bf16 and consumed as the MFMA B operand by all waves.  The LDS tile is
@@ -29,15 +29,17 @@ namespace of3 {
 
 namespace {
 
-// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only
-template <int C, int CH, int PART>
-__global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int panels, int whole_tiles, int total_items) {
+int panels_of(const TrimulProjArgs& a) { return (a.N + 31) / 32; }  // the panels that hold a k below N; the contraction reads no others
+
+// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only.
+// NW: waves per work-group
+template <int C, int CH, int PART, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void trimul_proj_kernel(TrimulProjArgs p, int panels, int whole_tiles, int total_items) {
   constexpr int NCH = C / 8;        // 16-byte chunks per position
   constexpr int LPP = NCH;          // lanes sharing one position in the LayerNorm phase
   constexpr int PPI = 64 / LPP;     // positions per wave instruction
   constexpr int TP = 128;           // positions per tile: TR rows x one 32-wide k-panel
   constexpr int TR = TP / 32;
-  constexpr int NW = 8;             // waves per work-group (two per SIMD)
   constexpr int LN_ITERS = (TP / NW) / PPI;
   constexpr int LN_STEP = NW * PPI; // positions that the waves normalise at a time where they share a row
   constexpr int KS = C / 16;        // MFMA k-steps
@@ -242,23 +244,19 @@ __global__ __launch_bounds__(512) void trimul_proj_kernel(TrimulProjArgs p, int 
   }
 }
 
-template <int C, int CH, int PART>
-hipError_t launch(const TrimulProjArgs& a, int panels, const LastRound& r, int grid, hipStream_t stream) {
-  hipLaunchKernelGGL((trimul_proj_kernel<C, CH, PART>), dim3(grid), dim3(512), 0, stream, a, panels, r.whole, r.items);
-  return hipGetLastError();
-}
-template <int C, int CH>
-hipError_t launch(const TrimulProjArgs& a, hipStream_t stream) {
+template <int C, int CH, int NW>
+hipError_t launch(const TrimulProjArgs& a, long tiles, hipStream_t stream) {
   static int cache[kMaxDevices];
   int grid_cap = 0;
-  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(trimul_proj_kernel<C, CH, 128>, 512, dev, v); }, &grid_cap);
+  hipError_t e = per_device(cache, [&](int dev, int* v) { return resident_blocks(trimul_proj_kernel<C, CH, 128, NW>, 64 * NW, dev, v); }, &grid_cap);
   if (e != hipSuccess) return e;
-  const int panels = (a.N + 31) / 32;  // the panels that hold a k below N; the contraction reads no others
-  const LastRound r = last_round((long)a.B * ((a.N + 3) / 4) * panels, grid_cap);
+  const LastRound r = last_round(tiles, grid_cap);
   const int grid = r.items < grid_cap ? r.items : grid_cap;
-  if (r.piece == 32) return launch<C, CH, 32>(a, panels, r, grid, stream);
-  if (r.piece == 64) return launch<C, CH, 64>(a, panels, r, grid, stream);
-  return launch<C, CH, 128>(a, panels, r, grid, stream);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), 0, stream, a, panels_of(a), r.whole, r.items); };
+  if (r.piece == 32) go(trimul_proj_kernel<C, CH, 32, NW>);
+  else if (r.piece == 64) go(trimul_proj_kernel<C, CH, 64, NW>);
+  else go(trimul_proj_kernel<C, CH, 128, NW>);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -272,8 +270,18 @@ hipError_t trimul_proj_launch(const TrimulProjArgs& args, int C, int CH, hipStre
   const hipError_t e = small_pass(args.B, args.N, 1, &small);
   if (e != hipSuccess) return e;
   if (small) return trimul_proj_panels_launch(args, C, stream);
-  if (C == 128) return launch<128, 128>(args, stream);
-  return launch<64, 64>(args, stream);
+  const long tiles = (long)args.B * ((args.N + 3) / 4) * panels_of(args);
+  if (C == 128) return launch<128, 128, 8>(args, tiles, stream);
+  // 64 channels: from more than two tiles per CU on two work-groups of four waves to a CU, whose LayerNorms and products do not coincide, in the
+  // place of one of eight in which two waves share a tile's positions.  us a launch, eight / four waves: 350 tiles (200 tokens) 9.9 / 10.4, 360 10.4 / 10.6,
+  // 564 (two templates of 187) 13.4 / 12.4, three templates of 300 31.0 / 29.2, four of 512 103.4 / 93.2; three to a CU, at 168 registers, 21 of
+  // them spilled, 122.7 for the last.  128 channels have twice the matrices: two pairs to a wave, on tiles of 64 positions, spill too and store 4 bytes a
+  // lane (N = 384 38.2 / 39.5, 768 124 / 158).
+  static int cache[kMaxDevices];
+  int cus = 0;
+  const hipError_t s = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  if (s != hipSuccess) return s;
+  return tiles > 2L * cus ? launch<64, 64, 4>(args, tiles, stream) : launch<64, 64, 8>(args, tiles, stream);
 }
 
 }  // namespace of3

@@ -13,3 +13,12 @@ def test_stages(c, d, n, batch):
     stages.test_trimul_out(1, c, n, batch)
     for starting in (False, True):
         stages.test_triattn_out(starting, 1, c, d, n, batch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,batch", [(256, 1), (257, 1), (187, 2), (200, 2), (331, 1), (63, 9)])
+def test_input_pass_64(n, batch):
+    """64 channels on both sides of two tiles per CU (256 CUs: 512 tiles at 256 tokens, 585 at 257), where work-groups of four waves take over from
+    those of eight, with pieces of both sizes in the last round and without."""
+    for incoming in (False, True):
+        stages.test_trimul_proj(incoming, 64, n, batch)
