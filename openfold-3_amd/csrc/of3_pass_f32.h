@@ -242,11 +242,19 @@ template <int C, bool W_ROWS>
 __device__ __forceinline__ f32x16_t unit_product(const HalfTile<C>& t, const u32x4_t (&w)[C / 16][2]) {
   HalfSum<C, W_ROWS> sum;
   const Lane at = lane_here();
+  u32x4_t nxt[2];
+  auto read = [&](int s) {
+    const u32x4_t* x = t.s + HalfTile<C>::slot(at.l32, 2 * s + at.lh);
+    nxt[0] = x[0], nxt[1] = x[HalfTile<C>::PLANE];
+  };
+  read(0);
 #pragma unroll
   for (int s = 0; s < C / 16; ++s) {
-    const u32x4_t* x = t.s + HalfTile<C>::slot(at.l32, 2 * s + at.lh);
-    const u32x4_t op[2] = {x[0], x[HalfTile<C>::PLANE]};
+    const u32x4_t op[2] = {nxt[0], nxt[1]};
+    if (s + 1 < C / 16) read(s + 1);
+    __builtin_amdgcn_sched_barrier(0);
     sum.step(w[s], op);
+    __builtin_amdgcn_sched_barrier(0);
   }
   return sum.total();
 }
