@@ -3,9 +3,10 @@
 // (pair_pass_f32.hip); pair_f32.hip has the cores for every other shape.
 //
 // Work-group = 4 waves = 2 consecutive rows i x 2 halves of one (head, 128-query range); a wave owns 64 queries (two
-// 32-query tiles) of one row.  Three work-groups share a CU, so that the products of one run under the exponentials and
+// 32-query tiles) of one row.  Three work-groups share a CU (heads of 16: four), so that the products of one run under the exponentials and
 // splits of the others.  Bound by matrix and vector time at the clock that both leave (N = 768, heads of 32: 901 us a launch, matrix
 // pipe 48 %, vector pipe 63 %, 1.67 GHz; three bf16 terms 1446; heads of 16, three templates of 200: 54 us, 22 and 59 %; 88).
+// A 32 x 32 tile is 80 vector instructions (169 ns on a SIMD alone) and 12 products (180, 300 with all CUs busy).
 //   S^T = K Q^T  (rows = keys, columns = queries), three products per k-step, started from the triangle bias (the
 //                accumulator is loaded with it).  Logits are in natural units times the scales of q and k, a power of
 //                two that the bias and the mask bias carry too, and not pre-multiplied by log2(e): a row of masked keys
@@ -18,10 +19,11 @@
 //                all four of the terms.
 // Per 32-key tile the work-group brings in the bias slice of its query range (it does not depend on i: shared by its
 // rows) and each row's K and V^T operands (shared by the row's two waves) with direct-to-LDS buffer loads, one tile
-// ahead, the bias and (width 16) the operands into double buffers: no registers are held for data in flight, and the only wait for
-// loads is one vmcnt(0) + barrier per key tile, a whole tile of arithmetic after they were issued.  At width 32 the operands
-// have one place, which a second barrier frees once they are in registers: with two, only two work-groups fit (N = 768 4744 / 4596 us a pass).  The bias slice is XOR-swizzled on the global side
-// (a lane picks which 16-byte chunk it fetches for its fixed LDS slot).
+// ahead, the bias into double buffers: no registers are held for data in flight, and the only wait for
+// loads is one vmcnt(0) + barrier per key tile, a whole tile of arithmetic after they were issued.  The operands have one place, which a
+// second barrier frees once they are in registers: with two, one work-group fewer fits (width 32, three / two, N = 768: 4596 / 4744 us a pass;
+// width 16, four / three, us a launch: three templates of 150 34.2 / 36.4, of 250 83.8 / 88.0, two of 384 174 / 185, one of 150 16.9 / 16.6).
+// The bias slice is XOR-swizzled on the global side (a lane picks which 16-byte chunk it fetches for its fixed LDS slot).
 //
 // Softmax weights as fp16 terms have to lie between 2^-13 (below it their second terms lose bits) and 2^16.  The first
 // pass takes as a query's offset the largest logit of the first key tile that has an unmasked key, and lifts the weights by 2^kLift
@@ -49,17 +51,16 @@ constexpr int kTbI = kTb / (64 * 2 * kRows);    // load instructions of a wave f
 template <int STEPS>
 struct CoreH2 {
   static constexpr int kKv = 2 * STEPS * 64;    // K (steps x terms), and as many of V^T (two steps x terms, or x 1 at width 16)
-  static constexpr int kStages = STEPS == 2 ? 1 : 2;  // of K and V^T
-  static constexpr size_t kLds = (size_t)(2 * kTb + kRows * kStages * 2 * kKv) * 16;
+  static constexpr size_t kLds = (size_t)(2 * kTb + kRows * 2 * kKv) * 16;
 };
 
 template <int STEPS>
-__global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32 p, int n_qc, int n_rg, int total, int per_xcd) {
+__global__ __launch_bounds__(128 * kRows, STEPS == 2 ? 3 : 4) void triattn_core_h2_f32(TriattnF32 p, int n_qc, int n_rg, int total, int per_xcd) {
   typedef CoreH2<STEPS> L;
   constexpr int QT = 2, D = 16 * STEPS;
   extern __shared__ u32x4_t lds4[];
   u32x4_t* tb_lds = lds4;                 // [2][kTb]
-  u32x4_t* kv_lds = lds4 + 2 * kTb;    // [kRows][kStages][K, V^T]
+  u32x4_t* kv_lds = lds4 + 2 * kTb;    // [kRows][K, V^T]
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row = wave >> 1, qh = wave & 1;
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
                                              buffer_rsrc(kvp + kv_plane, STEPS == 1 && qh ? kv_bytes - 1024 : kv_bytes)};
   const __amdgpu_buffer_rsrc_t tb_rsrc = buffer_rsrc(tbp, (size_t)N * Jp * sizeof(float));
   const uint32_t lane_off = lane * 16;
-  u32x4_t* kv_row = kv_lds + row * (L::kStages * 2 * L::kKv);
+  u32x4_t* kv_row = kv_lds + row * (2 * L::kKv);
   auto issue_bias = [&](int kt, int buf) {  // buf is a constant at every call site
     u32x4_t* tdst = tb_lds + buf * kTb + 64 * kTbI * wave;
 #pragma unroll
@@ -130,8 +131,8 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
       __builtin_amdgcn_raw_ptr_buffer_load_lds(tb_rsrc, (void OF3_LDS_AS*)(tdst + 64 * n), 16, tb_off[n],
                                                kt * (32 * (int)sizeof(float)), 0, 0);
   };
-  auto issue_kv = [&](int kt, int buf) {
-    u32x4_t* kdst = kv_row + (2 * (L::kStages == 2 ? buf : 0) + qh) * L::kKv;
+  auto issue_kv = [&](int kt) {
+    u32x4_t* kdst = kv_row + qh * L::kKv;
 #pragma unroll
     for (int n = 0; n < 2 * STEPS; ++n)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(kv_rsrc[n & 1], (void OF3_LDS_AS*)(kdst + 64 * n), 16, lane_off,
@@ -176,8 +177,8 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
   struct Operands {
     u32x4_t k[STEPS][2], v[2][STEPS];
   };
-  auto read_operands = [&](int buf) {
-    const u32x4_t* kvb = kv_row + (L::kStages == 2 ? buf : 0) * (2 * L::kKv) + lane;
+  auto read_operands = [&]() {
+    const u32x4_t* kvb = kv_row + lane;
     Operands o;
 #pragma unroll
     for (int st = 0; st < STEPS; ++st)
@@ -191,14 +192,13 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
   };
   uint32_t uneven[QT];  // level pass: bits in which a logit of the lane's query differed from level_at's
   uint32_t level_at = 0u;
-  auto tile = [&](auto kind, int buf, float mb, const Operands& given, int keys_left) {
+  auto tile = [&](auto kind, int buf, float mb, const Operands& op, int keys_left) {
     constexpr bool kTrack = decltype(kind)::value == kTracked, kLevel = decltype(kind)::value == kLevelled;
     if (!wave_has_work) return;
     // first pass: a tile whose keys are all masked or padded adds exp(-1e9 + logit) = 0 exactly to every sum
     if (!kTrack && !kLevel && __builtin_amdgcn_ballot_w64(mb > -1e8f) == 0) return;
     const bool has_mb = __builtin_amdgcn_ballot_w64(mb != 0.f) != 0;
     const u32x4_t* tbuf = tb_lds + buf * kTb + (64 * qh + l32) * 8;
-    const Operands op = L::kStages == 1 ? given : read_operands(buf);
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       if (qt > 0 && q0 + 32 * qt >= N) continue;
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
   auto first_loads = [&]() {
     mv_next = load_mask(0);
     issue_bias(0, 0);
-    issue_kv(0, 0);
+    issue_kv(0);
   };
   auto pass = [&](auto kind) {
     constexpr bool kLevel = decltype(kind)::value == kLevelled;
@@ -314,14 +314,11 @@ __global__ __launch_bounds__(128 * kRows, 3) void triattn_core_h2_f32(TriattnF32
       const int ktn = kt + 1 < nkt ? kt + 1 : nkt - 1;
       mv_next = load_mask(ktn);
       issue_bias(ktn, buf ^ 1);
-      Operands op;
-      if (L::kStages == 1) {
-        op = read_operands(buf);
-        wait_lds_reads();
-        __builtin_amdgcn_s_barrier();  // both waves of the row hold the operands in registers: their place is free
-        compiler_fence();
-      }
-      issue_kv(ktn, buf ^ 1);
+      const Operands op = read_operands();
+      wait_lds_reads();
+      __builtin_amdgcn_s_barrier();  // both waves of the row hold the operands in registers: their place is free
+      compiler_fence();
+      issue_kv(ktn);
       tile(kind, buf, mb, op, N - 32 * kt);
       compiler_fence();
     };
