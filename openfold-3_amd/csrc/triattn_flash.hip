@@ -7,9 +7,9 @@
 // With head width 16 or 32 the kernel is bound by the softmax's vector instructions (a SIMD spends
 // matrix time plus vector time), so the organisation removes vector work and keeps four waves per
 // SIMD to cover each other's waits:
-//  * work-group = 4 consecutive rows i x one (head, query range); a wave owns two (four) 32-query tiles of one row.  Long
-//    launches with heads of 32: 8 waves, 128 queries, two work-groups per CU (64 KB of LDS and 128 registers per lane
-//    each); otherwise 4 waves, 64 or 128 queries, three or four work-groups per CU.  The triangle bias of the query range
+//  * work-group = 4 consecutive rows i x one (head, query range); a wave owns two, three or four 32-query tiles of one row:
+//    4 waves, 64, 96 or (heads of 16) 128 queries, three or four work-groups per CU, or, heads of 32, 8 waves, 128 queries, two
+//    work-groups per CU (64 KB of LDS and 128 registers per lane each).  The triangle bias of the query range
 //    does not depend on i: each 32-key slice of it is brought into LDS once per work-group and every wave reads it
 //    straight into the MFMA accumulator, which adds it for free.
 //  * everything a key tile needs (the work-group's bias slice, each row's K tile and V^T tile,
@@ -84,13 +84,15 @@ constexpr float kMaskedBelow = -1e8f;  // a mask bias below this sends exp2 of a
 // reader there, and the maximum then is that of the logits before their last k-step
 __device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
-// QW = waves per row, RQ = 32-query tiles per wave: a work-group is 4 rows x 32 QW RQ queries.  Two waves (128 queries, two
-// work-groups of 8 waves per CU) move the fewest K and V^T bytes into LDS; one wave (64 or 128 queries, four or three work-groups
-// of 4 waves per CU) needs one K / V^T stage in place of two, and its smaller work-groups fill a short launch better.  Which
-// is taken where: triattn_flash_launch.  (Four waves, one work-group per CU, were slower everywhere: N = 768 395 against 375 us;
-// one 32-query tile per wave, too: 4 x 512 with head width 16 443 against 392 us.)
+// QW = waves per row, RQ = 32-query tiles per wave: a work-group is 4 rows x 32 QW RQ queries.  A K / V^T tile read from LDS serves
+// RQ tiles of logits, so more of them are less work per logit, as long as registers leave three waves per SIMD: four tiles
+// of heads of 32 do not (24 registers spilled at 168: N = 768 520 against 360 us).  One wave per row needs one K / V^T stage in place of
+// two; two waves (128 queries of heads of 32) move the fewest bytes into LDS.  Which is taken where: triattn_flash_launch.
+// (Four waves, one work-group per CU, were slower everywhere: N = 768 395 against 375 us; one 32-query tile per wave, too:
+// 4 x 512 with head width 16 443 against 392 us.)
+constexpr int groups_per_cu(int D, int QW, int RQ) { return QW == 2 ? 2 : RQ == 4 || (RQ == 3 && D == 32) ? 3 : 4; }
 template <int D, int QW, int RQ>
-__global__ __launch_bounds__(64 * kRows * QW, RQ == 4 ? 3 : 4) void triattn_flash_kernel(TriattnFlashArgs p, int n_qc, int n_rg, int total,
+__global__ __launch_bounds__(64 * kRows * QW, QW * groups_per_cu(D, QW, RQ)) void triattn_flash_kernel(TriattnFlashArgs p, int n_qc, int n_rg, int total,
                                                                                         int per_xcd) {
   constexpr int kWaves = kRows * QW;
   constexpr int kRQ = RQ, kQW = 32 * RQ;  // queries per wave
@@ -545,19 +547,35 @@ hipError_t triattn_flash_launch(const TriattnFlashArgs& args, int D, hipStream_t
   int cus = 0;
   const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
   if (e != hipSuccess) return e;
-  // work-groups that launches of 128 queries each have
-  const long ranges = (args.N + 127) / 128, wide = ranges * ((args.N + kRows - 1) / kRows) * args.B * args.H;
+  // A launch of ranges of 64, 96 or 128 queries takes its rounds (work-groups over places on the chip) times a round's time in
+  // that form; a round that is not full takes 0.4 of it and the share of its places that are taken of the other 0.6.  Fitted to launches
+  // by themselves, 52 lengths of heads of 32 between 160 and 2048 and 27 of 1 to 4 templates: the form taken is 0.5 % from the best on
+  // average, with work-groups of 96 left out 2.6 %.
+  auto estimate = [&](int queries, int per_cu, double round) {
+    const long items = (long)((args.N + queries - 1) / queries) * ((args.N + kRows - 1) / kRows) * args.B * args.H, places = (long)per_cu * cus;
+    const double part = (double)(items % places) / (double)places;
+    return round * ((double)(items / places) + (part > 0 ? 0.4 + 0.6 * part : 0.0));
+  };
+  // up to three work-groups of 64 queries per CU nothing else has enough of them (heads of 32, N = 128: 6.3 against 8.0 for 128, 192: 14.0, 14.2
+  // for 96; heads of 16, 1 x 150: 9.8 and 11.3 for 96)
+  const bool few = (long)((args.N + 63) / 64) * ((args.N + kRows - 1) / kRows) * args.B * args.H <= 3L * cus;
   if (D == 32) {
-    // Head width 32, 64 against 128 queries, us (256 CUs): N = 128 6.3 / 8.0, 160 9.0 / 12.7, 192 13.1 / 15.3, 300 32 / 39, 384 53 / 58,
-    // 450 94 / 96, 512 115 / 114, 768 365 / 343, 1280 1652 / 1544: up to three rounds of the latter.  Not where those are
-    // between one and two per CU and nearly full (N = 200 16.9 / 16.6, 230 19.2 / 18.6, 256 20.6 / 19.9).
-    const bool full = wide > cus && wide <= 2L * cus && (args.N + 63) / 64 == 2 * ranges;
-    return wide <= 6L * cus && !full ? launch<32, 1, 2>(args, stream) : launch<32, 2, 2>(args, stream);
+    // us a launch, 64 / 96 / 128 queries (256 CUs): N = 160 10.3 / 12.4 / 14.0, 256 22.0 / 22.0 / 21.8, 300 36 / 40 / 43, 384 63.5 / 60.1 / 65.5,
+    // 400 75 / 80 / 90, 450 111 / 103 / 118, 512 143 / 146 / 140, 576 202 / 187 / 203, 768 429 / 400 / 405, 900 683 / 649 / 681, 1024 902 / 891 / 865,
+    // 1280 1658 / 1685 / 1608, 1728 3946 / 3813 / 3883, 2048 6380 / 6632 / 6190.
+    const double t64 = estimate(64, groups_per_cu(32, 1, 2), 1.06), t96 = estimate(96, groups_per_cu(32, 1, 3), 1.11),
+                 t128 = estimate(128, groups_per_cu(32, 2, 2), 1.0);
+    if (few || (t64 <= t96 && t64 <= t128)) return launch<32, 1, 2>(args, stream);
+    return t96 <= t128 ? launch<32, 1, 3>(args, stream) : launch<32, 2, 2>(args, stream);
   }
   if (D == 16) {
-    // Head width 16, one wave per row: 64 / 128 queries, and 128 with two waves: 2 x 187 15.6 / 16.9 / 18.2, 3 x 256 38.8 / 40.2 / 41.6,
-    // 2 x 400 (28 % of the 128-query ranges empty) 92 / 105 / 112, 1 x 512 84.8 / 83.1 / 88.3, 4 x 512 370 / 339 / 367.
-    return wide >= 12L * cus && 128 * ranges * 100 <= 115L * args.N ? launch<16, 1, 4>(args, stream) : launch<16, 1, 2>(args, stream);
+    // us a launch, 64 / 96 / 128 queries: 1 x 100 6.4 / 7.4 / 8.1, 2 x 187 17.3 / 16.1 / 18.3, 2 x 288 46 / 43 / 50, 3 x 256 47 / 49 / 47, 4 x 280 89 / 80 / 90,
+    // 2 x 384 91 / 85 / 88, 4 x 400 232 / 213 / 219, 3 x 480 264 / 236 / 237, 4 x 512 400 / 377 / 360.  (Two waves to a row, 128 queries: 4 x 512 367
+    // against 339.)
+    const double t64 = estimate(64, groups_per_cu(16, 1, 2), 0.55), t96 = estimate(96, groups_per_cu(16, 1, 3), 0.72),
+                 t128 = estimate(128, groups_per_cu(16, 1, 4), 0.75);
+    if (few || (t64 <= t96 && t64 <= t128)) return launch<16, 1, 2>(args, stream);
+    return t96 <= t128 ? launch<16, 1, 3>(args, stream) : launch<16, 1, 4>(args, stream);
   }
   return hipErrorInvalidValue;
 }
