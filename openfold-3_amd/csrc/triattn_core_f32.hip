@@ -2,8 +2,8 @@
 // (of3_split.h), head width 16 * STEPS (32 or 16), for the shapes whose projection pass delivers them
 // (pair_pass_f32.hip); pair_f32.hip has the cores for every other shape.
 //
-// Work-group = 4 waves = 2 consecutive rows i x 2 halves of one (head, 128-query range); a wave owns 64 queries (two
-// 32-query tiles) of one row.  Three work-groups share a CU (heads of 16: four), so that the products of one run under the exponentials and
+// Work-group = 4 waves = 2 consecutive rows i x 2 halves of one (head, 128-query range), or 4 rows x one of 64 queries; a wave owns 64
+// queries (two 32-query tiles) of one row.  Three work-groups share a CU (heads of 16: four), so that the products of one run under the exponentials and
 // splits of the others.  Bound by matrix and vector time at the clock that both leave (N = 768, heads of 32: 901 us a launch, matrix
 // pipe 48 %, vector pipe 63 %, 1.67 GHz; three bf16 terms 1446; heads of 16, three templates of 200: 54 us, 22 and 59 %; 88).
 // A 32 x 32 tile is 80 vector instructions (169 ns on a SIMD alone) and 12 products (180, 300 with all CUs busy).
@@ -18,10 +18,10 @@
 //                Width 16: the operand's free rows hold V^T's second terms, [vh; vl] p, added at the end: two products,
 //                all four of the terms.
 // Per 32-key tile the work-group brings in the bias slice of its query range (it does not depend on i: shared by its
-// rows) and each row's K and V^T operands (shared by the row's two waves) with direct-to-LDS buffer loads, one tile
+// rows) and each row's K and V^T operands (shared by the row's waves) with direct-to-LDS buffer loads, one tile
 // ahead, the bias into double buffers: no registers are held for data in flight, and the only wait for
-// loads is one vmcnt(0) + barrier per key tile, a whole tile of arithmetic after they were issued.  The operands have one place, which a
-// second barrier frees once they are in registers: with two, one work-group fewer fits (width 32, three / two, N = 768: 4596 / 4744 us a pass;
+// loads is one vmcnt(0) + barrier per key tile, a whole tile of arithmetic after they were issued.  The operands have one place, which (two
+// waves to a row) a second barrier frees once they are in registers: with two, one work-group fewer fits (width 32, three / two, N = 768: 4596 / 4744 us a pass;
 // width 16, four / three, us a launch: three templates of 150 34.2 / 36.4, of 250 83.8 / 88.0, two of 384 174 / 185, one of 150 16.9 / 16.6).
 // The bias slice is XOR-swizzled on the global side (a lane picks which 16-byte chunk it fetches for its fixed LDS slot).
 //
@@ -42,28 +42,34 @@ namespace of3 {
 
 namespace {
 
-constexpr int kRows = 2;
+constexpr int kWaves = 4;
+template <int STEPS>
+constexpr int kPerCu = STEPS == 2 ? 3 : 4;  // work-groups
 constexpr float kLift = 4.f, kHigh = 0x1p15f;
 constexpr float kFloor = -3e38f;  // in place of -infinity as an offset
 enum { kFirst, kTracked, kLevelled };  // what a pass over the keys does
-constexpr int kTb = 128 * 8;                    // bias slice [128 queries][32 keys] fp32 in 16-byte slots
-constexpr int kTbI = kTb / (64 * 2 * kRows);    // load instructions of a wave for it
-template <int STEPS>
+template <int STEPS, int QW>
 struct CoreH2 {
+  static constexpr int kRows = kWaves / QW;
+  static constexpr int kQueries = 64 * QW;
+  static constexpr int kTb = kQueries * 8;           // bias slice [queries][32 keys] fp32 in 16-byte slots
+  static constexpr int kTbI = kTb / (64 * kWaves);   // load instructions of a wave for it
   static constexpr int kKv = 2 * STEPS * 64;    // K (steps x terms), and as many of V^T (two steps x terms, or x 1 at width 16)
   static constexpr size_t kLds = (size_t)(2 * kTb + kRows * 2 * kKv) * 16;
 };
 
-template <int STEPS>
-__global__ __launch_bounds__(128 * kRows, STEPS == 2 ? 3 : 4) void triattn_core_h2_f32(TriattnF32 p, int n_qc, int n_rg, int total, int per_xcd) {
-  typedef CoreH2<STEPS> L;
+// QW: waves of a row, 1 or 2 (kWaves / QW rows, 64 QW queries)
+template <int STEPS, int QW>
+__global__ __launch_bounds__(64 * kWaves, kPerCu<STEPS>) void triattn_core_h2_f32(TriattnF32 p, int n_qc, int n_rg, int total, int per_xcd) {
+  typedef CoreH2<STEPS, QW> L;
+  constexpr int kRows = L::kRows, kQueries = L::kQueries, kTb = L::kTb, kTbI = L::kTbI;
   constexpr int QT = 2, D = 16 * STEPS;
   extern __shared__ u32x4_t lds4[];
   u32x4_t* tb_lds = lds4;                 // [2][kTb]
   u32x4_t* kv_lds = lds4 + 2 * kTb;    // [kRows][K, V^T]
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int row = wave >> 1, qh = wave & 1;
+  const int row = wave / QW, qh = wave % QW;
   const int lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int N = p.N, H = p.H, Jp = p.Jp, nt = Jp / 32;
   const int logical = xcd_logical_block(blockIdx.x, per_xcd);
@@ -73,7 +79,7 @@ __global__ __launch_bounds__(128 * kRows, STEPS == 2 ? 3 : 4) void triattn_core_
   const bool row_valid = i_raw < N;  // wave-uniform; idle waves still take part in the loads and barriers
   const int i = row_valid ? i_raw : N - 1;
   const int b = bh / H, h = bh % H;
-  const int q0 = qc * 128 + 64 * qh;
+  const int q0 = qc * kQueries + 64 * qh;
   const size_t bih = ((size_t)b * N + i) * H + h;
   const long plane = p.qk_plane / 8;  // in 16-byte slots
   const u32x4_t* Q = reinterpret_cast<const u32x4_t*>(p.qs) + bih * nt * (64 * STEPS) + lane;
@@ -103,24 +109,30 @@ __global__ __launch_bounds__(128 * kRows, STEPS == 2 ? 3 : 4) void triattn_core_
 
   // bias slice: instruction n of wave w fills slots 64 (kTbI w + n) .. + 63; slot t holds chunk
   // (t & 7) ^ ((q >> 1) & 7) of query q = t >> 3 of the work-group's range
-  uint32_t tb_off[kTbI];
+  uint32_t tb_off[4];  // kTbI of them: with the dependent size clang leaves the kernel out of the host code
+  static_assert(kTbI <= 4, "");
 #pragma unroll
   for (int n = 0; n < kTbI; ++n) {
     const int t = 64 * (kTbI * wave + n) + lane;
     const int qloc = t >> 3, chunk = (t & 7) ^ ((qloc >> 1) & 7);
-    int qrow = qc * 128 + qloc;
+    int qrow = qc * kQueries + qloc;
     qrow = qrow < N ? qrow : N - 1;
     tb_off[n] = (uint32_t)(((size_t)qrow * Jp + 4 * chunk) * sizeof(float));
   }
   // This wave's share of its row's tile: the K operands (first wave of the row) or the V^T operands, 2 STEPS instructions of
-  // 1 KB.  Width 32: step n / 2, term n % 2, a descriptor per term (a plane can be larger than a descriptor's range); width
-  // 16: the term n of K's step, or the step n of V^T's plane, which begins 1 KB further on
-  const long kv_plane = STEPS == 2 ? (qh ? p.v_plane : p.qk_plane) : (qh ? 512 : p.qk_plane);
-  const int kv_tile = STEPS == 2 || qh ? 2048 : 1024;  // bytes of a key tile in a plane
-  const bf16_t* kvp = (qh ? p.vs : p.ks) + bih * nt * (kv_tile / 2);
+  // 1 KB, or (QW = 1) both.  Width 32: step n / 2, term n % 2, a descriptor per term (a plane can be larger than a descriptor's range);
+  // width 16: the term n of K's step, or the step n of V^T's plane, which begins 1 KB further on
+  const bool is_v = QW == 2 && qh;  // what its first 2 STEPS instructions bring
+  const long kv_plane = STEPS == 2 ? (is_v ? p.v_plane : p.qk_plane) : (is_v ? 512 : p.qk_plane);
+  const int kv_tile = STEPS == 2 || is_v ? 2048 : 1024;  // bytes of a key tile in a plane
+  const bf16_t* kvp = (is_v ? p.vs : p.ks) + bih * nt * (kv_tile / 2);
   const size_t kv_bytes = (size_t)nt * kv_tile;
   const __amdgpu_buffer_rsrc_t kv_rsrc[2] = {buffer_rsrc(kvp, kv_bytes),
-                                             buffer_rsrc(kvp + kv_plane, STEPS == 1 && qh ? kv_bytes - 1024 : kv_bytes)};
+                                             buffer_rsrc(kvp + kv_plane, STEPS == 1 && is_v ? kv_bytes - 1024 : kv_bytes)};
+  const bf16_t* vp = p.vs + bih * nt * 1024;
+  const long v_plane = STEPS == 2 ? p.v_plane : 512;
+  const __amdgpu_buffer_rsrc_t v_rsrc[2] = {buffer_rsrc(vp, (size_t)nt * 2048),  // QW = 1
+                                            buffer_rsrc(vp + v_plane, (size_t)nt * 2048 - (STEPS == 1 ? 1024 : 0))};
   const __amdgpu_buffer_rsrc_t tb_rsrc = buffer_rsrc(tbp, (size_t)N * Jp * sizeof(float));
   const uint32_t lane_off = lane * 16;
   u32x4_t* kv_row = kv_lds + row * (2 * L::kKv);
@@ -137,6 +149,12 @@ __global__ __launch_bounds__(128 * kRows, STEPS == 2 ? 3 : 4) void triattn_core_
     for (int n = 0; n < 2 * STEPS; ++n)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(kv_rsrc[n & 1], (void OF3_LDS_AS*)(kdst + 64 * n), 16, lane_off,
                                                kt * kv_tile + (n >> 1) * 1024, 0, 0);
+    if (QW == 1) {
+#pragma unroll
+      for (int n = 0; n < 2 * STEPS; ++n)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rsrc[n & 1], (void OF3_LDS_AS*)(kdst + L::kKv + 64 * n), 16, lane_off,
+                                                 kt * 2048 + (n >> 1) * 1024, 0, 0);
+    }
   };
   // mask value of key 32 kt + l32 (clamped to a real key; some bias value when there is no mask: not used)
   const float* mrow = p.mask ? p.mask + b * p.mv.stride_b + i * p.mv.stride_r : tbp;
@@ -316,7 +334,7 @@ __global__ __launch_bounds__(128 * kRows, STEPS == 2 ? 3 : 4) void triattn_core_
       issue_bias(ktn, buf ^ 1);
       const Operands op = read_operands();
       wait_lds_reads();
-      __builtin_amdgcn_s_barrier();  // both waves of the row hold the operands in registers: their place is free
+      if (QW == 2) __builtin_amdgcn_s_barrier();  // both waves of the row hold the operands in registers: their place is free
       compiler_fence();
       issue_kv(ktn);
       tile(kind, buf, mb, op, N - 32 * kt);
@@ -356,7 +374,7 @@ __global__ __launch_bounds__(128 * kRows, STEPS == 2 ? 3 : 4) void triattn_core_
     __syncthreads();
     uint32_t any = 0;
 #pragma unroll
-    for (int w = 0; w < 2 * kRows; ++w) any |= votes[w];
+    for (int w = 0; w < kWaves; ++w) any |= votes[w];
     const bool result = __builtin_amdgcn_readfirstlane(any) != 0;
     if (result) {
       __syncthreads();  // every wave has read the votes before loads land on them
@@ -401,23 +419,37 @@ __global__ __launch_bounds__(128 * kRows, STEPS == 2 ? 3 : 4) void triattn_core_
   }
 }
 
-template <int STEPS>
+template <int STEPS, int QW>
 hipError_t launch(const TriattnF32& p, hipStream_t stream) {
-  constexpr size_t lds = CoreH2<STEPS>::kLds;
-  const hipError_t e = allow_dynamic_lds<triattn_core_h2_f32<STEPS>>(lds);
+  typedef CoreH2<STEPS, QW> L;
+  const hipError_t e = allow_dynamic_lds<triattn_core_h2_f32<STEPS, QW>>(L::kLds);
   if (e != hipSuccess) return e;
-  const int n_qc = (p.N + 127) / 128, n_rg = (p.N + kRows - 1) / kRows;
+  const int n_qc = (p.N + L::kQueries - 1) / L::kQueries, n_rg = (p.N + L::kRows - 1) / L::kRows;
   const long total = (long)n_qc * n_rg * p.B * p.H;
   if (total > 0x7fffffffL - 8) return hipErrorInvalidValue;
   const int per_xcd = (int)((total + 7) / 8);
-  hipLaunchKernelGGL(triattn_core_h2_f32<STEPS>, dim3(per_xcd * 8), dim3(128 * kRows), lds, stream, p, n_qc, n_rg, (int)total, per_xcd);
+  hipLaunchKernelGGL((triattn_core_h2_f32<STEPS, QW>), dim3(per_xcd * 8), dim3(64 * kWaves), L::kLds, stream, p, n_qc, n_rg, (int)total, per_xcd);
   return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t triattn_core_h2_f32_launch(const TriattnF32& p, hipStream_t stream) {
-  return p.D == 32 ? launch<2>(p, stream) : launch<1>(p, stream);
+  // 64 queries of four rows instead of 128 of two, with one barrier a key tile less and twice the K and V^T through LDS, where the last range of
+  // 128 would be at most half full.  us a launch, 64 / 128: heads of 16, templates 1 x 140 13.7 / 16.6, 2 x 187 30.6 / 34.1, 4 x 300 190 / 205, 1 x 400 109
+  // / 119; others level (2 x 384 171.5 / 170.5, a pass of 3 x 200 874 / 870).  Heads of 32, whose K and V^T are twice as long: N = 300 80 / 87, 400
+  // 177 / 184, 550 396 / 399, 700 level; others slower (128 12.6 / 12.3, 384 147 / 141, 768 931 / 891); and where 128 leave no second round only if
+  // the last of those is a quarter (150 18.7 / 21.4; 180 27.0 / 26.2).
+  static int cache[kMaxDevices];
+  int cus = 0;
+  const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+  if (e != hipSuccess) return e;
+  typedef CoreH2<2, 2> Wide;
+  const int last = p.N > Wide::kQueries ? p.N % Wide::kQueries : 0;
+  if (p.D == 16) return last > 0 && last <= 64 ? launch<1, 1>(p, stream) : launch<1, 2>(p, stream);
+  const long wide = (long)((p.N + Wide::kQueries - 1) / Wide::kQueries) * ((p.N + Wide::kRows - 1) / Wide::kRows) * p.B * p.H;
+  const bool narrow = p.N <= 640 && last > 0 && last <= (wide > (long)kPerCu<2> * cus ? 64 : 32);
+  return narrow ? launch<2, 1>(p, stream) : launch<2, 2>(p, stream);
 }
 
 }  // namespace of3

@@ -3,6 +3,7 @@ waves per row (heads of 32) and of one wave per row (heads of 16), and 96 of one
 32-query tiles, at ragged lengths, with masked rows and runs, and with logits that need the second pass; lengths on either side of the rule."""
 import pytest
 
+import test_gpu_fp32 as fp32
 import test_gpu_stages as stages
 
 pytestmark = pytest.mark.gpu
@@ -20,3 +21,10 @@ def test_forms(D, n, B, logit_scale):
                                         (16, 187, 2, "tail"), (16, 288, 2, "middle"), (16, 250, 8, "tail"), (16, 240, 8, "head")])
 def test_padding(D, n, B, pads):
     stages.test_triattn_flash_padding_masks(D, n, B, pads)
+
+
+# fp32: work-groups of 64 queries (a last range of 128 that is at most half full; heads of 32, one round of launches: a quarter) and of 128, with masked rows and columns
+@pytest.mark.parametrize("c,d,n,batch", [(128, 32, 129, ()), (128, 32, 160, ()), (128, 32, 161, ()), (128, 32, 161, (2,)), (128, 32, 193, ()),
+                                         (128, 32, 290, ()), (64, 16, 129, (2,)), (64, 16, 192, ()), (64, 16, 193, ())])
+def test_fp32_forms(c, d, n, batch):
+    fp32.test_triattn_fp32(True, c, d, 4, n, batch, True)
