@@ -29,6 +29,13 @@ template <int C, int CH, bool RAGGED, int PART, int TP>
 __global__ __launch_bounds__(4 * TP, C == 64 && TP == 64 ? 3 : 2) void trimul_out_kernel(TrimulOutArgs p, int full_per_row, int tail_shift, int tiles_per_batch,
                                                            int whole_tiles, int total_items) {
   static_assert(C == CH, "position-major x tile shares the z tile geometry");
+  // 64 channels, tiles of 64: every tile issues the same loads and stores (indices past the end are clamped, a store past the end is beyond its
+  // buffer), so that the compiler's wait for a tile's values counts the stores of the tile before it and leaves them in flight; with a load or a store
+  // under a condition it waits for all of them.  Rows leave whole: the waves put their channels in the residual's place and the lanes that loaded a
+  // row store it, 1 KB of it per instruction in the place of 16 bytes of each of 64 pieces of rows.  us a launch, before / now: three templates of 400
+  // 46.1 / 44.2, of 500 68.3 / 65.0, four of 384 53.5 / 51.2, of 512 88.5 / 81.8; up to three rounds level.  At 128 channels the counted waits
+  // are within 2 % (N = 300 23.3 / 23.5, 768 117.5 / 118.3) and whole rows lose 4 % (768 122): two work-groups to a CU, all registers taken.
+  constexpr bool ROWS = C == 64 && TP == 64;
   constexpr int NCH = C / 8;
   constexpr int LPP = NCH;
   constexpr int PPI = 64 / LPP;
@@ -96,8 +103,15 @@ __global__ __launch_bounds__(4 * TP, C == 64 && TP == 64 ? 3 : 2) void trimul_ou
     const bf16_t* zrow = p.z + b * p.z_view.stride_b + i0 * p.z_view.stride_r;  // the tile's first row (scalar)
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      const int pos = piece.first + ln_position(piece.count < TP, it);
-      const int di = RAGGED ? pos >> shift : 0, j = j0 + (RAGGED ? pos & jmask : pos);  // di = 0 in the whole-row pieces
+      int in_item = ln_position(piece.count < TP, it);
+      if (ROWS && PART < TP) in_item = in_item < piece.count ? in_item : piece.count - 1;
+      const int pos = piece.first + in_item;
+      int di = RAGGED ? pos >> shift : 0, j = j0 + (RAGGED ? pos & jmask : pos);  // di = 0 in the whole-row pieces
+      if (ROWS) {
+        if (RAGGED) di = i0 + di < N ? di : N - 1 - i0, j = j < N ? j : N - 1;
+        zraw[it] = *reinterpret_cast<const u32x4_t*>(zrow + di * p.z_view.stride_r + j * p.z_view.stride_k + 8 * ln_chunk);
+        continue;
+      }
       u32x4_t v = {0u, 0u, 0u, 0u};
       if ((PART == TP || it * LN_STEP < piece.count) && (!RAGGED || i0 + di < N) && j < N) v = *reinterpret_cast<const u32x4_t*>(zrow + di * p.z_view.stride_r + j * p.z_view.stride_k + 8 * ln_chunk);
       zraw[it] = v;
@@ -106,8 +120,10 @@ __global__ __launch_bounds__(4 * TP, C == 64 && TP == 64 ? 3 : 2) void trimul_ou
     for (int rr = 0; rr < XROUNDS; ++rr) {
       const int item = rr * NTH + tid;
       // channels 2cp, 2cp+1; positions 8pg..8pg+7: one row, as the width is >= 8
-      const int cp = item >> piece.group_bits, pg = (piece.first >> 3) + (item & ((1 << piece.group_bits) - 1));
-      if (PART < TP && cp >= CH / 2) break;
+      int cp = item >> piece.group_bits;
+      const int pg = (piece.first >> 3) + (item & ((1 << piece.group_bits) - 1));
+      if (PART < TP && ROWS) cp = cp < CH / 2 ? cp : CH / 2 - 1;
+      else if (PART < TP && cp >= CH / 2) break;
       int i = i0 + (RAGGED ? (8 * pg) >> shift : 0);
       const int j = j0 + (RAGGED ? (8 * pg) & jmask : 8 * pg);  // < Np: the planes are padded to whole 128-wide pieces
       if (RAGGED) i = i < Np ? i : Np - 1;    // rows of a last piece past the end of the plane: any row, never used
@@ -116,7 +132,12 @@ __global__ __launch_bounds__(4 * TP, C == 64 && TP == 64 ? 3 : 2) void trimul_ou
       xb[rr] = *reinterpret_cast<const u32x4_t*>(src + (size_t)Np * Np);
     }
   };
-  if ((int)blockIdx.x < total_items) load_tile(blockIdx.x);
+  if ((int)blockIdx.x >= total_items) return;
+  load_tile(blockIdx.x);
+  if (ROWS) {  // the weights count as used here: no wait for them, which would be one for the next tile's loads, inside the loop
+#pragma unroll
+    for (int s = 0; s < KS; ++s) __asm__ volatile("" : "+v"(wz[s]), "+v"(wgt[s]));
+  }
 
   auto do_tile = [&](auto positions, int item) {
     constexpr int P = decltype(positions)::value;
@@ -129,6 +150,7 @@ __global__ __launch_bounds__(4 * TP, C == 64 && TP == 64 ? 3 : 2) void trimul_ou
     const int shift = RAGGED ? shift_rt : WHOLE;
     const int jmask = (1 << shift) - 1;
     bf16_t* orow0 = p.out + b * p.z_view.stride_b + i0 * p.z_view.stride_r;  // the tile's first row (scalar)
+    if (ROWS && P < TP) __syncthreads();  // a whole tile's rows have left before other lanes write their places
 
     // x: transpose into xtile[pos][c] with 4-byte (channel pair) writes
 #pragma unroll
@@ -140,7 +162,7 @@ __global__ __launch_bounds__(4 * TP, C == 64 && TP == 64 ? 3 : 2) void trimul_ou
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const uint32_t ua = xa[rr][e >> 1], ub = xb[rr][e >> 1];
-        const uint32_t w = (e & 1) ? ((ua >> 16) | (ub & 0xffff0000u)) : ((ua & 0xffffu) | (ub << 16));
+        const uint32_t w = __builtin_amdgcn_perm(ub, ua, (e & 1) ? 0x07060302u : 0x05040100u);
         const int pos = 8 * pg + e;
         xt32[tile_slot<NCH, 0>(pos, chunk) * 4 + (within >> 1)] = w;
       }
@@ -180,7 +202,7 @@ __global__ __launch_bounds__(4 * TP, C == 64 && TP == 64 ? 3 : 2) void trimul_ou
         accg = mfma_32x32x16(wgt[s], bz, accg);
       }
       const int di = RAGGED ? pos >> shift : 0, j = j0 + (RAGGED ? pos & jmask : pos);
-      if ((!RAGGED || i0 + di < N) && j < N) {
+      if ((ROWS && P == TP) || ((!RAGGED || i0 + di < N) && j < N)) {
         bf16_t* orow = orow0;
         const int64_t off = di * p.z_view.stride_r + j * p.z_view.stride_k + 32 * ot + 16 * lh;
         float res[16];
@@ -203,15 +225,38 @@ __global__ __launch_bounds__(4 * TP, C == 64 && TP == 64 ? 3 : 2) void trimul_ou
           o0[q] = pack_bf16(res[2 * q], res[2 * q + 1]);
           o1[q] = pack_bf16(res[8 + 2 * q], res[8 + 2 * q + 1]);
         }
-        *reinterpret_cast<u32x4_t*>(orow + off) = o0;
-        *reinterpret_cast<u32x4_t*>(orow + off + 8) = o1;
+        if (ROWS && P == TP) {
+          rtile[tile_slot<NCH, 0>(pos, 4 * ot + 2 * lh)] = o0;
+          rtile[tile_slot<NCH, 0>(pos, 4 * ot + 2 * lh + 1)] = o1;
+        } else {
+          *reinterpret_cast<u32x4_t*>(orow + off) = o0;
+          *reinterpret_cast<u32x4_t*>(orow + off + 8) = o1;
+        }
       }
     }
     if (P == TP) __syncthreads();  // both tiles are rewritten by the next iteration
+    if (ROWS && P == TP) {
+      const __amdgpu_buffer_rsrc_t rows = buffer_rsrc(orow0 + j0 * p.z_view.stride_k, 0x7fffffffu);
+      const int sr = (int)p.z_view.stride_r, sk = (int)p.z_view.stride_k;  // a tile's offsets fit 31 bits (trimul_out_launch)
+#pragma unroll
+      for (int it = 0; it < LN_ITERS; ++it) {
+        const int pos = ln_position(false, it), di = RAGGED ? pos >> shift : 0, dj = RAGGED ? pos & jmask : pos;
+        const bool there = !RAGGED || (i0 + di < N && j0 + dj < N);
+        const uint32_t off = there ? (uint32_t)(di * sr + dj * sk + 8 * ln_chunk) * 2u : 0x80000000u;
+        __builtin_amdgcn_raw_buffer_store_b128(rtile[tile_slot<NCH, 0>(pos, ln_chunk)], rows, off, 0, 0);
+      }
+    }
   };
   typedef std::integral_constant<int, TP> Whole;
   int item = blockIdx.x;
-  for (; item < whole_tiles; item += gridDim.x) do_tile(Whole{}, item);
+  if constexpr (ROWS) {
+    if (item < whole_tiles) {  // peeled: the loop proper is only entered with a tile's stores in flight
+      do_tile(Whole{}, item);
+      for (item += gridDim.x; item < whole_tiles; item += gridDim.x) do_tile(Whole{}, item);
+    }
+  } else {
+    for (; item < whole_tiles; item += gridDim.x) do_tile(Whole{}, item);
+  }
   if constexpr (PART < TP) {
     if (item < total_items) do_tile(std::integral_constant<int, PART>{}, item);  // one piece: the last round
   }
@@ -253,7 +298,9 @@ hipError_t trimul_out_launch(const TrimulOutArgs& args, int C, int CH, hipStream
   const hipError_t e = small_pass(args.B, args.N, C == 128 ? 2 : 1, &small);
   if (e != hipSuccess) return e;
   if (small) return trimul_out_panels_launch(args, C, stream);
-  const bool half = out_tile_positions(C, args.N, true) == 64;
+  // at 64 channels the stores of a tile of 64 have 32-bit offsets from its first position: 8 rows, 64 columns
+  const bool fits = C != 64 || 8 * args.z_view.stride_r + 64 * args.z_view.stride_k + C < (1l << 30);
+  const bool half = fits && out_tile_positions(C, args.N, true) == 64;
   if (C == 128) return half ? launch_tiles<128, 64>(args, stream) : launch_tiles<128, 128>(args, stream);
   return half ? launch_tiles<64, 64>(args, stream) : launch_tiles<64, 128>(args, stream);
 }
