@@ -26,6 +26,11 @@ namespace {
 template <int C, int HD, int MODE, int PART, int TP>
 __global__ __launch_bounds__(4 * TP, C == 64 ? 4 : 2) void triattn_out_kernel(TriattnOutArgs p, uint32_t total_pos, int whole_tiles, int total_items) {
   static_assert(C == HD, "o tile shares the x tile geometry");
+  // Unconditional loads and stores and rows that leave whole, as in trimul_out.hip, in launches without pieces.  Past the end, which only the last
+  // tile of all has, the last position is loaded and stored again.  us a launch, before / now, 64 channels: three templates of 256 19.3 / 18.1, of 400
+  // 39.0 / 37.0, of 500 56.9 / 53.1, four of 384 45.7 / 41.5, of 512 78.7 / 70.8.  128 channels, tiles of 64 inside one row: N = 384 30.9 / 30.3, 512
+  // 53.3 / 50.8, 768 105.7 / 101.2; where a tile may lie in two rows level (451 42.5 / 43.2, 1100 208 / 208), and on tiles of 128 1700 491 / 496.
+  constexpr bool ROWS = PART == TP && (C == 64 ? MODE < 2 : MODE == 0 && TP == 64);
   constexpr int NCH = C / 8;
   constexpr int LPP = NCH;
   constexpr int PPI = 64 / LPP;
@@ -84,7 +89,13 @@ __global__ __launch_bounds__(4 * TP, C == 64 ? 4 : 2) void triattn_out_kernel(Tr
     const uint32_t p0 = (uint32_t)piece.tile * TP;
 #pragma unroll
     for (int it = 0; it < LN_ITERS; ++it) {
-      const int d = piece.first + ln_position(piece.count < TP, it);
+      int d = piece.first + ln_position(piece.count < TP, it);
+      if (ROWS) {
+        if (MODE != 0) d = p0 + d < total_pos ? d : (int)(total_pos - 1 - p0);
+        xraw[it] = *reinterpret_cast<const u32x4_t*>(p.x + view_offset(t, d) + 8 * ln_chunk);
+        oraw[it] = *reinterpret_cast<const u32x4_t*>(p.o + (size_t)(p0 + d) * HD + 8 * ln_chunk);
+        continue;
+      }
       u32x4_t vx = {0u, 0u, 0u, 0u}, vo = {0u, 0u, 0u, 0u};
       if ((PART == TP || it * LN_STEP < piece.count) && p0 + d < total_pos) {
         vx = *reinterpret_cast<const u32x4_t*>(p.x + view_offset(t, d) + 8 * ln_chunk);
@@ -94,7 +105,12 @@ __global__ __launch_bounds__(4 * TP, C == 64 ? 4 : 2) void triattn_out_kernel(Tr
       oraw[it] = vo;
     }
   };
-  if ((int)blockIdx.x < total_items) load_tile(blockIdx.x);
+  if ((int)blockIdx.x >= total_items) return;
+  load_tile(blockIdx.x);
+  if (ROWS) {  // the weights count as used here
+#pragma unroll
+    for (int s = 0; s < KS; ++s) __asm__ volatile("" : "+v"(wg[s]), "+v"(wo[s]));
+  }
 
   auto do_tile = [&](auto positions, int item) {
     constexpr int P = decltype(positions)::value;
@@ -146,9 +162,9 @@ __global__ __launch_bounds__(4 * TP, C == 64 ? 4 : 2) void triattn_out_kernel(Tr
       f32x16_t acc = zero16();
 #pragma unroll
       for (int s = 0; s < KS; ++s) acc = mfma_32x32x16(wo[s], otile[tile_slot<NCH, 0>(pos, 2 * s + lh)], acc);
-      if (p0 + pos < total_pos) {
+      if (ROWS || p0 + pos < total_pos) {
         bf16_t* outrow = p.out;
-        const int64_t off = view_offset(t, pos) + 32 * ot + 16 * lh;
+        const int64_t off = ROWS ? 0 : view_offset(t, pos) + 32 * ot + 16 * lh;
         float res[16];
 #pragma unroll
         for (int v = 0; v < 16; ++v) res[v] = acc[v];
@@ -169,14 +185,31 @@ __global__ __launch_bounds__(4 * TP, C == 64 ? 4 : 2) void triattn_out_kernel(Tr
           o0[q] = pack_bf16(res[2 * q], res[2 * q + 1]);
           o1[q] = pack_bf16(res[8 + 2 * q], res[8 + 2 * q + 1]);
         }
-        *reinterpret_cast<u32x4_t*>(outrow + off) = o0;
-        *reinterpret_cast<u32x4_t*>(outrow + off + 8) = o1;
+        if (ROWS) {
+          rtile[tile_slot<NCH, 0>(pos, 4 * ot + 2 * lh)] = o0;
+          rtile[tile_slot<NCH, 0>(pos, 4 * ot + 2 * lh + 1)] = o1;
+        } else {
+          *reinterpret_cast<u32x4_t*>(outrow + off) = o0;
+          *reinterpret_cast<u32x4_t*>(outrow + off + 8) = o1;
+        }
       }
     }
     if (P == TP) __syncthreads();
+    if (ROWS) {
+#pragma unroll
+      for (int it = 0; it < LN_ITERS; ++it) {
+        int d = ln_position(false, it);
+        if (MODE != 0) d = p0 + d < total_pos ? d : (int)(total_pos - 1 - p0);
+        *reinterpret_cast<u32x4_t*>(p.out + view_offset(t, d) + 8 * ln_chunk) = rtile[tile_slot<NCH, 0>(d, ln_chunk)];
+      }
+    }
   };
   typedef std::integral_constant<int, TP> Whole;
   int item = blockIdx.x;
+  if constexpr (ROWS) {
+    do_tile(Whole{}, item);  // peeled: the loop proper is only entered with a tile's stores in flight
+    item += gridDim.x;
+  }
   for (; item < whole_tiles; item += gridDim.x) do_tile(Whole{}, item);
   if constexpr (PART < TP) {
     if (item < total_items) do_tile(std::integral_constant<int, PART>{}, item);  // one piece: the last round
