@@ -180,7 +180,7 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_kernel(TrimulProjArgs 
     // previous tile's matrix phase before arriving, the other buffer may be overwritten by
     // the next LayerNorm phase.
     __syncthreads();
-    if (32 * T * tgroup >= P) return;
+    if (P < TP && 32 * T * tgroup >= P) return;  // of a whole tile every wave has a part, which the compiler cannot tell: it would count no stores
 
     // ---- projection phase
     float res[T][16];
