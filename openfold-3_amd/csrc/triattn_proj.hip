@@ -197,13 +197,22 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
 
       // ---- projection phase
       auto bias_tile = [&](int tt) {  // triangle bias of position tile tt (wave-uniform, may be a run-time value)
-        const int pos = 32 * tt + l32, i = tile_row(tt), j = tile_col(tt) + l32;
+        const int pos = 32 * tt + l32, i = tile_row(tt), j0 = tile_col(tt), j = j0 + l32;
         f32x16_t acc = zero16();
 #pragma unroll
         for (int s = 0; s < KS; ++s)
           acc = mfma_32x32x16(wb_lds[s * 64 + lane], tile[buf][proj_slot<NCH>(pos, 2 * s + lh)], acc);
         // rows 0..3 of the result sit in registers 0..3 of lanes 0..31
-        if (lh == 0) {
+        if constexpr (ROLE == 2) {
+          // Lanes 32..63 store past the end of their buffer: with the stores under a condition, and no others in this role, the compiler waits for all of
+          // them at the top of the loop (three templates of 300 34.2 / 32.9 us, four of 512 116.8 / 114.8; at 128 channels, where v's come after, no
+          // difference).
+#pragma unroll
+          for (int h = 0; h < H; ++h) {
+            const __amdgpu_buffer_rsrc_t row = buffer_rsrc(p.tbias + (((size_t)b * H + h) * N + i) * Jp + j0, 32 * sizeof(float));
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(j < N ? acc[h] * kLog2e : 0.f), row, 4 * l32 + 128 * lh, 0, 0);
+          }
+        } else if (lh == 0) {
 #pragma unroll
           for (int h = 0; h < H; ++h) p.tbias[(((size_t)b * H + h) * N + i) * Jp + j] = (j < N) ? acc[h] * kLog2e : 0.f;
         }
