@@ -47,9 +47,9 @@ __device__ __forceinline__ int proj_slot(int pos, int chunk) {
   return pos * NCH + (chunk ^ key);
 }
 
-// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only
-template <int C, int D, int NW, bool RAGGED, int PART>
-__global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p, int full_per_row, int tail_shift,
+// PART: positions of the pieces that the tiles of the last round are dealt in (last_round in of3_tiles.h), 128: whole tiles only.  PER_CU: work-groups
+template <int C, int D, int NW, bool RAGGED, int PART, int PER_CU>
+__global__ __launch_bounds__(64 * NW, PER_CU == 2 ? NW / 2 : 1) void triattn_proj_kernel(TriattnProjArgs p, int full_per_row, int tail_shift,
                                                                int tiles_per_batch, int whole_tiles, int total_items) {
   constexpr int H = 4;
   constexpr int HD = H * D;
@@ -309,28 +309,42 @@ __global__ __launch_bounds__(64 * NW) void triattn_proj_kernel(TriattnProjArgs p
   }
 }
 
-template <int C, int D, int NW, bool RAGGED>
-hipError_t launch(const TriattnProjArgs& a, hipStream_t stream) {
+template <int C, int D, int NW, bool RAGGED, int PER_CU>
+hipError_t launch(const TriattnProjArgs& a, const RaggedTiles& t, long total, hipStream_t stream) {
   static int cache[kMaxDevices];
   int grid_cap = 0;
-  // one work-group per CU at 64 channels too, where some instances would let two share it (4 x 512^2: 121 us against 112)
   hipError_t e = per_device(
-      cache, [&](int dev, int* v) { return C == 64 ? cu_count(dev, v) : resident_blocks(triattn_proj_kernel<C, D, NW, RAGGED, 128>, 64 * NW, dev, v); },
+      cache, [&](int dev, int* v) { return C == 64 ? cu_count(dev, v) : resident_blocks(triattn_proj_kernel<C, D, NW, RAGGED, 128, PER_CU>, 64 * NW, dev, v); },
       &grid_cap);
   if (e != hipSuccess) return e;
-  RaggedTiles t = {a.Jp / 128, 7, a.N * (a.Jp / 128)};  // whole (padded) rows in 128-wide pieces
-  if (RAGGED) t = ragged_tiles(a.N, 5);                 // pieces of whole 32-key panels
-  const long total = (long)a.B * t.per_batch;
-  if (total > 0x7fffffffL) return hipErrorInvalidValue;
+  if (C == 64) grid_cap *= PER_CU;
   const LastRound r = last_round(total, grid_cap);
   const int grid = r.items < grid_cap ? r.items : grid_cap;
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), 0, stream, a, t.full_per_row, t.tail_shift, t.per_batch, r.whole, r.items);
   };
-  if (r.piece == 32) go(triattn_proj_kernel<C, D, NW, RAGGED, 32>);
-  else if (r.piece == 64) go(triattn_proj_kernel<C, D, NW, RAGGED, 64>);
-  else go(triattn_proj_kernel<C, D, NW, RAGGED, 128>);
+  if (r.piece == 32) go(triattn_proj_kernel<C, D, NW, RAGGED, 32, PER_CU>);
+  else if (r.piece == 64) go(triattn_proj_kernel<C, D, NW, RAGGED, 64, PER_CU>);
+  else go(triattn_proj_kernel<C, D, NW, RAGGED, 128, PER_CU>);
   return hipGetLastError();
+}
+template <int C, int D, int NW, bool RAGGED>
+hipError_t launch_tiles(const TriattnProjArgs& a, hipStream_t stream) {
+  RaggedTiles t = {a.Jp / 128, 7, a.N * (a.Jp / 128)};  // whole (padded) rows in 128-wide pieces
+  if (RAGGED) t = ragged_tiles(a.N, 5);                 // pieces of whole 32-key panels
+  const long total = (long)a.B * t.per_batch;
+  if (total > 0x7fffffffL) return hipErrorInvalidValue;
+  if constexpr (C == 64) {
+    // Two work-groups to a CU, whose barriers do not coincide, from more than one tile per CU up to sixteen; us a launch, one / two: templates 2 x 300 24.9 /
+    // 23.3, 4 x 300 43.3 / 40.5, 3 x 400 58.6 / 56.2, 1 x 512 31.0 / 29.8, 2 x 384 34.0 / 33.6; beyond, where the passes move 5 TB/s, 4 x 384 64.4 / 64.2, 3 x 500
+    // 93.9 / 95.6, 4 x 450 101.2 / 104.6.  (Whole rows in 128 registers spill 10, which costs long launches 3 %.)
+    static int cache[kMaxDevices];
+    int cus = 0;
+    const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
+    if (e != hipSuccess) return e;
+    if (total > cus && total <= 16L * cus) return launch<C, D, NW, RAGGED, 2>(a, t, total, stream);
+  }
+  return launch<C, D, NW, RAGGED, 1>(a, t, total, stream);
 }
 
 }  // namespace
@@ -345,8 +359,8 @@ hipError_t triattn_proj_launch(const TriattnProjArgs& args, int C, int D, hipStr
   if (small) return triattn_proj_panels_launch(args, C, stream);
   // ragged pieces hold up to four rows, all of which must exist
   const bool ragged = args.N % 128 != 0 && args.N >= 4;
-  if (C == 128) return ragged ? launch<128, 32, OF3_TP_WAVES, true>(args, stream) : launch<128, 32, OF3_TP_WAVES, false>(args, stream);
-  return ragged ? launch<64, 16, 8, true>(args, stream) : launch<64, 16, 8, false>(args, stream);
+  if (C == 128) return ragged ? launch_tiles<128, 32, OF3_TP_WAVES, true>(args, stream) : launch_tiles<128, 32, OF3_TP_WAVES, false>(args, stream);
+  return ragged ? launch_tiles<64, 16, 8, true>(args, stream) : launch_tiles<64, 16, 8, false>(args, stream);
 }
 
 }  // namespace of3

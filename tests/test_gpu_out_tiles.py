@@ -23,3 +23,12 @@ def test_input_pass_64(n, batch):
     those of eight, with pieces of both sizes in the last round and without."""
     for incoming in (False, True):
         stages.test_trimul_proj(incoming, 64, n, batch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,batch", [(230, 1), (257, 1), (384, 1), (300, 2), (256, 4), (512, 2), (513, 2), (500, 3)])
+def test_attention_input_pass_64(n, batch):
+    """Two work-groups to a CU from one tile of 128 positions per CU (256 CUs) up to sixteen (512 tokens, two tensors: 4096 tiles; 513: more), with pieces in the
+    last round and without, whole rows and ragged ones."""
+    for ending in (False, True):
+        stages.test_triattn_proj(ending, 64, 16, n, batch)
