@@ -69,7 +69,7 @@ __device__ __forceinline__ int key2(int row) { return (row >> 4) & 1; }  // 2 ch
 // Every iteration of the tile loop issues the same loads (indices past the end are clamped, their
 // data is never read), so that the compiler can count the loads in flight and its own waits do not
 // drain the ring.
-constexpr int kRows = 4, kStages = 2;
+constexpr int kRows = kFlashRows, kStages = 2;
 #ifndef OF3_FLASH_RG_BLOCK
 #define OF3_FLASH_RG_BLOCK 8
 #endif
@@ -87,12 +87,11 @@ __device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(
 // QW = waves per row, RQ = 32-query tiles per wave: a work-group is 4 rows x 32 QW RQ queries.  A K / V^T tile read from LDS serves
 // RQ tiles of logits, so more of them are less work per logit, as long as registers leave three waves per SIMD: four tiles
 // of heads of 32 do not (24 registers spilled at 168: N = 768 520 against 360 us).  One wave per row needs one K / V^T stage in place of
-// two; two waves (128 queries of heads of 32) move the fewest bytes into LDS.  Which is taken where: triattn_flash_launch.
+// two; two waves (128 queries of heads of 32) move the fewest bytes into LDS.  Which is taken where: flash_queries in of3_tiles.h.
 // (Four waves, one work-group per CU, were slower everywhere: N = 768 395 against 375 us; one 32-query tile per wave, too:
 // 4 x 512 with head width 16 443 against 392 us.)
-constexpr int groups_per_cu(int D, int QW, int RQ) { return QW == 2 ? 2 : RQ == 4 || (RQ == 3 && D == 32) ? 3 : 4; }
 template <int D, int QW, int RQ>
-__global__ __launch_bounds__(64 * kRows * QW, QW * groups_per_cu(D, QW, RQ)) void triattn_flash_kernel(TriattnFlashArgs p, int n_qc, int n_rg, int total,
+__global__ __launch_bounds__(64 * kRows * QW, QW * flash_groups_per_cu(D, 32 * QW * RQ)) void triattn_flash_kernel(TriattnFlashArgs p, int n_qc, int n_rg, int total,
                                                                                         int per_xcd) {
   constexpr int kWaves = kRows * QW;
   constexpr int kRQ = RQ, kQW = 32 * RQ;  // queries per wave
@@ -547,37 +546,14 @@ hipError_t triattn_flash_launch(const TriattnFlashArgs& args, int D, hipStream_t
   int cus = 0;
   const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
   if (e != hipSuccess) return e;
-  // A launch of ranges of 64, 96 or 128 queries takes its rounds (work-groups over places on the chip) times a round's time in
-  // that form; a round that is not full takes 0.4 of it and the share of its places that are taken of the other 0.6.  Fitted to launches
-  // by themselves, 52 lengths of heads of 32 between 160 and 2048 and 27 of 1 to 4 templates: the form taken is 0.5 % from the best on
-  // average, with work-groups of 96 left out 2.6 %.
-  auto estimate = [&](int queries, int per_cu, double round) {
-    const long items = (long)((args.N + queries - 1) / queries) * ((args.N + kRows - 1) / kRows) * args.B * args.H, places = (long)per_cu * cus;
-    const double part = (double)(items % places) / (double)places;
-    return round * ((double)(items / places) + (part > 0 ? 0.4 + 0.6 * part : 0.0));
-  };
-  // up to three work-groups of 64 queries per CU nothing else has enough of them (heads of 32, N = 128: 6.3 against 8.0 for 128, 192: 14.0, 14.2
-  // for 96; heads of 16, 1 x 150: 9.8 and 11.3 for 96)
-  const bool few = (long)((args.N + 63) / 64) * ((args.N + kRows - 1) / kRows) * args.B * args.H <= 3L * cus;
+  if (D != 32 && D != 16) return hipErrorInvalidValue;
+  const int queries = flash_queries(args.N, (long)args.B * args.H, D, cus);
   if (D == 32) {
-    // us a launch, 64 / 96 / 128 queries (256 CUs): N = 160 10.3 / 12.4 / 14.0, 256 22.0 / 22.0 / 21.8, 300 36 / 40 / 43, 384 63.5 / 60.1 / 65.5,
-    // 400 75 / 80 / 90, 450 111 / 103 / 118, 512 143 / 146 / 140, 576 202 / 187 / 203, 768 429 / 400 / 405, 900 683 / 649 / 681, 1024 902 / 891 / 865,
-    // 1280 1658 / 1685 / 1608, 1728 3946 / 3813 / 3883, 2048 6380 / 6632 / 6190.
-    const double t64 = estimate(64, groups_per_cu(32, 1, 2), 1.06), t96 = estimate(96, groups_per_cu(32, 1, 3), 1.11),
-                 t128 = estimate(128, groups_per_cu(32, 2, 2), 1.0);
-    if (few || (t64 <= t96 && t64 <= t128)) return launch<32, 1, 2>(args, stream);
-    return t96 <= t128 ? launch<32, 1, 3>(args, stream) : launch<32, 2, 2>(args, stream);
+    if (queries == 64) return launch<32, 1, 2>(args, stream);
+    return queries == 96 ? launch<32, 1, 3>(args, stream) : launch<32, 2, 2>(args, stream);
   }
-  if (D == 16) {
-    // us a launch, 64 / 96 / 128 queries: 1 x 100 6.4 / 7.4 / 8.1, 2 x 187 17.3 / 16.1 / 18.3, 2 x 288 46 / 43 / 50, 3 x 256 47 / 49 / 47, 4 x 280 89 / 80 / 90,
-    // 2 x 384 91 / 85 / 88, 4 x 400 232 / 213 / 219, 3 x 480 264 / 236 / 237, 4 x 512 400 / 377 / 360.  (Two waves to a row, 128 queries: 4 x 512 367
-    // against 339.)
-    const double t64 = estimate(64, groups_per_cu(16, 1, 2), 0.55), t96 = estimate(96, groups_per_cu(16, 1, 3), 0.72),
-                 t128 = estimate(128, groups_per_cu(16, 1, 4), 0.75);
-    if (few || (t64 <= t96 && t64 <= t128)) return launch<16, 1, 2>(args, stream);
-    return t96 <= t128 ? launch<16, 1, 3>(args, stream) : launch<16, 1, 4>(args, stream);
-  }
-  return hipErrorInvalidValue;
+  if (queries == 64) return launch<16, 1, 2>(args, stream);
+  return queries == 96 ? launch<16, 1, 3>(args, stream) : launch<16, 1, 4>(args, stream);
 }
 
 }  // namespace of3
