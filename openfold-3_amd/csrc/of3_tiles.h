@@ -160,22 +160,22 @@ constexpr int kFlashRows = 4;
 constexpr int flash_groups_per_cu(int D, int queries) { return D == 32 ? (queries == 64 ? 4 : queries == 96 ? 3 : 2) : (queries == 128 ? 3 : 4); }
 // Queries of a work-group's range, 64, 96 or 128: the form with the least estimated time, its rounds (work-groups over places on the chip)
 // times a round's time in that form.  What is left for a last round is dealt to the CUs one by one, so that round takes as long as the CU with the
-// most of them, k of its `places`: `alone` of a round for the first, and the rest of it in equal steps for the others.  (In proportion to
-// what is left instead, with one `alone` of 0.4 for all forms, work-groups of 96 won a round early: us a launch, those / the form taken now: heads of 32, N = 257
-// 29.7 / 27.3, 281 30.2 / 28.4, two tensors of 129 15.1 / 13.9; of 128, two of 207 30.0 / 27.6; heads of 16, of 128, 3 x 228 38.5 / 36.5.)  Rounds' times and `alone` were
-// fitted to 306 launches by themselves (heads of 32: one tensor of 129 to 2030 tokens, two of 129 to 519; of 16: one to four of 129 to 512): the form taken is 0.12 and
-// 0.22 % from the best on average, at most 2.4 and 4.6 %.  us a launch, 64 / 96 / 128 queries (256 CUs): heads of 32, N = 257 27.3 / 29.7 / 31.2, 345 45.4 / 46.5 / 49.3,
-// 449 105 / 93 / 102, 512 129 / 130 / 120, 697 306 / 302 / 302, 768 386 / 368 / 369, 964 775 / 766 / 744, 1224 1523 / 1438 / 1446, 1940 5622 / 5707 / 5499, 2048 6332 / 6589 / 6128; heads
-// of 16, 2 x 187 17.1 / 15.9 / 18.4, 3 x 228 36.5 / 37.7 / 38.5, 4 x 300 103 / 101 / 100, 4 x 400 217 / 205 / 217, 4 x 512 386 / 371 / 357.
+// most of them, k of its places: `alone` of a round for the first, and the rest of it in equal steps for the others.  Rounds' times and `alone` were
+// fitted to whole passes, 238 of them in each form (launches by themselves favour the larger forms: one after another they run at a lower clock): the form taken costs a
+// pass 0.06 % (heads of 32) and 0.12 % (16) against the best on average, 1.3 % at most; with a last round in proportion to what is left, 0.42 and 0.19 % on
+// average, 3.6 % at most.  us a pass, 64 / 96 / 128 queries (256 CUs): pair stack 257 tokens 239 / 243 / 244, 345 350 / 350 / 356, 453 635 / 620 / 632, 512 764 /
+// 760 / 751, 700 1657 / 1606 / 1629, 768 1953 / 1888 / 1886, 969 3571 / 3525 / 3474, two tensors of 221 279 / 287 / 286; templates 3 x 228 546 / 550 /
+// 553, 3 x 294 852 / 864 / 853, 4 x 404 2309 / 2241 / 2251, 4 x 503 3600 / 3519 / 3491.
 inline int flash_queries(int N, long slices, int D, int cus) {  // slices: batch elements times heads
   struct Form {
     int queries;
     double round, alone;
   };
-  const Form forms[2][3] = {{{64, 0.72, 0.1}, {96, 0.93, 0.3}, {128, 1.0, 0.25}}, {{64, 1.1, 0.0}, {96, 1.15, 0.2}, {128, 1.0, 0.45}}};
+  const Form forms[2][3] = {{{64, 0.71, 0.24}, {96, 1.08, 0.0}, {128, 1.0, 0.17}}, {{64, 1.1, 0.0}, {96, 1.15, 0.2}, {128, 1.0, 0.45}}};
   auto groups = [&](int queries) { return (long)((N + queries - 1) / queries) * ((N + kFlashRows - 1) / kFlashRows) * slices; };
   // up to three work-groups of 64 queries per CU nothing else has enough of them (heads of 32, N = 128: 6.3 against 8.0 for 128; heads of 16, 1 x 150: 8.7 and
-  // 10.0 for 96); beyond four rounds of them, which read every K and V^T tile the most times, they were never more than 0.3 % ahead
+  // 10.0 for 96); beyond four rounds of them, which read every K and V^T tile the most times, they were behind but
+  // for three templates of 294 to 316, by 0.1 to 1 % of a pass
   const long small = groups(64), places64 = (long)flash_groups_per_cu(D, 64) * cus;
   if (small <= 3L * cus) return 64;
   int best = 0;

@@ -1,5 +1,5 @@
-"""The form of a launch of the bf16 attention core (flash_queries in openfold-3_amd/csrc/of3_tiles.h) against launches that were timed in all
-three forms on a part of 256 CUs: at no length more than 5 % from the best of them, at lengths around the edges of rounds."""
+"""The form of a launch of the bf16 attention core (flash_queries in openfold-3_amd/csrc/of3_tiles.h) against whole passes that were timed with each of the
+three forms on a part of 256 CUs: at lengths around the edges of rounds, never more than 1.5 % from the best of them (two runs of a pass differ by up to 1 %)."""
 import os
 import shutil
 import subprocess
@@ -8,37 +8,62 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
-# head width, batch, tokens; us a launch with 64, 96 and 128 queries to a work-group
+# head width, batch, tokens; us a pass (pair stack; head width 16: two blocks of `batch` templates) with 64, 96 and 128 queries to a work-group
 TIMED = """
-32 1 130   9.4 11.6 13.3
-32 1 209  17.7 17.7 17.2
-32 1 257  27.3 29.7 31.2
-32 1 281  28.4 30.2 32.6
-32 1 300  31.7 37.4 37.6
-32 1 345  45.4 46.5 49.3
-32 1 400  75.6 77.3 82.2
-32 1 449 105.2 93.4 102.4
-32 1 512 129.4 130.4 120.1
-32 1 576 179.9 166.9 182.9
-32 1 697 306.4 302.0 302.5
-32 1 753 379.9 360.7 361.9
-32 1 964 775.4 765.8 744.2
-32 1 1264 1626.5 1625.2 1556.1
-32 1 1940 5621.9 5707.1 5498.6
-32 1 2048 6331.8 6589.3 6127.6
-32 2 129  13.9 15.1 17.7
-32 2 155  15.1 16.2 19.8
-32 2 207  27.6 28.9 30.0
-32 2 467 214.7 196.8 201.1
-16 1 150   8.7 10.0 11.6
-16 1 450  75.2 65.6 76.3
-16 2 187  17.1 15.9 18.4
-16 2 309  47.6 52.0 50.7
-16 3 228  36.5 37.7 38.5
-16 4 201  37.1 37.1 38.5
-16 4 300 103.0 100.7 99.5
-16 4 400 217.2 204.9 216.6
-16 4 512 385.6 371.3 357.3
+32 1 129  106.6 110.0 113.2
+32 1 201  160.0 158.2 156.3
+32 1 255  198.9 201.8 198.6
+32 1 257  238.5 243.2 243.5
+32 1 273  249.1 255.6 255.6
+32 1 288  259.7 265.4 266.4
+32 1 300  280.4 291.0 287.7
+32 1 345  349.5 349.9 355.5
+32 1 399  478.5 480.2 495.1
+32 1 453  634.5 620.4 632.0
+32 1 498  742.7 744.1 733.2
+32 1 516  927.3 896.4 914.0
+32 1 588  1194.4 1166.8 1154.7
+32 1 690  1630.3 1575.4 1595.8
+32 1 700  1656.5 1605.8 1629.3
+32 1 768  1952.8 1887.5 1886.0
+32 1 969  3571.1 3525.1 3473.9
+32 1 1850  18065.5 17868.5 17777.4
+32 1 1940  20725.0 20777.6 20278.5
+32 1 2047  22888.4 23289.3 22347.7
+32 2 129  150.3 151.3 157.2
+32 2 152  166.9 168.6 176.0
+32 2 198  253.4 254.1 257.9
+32 2 221  279.1 287.4 285.9
+32 2 405  1029.0 1000.1 993.6
+32 2 428  1136.5 1110.7 1122.2
+32 2 474  1361.1 1302.7 1300.2
+16 1 129  176.2 179.5 186.2
+16 1 209  246.1 247.9 248.7
+16 1 305  427.3 431.5 443.5
+16 1 401  637.2 636.2 662.8
+16 1 449  799.5 771.3 799.6
+16 1 497  908.6 915.9 895.7
+16 2 193  345.0 352.0 355.0
+16 2 305  640.7 647.0 643.6
+16 2 385  1052.0 1043.6 1070.1
+16 2 433  1324.0 1318.1 1332.8
+16 2 481  1675.6 1662.6 1644.8
+16 3 206  464.6 468.2 465.8
+16 3 228  546.0 550.4 553.1
+16 3 294  852.0 863.8 852.9
+16 3 316  936.0 942.6 945.5
+16 3 360  1283.0 1239.3 1230.2
+16 3 404  1736.3 1677.9 1679.4
+16 3 470  2429.6 2325.1 2300.9
+16 3 503  2776.8 2704.0 2638.5
+16 4 129  327.9 327.8 347.1
+16 4 206  571.6 573.0 572.0
+16 4 228  679.8 673.8 680.1
+16 4 294  1121.6 1131.2 1122.6
+16 4 338  1498.8 1454.2 1441.2
+16 4 382  1919.8 1857.3 1824.7
+16 4 404  2308.6 2241.4 2251.2
+16 4 503  3600.4 3519.3 3491.2
 """
 
 CHECK = r"""
@@ -63,4 +88,4 @@ def test_no_form_far_from_the_best(tmp_path):
     assert out.returncode == 0
     for row, queries in zip(rows, out.stdout.split()):
         times = dict(zip(("64", "96", "128"), map(float, row[3:])))
-        assert times[queries] <= 1.05 * min(times.values()), (row, queries)
+        assert times[queries] <= 1.015 * min(times.values()), (row, queries)
