@@ -78,13 +78,12 @@ def test_triattn_fp32(starting, c, d, heads, n, batch, masked):
 
 
 @pytest.mark.parametrize("d,heads,pads", [(32, 2, 0), (16, 4, 0), (32, 2, 50)])
-def test_triattn_fp32_large_logits_and_padding(d, heads, pads):
+def test_triattn_fp32_large_logits_and_padding(d, heads, pads, c=64, n=150):
     """Logits far outside the range in which a softmax with the offset 0 is exact (queries whose largest
     logit lies beyond +-60 in base 2): the work-groups concerned must repeat the pass with running
     maxima, next to work-groups that never need it; with a padded tail (runs of masked keys the first
     pass leaves out, padded rows that only the second pass serves)."""
     lib()
-    c, n = 64, 150
     gen = torch.Generator().manual_seed(4400 + d + pads)
     p = orc.make_triattn_params(gen, c, d, heads)
     p["mha.linear_q.weight"] = p["mha.linear_q.weight"] * 14.0   # q.k / sqrt(d) of +-40 and more
@@ -97,6 +96,13 @@ def test_triattn_fp32_large_logits_and_padding(d, heads, pads):
     if pads:  # padded rows: -1e9 absorbs moderate logits only, and these are not moderate; compare the real rows
         got, want = got[: n - pads], want[: n - pads]
     _maxerr("triattn fp32 large logits", got, want)
+
+
+# the core of of3_split.h's shapes in both of its forms: work-groups of 64 queries (a last range of 128 would hold 22, 4), of 128 (72, 102 or all in the last)
+@pytest.mark.parametrize("c,d,pads,n", [(128, 32, 0, 150), (128, 32, 0, 200), (128, 32, 40, 256), (128, 32, 0, 100), (64, 16, 0, 132), (64, 16, 0, 200),
+                                        (64, 16, 50, 230)])
+def test_triattn_fp32_large_logits_both_forms(c, d, pads, n):
+    test_triattn_fp32_large_logits_and_padding(d, 4, pads, c, n)
 
 
 def test_trimul_fp32_reference_unit_test_shape():

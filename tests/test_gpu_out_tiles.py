@@ -17,6 +17,20 @@ def test_stages(c, d, n, batch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("transposed", [False, True])
+def test_attention_long_rows(transposed):
+    """Above 1536 tokens the attention's pass takes tiles of 128: here off their multiples, so that a tile lies in two rows."""
+    stages.test_triattn_out(transposed, 1, 128, 32, 1537, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [897, 1024])
+def test_planes_of_1024(n):
+    """64 channels: the planes of x are 1024 wide and the pass that reads them takes tiles of 128, ragged rows and whole ones."""
+    stages.test_trimul_out(1, 64, n, 1)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,batch", [(256, 1), (257, 1), (187, 2), (200, 2), (331, 1), (63, 9)])
 def test_input_pass_64(n, batch):
     """64 channels on both sides of two tiles per CU (256 CUs: 512 tiles at 256 tokens, 585 at 257), where work-groups of four waves take over from
