@@ -606,6 +606,7 @@ hipError_t launch_contract8(const bf16_t* a, const bf16_t* b, bf16_t* x, int pla
 // quarters of the bytes through the CU's L1, and 1024 work-groups for 128 planes, all of them at once): us a launch, tiles of 64 x 64 with four
 // panels / with three / 64 x 128: N = 200 11.7 / 11.3 / 10.5, 170 8.9 / 8.2 / 8.3, two templates of 187 8.9 / 8.4 / 8.3, 128 5.1 / 5.1 / 5.4.
 constexpr int kShortM = 64, kShortRing = 3;
+static_assert(kShortRing == 3, "panel_ready waits for all but one panel");
 constexpr int kShortSide = kShortM * 4;  // u32x4 slots of the m side of a panel
 constexpr int short_panel(int tn) { return (kShortM + tn) * 4; }
 constexpr size_t short_lds(int tn) { return (size_t)kShortRing * short_panel(tn) * 16; }
@@ -663,9 +664,7 @@ __global__ __launch_bounds__(256) void contract_short_kernel(const bf16_t* __res
   const int ahead = nk < kShortRing - 1 ? nk : kShortRing - 1;
   for (int q = 0; q < ahead; ++q) issue(q);
   auto panel_ready = [&](int p) {
-    const int newer = nk - 1 - p;  // panels requested after this one: up to two, two loads each
-    if (newer >= kShortRing - 2) wait_vmcnt<(kShortRing - 2) * (1 + NT)>();
-    else if (newer == 1) wait_vmcnt<1 + NT>();
+    if (p + 1 < nk) wait_vmcnt<1 + NT>();  // the loads of the one panel requested after this one
     else wait_vmcnt<0>();
     wait_lds_reads();  // of the panel before
     __builtin_amdgcn_s_barrier();
@@ -740,7 +739,9 @@ hipError_t trimul_contract_launch(const bf16_t* a, const bf16_t* b, bf16_t* x, i
     const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
     if (e != hipSuccess) return e;
     // Above 192 tokens while the 256-wide tiles are up to two rounds, us a launch with those / with these: 128 planes, 256 tokens 14.2 / 11.4 (these on
-    // tiles of 64 x 64: already level), 192, three templates of 230 18.9 / 15.7, 256, four of 240 20.9 / 19.9.
+    // tiles of 64 x 64: already level), 192, three templates of 230 18.9 / 15.7, 256, four of 240 20.9 / 19.9.  At 256 planes by whole passes, whose projection
+    // leaves the operands in the caches: four templates of 193 tokens 559 / 553, 208 567 / 561, 224 611 / 600, 225 670 / 661, 240 704 / 698, 249 719 / 715, 256 729 /
+    // 725, three of 225 550 / 541.  With operands from memory the 256-wide ones win there: 200 17.1 / 17.6, 225 22.2 / 24.6, 256 22.3 / 24.0.
     if (transposed || nk <= 6 || planes <= cus) {
       const int order = variant == 2 ? 128 : 256;
       return short_tile_n(nk) == 128 ? launch_contract_short<128>(a, b, x, planes, Np, nk, order, transposed, stream)

@@ -1,6 +1,6 @@
 """The bf16 contraction's tiles of 64 x 64, from 193 tokens on of 64 x 128 (contract_short_kernel): one to eight panels (fewer than its ring holds, as many, more), tiles that
 are full, hold one 32 x 32 part in use, or leave waves without any.  The transposed form: test_gpu_pair_join.py, against this one.
-Beside them the tiles of 256 x 128 and 256 x 256 at 193 to 256 tokens, which more planes than half of the CUs take there."""
+Beside them the tiles of 256 x 128 and 256 x 256 at 193 to 256 tokens, which more planes than CUs take there."""
 import pytest
 import torch
 
