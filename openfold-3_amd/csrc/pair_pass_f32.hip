@@ -150,7 +150,8 @@ __global__ __launch_bounds__(64 * NW, 2) void trimul_proj_pass(TrimulF32 p, int 
     wait_vmcnt<0>();  // the rows in flight since a product ago, ahead of the stores, so that nobody waits for these
     // channels in the lanes, positions in the registers: registers 8 st .. + 7 are the k-values 16 st + 8 (e >> 2)
     // + 4 lh + (e & 3), stored as the 8 consecutive columns 16 st + 8 lh .. of the panel row (a and b in the same
-    // order, which is all a sum over k needs); positions past N are zero rows and store the panel's padding
+    // order, which is all a sum over k needs); positions past N are copies of a real row, and the zeros of msk make the
+    // panel's padding of them
     if (t.r < N) {
       const Lane out = lane_here();
       const int l32 = out.l32, lh = out.lh;
@@ -498,6 +499,8 @@ __global__ __launch_bounds__(6 * C / PARTS) void triattn_proj_pass(TriattnF32 p,
     // registers, positions in the lanes; v the other way round.  Registers 8 st .. + 7 of a lane are its operand
     // for step st (narrow heads: q, k have one step, that of head 2 ot + st; lane l32 of the v tile is row
     // l32 % 16 of head 2 ot + l32 / 16, its second term row 16 + l32 % 16).
+    // Positions past N store copies of the last real one: their keys and values are the reader's to leave out (a bias of -infinity there in the
+    // core, which gives them no weight; a value that is not a number makes its real copy's result one as well), their queries' results nobody stores.
     f32x16_t acc;
     bf16_t* dst;
     long second;

@@ -6,7 +6,8 @@
 // queries (two 32-query tiles) of one row.  Three work-groups share a CU (heads of 16: four), so that the products of one run under the exponentials and
 // splits of the others.  Bound by matrix and vector time at the clock that both leave (N = 768, heads of 32: 901 us a launch, matrix
 // pipe 48 %, vector pipe 63 %, 1.67 GHz; three bf16 terms 1446; heads of 16, three templates of 200: 54 us, 22 and 59 %; 88).
-// A 32 x 32 tile is 80 vector instructions (169 ns on a SIMD alone) and 12 products (180, 300 with all CUs busy).
+// A 32 x 32 tile is 98 vector instructions, 80 of them 16 each of exponentials, fused multiply-adds and additions and 32 of the splits (169 ns on a SIMD
+// alone), the rest the loop's own, and 12 products (180, 300 with all CUs busy).
 //   S^T = K Q^T  (rows = keys, columns = queries), three products per k-step, started from the triangle bias (the
 //                accumulator is loaded with it).  Logits are in natural units times the scales of q and k, a power of
 //                two that the bias and the mask bias carry too, and not pre-multiplied by log2(e): a row of masked keys

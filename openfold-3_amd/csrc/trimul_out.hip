@@ -6,7 +6,8 @@
 // LDS; the gate is recomputed from z instead of being stored by the input pass, which
 // saves one full write and one full read of a z-sized tensor.
 //
-// HBM bound: reads x and z once, writes out once.
+// Reads x and z once, writes out once.  Bound by its instructions beside the bytes: at N = 768 (128 channels) 4.1 TB/s, where a large copy has 4.8, with the
+// vector pipe 64 % busy.
 //
 // Tiles are TP = 128 or 64 positions: the whole TP-wide pieces of every row first, then, when N is not a multiple
 // of TP, the remaining columns in pieces of 2^s columns x TP / 2^s consecutive rows (2^s the smallest
@@ -300,7 +301,7 @@ hipError_t trimul_out_launch(const TrimulOutArgs& args, int C, int CH, hipStream
   if (small) return trimul_out_panels_launch(args, C, stream);
   // at 64 channels the stores of a tile of 64 have 32-bit offsets from its first position: 8 rows, 64 columns
   const bool fits = C != 64 || 8 * args.z_view.stride_r + 64 * args.z_view.stride_k + C < (1l << 30);
-  const bool half = fits && out_tile_positions(C, args.N, true) == 64;
+  const bool half = fits && out_tile_positions(args.N, true) == 64;
   if (C == 128) return half ? launch_tiles<128, 64>(args, stream) : launch_tiles<128, 128>(args, stream);
   return half ? launch_tiles<64, 64>(args, stream) : launch_tiles<64, 128>(args, stream);
 }
