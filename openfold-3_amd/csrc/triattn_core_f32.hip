@@ -439,8 +439,9 @@ hipError_t triattn_core_h2_f32_launch(const TriattnF32& p, hipStream_t stream) {
   // 64 queries of four rows instead of 128 of two, with one barrier a key tile less and twice the K and V^T through LDS, where the last range of
   // 128 would be at most half full.  us a launch, 64 / 128: heads of 16, templates 1 x 140 13.7 / 16.6, 2 x 187 30.6 / 34.1, 4 x 300 190 / 205, 1 x 400 109
   // / 119; others level (2 x 384 171.5 / 170.5, a pass of 3 x 200 874 / 870).  Heads of 32, whose K and V^T are twice as long: N = 300 80 / 87, 400
-  // 177 / 184, 550 396 / 399, 700 level; others slower (128 12.6 / 12.3, 384 147 / 141, 768 931 / 891); and where 128 leave no second round only if
-  // the last of those is a quarter (150 18.7 / 21.4; 180 27.0 / 26.2).
+  // 177 / 184; others slower (128 12.6 / 12.3, 384 147 / 141, 768 931 / 891); and where 128 leave no second round only if the last of those is a quarter
+  // (150 18.7 / 21.4; 180 27.0 / 26.2).  Beyond 512 tokens the unused half is at most a tenth of a launch, which the second reading of K and V^T costs: whole pair
+  // stacks 64 / 128, us, 300 578 / 587, 390 1044 / 1053, 430 1233 / 1253, 448 1298 / 1304, but 520 1946 / 1929, 550 2202 / 2183, 576 2286 / 2293, 660 3244 / 3257.
   static int cache[kMaxDevices];
   int cus = 0;
   const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
@@ -449,7 +450,7 @@ hipError_t triattn_core_h2_f32_launch(const TriattnF32& p, hipStream_t stream) {
   const int last = p.N > Wide::kQueries ? p.N % Wide::kQueries : 0;
   if (p.D == 16) return last > 0 && last <= 64 ? launch<1, 1>(p, stream) : launch<1, 2>(p, stream);
   const long wide = (long)((p.N + Wide::kQueries - 1) / Wide::kQueries) * ((p.N + Wide::kRows - 1) / Wide::kRows) * p.B * p.H;
-  const bool narrow = p.N <= 640 && last > 0 && last <= (wide > (long)kPerCu<2> * cus ? 64 : 32);
+  const bool narrow = p.N <= 512 && last > 0 && last <= (wide > (long)kPerCu<2> * cus ? 64 : 32);
   return narrow ? launch<2, 1>(p, stream) : launch<2, 2>(p, stream);
 }
 
