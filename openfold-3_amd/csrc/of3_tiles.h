@@ -147,6 +147,8 @@ inline LastRound last_round(long tiles, int grid) {
 // the multiplication's pass at 128 channels: N = 300 24.7 / 22.9, 384 35.0 / 32.0, 451 52.8 / 47.8, 768 118 / 116, 850 157 / 148, 1100 236 / 226, 1700
 // 546 / 536; at 64, three templates of 300 30.8 / 25.8, four of 512 95.0 / 86.9.  Of the attention's at 128: N = 300 21.5 / 21.4, 384 31.9 /
 // 28.5, 640 79.8 / 75.1, 896 148 / 143, 1280 275 / 269; at 64 its launch does not ask: two work-groups of eight waves share a CU there, 42.4 / 42.7 for two of 512.
+// Launches by themselves of the attention's off multiples of 64 between 500 and 740 tokens prefer 128 (540 52.0 / 54.3, 600 61.4 / 64.6, 720 85.9 / 89.3), whole
+// passes do not: pair stack 540 963 / 961, 600 1209 / 1201, 720 1741 / 1736, and 257 261 / 255, 580 1173 / 1157, 1000 3702 / 3707.
 // Beyond 1536 tokens the attention's lose (1536 401 / 402, 1792 528 / 546, 2048 708 / 742: more rows open in memory at once).  The multiplication's go
 // either way there (128 channels 1600 462 / 450, 1700 521 / 522, 1792 564 / 571, others within 1 %; 64 channels 1600 221 / 202, 1700 250 / 240, 1792 263 / 273, 1920 302 / 314)
 // and keep to the same line.  x loses at whole multiples of 1024, where the 128-byte pieces of a tile's planes are a power of two apart (929 170 /

@@ -337,7 +337,9 @@ hipError_t launch_tiles(const TriattnProjArgs& a, hipStream_t stream) {
   if constexpr (C == 64) {
     // Two work-groups to a CU, whose barriers do not coincide, from more than one tile per CU up to sixteen; us a launch, one / two: templates 2 x 300 24.9 /
     // 23.3, 4 x 300 43.3 / 40.5, 3 x 400 58.6 / 56.2, 1 x 512 31.0 / 29.8, 2 x 384 34.0 / 33.6; beyond, where the passes move 5 TB/s, 4 x 384 64.4 / 64.2, 3 x 500
-    // 93.9 / 95.6, 4 x 450 101.2 / 104.6.  (Whole rows in 128 registers spill 10, which costs long launches 3 %.)
+    // 93.9 / 95.6, 4 x 450 101.2 / 104.6.  Launches one after another prefer one earlier (2 x 450 47.1 / 48.9, 3 x 360 43.8 / 46.2), whole passes do not: 2 x 390
+    // 1120 / 1109, 2 x 450 1441 / 1433, 3 x 360 1303 / 1288, 3 x 430 2008 / 1990, 2 x 512 1769 / 1772, 4 x 256 773 / 776; beyond, 3 x 512 2695 / 2712, 4 x 512 3489 /
+    // 3517.  (Whole rows in 128 registers spill 10, which costs long launches 3 %.)
     static int cache[kMaxDevices];
     int cus = 0;
     const hipError_t e = per_device(cache, [](int dev, int* v) { return cu_count(dev, v); }, &cus);
